@@ -6,9 +6,10 @@ There is no CPU or eager fallback.
 import ctypes
 import os
 
-from .build import LIB_PATH
+from .build import LIB_PATH, NATIVE_PATH
 
 _lib = None
+_native = None
 
 c_i32, c_i64, c_u32, c_f32 = ctypes.c_int32, ctypes.c_int64, ctypes.c_uint32, ctypes.c_float
 c_vp, c_sz, c_int = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int
@@ -20,8 +21,12 @@ SIGNATURES = {
     "fo_num_cu": ([], c_int),
     "fo_packbits": ([c_vp, c_i64, c_int, c_vp, c_vp], c_int),
     "fo_segment_packbits": ([c_vp, c_vp, c_vp, c_i32, c_int, c_vp, c_vp], c_int),
+    "fo_segment_packbits_scan": ([c_vp, c_i64, c_vp, c_int, c_i32, c_int, c_vp, c_i64, c_vp, c_vp, c_u32, c_vp],
+                                 c_int),
     "fo_prefill_plan": ([c_vp, c_sz, c_vp, c_vp, c_sz, c_vp, c_vp, c_u32, c_u32, c_u32, c_u32,
                          c_u32, c_u32, c_u32, c_int, c_u32, c_int, c_vp, c_vp], c_int),
+    "fo_plan_batch": ([c_vp, c_vp, c_i32, c_i32, c_i32, c_int, c_vp], c_int),
+    "fo_plan_tables": ([c_vp, c_vp, c_i32, c_i32, c_i32, c_int, c_vp, c_vp], c_int),
     "fo_sparse_block_table": ([c_vp, c_u32, c_u32, c_vp, c_vp, c_i64, c_vp], c_int),
     "fo_decode_sizes": ([c_vp, c_vp, c_u32, c_u32, c_u32, c_u32, c_vp, c_vp, c_vp], c_int),
     "fo_decode_sparse": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 9 + [c_vp, c_vp], c_int),
@@ -63,6 +68,24 @@ def lib():
             fn.restype = restype
         _lib = handle
     return _lib
+
+
+def native():
+    """Load (once) and return the extension that makes the ordinary calls (bindings.cpp).  torch is
+    imported by then, so the HIP runtime the extension finds is torch's own."""
+    global _native
+    if _native is None:
+        lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(
+                "flashomni_amd: %s is missing; build it with `python -m flashomni_amd.build` "
+                "(there is no fallback path)" % NATIVE_PATH)
+        import torch  # noqa: F401
+        from . import _native as module
+        from .gemm import _gemm_scratch_at
+        module.set_gemm_scratch(_gemm_scratch_at)
+        _native = module
+    return _native
 
 
 def check(rc):

@@ -92,10 +92,8 @@ class PlannedBatch:
     def __init__(self, float_workspace_buffer, qo_indptr_host, kv_indptr_host, qo_indptr_dev,
                  kv_indptr_dev, num_qo_heads, num_kv_heads, block_q, block_kv, share_rows=True,
                  worklist=None, gqa_packed=False):
-        L = _lib.lib()
         self.device = float_workspace_buffer.device
         self.float_ws = float_workspace_buffer
-        self.qo_indptr, self.kv_indptr = qo_indptr_dev, kv_indptr_dev
         self.num_qo_heads, self.num_kv_heads = num_qo_heads, num_kv_heads
         self.block_q, self.block_kv = block_q, block_kv
         batch_size = qo_indptr_host.numel() - 1
@@ -107,52 +105,35 @@ class PlannedBatch:
         # whose requests are `group` times as long, with num_kv_heads heads.
         self.gqa_packed = bool(gqa_packed) and num_kv_heads != num_qo_heads
         self.symbol_heads = num_kv_heads if self.gqa_packed else num_qo_heads
-        qo_rows_host = qo_indptr_host
-        if self.gqa_packed:
-            rows = qo_indptr_host.to(torch.int64) * (num_qo_heads // num_kv_heads)
-            if int(rows[-1]) >= 2 ** 31:
-                raise RuntimeError("Failed to plan prefill with error: too many packed q rows")
-            qo_rows_host = rows.to(torch.int32).contiguous()
-        n_blk = torch.zeros(3, dtype=torch.int64)
-        _lib.check(L.fo_decode_sizes(_lib.ptr(qo_rows_host), _lib.ptr(kv_indptr_host), batch_size,
-                                     self.symbol_heads, block_q, block_kv,
-                                     n_blk[0:].data_ptr(), n_blk[1:].data_ptr(), n_blk[2:].data_ptr()))
-        n_q_blk, max_rows, max_nnz = (int(v) for v in n_blk)
-        if max_nnz >= 2 ** 31:
-            raise RuntimeError("Failed to plan prefill with error: work list too large")
-        table = torch.empty((2, max(n_q_blk, 1)), dtype=torch.int32)
-        _lib.check(L.fo_sparse_block_table(_lib.ptr(qo_rows_host), batch_size, block_q,
-                                           table[0].data_ptr(), table[1].data_ptr(), n_q_blk,
-                                           n_blk[0:].data_ptr()))
-        self.blk_table = table.to(self.device)
-        self.n_q_blk = n_q_blk
-        qlen = (qo_indptr_host[1:] - qo_indptr_host[:-1]).to(torch.int64)
-        klen = (kv_indptr_host[1:] - kv_indptr_host[:-1]).to(torch.int64)
-        q_base = torch.zeros(batch_size + 1, dtype=torch.int64)
-        kv_base = torch.zeros(batch_size + 1, dtype=torch.int64)
-        q_base[1:] = torch.cumsum((qlen + block_q - 1) // block_q, 0)
-        kv_base[1:] = torch.cumsum((klen + block_kv - 1) // block_kv, 0)
-        self.q_blk_base = q_base.to(torch.int32).to(self.device)
-        self.kv_blk_base = kv_base.to(torch.int32).to(self.device)
-        self.n_kv_blk = int(kv_base[-1])
-        self.max_kv_len = int(klen.max()) if klen.numel() else 0
-        # sizes the tensors given to run() must have (checked there without reading the device):
-        # token counts, and the packed bytes of the byte-aligned per-request segments
-        self.total_q_rows = int(qo_indptr_host[-1]) if qo_indptr_host.numel() else 0
-        self.total_kv_rows = int(kv_indptr_host[-1]) if kv_indptr_host.numel() else 0
-        qrows = (qo_rows_host[1:] - qo_rows_host[:-1]).to(torch.int64)
-        nqb = (qrows + block_q - 1) // block_q   # symbol rows (q blocks or packed tiles) per request
-        nkb = kv_base[1:] - kv_base[:-1]
-        self.min_info_bytes = int(((nqb * self.symbol_heads + 7) // 8).sum())
-        self.min_kv_info_bytes = int(((nqb * nkb * self.symbol_heads + 7) // 8).sum())
-        if worklist is None or worklist.max_rows < max_rows or worklist.max_nnz < max_nnz:
-            worklist = DecodedWorkList(max_rows, max_nnz, self.symbol_heads, self.device)
+        # Sizes and tables of the batch.  total_q_rows / total_kv_rows / min_*_bytes are what the
+        # tensors given to run() must have (checked there without reading the device): token counts,
+        # and the packed bytes of the byte-aligned per-request segments.
+        index = self.device.index if self.device.index is not None else torch.cuda.current_device()
+        self.native, self.tables, sizes = _lib.native().plan(
+            qo_indptr_host, kv_indptr_host, num_qo_heads, num_kv_heads, self.gqa_packed, index,
+            qo_indptr_dev, kv_indptr_dev)
+        (self.n_q_blk, self.n_kv_blk, self.max_rows, self.max_nnz, self.total_q_rows, self.total_kv_rows,
+         self.min_info_bytes, self.min_kv_info_bytes, self.max_kv_len, *self._table_at) = sizes
+        self.qo_indptr = self.table(0) if qo_indptr_dev is None else qo_indptr_dev
+        self.kv_indptr = self.table(1) if kv_indptr_dev is None else kv_indptr_dev
+        if worklist is None or worklist.max_rows < self.max_rows or worklist.max_nnz < self.max_nnz:
+            worklist = DecodedWorkList(self.max_rows, self.max_nnz, self.symbol_heads, self.device)
         self.worklist = worklist
-        self.max_rows = max_rows
         self.share_rows = share_rows
         self.split_ok = self._split_ws_ok()
         # [is_full, stream, streams already ordered after it] of the list the work-list buffers hold
         self.decoded = None
+
+    def table(self, i: int) -> torch.Tensor:
+        """One of the device tables (order: see fo_batch_sizes): the indptrs of the q and kv tokens, of their
+        128-token blocks and of the symbol bits, then the request and q block of every symbol row."""
+        return self.tables.narrow(0, self._table_at[(0, 1, 4, 5, 6, 7, 2, 3)[i]],
+                                  self.batch_size + 1 if i < 6 else max(self.n_q_blk, 1))
+
+    blk_req = property(lambda self: self.table(6))
+    blk_qb = property(lambda self: self.table(7))
+    q_blk_base = property(lambda self: self.table(2))
+    kv_blk_base = property(lambda self: self.table(3))
 
     def float_ws_bytes(self) -> int:
         return self.float_ws.numel() * self.float_ws.element_size()
@@ -195,7 +176,7 @@ class PlannedBatch:
         with _lib.device_guard(self.device):
             _lib.check(_lib.lib().fo_decode_sparse(
                 _lib.ptr(tensors[0]), _lib.ptr(tensors[1]), _lib.ptr(tensors[2]), _lib.ptr(tensors[3]),
-                _lib.ptr(self.blk_table[0]), _lib.ptr(self.blk_table[1]), _lib.ptr(self.kv_indptr),
+                _lib.ptr(self.blk_req), _lib.ptr(self.blk_qb), _lib.ptr(self.kv_indptr),
                 self.n_q_blk, self.symbol_heads, self.block_kv, int(bool(is_full)),
                 _lib.ptr(wl.row_req), _lib.ptr(wl.row_qb), _lib.ptr(wl.row_head), _lib.ptr(wl.kv_row_ptr),
                 _lib.ptr(wl.kv_idx), _lib.ptr(wl.counts), _lib.ptr(wl.order), _lib.ptr(wl.sched),
@@ -205,6 +186,20 @@ class PlannedBatch:
         # stream must be ordered after it)
         self.decoded = (bool(is_full), stream, [])
         return wl
+
+    def attention(self, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full,
+                  out, lse, return_lse, sm_scale, logits_soft_cap, hnd):
+        """Decode and attention of an ordinary call (16-bit operands, nothing to convert) in one native
+        call; None where the call needs the general path."""
+        wl = self.worklist
+        r = _lib.native().attention(
+            self.native, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full, out,
+            lse, return_lse, sm_scale, logits_soft_cap, hnd,
+            (wl.row_req, wl.row_qb, wl.row_head, wl.kv_row_ptr, wl.kv_idx, wl.counts, wl.order, wl.sched, wl.scratch,
+             wl.shares), self.float_ws if self.split_ok else None)
+        if r is not None:
+            self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
+        return r
 
     def reuse_decoded(self, is_full: bool) -> DecodedWorkList:
         """The work list of the last decode, ordered before the current stream's work."""
@@ -358,6 +353,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         self._backend = backend  # accepted for compatibility; there is one HIP code path
         self._plan_info = None
         self._planned = None  # PlannedBatch of the last plan()
+        self._pin_offset = 0  # free part of the pinned mirror (plans are laid out one behind the other)
 
     @property
     def is_cuda_graph_enabled(self) -> bool:
@@ -370,6 +366,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         self._pin_memory_int_workspace_buffer = torch.empty(
             self._int_workspace_buffer.shape, dtype=self._int_workspace_buffer.dtype, device="cpu",
             pin_memory=True)
+        self._pin_offset = 0
         # whether rows may be shared between workgroups depends on the float workspace, and a list
         # decoded for the old buffers' share table must not be reused
         if self._planned is not None:
@@ -470,38 +467,30 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
                         batch_size, self._fixed_batch_size))
             self._qo_indptr_buf.copy_(qo_indptr)
             self._kv_indptr_buf.copy_(kv_indptr)
-        else:
-            self._qo_indptr_buf = qo_indptr_host.to(self.device)
-            self._kv_indptr_buf = kv_indptr_host.to(self.device)
 
         self._cached_q_data_type = q_data_type
         self._cached_kv_data_type = kv_data_type
 
-        L = _lib.lib()
-        stream = _lib.current_stream(self.device)
         plan_info = torch.empty(15, dtype=torch.int64)
-        with torch.cuda.device(self.device):
+        graph = self.is_cuda_graph_enabled
+        with _lib.device_guard(self.device):
             try:
-                _lib.check(L.fo_prefill_plan(
-                    _lib.ptr(self._float_workspace_buffer),
-                    self._float_workspace_buffer.numel() * self._float_workspace_buffer.element_size(),
-                    _lib.ptr(self._int_workspace_buffer),
-                    _lib.ptr(self._pin_memory_int_workspace_buffer),
-                    self._int_workspace_buffer.numel() * self._int_workspace_buffer.element_size(),
-                    _lib.ptr(qo_indptr_host), _lib.ptr(kv_indptr_host),
-                    self._max_total_num_rows or total_num_rows, batch_size, num_qo_heads,
-                    num_kv_heads, head_dim_qk, head_dim_vo, 1, int(self.is_cuda_graph_enabled),
-                    q_data_type.itemsize, 0, _lib.ptr(plan_info), stream))
+                self._pin_offset = _lib.native().host_plan(
+                    self._float_workspace_buffer, self._int_workspace_buffer,
+                    self._pin_memory_int_workspace_buffer, self._pin_offset, qo_indptr_host, kv_indptr_host,
+                    self._max_total_num_rows or total_num_rows, num_qo_heads, num_kv_heads, graph,
+                    q_data_type.itemsize, plan_info)
             except RuntimeError as e:  # same wording as csrc/batch_sparseFA.cu:61
                 raise RuntimeError("Failed to plan prefill with error: " + str(e)) from None
-        self._plan_info = plan_info
-
-        self._planned = PlannedBatch(
-            self._float_workspace_buffer, qo_indptr_host, kv_indptr_host, self._qo_indptr_buf,
-            self._kv_indptr_buf, num_qo_heads, num_kv_heads, sparse_block_size_for_q,
-            sparse_block_size_for_kv, share_rows=self._share_rows,
-            worklist=self._planned.worklist if self._planned is not None else None,
-            gqa_packed=gqa_symbols != "per_q_head")
+            self._plan_info = plan_info
+            self._planned = PlannedBatch(
+                self._float_workspace_buffer, qo_indptr_host, kv_indptr_host,
+                self._qo_indptr_buf if graph else None, self._kv_indptr_buf if graph else None, num_qo_heads,
+                num_kv_heads, sparse_block_size_for_q, sparse_block_size_for_kv, share_rows=self._share_rows,
+                worklist=self._planned.worklist if self._planned is not None else None,
+                gqa_packed=gqa_symbols != "per_q_head")
+        if not graph:
+            self._qo_indptr_buf, self._kv_indptr_buf = self._planned.qo_indptr, self._planned.kv_indptr
 
         self._num_qo_heads = num_qo_heads
         self._num_kv_heads = num_kv_heads
@@ -515,15 +504,17 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         self._rope_scale = rope_scale
         self._rope_theta = rope_theta
 
-        self._sparse_info_indptr_base = _compute_sparse_info_indptr(
-            self._qo_indptr_buf, num_qo_heads, self._sparse_block_size_for_q, device=self.device)
-        self._sparse_kv_info_indptr_base = _compute_sparse_kv_info_indptr(
-            self._qo_indptr_buf, self._kv_indptr_buf, num_qo_heads, self._sparse_block_size_for_q,
-            self._sparse_block_size_for_kv, device=self.device)
-
     begin_forward = plan
 
     # names kept for callers that inspect the wrapper
+    @property
+    def _sparse_info_indptr_base(self):
+        return self._planned.table(4)
+
+    @property
+    def _sparse_kv_info_indptr_base(self):
+        return self._planned.table(5)
+
     @property
     def _worklist(self):
         return None if self._planned is None else self._planned.worklist
@@ -586,6 +577,14 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         same from here.  Pass True to skip the decode and run the work list of the previous
         ``decode``/``run``: the caller then vouches that the four symbol tensors have not changed.
         """
+        pb = self._planned
+        if pb is not None and not reuse_decoded and q_scale is None and k_scale is None and q_lo is None \
+                and k_lo is None and q.dtype is self._cached_q_data_type and k.dtype is self._cached_kv_data_type:
+            r = pb.attention(q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full,
+                             out, lse, return_lse, self._sm_scale, self._logits_soft_cap or 0.0,
+                             self._kv_layout == "HND")
+            if r is not None:
+                return r
         if self._plan_info is None:
             raise RuntimeError("plan() must be called before run()")
         if q.dim() != 3 or v.dim() != 3:
@@ -604,7 +603,6 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
             out = torch.zeros(q.shape[:-1] + v.shape[-1:], dtype=out_dtype, device=q.device)
         else:
             _check_shape_dtype_device(out, q.shape[:-1] + v.shape[-1:], out_dtype, q.device, "out")
-        pb = self._planned
         if reuse_decoded:
             pb.reuse_decoded(is_full)
         else:

@@ -1,0 +1,550 @@
+// Native call path of the Python API: argument checks, allocation and the C-ABI call of an ordinary
+// call in one step.
+//
+// A call of the package is a handful of tensors and numbers.  Checked attribute by attribute in Python
+// and passed through ctypes (25 + 45 arguments for one attention call), its host side took 15 us per
+// GEMM and 39 us per attention call, more than the GPU needs for a small one (attention over 384 tokens
+// of two heads: 28 us of kernels).  Here the same checks read the tensors' C++ fields.
+//
+// Every function returns None when a call is not an ordinary one (another device than the current one, a
+// tensor that has to be converted first, a wrong shape or type): the Python code then goes through its
+// own checks, converts or raises, so that errors have one source and this file none.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <cstring>
+#include <memory>
+#include <vector>
+
+#include "../../include/flashomni_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+// None or a tensor
+bool opt_tensor(PyObject* o, const Tensor** t) {
+  if (o == Py_None) {
+    *t = nullptr;
+    return true;
+  }
+  if (!THPVariable_Check(o)) return false;
+  *t = &THPVariable_Unpack(o);
+  return true;
+}
+
+bool whole(PyObject* o, int64_t* v) {
+  if (!PyLong_Check(o)) return false;
+  *v = PyLong_AsLongLong(o);
+  if (*v == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+bool real(PyObject* o, double* v) {
+  if (!PyFloat_Check(o) && !PyLong_Check(o)) return false;
+  *v = PyFloat_AsDouble(o);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
+
+void* data(const Tensor* t) { return t ? t->data_ptr() : nullptr; }
+
+bool on(const Tensor& t, int dev) { return t.is_cuda() && t.get_device() == dev; }
+
+// a contiguous tensor of the given type on the device
+bool flat(const Tensor& t, at::ScalarType type, int dev) {
+  return on(t, dev) && t.scalar_type() == type && t.is_contiguous();
+}
+
+int act_code(at::ScalarType t) { return t == at::kBFloat16 ? FO_BF16 : t == at::kHalf ? FO_F16 : -1; }
+
+void* stream_of(int dev) { return c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream(); }
+
+Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType type, int dev) {
+  return at::empty(sizes, at::TensorOptions().dtype(type).device(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(dev))));
+}
+
+PyObject* raise_last() {
+  PyErr_SetString(PyExc_RuntimeError, fo_last_error());
+  return nullptr;
+}
+
+#define FALL_BACK_UNLESS(cond) \
+  do {                         \
+    if (!(cond)) Py_RETURN_NONE; \
+  } while (0)
+
+#define TORCH_GUARD_BEGIN try {
+#define TORCH_GUARD_END                              \
+  }                                                  \
+  catch (const std::exception& e) {                  \
+    PyErr_SetString(PyExc_RuntimeError, e.what());   \
+    return nullptr;                                  \
+  }
+
+// x [B, M, K] and w [N, K] of a GEMM: contiguous, one 16-bit type, on the current device
+bool gemm_operands(const Tensor& a, const Tensor& b, int* dev, int* code) {
+  if (!a.is_cuda() || a.dim() != 3 || b.dim() != 2) return false;
+  *dev = a.get_device();
+  *code = act_code(a.scalar_type());
+  return *code >= 0 && *dev == c10::hip::current_device() && a.is_contiguous() && flat(b, a.scalar_type(), *dev) &&
+         a.size(2) == b.size(1) && a.size(0) > 0 && a.size(1) > 0 && a.size(0) < (1 << 30) && a.size(1) < (1 << 30) &&
+         b.size(0) < (1 << 30) && a.size(2) < (1 << 30);
+}
+
+bool gemm_symbols(const Tensor* info, const Tensor* indptr, int dev, int64_t batch, int64_t m, int64_t heads,
+                  int64_t text, int64_t q_size) {
+  if (!info || !indptr || !flat(*info, at::kByte, dev) || !flat(*indptr, at::kInt, dev)) return false;
+  const int64_t last = (text + m - 1) / q_size;
+  return indptr->numel() == batch + 1 && info->numel() >= ((last + 1) * heads + 7) / 8;
+}
+
+// scratch of the long launches: the pool that the Python side keeps per device and stream
+PyObject* g_gemm_scratch = nullptr;  // callable (device index, stream, bytes) -> tensor
+
+PyObject* set_gemm_scratch(PyObject*, PyObject* fn) {
+  Py_INCREF(fn);
+  Py_XDECREF(g_gemm_scratch);
+  g_gemm_scratch = fn;
+  Py_RETURN_NONE;
+}
+
+bool gemm_scratch(int dev, void* stream, int64_t bytes, Tensor* out) {
+  PyObject* r = PyObject_CallFunction(g_gemm_scratch, "iKL", dev, static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(stream)),
+                                      static_cast<long long>(bytes));
+  if (!r) return false;
+  *out = THPVariable_Unpack(r);
+  Py_DECREF(r);
+  return true;
+}
+
+// (A, B, num_qo_heads, sparse_info, sparse_info_indptr, num_text_tokens, bias, out, sparse_q_size, is_full)
+PyObject* gemm_q(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  const Tensor *a, *b, *info, *indptr, *bias, *out;
+  int64_t heads, text, q_size;
+  FALL_BACK_UNLESS(n == 10 && opt_tensor(args[0], &a) && a && opt_tensor(args[1], &b) && b && whole(args[2], &heads) &&
+                   opt_tensor(args[3], &info) && opt_tensor(args[4], &indptr) && whole(args[5], &text) &&
+                   opt_tensor(args[6], &bias) && opt_tensor(args[7], &out) && whole(args[8], &q_size));
+  const bool full = truth(args[9]);
+  int dev, code;
+  FALL_BACK_UNLESS(gemm_operands(*a, *b, &dev, &code));
+  const int64_t batch = a->size(0), m = a->size(1), k = a->size(2), cols = b->size(0);
+  FALL_BACK_UNLESS(heads > 0 && heads < (1 << 20) && cols % heads == 0 && text >= 0 && text < (1 << 30) && q_size > 0 &&
+                   q_size < (1 << 30));
+  FALL_BACK_UNLESS(full || gemm_symbols(info, indptr, dev, batch, m, heads, text, q_size));
+  FALL_BACK_UNLESS(!bias || (flat(*bias, a->scalar_type(), dev) && bias->numel() == cols));
+  FALL_BACK_UNLESS(!out || (flat(*out, a->scalar_type(), dev) && out->dim() == 3 && out->size(0) == batch &&
+                            out->size(1) == m && out->size(2) == cols));
+  Tensor fresh, scratch;
+  if (!out) fresh = new_tensor({batch, m, cols}, a->scalar_type(), dev);
+  const Tensor& y = out ? *out : fresh;
+  void* stream = stream_of(dev);
+  const int64_t need = full ? 0 : fo_gemm_workspace_bytes(batch, m, cols);
+  if (need && !gemm_scratch(dev, stream, need, &scratch)) return nullptr;
+  if (fo_gemm_q(a->data_ptr(), b->data_ptr(), data(bias), y.data_ptr(), code, batch, m, cols, k, q_size, heads,
+                full ? nullptr : static_cast<const uint8_t*>(data(info)),
+                full ? nullptr : static_cast<const int32_t*>(data(indptr)), text, full, need ? scratch.data_ptr() : nullptr,
+                need, stream))
+    return raise_last();
+  if (out) {
+    Py_INCREF(args[7]);
+    return args[7];
+  }
+  return THPVariable_Wrap(std::move(fresh));
+  TORCH_GUARD_END
+}
+
+// (A, B, num_qo_heads, sparse_info, sparse_info_indptr, num_text_tokens, bias, is_for_cache, sparse_q_size,
+//  fp32 output)
+PyObject* gemm_o(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  const Tensor *a, *b, *info, *indptr, *bias;
+  int64_t heads, text, q_size;
+  FALL_BACK_UNLESS(n == 10 && opt_tensor(args[0], &a) && a && opt_tensor(args[1], &b) && b && whole(args[2], &heads) &&
+                   opt_tensor(args[3], &info) && opt_tensor(args[4], &indptr) && whole(args[5], &text) &&
+                   opt_tensor(args[6], &bias) && whole(args[8], &q_size));
+  const bool cache = truth(args[7]), f32 = truth(args[9]);
+  int dev, code;
+  FALL_BACK_UNLESS(gemm_operands(*a, *b, &dev, &code));
+  const int64_t batch = a->size(0), m = a->size(1), k = a->size(2), cols = b->size(0);
+  FALL_BACK_UNLESS(heads > 0 && heads < (1 << 20) && text >= 0 && text < (1 << 30) && q_size > 0 && q_size < (1 << 30) &&
+                   cols % heads == 0 && gemm_symbols(info, indptr, dev, batch, m, heads, text, q_size));
+  int kind = FO_BIAS_NONE, bias_code = code;
+  if (bias && cache) {
+    FALL_BACK_UNLESS(flat(*bias, a->scalar_type(), dev) && bias->numel() == cols);
+    kind = FO_BIAS_VECTOR;
+  } else if (bias) {
+    FALL_BACK_UNLESS(on(*bias, dev) && bias->is_contiguous() && bias->numel() == batch * m * cols &&
+                     (bias->scalar_type() == a->scalar_type() || bias->scalar_type() == at::kFloat));
+    kind = FO_BIAS_MATRIX;
+    if (bias->scalar_type() == at::kFloat) bias_code = FO_F32;
+  }
+  Tensor y = new_tensor({batch, m, cols}, f32 ? at::kFloat : a->scalar_type(), dev), scratch;
+  void* stream = stream_of(dev);
+  if (!gemm_scratch(dev, stream, 256, &scratch)) return nullptr;
+  if (fo_gemm_o(a->data_ptr(), b->data_ptr(), data(bias), y.data_ptr(), code, kind, bias_code, f32 ? FO_F32 : code, batch,
+                m, cols, k, q_size, heads, static_cast<const uint8_t*>(data(info)),
+                static_cast<const int32_t*>(data(indptr)), text, cache, scratch.data_ptr(), 256, stream))
+    return raise_last();
+  return THPVariable_Wrap(std::move(y));
+  TORCH_GUARD_END
+}
+
+// ---- attention -----------------------------------------------------------------------------------
+// What plan() derives from a batch: sizes, and one int32 tensor on the device that holds every table
+// (see fo_plan_tables).
+struct Plan {
+  PyObject_HEAD
+  Tensor tables;
+  const int32_t *qo_indptr, *kv_indptr;  // the tables' own, or the caller's (graph mode)
+  Tensor qo_keep, kv_keep;
+  int dev, batch, num_qo, num_kv, symbol_heads, packed;
+  fo_batch_sizes z;
+};
+
+PyTypeObject* g_plan_type = nullptr;
+
+void plan_dealloc(PyObject* self) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  p->tables.~Tensor();
+  p->qo_keep.~Tensor();
+  p->kv_keep.~Tensor();
+  PyTypeObject* t = Py_TYPE(self);
+  t->tp_free(self);
+  Py_DECREF(t);
+}
+
+// (qo_indptr, kv_indptr: int32 on the host; num_qo_heads, num_kv_heads, packed, device index,
+//  qo_indptr, kv_indptr of the device or None) -> (Plan, tables, sizes)
+PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  const Tensor *qo, *kv, *qo_dev, *kv_dev;
+  int64_t hq, hkv, dev;
+  if (!(n == 8 && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
+        whole(args[3], &hkv) && whole(args[5], &dev) && opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
+        qo->scalar_type() == at::kInt && kv->scalar_type() == at::kInt && qo->is_contiguous() && kv->is_contiguous() &&
+        qo->is_cpu() && kv->is_cpu() && qo->numel() == kv->numel() && qo->numel() >= 1)) {
+    PyErr_SetString(PyExc_RuntimeError, "plan: bad argument");
+    return nullptr;
+  }
+  const int batch = static_cast<int>(qo->numel()) - 1;
+  const bool packed = truth(args[4]);
+  fo_batch_sizes z;
+  if (fo_plan_batch(qo->data_ptr<int32_t>(), kv->data_ptr<int32_t>(), batch, hq, hkv, packed, &z)) return raise_last();
+  PyObject* self = g_plan_type->tp_alloc(g_plan_type, 0);
+  if (!self) return nullptr;
+  Plan* p = reinterpret_cast<Plan*>(self);
+  new (&p->tables) Tensor();
+  new (&p->qo_keep) Tensor();
+  new (&p->kv_keep) Tensor();
+  p->dev = dev;
+  p->batch = batch;
+  p->num_qo = hq;
+  p->num_kv = hkv;
+  p->packed = packed;
+  p->symbol_heads = packed ? hkv : hq;
+  p->z = z;
+  int rc = 0;
+  try {
+    p->tables = new_tensor({z.table_ints}, at::kInt, dev);
+    rc = fo_plan_tables(qo->data_ptr<int32_t>(), kv->data_ptr<int32_t>(), batch, hq, hkv, packed,
+                        p->tables.data_ptr<int32_t>(), stream_of(dev));
+  } catch (...) {
+    Py_DECREF(self);
+    throw;
+  }
+  if (rc) {
+    Py_DECREF(self);
+    return raise_last();
+  }
+  int32_t* t = p->tables.data_ptr<int32_t>();
+  p->qo_indptr = t + z.qo_indptr;
+  p->kv_indptr = t + z.kv_indptr;
+  if (qo_dev && kv_dev) {  // (graph mode: a replay reads the caller's buffers)
+    p->qo_keep = *qo_dev;
+    p->kv_keep = *kv_dev;
+    p->qo_indptr = qo_dev->data_ptr<int32_t>();
+    p->kv_indptr = kv_dev->data_ptr<int32_t>();
+  }
+  const int64_t v[] = {z.n_q_blocks, z.n_kv_blocks, z.max_rows,   z.max_nnz,       z.total_q,     z.total_kv,
+                       z.min_info,   z.min_kv_info, z.max_kv_len, z.qo_indptr,     z.kv_indptr,   z.blk_req,
+                       z.blk_qb,     z.q_blk_base,  z.kv_blk_base, z.info_indptr,  z.kv_info_indptr};
+  PyObject* sizes = PyTuple_New(17);
+  for (int i = 0; i < 17; ++i) PyTuple_SET_ITEM(sizes, i, PyLong_FromLongLong(v[i]));
+  return Py_BuildValue("(NNN)", self, THPVariable_Wrap(p->tables), sizes);
+  TORCH_GUARD_END
+}
+
+// The host planner and the copy of its arrays into the integer workspace: (float workspace, integer
+// workspace, pinned mirror, offset of the mirror's free part, qo_indptr, kv_indptr (host), rows, heads,
+// kv heads, graph mode, element size, plan vector) -> the mirror's new offset.
+// Plans are laid out one behind the other in the pinned mirror: the copy that an earlier plan queued may
+// still be reading its part, and waiting for it would mean waiting for everything queued before it.
+// Only when the mirror is full the device is waited for.
+PyObject* host_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  const Tensor *fws, *iws, *pin, *qo, *kv, *info;
+  int64_t off, rows, hq, hkv, elem;
+  if (!(n == 12 && opt_tensor(args[0], &fws) && fws && opt_tensor(args[1], &iws) && iws && opt_tensor(args[2], &pin) &&
+        pin && whole(args[3], &off) && opt_tensor(args[4], &qo) && qo && opt_tensor(args[5], &kv) && kv &&
+        whole(args[6], &rows) && whole(args[7], &hq) && whole(args[8], &hkv) && whole(args[10], &elem) &&
+        opt_tensor(args[11], &info) && info && info->scalar_type() == at::kLong && info->numel() == 15)) {
+    PyErr_SetString(PyExc_RuntimeError, "plan: bad argument");
+    return nullptr;
+  }
+  const bool graph = truth(args[9]);
+  const int batch = static_cast<int>(qo->numel()) - 1;
+  const size_t bytes = iws->numel() * iws->element_size(), pin_bytes = pin->numel() * pin->element_size();
+  // (the planner writes the used prefix only: the rest of the scratch is never touched)
+  static thread_local std::unique_ptr<char[]> scratch;
+  static thread_local size_t scratch_bytes = 0;
+  if (scratch_bytes < bytes) {
+    scratch.reset(new char[bytes]);
+    scratch_bytes = bytes;
+  }
+  int64_t* v = info->data_ptr<int64_t>();
+  if (fo_prefill_plan(fws->data_ptr(), fws->numel() * fws->element_size(), nullptr, scratch.get(), bytes,
+                      qo->data_ptr<int32_t>(), kv->data_ptr<int32_t>(), rows, batch, hq, hkv, 128, 128, 1, graph, elem, 0,
+                      v, nullptr))
+    return raise_last();
+  // end of the last array: block_valid_mask, else the row count (graph mode), else the chunk size
+  const size_t used = v[14] ? v[12] + v[0] : (v[13] ? v[2] : v[9]) + 4;
+  if (used > pin_bytes) {
+    PyErr_SetString(PyExc_RuntimeError, "the pinned mirror is smaller than the integer workspace");
+    return nullptr;
+  }
+  if (off + used > pin_bytes) {
+    if (hipDeviceSynchronize() != hipSuccess) {
+      PyErr_SetString(PyExc_RuntimeError, "hipDeviceSynchronize failed");
+      return nullptr;
+    }
+    off = 0;
+  }
+  char* host = static_cast<char*>(pin->data_ptr()) + off;
+  std::memcpy(host, scratch.get(), used);
+  if (hipMemcpyAsync(iws->data_ptr(), host, used, hipMemcpyHostToDevice,
+                     static_cast<hipStream_t>(stream_of(iws->get_device()))) != hipSuccess) {
+    PyErr_SetString(PyExc_RuntimeError, "the copy into the integer workspace failed");
+    return nullptr;
+  }
+  return PyLong_FromLongLong((off + used + 255) / 256 * 256);
+  TORCH_GUARD_END
+}
+
+// attention of an ordinary call: (plan, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr,
+// sparse_kv_info_indptr, is_full, out, lse, return_lse, sm_scale, logits_soft_cap, HND, work-list tensors,
+// float workspace or None) -> out or (out, lse)
+PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  FALL_BACK_UNLESS(n == 17 && Py_TYPE(args[0]) == g_plan_type);
+  Plan* p = reinterpret_cast<Plan*>(args[0]);
+  const int dev = p->dev;
+  const Tensor *q, *k, *v, *sym[4], *out, *lse, *ws;
+  double sm_scale, cap;
+  FALL_BACK_UNLESS(dev == c10::hip::current_device() && opt_tensor(args[1], &q) && q && opt_tensor(args[2], &k) && k &&
+                   opt_tensor(args[3], &v) && v && opt_tensor(args[4], &sym[0]) && opt_tensor(args[5], &sym[1]) &&
+                   opt_tensor(args[6], &sym[2]) && opt_tensor(args[7], &sym[3]) && opt_tensor(args[9], &out) &&
+                   opt_tensor(args[10], &lse) && real(args[13], &cap) && opt_tensor(args[16], &ws));
+  const bool full = truth(args[8]), want_lse = truth(args[11]), hnd = truth(args[14]);
+  const int code = act_code(q->scalar_type());
+  FALL_BACK_UNLESS(code >= 0 && on(*q, dev) && on(*k, dev) && on(*v, dev) && k->scalar_type() == q->scalar_type() &&
+                   v->scalar_type() == q->scalar_type() && q->dim() == 3 && k->dim() == 3 && v->dim() == 3);
+  const int kn = hnd ? 1 : 0, kh = 1 - kn;
+  FALL_BACK_UNLESS(q->size(1) == p->num_qo && q->size(2) == 128 && k->size(2) == 128 && v->size(2) == 128 &&
+                   k->size(kh) == p->num_kv && v->size(kh) == p->num_kv && q->size(0) >= p->z.total_q &&
+                   k->size(kn) >= p->z.total_kv && v->size(kn) >= p->z.total_kv && q->stride(2) == 1 &&
+                   k->stride(2) == 1 && v->stride(2) == 1);
+  if (args[12] == Py_None) {
+    sm_scale = 1.0 / std::sqrt(128.0);
+  } else {
+    FALL_BACK_UNLESS(real(args[12], &sm_scale));
+  }
+  if (!full) {
+    FALL_BACK_UNLESS(sym[0] && sym[1] && sym[2] && sym[3] && flat(*sym[0], at::kByte, dev) &&
+                     flat(*sym[1], at::kByte, dev) && flat(*sym[2], at::kInt, dev) && flat(*sym[3], at::kInt, dev) &&
+                     sym[0]->numel() >= p->z.min_info && sym[1]->numel() >= p->z.min_kv_info &&
+                     sym[2]->numel() == p->batch + 1 && sym[3]->numel() == p->batch + 1);
+  }
+  FALL_BACK_UNLESS(!out || (on(*out, dev) && out->scalar_type() == q->scalar_type() && out->sizes() == q->sizes() &&
+                            out->stride(2) == 1));
+  FALL_BACK_UNLESS(!want_lse || !lse || (flat(*lse, at::kFloat, dev) && lse->dim() == 2 && lse->size(0) == q->size(0) &&
+                                         lse->size(1) == q->size(1)));
+  // work-list buffers, in the order of fo_decode_sparse's outputs
+  FALL_BACK_UNLESS(PyTuple_Check(args[15]) && PyTuple_GET_SIZE(args[15]) == 10);
+  int32_t* wl[10];
+  for (int i = 0; i < 10; ++i) {
+    PyObject* o = PyTuple_GET_ITEM(args[15], i);
+    FALL_BACK_UNLESS(THPVariable_Check(o));
+    wl[i] = static_cast<int32_t*>(THPVariable_Unpack(o).data_ptr());
+  }
+  int32_t* shares = ws ? wl[9] : nullptr;
+
+  Tensor fresh, fresh_lse;
+  if (!out) fresh = at::zeros(q->sizes(), q->options());
+  const Tensor& o = out ? *out : fresh;
+  if (want_lse && !lse) fresh_lse = new_tensor({q->size(0), q->size(1)}, at::kFloat, dev);
+  float* lse_ptr = !want_lse ? nullptr : lse ? lse->data_ptr<float>() : fresh_lse.data_ptr<float>();
+  void* stream = stream_of(dev);
+  const int32_t* t = p->tables.data_ptr<int32_t>();
+  auto bytes = [&](int i) { return full ? nullptr : static_cast<const uint8_t*>(sym[i]->data_ptr()); };
+  auto ints = [&](int i) { return full ? nullptr : static_cast<const int32_t*>(sym[i]->data_ptr()); };
+  if (fo_decode_sparse(bytes(0), bytes(1), ints(2), ints(3), t + p->z.blk_req, t + p->z.blk_qb, p->kv_indptr,
+                       p->z.n_q_blocks, p->symbol_heads, 128, full, wl[0], wl[1], wl[2], wl[3], wl[4], wl[5], wl[6],
+                       wl[7], wl[8], shares, stream))
+    return raise_last();
+  if (fo_sparse_fa_run(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), lse_ptr, code, nullptr, nullptr, nullptr,
+                       nullptr, q->stride(0), q->stride(1), k->stride(kn), k->stride(kh), v->stride(kn), v->stride(kh),
+                       o.stride(0), o.stride(1), p->qo_indptr, p->kv_indptr, t + p->z.q_blk_base, t + p->z.kv_blk_base,
+                       p->z.n_q_blocks, p->z.n_kv_blocks, wl[0], wl[1], wl[2], wl[3], wl[4], wl[6], wl[7], p->z.max_rows,
+                       p->num_qo, p->num_kv, p->packed, 128, 128, 128, static_cast<float>(sm_scale),
+                       static_cast<float>(cap), shares, ws ? ws->data_ptr() : nullptr,
+                       ws ? ws->numel() * ws->element_size() : 0, stream))
+    return raise_last();
+  PyObject* ret = args[9];
+  if (out) {
+    Py_INCREF(ret);
+  } else {
+    ret = THPVariable_Wrap(std::move(fresh));
+  }
+  if (!want_lse || !ret) return ret;
+  PyObject* l = args[10];
+  if (lse) {
+    Py_INCREF(l);
+  } else {
+    l = THPVariable_Wrap(std::move(fresh_lse));
+  }
+  return Py_BuildValue("(NN)", ret, l);
+  TORCH_GUARD_END
+}
+
+// ---- bit packing ---------------------------------------------------------------------------------
+bool bool_bytes(const Tensor* x, int* dev) {
+  if (!x || !x->is_cuda() || !x->is_contiguous()) return false;
+  *dev = x->get_device();
+  const auto t = x->scalar_type();
+  return *dev == c10::hip::current_device() && (t == at::kBool || t == at::kByte || t == at::kChar);
+}
+
+// (x, bit order code) -> y
+PyObject* packbits(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  const Tensor* x;
+  int64_t code;
+  int dev;
+  FALL_BACK_UNLESS(n == 2 && opt_tensor(args[0], &x) && bool_bytes(x, &dev) && whole(args[1], &code));
+  Tensor y = new_tensor({(x->numel() + 7) / 8}, at::kByte, dev);
+  if (fo_packbits(static_cast<const uint8_t*>(x->data_ptr()), x->numel(), code, static_cast<uint8_t*>(y.data_ptr()),
+                  stream_of(dev)))
+    return raise_last();
+  return THPVariable_Wrap(std::move(y));
+  TORCH_GUARD_END
+}
+
+// Words of pinned memory that kernels leave a length in.  A call takes one and puts it back; there are
+// as many as calls have ever waited at the same time (guarded by the interpreter's lock).
+std::vector<uint64_t*> g_words;
+uint32_t g_ticket = 0;
+
+// (x, indptr, bit order code) -> (y, indptr of y)
+PyObject* segment_packbits(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  const Tensor *x, *ip;
+  int64_t code;
+  int dev;
+  FALL_BACK_UNLESS(n == 3 && opt_tensor(args[0], &x) && bool_bytes(x, &dev) && opt_tensor(args[1], &ip) && ip &&
+                   on(*ip, dev) && ip->dim() == 1 && ip->is_contiguous() && ip->numel() >= 2 && ip->numel() <= 1025 &&
+                   (ip->scalar_type() == at::kInt || ip->scalar_type() == at::kLong) && whole(args[2], &code));
+  hipStream_t stream = static_cast<hipStream_t>(stream_of(dev));
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  FALL_BACK_UNLESS(hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone);
+  const int64_t segments = ip->numel() - 1, capacity = (x->numel() + 7 * segments) / 8;
+  FALL_BACK_UNLESS(capacity < (int64_t(1) << 31));
+  if (g_words.empty()) {
+    void* w = nullptr;
+    if (hipHostMalloc(&w, 64, hipHostMallocCoherent) != hipSuccess) {
+      PyErr_SetString(PyExc_RuntimeError, "hipHostMalloc failed");
+      return nullptr;
+    }
+    g_words.push_back(static_cast<uint64_t*>(w));
+  }
+  Tensor y = new_tensor({capacity}, at::kByte, dev), out_ip = new_tensor({segments + 1}, at::kInt, dev);
+  uint64_t* word = g_words.back();
+  g_words.pop_back();
+  const uint32_t ticket = ++g_ticket;
+  *static_cast<volatile uint64_t*>(word) = static_cast<uint64_t>(~ticket) << 32;
+  const int rc = fo_segment_packbits_scan(static_cast<const uint8_t*>(x->data_ptr()), x->numel(), ip->data_ptr(),
+                                          ip->scalar_type() == at::kLong, segments, code,
+                                          static_cast<uint8_t*>(y.data_ptr()), capacity, out_ip.data_ptr<int32_t>(), word,
+                                          ticket, stream);
+  uint64_t got = 0;
+  bool arrived = false;
+  hipError_t err = hipSuccess;
+  if (!rc) {
+    // The word arrives a few microseconds after the kernel's start: looked at for about as long, then the
+    // stream is waited for (the kernel may be behind other work).
+    Py_BEGIN_ALLOW_THREADS
+    for (int spin = 0; spin < 20000 && !arrived; ++spin) {
+      got = *static_cast<volatile uint64_t*>(word);
+      arrived = got >> 32 == ticket;
+    }
+    if (!arrived) {
+      err = hipStreamSynchronize(stream);
+      got = *static_cast<volatile uint64_t*>(word);
+      arrived = got >> 32 == ticket;
+    }
+    Py_END_ALLOW_THREADS
+  }
+  g_words.push_back(word);
+  if (rc) return raise_last();
+  if (err != hipSuccess || !arrived) {
+    PyErr_SetString(PyExc_RuntimeError, hipGetErrorString(err));
+    return nullptr;
+  }
+  const int32_t total = static_cast<int32_t>(static_cast<uint32_t>(got));
+  FALL_BACK_UNLESS(total >= 0);
+  if (total != capacity) y = y.narrow(0, 0, total);
+  return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(out_ip)));
+  TORCH_GUARD_END
+}
+
+#define FASTCALL(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL
+PyMethodDef g_methods[] = {
+    {"gemm_q", FASTCALL(gemm_q), nullptr},
+    {"gemm_o", FASTCALL(gemm_o), nullptr},
+    {"plan", FASTCALL(plan), nullptr},
+    {"host_plan", FASTCALL(host_plan), nullptr},
+    {"attention", FASTCALL(attention), nullptr},
+    {"packbits", FASTCALL(packbits), nullptr},
+    {"segment_packbits", FASTCALL(segment_packbits), nullptr},
+    {"set_gemm_scratch", set_gemm_scratch, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+PyType_Slot g_plan_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(plan_dealloc)}, {0, nullptr}};
+PyType_Spec g_plan_spec = {"flashomni_amd._native.Plan", sizeof(Plan), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_DISALLOW_INSTANTIATION,
+                           g_plan_slots};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) {
+  g_plan_type = reinterpret_cast<PyTypeObject*>(PyType_FromSpec(&g_plan_spec));
+  if (!g_plan_type) return nullptr;
+  return PyModule_Create(&g_module);
+}

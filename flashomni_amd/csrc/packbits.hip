@@ -74,6 +74,88 @@ __global__ void __launch_bounds__(kThreads) segment_packbits_kernel(
   }
 }
 
+// Segments with their output offsets worked out here: x holds n bools, segment i packs
+// x[indptr[i] : indptr[i+1]] and begins at the next output byte.  Every workgroup takes the prefix sum of
+// the segments' byte counts itself (at most kMaxScanSegments, one batch of loads and a scan), so there is
+// no pass in front of this one; a lane then owns 8 output bytes.  Inside a segment that is 64 bools through
+// four 16-byte loads of any alignment and one 8-byte store, otherwise byte by byte.  Bound by launch
+// latency at the sizes of a mask (1.6 M bools of a 33 k token video layer: 2.6 us).  Workgroup 0 writes
+// the output's indptr, and the total with the caller's ticket to `total` (pinned host memory, or null):
+// the host reads the length there, and waits neither for a copy nor for the rest of the stream's work.
+// An indptr that descends, leaves x or needs more than `capacity` bytes packs nothing: total = -1.
+constexpr int kMaxScanSegments = 1024;
+template <typename I>
+__global__ void __launch_bounds__(kThreads) segment_packbits_scan_kernel(
+    const uint8_t* __restrict__ x, int64_t n, const I* __restrict__ indptr, int num_segments, int little,
+    uint8_t* __restrict__ y, int64_t capacity, int32_t* __restrict__ out_indptr, uint64_t* total, uint32_t ticket) {
+  __shared__ int64_t s_begin[kMaxScanSegments + 1];
+  __shared__ int32_t s_out[kMaxScanSegments + 1];
+  __shared__ int64_t s_wave[kThreads / 64];
+  __shared__ int s_bad;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) s_bad = 0;
+  for (int i = tid; i <= num_segments; i += kThreads) s_begin[i] = indptr[i];
+  __syncthreads();
+  int64_t carry = 0;
+  for (int base = 0; base < num_segments; base += kThreads) {
+    const int i = base + tid;
+    int64_t bytes = 0;
+    if (i < num_segments) {
+      const int64_t len = s_begin[i + 1] - s_begin[i];
+      if (len < 0 || s_begin[i] < 0 || s_begin[i + 1] > n) s_bad = 1; else bytes = (len + 7) >> 3;
+    }
+    int64_t incl = bytes;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t up = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += up;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    int64_t before = carry;
+    for (int w = 0; w < kThreads / 64; ++w) {
+      if (w < wave) before += s_wave[w];
+      carry += s_wave[w];
+    }
+    if (i < num_segments) s_out[i] = static_cast<int32_t>(before + incl - bytes);
+    __syncthreads();
+  }
+  if (tid == 0) s_out[num_segments] = static_cast<int32_t>(carry);
+  __syncthreads();
+  const bool bad = s_bad != 0 || carry > capacity;
+  if (blockIdx.x == 0) {
+    if (!bad)
+      for (int i = tid; i <= num_segments; i += kThreads) out_indptr[i] = s_out[i];
+    if (tid == 0 && total)
+      __hip_atomic_store(total, static_cast<uint64_t>(ticket) << 32 | static_cast<uint32_t>(bad ? -1 : static_cast<int32_t>(carry)),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (bad) return;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * 8;
+  for (int64_t o = (static_cast<int64_t>(blockIdx.x) * kThreads + tid) * 8; o < carry; o += stride) {
+    int lo = 0, hi = num_segments;  // last segment that begins at or before output byte o
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (s_out[mid] <= o) lo = mid; else hi = mid;
+    }
+    const uint8_t* src = x + s_begin[lo] + (o - s_out[lo]) * 8;
+    if (src + 64 <= x + s_begin[lo + 1]) {
+      uint64_t v[8], out = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) __builtin_memcpy(&v[2 * j], src + 16 * j, 16);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) out |= static_cast<uint64_t>(pack8(v[j], little)) << (8 * j);
+      *reinterpret_cast<uint64_t*>(y + o) = out;
+      continue;
+    }
+    for (int64_t b = o; b < min(o + 8, carry); ++b) {
+      while (lo + 1 < num_segments && s_out[lo + 1] <= b) ++lo;  // (empty segments share a byte offset)
+      const int64_t at = s_begin[lo] + (b - s_out[lo]) * 8;
+      y[b] = pack8(load8_guarded(x + at, s_begin[lo + 1] - at), little);
+    }
+  }
+}
+
 int grid_for(int64_t nbytes) {
   int64_t g = (nbytes + kThreads - 1) / kThreads;
   if (g < 1) g = 1;
@@ -113,6 +195,29 @@ extern "C" int fo_segment_packbits(const uint8_t* x, const int32_t* in_indptr,
   dim3 grid(num_segments == 1 ? 1024 : 64, num_segments);
   segment_packbits_kernel<<<grid, kThreads, 0, static_cast<hipStream_t>(stream)>>>(
       x, in_indptr, out_indptr, bitorder == FO_BITORDER_LITTLE, y);
+  FO_CHECK_LAUNCH();
+  return FO_OK;
+}
+
+extern "C" int fo_segment_packbits_scan(const uint8_t* x, int64_t n, const void* indptr, int indptr_int64,
+                                        int32_t num_segments, int bitorder, uint8_t* y, int64_t capacity,
+                                        int32_t* out_indptr, uint64_t* total, uint32_t ticket, void* stream) {
+  FO_REQUIRE(bitorder == FO_BITORDER_BIG || bitorder == FO_BITORDER_LITTLE,
+             "bitorder must be 'big' or 'little'");
+  FO_REQUIRE(num_segments >= 1 && num_segments <= kMaxScanSegments && n >= 0 && capacity >= 0 &&
+                 capacity < (int64_t(1) << 31),
+             "segment_packbits: bad sizes (1 to %d segments)", kMaxScanSegments);
+  FO_REQUIRE(indptr && out_indptr && (x || n == 0) && (y || capacity == 0), "segment_packbits: null pointer");
+  FO_REQUIRE((reinterpret_cast<uintptr_t>(y) & 7) == 0, "segment_packbits: y must be 8-byte aligned");
+  const int grid = grid_for((capacity + 7) / 8), little = bitorder == FO_BITORDER_LITTLE;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (indptr_int64) {
+    segment_packbits_scan_kernel<<<grid, kThreads, 0, s>>>(x, n, static_cast<const int64_t*>(indptr), num_segments, little,
+                                                           y, capacity, out_indptr, total, ticket);
+  } else {
+    segment_packbits_scan_kernel<<<grid, kThreads, 0, s>>>(x, n, static_cast<const int32_t*>(indptr), num_segments, little,
+                                                           y, capacity, out_indptr, total, ticket);
+  }
   FO_CHECK_LAUNCH();
   return FO_OK;
 }

@@ -33,7 +33,129 @@ uint32_t cta_tile_q_for(int64_t avg_packed_qo_len, uint32_t head_dim) {
   return avg_packed_qo_len > 16 ? 64 : 16;
 }
 
+// Tables of a batch (see fo_plan_tables).  An array of ~20 ints per request does not pay for a copy of its
+// own (staging, a DMA packet, a wait for the staging buffer): the indptrs travel as kernel arguments
+// and the kernel derives the rest.  Bound by launch latency.
+constexpr int kMaxArgBatch = 400;  // 2 x 401 ints fit the 4 KB that a kernel's arguments may take
+struct TableArgs {
+  int32_t batch, group, num_qo;
+  int32_t n_blk;
+  int32_t off[8];  // qo, kv, q base, kv base, info, kv info, blk_req, blk_qb
+  int32_t indptr[2][kMaxArgBatch + 1];
+};
+static_assert(sizeof(TableArgs) <= 4096, "kernel arguments");
+
+__global__ void __launch_bounds__(256) plan_tables_kernel(const TableArgs a, int32_t* __restrict__ out) {
+  __shared__ int32_t s_rows[kMaxArgBatch + 1];  // first symbol row of every request
+  const int tid = threadIdx.x;
+  if (tid < 5) {  // five running sums, a lane each; lane 0's also stays in LDS
+    int64_t sum = 0;
+    for (int r = 0; r <= a.batch; ++r) {
+      const int32_t v = static_cast<int32_t>(sum);
+      if (tid == 0) s_rows[r] = v;
+      else if (blockIdx.x == 0) out[a.off[1 + tid] + r] = v;
+      if (r < a.batch) {
+        const int64_t ql = a.indptr[0][r + 1] - a.indptr[0][r], kl = a.indptr[1][r + 1] - a.indptr[1][r];
+        const int64_t nq = (ql + 127) / 128, nk = (kl + 127) / 128;
+        sum += tid == 0 ? (ql * a.group + 127) / 128 : tid == 1 ? nq : tid == 2 ? nk : tid == 3 ? nq * a.num_qo
+                                                                                                : nq * nk * a.num_qo;
+      }
+    }
+  }
+  if (blockIdx.x == 0)
+    for (int i = tid; i <= a.batch; i += 256) {
+      out[a.off[0] + i] = a.indptr[0][i];
+      out[a.off[1] + i] = a.indptr[1][i];
+    }
+  __syncthreads();
+  for (int i = blockIdx.x * 256 + tid; i < a.n_blk; i += gridDim.x * 256) {
+    int lo = 0, hi = a.batch;  // last request that begins at or before row i
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (s_rows[mid] <= i) lo = mid; else hi = mid;
+    }
+    out[a.off[6] + i] = lo;
+    out[a.off[7] + i] = i - s_rows[lo];
+  }
+}
+
 }  // namespace
+
+extern "C" int fo_plan_batch(const int32_t* qo, const int32_t* kv, int32_t batch, int32_t num_qo, int32_t num_kv,
+                             int packed, void* sizes) {
+  FO_REQUIRE(qo && kv && sizes && batch >= 0 && num_qo > 0 && num_kv > 0 && num_qo % num_kv == 0, "plan batch: bad argument");
+  fo_batch_sizes z{};
+  const int64_t group = packed ? num_qo / num_kv : 1, heads = packed ? num_kv : num_qo;
+  FO_REQUIRE(qo[batch] * group < (int64_t(1) << 31), "Failed to plan prefill with error: too many packed q rows");
+  for (int32_t r = 0; r < batch; ++r) {
+    const int64_t ql = int64_t(qo[r + 1]) - qo[r], kl = int64_t(kv[r + 1]) - kv[r];
+    FO_REQUIRE(ql >= 0 && kl >= 0, "indptr should be non-decreasing");
+    const int64_t rows = (ql * group + 127) / 128, nk = (kl + 127) / 128;
+    z.n_q_blocks += rows;
+    z.n_kv_blocks += nk;
+    z.max_nnz += rows * nk * heads;
+    z.min_info += (rows * heads + 7) / 8;
+    z.min_kv_info += (rows * nk * heads + 7) / 8;
+    z.max_kv_len = std::max(z.max_kv_len, kl);
+  }
+  z.max_rows = z.n_q_blocks * heads;
+  FO_REQUIRE(z.max_nnz < (int64_t(1) << 31), "Failed to plan prefill with error: work list too large");
+  z.total_q = qo[batch];
+  z.total_kv = kv[batch];
+  int64_t at = 0;
+  for (int64_t* o : {&z.qo_indptr, &z.kv_indptr, &z.q_blk_base, &z.kv_blk_base, &z.info_indptr, &z.kv_info_indptr}) {
+    *o = at;
+    at += batch + 1;
+  }
+  z.blk_req = at;
+  z.blk_qb = at + std::max<int64_t>(z.n_q_blocks, 1);
+  z.table_ints = z.blk_qb + std::max<int64_t>(z.n_q_blocks, 1);
+  std::memcpy(sizes, &z, sizeof(z));
+  return FO_OK;
+}
+
+extern "C" int fo_plan_tables(const int32_t* qo, const int32_t* kv, int32_t batch, int32_t num_qo, int32_t num_kv,
+                              int packed, int32_t* tables, void* stream) {
+  FO_REQUIRE(tables, "plan tables: null pointer");
+  fo_batch_sizes z;
+  if (int rc = fo_plan_batch(qo, kv, batch, num_qo, num_kv, packed, &z)) return rc;
+  const int64_t group = packed ? num_qo / num_kv : 1;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int64_t off[8] = {z.qo_indptr, z.kv_indptr, z.q_blk_base, z.kv_blk_base, z.info_indptr, z.kv_info_indptr,
+                          z.blk_req,   z.blk_qb};
+  if (batch <= kMaxArgBatch && z.table_ints < (int64_t(1) << 31)) {
+    TableArgs a;
+    a.batch = batch;
+    a.group = static_cast<int32_t>(group);
+    a.num_qo = num_qo;
+    a.n_blk = static_cast<int32_t>(z.n_q_blocks);
+    for (int i = 0; i < 8; ++i) a.off[i] = static_cast<int32_t>(off[i]);
+    std::memcpy(a.indptr[0], qo, 4 * (batch + 1));
+    std::memcpy(a.indptr[1], kv, 4 * (batch + 1));
+    const int64_t grid = std::min<int64_t>(64, std::max<int64_t>(1, z.n_q_blocks / 1024));
+    plan_tables_kernel<<<static_cast<unsigned>(grid), 256, 0, s>>>(a, tables);
+    FO_CHECK_LAUNCH();
+    return FO_OK;
+  }
+  std::vector<int32_t> h(z.table_ints);
+  std::memcpy(&h[off[0]], qo, 4 * (batch + 1));
+  std::memcpy(&h[off[1]], kv, 4 * (batch + 1));
+  int64_t at = 0, sum[4] = {0, 0, 0, 0};
+  for (int32_t r = 0; r <= batch; ++r) {
+    for (int i = 0; i < 4; ++i) h[off[2 + i] + r] = static_cast<int32_t>(sum[i]);
+    if (r == batch) break;
+    const int64_t ql = qo[r + 1] - qo[r], nq = (ql + 127) / 128, nk = (int64_t(kv[r + 1]) - kv[r] + 127) / 128;
+    const int64_t add[4] = {nq, nk, nq * num_qo, nq * nk * num_qo};
+    for (int i = 0; i < 4; ++i) sum[i] += add[i];
+    for (int64_t b = 0; b < (ql * group + 127) / 128; ++b, ++at) {
+      h[off[6] + at] = r;
+      h[off[7] + at] = static_cast<int32_t>(b);
+    }
+  }
+  FO_HIP_CALL(hipMemcpyAsync(tables, h.data(), 4 * h.size(), hipMemcpyHostToDevice, s));
+  FO_HIP_CALL(hipStreamSynchronize(s));
+  return FO_OK;
+}
 
 extern "C" int fo_prefill_plan(void* float_ws, size_t float_ws_bytes, void* int_ws_dev,
                                void* int_ws_host, size_t int_ws_bytes,

@@ -68,6 +68,10 @@ def _gemm_workspace(device, stream, nbytes):
     return bufs[-1]
 
 
+def _gemm_scratch_at(index, stream, nbytes):
+    return _gemm_workspace(torch.device("cuda", index), stream, nbytes)
+
+
 def flashomni_gemm(
     A: torch.Tensor,
     B: torch.Tensor,
@@ -97,6 +101,11 @@ def flashomni_gemm(
     ``out=False`` the 16-bit result is not written at all.  Returns ``out``, or ``(out, q8, scale)``
     resp. ``(out, q8, scale, q8_lo)`` when ``quant_out`` is given (``out`` is None if it was not
     written)."""
+    if quant_out is None:
+        y = _lib.native().gemm_q(A, B, num_qo_heads, sparse_info, sparse_info_indptr, num_text_tokens, bias, out,
+                                 sparse_q_size, is_full)
+        if y is not None:
+            return y
     _check_gemm_operands(A, B, "flashomni_gemm")
     skip_out = out is False
     if skip_out:
@@ -183,6 +192,11 @@ def flashomni_gemm_reduction(
 
     ``out_dtype`` (extension; the reference always returns ``A.dtype``): pass ``torch.float32``
     to keep the cached partial in fp32; the second call accepts an fp32 ``bias`` matrix."""
+    if out_dtype is None or out_dtype is torch.float32:
+        y = _lib.native().gemm_o(A, B, num_qo_heads, sparse_info, sparse_info_indptr, num_text_tokens, bias,
+                                 is_for_cache, sparse_q_size, out_dtype is not None)
+        if y is not None:
+            return y
     _check_gemm_operands(A, B, "flashomni_gemm_reduction")
     if sparse_info is None or sparse_info_indptr is None:
         raise RuntimeError("flashomni_gemm_reduction: sparse_info and sparse_info_indptr are required")

@@ -69,7 +69,7 @@ def batch_sparseFA_with_kv_plan(float_workspace_buffer, int_workspace_buffer,
         # the plan goes when the workspace's memory does: another tensor at the same address later must
         # not find it
         weakref.finalize(int_workspace_buffer.untyped_storage(), _plans.pop, key, None)
-    _plans[key] = PlannedBatch(float_workspace_buffer, qo_host, kv_host, qo_host.to(dev), kv_host.to(dev),
+    _plans[key] = PlannedBatch(float_workspace_buffer, qo_host, kv_host, None, None,
                                num_qo_heads, num_kv_heads, 128, 128,
                                worklist=old.worklist if old is not None else None,
                                # grouped-query attention: the reference's symbols, one bit per (tile of

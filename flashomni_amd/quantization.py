@@ -33,6 +33,9 @@ def packbits(x: torch.Tensor, bitorder: str = "big") -> torch.Tensor:
     ['0b10110011']
     """
     code = _bitorder_code(bitorder)
+    y = _lib.native().packbits(x, code)
+    if y is not None:
+        return y
     _require_gpu_tensor(x, "x")
     xb = _as_bool_bytes(x.reshape(-1))
     y = torch.empty((xb.size(0) + 7) // 8, dtype=torch.uint8, device=x.device)
@@ -58,6 +61,9 @@ def segment_packbits(x: torch.Tensor, indptr: torch.Tensor,
     (as the reference does, flashomni/quantization.py:152).
     """
     code = _bitorder_code(bitorder)
+    r = _lib.native().segment_packbits(x, indptr, code)
+    if r is not None:
+        return r
     _require_gpu_tensor(x, "x")
     seglen = indptr[1:] - indptr[:-1]
     packed_len = (seglen + 7) // 8

@@ -51,6 +51,14 @@ int fo_num_cu(void);
 int fo_packbits(const uint8_t* x, int64_t n, int bitorder, uint8_t* y, void* stream);
 int fo_segment_packbits(const uint8_t* x, const int32_t* in_indptr, const int32_t* out_indptr,
                         int32_t num_segments, int bitorder, uint8_t* y, void* stream);
+/* The segment form with the output's offsets worked out on the device: x holds n bools, indptr
+ * [num_segments + 1] is int32 or int64, 1 <= num_segments <= 1024.  out_indptr (int32) receives the byte
+ * offsets, y (8-byte aligned, `capacity` bytes) the bits.  total (optional): a word of pinned host memory
+ * that receives ticket << 32 | total bytes as soon as the kernel has them.  An indptr that descends,
+ * leaves x or needs more than capacity bytes writes nothing but a total of -1. */
+int fo_segment_packbits_scan(const uint8_t* x, int64_t n, const void* indptr, int indptr_int64,
+                             int32_t num_segments, int bitorder, uint8_t* y, int64_t capacity,
+                             int32_t* out_indptr, uint64_t* total, uint32_t ticket, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Host planner.
@@ -69,6 +77,31 @@ int fo_prefill_plan(void* float_ws, size_t float_ws_bytes, void* int_ws_dev, voi
                     uint32_t num_qo_heads, uint32_t num_kv_heads, uint32_t head_dim_qk,
                     uint32_t head_dim_vo, uint32_t page_size, int enable_graph,
                     uint32_t sizeof_dtype_o, int num_cu, int64_t plan_info_out[15], void* stream);
+
+/* ---------------------------------------------------------------------------------------------
+ * Sizes and device tables of a ragged batch: what the decoder and the attention kernel read beside
+ * the tensors.  No counterpart in the reference (its kernels derive the same from the plan arrays).
+ * fo_plan_batch fills `sizes` from the host indptrs; packed != 0 (with num_kv_heads < num_qo_heads):
+ * symbol rows are tiles of 128 (token, q head of the group) pairs per kv head, see fo_sparse_fa_run.
+ * fo_plan_tables writes sizes.table_ints int32 to `tables` on the device: the arrays that start at
+ * the offsets (in ints) below.  Batches of up to 400 requests travel as the arguments of one launch
+ * (nothing of the caller's is read after the call); larger ones are copied and waited for.
+ * ------------------------------------------------------------------------------------------- */
+typedef struct fo_batch_sizes {
+  int64_t n_q_blocks, n_kv_blocks;  /* symbol rows / 128 (blk_req, blk_qb entries), kv blocks */
+  int64_t max_rows, max_nnz;        /* work-list bounds: every bit set */
+  int64_t total_q, total_kv;        /* tokens */
+  int64_t min_info, min_kv_info;    /* bytes of the packed symbols, every request byte-aligned */
+  int64_t max_kv_len;
+  /* offsets inside the tables: [batch + 1] each ... */
+  int64_t qo_indptr, kv_indptr, q_blk_base, kv_blk_base, info_indptr, kv_info_indptr;
+  int64_t blk_req, blk_qb;          /* ... and [n_q_blocks] each */
+  int64_t table_ints;
+} fo_batch_sizes;
+int fo_plan_batch(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, int32_t batch_size,
+                  int32_t num_qo_heads, int32_t num_kv_heads, int packed, void* sizes);
+int fo_plan_tables(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, int32_t batch_size,
+                   int32_t num_qo_heads, int32_t num_kv_heads, int packed, int32_t* tables, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Sparse-symbol decoder: packed symbols -> compacted, canonically ordered work list.
