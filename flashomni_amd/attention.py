@@ -71,6 +71,8 @@ class DecodedWorkList:
         self.sched = torch.zeros(1024, dtype=torch.int32, device=device)
         self.shares = torch.zeros(512 + 8 * (n + 1), dtype=torch.int32, device=device)
         self.scratch = torch.empty(2 * n + 8192, dtype=torch.int32, device=device)
+        self.buffers = (self.row_req, self.row_qb, self.row_head, self.kv_row_ptr, self.kv_idx, self.counts, self.order,
+                        self.sched, self.scratch, self.shares)
 
     def sizes(self) -> Tuple[int, int]:
         c = self.counts.cpu()
@@ -116,13 +118,21 @@ class PlannedBatch:
          self.min_info_bytes, self.min_kv_info_bytes, self.max_kv_len, *self._table_at) = sizes
         self.qo_indptr = self.table(0) if qo_indptr_dev is None else qo_indptr_dev
         self.kv_indptr = self.table(1) if kv_indptr_dev is None else kv_indptr_dev
-        if worklist is None or worklist.max_rows < self.max_rows or worklist.max_nnz < self.max_nnz:
-            worklist = DecodedWorkList(self.max_rows, self.max_nnz, self.symbol_heads, self.device)
-        self.worklist = worklist
+        # buffers of an earlier plan are taken over where they are large enough; made when first needed
+        # (a run that takes its rows straight from the symbols needs none)
+        self._list = worklist
+        if worklist is not None and (worklist.max_rows < self.max_rows or worklist.max_nnz < self.max_nnz):
+            self._list = None
         self.share_rows = share_rows
         self.split_ok = self._split_ws_ok()
         # [is_full, stream, streams already ordered after it] of the list the work-list buffers hold
         self.decoded = None
+
+    @property
+    def worklist(self) -> DecodedWorkList:
+        if self._list is None:
+            self._list = DecodedWorkList(self.max_rows, self.max_nnz, self.symbol_heads, self.device)
+        return self._list
 
     def table(self, i: int) -> torch.Tensor:
         """One of the device tables (order: see fo_batch_sizes): the indptrs of the q and kv tokens, of their
@@ -185,24 +195,43 @@ class PlannedBatch:
         # remembered for reuse_decoded: which stream the list was decoded on (a run on another
         # stream must be ordered after it)
         self.decoded = (bool(is_full), stream, [])
+        self.native.state = 0
         return wl
 
     def attention(self, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full,
-                  out, lse, return_lse, sm_scale, logits_soft_cap, hnd):
+                  out, lse, return_lse, sm_scale, logits_soft_cap, hnd, qo_indptr=None, kv_indptr=None):
         """Decode and attention of an ordinary call (16-bit operands, nothing to convert) in one native
         call; None where the call needs the general path."""
-        wl = self.worklist
-        r = _lib.native().attention(
-            self.native, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full, out,
-            lse, return_lse, sm_scale, logits_soft_cap, hnd,
-            (wl.row_req, wl.row_qb, wl.row_head, wl.kv_row_ptr, wl.kv_idx, wl.counts, wl.order, wl.sched, wl.scratch,
-             wl.shares), self.float_ws if self.split_ok else None)
-        if r is not None:
+        native = _lib.native()
+        ws = self.float_ws if self.split_ok else None
+        wl = self._list
+        r = False
+        while r is False:
+            r = native.attention(
+                self.native, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full,
+                out, lse, return_lse, sm_scale, logits_soft_cap, hnd, None if wl is None else wl.buffers, ws,
+                qo_indptr, kv_indptr)
+            if r is False:
+                wl = self.worklist
+        if r is not None and self.native.state == 0:
             self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
         return r
 
+    def listed(self) -> DecodedWorkList:
+        """The work list of the last run or decode.  A run that took its rows straight from the symbols
+        has kept a copy of them: decoded here, on the current stream, behind that run."""
+        if self.native.state:
+            cur = torch.cuda.current_stream(self.device)
+            if self.native.stream != cur.cuda_stream and not torch.cuda.is_current_stream_capturing():
+                cur.wait_stream(torch.cuda.ExternalStream(self.native.stream, device=self.device))
+            full = self.native.state == 2
+            info, kv_info, info_ip, kv_ip = (None,) * 4 if full else _lib.native().kept_symbols(self.native)
+            self.decode(info, kv_info, info_ip, kv_ip, full)
+        return self.worklist
+
     def reuse_decoded(self, is_full: bool) -> DecodedWorkList:
         """The work list of the last decode, ordered before the current stream's work."""
+        self.listed()
         if self.decoded is None:
             raise RuntimeError("reuse_decoded=True needs an earlier decode() or run() after plan()")
         was_full, stream, ordered = self.decoded
@@ -373,6 +402,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
             self._planned.float_ws = float_workspace_buffer
             self._planned.split_ok = self._planned._split_ws_ok()
             self._planned.decoded = None
+            self._planned.native.state = 0
 
     # ------------------------------------------------------------------------------------------
     def plan(
@@ -487,7 +517,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
                 self._float_workspace_buffer, qo_indptr_host, kv_indptr_host,
                 self._qo_indptr_buf if graph else None, self._kv_indptr_buf if graph else None, num_qo_heads,
                 num_kv_heads, sparse_block_size_for_q, sparse_block_size_for_kv, share_rows=self._share_rows,
-                worklist=self._planned.worklist if self._planned is not None else None,
+                worklist=self._planned._list if self._planned is not None else None,
                 gqa_packed=gqa_symbols != "per_q_head")
         if not graph:
             self._qo_indptr_buf, self._kv_indptr_buf = self._planned.qo_indptr, self._planned.kv_indptr
@@ -517,7 +547,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
 
     @property
     def _worklist(self):
-        return None if self._planned is None else self._planned.worklist
+        return None if self._planned is None else self._planned.listed()
 
     @property
     def _split_ok(self):

@@ -11,6 +11,7 @@
 // own checks, converts or raises, so that errors have one source and this file none.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <structmember.h>
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
@@ -210,10 +211,16 @@ PyObject* gemm_o(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // (see fo_plan_tables).
 struct Plan {
   PyObject_HEAD
-  Tensor tables;
+  Tensor tables, keep;
   const int32_t *qo_indptr, *kv_indptr;  // the tables' own, or the caller's (graph mode)
   Tensor qo_keep, kv_keep;
   int dev, batch, num_qo, num_kv, symbol_heads, packed;
+  bool from_zero;  // the first request begins at token 0
+  // What the last run left behind.  state 0: the list that the Python side decoded; 1: rows taken straight
+  // from the symbols, of which `keep` holds a copy (info at 0, kv_info at keep_at[0], the indptrs at
+  // keep_at[1], in bytes); 2: every row (is_full).  stream: where it ran.
+  int state;
+  long long stream, keep_at[2], keep_bytes[2];
   fo_batch_sizes z;
 };
 
@@ -222,6 +229,7 @@ PyTypeObject* g_plan_type = nullptr;
 void plan_dealloc(PyObject* self) {
   Plan* p = reinterpret_cast<Plan*>(self);
   p->tables.~Tensor();
+  p->keep.~Tensor();
   p->qo_keep.~Tensor();
   p->kv_keep.~Tensor();
   PyTypeObject* t = Py_TYPE(self);
@@ -250,6 +258,7 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!self) return nullptr;
   Plan* p = reinterpret_cast<Plan*>(self);
   new (&p->tables) Tensor();
+  new (&p->keep) Tensor();
   new (&p->qo_keep) Tensor();
   new (&p->kv_keep) Tensor();
   p->dev = dev;
@@ -259,6 +268,8 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   p->packed = packed;
   p->symbol_heads = packed ? hkv : hq;
   p->z = z;
+  p->from_zero = qo->data_ptr<int32_t>()[0] == 0;
+  p->state = 0;
   int rc = 0;
   try {
     p->tables = new_tensor({z.table_ints}, at::kInt, dev);
@@ -346,20 +357,40 @@ PyObject* host_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_END
 }
 
+// (Plan) -> (sparse_info, sparse_kv_info, the two indptrs) as the last run read them (state 1)
+PyObject* kept_symbols(PyObject*, PyObject* arg) {
+  TORCH_GUARD_BEGIN
+  if (Py_TYPE(arg) != g_plan_type || reinterpret_cast<Plan*>(arg)->state != 1) {
+    PyErr_SetString(PyExc_RuntimeError, "no symbols kept");
+    return nullptr;
+  }
+  Plan* p = reinterpret_cast<Plan*>(arg);
+  const int64_t n = p->batch + 1;
+  Tensor ip = p->keep.narrow(0, p->keep_at[1], 8 * n).view(at::kInt);
+  return Py_BuildValue("(NNNN)", THPVariable_Wrap(p->keep.narrow(0, 0, p->keep_bytes[0])),
+                       THPVariable_Wrap(p->keep.narrow(0, p->keep_at[0], p->keep_bytes[1])),
+                       THPVariable_Wrap(ip.narrow(0, 0, n)), THPVariable_Wrap(ip.narrow(0, n, n)));
+  TORCH_GUARD_END
+}
+
 // attention of an ordinary call: (plan, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr,
-// sparse_kv_info_indptr, is_full, out, lse, return_lse, sm_scale, logits_soft_cap, HND, work-list tensors,
-// float workspace or None) -> out or (out, lse)
+// sparse_kv_info_indptr, is_full, out, lse, return_lse, sm_scale, logits_soft_cap, HND, work-list tensors
+// or None, float workspace or None, indptrs of the q and kv tokens or None: the plan's) -> out or (out, lse);
+// False: needs the work-list tensors
 PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_BEGIN
-  FALL_BACK_UNLESS(n == 17 && Py_TYPE(args[0]) == g_plan_type);
+  FALL_BACK_UNLESS(n == 19 && Py_TYPE(args[0]) == g_plan_type);
   Plan* p = reinterpret_cast<Plan*>(args[0]);
   const int dev = p->dev;
-  const Tensor *q, *k, *v, *sym[4], *out, *lse, *ws;
+  const Tensor *q, *k, *v, *sym[4], *out, *lse, *ws, *ip[2];
   double sm_scale, cap;
   FALL_BACK_UNLESS(dev == c10::hip::current_device() && opt_tensor(args[1], &q) && q && opt_tensor(args[2], &k) && k &&
                    opt_tensor(args[3], &v) && v && opt_tensor(args[4], &sym[0]) && opt_tensor(args[5], &sym[1]) &&
                    opt_tensor(args[6], &sym[2]) && opt_tensor(args[7], &sym[3]) && opt_tensor(args[9], &out) &&
-                   opt_tensor(args[10], &lse) && real(args[13], &cap) && opt_tensor(args[16], &ws));
+                   opt_tensor(args[10], &lse) && real(args[13], &cap) && opt_tensor(args[16], &ws) &&
+                   opt_tensor(args[17], &ip[0]) && opt_tensor(args[18], &ip[1]));
+  for (const Tensor* t : ip)
+    FALL_BACK_UNLESS(!t || (flat(*t, at::kInt, dev) && t->numel() == p->batch + 1));
   const bool full = truth(args[8]), want_lse = truth(args[11]), hnd = truth(args[14]);
   const int code = act_code(q->scalar_type());
   FALL_BACK_UNLESS(code >= 0 && on(*q, dev) && on(*k, dev) && on(*v, dev) && k->scalar_type() == q->scalar_type() &&
@@ -385,36 +416,95 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   FALL_BACK_UNLESS(!want_lse || !lse || (flat(*lse, at::kFloat, dev) && lse->dim() == 2 && lse->size(0) == q->size(0) &&
                                          lse->size(1) == q->size(1)));
   // work-list buffers, in the order of fo_decode_sparse's outputs
-  FALL_BACK_UNLESS(PyTuple_Check(args[15]) && PyTuple_GET_SIZE(args[15]) == 10);
-  int32_t* wl[10];
-  for (int i = 0; i < 10; ++i) {
-    PyObject* o = PyTuple_GET_ITEM(args[15], i);
-    FALL_BACK_UNLESS(THPVariable_Check(o));
-    wl[i] = static_cast<int32_t*>(THPVariable_Unpack(o).data_ptr());
+  int32_t* wl[10] = {};
+  if (args[15] != Py_None) {
+    FALL_BACK_UNLESS(PyTuple_Check(args[15]) && PyTuple_GET_SIZE(args[15]) == 10);
+    for (int i = 0; i < 10; ++i) {
+      PyObject* o = PyTuple_GET_ITEM(args[15], i);
+      FALL_BACK_UNLESS(THPVariable_Check(o));
+      wl[i] = static_cast<int32_t*>(THPVariable_Unpack(o).data_ptr());
+    }
   }
-  int32_t* shares = ws ? wl[9] : nullptr;
 
-  Tensor fresh, fresh_lse;
-  if (!out) fresh = at::zeros(q->sizes(), q->options());
-  const Tensor& o = out ? *out : fresh;
-  if (want_lse && !lse) fresh_lse = new_tensor({q->size(0), q->size(1)}, at::kFloat, dev);
-  float* lse_ptr = !want_lse ? nullptr : lse ? lse->data_ptr<float>() : fresh_lse.data_ptr<float>();
   void* stream = stream_of(dev);
-  const int32_t* t = p->tables.data_ptr<int32_t>();
+  int32_t* t = p->tables.data_ptr<int32_t>();
   auto bytes = [&](int i) { return full ? nullptr : static_cast<const uint8_t*>(sym[i]->data_ptr()); };
   auto ints = [&](int i) { return full ? nullptr : static_cast<const int32_t*>(sym[i]->data_ptr()); };
-  if (fo_decode_sparse(bytes(0), bytes(1), ints(2), ints(3), t + p->z.blk_req, t + p->z.blk_qb, p->kv_indptr,
-                       p->z.n_q_blocks, p->symbol_heads, 128, full, wl[0], wl[1], wl[2], wl[3], wl[4], wl[5], wl[6],
-                       wl[7], wl[8], shares, stream))
-    return raise_last();
-  if (fo_sparse_fa_run(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), lse_ptr, code, nullptr, nullptr, nullptr,
-                       nullptr, q->stride(0), q->stride(1), k->stride(kn), k->stride(kh), v->stride(kn), v->stride(kh),
-                       o.stride(0), o.stride(1), p->qo_indptr, p->kv_indptr, t + p->z.q_blk_base, t + p->z.kv_blk_base,
-                       p->z.n_q_blocks, p->z.n_kv_blocks, wl[0], wl[1], wl[2], wl[3], wl[4], wl[6], wl[7], p->z.max_rows,
-                       p->num_qo, p->num_kv, p->packed, 128, 128, 128, static_cast<float>(sm_scale),
-                       static_cast<float>(cap), shares, ws ? ws->data_ptr() : nullptr,
-                       ws ? ws->numel() * ws->element_size() : 0, stream))
-    return raise_last();
+  Tensor fresh_lse;
+  if (want_lse && !lse) fresh_lse = new_tensor({q->size(0), q->size(1)}, at::kFloat, dev);
+
+  fo_attention_args a{};
+  a.q = q->data_ptr(); a.k = k->data_ptr(); a.v = v->data_ptr();
+  a.lse = !want_lse ? nullptr : lse ? lse->data_ptr<float>() : fresh_lse.data_ptr<float>();
+  a.q_stride_n = q->stride(0); a.q_stride_h = q->stride(1);
+  a.k_stride_n = k->stride(kn); a.k_stride_h = k->stride(kh);
+  a.v_stride_n = v->stride(kn); a.v_stride_h = v->stride(kh);
+  a.info = bytes(0); a.kv_info = bytes(1); a.info_indptr = ints(2); a.kv_info_indptr = ints(3);
+  a.qo_indptr = ip[0] ? ip[0]->data_ptr<int32_t>() : p->qo_indptr;
+  a.kv_indptr = ip[1] ? ip[1]->data_ptr<int32_t>() : p->kv_indptr;
+  a.blk_req = t + p->z.blk_req; a.blk_qb = t + p->z.blk_qb;
+  a.sched = t + p->z.sched;
+  a.split_ws = ws ? ws->data_ptr() : nullptr;
+  a.split_ws_bytes = ws ? ws->numel() * ws->element_size() : 0;
+  a.max_nnz = p->z.max_nnz;
+  a.dtype = code; a.n_blk = p->z.n_q_blocks; a.batch = p->batch; a.symbol_heads = p->symbol_heads;
+  a.num_heads = p->num_qo; a.num_kv_heads = p->num_kv; a.gqa_packed = p->packed; a.is_full = full;
+  a.sm_scale = static_cast<float>(sm_scale); a.logits_soft_cap = static_cast<float>(cap);
+  a.stream = stream;
+
+  Tensor fresh;
+  // the launch without a decoded list (it clears what it skips: every row of a fresh output is its own)
+  const bool own = !out && p->from_zero && q->size(0) == p->z.total_q;
+  // (symbol tensors much larger than the batch needs are not worth copying)
+  const bool small = full || (sym[0]->numel() <= p->z.min_info + 4096 && sym[1]->numel() <= p->z.min_kv_info + 4096);
+  int rc = FO_NOT_DIRECT;
+  if (small && p->z.max_rows > 0 && fo_sparse_attention_direct_serves(&a)) {
+    if (!out) fresh = own ? at::empty(q->sizes(), q->options()) : at::zeros(q->sizes(), q->options());
+    const Tensor& o = out ? *out : fresh;
+    a.o = o.data_ptr();
+    a.o_stride_n = o.stride(0);
+    a.o_stride_h = o.stride(1);
+    a.zero_skipped = own;
+    if (!full) {
+      auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+      p->keep_bytes[0] = sym[0]->numel();
+      p->keep_bytes[1] = sym[1]->numel();
+      p->keep_at[0] = up(p->keep_bytes[0]);
+      p->keep_at[1] = p->keep_at[0] + up(p->keep_bytes[1]);
+      const int64_t need = p->keep_at[1] + 8 * (p->batch + 1);
+      if (!p->keep.defined() || p->keep.numel() < need) p->keep = new_tensor({need}, at::kByte, dev);
+      uint8_t* kept = p->keep.data_ptr<uint8_t>();
+      a.keep_info = kept;
+      a.keep_kv_info = kept + p->keep_at[0];
+      a.keep_indptr = reinterpret_cast<int32_t*>(kept + p->keep_at[1]);
+      a.info_bytes = p->keep_bytes[0];
+      a.kv_info_bytes = p->keep_bytes[1];
+    }
+    rc = fo_sparse_attention_direct(&a);
+    if (rc < 0) return raise_last();
+    if (rc == FO_OK) {
+      p->state = full ? 2 : 1;
+      p->stream = reinterpret_cast<long long>(stream);
+    }
+  }
+  if (rc == FO_NOT_DIRECT) {
+    if (args[15] == Py_None) Py_RETURN_FALSE;
+    if (!out && !fresh.defined()) fresh = at::zeros(q->sizes(), q->options());
+    const Tensor& o = out ? *out : fresh;
+    int32_t* shares = ws ? wl[9] : nullptr;
+    if (fo_decode_sparse(a.info, a.kv_info, a.info_indptr, a.kv_info_indptr, a.blk_req, a.blk_qb, a.kv_indptr,
+                         p->z.n_q_blocks, p->symbol_heads, 128, full, wl[0], wl[1], wl[2], wl[3], wl[4], wl[5], wl[6],
+                         wl[7], wl[8], shares, stream))
+      return raise_last();
+    if (fo_sparse_fa_run(a.q, a.k, a.v, o.data_ptr(), a.lse, code, nullptr, nullptr, nullptr, nullptr, a.q_stride_n,
+                         a.q_stride_h, a.k_stride_n, a.k_stride_h, a.v_stride_n, a.v_stride_h, o.stride(0), o.stride(1),
+                         a.qo_indptr, a.kv_indptr, t + p->z.q_blk_base, t + p->z.kv_blk_base, p->z.n_q_blocks,
+                         p->z.n_kv_blocks, wl[0], wl[1], wl[2], wl[3], wl[4], wl[6], wl[7], p->z.max_rows, p->num_qo,
+                         p->num_kv, p->packed, 128, 128, 128, a.sm_scale, a.logits_soft_cap, shares, a.split_ws,
+                         a.split_ws_bytes, stream))
+      return raise_last();
+    p->state = 0;
+  }
   PyObject* ret = args[9];
   if (out) {
     Py_INCREF(ret);
@@ -529,6 +619,7 @@ PyMethodDef g_methods[] = {
     {"plan", FASTCALL(plan), nullptr},
     {"host_plan", FASTCALL(host_plan), nullptr},
     {"attention", FASTCALL(attention), nullptr},
+    {"kept_symbols", kept_symbols, METH_O, nullptr},
     {"packbits", FASTCALL(packbits), nullptr},
     {"segment_packbits", FASTCALL(segment_packbits), nullptr},
     {"set_gemm_scratch", set_gemm_scratch, METH_O, nullptr},
@@ -537,7 +628,12 @@ PyMethodDef g_methods[] = {
 
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
-PyType_Slot g_plan_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(plan_dealloc)}, {0, nullptr}};
+PyMemberDef g_plan_members[] = {{"state", T_INT, offsetof(Plan, state), 0, nullptr},
+                                {"stream", T_LONGLONG, offsetof(Plan, stream), READONLY, nullptr},
+                                {nullptr, 0, 0, 0, nullptr}};
+PyType_Slot g_plan_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(plan_dealloc)},
+                              {Py_tp_members, g_plan_members},
+                              {0, nullptr}};
 PyType_Spec g_plan_spec = {"flashomni_amd._native.Plan", sizeof(Plan), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_DISALLOW_INSTANTIATION,
                            g_plan_slots};
 

@@ -36,11 +36,12 @@ uint32_t cta_tile_q_for(int64_t avg_packed_qo_len, uint32_t head_dim) {
 // Tables of a batch (see fo_plan_tables).  An array of ~20 ints per request does not pay for a copy of its
 // own (staging, a DMA packet, a wait for the staging buffer): the indptrs travel as kernel arguments
 // and the kernel derives the rest.  Bound by launch latency.
+constexpr int kSchedInts = 1024;
 constexpr int kMaxArgBatch = 400;  // 2 x 401 ints fit the 4 KB that a kernel's arguments may take
 struct TableArgs {
   int32_t batch, group, num_qo;
   int32_t n_blk;
-  int32_t off[8];  // qo, kv, q base, kv base, info, kv info, blk_req, blk_qb
+  int32_t off[9];  // qo, kv, q base, kv base, info, kv info, blk_req, blk_qb, sched
   int32_t indptr[2][kMaxArgBatch + 1];
 };
 static_assert(sizeof(TableArgs) <= 4096, "kernel arguments");
@@ -67,6 +68,8 @@ __global__ void __launch_bounds__(256) plan_tables_kernel(const TableArgs a, int
       out[a.off[0] + i] = a.indptr[0][i];
       out[a.off[1] + i] = a.indptr[1][i];
     }
+  if (blockIdx.x == 0)
+    for (int i = tid; i < kSchedInts; i += 256) out[a.off[8] + i] = 0;
   __syncthreads();
   for (int i = blockIdx.x * 256 + tid; i < a.n_blk; i += gridDim.x * 256) {
     int lo = 0, hi = a.batch;  // last request that begins at or before row i
@@ -109,7 +112,8 @@ extern "C" int fo_plan_batch(const int32_t* qo, const int32_t* kv, int32_t batch
   }
   z.blk_req = at;
   z.blk_qb = at + std::max<int64_t>(z.n_q_blocks, 1);
-  z.table_ints = z.blk_qb + std::max<int64_t>(z.n_q_blocks, 1);
+  z.sched = z.blk_qb + std::max<int64_t>(z.n_q_blocks, 1);
+  z.table_ints = z.sched + kSchedInts;
   std::memcpy(sizes, &z, sizeof(z));
   return FO_OK;
 }
@@ -121,15 +125,15 @@ extern "C" int fo_plan_tables(const int32_t* qo, const int32_t* kv, int32_t batc
   if (int rc = fo_plan_batch(qo, kv, batch, num_qo, num_kv, packed, &z)) return rc;
   const int64_t group = packed ? num_qo / num_kv : 1;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t off[8] = {z.qo_indptr, z.kv_indptr, z.q_blk_base, z.kv_blk_base, z.info_indptr, z.kv_info_indptr,
-                          z.blk_req,   z.blk_qb};
+  const int64_t off[9] = {z.qo_indptr, z.kv_indptr, z.q_blk_base, z.kv_blk_base, z.info_indptr, z.kv_info_indptr,
+                          z.blk_req,   z.blk_qb,    z.sched};
   if (batch <= kMaxArgBatch && z.table_ints < (int64_t(1) << 31)) {
     TableArgs a;
     a.batch = batch;
     a.group = static_cast<int32_t>(group);
     a.num_qo = num_qo;
     a.n_blk = static_cast<int32_t>(z.n_q_blocks);
-    for (int i = 0; i < 8; ++i) a.off[i] = static_cast<int32_t>(off[i]);
+    for (int i = 0; i < 9; ++i) a.off[i] = static_cast<int32_t>(off[i]);
     std::memcpy(a.indptr[0], qo, 4 * (batch + 1));
     std::memcpy(a.indptr[1], kv, 4 * (batch + 1));
     const int64_t grid = std::min<int64_t>(64, std::max<int64_t>(1, z.n_q_blocks / 1024));

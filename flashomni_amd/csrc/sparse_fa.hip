@@ -147,6 +147,20 @@ struct FaParams {
   // cap * tanh(q.k * sm_scale / cap).  cap_log2 = cap * log2(e), and sm_scale_log2 then holds
   // 2 * log2(e) * sm_scale / cap, so that exp2 of the scaled product is exp(2x) of tanh's argument.
   float cap_log2;
+  // rows straight from the packed symbols (kDirect), see direct_schedule below
+  const uint8_t* info;
+  const uint8_t* kv_info;
+  const int32_t* info_indptr;
+  const int32_t* kv_info_indptr;
+  const int32_t* blk_req;
+  const int32_t* blk_qb;
+  int32_t n_blk, batch, symbol_heads, is_full;
+  int32_t zero_skipped;  // `o` is fresh: the rows of q blocks that are not computed are cleared
+  // copy of the symbols for a later decode of the same rows (or null): bytes, and the two indptrs
+  uint8_t* keep_info;
+  uint8_t* keep_kv_info;
+  int32_t* keep_indptr;
+  int32_t info_bytes, kv_info_bytes;
 };
 
 template <typename T>
@@ -270,6 +284,42 @@ __device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q,
   return -1;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wavefront: rows of 16 lanes by lane shifts, then the row totals
+// through scalar registers.
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  const int t0 = __builtin_amdgcn_readlane(v, 15), t1 = __builtin_amdgcn_readlane(v, 31), t2 = __builtin_amdgcn_readlane(v, 47);
+  const int row = (threadIdx.x & 63) >> 4;
+  return v + (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
+}
+
+// The bits [bit, bit + n) of a byte-aligned segment as 32-bit words: word i of the range, bits outside of it
+// cleared; `first` (the bit position of the range inside the first word) comes with the pointer.  Words
+// are read aligned: the ends may hold bytes of the neighbouring rows, never of another allocation.
+struct BitRange {
+  const uint32_t* words;
+  int first, n;
+  __device__ __forceinline__ BitRange(const uint8_t* seg, int64_t bit, int n_) : n(n_) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(seg) + (bit >> 3);
+    words = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
+    first = static_cast<int>(a & 3) * 8 + static_cast<int>(bit & 7);
+  }
+  __device__ __forceinline__ int count() const { return (first + n + 31) >> 5; }
+  __device__ __forceinline__ uint32_t trim(uint32_t v, int i) const {
+    if (i == 0) v &= 0xffffffffu << first;
+    const int left = first + n - 32 * i;
+    if (left < 32) v &= (1u << left) - 1u;
+    return v;
+  }
+};
+
+constexpr int kDirectMaxCand = 1024;  // candidates (symbol row, head): two per thread of a workgroup
+constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
+constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologue, epilogue and exchange cost about as many
+
 // T: element type of V, P and O (and of Q, K unless kFp8).  kFp8: Q and K are e4m3fn bytes with one
 // dequantisation scale per (head, 128-token block); S^T then comes from
 // v_mfma_scale_f32_32x32x64_f8f6f4 (64 d per instruction, unit block scale) and the two per-block
@@ -288,7 +338,7 @@ __device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q,
 // their phases together, there is no merge, and one's row prologue / epilogue overlaps the other's
 // main loop.  A row takes twice as long, so this is the form for long lists (many rows per CU).
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false>
+          bool kCap = false, bool kDirect = false>
 __global__ void __launch_bounds__(kGroups * kGroupThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 sparse_fa_kernel(const FaParams p) {
   static_assert(kPipe == (kGroups == 1), "one kv group runs the software-pipelined loop, two the two-phase loop");
@@ -312,6 +362,10 @@ sparse_fa_kernel(const FaParams p) {
     int row, part, parts, slot, req, qb, head, q_begin, q_rows, kv_begin, kv_len, ptr0, nb;
     float q_scale;  // fp8: dequantisation scale of the row's q block
     int k_scale0;   // fp8: position of the request's first kv block in k_scale (the kv head's row)
+    // kDirect: the row's keep bits (words, position of its first bit, kv blocks of the request); ptr0 is then the
+    // first kept block of this part among the row's kept blocks
+    const uint32_t* mask;
+    int mask_first, nkv;
   };
   // (fetched with the rest of the record: read in the row's prologue, they would wait behind every
   // tile copy in flight)
@@ -395,10 +449,12 @@ sparse_fa_kernel(const FaParams p) {
 
   // The next row is popped by kv group 1 while kv group 0 combines and stores the current one
   // (group 1 has nothing else to do then), so the queue atomics are off the critical path.
-  if (tid < 9) s_queue[tid] = p.sched[tid];
-  if (tid >= 64 && tid < 64 + 6) s_queue[9 + tid - 64] = p.sched[kSchedEven + tid - 64];
-  if (tid == 128) s_guess = 0;
-  __syncthreads();
+  if constexpr (!kDirect) {
+    if (tid < 9) s_queue[tid] = p.sched[tid];
+    if (tid >= 64 && tid < 64 + 6) s_queue[9 + tid - 64] = p.sched[kSchedEven + tid - 64];
+    if (tid == 128) s_guess = 0;
+    __syncthreads();
+  }
   // Even shares: the decoder has laid the rows out head by head and given every row a cost
   // (kRowOverhead + its kv blocks); share j is the cost range [j * share, (j + 1) * share), and a
   // row that straddles share boundaries is computed in parts by the shares it touches.  Every
@@ -408,15 +464,15 @@ sparse_fa_kernel(const FaParams p) {
   // rows only the kv block list has to be fetched.
   // (workgroup-uniform words: made scalar, so that none of them occupies a vector register for the
   // whole launch)
-  auto queue_word = [&](int i) { return __builtin_amdgcn_readfirstlane(s_queue[i]); };
-  const int ev_share = queue_word(10), ev_total = queue_word(11), ev_n = queue_word(12), ev_rows = queue_word(13);
+  auto queue_word = [&](int i) { return kDirect ? 0 : __builtin_amdgcn_readfirstlane(s_queue[i]); };
+  const int ev_share = kDirect ? 1 : queue_word(10), ev_total = queue_word(11), ev_n = queue_word(12), ev_rows = queue_word(13);
   const bool even = kGroups == 2 && queue_word(9) != 0 && p.shares != nullptr && p.split_ws != nullptr &&
                     static_cast<int>(gridDim.x) == ev_n;
   const int ev_j = (ev_n & (kXcds - 1)) == 0 ? (blockIdx.x & (kXcds - 1)) * (ev_n / kXcds) + blockIdx.x / kXcds
                                              : static_cast<int>(blockIdx.x);
   auto fill_items = [&](int batch_base) {
     const int lane = fresh_lane();
-    if (lane < kItemBatch) {
+    if (!kDirect && lane < kItemBatch) {
       RowInfo it;
       it.row = -1;
       it.ptr0 = 0;
@@ -578,13 +634,261 @@ sparse_fa_kernel(const FaParams p) {
     // loads as pending to the top of the row loop and wait there, behind the previous row's stores)
     __builtin_amdgcn_s_waitcnt(0x0f70);
   };
-  if (wv == 0) {
-    if (even) {
-      if (lane == 0) s_share[0] = 0;
-      fill_items(0);
+  // ---- kDirect: rows straight from the packed symbols (short lists) ----
+  // Every workgroup reads all flags and keep bits itself, two candidates (symbol row, head) per thread in
+  // head-major order, and works out with two or three workgroup scans which rows or parts of rows are its
+  // own.  A decode launch in front of this one costs 8-15 us and a launch gap at these sizes, most of it
+  // latency of a single workgroup; here the same trips to memory (two, for a batch of one request) replace
+  // the three that fetching the decoded schedule costs.
+  //   * No more rows than workgroups: one workgroup per row, or per part of it where workgroups are left
+  //     over and a part still has kDirectMinPart kv blocks.  (Even shares would cut short rows at share
+  //     boundaries here and give workgroups two pieces.)
+  //   * More: even shares as the decoder lays them out (a row costs kRowOverhead + its kv blocks, share j
+  //     is the cost range [j * share, (j + 1) * share)), with the table of rows in LDS.
+  __shared__ int s_wave[4][8];
+  __shared__ uint16_t s_row_cand[kDirect ? kDirectMaxCand : 1];  // even shares: candidate of every active row ...
+  __shared__ int s_row_u[kDirect ? kDirectMaxCand + 1 : 1];      // ... and the cost at which its kv blocks begin
+  __shared__ uint16_t s_zero[kDirect ? 64 : 1];                  // candidates this workgroup clears
+  __shared__ int s_dir[4];                         // first row of the share, candidates to clear
+  int dir_rows = 0, dir_share = 0, dir_total = 0;                // even shares; rows = 0: one item at most
+  const int dir_g = (gridDim.x & (kXcds - 1)) == 0 ? (blockIdx.x & (kXcds - 1)) * (gridDim.x / kXcds) + blockIdx.x / kXcds
+                                                   : static_cast<int>(blockIdx.x);
+  // everything about candidate `cand` but its part
+  auto direct_row = [&](int cand, RowInfo& it) {
+    const int h = cand / p.n_blk, t = cand - h * p.n_blk;
+    it.row = cand;
+    it.req = p.batch == 1 ? 0 : p.blk_req[t];
+    it.qb = p.batch == 1 ? t : p.blk_qb[t];
+    it.head = h;
+    set_q_range(it);
+    it.kv_begin = p.kv_indptr[it.req];
+    it.kv_len = p.kv_indptr[it.req + 1] - it.kv_begin;
+    it.nkv = (it.kv_len + kBlockKV - 1) / kBlockKV;
+    it.mask = nullptr;
+    it.mask_first = 0;
+    if (!p.is_full) {
+      const BitRange r(p.kv_info + p.kv_info_indptr[it.req],
+                       (static_cast<int64_t>(it.qb) * p.symbol_heads + h) * it.nkv, it.nkv);
+      it.mask = r.words;
+      it.mask_first = r.first;
     }
-    fetch_next(0);
+    it.q_scale = 1.f;
+    it.k_scale0 = 0;
+  };
+  auto direct_schedule = [&]() {
+    const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads;
+    bool act[2];
+    int n[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int cand = 2 * tid + u;
+      act[u] = false;
+      n[u] = 0;
+      if (cand < n_cand) {
+        const int h = cand / p.n_blk, t = cand - h * p.n_blk;
+        const int req = p.batch == 1 ? 0 : p.blk_req[t], qb = p.batch == 1 ? t : p.blk_qb[t];
+        const int nkv = (p.kv_indptr[req + 1] - p.kv_indptr[req] + kBlockKV - 1) / kBlockKV;
+        act[u] = true;
+        n[u] = nkv;
+        if (!p.is_full) {
+          const int64_t bit = static_cast<int64_t>(qb) * p.symbol_heads + h;
+          const uint8_t flags = p.info[p.info_indptr[req] + (bit >> 3)];
+          const BitRange r(p.kv_info + p.kv_info_indptr[req], bit * nkv, nkv);
+          int kept = 0;
+          const int words = r.count();
+          for (int i = 0; i < words; ++i) kept += __popc(r.trim(r.words[i], i));
+          act[u] = (flags >> (bit & 7)) & 1;
+          n[u] = act[u] ? kept : 0;
+        }
+      }
+    }
+    if (tid < 4) s_dir[tid] = tid == 0 ? 0x7fffffff : 0;
+    const int rows_mine = act[0] + act[1], n_mine = n[0] + n[1];
+    const int rows_incl = wave_scan(rows_mine), n_incl = wave_scan(n_mine);
+    int mx = max(n[0], n[1]);
+    for (int off = 32; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off, 64));
+    if (lane == 63) {
+      s_wave[0][wv] = rows_incl;
+      s_wave[1][wv] = n_incl;
+      s_wave[2][wv] = mx;
+    }
+    __syncthreads();
+    int rows = 0, blocks = 0, max_n = 0, row = rows_incl - rows_mine, before = n_incl - n_mine;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      if (w < wv) {
+        row += s_wave[0][w];
+        before += s_wave[1][w];
+      }
+      rows += s_wave[0][w];
+      blocks += s_wave[1][w];
+      max_n = max(max_n, s_wave[2][w]);
+    }
+    // q blocks that are not computed are cleared by turns
+    if (p.zero_skipped) {
+      int skipped = 2 * tid - row;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (2 * tid + u < n_cand && !act[u]) {
+          if (skipped % n_wg == dir_g) {
+            s_zero[skipped / n_wg] = static_cast<uint16_t>(2 * tid + u);
+            atomicAdd(&s_dir[1], 1);
+          }
+          ++skipped;
+        }
+    }
+    if (rows <= n_wg) {
+      const int spare = n_wg - rows;
+      const int want = max(max(spare > 0 ? (blocks + spare - 1) / spare : max_n, (max_n + kDirectMaxParts - 1) / kDirectMaxParts),
+                           kDirectMinPart);
+      int parts[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) parts[u] = act[u] ? max((n[u] + want - 1) / want, 1) : 0;
+      const int parts_mine = parts[0] + parts[1], parts_incl = wave_scan(parts_mine);
+      if (lane == 63) s_wave[3][wv] = parts_incl;
+      if (tid < kItemBatch) s_items[tid].row = -1;
+      __syncthreads();
+      int first = parts_incl - parts_mine;
+      for (int w = 0; w < wv; ++w) first += s_wave[3][w];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (first <= dir_g && dir_g < first + parts[u]) {
+          RowInfo it;
+          direct_row(2 * tid + u, it);
+          const int per = (n[u] + parts[u] - 1) / parts[u];
+          it.part = dir_g - first;
+          it.parts = parts[u];
+          it.slot = first;
+          it.ptr0 = it.part * per;
+          it.nb = max(min(n[u] - it.ptr0, per), 0);
+          // (the parts are as long as ceil allows: the last one may be empty)
+          s_items[0] = it;
+        }
+        first += parts[u];
+      }
+      __syncthreads();
+      return;
+    }
+    dir_rows = rows;
+    dir_total = kRowOverhead * rows + blocks;
+    dir_share = max(max((dir_total + n_wg - 1) / n_wg, (max_n + 2) / 3), 1);
+    const int a = dir_g * dir_share;
+    int cost = kRowOverhead * row + before;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (act[u]) {
+        s_row_cand[row] = static_cast<uint16_t>(2 * tid + u);
+        s_row_u[row] = cost + kRowOverhead;
+        cost += kRowOverhead + n[u];
+        // first row of the share: the first one that ends behind the share's lower bound
+        if (cost > a) atomicMin(&s_dir[0], row);
+        ++row;
+      }
+    if (tid == 0) s_row_u[rows] = dir_total + kRowOverhead;
+    __syncthreads();
+  };
+  // sixteen items of the share from `batch_base` on
+  auto direct_items = [&](int batch_base) {
+    const int lane = fresh_lane();
+    if (lane < kItemBatch) {
+      RowInfo it;
+      it.row = -1;
+      const int a = dir_g * dir_share, b = min(a + dir_share, dir_total), i = s_dir[0] + batch_base + lane;
+      if (a < dir_total && i >= 0 && i < dir_rows) {
+        const int u = s_row_u[i], e = s_row_u[i + 1] - kRowOverhead;  // kv blocks cost [u, e)
+        // (a row without kv blocks stands for the last unit of its own overhead)
+        if ((e > u ? u : u - 1) < b) {
+          direct_row(s_row_cand[i], it);
+          it.part = 0;
+          it.parts = 1;
+          it.slot = 0;
+          if (e > u) {
+            const int j_lo = u / dir_share, j_hi = (e - 1) / dir_share;
+            it.part = dir_g - j_lo;
+            it.parts = j_hi - j_lo + 1;
+            it.slot = j_lo;
+          }
+          it.ptr0 = max(a, u) - u;
+          it.nb = max(min(b, e) - u - it.ptr0, 0);
+        }
+      }
+      s_items[lane] = it;
+    }
+  };
+  // One wavefront: the next item and its kv block list, from the row's keep bits
+  auto direct_next = [&](int slot_idx) {
+    slot_idx = __builtin_amdgcn_readfirstlane(slot_idx);
+    const int lane = fresh_lane();
+    const int at = __builtin_amdgcn_readfirstlane(s_share[0]);  // items handed out so far
+    if (at > 0 && (at & (kItemBatch - 1)) == 0) direct_items(at);
+    const RowInfo& it = s_items[at & (kItemBatch - 1)];
+    if (lane == 0) {
+      s_next_row[slot_idx] = it;
+      s_share[0] = at + 1;
+    }
+    if (__builtin_amdgcn_readfirstlane(it.row) >= 0) {
+      const int lo = __builtin_amdgcn_readfirstlane(it.ptr0), n = __builtin_amdgcn_readfirstlane(it.nb);
+      if (p.is_full) {
+        for (int i = lane; i < n; i += 64) s_blk2[slot_idx][i] = static_cast<uint16_t>(lo + i);
+      } else {
+        BitRange r(nullptr, 0, __builtin_amdgcn_readfirstlane(it.nkv));
+        r.first = __builtin_amdgcn_readfirstlane(it.mask_first);
+        const uint64_t m = reinterpret_cast<uint64_t>(it.mask);
+        r.words = reinterpret_cast<const uint32_t*>(
+            static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m >> 32)))) << 32 |
+            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m))));
+        int seen = 0;
+        for (int w0 = 0; w0 < r.count(); w0 += 64) {
+          const int w = w0 + lane;
+          uint32_t bits = w < r.count() ? r.trim(r.words[w], w) : 0u;
+          const int incl = wave_scan(__popc(bits));
+          int at_bit = seen + incl - __popc(bits) - lo;
+          while (bits) {
+            const int b = __ffs(bits) - 1;
+            bits &= bits - 1;
+            if (at_bit >= 0 && at_bit < n) s_blk2[slot_idx][at_bit] = static_cast<uint16_t>(32 * w + b - r.first);
+            ++at_bit;
+          }
+          seen += __builtin_amdgcn_readlane(incl, 63);
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // (see fetch_next)
+  };
+  if constexpr (kDirect) {
+    // (the copy of the symbols for a later decode: requested first, so that it passes beside the scans)
+    if (p.keep_info != nullptr) {
+      const int step = gridDim.x * kThreads, at = blockIdx.x * kThreads + tid;
+      for (int i = at; i < p.kv_info_bytes; i += step) p.keep_kv_info[i] = p.kv_info[i];
+      for (int i = at; i < p.info_bytes; i += step) p.keep_info[i] = p.info[i];
+      for (int i = at; i <= p.batch; i += step) {
+        p.keep_indptr[i] = p.info_indptr[i];
+        p.keep_indptr[p.batch + 1 + i] = p.kv_info_indptr[i];
+      }
+    }
+    direct_schedule();
+    if (wv == 0) {
+      if (lane == 0) s_share[0] = 0;
+      if (dir_rows > 0) direct_items(0);
+      direct_next(0);
+    }
   }
+  if constexpr (!kDirect) {
+    if (wv == 0) {
+      if (even) {
+        if (lane == 0) s_share[0] = 0;
+        fill_items(0);
+      }
+      fetch_next(0);
+    }
+  }
+  auto next_item = [&](int slot_idx) __attribute__((always_inline)) {
+    if constexpr (kDirect) {
+      direct_next(slot_idx);
+    } else {
+      fetch_next(slot_idx);
+    }
+  };
   for (int row_it = 0;; ++row_it) {
     // s_next_row is published; everyone is done with the previous row's LDS data.  (Not
     // __syncthreads(): its fence would also wait for the row just stored to be acknowledged by
@@ -644,7 +948,7 @@ sparse_fa_kernel(const FaParams p) {
         for (int j = 0; j < 8; ++j) reinterpret_cast<u32x4*>(dst)[j] = z;
         if (p.lse && g_p == 0) p.lse[q_tok * p.num_heads + my_head] = kNegInf;
       }
-      if (wv == kFetchWave) fetch_next((row_it + 1) & 1);
+      if (wv == kFetchWave) next_item((row_it + 1) & 1);
       continue;
     }
 
@@ -1473,7 +1777,7 @@ sparse_fa_kernel(const FaParams p) {
       }
       __syncthreads();
     }
-    if (wv == kFetchWave) fetch_next((row_it + 1) & 1);
+    if (wv == kFetchWave) next_item((row_it + 1) & 1);
     float m_all = 0.f, d_all = 0.f;  // kv group 0: row maximum and row sum over both groups
     // A lane owns one q row and runs of four d: stored from here, a row would leave as 32 scattered
     // 8-byte pieces per instruction (measured: ~12 k cycles per row).  The finished row goes through
@@ -1578,7 +1882,8 @@ sparse_fa_kernel(const FaParams p) {
           auto part_base = [&](int i) {
             return p.split_ws + static_cast<int64_t>(part_area(split_slot, i)) * kSplitPartFloats;
           };
-          float m_p[kMaxSplitParts], d_p[kMaxSplitParts];
+          constexpr int kParts = kDirect ? kDirectMaxParts : kMaxSplitParts;
+          float m_p[kParts], d_p[kParts];
           const float m_own = m_all, d_own = d_all;
           m_all = kNegInf;
           for (int i = 0; i < parts; ++i) {
@@ -1666,6 +1971,31 @@ sparse_fa_kernel(const FaParams p) {
     }
   }
 
+  if constexpr (kDirect) {
+    // q blocks that are not computed, of a fresh output: zeros (left to the end: a workgroup that has no row
+    // comes here at once)
+    const int n_zero = __builtin_amdgcn_readfirstlane(s_dir[1]);
+    for (int z = 0; z < n_zero; ++z) {
+      RowInfo it;
+      direct_row(s_zero[z], it);
+      const int gq = kGqaPack ? p.gqa_pack : 0;
+      T* dst = op + static_cast<int64_t>(it.q_begin) * p.o_sn + static_cast<int64_t>(gq ? it.head * gq : it.head) * p.o_sh;
+      for (int i = tid; i < it.q_rows * 16; i += kThreads) {
+        const int r = i >> 4;
+        int64_t off;
+        if constexpr (kGqaPack) {
+          const uint32_t pr = static_cast<uint32_t>(it.qb) * kBlockQ + r;
+          const int tok = static_cast<int>(pr / static_cast<uint32_t>(gq));
+          off = tok * p.o_sn + static_cast<int64_t>(pr - tok * gq) * p.o_sh;
+        } else {
+          off = r * p.o_sn;
+        }
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        __builtin_nontemporal_store(zero, reinterpret_cast<u32x4*>(dst + off) + (i & 15));
+      }
+    }
+    return;
+  }
   // the last workgroup to leave rewinds the queues for the next launch
   if (tid == 0) {
     __threadfence();
@@ -1678,7 +2008,7 @@ sparse_fa_kernel(const FaParams p) {
 }
 
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups = 2, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false>
+          bool kCap = false, bool kDirect = false>
 int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   constexpr int kSmemBytes = Geom<kFp8, kKLo, kGroups>::kSmemBytes;
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
@@ -1687,7 +2017,7 @@ int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
-    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap>),
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes));
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
@@ -1695,8 +2025,8 @@ int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "sparse_fa: no device");
   int64_t grid = num_cu * (3 - kGroups);  // persistent workgroups: one per CU, or two of one kv group each (LDS bound)
   // (with even shares every workgroup may hold a part of a row; otherwise at most one row each)
-  if (!(p.split_ws && p.shares) && grid > max_rows) grid = max_rows;
-  sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap><<<static_cast<unsigned>(grid), kGroups * kGroupThreads, kSmemBytes, stream>>>(p);
+  if (!kDirect && !(p.split_ws && p.shares) && grid > max_rows) grid = max_rows;
+  sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect><<<static_cast<unsigned>(grid), kGroups * kGroupThreads, kSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
 }
@@ -1839,4 +2169,74 @@ extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, voi
   if (k_lo != nullptr) return launch<__bf16, true, true, true>(p, max_rows, s);
   if (q_lo != nullptr) return launch<__bf16, true, true, false>(p, max_rows, s);
   return launch<__bf16, true, false, false>(p, max_rows, s);
+}
+
+extern "C" int fo_sparse_attention_direct_serves(const void* args) {
+  const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
+  const int num_cu = fo_num_cu();
+  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  // Two candidates per thread at most, and keep bits that every workgroup can afford to read (2^20 bits =
+  // 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also sorts
+  // their rows.
+  return (a.dtype == FO_BF16 || a.dtype == FO_F16) && g_variant.load(std::memory_order_relaxed) != 1 && n_cand >= 1 &&
+         n_cand <= kDirectMaxCand && a.max_nnz <= (1 << 20) && num_cu >= 16 && num_cu <= kMaxShares && a.split_ws &&
+         a.split_ws_bytes >= fo_sparse_fa_split_workspace_bytes() && (reinterpret_cast<uintptr_t>(a.split_ws) & 15) == 0;
+}
+
+extern "C" int fo_sparse_attention_direct(const void* args) {
+  FO_REQUIRE(args, "sparse_attention: null pointer");
+  const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
+  if (!fo_sparse_attention_direct_serves(args)) return FO_NOT_DIRECT;
+  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  FO_REQUIRE(a.q && a.k && a.v && a.o && a.qo_indptr && a.kv_indptr && a.blk_req && a.blk_qb && a.sched,
+             "sparse_attention: null pointer");
+  FO_REQUIRE(a.is_full || (a.info && a.kv_info && a.info_indptr && a.kv_info_indptr), "sparse_attention: null symbols");
+  FO_REQUIRE(a.num_kv_heads > 0 && a.num_heads % a.num_kv_heads == 0, "sparse_attention: bad head counts");
+  FO_REQUIRE(a.logits_soft_cap >= 0.f && a.logits_soft_cap < __builtin_inff(),
+             "sparse_attention: logits_soft_cap must be a finite value >= 0 (0: no cap)");
+  const int64_t strides[8] = {a.q_stride_n, a.q_stride_h, a.k_stride_n, a.k_stride_h,
+                              a.v_stride_n, a.v_stride_h, a.o_stride_n, a.o_stride_h};
+  for (int i = 0; i < 8; ++i)
+    FO_REQUIRE(strides[i] % 8 == 0 && strides[i] > 0,
+               "sparse_fa: strides must be positive multiples of 16 bytes (128-bit accesses)");
+  FO_REQUIRE(a.q_stride_n < (int64_t(1) << 23) && a.k_stride_n < (int64_t(1) << 23) && a.v_stride_n < (int64_t(1) << 23),
+             "sparse_fa: q/k/v token strides must be below 2^23 elements (32-bit tile offsets)");
+  for (const void* ptr : {a.q, a.k, a.v, static_cast<const void*>(a.o)})
+    FO_REQUIRE((reinterpret_cast<uintptr_t>(ptr) & 15) == 0, "sparse_fa: q/k/v/o must be 16-byte aligned");
+  FaParams p{};
+  p.q = a.q; p.k = a.k; p.v = a.v; p.o = a.o; p.lse = a.lse;
+  p.q_sn = a.q_stride_n; p.q_sh = a.q_stride_h; p.k_sn = a.k_stride_n; p.k_sh = a.k_stride_h;
+  p.v_sn = a.v_stride_n; p.v_sh = a.v_stride_h; p.o_sn = a.o_stride_n; p.o_sh = a.o_stride_h;
+  p.qo_indptr = a.qo_indptr; p.kv_indptr = a.kv_indptr; p.sched = a.sched;
+  p.split_ws = static_cast<float*>(a.split_ws);
+  p.num_heads = a.num_heads;
+  const bool packed = a.gqa_packed && a.num_heads != a.num_kv_heads;
+  p.kv_group = packed ? 1 : a.num_heads / a.num_kv_heads;
+  p.gqa_pack = packed ? a.num_heads / a.num_kv_heads : 0;
+  p.sm_scale_log2 = a.sm_scale * 1.44269504088896340736f;
+  p.info = a.info; p.kv_info = a.kv_info; p.info_indptr = a.info_indptr; p.kv_info_indptr = a.kv_info_indptr;
+  p.blk_req = a.blk_req; p.blk_qb = a.blk_qb;
+  p.n_blk = a.n_blk; p.batch = a.batch; p.symbol_heads = a.symbol_heads; p.is_full = a.is_full;
+  p.zero_skipped = a.zero_skipped && !a.is_full;
+  if (!a.is_full && a.keep_info) {
+    FO_REQUIRE(a.keep_kv_info && a.keep_indptr, "sparse_attention: null pointer");
+    p.keep_info = a.keep_info; p.keep_kv_info = a.keep_kv_info; p.keep_indptr = a.keep_indptr;
+    p.info_bytes = a.info_bytes; p.kv_info_bytes = a.kv_info_bytes;
+  }
+  hipStream_t s = static_cast<hipStream_t>(a.stream);
+  const bool bf16 = a.dtype == FO_BF16;
+  if (a.logits_soft_cap > 0.f) {
+    p.cap_log2 = a.logits_soft_cap * 1.44269504088896340736f;
+    p.sm_scale_log2 = 2.f * 1.44269504088896340736f * a.sm_scale / a.logits_soft_cap;
+    if (packed)
+      return bf16 ? launch<__bf16, false, false, false, 2, false, true, true, true>(p, n_cand, s)
+                  : launch<_Float16, false, false, false, 2, false, true, true, true>(p, n_cand, s);
+    return bf16 ? launch<__bf16, false, false, false, 2, false, false, true, true>(p, n_cand, s)
+                : launch<_Float16, false, false, false, 2, false, false, true, true>(p, n_cand, s);
+  }
+  if (packed)
+    return bf16 ? launch<__bf16, false, false, false, 2, false, true, false, true>(p, n_cand, s)
+                : launch<_Float16, false, false, false, 2, false, true, false, true>(p, n_cand, s);
+  return bf16 ? launch<__bf16, false, false, false, 2, false, false, false, true>(p, n_cand, s)
+              : launch<_Float16, false, false, false, 2, false, false, false, true>(p, n_cand, s);
 }

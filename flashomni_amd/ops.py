@@ -71,7 +71,7 @@ def batch_sparseFA_with_kv_plan(float_workspace_buffer, int_workspace_buffer,
         weakref.finalize(int_workspace_buffer.untyped_storage(), _plans.pop, key, None)
     _plans[key] = PlannedBatch(float_workspace_buffer, qo_host, kv_host, None, None,
                                num_qo_heads, num_kv_heads, 128, 128,
-                               worklist=old.worklist if old is not None else None,
+                               worklist=old._list if old is not None else None,
                                # grouped-query attention: the reference's symbols, one bit per (tile of
                                # 128 packed rows, kv head) (prefill.cuh:1283-1290)
                                gqa_packed=True)
@@ -123,6 +123,10 @@ def batch_sparseFA_with_ragged_kv_run(float_workspace_buffer, int_workspace_buff
         pb.float_ws = float_workspace_buffer
         pb.split_ok = pb._split_ws_ok()
     pb.qo_indptr, pb.kv_indptr = qo_indptr, kv_indptr
+    if pb.attention(q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full, o,
+                    maybe_lse, maybe_lse is not None, sm_scale, logits_soft_cap, layout == 1, qo_indptr,
+                    kv_indptr) is not None:
+        return
     try:
         pb.decode(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full)
         pb.launch(q, k, v, o, maybe_lse, "NHD" if layout == 0 else "HND", sm_scale,

@@ -96,6 +96,7 @@ typedef struct fo_batch_sizes {
   /* offsets inside the tables: [batch + 1] each ... */
   int64_t qo_indptr, kv_indptr, q_blk_base, kv_blk_base, info_indptr, kv_info_indptr;
   int64_t blk_req, blk_qb;          /* ... and [n_q_blocks] each */
+  int64_t sched;                    /* 1024 zeros: see fo_sparse_attention_direct */
   int64_t table_ints;
 } fo_batch_sizes;
 int fo_plan_batch(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, int32_t batch_size,
@@ -256,6 +257,38 @@ int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float
                      int32_t* sched, int64_t max_rows, int32_t num_heads, int32_t num_kv_heads, int32_t gqa_packed,
                      int32_t head_dim, int32_t block_q, int32_t block_kv, float sm_scale, float logits_soft_cap,
                      const int32_t* shares, void* split_workspace, int64_t split_workspace_bytes, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
+ * The same attention straight from the packed symbols, without a decoded list: short lists whose rows
+ * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
+ * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
+ * candidates, more than 2^20 keep bits, no split workspace of fo_sparse_fa_split_workspace_bytes() bytes.
+ * Arguments as in fo_decode_sparse (symbols, blk_req, blk_qb, is_full; n_blk symbol rows of symbol_heads
+ * heads) and fo_sparse_fa_run.  sched: 1024 int32, zero before the first launch and left zero by every
+ * one.  zero_skipped: the rows of q blocks that are not computed are cleared in o.  keep_info,
+ * keep_kv_info, keep_indptr (optional): receive the info_bytes / kv_info_bytes of symbols and the two
+ * indptrs ([2 * (batch + 1)]) that this launch read, for a decode of the same list later.  Launches that share sched or split_ws must not overlap in time.
+ * ------------------------------------------------------------------------------------------- */
+typedef struct fo_attention_args {
+  const void *q, *k, *v;
+  void* o;
+  float* lse;
+  int64_t q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n, v_stride_h, o_stride_n, o_stride_h;
+  const uint8_t *info, *kv_info;
+  const int32_t *info_indptr, *kv_info_indptr, *qo_indptr, *kv_indptr, *blk_req, *blk_qb;
+  int32_t* sched;
+  void* split_ws;
+  int64_t split_ws_bytes;
+  uint8_t *keep_info, *keep_kv_info;
+  int32_t* keep_indptr;
+  int64_t max_nnz;
+  int32_t info_bytes, kv_info_bytes, dtype, n_blk, batch, symbol_heads, num_heads, num_kv_heads, gqa_packed, is_full, zero_skipped;
+  float sm_scale, logits_soft_cap;
+  void* stream;
+} fo_attention_args;
+enum { FO_NOT_DIRECT = 1 };
+int fo_sparse_attention_direct_serves(const void* args);  /* 1: fo_sparse_attention_direct takes the batch */
+int fo_sparse_attention_direct(const void* args);
 
 /* ---------------------------------------------------------------------------------------------
  * GEMM-Q: y[b, tile] = x[b] . w^T + bias for every (128-row, 128-column) tile whose symbol bit

@@ -1,0 +1,82 @@
+"""GPU: run() without a decode launch (rows taken straight from the packed symbols) against the oracle, at
+the edges of its range: one candidate, 1024 and one more, rows in eight parts, even shares, batches, a
+fresh output whose skipped q blocks the launch clears itself, and a list reused afterwards."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import make_ragged_masks, max_abs, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    ([1], [1], 1, 1.0),
+    ([640], [20000], 1, 1.0),                 # 5 rows of ~80 kept blocks: eight parts each
+    ([300, 1, 128, 1000, 129], [77, 513, 128, 1100, 64], 3, 0.6),
+    ([2048], [300], 64, 0.7),                 # 1024 candidates, ~720 rows: even shares
+    ([2049], [300], 64, 0.7),                 # 1088 candidates: decoded
+    ([1200, 900], [1300, 2500], 24, 0.95),    # more rows than workgroups, rows cut at share boundaries
+    ([512], [512], 2, 0.0),                   # nothing to compute
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("is_full", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_from_the_symbols(dev, case, is_full, dtype):
+    import flashomni_amd as fo
+    ql, kl, heads, pa = case
+    m = make_ragged_masks(ql, kl, heads, pa, 0.5, seed=3)
+    g = torch.Generator().manual_seed(3)
+    nq, nk = sum(ql), sum(kl)
+    q, k, v = (torch.randn(n, heads, 128, generator=g).to(dtype) for n in (nq, nk, nk))
+    t = lambda n: torch.from_numpy(m[n]).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t("qo_indptr"), t("kv_indptr"), heads, heads, 128, q_data_type=dtype)
+    sym = [t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    args = (q.to(dev), k.to(dev), v.to(dev), *sym, is_full)
+    lse = torch.full((nq, heads), 7.0, device=dev)
+    junk = torch.full((64 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
+    del junk
+    out, lse = w.run(*args, lse=lse, return_lse=True)
+    again, lse2 = w.run(*args, lse=lse.clone(), return_lse=True)
+    assert torch.equal(out, again) and torch.equal(lse, lse2)
+    exp_lse = torch.full((nq, heads), 7.0)
+    exp = oracle.sparse_attention(q, k, v, m["packed_info"], m["packed_keep"], m["info_indptr"], m["keep_indptr"],
+                                  m["qo_indptr"], m["kv_indptr"], is_full=is_full, out=torch.zeros_like(q), lse=exp_lse)
+    got = out.cpu()
+    cached = torch.zeros(nq, heads, dtype=torch.bool)
+    for r, info in enumerate(m["info"]):
+        for qb in range(0 if is_full else info.shape[0]):
+            rows = slice(int(m["qo_indptr"][r]) + qb * 128, min(int(m["qo_indptr"][r]) + qb * 128 + 128, int(m["qo_indptr"][r + 1])))
+            cached[rows] = torch.from_numpy(~info[qb])
+    assert not got[cached].any()
+    assert max_abs(got, exp) <= 2e-2 and rel_l2(got, exp) <= 1e-2
+    assert torch.allclose(lse.cpu(), exp_lse, atol=2e-3, rtol=1e-3)
+    # the list of that run, reused after the symbols were overwritten
+    for s in sym[:2]:
+        s.fill_(0xff)
+    listed = torch.zeros_like(out)
+    w.run(*args, out=listed, reuse_decoded=True)
+    assert max_abs(listed.cpu(), got) <= 8e-3
+
+
+@pytest.mark.parametrize("group", [2, 7])
+def test_fresh_output_of_packed_tiles(dev, group):
+    """Skipped tiles of grouped-query attention: the rows of a tile are spread over the group's q heads."""
+    import flashomni_amd as fo
+    hkv, ql, kl = 2, [300, 1, 640], [77, 513, 640]
+    hq = hkv * group
+    m = make_ragged_masks([n * group for n in ql], kl, hkv, 0.5, 0.5, seed=4)
+    qo = torch.from_numpy(np.concatenate([[0], np.cumsum(ql)]).astype(np.int32))
+    g = torch.Generator(device=dev).manual_seed(4)
+    q, k, v = (torch.randn(n, h, 128, generator=g, device=dev).to(torch.bfloat16) for n, h in ((941, hq), (1230, hkv), (1230, hkv)))
+    t = lambda n: torch.from_numpy(m[n]).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(512 << 20, dtype=torch.uint8, device=dev))
+    w.plan(qo, t("kv_indptr"), hq, hkv, 128, q_data_type=torch.bfloat16)
+    sym = [t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    exp = w.run(q, k, v, *sym, out=torch.zeros_like(q))
+    junk = torch.full((64 << 20,), 0x7f, dtype=torch.uint8, device=dev)
+    del junk
+    assert torch.equal(w.run(q, k, v, *sym), exp)
