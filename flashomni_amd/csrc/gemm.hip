@@ -1053,7 +1053,9 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
           // (stored with the streaming hint, cache policy 2: the output is not read again by this launch
           // and should not push operand tiles out of the L2; 0.5-1.5 % at both sizes)
           if constexpr (kOutF32) {
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, el_off * 4, row_off(i, 4), 2);
+            // (the row offset travels in the lane's: with one in a scalar register the compiler may write the
+            // first data register in the very next instruction, and the last lanes then store that value)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, el_off * 4 + row_off(i, 4), 0, 2);
           } else {
             x4 out;
 #pragma unroll

@@ -443,6 +443,30 @@ def test_gemm_o_cursors_and_fixed_stride_agree(dev, shape):
     assert rel_l2(got[0, :256].cpu(), dense) <= REL_L2
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch", [1, 2, 5])
+def test_fp32_output_rounds_to_the_16_bit_one(dev, batch, dtype):
+    """GEMM-O forms the same fp32 value whatever it stores: the fp32 result rounded is the 16-bit result,
+    without a bias, with a bias vector and with a cached partial, in launches of few and of many units.
+    (The fp32 store once read a data register that the next instruction had already overwritten: runs
+    of four rows whose every fourth column held another row's value.)"""
+    import flashomni_amd as fo
+    m, n, heads = 3000, 2048, 8
+    info, packed, indptr = _flags(batch, (m + 127) // 128, heads, 0.6, seed=5)
+    g = torch.Generator(device=dev).manual_seed(6)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    part = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 0, bias=b, is_for_cache=True)
+    for bias, cache in ((None, True), (b, True), (part, False), (part.float(), False)):
+        short = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 0, bias=bias, is_for_cache=cache)
+        for _ in range(4):
+            wide = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 0, bias=bias, is_for_cache=cache,
+                                               out_dtype=torch.float32)
+            assert torch.equal(wide.to(dtype), short)
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_random_gemm_shapes(dev, seed):
     """Seeded random shapes through GEMM-Q (flags or is_full) and the two passes of GEMM-O (the cached
