@@ -86,6 +86,8 @@ constexpr int kUnitBytes = kTile * kRowBytes;      // one 128-row operand tile: 
 constexpr int kStageBytes = 4 * kUnitBytes;        // X0, X1, W0, W1
 constexpr int kStages = 2;
 constexpr int kSmemBytes = kStages * kStageBytes;  // 128 KB
+constexpr int kUnitSmemBytes = kStages * 2 * kUnitBytes;  // workgroup per unit: 64 KB, two workgroups per CU
+constexpr int kUnitWindow = 8;  // ... token blocks per scheduling window
 constexpr int kZeroFirst = 1 << 18, kZeroSecond = 1 << 19;  // slab entry: half of the slab does not count
 constexpr int kMaxHeads = 256;
 constexpr int kMaxSteps = 2048;  // GEMM-O: k steps of one work item (K <= 65536)
@@ -1111,6 +1113,318 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Short launches: a workgroup per unit.  Quads keep a CU busy with one work item of four units for
+// its whole k range, so a launch lasts whole rounds of quads however few units are in them: nine
+// token blocks x eight heads fill 36 of 256 CUs, and one unit in ten flagged over 16 k tokens is
+// ~200 items of one or two units that each take as long as four.  Here the four wavefronts share one
+// unit (64 x 64 each: 64 accumulators, 182 registers), two workgroups fit a CU (72 KB of LDS), one's
+// prologue and epilogue run beside the other's loop, and GEMM-O walks the heads of one token block
+// instead of the union of two.  The price is twice the operand bytes per flop over the L2 -> CU path
+// (32 KB per 128 x 128 x 64 step, ~550 cycles of it beside 512 of matrix core), so long launches keep
+// the quads.  The loop is the quads': staging registers a slab ahead, two LDS slab buffers, one
+// barrier per slab, the same mix of MFMAs, operand reads, LDS writes and loads in every substep; the
+// k order is the same, and so are the results, bit for bit.
+// ---------------------------------------------------------------------------------------------
+template <typename T, bool kReduce, bool kHalf, bool kPartial>
+__global__ void __launch_bounds__(kThreads, 2) gemm_unit_kernel(const GemmParams p) {
+  using TT = Types<T>;
+  using x8 = typename TT::x8;
+  using x4 = typename TT::x4;
+  constexpr int NT = 2, MT = 2;  // wavefront tile: 64 columns (W rows) x 64 token rows (X rows)
+  constexpr int P = 8, PS = P / 4;  // 8-row pieces per wavefront and slab (0..3 X, 4..7 W), per substep
+  constexpr int kStage = 2 * kUnitBytes;  // X, W
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ int32_t s_heads[kReduce ? kMaxHeads : 1];
+  __shared__ int32_t s_nsel;
+  __shared__ int32_t s_step[kReduce ? kMaxSteps + 4 : 1];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, g = lane >> 5;
+  const int wr = wv >> 1, wc = wv & 1;  // half of the unit's rows, of its columns
+
+  // ---- which unit: XCD x owns the x-th eighth of the units, ordered batch, window of eight token
+  // blocks, column, row: the ~64 units an XCD works on at a time share 8 + 8 operand tiles in its L2 ----
+  const int units_per_batch = p.n_row_tiles * p.n_col_tiles;
+  const int64_t total = static_cast<int64_t>(units_per_batch) * p.batch;
+  const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
+  const int u_lo = static_cast<int>(total * xcd / kXcds);
+  const int u = u_lo + slot;
+  if (u >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
+  const int bz = u / units_per_batch;
+  const int rem = u - bz * units_per_batch;
+  const int win = rem / (kUnitWindow * p.n_col_tiles);
+  const int in_win = rem - win * kUnitWindow * p.n_col_tiles;
+  const int win_rows = min(kUnitWindow, p.n_row_tiles - win * kUnitWindow);
+  const int col = in_win / win_rows;
+  const int row = win * kUnitWindow + in_win - col * win_rows;
+  const int m0 = row * kTile, n0 = col * kTile;
+  const uint32_t flag_row =
+      static_cast<uint32_t>(p.num_text_tokens + m0) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
+  if constexpr (!kReduce) {
+    if (p.flag == 0) {
+      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+      if (!flag_bit(info, flag_row + static_cast<uint32_t>(n0) / p.head_dim)) return;
+    }
+  }
+
+  // ---- k steps (entries as in gemm_kernel) ----
+  int n_iter;
+  if constexpr (kReduce) {
+    if (wv == 0) {
+      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+      const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
+      const int n_slices = p.k / p.head_dim;
+      int count = 0;
+      for (int h0 = 0; h0 < n_slices; h0 += 64) {
+        const int h = h0 + lane;
+        const bool sel = h < n_slices && flag_bit(info, flag_row + h) == pick;
+        const unsigned long long mask = __ballot(sel);
+        if (sel) s_heads[count + __popcll(mask & ((1ull << lane) - 1ull))] = h;
+        count += __popcll(mask);
+      }
+      if (lane == 0) s_nsel = count;
+    }
+    __syncthreads();
+    const int iph = (p.head_dim + kBK - 1) / kBK;
+    n_iter = __builtin_amdgcn_readfirstlane(s_nsel) * iph;
+    for (int i = tid; i < n_iter + 4 && n_iter > 0; i += kThreads) {
+      const int ii = i < n_iter ? i : n_iter - 1;
+      const int k0 = s_heads[ii / iph] * p.head_dim + (ii % iph) * kBK;
+      int e = k0;
+      if ((ii % iph) * kBK + kBK > p.head_dim) e = k0 >= 32 ? (k0 - 32) | kZeroFirst : k0 | kZeroSecond;
+      s_step[i] = e;
+    }
+    __syncthreads();
+  } else {
+    n_iter = (p.k + kBK - 1) / kBK;
+  }
+  auto step_entry_raw = [&](int it) -> int {
+    if constexpr (kReduce) {
+      return s_step[it];
+    } else {
+      const int i = it < n_iter ? it : n_iter - 1;
+      return (i + 1) * kBK <= p.k ? i * kBK : (p.k - kBK) | kZeroFirst;
+    }
+  };
+  auto step_entry = [&](int it) -> int { return __builtin_amdgcn_readfirstlane(step_entry_raw(it)); };
+
+  // ---- operand tiles (rows past M read as zeros through the descriptor's range check) ----
+  const T* __restrict__ xg = static_cast<const T*>(p.x);
+  const T* __restrict__ wg = static_cast<const T*>(p.w);
+  const int rows_here = min(p.m - m0, kTile);
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(xg + (static_cast<int64_t>(bz) * p.m + m0) * p.k), 0, rows_here * p.k * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(wg + static_cast<int64_t>(n0) * p.k), 0, kTile * p.k * 2, 0x00020000);
+  const int ld_chunk = lane & 7;
+  int wr_off[2];
+#pragma unroll
+  for (int par = 0; par < 2; ++par)
+    wr_off[par] = (lane >> 3) * kRowBytes + ((ld_chunk ^ ((4 * par + (lane >> 4)) & 7)) << 4);
+  const unsigned mask_first = ld_chunk < 4 ? 0xFFFFFFFFu : 0u;
+  const int rd_x = (g ^ ((l32 >> 1) & 7)) << 4;
+  int ld_off[4];
+#pragma unroll
+  for (int jj = 0; jj < 4; ++jj) ld_off[jj] = (32 * wv + 8 * jj + (lane >> 3)) * p.k * 2 + ld_chunk * 16;
+  u32x4 stg[P];
+  auto gload = [&](int j, int entry) {
+    stg[j] = __builtin_amdgcn_raw_buffer_load_b128(j < 4 ? rsrc_x : rsrc_w, ld_off[j & 3], (entry & 0xFFFF) * 2, 0);
+  };
+  auto keep_of = [&](int entry) -> unsigned {
+    return (entry & kZeroFirst) ? ~mask_first : ((entry & kZeroSecond) ? mask_first : 0xFFFFFFFFu);
+  };
+  auto lwrite = [&](int j, int stage, unsigned keep) {
+    uint8_t* dst = smem + stage * kStage + (j >> 2) * kUnitBytes + (32 * wv + 8 * (j & 3)) * kRowBytes + wr_off[j & 1];
+    u32x4 v = stg[j];
+    if constexpr (kHalf) {
+      if (j < 4) v &= keep;
+    }
+    *reinterpret_cast<u32x4*>(dst) = v;
+  };
+
+  // acc[nt][mt][i]: column wc*64 + nt*32 + (i/4)*8 + g*4 + i%4, row wr*64 + mt*32 + l32 of the unit
+  f32x16 acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
+
+  if (n_iter > 0) {
+    const int a_base = kUnitBytes + (wc * 64 + l32) * kRowBytes;  // W rows
+    const int b_base = (wr * 64 + l32) * kRowBytes;               // X rows
+    // Operands are read two substeps ahead of their MFMAs (register set = substep): one ahead is 128 cycles
+    // of MFMAs, less than the LDS pipe's queue of four wavefronts (256 units of K = 2048: 24.4 -> 22.5 us).
+    x8 a[4][NT], b[4][MT];
+    auto lread = [&](int stage, int sub, int idx) {  // W rows 0, both X row groups, W rows 1
+      const uint8_t* st = smem + stage * kStage;
+      const int x = rd_x ^ (sub << 5);
+      if (idx == 0) {
+        a[sub][0] = *reinterpret_cast<const x8*>(st + a_base + x);
+      } else if (idx <= MT) {
+        b[sub][idx - 1] = *reinterpret_cast<const x8*>(st + b_base + (idx - 1) * 32 * kRowBytes + x);
+      } else {
+        a[sub][idx - MT] = *reinterpret_cast<const x8*>(st + a_base + (idx - MT) * 32 * kRowBytes + x);
+      }
+    };
+    auto substep = [&](int set, int rstage, int rsub, int wstage, int j0, unsigned keep, int lentry) {
+#pragma unroll
+      for (int i = 0; i < NT * MT; ++i) {
+        const int nt = i / MT, mt = i % MT;
+        acc[nt][mt] = TT::mfma(a[set][nt], b[set][mt], acc[nt][mt]);
+        lread(rstage, rsub, i);
+        if (i & 1) {
+          lwrite(j0 + (i >> 1), wstage, keep);
+          gload(j0 + (i >> 1), lentry);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    int en1, en2, en3;
+    {
+      const int e0 = step_entry(0);
+#pragma unroll
+      for (int j = 0; j < P; ++j) gload(j, e0);
+      en1 = step_entry(1), en2 = step_entry(2), en3 = step_entry(3);
+      const unsigned keep0 = keep_of(e0), keep1 = keep_of(en1);
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        lwrite(j, 0, keep0);
+        gload(j, en1);
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * PS; ++j) {
+        lwrite(j, 1, keep1);
+        gload(j, en2);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int idx = 0; idx < NT + MT; ++idx) lread(0, sub, idx);
+    // Iteration it: stage it % 2 holds slab it; substeps 0 and 1 complete slab it+1 in the other stage,
+    // then (everyone has read all of slab it and written all of slab it+1) substeps 2 and 3 begin slab
+    // it+2 in this one.  A piece is requested again, a slab on, once it is written.
+    for (int it = 0; it < n_iter; ++it) {
+      const int st = it & 1;
+      const int en4_raw = step_entry_raw(it + 4);
+      const unsigned keep1 = keep_of(en1), keep2 = keep_of(en2);
+      substep(0, st, 2, st ^ 1, 2 * PS, keep1, en2);
+      substep(1, st, 3, st ^ 1, 3 * PS, keep1, en2);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): my reads of slab it and my writes of slab it+1 are done
+      __builtin_amdgcn_s_barrier();        // ... for every wavefront
+      const int en4 = __builtin_amdgcn_readfirstlane(en4_raw);
+      substep(2, st ^ 1, 0, st, 0, keep2, en3);
+      substep(3, st ^ 1, 1, st, PS, keep2, en3);
+      en1 = en2;
+      en2 = en3;
+      en3 = en4;
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring
+
+  // ---- epilogue: each wavefront turns its 64 x 64 block through its quarter of the ring in fp32, into
+  // a layout in which 16 consecutive lanes cover a row; bias or partial is added there, the result
+  // rounded once.  Output and partial go through descriptors that end with the matrix. ----
+  uint8_t* const region = smem + wv * (kUnitSmemBytes / 4);
+  const int col4 = lane & 15, rsub = lane >> 4;
+  const int el_off = n0 + wc * 64 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 4*i
+  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
+  auto out_rsrc = [&](const void* base, int elem_bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
+        rows_here * p.n * elem_bytes, 0x00020000);
+  };
+  auto turn = [&](auto bias_tag, auto f32_tag) {
+    using BiasT = decltype(bias_tag);
+    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
+    constexpr bool kOutF32 = decltype(f32_tag)::value;
+    constexpr int kBytes = sizeof(BiasT);
+    BiasVec bm[16];
+    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (kPartial) {
+      // sixteen pieces in flight together while the rows turn through LDS
+      const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if constexpr (kBytes == 4) {
+          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, 4 * i * p.n * 4, 0));
+        } else {
+          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, 4 * i * p.n * 2, 0));
+        }
+      }
+    } else if (p.bias_kind == FO_BIAS_VECTOR) {
+      const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + wc * 64 + col4 * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+    }
+    // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 256 bytes = 16 chunks)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          f32x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = acc[nt][mt][i4 * 4 + j];
+          const int chunk = nt * 8 + i4 * 2 + g;
+          *reinterpret_cast<f32x4*>(region + (mt * 32 + l32) * 256 + ((chunk ^ (l32 & 15)) << 4)) = v;
+        }
+    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
+    f32x4 vals[8];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if ((i & 7) == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int rk = (i + k) * 4 + rsub;
+          vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 256 + ((col4 ^ (rk & 15)) << 4));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      f32x4 v = vals[i & 7];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (kPartial) {
+          v[j] += static_cast<float>(bm[i][j]);
+        } else {
+          v[j] += bvec[j];
+        }
+      }
+      if constexpr (kOutF32) {
+        // (no scalar offset: see the quads' store)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + 4 * i * p.n) * 4, 0, 2);
+      } else {
+        x4 out;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+        typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, 4 * i * p.n * 2, 2);
+      }
+    }
+  };
+  using std::false_type;
+  using std::true_type;
+  if constexpr (!kReduce) {
+    turn(T{}, false_type{});
+  } else if constexpr (kPartial) {
+    if (p.bias_f32) {
+      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
+    } else {
+      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+    }
+  } else {
+    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+  }
+}
+
 ListGeom make_geom(int32_t batch, int32_t m, int32_t n) {
   ListGeom gm;
   gm.batch = batch;
@@ -1128,8 +1442,39 @@ int64_t workspace_ints(const ListGeom& gm, int64_t* max_quads_out) {
   return 16 + kQuadInts * max_quads;
 }
 
+// a workgroup per unit
+template <typename T, bool kReduce, bool kHalf, bool kAux>
+int launch_units(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
+  static std::atomic<bool> attr_set[64] = {};
+  int dev = 0;
+  FO_HIP_CALL(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_unit_kernel<T, kReduce, kHalf, kAux>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kUnitSmemBytes));
+    if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
+  }
+  p.n_row_tiles = gm.n_row_tiles;
+  p.n_col_tiles = gm.n_col_tiles;
+  const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
+  const int64_t grid = (units + kXcds - 1) / kXcds * kXcds;
+  gemm_unit_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kUnitSmemBytes, stream>>>(p);
+  FO_CHECK_LAUNCH();
+  return FO_OK;
+}
+
 template <typename T, bool kReduce, bool kHalf, bool kAux>
 int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace, hipStream_t stream) {
+  const int num_cu = fo_num_cu();
+  if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
+  // A workgroup per unit while all of them fit the chip at once, two per CU: quads would leave most CUs
+  // idle or without their fourth unit.  Measured (us, quads -> units): 144 units of K = 1024 28 -> 12,
+  // 256 of K = 2048 46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged.  Above
+  // that it depends on the flags, which the host does not see: 864 units of K = 3072 83 -> 98 dense,
+  // 59 -> 43 with a quarter flagged.  (The fused quantiser needs a unit's absmax: quads only.)
+  if constexpr (kReduce || !kAux) {
+    if (static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles <= 2 * num_cu)
+      return launch_units<T, kReduce, kHalf, kAux>(p, gm, stream);
+  }
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
   // are atomic because host threads may launch concurrently, and setting it twice is harmless)
   static std::atomic<bool> attr_set[64] = {};
@@ -1147,8 +1492,6 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
   p.n_cp = gm.n_cp;
   p.n_win = gm.n_win;
   p.inline_cells = 0;
-  int num_cu = fo_num_cu();
-  if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
   int64_t grid = (num_cu + kXcds - 1) / kXcds * kXcds;  // one persistent workgroup per CU
   const int64_t cap = (max_quads + kXcds - 1) / kXcds * kXcds;
   if (grid > cap) grid = cap;

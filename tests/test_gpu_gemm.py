@@ -443,6 +443,44 @@ def test_gemm_o_cursors_and_fixed_stride_agree(dev, shape):
     assert rel_l2(got[0, :256].cpu(), dense) <= REL_L2
 
 
+@pytest.mark.parametrize("case", [(1, 128, 1), (129, 128, 1), (1100, 64, 4), (1100, 128, 8), (2176, 96, 4), (3000, 256, 8),
+                                  (130, 32, 12)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_workgroup_per_unit_equals_quads(dev, case, dtype):
+    """Launches of few units give each a workgroup of its own, longer ones compute quads: the same
+    inputs alone (few units) and as one of many batch entries (more than two units per CU) give the same
+    bits, because both add a unit's k steps in the same order.  One and two token rows past a block,
+    heads of 32 to 256 columns (slabs that count for one half only), every unit of the chip in use
+    (3000 x 2048: 384 units)."""
+    import flashomni_amd as fo
+    m, hd, heads = case
+    n = heads * hd
+    units = -(-m // 128) * (n // 128)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert units <= 2 * cus
+    batch = 2 * cus // units + 1
+    info, packed, indptr = _flags(batch, -(-m // 128) + 1, heads, 0.6, seed=m + hd)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+
+    def chain(x, ip):
+        q = torch.full_like(x, -3.0)
+        fo.flashomni_gemm(x, w, heads, pk, ip, 128, b, out=q)
+        full = fo.flashomni_gemm(x, w, heads, num_text_tokens=0, bias=b, is_full=True)
+        part = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=b, is_for_cache=True)
+        part32 = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, is_for_cache=True, out_dtype=torch.float32)
+        return [q, full, part, part32, fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part),
+                fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part32)]
+
+    many = chain(x, ip)
+    for i in sorted({0, batch // 2, batch - 1}):
+        for k, (one, all_) in enumerate(zip(chain(x[i:i + 1].contiguous(), ip[i:i + 2].contiguous()), many)):
+            assert torch.equal(one[0], all_[i]), (i, k)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch", [1, 2, 5])
 def test_fp32_output_rounds_to_the_16_bit_one(dev, batch, dtype):
