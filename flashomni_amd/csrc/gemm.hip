@@ -266,6 +266,32 @@ __device__ __forceinline__ void for_each_quad(uint32_t m0, uint32_t m1, bool col
   }
 }
 
+// The same for work items of at most two units that share a tile (`pairs`, see gemm_kernel): two rows of a
+// column, or both columns of a row, or one unit.
+template <typename F>
+__device__ __forceinline__ void for_each_pair(uint32_t m0, uint32_t m1, F&& f) {
+  while (__popc(m0) >= 2) {
+    const int r0 = pop_lowest(&m0), r1 = pop_lowest(&m0);
+    f(r0, r1, 0x5, 0);
+  }
+  while (__popc(m1) >= 2) {
+    const int r0 = pop_lowest(&m1), r1 = pop_lowest(&m1);
+    f(r0, r1, 0xA, 0);
+  }
+  if (m0 && m0 == m1) {
+    f(pop_lowest(&m0), -1, 0x3, 0);
+  } else {
+    if (m0) f(pop_lowest(&m0), -1, 0x1, 0);
+    if (m1) f(pop_lowest(&m1), -1, 0x2, 0);
+  }
+}
+// how many that are: of an odd number of rows the last one is left over
+__device__ __forceinline__ int count_pairs(uint32_t m0, uint32_t m1) {
+  const int n0 = __popc(m0), n1 = __popc(m1);
+  const bool together = (n0 & n1 & 1) && __clz(m0) == __clz(m1);
+  return (n0 + 1) / 2 + (n1 + 1) / 2 - (together ? 1 : 0);
+}
+
 struct ListArgs {
   const uint8_t* sparse_info;
   const int32_t* sparse_info_indptr;
@@ -396,6 +422,14 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   int q_lo, q_len;
   bool inline_list = false;
   if constexpr (!kReduce) inline_list = p.inline_cells > 0;
+  // Few flagged units (GEMM-Q that lists its own work): a quad would keep one CU busy for four units' time
+  // while others idle.  If items of at most two units are no more than the workgroups, the list is made of
+  // those, and two wavefronts share a unit: each takes two of a slab's four substeps (half of k), and the
+  // halves are added through LDS at the end.  Measured with K = 3072 (us, quads -> pairs): 16 k tokens x 24
+  // heads with one unit in ten flagged 60 -> 45, 4.6 k tokens with a quarter flagged 60 -> 43.  The error
+  // against 64-bit sums is the same (bf16 1.66e-3, fp16 2.08e-4: the rounding of the result).
+  constexpr bool kPairs = !kReduce && !kAux;
+  bool pairs = false;
   if (inline_list) {
     if constexpr (!kReduce) {
       // thread = cell: masks, quad count, workgroup-wide inclusive scan of the counts
@@ -412,6 +446,9 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         cell_masks(gm, tid, true, p.sparse_info, p.sparse_info_indptr, p.sparse_q_size, p.num_heads,
                    p.head_dim, p.num_text_tokens, &b, &row0, &cp, &m0, &m1);
         for_each_quad(m0, m1, true, [&](int, int, int, int) { ++cnt; });
+        if constexpr (kPairs) {  // (both counts in one scan: at most 16 per cell and kInlineCells cells)
+          cnt += count_pairs(m0, m1) << 16;
+        }
         s_cell_mask[2 * tid] = m0;
         s_cell_mask[2 * tid + 1] = m1;
       }
@@ -430,7 +467,13 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         if (w < wv) base += t;
         total += t;
       }
-      if (tid < kInlineCells) s_cell_pref[tid + 1] = base + incl;
+      incl += base;
+      if constexpr (kPairs) {
+        pairs = (total >> 16) <= static_cast<int>(gridDim.x);
+        total = pairs ? total >> 16 : total & 0xFFFF;
+        incl = pairs ? incl >> 16 : incl & 0xFFFF;
+      }
+      if (tid < kInlineCells) s_cell_pref[tid + 1] = incl;
       if (tid == 0) s_cell_pref[0] = 0;
       q_lo = static_cast<int>(static_cast<int64_t>(total) * xcd / kXcds);
       q_len = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / kXcds) - q_lo;
@@ -470,7 +513,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
           const int cp = tid % p.n_cp, t = tid / p.n_cp;
           const int w = t % p.n_win, b = t / p.n_win;
           int k = q - s_cell_pref[tid];
-          for_each_quad(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], true, [&](int r0, int r1, int v, int r2) {
+          auto entry = [&](int r0, int r1, int v, int r2) {
             if (k == 0) {
               s_entry[0] = b;
               s_entry[1] = w * kWindow + r0;
@@ -485,7 +528,12 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
               s_entry[6] = w * kWindow + r2;
             }
             --k;
-          });
+          };
+          if (kPairs && pairs) {
+            for_each_pair(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], entry);
+          } else {
+            for_each_quad(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], true, entry);
+          }
         }
         __syncthreads();
         bz = s_entry[0];
@@ -717,6 +765,199 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   auto pop = [&]() {
     if (tid == 0) popped = per_xcd + atomicAdd(p.cursor + xcd, 1);  // (the first per_xcd items are dealt by slot)
   };
+  if constexpr (kPairs) {
+    if (pairs) {
+      // One item of at most two units (no more items than workgroups), two wavefronts each.
+      if (slot >= q_len) return;
+      const Item item = decode_item(slot);
+      n_iter = build_steps(item, 0);
+      // Three tiles at most: X r0, X r1, W of a column pair; X, W c0, W c1 of a row's two units; X, none, W.
+      // (What the loop waits for is the vector memory path: a CU takes ~37 bytes per clock through it, and
+      // loads that fetch nothing hold it up as well: with four tiles, one or two of them empty, 51 and 47 us.
+      // Two slabs in flight in staging registers, against the latency of a tile's first touch, do not fit
+      // the registers beside 256 accumulators: 757 spilled.)
+      constexpr int PP = 12;  // pieces per wavefront and slab
+      make_rsrc(item);
+      const bool two_cols = item.valid == 0x3;
+      rsrc[1] = two_cols ? rsrc[2] : (item.valid & (item.valid - 1)) ? rsrc[1] : rsrc_none;
+      if (two_cols || !(item.valid & 0x5)) rsrc[2] = rsrc[3];
+      // wavefronts 0, 1: the lowest unit of the mask, 2, 3: the other one, if there is one
+      const int first = __builtin_ctz(item.valid), rest = item.valid & (item.valid - 1);
+      const int unit = wv < 2 || !rest ? first : __builtin_ctz(rest);
+      const int m0 = (unit >> 1 ? item.r[1] : item.r[0]) * kTile, n0 = (unit & 1 ? item.c[1] : item.c[0]) * kTile;
+      auto barrier = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+      };
+      {
+        const int e0 = step_entry(0), e1 = step_entry(1), e2 = step_entry(2);
+        const unsigned keep0 = keep_of(e0), keep1 = keep_of(e1);
+#pragma unroll
+        for (int j = 0; j < PP; ++j) gload(j, e0);
+#pragma unroll
+        for (int j = 0; j < PP; ++j) {
+          lwrite(j, 0, keep0);
+          gload(j, e1);
+        }
+#pragma unroll
+        for (int j = 0; j < PP / 2; ++j) {
+          lwrite(j, 1, keep1);
+          gload(j, e2);
+        }
+        barrier();
+      }
+      // Iteration it: stage it % 2 holds slab it; beside the first substep the second half of the pieces
+      // completes slab it+1 in the other stage, the barrier, beside the second the first half begins slab
+      // it+2 in this one.
+      if (wv >= 2 && !rest) {  // no unit: moves its pieces and keeps the barrier sequence of the others
+        for (int it = 0; it < n_iter; ++it) {
+          const int st = it & 1;
+          const int en1 = step_entry(it + 1), en2 = step_entry(it + 2), en3 = step_entry(it + 3);
+#pragma unroll
+          for (int j = PP / 2; j < PP; ++j) {
+            lwrite(j, st ^ 1, keep_of(en1));
+            gload(j, en2);
+          }
+          barrier();
+#pragma unroll
+          for (int j = 0; j < PP / 2; ++j) {
+            lwrite(j, st, keep_of(en2));
+            gload(j, en3);
+          }
+        }
+        barrier();
+        barrier();
+        barrier();
+        return;
+      }
+      f32x16 acc[NT][MT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
+      const int a_base = (two_cols && unit == 0 ? 1 : 2) * kUnitBytes + l32 * kRowBytes;
+      const int b_base = (two_cols ? 0 : wv >> 1) * kUnitBytes + l32 * kRowBytes;
+      const int sub0 = 2 * (wv & 1);  // my substeps: sub0, sub0 + 1
+      x8 a[2][NT], b[2][MT];
+      auto lread = [&](int set, int stage, int sub, int idx) __attribute__((always_inline)) {
+        const uint8_t* st = smem + stage * kStageBytes;
+        const int x = rd_x ^ (sub << 5);
+        if (idx == 0) {
+          a[set][0] = *reinterpret_cast<const x8*>(st + a_base + x);
+        } else if (idx <= MT) {
+          b[set][idx - 1] = *reinterpret_cast<const x8*>(st + b_base + (idx - 1) * 32 * kRowBytes + x);
+        } else {
+          a[set][idx - MT] = *reinterpret_cast<const x8*>(st + a_base + (idx - MT) * 32 * kRowBytes + x);
+        }
+      };
+      auto substep = [&](int set, int rstage, int rsub, int wstage, int j0, unsigned keep, int lentry)
+                         __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NT * MT; ++i) {
+          const int nt = i / MT, mt = i % MT;
+          acc[nt][mt] = TT::mfma(a[set][nt], b[set][mt], acc[nt][mt]);
+          if ((i & 1) == 0) {
+            lread(set ^ 1, rstage, rsub, i >> 1);
+          } else {
+            if ((i >> 1) < PP / 2) {
+              lwrite(j0 + (i >> 1), wstage, keep);
+              gload(j0 + (i >> 1), lentry);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+#pragma unroll
+      for (int idx = 0; idx < NT + MT; ++idx) lread(0, 0, sub0, idx);
+      for (int it = 0; it < n_iter; ++it) {
+        const int st = it & 1;
+        const int en1 = step_entry(it + 1), en2 = step_entry(it + 2), en3 = step_entry(it + 3);
+        substep(0, st, sub0 + 1, st ^ 1, PP / 2, keep_of(en1), en2);
+        barrier();
+        substep(1, st ^ 1, sub0, st, 0, keep_of(en2), en3);
+      }
+      barrier();
+      // The two wavefronts of a unit hold sums over different k: each hands half of the rows over through
+      // its quarter of the ring (32 KB, 16 bytes per lane and instruction), adds what it gets to the rows
+      // it keeps, turns those as in the epilogue below and stores them.
+      // (even wavefronts keep rows 0..63, odd ones 64..127: chosen value by value, a branch makes the
+      // compiler copy all accumulators)
+      {
+        const bool odd = wv & 1;
+        const int keep_row = odd ? 64 : 0;
+        uint8_t* const region = smem + wv * (kSmemBytes / 4);
+        const uint8_t* const other = smem + (wv ^ 1) * (kSmemBytes / 4);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+              f32x4 v;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) v[j] = odd ? acc[nt][h][i4 * 4 + j] : acc[nt][2 + h][i4 * 4 + j];
+              *reinterpret_cast<f32x4*>(region + ((h * NT + nt) * 4 + i4) * 1024 + lane * 16) = v;
+              __builtin_amdgcn_sched_barrier(0);
+            }
+        barrier();  // every wavefront's pieces are written
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            f32x4 v[4];
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4)
+              v[i4] = *reinterpret_cast<const f32x4*>(other + ((h * NT + nt) * 4 + i4) * 1024 + lane * 16);
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) acc[nt][h][i4 * 4 + j] = (odd ? acc[nt][2 + h][i4 * 4 + j] : acc[nt][h][i4 * 4 + j]) + v[i4][j];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        barrier();  // ... and read
+        const int col4 = l32;
+        float bvec[4] = {0.f, 0.f, 0.f, 0.f};
+        if (p.bias_kind == FO_BIAS_VECTOR) {
+          const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + col4 * 4);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+        }
+        const int64_t row0 = static_cast<int64_t>(item.bz) * p.m + m0;
+        const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
+            static_cast<T*>(p.y) + row0 * p.n, 0, min(p.m - m0, kTile) * p.n * 2, 0x00020000);
+        const int el_off = n0 + col4 * 4 + g * p.n;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          uint8_t* const half = region + h * (kSmemBytes / 8);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+              f32x4 v;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) v[j] = acc[nt][h][i4 * 4 + j];
+              *reinterpret_cast<f32x4*>(half + l32 * 512 + (((nt * 8 + i4 * 2 + g) ^ l32) << 4)) = v;
+              __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int rk = 2 * i + g;
+            const f32x4 v = *reinterpret_cast<const f32x4*>(half + rk * 512 + ((col4 ^ rk) << 4));
+            x4 out;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j] + bvec[j]);
+            typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2,
+                                                  (keep_row + h * 32 + 2 * i) * p.n * 2, 2);
+            if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+      return;
+    }
+  }
   if (popping) pop();
   int work = slot;
   bool have = work < q_len;
