@@ -316,6 +316,14 @@ struct BitRange {
   }
 };
 
+// what a row's record holds besides, kDirect only (in the other kernels' records it cost the two-term fp8
+// launch at 76 k tokens x 40 heads 1 %): the row's keep bits (words, position of its first bit, kv blocks
+// of the request); ptr0 is then the first kept block of this part among the row's kept blocks
+struct DirectMask {
+  const uint32_t* mask;
+  int mask_first, nkv;
+};
+struct NoMask {};
 constexpr int kDirectMaxCand = 1024;  // candidates (symbol row, head): two per thread of a workgroup
 constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
 constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologue, epilogue and exchange cost about as many
@@ -358,14 +366,10 @@ sparse_fa_kernel(const FaParams p) {
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   // this item / the next one, with everything the row's prologue needs: fetched by the popping lane
   // while the rest of the workgroup finishes the current row
-  struct RowInfo {
+  struct RowInfo : std::conditional<kDirect, DirectMask, NoMask>::type {
     int row, part, parts, slot, req, qb, head, q_begin, q_rows, kv_begin, kv_len, ptr0, nb;
     float q_scale;  // fp8: dequantisation scale of the row's q block
     int k_scale0;   // fp8: position of the request's first kv block in k_scale (the kv head's row)
-    // kDirect: the row's keep bits (words, position of its first bit, kv blocks of the request); ptr0 is then the
-    // first kept block of this part among the row's kept blocks
-    const uint32_t* mask;
-    int mask_first, nkv;
   };
   // (fetched with the rest of the record: read in the row's prologue, they would wait behind every
   // tile copy in flight)
@@ -663,14 +667,16 @@ sparse_fa_kernel(const FaParams p) {
     set_q_range(it);
     it.kv_begin = p.kv_indptr[it.req];
     it.kv_len = p.kv_indptr[it.req + 1] - it.kv_begin;
-    it.nkv = (it.kv_len + kBlockKV - 1) / kBlockKV;
-    it.mask = nullptr;
-    it.mask_first = 0;
-    if (!p.is_full) {
-      const BitRange r(p.kv_info + p.kv_info_indptr[it.req],
-                       (static_cast<int64_t>(it.qb) * p.symbol_heads + h) * it.nkv, it.nkv);
-      it.mask = r.words;
-      it.mask_first = r.first;
+    if constexpr (kDirect) {
+      it.nkv = (it.kv_len + kBlockKV - 1) / kBlockKV;
+      it.mask = nullptr;
+      it.mask_first = 0;
+      if (!p.is_full) {
+        const BitRange r(p.kv_info + p.kv_info_indptr[it.req],
+                         (static_cast<int64_t>(it.qb) * p.symbol_heads + h) * it.nkv, it.nkv);
+        it.mask = r.words;
+        it.mask_first = r.first;
+      }
     }
     it.q_scale = 1.f;
     it.k_scale0 = 0;
@@ -830,7 +836,7 @@ sparse_fa_kernel(const FaParams p) {
       const int lo = __builtin_amdgcn_readfirstlane(it.ptr0), n = __builtin_amdgcn_readfirstlane(it.nb);
       if (p.is_full) {
         for (int i = lane; i < n; i += 64) s_blk2[slot_idx][i] = static_cast<uint16_t>(lo + i);
-      } else {
+      } else if constexpr (kDirect) {
         BitRange r(nullptr, 0, __builtin_amdgcn_readfirstlane(it.nkv));
         r.first = __builtin_amdgcn_readfirstlane(it.mask_first);
         const uint64_t m = reinterpret_cast<uint64_t>(it.mask);
@@ -882,13 +888,6 @@ sparse_fa_kernel(const FaParams p) {
       fetch_next(0);
     }
   }
-  auto next_item = [&](int slot_idx) __attribute__((always_inline)) {
-    if constexpr (kDirect) {
-      direct_next(slot_idx);
-    } else {
-      fetch_next(slot_idx);
-    }
-  };
   for (int row_it = 0;; ++row_it) {
     // s_next_row is published; everyone is done with the previous row's LDS data.  (Not
     // __syncthreads(): its fence would also wait for the row just stored to be acknowledged by
@@ -948,7 +947,9 @@ sparse_fa_kernel(const FaParams p) {
         for (int j = 0; j < 8; ++j) reinterpret_cast<u32x4*>(dst)[j] = z;
         if (p.lse && g_p == 0) p.lse[q_tok * p.num_heads + my_head] = kNegInf;
       }
-      if (wv == kFetchWave) next_item((row_it + 1) & 1);
+      if (wv == kFetchWave) {
+        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1);
+      }
       continue;
     }
 
@@ -1777,7 +1778,9 @@ sparse_fa_kernel(const FaParams p) {
       }
       __syncthreads();
     }
-    if (wv == kFetchWave) next_item((row_it + 1) & 1);
+    if (wv == kFetchWave) {
+        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1);
+      }
     float m_all = 0.f, d_all = 0.f;  // kv group 0: row maximum and row sum over both groups
     // A lane owns one q row and runs of four d: stored from here, a row would leave as 32 scattered
     // 8-byte pieces per instruction (measured: ~12 k cycles per row).  The finished row goes through
