@@ -489,12 +489,18 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   if (rc == FO_NOT_DIRECT) {
     if (args[15] == Py_None) Py_RETURN_FALSE;
-    if (!out && !fresh.defined()) fresh = at::zeros(q->sizes(), q->options());
+    // (the decoder's launches for longer lists clear the rows of a fresh output that nothing computes)
+    const bool clears = own && int64_t(p->z.n_q_blocks) * p->symbol_heads >= fo_decode_sparse_clear_min_pairs();
+    if (!out) fresh = clears ? at::empty(q->sizes(), q->options()) : at::zeros(q->sizes(), q->options());
     const Tensor& o = out ? *out : fresh;
     int32_t* shares = ws ? wl[9] : nullptr;
-    if (fo_decode_sparse(a.info, a.kv_info, a.info_indptr, a.kv_info_indptr, a.blk_req, a.blk_qb, a.kv_indptr,
-                         p->z.n_q_blocks, p->symbol_heads, 128, full, wl[0], wl[1], wl[2], wl[3], wl[4], wl[5], wl[6],
-                         wl[7], wl[8], shares, stream))
+    if (clears ? fo_decode_sparse_clear(a.info, a.kv_info, a.info_indptr, a.kv_info_indptr, a.blk_req, a.blk_qb,
+                                        a.kv_indptr, p->z.n_q_blocks, p->symbol_heads, 128, full, wl[0], wl[1], wl[2],
+                                        wl[3], wl[4], wl[5], wl[6], wl[7], wl[8], shares, o.data_ptr(), o.stride(0),
+                                        o.stride(1), a.qo_indptr, p->packed ? p->num_qo / p->num_kv : 1, stream)
+               : fo_decode_sparse(a.info, a.kv_info, a.info_indptr, a.kv_info_indptr, a.blk_req, a.blk_qb, a.kv_indptr,
+                                  p->z.n_q_blocks, p->symbol_heads, 128, full, wl[0], wl[1], wl[2], wl[3], wl[4], wl[5],
+                                  wl[6], wl[7], wl[8], shares, stream))
       return raise_last();
     if (fo_sparse_fa_run(a.q, a.k, a.v, o.data_ptr(), a.lse, code, nullptr, nullptr, nullptr, nullptr, a.q_stride_n,
                          a.q_stride_h, a.k_stride_n, a.k_stride_h, a.v_stride_n, a.v_stride_h, o.stride(0), o.stride(1),

@@ -573,6 +573,29 @@ __global__ void __launch_bounds__(kScanThreads) decode_small_kernel(
   }
 }
 
+// A fresh attention output whose rows of q blocks that are not computed the fill kernel clears (o = null: none).
+// The whole output was cleared by a launch of its own before: 26 us at 33 k tokens x 24 heads, where three
+// tenths of the rows are skipped, 16 us at 16.9 k x 24 where none is; here TIMES.
+struct ClearRows {
+  uint8_t* o;
+  int64_t stride_n, stride_h;  // bytes
+  const int32_t* qo_indptr;
+  int32_t gqa_pack;  // > 1: a row is a (token, q head of the group) pair
+};
+
+// one wavefront: the rows of q block qb of request req and (kv) head `head`, 256 bytes each, 16 bytes a lane
+__device__ __forceinline__ void clear_rows(const ClearRows& z, int req, int qb, int head, int lane) {
+  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+  const int q0 = z.qo_indptr[req], gq = z.gqa_pack;
+  const int rows = min(128, (z.qo_indptr[req + 1] - q0) * gq - qb * 128);
+  uint8_t* const dst = z.o + q0 * z.stride_n + head * gq * z.stride_h + (lane & 15) * 16;
+  for (int r = lane >> 4; r < rows; r += 4) {
+    const int pr = qb * 128 + r, tok = gq > 1 ? pr / gq : pr;
+    __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u},
+                                reinterpret_cast<u32x4*>(dst + tok * z.stride_n + (pr - tok * gq) * z.stride_h));
+  }
+}
+
 __global__ void __launch_bounds__(kCountThreads) decode_fill_kernel(
     const uint8_t* __restrict__ sparse_info, const uint8_t* __restrict__ sparse_kv_info,
     const int32_t* __restrict__ sparse_info_indptr,
@@ -584,12 +607,16 @@ __global__ void __launch_bounds__(kCountThreads) decode_fill_kernel(
     int32_t* __restrict__ kv_row_ptr, int32_t* __restrict__ kv_idx,
     int32_t* __restrict__ head_cursor, int32_t* __restrict__ order,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ sched,
-    int32_t* __restrict__ shares) {
+    int32_t* __restrict__ shares, ClearRows clear) {
   const int lane = threadIdx.x % kWave;
   const int64_t c = static_cast<int64_t>(blockIdx.x) * (kCountThreads / kWave) + threadIdx.x / kWave;
   if (c >= n_cand) return;
   const int32_t pos = row_pos[c];
-  if (pos < 0) return;
+  if (pos < 0) {
+    const int32_t t = static_cast<int32_t>(c / num_heads);
+    if (clear.o) clear_rows(clear, blk_req[t], blk_qb[t], static_cast<int32_t>(c - static_cast<int64_t>(t) * num_heads), lane);
+    return;
+  }
   const Candidate cd = load_candidate(c, num_heads, block_kv, is_full, sparse_info,
                                       sparse_info_indptr, blk_req, blk_qb, kv_indptr);
   int32_t out = kv_pos[c];
@@ -664,7 +691,8 @@ int decode_impl(const uint8_t* sparse_info, const uint8_t* sparse_kv_info, const
                 const int32_t* kv_indptr, int32_t n_blk, int32_t num_heads, int32_t block_kv, int is_full,
                 int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr, int32_t* kv_idx,
                 int32_t* counts, int32_t* order, int32_t* sched, int32_t* scratch_ptr, int32_t* shares,
-                void* stream) {
+                void* stream,
+                const ClearRows& clear = ClearRows{}) {
   FO_REQUIRE(n_blk >= 0 && num_heads > 0 && num_heads <= kMaxHeads && block_kv > 0,
              "decode: bad sizes");
   FO_REQUIRE(counts && kv_row_ptr && order && sched, "decode: null output");
@@ -709,7 +737,7 @@ int decode_impl(const uint8_t* sparse_info, const uint8_t* sparse_kv_info, const
     decode_fill_kernel<<<grid, kCountThreads, 0, s>>>(
         sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
         kv_indptr, n_cand, num_heads, block_kv, is_full, act, cnt, row_req, row_qb, row_head,
-        kv_row_ptr, kv_idx, head_cursor, order, counts, sched, shares);
+        kv_row_ptr, kv_idx, head_cursor, order, counts, sched, shares, clear);
     FO_CHECK_LAUNCH();
   }
   return FO_OK;
@@ -748,6 +776,27 @@ extern "C" int fo_decode_sparse(const uint8_t* sparse_info, const uint8_t* spars
   return decode_impl(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
                      kv_indptr, n_blk, num_heads, block_kv, is_full, row_req, row_qb, row_head, kv_row_ptr,
                      kv_idx, counts, order, sched, scratch, shares, stream);
+}
+
+extern "C" int32_t fo_decode_sparse_clear_min_pairs(void) { return kScanThreads + 1; }
+
+extern "C" int fo_decode_sparse_clear(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
+                                      const int32_t* sparse_info_indptr, const int32_t* sparse_kv_info_indptr,
+                                      const int32_t* blk_req, const int32_t* blk_qb, const int32_t* kv_indptr,
+                                      int32_t n_blk, int32_t num_heads, int32_t block_kv, int is_full, int32_t* row_req,
+                                      int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr, int32_t* kv_idx,
+                                      int32_t* counts, int32_t* order, int32_t* sched, int32_t* scratch, int32_t* shares,
+                                      void* o, int64_t o_stride_n, int64_t o_stride_h, const int32_t* qo_indptr,
+                                      int32_t gqa_pack, void* stream) {
+  FO_REQUIRE(static_cast<int64_t>(n_blk) * num_heads >= fo_decode_sparse_clear_min_pairs(),
+             "decode: lists of up to %d (q-block, head) pairs are decoded without clearing", kScanThreads);
+  FO_REQUIRE(o && qo_indptr && gqa_pack >= 1, "decode: null pointer or bad group");
+  FO_REQUIRE((reinterpret_cast<uintptr_t>(o) & 15) == 0 && o_stride_n % 8 == 0 && o_stride_h % 8 == 0,
+             "decode: the rows of o must be 16-byte aligned");
+  const ClearRows clear = {static_cast<uint8_t*>(o), 2 * o_stride_n, 2 * o_stride_h, qo_indptr, gqa_pack};
+  return decode_impl(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
+                     kv_indptr, n_blk, num_heads, block_kv, is_full, row_req, row_qb, row_head, kv_row_ptr,
+                     kv_idx, counts, order, sched, scratch, shares, stream, clear);
 }
 
 extern "C" int64_t fo_decode_sparse_static_max_pairs(void) { return (kStaticScratchInts - kHistSlots) / 2; }

@@ -165,6 +165,23 @@ int fo_decode_sparse(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
                      int32_t* scratch, int32_t* shares, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * fo_decode_sparse that also clears, in a fresh 16-bit attention output o [nnz_q, H, 128] (strides in
+ * elements, rows 16-byte aligned), the rows of the (q block, head) pairs that are not listed.  Lists of
+ * at least fo_decode_sparse_clear_min_pairs() pairs; gqa_pack = H / H_kv where the rows are packed
+ * (fo_sparse_fa_run's gqa_packed), else 1.  qo_indptr [batch+1] on the device.  No counterpart in the
+ * reference (it clears the whole output first).
+ * ------------------------------------------------------------------------------------------- */
+int32_t fo_decode_sparse_clear_min_pairs(void);
+int fo_decode_sparse_clear(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
+                           const int32_t* sparse_info_indptr, const int32_t* sparse_kv_info_indptr,
+                           const int32_t* blk_req, const int32_t* blk_qb, const int32_t* kv_indptr,
+                           int32_t n_blk, int32_t num_heads, int32_t block_kv, int is_full,
+                           int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr,
+                           int32_t* kv_idx, int32_t* counts, int32_t* order, int32_t* sched,
+                           int32_t* scratch, int32_t* shares, void* o, int64_t o_stride_n,
+                           int64_t o_stride_h, const int32_t* qo_indptr, int32_t gqa_pack, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * fo_decode_sparse without the `scratch` argument, for callers that cannot allocate device memory
  * for it (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  The decoder's scratch (2*n_blk*H + 8192 int32) lives in a 1 MiB

@@ -80,3 +80,28 @@ def test_fresh_output_of_packed_tiles(dev, group):
     junk = torch.full((64 << 20,), 0x7f, dtype=torch.uint8, device=dev)
     del junk
     assert torch.equal(w.run(q, k, v, *sym), exp)
+
+
+@pytest.mark.parametrize("case", [([2000, 1, 130, 1500], [300, 77, 513, 640], 40, 1, 0.5),
+                                  ([5000, 129, 1], [640, 300, 77], 8, 4, 0.3), ([9000], [300], 16, 1, 0.0)])
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+def test_fresh_output_of_decoded_lists(dev, case, layout):
+    """Lists above 1024 pairs: the decoder's launches clear the skipped rows of a fresh output (ragged last
+    tiles, tiles of grouped-query rows, nothing to compute); the same bits as over a cleared output."""
+    import flashomni_amd as fo
+    ql, kl, hkv, group, pa = case
+    hq = hkv * group
+    m = make_ragged_masks([n * group for n in ql], kl, hkv, pa, 0.5, seed=6)
+    qo = torch.from_numpy(np.concatenate([[0], np.cumsum(ql)]).astype(np.int32))
+    g = torch.Generator(device=dev).manual_seed(6)
+    kv_shape = (sum(kl), hkv, 128) if layout == "NHD" else (hkv, sum(kl), 128)
+    q, k, v = (torch.randn(*s, generator=g, device=dev).to(torch.bfloat16) for s in ((sum(ql), hq, 128), kv_shape, kv_shape))
+    t = lambda n: torch.from_numpy(m[n]).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev), layout)
+    w.plan(qo, t("kv_indptr"), hq, hkv, 128, q_data_type=torch.bfloat16)
+    sym = [t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    exp = w.run(q, k, v, *sym, out=torch.zeros_like(q))
+    for _ in range(3):
+        junk = torch.full((256 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
+        del junk
+        assert torch.equal(w.run(q, k, v, *sym), exp)
