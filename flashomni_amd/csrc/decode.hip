@@ -575,7 +575,7 @@ __global__ void __launch_bounds__(kScanThreads) decode_small_kernel(
 
 // A fresh attention output whose rows of q blocks that are not computed the fill kernel clears (o = null: none).
 // The whole output was cleared by a launch of its own before: 26 us at 33 k tokens x 24 heads, where three
-// tenths of the rows are skipped, 16 us at 16.9 k x 24 where none is; here TIMES.
+// tenths of the rows are skipped, 16 us at 16.9 k x 24 where none is (1.1 % and 1.9 % of those calls).
 struct ClearRows {
   uint8_t* o;
   int64_t stride_n, stride_h;  // bytes
