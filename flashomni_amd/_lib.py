@@ -30,6 +30,9 @@ SIGNATURES = {
     "fo_sparse_block_table": ([c_vp, c_u32, c_u32, c_vp, c_vp, c_i64, c_vp], c_int),
     "fo_decode_sizes": ([c_vp, c_vp, c_u32, c_u32, c_u32, c_u32, c_vp, c_vp, c_vp], c_int),
     "fo_decode_sparse": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 9 + [c_vp, c_vp], c_int),
+    "fo_decode_sparse_clear_min_pairs": ([], c_i32),
+    "fo_decode_sparse_clear": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 9 + [c_vp, c_vp, c_i64, c_i64, c_vp, c_i32, c_vp],
+                               c_int),
     "fo_decode_sparse_static_max_pairs": ([], c_i64),
     "fo_decode_sparse_static": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 8 + [c_vp, c_vp], c_int),
     "fo_sparse_fa_split_workspace_bytes": ([], c_i64),
