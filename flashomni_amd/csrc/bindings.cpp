@@ -456,7 +456,9 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   // the launch without a decoded list (it clears what it skips: every row of a fresh output is its own)
   const bool own = !out && p->from_zero && q->size(0) == p->z.total_q;
   // (symbol tensors much larger than the batch needs are not worth copying)
-  const bool small = full || (sym[0]->numel() <= p->z.min_info + 4096 && sym[1]->numel() <= p->z.min_kv_info + 4096);
+  // (nor is a request served whose rows may list more kv blocks than the kernel has room for, 4096: the decoded
+  // forms take whole rows of it up to that many)
+  const bool small = p->z.max_kv_len <= 4096 * 128 && (full || (sym[0]->numel() <= p->z.min_info + 4096 && sym[1]->numel() <= p->z.min_kv_info + 4096));
   int rc = FO_NOT_DIRECT;
   if (small && p->z.max_rows > 0 && fo_sparse_attention_direct_serves(&a)) {
     if (!out) fresh = own ? at::empty(q->sizes(), q->options()) : at::zeros(q->sizes(), q->options());

@@ -769,8 +769,10 @@ sparse_fa_kernel(const FaParams p) {
           it.parts = parts[u];
           it.slot = first;
           it.ptr0 = it.part * per;
-          it.nb = max(min(n[u] - it.ptr0, per), 0);
-          // (the parts are as long as ceil allows: the last one may be empty)
+          // (no part is empty but that of a row without kv blocks: per <= want, so parts - 1 of them are fewer
+          // than n blocks.  Longer than the LDS list, a part is cut, as the other forms cut a row: callers that plan a
+          // batch send requests of more than kRowBlocks kv blocks to the decoder)
+          it.nb = min(max(min(n[u] - it.ptr0, per), 0), kRowBlocks);
           s_items[0] = it;
         }
         first += parts[u];
@@ -818,7 +820,7 @@ sparse_fa_kernel(const FaParams p) {
             it.slot = j_lo;
           }
           it.ptr0 = max(a, u) - u;
-          it.nb = max(min(b, e) - u - it.ptr0, 0);
+          it.nb = min(max(min(b, e) - u - it.ptr0, 0), kRowBlocks);
         }
       }
       s_items[lane] = it;

@@ -205,6 +205,23 @@ def test_symbols_rewritten_in_place_are_decoded_again(dev):
     assert max_abs(o_reuse.cpu()[touched], exp_b[touched]) <= 2e-2
 
 
+def test_attention_ops_request_beyond_the_lds_list(dev):
+    """A request of 4700 kv blocks, half of them kept: a short list, but its rows may hold more blocks than the
+    4096 that a workgroup can list, so it is decoded (the wrapper refuses such requests, the operators do not)."""
+    from flashomni_amd.ops import _plans
+    m = make_ragged_masks([200], [4700 * 128 - 5], 1, 1.0, 0.5, seed=34)
+    g = torch.Generator().manual_seed(34)
+    q, k, v = (torch.randn(n, 1, 128, generator=g).to(torch.bfloat16) for n in (200, 4700 * 128 - 5, 4700 * 128 - 5))
+    state = _plan(dev, m, 1)
+    o = torch.zeros(200, 1, 128, dtype=torch.bfloat16, device=dev)
+    _run(dev, state, q.to(dev), k.to(dev), v.to(dev), m, o)
+    assert _plans[(o.device.index, state[1].data_ptr())].native.state == 0
+    exp = oracle.sparse_attention(q, k, v, m["packed_info"], m["packed_keep"], m["info_indptr"], m["keep_indptr"],
+                                  m["qo_indptr"], m["kv_indptr"], out=torch.zeros_like(q))
+    # (sums over 3 x 10^5 keys: the output is of the order of 2e-3, so the bound is relative)
+    assert rel_l2(o.cpu(), exp) <= 1e-2
+
+
 def test_attention_ops_logits_soft_cap(dev):
     """The run operator's logits_soft_cap argument (csrc/batch_sparseFA.cu:67-201 passes it to the
     variant, variants.cuh:43-56): equal to the wrapper planned with the same cap, and within the path's
