@@ -18,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -593,13 +594,17 @@ PyObject* segment_packbits(PyObject*, PyObject* const* args, Py_ssize_t n) {
   bool arrived = false;
   hipError_t err = hipSuccess;
   if (!rc) {
-    // The word arrives a few microseconds after the kernel's start: looked at for about as long, then the
-    // stream is waited for (the kernel may be behind other work).
+    // The word arrives 8-11 us after the call where nothing else is queued: looked at for 50 us, then the stream
+    // is waited for (the kernel may be behind other work; that wait takes 12 us by itself.  A limit of 20000
+    // looks was about 10 us long: calls fell on either side of it, 11 or 23 us, with the code around the loop.)
     Py_BEGIN_ALLOW_THREADS
-    for (int spin = 0; spin < 20000 && !arrived; ++spin) {
-      got = *static_cast<volatile uint64_t*>(word);
-      arrived = got >> 32 == ticket;
-    }
+    const auto limit = std::chrono::steady_clock::now() + std::chrono::microseconds(50);
+    do {
+      for (int look = 0; look < 64 && !arrived; ++look) {
+        got = *static_cast<volatile uint64_t*>(word);
+        arrived = got >> 32 == ticket;
+      }
+    } while (!arrived && std::chrono::steady_clock::now() < limit);
     if (!arrived) {
       err = hipStreamSynchronize(stream);
       got = *static_cast<volatile uint64_t*>(word);
