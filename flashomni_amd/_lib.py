@@ -27,6 +27,7 @@ SIGNATURES = {
                          c_u32, c_u32, c_u32, c_int, c_u32, c_int, c_vp, c_vp], c_int),
     "fo_plan_batch": ([c_vp, c_vp, c_i32, c_i32, c_i32, c_int, c_vp], c_int),
     "fo_plan_tables": ([c_vp, c_vp, c_i32, c_i32, c_i32, c_int, c_vp, c_vp], c_int),
+    "fo_plan_tables_signal": ([c_vp, c_vp, c_i32, c_i32, c_i32, c_int, c_vp, c_vp, c_u32, c_vp], c_int),
     "fo_sparse_block_table": ([c_vp, c_u32, c_u32, c_vp, c_vp, c_i64, c_vp], c_int),
     "fo_decode_sizes": ([c_vp, c_vp, c_u32, c_u32, c_u32, c_u32, c_vp, c_vp, c_vp], c_int),
     "fo_decode_sparse": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 9 + [c_vp, c_vp], c_int),

@@ -61,16 +61,15 @@ class DecodedWorkList:
     def __init__(self, max_rows: int, max_nnz: int, num_heads: int, device):
         self.max_rows, self.max_nnz = max_rows, max_nnz
         n = max(max_rows, 1)
-        self.row_req = torch.empty(n, dtype=torch.int32, device=device)
-        self.row_qb = torch.empty(n, dtype=torch.int32, device=device)
-        self.row_head = torch.empty(n, dtype=torch.int32, device=device)
-        self.kv_row_ptr = torch.empty(n + 1, dtype=torch.int32, device=device)
-        self.kv_idx = torch.empty(max(max_nnz, 1), dtype=torch.int32, device=device)
-        self.counts = torch.zeros(4, dtype=torch.int32, device=device)
-        self.order = torch.empty(n, dtype=torch.int32, device=device)
-        self.sched = torch.zeros(1024, dtype=torch.int32, device=device)
-        self.shares = torch.zeros(512 + 8 * (n + 1), dtype=torch.int32, device=device)
-        self.scratch = torch.empty(2 * n + 8192, dtype=torch.int32, device=device)
+        # one allocation (a stream that uses the list holds one block, not ten); the ones to be cleared at the end
+        sizes = (n, n, n, n + 1, max(max_nnz, 1), n, 2 * n + 8192, 4, 1024, 512 + 8 * (n + 1))
+        starts = [0]
+        for size in sizes:
+            starts.append(starts[-1] + -(-size // 64) * 64)
+        self.base = torch.empty(starts[-1], dtype=torch.int32, device=device)
+        self.base[starts[7]:].zero_()
+        (self.row_req, self.row_qb, self.row_head, self.kv_row_ptr, self.kv_idx, self.order, self.scratch, self.counts,
+         self.sched, self.shares) = (self.base.narrow(0, a, size) for a, size in zip(starts, sizes))
         self.buffers = (self.row_req, self.row_qb, self.row_head, self.kv_row_ptr, self.kv_idx, self.counts, self.order,
                         self.sched, self.scratch, self.shares)
 
@@ -116,8 +115,8 @@ class PlannedBatch:
             qo_indptr_dev, kv_indptr_dev)
         (self.n_q_blk, self.n_kv_blk, self.max_rows, self.max_nnz, self.total_q_rows, self.total_kv_rows,
          self.min_info_bytes, self.min_kv_info_bytes, self.max_kv_len, *self._table_at) = sizes
-        self.qo_indptr = self.table(0) if qo_indptr_dev is None else qo_indptr_dev
-        self.kv_indptr = self.table(1) if kv_indptr_dev is None else kv_indptr_dev
+        self.qo_indptr = self._table(0) if qo_indptr_dev is None else qo_indptr_dev
+        self.kv_indptr = self._table(1) if kv_indptr_dev is None else kv_indptr_dev
         # buffers of an earlier plan are taken over where they are large enough; made when first needed
         # (a run that takes its rows straight from the symbols needs none)
         self._list = worklist
@@ -132,11 +131,17 @@ class PlannedBatch:
     def worklist(self) -> DecodedWorkList:
         if self._list is None:
             self._list = DecodedWorkList(self.max_rows, self.max_nnz, self.symbol_heads, self.device)
+        _lib.native().enter_plan(self.native, self._list.base)
         return self._list
 
     def table(self, i: int) -> torch.Tensor:
         """One of the device tables (order: see fo_batch_sizes): the indptrs of the q and kv tokens, of their
-        128-token blocks and of the symbol bits, then the request and q block of every symbol row."""
+        128-token blocks and of the symbol bits, then the request and q block of every symbol row.  Ordered
+        before the current stream's work."""
+        _lib.native().enter_plan(self.native, None)
+        return self._table(i)
+
+    def _table(self, i: int) -> torch.Tensor:
         return self.tables.narrow(0, self._table_at[(0, 1, 4, 5, 6, 7, 2, 3)[i]],
                                   self.batch_size + 1 if i < 6 else max(self.n_q_blk, 1))
 

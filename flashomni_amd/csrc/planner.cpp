@@ -46,7 +46,16 @@ struct TableArgs {
 };
 static_assert(sizeof(TableArgs) <= 4096, "kernel arguments");
 
-__global__ void __launch_bounds__(256) plan_tables_kernel(const TableArgs a, int32_t* __restrict__ out) {
+// `word` (pinned host memory, or null): receives ticket << 32 when everything queued so far is in memory
+__device__ __forceinline__ void signal_host(uint64_t* word, uint32_t ticket) {
+  __hip_atomic_store(word, static_cast<uint64_t>(ticket) << 32, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void plan_signal_kernel(uint64_t* word, uint32_t ticket) { signal_host(word, ticket); }
+
+// (word: launches of one workgroup only)
+__global__ void __launch_bounds__(256) plan_tables_kernel(const TableArgs a, int32_t* __restrict__ out, uint64_t* word,
+                                                          uint32_t ticket) {
   __shared__ int32_t s_rows[kMaxArgBatch + 1];  // first symbol row of every request
   const int tid = threadIdx.x;
   if (tid < 5) {  // five running sums, a lane each; lane 0's also stays in LDS
@@ -79,6 +88,10 @@ __global__ void __launch_bounds__(256) plan_tables_kernel(const TableArgs a, int
     }
     out[a.off[6] + i] = lo;
     out[a.off[7] + i] = i - s_rows[lo];
+  }
+  if (word != nullptr) {
+    __syncthreads();  // (the release of the word covers what the barrier ordered before it)
+    if (tid == 0) signal_host(word, ticket);
   }
 }
 
@@ -120,6 +133,11 @@ extern "C" int fo_plan_batch(const int32_t* qo, const int32_t* kv, int32_t batch
 
 extern "C" int fo_plan_tables(const int32_t* qo, const int32_t* kv, int32_t batch, int32_t num_qo, int32_t num_kv,
                               int packed, int32_t* tables, void* stream) {
+  return fo_plan_tables_signal(qo, kv, batch, num_qo, num_kv, packed, tables, nullptr, 0, stream);
+}
+
+extern "C" int fo_plan_tables_signal(const int32_t* qo, const int32_t* kv, int32_t batch, int32_t num_qo, int32_t num_kv,
+                                     int packed, int32_t* tables, uint64_t* word, uint32_t ticket, void* stream) {
   FO_REQUIRE(tables, "plan tables: null pointer");
   fo_batch_sizes z;
   if (int rc = fo_plan_batch(qo, kv, batch, num_qo, num_kv, packed, &z)) return rc;
@@ -137,8 +155,12 @@ extern "C" int fo_plan_tables(const int32_t* qo, const int32_t* kv, int32_t batc
     std::memcpy(a.indptr[0], qo, 4 * (batch + 1));
     std::memcpy(a.indptr[1], kv, 4 * (batch + 1));
     const int64_t grid = std::min<int64_t>(64, std::max<int64_t>(1, z.n_q_blocks / 1024));
-    plan_tables_kernel<<<static_cast<unsigned>(grid), 256, 0, s>>>(a, tables);
+    plan_tables_kernel<<<static_cast<unsigned>(grid), 256, 0, s>>>(a, tables, grid == 1 ? word : nullptr, ticket);
     FO_CHECK_LAUNCH();
+    if (word != nullptr && grid > 1) {
+      plan_signal_kernel<<<1, 1, 0, s>>>(word, ticket);
+      FO_CHECK_LAUNCH();
+    }
     return FO_OK;
   }
   std::vector<int32_t> h(z.table_ints);
@@ -158,6 +180,7 @@ extern "C" int fo_plan_tables(const int32_t* qo, const int32_t* kv, int32_t batc
   }
   FO_HIP_CALL(hipMemcpyAsync(tables, h.data(), 4 * h.size(), hipMemcpyHostToDevice, s));
   FO_HIP_CALL(hipStreamSynchronize(s));
+  if (word != nullptr) __atomic_store_n(word, static_cast<uint64_t>(ticket) << 32, __ATOMIC_RELEASE);
   return FO_OK;
 }
 

@@ -103,6 +103,13 @@ int fo_plan_batch(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, 
                   int32_t num_qo_heads, int32_t num_kv_heads, int packed, void* sizes);
 int fo_plan_tables(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, int32_t batch_size,
                    int32_t num_qo_heads, int32_t num_kv_heads, int packed, int32_t* tables, void* stream);
+/* The same; `word` (8 bytes of pinned host memory, or null) receives ticket << 32 when the tables and whatever
+ * the stream held before them are complete and visible to the whole device.  (An event behind the launch costs
+ * 3 us of a small batch that is planned anew for each call, and cannot be asked for while its stream is being
+ * captured.) */
+int fo_plan_tables_signal(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, int32_t batch_size,
+                          int32_t num_qo_heads, int32_t num_kv_heads, int packed, int32_t* tables, uint64_t* word,
+                          uint32_t ticket, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Sparse-symbol decoder: packed symbols -> compacted, canonically ordered work list.

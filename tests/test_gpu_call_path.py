@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import oracle
+from helpers import make_ragged_masks, max_abs, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +45,94 @@ def test_plan_tables(dev, batch, packed):
            np.concatenate([np.arange(r) for r in rows])]
     for i, e in enumerate(exp):
         np.testing.assert_array_equal(w._planned.table(i).cpu().numpy(), e, err_msg=str(i))
+
+
+def _small_problem(dev, lens, heads, seed):
+    m = make_ragged_masks(lens, lens, heads, 0.7, 0.6, seed=seed)
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(sum(lens), heads, 128, generator=g).to(torch.bfloat16) for _ in range(3))
+    sym = [torch.from_numpy(m[n]) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    exp = oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=torch.zeros_like(q))
+    return m, [t.to(dev) for t in (q, k, v)], [t.to(dev) for t in sym], exp
+
+
+@pytest.mark.parametrize("lens,heads", [([384, 130], 2), ([4500], 40)])     # rows from the symbols, a decoded list
+@pytest.mark.parametrize("plan_on_side,how", [(True, "eager"), (False, "eager"), (True, "captured"), (False, "captured"),
+                                              (True, "captured on the planning stream")])
+def test_plan_and_run_on_two_streams(dev, lens, heads, plan_on_side, how):
+    """The tables of a plan are complete when another stream reads them, although plan() does not wait: the
+    planning stream is busy when plan() queues them (the memory they land in held other values).  A captured run
+    may be replayed on any stream: the tables are complete before it is recorded."""
+    import flashomni_amd as fo
+    m, qkv, sym, exp = _small_problem(dev, lens, heads, 8)
+    qo, kv = torch.from_numpy(m["qo_indptr"]), torch.from_numpy(m["kv_indptr"])
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(qo, kv, heads, heads, 128, q_data_type=torch.bfloat16)
+    w.run(*qkv, *sym)          # (the kernels are loaded before the clock matters)
+    side, third = torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)
+    planner, runner = (side, torch.cuda.current_stream()) if plan_on_side else (torch.cuda.current_stream(), side)
+    out = torch.zeros(qkv[0].shape, dtype=torch.bfloat16, device=dev)
+    torch.cuda.synchronize(dev)
+    with torch.cuda.stream(planner):
+        busy = torch.empty(1 << 30, dtype=torch.uint8, device=dev)
+        for i in range(20):
+            busy.fill_(i)
+        w.plan(qo, kv, heads, heads, 128, q_data_type=torch.bfloat16)
+    if how == "captured on the planning stream":
+        third = side
+    if how == "eager":
+        with torch.cuda.stream(runner):
+            w.run(*qkv, *sym, out=out)
+        runner.synchronize()
+    else:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(third):
+            graph.capture_begin()
+            w.run(*qkv, *sym, out=out)
+            graph.capture_end()
+        with torch.cuda.stream(runner):
+            graph.replay()
+        runner.synchronize()
+    got = out.cpu()
+    assert max_abs(got, exp) <= 2e-2 and rel_l2(got, exp) <= 1e-2
+    torch.cuda.synchronize(dev)
+
+
+def test_plan_tables_outlive_the_plan_on_another_stream(dev):
+    """Planned on the current stream, run on a busy side stream, planned again: the memory of the first plan's
+    tables is not handed out before the side stream's launch has read them."""
+    import flashomni_amd as fo
+    m, qkv, sym, exp = _small_problem(dev, [384, 130], 2, 9)
+    qo, kv = torch.from_numpy(m["qo_indptr"]), torch.from_numpy(m["kv_indptr"])
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(qo, kv, 2, 2, 128, q_data_type=torch.bfloat16)
+    side = torch.cuda.Stream(device=dev)
+    out = torch.zeros(qkv[0].shape, dtype=torch.bfloat16, device=dev)
+    torch.cuda.synchronize(dev)
+    with torch.cuda.stream(side):
+        busy = torch.empty(1 << 30, dtype=torch.uint8, device=dev)
+        for i in range(20):
+            busy.fill_(i)
+        w.run(*qkv, *sym, out=out)
+    at, ints = w._planned.tables.data_ptr(), w._planned.tables.numel()
+    w._planned = None
+    again = [torch.empty(ints, dtype=torch.int32, device=dev) for _ in range(64)]
+    assert all(t.data_ptr() != at for t in again)
+    del again
+    side.synchronize()
+    assert max_abs(out.cpu(), exp) <= 2e-2
+
+
+def test_plan_is_refused_under_capture(dev):
+    import flashomni_amd as fo
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    ip = torch.tensor([0, 384], dtype=torch.int32)
+    graph, s = torch.cuda.CUDAGraph(), torch.cuda.Stream(device=dev)
+    torch.cuda.synchronize(dev)
+    with torch.cuda.stream(s):
+        graph.capture_begin()
+        with pytest.raises(RuntimeError, match="cannot be captured"):
+            w.plan(ip, ip, 2, 2, 128, q_data_type=torch.bfloat16)
+        torch.zeros(8, device=dev)
+        graph.capture_end()
+    w.plan(ip, ip, 2, 2, 128, q_data_type=torch.bfloat16)
