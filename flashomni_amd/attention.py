@@ -226,9 +226,7 @@ class PlannedBatch:
         """The work list of the last run or decode.  A run that took its rows straight from the symbols
         has kept a copy of them: decoded here, on the current stream, behind that run."""
         if self.native.state:
-            cur = torch.cuda.current_stream(self.device)
-            if self.native.stream != cur.cuda_stream and not torch.cuda.is_current_stream_capturing():
-                cur.wait_stream(torch.cuda.ExternalStream(self.native.stream, device=self.device))
+            _lib.native().follow_run(self.native)
             full = self.native.state == 2
             info, kv_info, info_ip, kv_ip = (None,) * 4 if full else _lib.native().kept_symbols(self.native)
             self.decode(info, kv_info, info_ip, kv_ip, full)

@@ -524,6 +524,34 @@ PyObject* host_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_END
 }
 
+// (Plan): the current stream waits for the stream of the last run (by its handle: torch has no stream object for
+// the default stream's, 0, but hands out one of its pool).  Under capture nothing is waited for: a replay is
+// ordered by whoever makes it.
+PyObject* follow_run(PyObject*, PyObject* arg) {
+  TORCH_GUARD_BEGIN
+  if (Py_TYPE(arg) != g_plan_type) {
+    PyErr_SetString(PyExc_RuntimeError, "not a plan");
+    return nullptr;
+  }
+  Plan* p = reinterpret_cast<Plan*>(arg);
+  const hipStream_t cur = static_cast<hipStream_t>(stream_of(p->dev)), ran = reinterpret_cast<hipStream_t>(p->stream);
+  if (cur == ran || capturing(cur)) Py_RETURN_NONE;
+  if (capturing(ran)) {
+    PyErr_SetString(PyExc_RuntimeError, "the stream of the last run() is being captured: its list cannot be reused on another");
+    return nullptr;
+  }
+  hipEvent_t ev;
+  hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+  if (e != hipSuccess) return raise_hip(e);
+  e = hipEventRecord(ev, ran);
+  if (e == hipSuccess) e = hipStreamWaitEvent(cur, ev, 0);
+  const hipError_t destroyed = hipEventDestroy(ev);  // (what was queued stays)
+  if (e == hipSuccess) e = destroyed;
+  if (e != hipSuccess) return raise_hip(e);
+  Py_RETURN_NONE;
+  TORCH_GUARD_END
+}
+
 // (Plan) -> (sparse_info, sparse_kv_info, the two indptrs) as the last run read them (state 1)
 PyObject* kept_symbols(PyObject*, PyObject* arg) {
   TORCH_GUARD_BEGIN
@@ -802,6 +830,7 @@ PyMethodDef g_methods[] = {
     {"host_plan", FASTCALL(host_plan), nullptr},
     {"attention", FASTCALL(attention), nullptr},
     {"enter_plan", FASTCALL(enter_plan), nullptr},
+    {"follow_run", follow_run, METH_O, nullptr},
     {"kept_symbols", kept_symbols, METH_O, nullptr},
     {"packbits", FASTCALL(packbits), nullptr},
     {"segment_packbits", FASTCALL(segment_packbits), nullptr},

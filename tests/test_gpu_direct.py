@@ -105,3 +105,37 @@ def test_fresh_output_of_decoded_lists(dev, case, layout):
         junk = torch.full((256 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
         del junk
         assert torch.equal(w.run(q, k, v, *sym), exp)
+
+
+@pytest.mark.parametrize("run_on_default", [True, False])
+def test_list_of_a_run_reused_on_another_stream(dev, run_on_default):
+    """A run that took its rows from the symbols is still to come on its (busy) stream when another stream
+    reuses its list: the reuse waits for that run, and does not decode what an earlier run left."""
+    import flashomni_amd as fo
+    heads, lens = 2, [384, 130]
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(sum(lens), heads, 128, generator=g).to(torch.bfloat16) for _ in range(3))
+    masks = [make_ragged_masks(lens, lens, heads, 0.7, 0.6, seed=s) for s in (50, 51)]
+    names = ("packed_info", "packed_keep", "info_indptr", "keep_indptr")
+    syms = [[torch.from_numpy(m[n]).to(dev) for n in names] for m in masks]
+    m = masks[1]
+    exp = oracle.sparse_attention(q, k, v, *(m[n] for n in names), m["qo_indptr"], m["kv_indptr"], out=torch.zeros_like(q))
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(torch.from_numpy(m["qo_indptr"]), torch.from_numpy(m["kv_indptr"]), heads, heads, 128, q_data_type=torch.bfloat16)
+    w.run(qd, kd, vd, *syms[0])
+    w.run(qd, kd, vd, *syms[0], reuse_decoded=True)    # (the list exists, and is the other symbols')
+    default, side = torch.cuda.current_stream(dev), torch.cuda.Stream(device=dev)
+    first, second = (default, side) if run_on_default else (side, default)
+    out, again = torch.zeros_like(qd), torch.zeros_like(qd)
+    torch.cuda.synchronize(dev)
+    with torch.cuda.stream(first):
+        busy = torch.empty(1 << 30, dtype=torch.uint8, device=dev)
+        for i in range(20):
+            busy.fill_(i)
+        w.run(qd, kd, vd, *syms[1], out=out)
+    with torch.cuda.stream(second):
+        w.run(qd, kd, vd, *syms[1], out=again, reuse_decoded=True)
+    torch.cuda.synchronize(dev)
+    for got in (out.cpu(), again.cpu()):
+        assert max_abs(got, exp) <= 2e-2 and rel_l2(got, exp) <= 1e-2
