@@ -267,6 +267,10 @@ bool wait_word(const Word& w) {
   return ok;
 }
 
+// kv tokens of a request whose rows the kernel without a decoded list can hold (4096 blocks; the decoder takes
+// longer requests)
+constexpr int64_t kMaxListed = 4096 * 128;
+
 hipError_t host_wait(hipEvent_t event) {
   hipError_t e;
   Py_BEGIN_ALLOW_THREADS
@@ -277,7 +281,7 @@ hipError_t host_wait(hipEvent_t event) {
 
 struct Plan {
   PyObject_HEAD
-  Tensor tables, keep;
+  Tensor tables;
   // plan() queues the tables on the stream that is current there, `home`, and does not wait.  Another stream
   // waits for `behind`, an event recorded on `home` when one first asks.  A stream that is being captured by then
   // takes no such event; the host can still see `word`, which the launch writes.  The default stream cannot be
@@ -293,10 +297,13 @@ struct Plan {
   int dev, batch, num_qo, num_kv, symbol_heads, packed;
   bool from_zero;  // the first request begins at token 0
   // What the last run left behind.  state 0: the list that the Python side decoded; 1: rows taken straight
-  // from the symbols, of which `keep` holds a copy (info at 0, kv_info at keep_at[0], the indptrs at
-  // keep_at[1], in bytes); 2: every row (is_full).  stream: where it ran.
+  // from the symbols, of which a copy is kept; 2: every row (is_full).  stream: where it ran.
   int state;
-  long long stream, keep_at[2], keep_bytes[2];
+  long long stream;
+  // The copy lies behind the tables, in one place for as long as the plan lives (a graph writes it at every
+  // replay): room for the symbols that such a run takes, at keep_at[0] info, [1] kv_info, [2] the indptrs (bytes
+  // from the start of the tables; keep_at[0] = 0: a batch that is always decoded).
+  int64_t keep_at[3], keep_room[2];
   fo_batch_sizes z;
 };
 
@@ -308,7 +315,6 @@ void plan_dealloc(PyObject* self) {
   give_word(p->word);
   p->used.~vector();
   p->tables.~Tensor();
-  p->keep.~Tensor();
   p->qo_keep.~Tensor();
   p->kv_keep.~Tensor();
   PyTypeObject* t = Py_TYPE(self);
@@ -417,7 +423,6 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!self) return nullptr;
   Plan* p = reinterpret_cast<Plan*>(self);
   new (&p->tables) Tensor();
-  new (&p->keep) Tensor();
   new (&p->used) std::vector<hipStream_t>();
   new (&p->qo_keep) Tensor();
   new (&p->kv_keep) Tensor();
@@ -431,8 +436,19 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   p->from_zero = qo->data_ptr<int32_t>()[0] == 0;
   p->state = 0;
   int rc = 0;
+  int64_t ints = z.table_ints;
+  if (z.max_rows > 0 && z.max_rows < fo_decode_sparse_clear_min_pairs() && z.max_nnz <= (1 << 20) && z.max_kv_len <= kMaxListed) {
+    auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+    // (symbol tensors much larger than the batch needs are not worth copying)
+    p->keep_room[0] = z.min_info + 4096;
+    p->keep_room[1] = z.min_kv_info + 4096;
+    p->keep_at[0] = up(4 * ints);
+    p->keep_at[1] = p->keep_at[0] + up(p->keep_room[0]);
+    p->keep_at[2] = p->keep_at[1] + up(p->keep_room[1]);
+    ints = p->keep_at[2] / 4 + 2 * (batch + 1);
+  }
   try {
-    p->tables = new_tensor({z.table_ints}, at::kInt, dev);
+    p->tables = new_tensor({ints}, at::kInt, dev);
     p->home = home;
     if (home && !take_word(&p->word)) {
       Py_DECREF(self);
@@ -560,11 +576,11 @@ PyObject* kept_symbols(PyObject*, PyObject* arg) {
     return nullptr;
   }
   Plan* p = reinterpret_cast<Plan*>(arg);
-  const int64_t n = p->batch + 1;
-  Tensor ip = p->keep.narrow(0, p->keep_at[1], 8 * n).view(at::kInt);
-  return Py_BuildValue("(NNNN)", THPVariable_Wrap(p->keep.narrow(0, 0, p->keep_bytes[0])),
-                       THPVariable_Wrap(p->keep.narrow(0, p->keep_at[0], p->keep_bytes[1])),
-                       THPVariable_Wrap(ip.narrow(0, 0, n)), THPVariable_Wrap(ip.narrow(0, n, n)));
+  const int64_t n = p->batch + 1, ip = p->keep_at[2] / 4;
+  const Tensor bytes = p->tables.view(at::kByte);
+  return Py_BuildValue("(NNNN)", THPVariable_Wrap(bytes.narrow(0, p->keep_at[0], p->keep_room[0])),
+                       THPVariable_Wrap(bytes.narrow(0, p->keep_at[1], p->keep_room[1])),
+                       THPVariable_Wrap(p->tables.narrow(0, ip, n)), THPVariable_Wrap(p->tables.narrow(0, ip + n, n)));
   TORCH_GUARD_END
 }
 
@@ -652,12 +668,9 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor fresh;
   // the launch without a decoded list (it clears what it skips: every row of a fresh output is its own)
   const bool own = !out && p->from_zero && q->size(0) == p->z.total_q;
-  // (symbol tensors much larger than the batch needs are not worth copying)
-  // (nor is a request served whose rows may list more kv blocks than the kernel has room for, 4096: the decoded
-  // forms take whole rows of it up to that many)
-  const bool small = p->z.max_kv_len <= 4096 * 128 && (full || (sym[0]->numel() <= p->z.min_info + 4096 && sym[1]->numel() <= p->z.min_kv_info + 4096));
+  const bool small = p->keep_at[0] && (full || (sym[0]->numel() <= p->keep_room[0] && sym[1]->numel() <= p->keep_room[1]));
   int rc = FO_NOT_DIRECT;
-  if (small && p->z.max_rows > 0 && fo_sparse_attention_direct_serves(&a)) {
+  if (small && fo_sparse_attention_direct_serves(&a)) {
     if (!out) fresh = own ? at::empty(q->sizes(), q->options()) : at::zeros(q->sizes(), q->options());
     const Tensor& o = out ? *out : fresh;
     a.o = o.data_ptr();
@@ -665,19 +678,11 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     a.o_stride_h = o.stride(1);
     a.zero_skipped = own;
     if (!full) {
-      auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
-      p->keep_bytes[0] = sym[0]->numel();
-      p->keep_bytes[1] = sym[1]->numel();
-      p->keep_at[0] = up(p->keep_bytes[0]);
-      p->keep_at[1] = p->keep_at[0] + up(p->keep_bytes[1]);
-      const int64_t need = p->keep_at[1] + 8 * (p->batch + 1);
-      if (!p->keep.defined() || p->keep.numel() < need) p->keep = new_tensor({need}, at::kByte, dev);
-      uint8_t* kept = p->keep.data_ptr<uint8_t>();
-      a.keep_info = kept;
-      a.keep_kv_info = kept + p->keep_at[0];
-      a.keep_indptr = reinterpret_cast<int32_t*>(kept + p->keep_at[1]);
-      a.info_bytes = p->keep_bytes[0];
-      a.kv_info_bytes = p->keep_bytes[1];
+      a.keep_info = reinterpret_cast<uint8_t*>(t) + p->keep_at[0];
+      a.keep_kv_info = reinterpret_cast<uint8_t*>(t) + p->keep_at[1];
+      a.keep_indptr = t + p->keep_at[2] / 4;
+      a.info_bytes = sym[0]->numel();
+      a.kv_info_bytes = sym[1]->numel();
     }
     rc = fo_sparse_attention_direct(&a);
     if (rc < 0) return raise_last();

@@ -171,3 +171,37 @@ def test_graph_captured_on_a_warm_stream_survives_workspace_growth(dev):
         torch.cuda.synchronize()
         assert torch.equal(out, ref), "replay %d differs from the eager call" % replay
         assert all(bool((j == 0x5a).all()) for j in junk), "a replay wrote outside its own scratch"
+
+
+def test_captured_short_run_keeps_its_symbols_in_place(dev):
+    """A run that takes its rows straight from the symbols keeps a copy of them for a later reuse.  A graph writes
+    that copy at every replay: eager runs with larger symbol tensors in between must not move it, and what the
+    replays write is what a reuse then decodes."""
+    import flashomni_amd as fo
+    heads, lens = 2, [384, 130]
+    n = sum(lens)
+    g = torch.Generator(device=dev).manual_seed(21)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    m = make_ragged_masks(lens, lens, heads, 0.7, 0.6, seed=21)
+    t = lambda name: torch.from_numpy(m[name]).to(dev)
+    sym = [t(s) for s in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    indptr = torch.from_numpy(m["qo_indptr"])
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(indptr, indptr, heads, heads, 128, q_data_type=torch.bfloat16)
+    exp = w.run(q, k, v, *sym, out=torch.zeros_like(q))
+    out = torch.zeros_like(q)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        w.run(q, k, v, *sym, out=out)
+    longer = [torch.cat([s, torch.full((3000,), 0xff, dtype=torch.uint8, device=dev)]) for s in sym[:2]] + sym[2:]
+    assert torch.equal(w.run(q, k, v, *longer, out=torch.zeros_like(q)), exp)
+    junk = [torch.full((1 << s,), 0x5a, dtype=torch.uint8, device=dev) for s in range(9, 15) for _ in range(32)]
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, exp)
+        assert all(bool((j == 0x5a).all()) for j in junk), "a replay wrote outside its own buffers"
+    listed = w.run(q, k, v, *sym, out=torch.zeros_like(q), reuse_decoded=True)
+    assert float((listed.float() - exp.float()).abs().max()) <= 8e-3
