@@ -31,6 +31,7 @@ SIGNATURES = {
     "fo_sparse_block_table": ([c_vp, c_u32, c_u32, c_vp, c_vp, c_i64, c_vp], c_int),
     "fo_decode_sizes": ([c_vp, c_vp, c_u32, c_u32, c_u32, c_u32, c_vp, c_vp, c_vp], c_int),
     "fo_decode_sparse": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 9 + [c_vp, c_vp], c_int),
+    "fo_decode_sparse_kept": ([c_vp] * 7 + [c_i32, c_i32, c_i32] + [c_vp] * 9 + [c_vp, c_vp], c_int),
     "fo_decode_sparse_clear_min_pairs": ([], c_i32),
     "fo_decode_sparse_clear": ([c_vp] * 7 + [c_i32, c_i32, c_i32, c_int] + [c_vp] * 9 + [c_vp, c_vp, c_i64, c_i64, c_vp, c_i32, c_vp],
                                c_int),

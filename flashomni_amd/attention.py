@@ -58,18 +58,24 @@ class DecodedWorkList:
     entry or, when there are only a few rows per CU, the table of even shares used instead.  The sizes live on the device;
     ``sizes()`` copies them back (one synchronisation) for tests and reports."""
 
-    def __init__(self, max_rows: int, max_nnz: int, num_heads: int, device):
+    def __init__(self, max_rows: int, max_nnz: int, num_heads: int, device, sched):
         self.max_rows, self.max_nnz = max_rows, max_nnz
         n = max(max_rows, 1)
-        # one allocation (a stream that uses the list holds one block, not ten); the ones to be cleared at the end
-        sizes = (n, n, n, n + 1, max(max_nnz, 1), n, 2 * n + 8192, 4, 1024, 512 + 8 * (n + 1))
+        # One allocation: a stream that uses the list holds one block.  Nothing has to be cleared (every decode
+        # writes what a launch reads), nor may it be where a graph is being recorded: the graph would clear it at
+        # every replay.
+        sizes = (n, n, n, n + 1, max(max_nnz, 1), 4, n, 2 * n + 8192, 512 + 8 * (n + 1))
         starts = [0]
         for size in sizes:
             starts.append(starts[-1] + -(-size // 64) * 64)
         self.base = torch.empty(starts[-1], dtype=torch.int32, device=device)
-        self.base[starts[7]:].zero_()
-        (self.row_req, self.row_qb, self.row_head, self.kv_row_ptr, self.kv_idx, self.order, self.scratch, self.counts,
-         self.sched, self.shares) = (self.base.narrow(0, a, size) for a, size in zip(starts, sizes))
+        (self.row_req, self.row_qb, self.row_head, self.kv_row_ptr, self.kv_idx, self.counts, self.order, self.scratch,
+         self.shares) = (self.base.narrow(0, a, size) for a, size in zip(starts, sizes))
+        self.use_sched(sched)
+
+    def use_sched(self, sched):
+        """The queue words belong to a plan (it clears them once, and its launches without a list share them)."""
+        self.sched = sched
         self.buffers = (self.row_req, self.row_qb, self.row_head, self.kv_row_ptr, self.kv_idx, self.counts, self.order,
                         self.sched, self.scratch, self.shares)
 
@@ -122,6 +128,8 @@ class PlannedBatch:
         self._list = worklist
         if worklist is not None and (worklist.max_rows < self.max_rows or worklist.max_nnz < self.max_nnz):
             self._list = None
+        if self._list is not None:
+            self._list.use_sched(self._sched())
         self.share_rows = share_rows
         self.split_ok = self._split_ws_ok()
         # [is_full, stream, streams already ordered after it] of the list the work-list buffers hold
@@ -130,7 +138,7 @@ class PlannedBatch:
     @property
     def worklist(self) -> DecodedWorkList:
         if self._list is None:
-            self._list = DecodedWorkList(self.max_rows, self.max_nnz, self.symbol_heads, self.device)
+            self._list = DecodedWorkList(self.max_rows, self.max_nnz, self.symbol_heads, self.device, self._sched())
         _lib.native().enter_plan(self.native, self._list.base)
         return self._list
 
@@ -140,6 +148,9 @@ class PlannedBatch:
         before the current stream's work."""
         _lib.native().enter_plan(self.native, None)
         return self._table(i)
+
+    def _sched(self) -> torch.Tensor:
+        return self.tables.narrow(0, self.native.sched_at, 1024)
 
     def _table(self, i: int) -> torch.Tensor:
         return self.tables.narrow(0, self._table_at[(0, 1, 4, 5, 6, 7, 2, 3)[i]],
@@ -197,11 +208,16 @@ class PlannedBatch:
                 _lib.ptr(wl.kv_idx), _lib.ptr(wl.counts), _lib.ptr(wl.order), _lib.ptr(wl.sched),
                 _lib.ptr(wl.scratch), _lib.ptr(wl.shares if self.split_ok else None),
                 stream.cuda_stream))
-        # remembered for reuse_decoded: which stream the list was decoded on (a run on another
-        # stream must be ordered after it)
-        self.decoded = (bool(is_full), stream, [])
-        self.native.state = 0
+        self._note_list(is_full)
         return wl
+
+    def _note_list(self, is_full):
+        """A list has been decoded on the current stream."""
+        _lib.native().note_list(self.native, is_full)
+        if not torch.cuda.is_current_stream_capturing():
+            # remembered for reuse_decoded: which stream the list was decoded on (a run on another stream must be
+            # ordered after it)
+            self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
 
     def attention(self, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full,
                   out, lse, return_lse, sm_scale, logits_soft_cap, hnd, qo_indptr=None, kv_indptr=None):
@@ -218,28 +234,52 @@ class PlannedBatch:
                 qo_indptr, kv_indptr)
             if r is False:
                 wl = self.worklist
-        if r is not None and self.native.state == 0:
+        if r is not None and self.native.state == 0 and not torch.cuda.is_current_stream_capturing():
             self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
         return r
 
     def listed(self) -> DecodedWorkList:
-        """The work list of the last run or decode.  A run that took its rows straight from the symbols
-        has kept a copy of them: decoded here, on the current stream, behind that run."""
-        if self.native.state:
-            _lib.native().follow_run(self.native)
-            full = self.native.state == 2
-            info, kv_info, info_ip, kv_ip = (None,) * 4 if full else _lib.native().kept_symbols(self.native)
-            self.decode(info, kv_info, info_ip, kv_ip, full)
+        """The work list of the last run or decode, ordered before the current stream's work.  A run that took
+        its rows straight from the symbols has kept a copy of them: decoded here, behind that run.  Where graphs
+        hold launches of this plan the device decides whether there is something to decode."""
+        native = _lib.native()
+        source, _ = native.list_source(self.native)
+        if source:
+            full = self._was_full()
+            if self.decoded is not None:
+                self._follow_list()
+            if self.native.state:
+                native.follow_run(self.native)
+            info, kv_info, info_ip, kv_ip = native.kept_symbols(self.native)
+            if source == 1:
+                self.decode(info, kv_info, info_ip, kv_ip, full)
+            else:
+                wl = self.worklist
+                with _lib.device_guard(self.device):
+                    _lib.check(_lib.lib().fo_decode_sparse_kept(
+                        _lib.ptr(info), _lib.ptr(kv_info), _lib.ptr(info_ip), _lib.ptr(kv_ip), _lib.ptr(self.blk_req),
+                        _lib.ptr(self.blk_qb), _lib.ptr(self.kv_indptr), self.n_q_blk, self.symbol_heads, self.block_kv,
+                        _lib.ptr(wl.row_req), _lib.ptr(wl.row_qb), _lib.ptr(wl.row_head), _lib.ptr(wl.kv_row_ptr),
+                        _lib.ptr(wl.kv_idx), _lib.ptr(wl.counts), _lib.ptr(wl.order), _lib.ptr(wl.sched),
+                        _lib.ptr(wl.scratch), _lib.ptr(wl.shares if self.split_ok else None),
+                        _lib.current_stream(self.device)))
+                self._note_list(full)
+        elif self.decoded is not None:
+            self._follow_list()
         return self.worklist
 
-    def reuse_decoded(self, is_full: bool) -> DecodedWorkList:
-        """The work list of the last decode, ordered before the current stream's work."""
-        self.listed()
-        if self.decoded is None:
-            raise RuntimeError("reuse_decoded=True needs an earlier decode() or run() after plan()")
-        was_full, stream, ordered = self.decoded
-        if was_full != bool(is_full):
-            raise RuntimeError("reuse_decoded=True: the last decode was made with is_full=%s" % was_full)
+    def _was_full(self):
+        """is_full of what the current list stands for, as far as the host knows; None: there is none."""
+        _, capture = _lib.native().list_source(self.native)
+        if self.native.recorded_in and (capture == self.native.recorded_in
+                                        or (self.decoded is None and not self.native.state)):
+            return bool(self.native.recorded_full)
+        if self.native.state:
+            return self.native.state == 2
+        return None if self.decoded is None else self.decoded[0]
+
+    def _follow_list(self):
+        _, stream, ordered = self.decoded
         cur = torch.cuda.current_stream(self.device)
         # one wait per (decode, stream): later work on a stream that has waited is behind the decode
         # already, and a wait in front of every launch costs each one 2-3 us
@@ -248,7 +288,15 @@ class PlannedBatch:
             ev.record(stream)
             cur.wait_event(ev)
             ordered.append(cur)
-        return self.worklist
+
+    def reuse_decoded(self, is_full: bool) -> DecodedWorkList:
+        """The work list of the last decode, ordered before the current stream's work."""
+        was_full = self._was_full()
+        if was_full is None:
+            raise RuntimeError("reuse_decoded=True needs an earlier decode() or run() after plan()")
+        if was_full != bool(is_full):
+            raise RuntimeError("reuse_decoded=True: the last decode was made with is_full=%s" % was_full)
+        return self.listed()
 
     def launch(self, q, k, v, out, lse, kv_layout, sm_scale, q_scale=None, k_scale=None, q_lo=None,
                k_lo=None, logits_soft_cap=0.0) -> None:
@@ -406,6 +454,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
             self._planned.split_ok = self._planned._split_ws_ok()
             self._planned.decoded = None
             self._planned.native.state = 0
+            self._planned.native.recorded_in = 0
 
     # ------------------------------------------------------------------------------------------
     def plan(

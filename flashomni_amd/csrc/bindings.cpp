@@ -296,10 +296,16 @@ struct Plan {
   Tensor qo_keep, kv_keep;
   int dev, batch, num_qo, num_kv, symbol_heads, packed;
   bool from_zero;  // the first request begins at token 0
-  // What the last run left behind.  state 0: the list that the Python side decoded; 1: rows taken straight
-  // from the symbols, of which a copy is kept; 2: every row (is_full).  stream: where it ran.
+  // What the last run (not: recorded in a graph) left behind.  state 0: the list that the Python side decoded; 1:
+  // rows taken straight from the symbols, of which a copy is kept; 2: every row (is_full).  stream: where it ran.
   int state;
   long long stream;
+  // Launches of the plan's that a graph holds run at times the host does not know: once there are any
+  // (`captured`), whether the list or the kept symbols are newer is read on the device (sched[33]).
+  // listed_in: the capture whose last launch on this plan was a decode; recorded_in, recorded_full: the last
+  // capture that recorded a decode or run, and its is_full.
+  int captured, recorded_full;
+  unsigned long long listed_in, recorded_in;
   // The copy lies behind the tables, in one place for as long as the plan lives (a graph writes it at every
   // replay): room for the symbols that such a run takes, at keep_at[0] info, [1] kv_info, [2] the indptrs (bytes
   // from the start of the tables; keep_at[0] = 0: a batch that is always decoded).
@@ -327,6 +333,27 @@ bool capturing(hipStream_t stream) {
   if (!stream) return false;
   hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
+// the capture that the stream is in, 0: none
+unsigned long long capture_of(hipStream_t stream) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (!stream || hipStreamGetCaptureInfo(stream, &s, &id) != hipSuccess || s == hipStreamCaptureStatusNone) return 0;
+  return id ? id : ~0ull;
+}
+
+// A launch that leaves a list (state 0) or takes rows without one (1, 2) has been queued on the stream.
+void note(Plan* p, hipStream_t stream, int state, bool full) {
+  if (const unsigned long long id = capture_of(stream)) {
+    p->captured = 1;
+    p->recorded_in = id;
+    p->recorded_full = full;
+    p->listed_in = state == 0 ? id : 0;
+  } else {
+    p->state = state;
+    p->stream = reinterpret_cast<long long>(stream);
+  }
 }
 
 PyObject* raise_captured_plan() {
@@ -568,10 +595,39 @@ PyObject* follow_run(PyObject*, PyObject* arg) {
   TORCH_GUARD_END
 }
 
-// (Plan) -> (sparse_info, sparse_kv_info, the two indptrs) as the last run read them (state 1)
+// (Plan, is_full): a list has been decoded on the current stream
+PyObject* note_list(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  if (n != 2 || Py_TYPE(args[0]) != g_plan_type) {
+    PyErr_SetString(PyExc_RuntimeError, "note_list: bad argument");
+    return nullptr;
+  }
+  Plan* p = reinterpret_cast<Plan*>(args[0]);
+  note(p, static_cast<hipStream_t>(stream_of(p->dev)), 0, truth(args[1]));
+  Py_RETURN_NONE;
+  TORCH_GUARD_END
+}
+
+// (Plan) -> how a reuse on the current stream gets its list: 0: as it is; 1: decoded from what the last run left
+// behind; 2: the device decides between the two (fo_decode_sparse_kept).  And the capture the stream is in.
+PyObject* list_source(PyObject*, PyObject* arg) {
+  TORCH_GUARD_BEGIN
+  if (Py_TYPE(arg) != g_plan_type) {
+    PyErr_SetString(PyExc_RuntimeError, "not a plan");
+    return nullptr;
+  }
+  Plan* p = reinterpret_cast<Plan*>(arg);
+  const unsigned long long id = capture_of(static_cast<hipStream_t>(stream_of(p->dev)));
+  if (id) p->captured = 1;
+  const int source = !p->keep_at[0] || (id && p->listed_in == id) ? 0 : p->captured ? 2 : p->state != 0;
+  return Py_BuildValue("(iK)", source, id);
+  TORCH_GUARD_END
+}
+
+// (Plan) -> room for (sparse_info, sparse_kv_info, the two indptrs) as the last run without a list read them
 PyObject* kept_symbols(PyObject*, PyObject* arg) {
   TORCH_GUARD_BEGIN
-  if (Py_TYPE(arg) != g_plan_type || reinterpret_cast<Plan*>(arg)->state != 1) {
+  if (Py_TYPE(arg) != g_plan_type || !reinterpret_cast<Plan*>(arg)->keep_at[0]) {
     PyErr_SetString(PyExc_RuntimeError, "no symbols kept");
     return nullptr;
   }
@@ -680,16 +736,13 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!full) {
       a.keep_info = reinterpret_cast<uint8_t*>(t) + p->keep_at[0];
       a.keep_kv_info = reinterpret_cast<uint8_t*>(t) + p->keep_at[1];
-      a.keep_indptr = t + p->keep_at[2] / 4;
       a.info_bytes = sym[0]->numel();
       a.kv_info_bytes = sym[1]->numel();
     }
+    a.keep_indptr = t + p->keep_at[2] / 4;
     rc = fo_sparse_attention_direct(&a);
     if (rc < 0) return raise_last();
-    if (rc == FO_OK) {
-      p->state = full ? 2 : 1;
-      p->stream = reinterpret_cast<long long>(stream);
-    }
+    if (rc == FO_OK) note(p, static_cast<hipStream_t>(stream), full ? 2 : 1, full);
   }
   if (rc == FO_NOT_DIRECT) {
     if (args[15] == Py_None) Py_RETURN_FALSE;
@@ -714,7 +767,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
                          p->num_kv, p->packed, 128, 128, 128, a.sm_scale, a.logits_soft_cap, shares, a.split_ws,
                          a.split_ws_bytes, stream))
       return raise_last();
-    p->state = 0;
+    note(p, static_cast<hipStream_t>(stream), 0, full);
   }
   PyObject* ret = args[9];
   if (out) {
@@ -836,6 +889,8 @@ PyMethodDef g_methods[] = {
     {"attention", FASTCALL(attention), nullptr},
     {"enter_plan", FASTCALL(enter_plan), nullptr},
     {"follow_run", follow_run, METH_O, nullptr},
+    {"note_list", FASTCALL(note_list), nullptr},
+    {"list_source", list_source, METH_O, nullptr},
     {"kept_symbols", kept_symbols, METH_O, nullptr},
     {"packbits", FASTCALL(packbits), nullptr},
     {"segment_packbits", FASTCALL(segment_packbits), nullptr},
@@ -846,7 +901,9 @@ PyMethodDef g_methods[] = {
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
 PyMemberDef g_plan_members[] = {{"state", T_INT, offsetof(Plan, state), 0, nullptr},
-                                {"stream", T_LONGLONG, offsetof(Plan, stream), READONLY, nullptr},
+                                {"recorded_in", T_ULONGLONG, offsetof(Plan, recorded_in), 0, nullptr},
+                                {"recorded_full", T_INT, offsetof(Plan, recorded_full), READONLY, nullptr},
+                                {"sched_at", T_LONGLONG, offsetof(Plan, z.sched), READONLY, nullptr},
                                 {nullptr, 0, 0, 0, nullptr}};
 PyType_Slot g_plan_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(plan_dealloc)},
                               {Py_tp_members, g_plan_members},

@@ -41,7 +41,7 @@ constexpr int kXcds = 8;
 constexpr int kHistSlots = 8192;  // (head, length class) counters of the order layout
 // even shares (see the attention kernel): words of `sched` and limits
 constexpr int kSchedEven = 26, kSchedShare = 27, kSchedTotal = 28, kSchedShares = 29, kSchedRows = 30,
-              kSchedRecords = 31, kSchedOrdered = 32, kSchedArrived = 64;
+              kSchedRecords = 31, kSchedOrdered = 32, kSchedKept = 33, kSchedArrived = 64;
 constexpr int kSchedWords = 40;      // words [0, kSchedWords) are rewritten by every decode
 constexpr int kRecordInts = 8;  // queue entry: row, request, q block, head, first kv slot, kv count, pad, pad
 constexpr int kMaxShares = 512;      // arrival counters in `sched`, first-row entries in `shares`
@@ -474,8 +474,13 @@ __global__ void __launch_bounds__(kScanThreads) decode_small_kernel(
     const int32_t* __restrict__ sparse_info_indptr, const int32_t* __restrict__ sparse_kv_info_indptr,
     const int32_t* __restrict__ blk_req, const int32_t* __restrict__ blk_qb,
     const int32_t* __restrict__ kv_indptr, int64_t n_cand, int32_t num_heads, int32_t block_kv, int is_full,
-    int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr, int32_t* kv_idx,
+    int kept, int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr, int32_t* kv_idx,
     int32_t* counts, int32_t* order, int32_t* sched, int32_t* shares, int32_t n_shares, int32_t n_wg) {
+  if (kept) {  // (every thread has read the word when the scan, behind its barriers, clears it)
+    const int32_t newer = sched[kSchedKept];
+    if (newer == 0) return;
+    is_full = newer == 2;
+  }
   // (flags, counts and cursors stay in LDS: every trip to memory between the phases costs about as
   // much as a phase's arithmetic)
   __shared__ int32_t s_rows[kScanThreads];
@@ -692,7 +697,7 @@ int decode_impl(const uint8_t* sparse_info, const uint8_t* sparse_kv_info, const
                 int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr, int32_t* kv_idx,
                 int32_t* counts, int32_t* order, int32_t* sched, int32_t* scratch_ptr, int32_t* shares,
                 void* stream,
-                const ClearRows& clear = ClearRows{}) {
+                const ClearRows& clear = ClearRows{}, int kept = 0) {
   FO_REQUIRE(n_blk >= 0 && num_heads > 0 && num_heads <= kMaxHeads && block_kv > 0,
              "decode: bad sizes");
   FO_REQUIRE(counts && kv_row_ptr && order && sched, "decode: null output");
@@ -714,7 +719,7 @@ int decode_impl(const uint8_t* sparse_info, const uint8_t* sparse_kv_info, const
     FO_REQUIRE(row_req && row_qb && row_head && kv_idx, "decode: null output");
     decode_small_kernel<<<1, kScanThreads, 0, s>>>(
         sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb, kv_indptr,
-        n_cand, num_heads, block_kv, is_full, row_req, row_qb, row_head, kv_row_ptr, kv_idx, counts, order,
+        n_cand, num_heads, block_kv, is_full, kept, row_req, row_qb, row_head, kv_row_ptr, kv_idx, counts, order,
         sched, shares, n_shares, n_wg);
     FO_CHECK_LAUNCH();
     return FO_OK;
@@ -776,6 +781,20 @@ extern "C" int fo_decode_sparse(const uint8_t* sparse_info, const uint8_t* spars
   return decode_impl(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
                      kv_indptr, n_blk, num_heads, block_kv, is_full, row_req, row_qb, row_head, kv_row_ptr,
                      kv_idx, counts, order, sched, scratch, shares, stream);
+}
+
+extern "C" int fo_decode_sparse_kept(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
+                                     const int32_t* sparse_info_indptr, const int32_t* sparse_kv_info_indptr,
+                                     const int32_t* blk_req, const int32_t* blk_qb, const int32_t* kv_indptr,
+                                     int32_t n_blk, int32_t num_heads, int32_t block_kv, int32_t* row_req,
+                                     int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr, int32_t* kv_idx,
+                                     int32_t* counts, int32_t* order, int32_t* sched, int32_t* scratch, int32_t* shares,
+                                     void* stream) {
+  const int64_t n_cand = static_cast<int64_t>(n_blk) * num_heads;
+  FO_REQUIRE(n_cand > 0 && n_cand <= kScanThreads, "decode: lists of 1 to %d (q-block, head) pairs only", kScanThreads);
+  return decode_impl(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
+                     kv_indptr, n_blk, num_heads, block_kv, 0, row_req, row_qb, row_head, kv_row_ptr, kv_idx, counts,
+                     order, sched, scratch, shares, stream, ClearRows{}, 1);
 }
 
 extern "C" int32_t fo_decode_sparse_clear_min_pairs(void) { return kScanThreads + 1; }

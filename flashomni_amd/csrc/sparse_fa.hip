@@ -161,6 +161,7 @@ struct FaParams {
   uint8_t* keep_kv_info;
   int32_t* keep_indptr;
   int32_t info_bytes, kv_info_bytes;
+  int32_t mark;  // value for sched[kSchedKept], or 0: the word stays
 };
 
 template <typename T>
@@ -238,7 +239,8 @@ __device__ __forceinline__ float max_across_halves(float x) {
 // cursors, [24] completion counter; [26] even shares in use, [27] cost share of a workgroup, [28]
 // total cost, [29] number of shares, [30] number of rows, [31] the share table holds one record per
 // queue entry; [64..575] arrival counters of the rows cut at share boundaries
-constexpr int kSchedEven = 26, kSchedArrived = 64;
+// sched[33]: 0, or this launch's rows (1: kept symbols, 2: every row) are newer than the decoded list
+constexpr int kSchedEven = 26, kSchedKept = 33, kSchedArrived = 64;
 constexpr int kRecordInts = 8;  // queue entry record: row, request, q block, head, first kv slot, kv count
 constexpr int kMaxShares = 512, kMaxSplitParts = 4, kRowOverhead = 3;
 constexpr int kItemBatch = 16;  // item records of a share gathered at a time
@@ -877,6 +879,7 @@ sparse_fa_kernel(const FaParams p) {
         p.keep_indptr[p.batch + 1 + i] = p.kv_info_indptr[i];
       }
     }
+    if (p.mark != 0 && blockIdx.x == 0 && tid == 0) p.sched[kSchedKept] = p.mark;
     direct_schedule();
     if (wv == 0) {
       if (lane == 0) s_share[0] = 0;
@@ -2226,11 +2229,12 @@ extern "C" int fo_sparse_attention_direct(const void* args) {
   p.blk_req = a.blk_req; p.blk_qb = a.blk_qb;
   p.n_blk = a.n_blk; p.batch = a.batch; p.symbol_heads = a.symbol_heads; p.is_full = a.is_full;
   p.zero_skipped = a.zero_skipped && !a.is_full;
-  if (!a.is_full && a.keep_info) {
-    FO_REQUIRE(a.keep_kv_info && a.keep_indptr, "sparse_attention: null pointer");
+  if (!a.is_full && (a.keep_info || a.keep_kv_info || a.keep_indptr)) {
+    FO_REQUIRE(a.keep_info && a.keep_kv_info && a.keep_indptr, "sparse_attention: null pointer");
     p.keep_info = a.keep_info; p.keep_kv_info = a.keep_kv_info; p.keep_indptr = a.keep_indptr;
     p.info_bytes = a.info_bytes; p.kv_info_bytes = a.kv_info_bytes;
   }
+  p.mark = a.keep_indptr == nullptr ? 0 : a.is_full ? 2 : 1;
   hipStream_t s = static_cast<hipStream_t>(a.stream);
   const bool bf16 = a.dtype == FO_BF16;
   if (a.logits_soft_cap > 0.f) {

@@ -96,7 +96,7 @@ typedef struct fo_batch_sizes {
   /* offsets inside the tables: [batch + 1] each ... */
   int64_t qo_indptr, kv_indptr, q_blk_base, kv_blk_base, info_indptr, kv_info_indptr;
   int64_t blk_req, blk_qb;          /* ... and [n_q_blocks] each */
-  int64_t sched;                    /* 1024 zeros: see fo_sparse_attention_direct */
+  int64_t sched;                    /* 1024 zeros: sched of a decoded list and of fo_sparse_attention_direct */
   int64_t table_ints;
 } fo_batch_sizes;
 int fo_plan_batch(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host, int32_t batch_size,
@@ -170,6 +170,20 @@ int fo_decode_sparse(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
                      int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr,
                      int32_t* kv_idx, int32_t* counts, int32_t* order, int32_t* sched,
                      int32_t* scratch, int32_t* shares, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
+ * fo_decode_sparse of what the last fo_sparse_attention_direct on the same `sched` computed, if that is newer
+ * than the list: sched[33] is 0 (every decode leaves it so) and the list stays, or 1 and the symbols given here
+ * are decoded (the ones that launch kept), or 2 and every bit counts as set.  For callers that cannot know which
+ * of two launches came last, because graphs hold them.  1 to 1024 (q block, head) pairs.
+ * ------------------------------------------------------------------------------------------- */
+int fo_decode_sparse_kept(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
+                          const int32_t* sparse_info_indptr, const int32_t* sparse_kv_info_indptr,
+                          const int32_t* blk_req, const int32_t* blk_qb, const int32_t* kv_indptr,
+                          int32_t n_blk, int32_t num_heads, int32_t block_kv,
+                          int32_t* row_req, int32_t* row_qb, int32_t* row_head, int32_t* kv_row_ptr,
+                          int32_t* kv_idx, int32_t* counts, int32_t* order, int32_t* sched,
+                          int32_t* scratch, int32_t* shares, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * fo_decode_sparse that also clears, in a fresh 16-bit attention output o [nnz_q, H, 128] (strides in
@@ -288,11 +302,13 @@ int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
  * candidates, more than 2^20 keep bits, no split workspace of fo_sparse_fa_split_workspace_bytes() bytes.
  * Arguments as in fo_decode_sparse (symbols, blk_req, blk_qb, is_full; n_blk symbol rows of symbol_heads
- * heads) and fo_sparse_fa_run.  sched: 1024 int32, zero before the first launch and left zero by every
- * one.  A workgroup lists at most 4096 kv blocks of a row, as in fo_sparse_fa_run.
+ * heads) and fo_sparse_fa_run.  sched: 1024 int32, its words [64, 576) zero before the first launch and left
+ * zero by every one (it may be the sched of a decoded list).  A workgroup lists at most 4096 kv blocks of a row, as in fo_sparse_fa_run.
  * zero_skipped: the rows of q blocks that are not computed are cleared in o.  keep_info,
  * keep_kv_info, keep_indptr (optional): receive the info_bytes / kv_info_bytes of symbols and the two
- * indptrs ([2 * (batch + 1)]) that this launch read, for a decode of the same list later.  Launches that share sched or split_ws must not overlap in time.
+ * indptrs ([2 * (batch + 1)]) that this launch read, for a decode of the same list later; with keep_indptr (also
+ * where is_full needs no copy) the launch sets sched[33] to 1 (is_full: 2), see fo_decode_sparse_kept.
+ * Launches that share sched or split_ws must not overlap in time.
  * ------------------------------------------------------------------------------------------- */
 typedef struct fo_attention_args {
   const void *q, *k, *v;

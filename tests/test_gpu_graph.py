@@ -205,3 +205,103 @@ def test_captured_short_run_keeps_its_symbols_in_place(dev):
         assert all(bool((j == 0x5a).all()) for j in junk), "a replay wrote outside its own buffers"
     listed = w.run(q, k, v, *sym, out=torch.zeros_like(q), reuse_decoded=True)
     assert float((listed.float() - exp.float()).abs().max()) <= 8e-3
+
+
+class _ShortList:
+    """Two short requests, a wrapper, and the result of every symbol set by the oracle."""
+
+    def __init__(self, dev, seed):
+        import flashomni_amd as fo
+        import oracle
+        self.dev, heads, lens = dev, 2, [384, 130]
+        g = torch.Generator().manual_seed(seed)
+        q, k, v = (torch.randn(sum(lens), heads, 128, generator=g).to(torch.bfloat16) for _ in range(3))
+        names = ("packed_info", "packed_keep", "info_indptr", "keep_indptr")
+        masks = [make_ragged_masks(lens, lens, heads, 0.7, 0.5, seed=seed + i) for i in range(3)]
+        self.sym = [[torch.from_numpy(m[n]).to(dev) for n in names] for m in masks]
+        self.exp = [oracle.sparse_attention(q, k, v, *(m[n] for n in names), m["qo_indptr"], m["kv_indptr"],
+                                            out=torch.zeros_like(q)) for m in masks]
+        self.full = oracle.sparse_attention(q, k, v, None, None, None, None, masks[0]["qo_indptr"], masks[0]["kv_indptr"],
+                                            is_full=True, out=torch.zeros_like(q))
+        self.qkv = [t.to(dev) for t in (q, k, v)]
+        self.buf = [t.clone() for t in self.sym[0]]    # rewritten in place between replays
+        indptr = torch.from_numpy(masks[0]["qo_indptr"])
+        self.w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+        self.w.plan(indptr, indptr, heads, heads, 128, q_data_type=torch.bfloat16)
+        self.out = torch.zeros_like(self.qkv[0])
+
+    def run(self, sym, reuse=False, is_full=False):
+        return self.w.run(*self.qkv, *sym, is_full, out=self.out, reuse_decoded=reuse)
+
+    def capture(self, fn):
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            fn()
+        return graph
+
+    def check(self, exp, fn, *args, **kw):
+        self.out.zero_()
+        fn(*args, **kw)
+        torch.cuda.synchronize()
+        got = self.out.cpu().float()
+        assert float((got - exp.float()).abs().max()) <= 2e-2
+        assert float((got - exp.float()).norm()) <= 1e-2 * float(exp.float().norm()) + 1e-6
+
+
+def test_captured_reuse_runs_the_list_of_the_moment(dev):
+    """A reuse in a graph runs, at every replay, what the last run or decode before it left, whether that was
+    decoded or took its rows from the symbols, eagerly or in another graph; recording it leaves the eager state
+    as it was."""
+    s = _ShortList(dev, 30)
+    a, b, c = s.sym
+    s.check(s.exp[0], s.run, a)                                   # rows from the symbols: no list yet
+    reuse = s.capture(lambda: s.run(a, reuse=True))
+    s.check(s.exp[0], s.run, a, reuse=True)                       # eagerly, before any replay
+    s.check(s.exp[0], reuse.replay)
+    s.run(b)
+    s.check(s.exp[1], reuse.replay)
+    s.check(s.exp[1], reuse.replay)
+    s.w.decode(*c)
+    s.check(s.exp[2], reuse.replay)
+    s.check(s.exp[2], s.run, c, reuse=True)
+    run = s.capture(lambda: s.run(s.buf))                         # a run in a graph, symbols rewritten in place
+    s.check(s.exp[2], s.run, c, reuse=True)                       # recording it has run nothing
+    for i in (1, 2, 0):
+        for dst, src in zip(s.buf, s.sym[i]):
+            dst.copy_(src)
+        s.check(s.exp[i], run.replay)
+        s.check(s.exp[i], s.run, s.buf, reuse=True)
+        s.check(s.exp[i], reuse.replay)
+        s.w.decode(*s.sym[(i + 1) % 3])
+        s.check(s.exp[(i + 1) % 3], reuse.replay)
+    s.run([None] * 4, is_full=True)
+    s.check(s.full, reuse.replay)
+    s.check(s.full, s.run, [None] * 4, reuse=True, is_full=True)
+
+
+def test_captured_decode_and_reuse(dev):
+    """decode() on a second stream and reuse of its list in one graph (no launch but those two), also on a plan that
+    has not run before; a reuse made before the first replay computes nothing."""
+    s = _ShortList(dev, 40)
+    side = torch.cuda.Stream(device=dev)
+
+    def step():
+        cur = torch.cuda.current_stream()
+        side.wait_stream(cur)
+        with torch.cuda.stream(side):
+            s.w.decode(*s.buf)
+        cur.wait_stream(side)
+        s.run(s.buf, reuse=True)
+
+    graph = s.capture(step)
+    s.check(torch.zeros_like(s.exp[0]), s.run, s.buf, reuse=True)
+    for i in (0, 1, 2):
+        for dst, src in zip(s.buf, s.sym[i]):
+            dst.copy_(src)
+        s.check(s.exp[i], graph.replay)
+        s.run(s.sym[(i + 1) % 3])
+        s.check(s.exp[i], graph.replay)
+        s.check(s.exp[i], s.run, s.buf, reuse=True)
+        with pytest.raises(RuntimeError, match="is_full=False"):
+            s.run(s.buf, reuse=True, is_full=True)
