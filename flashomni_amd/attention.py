@@ -98,7 +98,7 @@ class PlannedBatch:
 
     def __init__(self, float_workspace_buffer, qo_indptr_host, kv_indptr_host, qo_indptr_dev,
                  kv_indptr_dev, num_qo_heads, num_kv_heads, block_q, block_kv, share_rows=True,
-                 worklist=None, gqa_packed=False):
+                 worklist=None, gqa_packed=False, send=(0, None, None, None)):
         self.device = float_workspace_buffer.device
         self.float_ws = float_workspace_buffer
         self.num_qo_heads, self.num_kv_heads = num_qo_heads, num_kv_heads
@@ -118,7 +118,7 @@ class PlannedBatch:
         index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         self.native, self.tables, sizes = _lib.native().plan(
             qo_indptr_host, kv_indptr_host, num_qo_heads, num_kv_heads, self.gqa_packed, index,
-            qo_indptr_dev, kv_indptr_dev)
+            qo_indptr_dev, kv_indptr_dev, *send)
         (self.n_q_blk, self.n_kv_blk, self.max_rows, self.max_nnz, self.total_q_rows, self.total_kv_rows,
          self.min_info_bytes, self.min_kv_info_bytes, self.max_kv_len, *self._table_at) = sizes
         self.qo_indptr = self._table(0) if qo_indptr_dev is None else qo_indptr_dev
@@ -433,7 +433,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         self._backend = backend  # accepted for compatibility; there is one HIP code path
         self._plan_info = None
         self._planned = None  # PlannedBatch of the last plan()
-        self._pin_offset = 0  # free part of the pinned mirror (plans are laid out one behind the other)
+        self._pin_ring = _lib.native().new_ring()  # (plans are laid out in the pinned mirror one behind the other)
 
     @property
     def is_cuda_graph_enabled(self) -> bool:
@@ -446,7 +446,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         self._pin_memory_int_workspace_buffer = torch.empty(
             self._int_workspace_buffer.shape, dtype=self._int_workspace_buffer.dtype, device="cpu",
             pin_memory=True)
-        self._pin_offset = 0
+        self._pin_ring = _lib.native().new_ring()
         # whether rows may be shared between workgroups depends on the float workspace, and a list
         # decoded for the old buffers' share table must not be reused
         if self._planned is not None:
@@ -557,20 +557,20 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         graph = self.is_cuda_graph_enabled
         with _lib.device_guard(self.device):
             try:
-                self._pin_offset = _lib.native().host_plan(
-                    self._float_workspace_buffer, self._int_workspace_buffer,
-                    self._pin_memory_int_workspace_buffer, self._pin_offset, qo_indptr_host, kv_indptr_host,
+                sent = _lib.native().host_plan(
+                    self._float_workspace_buffer, self._int_workspace_buffer, qo_indptr_host, kv_indptr_host,
                     self._max_total_num_rows or total_num_rows, num_qo_heads, num_kv_heads, graph,
                     q_data_type.itemsize, plan_info)
             except RuntimeError as e:  # same wording as csrc/batch_sparseFA.cu:61
                 raise RuntimeError("Failed to plan prefill with error: " + str(e)) from None
-            self._plan_info = plan_info
             self._planned = PlannedBatch(
                 self._float_workspace_buffer, qo_indptr_host, kv_indptr_host,
                 self._qo_indptr_buf if graph else None, self._kv_indptr_buf if graph else None, num_qo_heads,
                 num_kv_heads, sparse_block_size_for_q, sparse_block_size_for_kv, share_rows=self._share_rows,
                 worklist=self._planned._list if self._planned is not None else None,
-                gqa_packed=gqa_symbols != "per_q_head")
+                gqa_packed=gqa_symbols != "per_q_head",
+                send=(sent, self._int_workspace_buffer, self._pin_memory_int_workspace_buffer, self._pin_ring))
+            self._plan_info = plan_info
         if not graph:
             self._qo_indptr_buf, self._kv_indptr_buf = self._planned.qo_indptr, self._planned.kv_indptr
 

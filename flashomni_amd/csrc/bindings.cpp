@@ -356,6 +356,111 @@ void note(Plan* p, hipStream_t stream, int state, bool full) {
   }
 }
 
+// host_plan()'s arrays, until plan() sends them
+thread_local std::unique_ptr<char[]> t_planned;
+thread_local size_t t_planned_size = 0;
+
+// The pinned mirror of an integer workspace.  Plans are laid out in it one behind the other: the copy that an
+// earlier plan queued may still be reading its part, and waiting for it would mean waiting for everything queued
+// before it.  A half of the mirror is written again when the copies out of it are done, which is looked at (and
+// fenced, on the default stream) only where a plan enters the other half: half a lap ago, so that there is rarely
+// anything left to wait for, and never for other streams.
+struct Ring {
+  PyObject_HEAD
+  size_t off;
+  int half;
+  struct Half {
+    bool on_default;                                    // copies on the default stream, fenced by ...
+    hipEvent_t fence;                                   // ... this, recorded when the half is left
+    std::vector<std::pair<hipStream_t, Word>> others;   // other streams: the last plan's word (written behind its copy)
+  } halves[2];
+};
+PyTypeObject* g_ring_type = nullptr;
+
+void ring_dealloc(PyObject* self) {
+  Ring* r = reinterpret_cast<Ring*>(self);
+  for (Ring::Half& h : r->halves) {
+    if (h.fence) (void)hipEventDestroy(h.fence);
+    h.others.~vector();
+  }
+  PyTypeObject* t = Py_TYPE(self);
+  t->tp_free(self);
+  Py_DECREF(t);
+}
+
+PyObject* new_ring(PyObject*, PyObject*) {
+  PyObject* self = g_ring_type->tp_alloc(g_ring_type, 0);
+  if (!self) return nullptr;
+  for (Ring::Half& h : reinterpret_cast<Ring*>(self)->halves) new (&h.others) std::vector<std::pair<hipStream_t, Word>>();
+  return self;
+}
+
+hipError_t leave_half(Ring::Half& h) {
+  if (!h.on_default) return hipSuccess;
+  c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);  // (another thread may be capturing)
+  if (!h.fence) {
+    const hipError_t e = hipEventCreateWithFlags(&h.fence, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+  }
+  return hipEventRecord(h.fence, nullptr);
+}
+
+hipError_t enter_half(Ring::Half& h) {
+  if (h.on_default) {
+    c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+    const hipError_t e = host_wait(h.fence);
+    if (e != hipSuccess) return e;
+    h.on_default = false;
+  }
+  const auto others = std::move(h.others);
+  h.others.clear();
+  for (const auto& o : others)
+    if (!wait_word(o.second)) return hipErrorNotReady;
+  return hipSuccess;
+}
+
+// a part of the mirror for `used` bytes
+hipError_t ring_take(Ring* r, size_t size, size_t used, size_t* at) {
+  const size_t mid = size / 2;
+  const bool large = used > mid;  // (then the whole mirror, alone)
+  size_t off = r->off;
+  int half = r->half;
+  if (large) {
+    hipError_t e = leave_half(r->halves[half]);
+    if (e == hipSuccess) e = enter_half(r->halves[half]);
+    if (e == hipSuccess) e = enter_half(r->halves[1 - half]);
+    if (e != hipSuccess) return e;
+    off = 0;
+    half = 1;
+  } else if (off + used > (half ? size : mid)) {
+    hipError_t e = leave_half(r->halves[half]);
+    if (e == hipSuccess) e = enter_half(r->halves[1 - half]);
+    if (e != hipSuccess) return e;
+    half = 1 - half;
+    off = half ? mid : 0;
+  }
+  *at = off;
+  r->off = large ? size : (off + used + 255) / 256 * 256;
+  r->half = half;
+  return hipSuccess;
+}
+
+// the copy out of the part just taken has been queued, and `word`'s launch behind it
+void ring_note(Ring* r, bool large, hipStream_t stream, const Word& word) {
+  for (int i = 0; i < 2; ++i) {
+    Ring::Half& h = r->halves[i];
+    if (i != r->half && !large) continue;
+    if (!stream) {
+      h.on_default = true;
+      if (i != r->half) (void)leave_half(h);
+      continue;
+    }
+    auto o = std::find_if(h.others.begin(), h.others.end(), [&](const auto& v) { return v.first == stream; });
+    if (o == h.others.end()) h.others.emplace_back(stream, word);
+    else o->second = word;
+  }
+}
+
 PyObject* raise_captured_plan() {
   PyErr_SetString(PyExc_RuntimeError, "plan() cannot be captured in a graph");
   return nullptr;
@@ -428,13 +533,15 @@ PyObject* enter_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // (qo_indptr, kv_indptr: int32 on the host; num_qo_heads, num_kv_heads, packed, device index,
-//  qo_indptr, kv_indptr of the device or None) -> (Plan, tables, sizes)
+//  qo_indptr, kv_indptr of the device or None; and, to send host_plan()'s arrays: their bytes, the integer
+//  workspace, its pinned mirror and the mirror's Ring, or 0 and None) -> (Plan, tables, sizes)
 PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_BEGIN
-  const Tensor *qo, *kv, *qo_dev, *kv_dev;
-  int64_t hq, hkv, dev;
-  if (!(n == 8 && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
-        whole(args[3], &hkv) && whole(args[5], &dev) && opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
+  const Tensor *qo, *kv, *qo_dev, *kv_dev, *iws, *pin;
+  int64_t hq, hkv, dev, sent;
+  if (!(n == 12 && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
+        whole(args[3], &hkv) && whole(args[5], &dev) && whole(args[8], &sent) && opt_tensor(args[9], &iws) &&
+        opt_tensor(args[10], &pin) && (sent == 0 || (iws && pin && Py_TYPE(args[11]) == g_ring_type)) && opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
         qo->scalar_type() == at::kInt && kv->scalar_type() == at::kInt && qo->is_contiguous() && kv->is_contiguous() &&
         qo->is_cpu() && kv->is_cpu() && qo->numel() == kv->numel() && qo->numel() >= 1)) {
     PyErr_SetString(PyExc_RuntimeError, "plan: bad argument");
@@ -482,8 +589,26 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
       PyErr_SetString(PyExc_RuntimeError, "hipHostMalloc failed");
       return nullptr;
     }
+    Ring* ring = sent ? reinterpret_cast<Ring*>(args[11]) : nullptr;
+    const size_t mirror = sent ? pin->numel() * pin->element_size() : 0;
+    if (ring) {
+      size_t at = 0;
+      hipError_t e = static_cast<size_t>(sent) > mirror ? hipErrorInvalidValue : ring_take(ring, mirror, sent, &at);
+      if (e == hipSuccess) {
+        char* host = static_cast<char*>(pin->data_ptr()) + at;
+        std::memcpy(host, t_planned.get(), sent);
+        e = hipMemcpyAsync(iws->data_ptr(), host, sent, hipMemcpyHostToDevice, home);
+      }
+      if (e != hipSuccess) {
+        Py_DECREF(self);
+        PyErr_Format(PyExc_RuntimeError, "the copy into the integer workspace failed: %s", hipGetErrorString(e));
+        return nullptr;
+      }
+    }
     rc = fo_plan_tables_signal(qo->data_ptr<int32_t>(), kv->data_ptr<int32_t>(), batch, hq, hkv, packed,
                                p->tables.data_ptr<int32_t>(), p->word.at, p->word.ticket, p->home);
+    if (rc) (void)hipStreamSynchronize(home);  // (no word to wait for)
+    else if (ring) ring_note(ring, static_cast<size_t>(sent) > mirror / 2, home, p->word);
   } catch (...) {
     Py_DECREF(self);
     throw;
@@ -510,60 +635,34 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_END
 }
 
-// The host planner and the copy of its arrays into the integer workspace: (float workspace, integer
-// workspace, pinned mirror, offset of the mirror's free part, qo_indptr, kv_indptr (host), rows, heads,
-// kv heads, graph mode, element size, plan vector) -> the mirror's new offset.
-// Plans are laid out one behind the other in the pinned mirror: the copy that an earlier plan queued may
-// still be reading its part, and waiting for it would mean waiting for everything queued before it.
-// Only when the mirror is full the device is waited for.
+// The host planner: (float workspace, integer workspace, qo_indptr, kv_indptr (host), rows, heads, kv heads, graph
+// mode, element size, plan vector) -> bytes of its arrays, which plan() sends to the integer workspace from this
+// thread's scratch.
 PyObject* host_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_BEGIN
-  const Tensor *fws, *iws, *pin, *qo, *kv, *info;
-  int64_t off, rows, hq, hkv, elem;
-  if (!(n == 12 && opt_tensor(args[0], &fws) && fws && opt_tensor(args[1], &iws) && iws && opt_tensor(args[2], &pin) &&
-        pin && whole(args[3], &off) && opt_tensor(args[4], &qo) && qo && opt_tensor(args[5], &kv) && kv &&
-        whole(args[6], &rows) && whole(args[7], &hq) && whole(args[8], &hkv) && whole(args[10], &elem) &&
-        opt_tensor(args[11], &info) && info && info->scalar_type() == at::kLong && info->numel() == 15)) {
+  const Tensor *fws, *iws, *qo, *kv, *info;
+  int64_t rows, hq, hkv, elem;
+  if (!(n == 10 && opt_tensor(args[0], &fws) && fws && opt_tensor(args[1], &iws) && iws && opt_tensor(args[2], &qo) && qo &&
+        opt_tensor(args[3], &kv) && kv && whole(args[4], &rows) && whole(args[5], &hq) && whole(args[6], &hkv) &&
+        whole(args[8], &elem) && opt_tensor(args[9], &info) && info && info->scalar_type() == at::kLong && info->numel() == 15)) {
     PyErr_SetString(PyExc_RuntimeError, "plan: bad argument");
     return nullptr;
   }
-  if (capturing(static_cast<hipStream_t>(stream_of(iws->get_device())))) return raise_captured_plan();
-  const bool graph = truth(args[9]);
+  const bool graph = truth(args[7]);
   const int batch = static_cast<int>(qo->numel()) - 1;
-  const size_t bytes = iws->numel() * iws->element_size(), pin_bytes = pin->numel() * pin->element_size();
+  const size_t bytes = iws->numel() * iws->element_size();
   // (the planner writes the used prefix only: the rest of the scratch is never touched)
-  static thread_local std::unique_ptr<char[]> scratch;
-  static thread_local size_t scratch_bytes = 0;
-  if (scratch_bytes < bytes) {
-    scratch.reset(new char[bytes]);
-    scratch_bytes = bytes;
+  if (t_planned_size < bytes) {
+    t_planned.reset(new char[bytes]);
+    t_planned_size = bytes;
   }
   int64_t* v = info->data_ptr<int64_t>();
-  if (fo_prefill_plan(fws->data_ptr(), fws->numel() * fws->element_size(), nullptr, scratch.get(), bytes,
+  if (fo_prefill_plan(fws->data_ptr(), fws->numel() * fws->element_size(), nullptr, t_planned.get(), bytes,
                       qo->data_ptr<int32_t>(), kv->data_ptr<int32_t>(), rows, batch, hq, hkv, 128, 128, 1, graph, elem, 0,
                       v, nullptr))
     return raise_last();
   // end of the last array: block_valid_mask, else the row count (graph mode), else the chunk size
-  const size_t used = v[14] ? v[12] + v[0] : (v[13] ? v[2] : v[9]) + 4;
-  if (used > pin_bytes) {
-    PyErr_SetString(PyExc_RuntimeError, "the pinned mirror is smaller than the integer workspace");
-    return nullptr;
-  }
-  if (off + used > pin_bytes) {
-    if (hipDeviceSynchronize() != hipSuccess) {
-      PyErr_SetString(PyExc_RuntimeError, "hipDeviceSynchronize failed");
-      return nullptr;
-    }
-    off = 0;
-  }
-  char* host = static_cast<char*>(pin->data_ptr()) + off;
-  std::memcpy(host, scratch.get(), used);
-  if (hipMemcpyAsync(iws->data_ptr(), host, used, hipMemcpyHostToDevice,
-                     static_cast<hipStream_t>(stream_of(iws->get_device()))) != hipSuccess) {
-    PyErr_SetString(PyExc_RuntimeError, "the copy into the integer workspace failed");
-    return nullptr;
-  }
-  return PyLong_FromLongLong((off + used + 255) / 256 * 256);
+  return PyLong_FromLongLong(v[14] ? v[12] + v[0] : (v[13] ? v[2] : v[9]) + 4);
   TORCH_GUARD_END
 }
 
@@ -886,6 +985,7 @@ PyMethodDef g_methods[] = {
     {"gemm_o", FASTCALL(gemm_o), nullptr},
     {"plan", FASTCALL(plan), nullptr},
     {"host_plan", FASTCALL(host_plan), nullptr},
+    {"new_ring", new_ring, METH_NOARGS, nullptr},
     {"attention", FASTCALL(attention), nullptr},
     {"enter_plan", FASTCALL(enter_plan), nullptr},
     {"follow_run", follow_run, METH_O, nullptr},
@@ -905,6 +1005,9 @@ PyMemberDef g_plan_members[] = {{"state", T_INT, offsetof(Plan, state), 0, nullp
                                 {"recorded_full", T_INT, offsetof(Plan, recorded_full), READONLY, nullptr},
                                 {"sched_at", T_LONGLONG, offsetof(Plan, z.sched), READONLY, nullptr},
                                 {nullptr, 0, 0, 0, nullptr}};
+PyType_Slot g_ring_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(ring_dealloc)}, {0, nullptr}};
+PyType_Spec g_ring_spec = {"flashomni_amd._native.Ring", sizeof(Ring), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_DISALLOW_INSTANTIATION,
+                           g_ring_slots};
 PyType_Slot g_plan_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(plan_dealloc)},
                               {Py_tp_members, g_plan_members},
                               {0, nullptr}};
@@ -914,6 +1017,8 @@ PyType_Spec g_plan_spec = {"flashomni_amd._native.Plan", sizeof(Plan), 0, Py_TPF
 }  // namespace
 
 PyMODINIT_FUNC PyInit__native(void) {
+  g_ring_type = reinterpret_cast<PyTypeObject*>(PyType_FromSpec(&g_ring_spec));
+  if (!g_ring_type) return nullptr;
   g_plan_type = reinterpret_cast<PyTypeObject*>(PyType_FromSpec(&g_plan_spec));
   if (!g_plan_type) return nullptr;
   return PyModule_Create(&g_module);

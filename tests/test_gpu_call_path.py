@@ -136,3 +136,79 @@ def test_plan_is_refused_under_capture(dev):
         torch.zeros(8, device=dev)
         graph.capture_end()
     w.plan(ip, ip, 2, 2, 128, q_data_type=torch.bfloat16)
+
+
+@pytest.mark.parametrize("stream", ["default", "side"])
+@pytest.mark.parametrize("capturing", [False, True])
+def test_plans_beyond_the_pinned_mirror(dev, stream, capturing):
+    """Plans one behind the other in a small pinned mirror, many laps of it, queued behind a busy stretch: every
+    copy arrives as it was planned, no other stream is waited for, and another thread may be capturing."""
+    import threading
+
+    import flashomni_amd as fo
+    ws = torch.empty(128 << 20, dtype=torch.uint8, device=dev)
+    batches = [torch.tensor(v, dtype=torch.int32) for v in ([0, 300, 640], [0, 1, 200, 2000], [0, 5000])]
+
+    def plan(w, ip):
+        w.plan(ip, ip, 4, 4, 128, q_data_type=torch.bfloat16)
+
+    def arrays(info, workspace, ip):      # (what lies between the aligned arrays is not defined)
+        n, rows = info[0], info[1]
+        parts = [(info[4], 4 * n), (info[5], 4 * n), (info[6], 4 * n), (info[8], 4 * ip.numel()), (info[9], 4)]
+        if info[14]:
+            parts += [(info[7], 4 * rows + 4), (info[12], n)]
+        return [workspace[a:a + size].tolist() for a, size in parts]
+
+    exp = []
+    for ip in batches:
+        w = fo.BatchFlashOmniFAWithRaggedKVWrapper(ws)
+        plan(w, ip)
+        exp.append((w._plan_info.tolist(), arrays(w._plan_info.tolist(), w._int_workspace_buffer.cpu(), ip)))
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(ws)
+    w.reset_workspace_buffer(ws, torch.zeros(40960, dtype=torch.uint8, device=dev))
+    other, third = torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)
+    planner = torch.cuda.current_stream(dev) if stream == "default" else torch.cuda.Stream(device=dev)
+    busy = torch.empty(1 << 30, dtype=torch.uint8, device=dev)
+    copies = torch.zeros(200, 40960, dtype=torch.uint8, device=dev)
+    with torch.cuda.stream(planner):     # (torch itself cannot take memory from the device while a thread captures)
+        plan(w, batches[1])
+        plan(w, batches[2])
+    torch.cuda.synchronize(dev)
+    graph, begun, planned, errors = torch.cuda.CUDAGraph(), threading.Event(), threading.Event(), []
+
+    def capture():
+        try:
+            with torch.cuda.stream(third):
+                graph.capture_begin()
+                begun.set()
+                planned.wait(60)
+                torch.zeros(8, device=dev)
+                graph.capture_end()
+        except Exception as e:
+            errors.append(e)
+            begun.set()
+
+    thread = threading.Thread(target=capture) if capturing else None
+    if thread:
+        thread.start()
+        begun.wait(60)
+    seen = []
+    with torch.cuda.stream(other):
+        for i in range(300):                      # ~0.1 s
+            busy.fill_(i & 1)
+    with torch.cuda.stream(planner):
+        for i in range(200):
+            w._int_workspace_buffer.zero_()
+            plan(w, batches[i % 3])
+            copies[i].copy_(w._int_workspace_buffer)
+            seen.append(w._plan_info.tolist())
+    waited = other.query() if not capturing else False
+    planned.set()
+    if thread:
+        thread.join(60)
+    torch.cuda.synchronize(dev)
+    assert not errors, errors
+    assert not waited, "the other stream was waited for"
+    for i, (info, got) in enumerate(zip(seen, copies.cpu())):
+        assert info == exp[i % 3][0]
+        assert arrays(info, got, batches[i % 3]) == exp[i % 3][1], i
