@@ -59,8 +59,11 @@
 #include <type_traits>
 
 #include "fo_common.h"
+#include "fo_device.h"
 
 namespace {
+
+using fo::wave_scan;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
@@ -284,18 +287,6 @@ __device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q,
   }
   *first = kXcds;
   return -1;
-}
-
-// Inclusive prefix sum over the 64 lanes of a wavefront: rows of 16 lanes by lane shifts, then the row totals
-// through scalar registers.
-__device__ __forceinline__ int wave_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);  // row_shr:8
-  const int t0 = __builtin_amdgcn_readlane(v, 15), t1 = __builtin_amdgcn_readlane(v, 31), t2 = __builtin_amdgcn_readlane(v, 47);
-  const int row = (threadIdx.x & 63) >> 4;
-  return v + (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
 }
 
 // The bits [bit, bit + n) of a byte-aligned segment as 32-bit words: word i of the range, bits outside of it
