@@ -151,6 +151,13 @@ class FluxLayer:
         self.attention(fresh_decode=False)
         return self.gemm_o_final()
 
+    def step_one_stream(self):
+        """The same calls one after the other on one stream."""
+        self.gemm_q()
+        self.decode()
+        self.attention(fresh_decode=False)
+        return self.gemm_o_final()
+
     def step_dropin(self):
         """The same pass as the reference's call sequence on one stream: flashomni_gemm, then
         wrapper.run(q, k, v, symbols...) (which decodes the symbols itself), then
@@ -528,19 +535,23 @@ def main():
     layer = FluxLayer(dev)
     kernels = {}
 
-    # the step's two-stream form must give what the plain sequence of calls gives
-    layer.gemm_q(); layer.attention(fresh_decode=True); ref_o = layer.gemm_o_final().clone()
-    ref_q, ref_fa = layer.out_q.clone(), layer.out_fa.clone()
-    layer.out_q.zero_(); layer.out_fa.zero_()
-    got_o = layer.step()
-    torch.cuda.synchronize()
-    # (run() takes the rows from the packed symbols and cuts them for the workgroups differently than the
-    # decoded list does: the probabilities are rounded against other running maxima, which shows as 1.4e-3 of
-    # the attention's norm and 1.9e-3 of the projection's; four times that is allowed)
+    def results(step):
+        layer.out_q.zero_(); layer.out_fa.zero_()
+        o = step()
+        torch.cuda.synchronize()
+        return layer.out_q.clone(), layer.out_fa.clone(), o.clone()
+
+    # the step's two-stream form must give the bits of the same calls on one stream
+    got, one, dropin = (results(step) for step in (layer.step, layer.step_one_stream, layer.step_dropin))
+    assert all(torch.equal(a, b) for a, b in zip(got, one)), "two-stream step differs from the calls on one stream"
+    # and, within rounding, what the plain sequence of calls gives.  (run() takes the rows from the packed symbols and
+    # cuts them for the workgroups differently than the decoded list does: the probabilities are rounded against other
+    # running maxima, which shows as 1.4e-3 of the attention's norm and 1.9e-3 of the projection's; four times that is
+    # allowed)
     close = lambda got, exp: float((got.float() - exp.float()).norm()) <= 8e-3 * float(exp.float().norm())
-    assert torch.equal(ref_q, layer.out_q) and close(layer.out_fa, ref_fa) and close(got_o, ref_o), \
-        "two-stream step differs from the sequential chain"
-    del ref_q, ref_fa, ref_o, got_o
+    assert torch.equal(got[0], dropin[0]) and close(got[1], dropin[1]) and close(got[2], dropin[2]), \
+        "two-stream step differs from the plain sequence of calls"
+    del got, one, dropin
 
     # ---- clock settle (fixed, whatever --warmup says), W warm-up steps, then the timed region ----
     t_settle = time.perf_counter()
