@@ -4,19 +4,23 @@
 One *step* is one sparse pass of a FLUX-shaped layer (configs 0-2 of the baseline):
 GEMM-Q over the flagged (token-block, head) tiles -> symbol decode + block-sparse FlashAttention
 -> GEMM-O that adds the non-cached heads to the cached partial.  ``value`` is the effective
-TFLOP/s of that chain, counting only computed blocks / tiles / head slices.
+TFLOP/s of that chain, counting only computed blocks / tiles / head slices, with the decode on a second
+stream beside GEMM-Q (``wrapper.decode()``, then ``run(reuse_decoded=True)``).  The plain sequence of calls
+on one stream, whose ``run()`` at this size takes its rows straight from the packed symbols (another launch
+of the attention kernel, no decode), is timed beside it as ``dropin_call_sequence``.
 
 The JSON line also carries
   * ``kernels``: per-kernel latency and effective TFLOP/s (or GB/s) for every config, each as a
     fraction of the MI355X peak that bounds it,
-  * ``roofline``: the dominant kernel (sparse FlashAttention at the FLUX shape) measured with HIP
-    events on the launch stream,
+  * ``roofline``: the dominant kernel (sparse FlashAttention at the FLUX shape, over the decoded list) measured
+    with HIP events on the launch stream; ``rows_from_symbols`` in it is the launch that a plain ``run()`` makes,
   * ``cpu_baseline``: the fp32 CPU path (the oracle) timed on this box's host cores: the whole FLUX
     layer, and under ``c3`` / ``c4`` a sample of the big configs' attention rows and token blocks
     with the extrapolation to the whole config labelled as such.
 
-Every attention config also carries ``run_dropin``: the reference's call sequence
-``wrapper.run(q, k, v, sparse_info, sparse_kv_info, indptrs)`` with a fresh decode in every call.
+Every attention config also carries ``run_dropin``: the reference's call
+``wrapper.run(q, k, v, sparse_info, sparse_kv_info, indptrs)``, which reads the symbols in every call
+(configs 3 and 4: a decode and the attention launch; config 0: one launch).
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--configs 0,1,2,3,4] [--no-cpu]
 """
@@ -48,16 +52,16 @@ def kernel_source_hash():
         return hashlib.sha256(f.read()).hexdigest()[:16]
 
 
-def traffic_from_profile():
+def traffic_from_profile(launch):
     """HBM bytes per sparse-FA launch at config 0, as recorded in the committed rocprofv3 summary
-    (line ``traffic_bytes_per_launch <kernel> = <bytes>``), and whether that summary was taken from the
+    (line ``traffic_bytes_per_launch <kernel> c0, <launch> = <bytes>``), and whether that summary was taken from the
     kernel source this run uses (line ``kernel_source_sha256 sparse_fa.hip = <first 16 hex digits>``).
     (None, reason) when the summary has no such line or describes another version of the kernel: a
     counter reading of other code is not this run's traffic."""
     value = recorded = None
     try:
         for line in open(TRAFFIC_PROFILE):
-            if line.startswith("traffic_bytes_per_launch sparse_fa_kernel<bf16>"):
+            if line.startswith("traffic_bytes_per_launch sparse_fa_kernel<bf16> c0, %s = " % launch):
                 value = float(line.split("=")[1].split()[0])
             if line.startswith("kernel_source_sha256 sparse_fa.hip"):
                 recorded = line.split("=")[1].split()[0]
@@ -125,10 +129,10 @@ class FluxLayer:
     def decode(self):
         return self.wrapper.decode(self.info, self.kv_info, self.info_ip, self.kv_ip)
 
-    def attention(self, fresh_decode=True):
-        """fresh_decode=False: run the list the last decode() left (ordered after it across streams)."""
+    def attention(self, from_symbols=True):
+        """from_symbols=False: run the list the last decode() left (ordered after it across streams)."""
         return self.wrapper.run(self.q, self.k, self.v, self.info, self.kv_info, self.info_ip,
-                                self.kv_ip, out=self.out_fa, reuse_decoded=not fresh_decode)
+                                self.kv_ip, out=self.out_fa, reuse_decoded=not from_symbols)
 
     def gemm_o_cache(self):
         return self.fo.flashomni_gemm_reduction(self.a, self.wo, 24, self.info, self.info_ip, 0,
@@ -148,22 +152,22 @@ class FluxLayer:
             self.decode()               # a fresh decode every step
         self.gemm_q()
         cur.wait_stream(self.side)
-        self.attention(fresh_decode=False)
+        self.attention(from_symbols=False)
         return self.gemm_o_final()
 
     def step_one_stream(self):
         """The same calls one after the other on one stream."""
         self.gemm_q()
         self.decode()
-        self.attention(fresh_decode=False)
+        self.attention(from_symbols=False)
         return self.gemm_o_final()
 
     def step_dropin(self):
         """The same pass as the reference's call sequence on one stream: flashomni_gemm, then
-        wrapper.run(q, k, v, symbols...) (which decodes the symbols itself), then
+        wrapper.run(q, k, v, symbols...) (which takes its rows from the symbols itself), then
         flashomni_gemm_reduction."""
         self.gemm_q()
-        self.attention(fresh_decode=True)
+        self.attention()
         return self.gemm_o_final()
 
     def chain_flops(self):
@@ -572,7 +576,7 @@ def main():
     value = chain_flops / (ms_per_step * 1e-3) / 1e12
     log("[bench] chain %.4f ms/step -> %.1f TFLOP/s" % (ms_per_step, value))
 
-    # ---- the reference's call sequence on one stream (the decode inside run(), nothing overlapped) ----
+    # ---- the reference's call sequence on one stream (rows from the symbols inside run(), nothing overlapped) ----
     for _ in range(W):
         layer.step_dropin()
     torch.cuda.synchronize()
@@ -603,15 +607,17 @@ def main():
     c0 = {}
     # (the attention launch first, straight after the step loop: the decoder's 17 us launches in between
     # would let the clocks fall back)
-    fa_ms = time_gpu(lambda: layer.attention(fresh_decode=False), KK, WW)
+    fa_ms = time_gpu(lambda: layer.attention(from_symbols=False), KK, WW)
     ms = time_gpu(layer.decode, KK, WW)
     rows, nnz = layer.wrapper._worklist.sizes()
     c0["decode"] = entry(ms, nbytes=w0.packed_info.numel() + w0.packed_kv_info.numel() + 4 * (4 * rows + 1 + nnz))
     c0["decode"]["rows"], c0["decode"]["kv_blocks"] = rows, nnz
     c0["sparse_fa_bf16"] = entry(fa_ms, flops=w0.attention_flops())
     c0["sparse_fa_bf16"]["computed_blocks"] = w0.computed_blocks
-    # the call a user of the reference makes: decode of the symbols + attention, every time
-    c0["run_dropin"] = entry(time_gpu(lambda: layer.attention(fresh_decode=True), KK, WW), flops=w0.attention_flops())
+    # the call a user of the reference makes (at this size one launch, rows from the symbols)
+    run_ms = time_gpu(layer.attention, KK, WW)
+    c0["run_dropin"] = entry(run_ms, flops=w0.attention_flops())
+    layer.decode()                  # (the layer is left with a decoded list)
     kernels[w0.shape.name] = c0
     ms = time_gpu(layer.gemm_q, KK, WW)
     kernels[layer.w1.shape.name] = {"gemm_q": entry(ms, flops=layer.w1.gemm_q_flops())}
@@ -671,9 +677,10 @@ def main():
     kernel_sum_ms = (kernels[layer.w1.shape.name]["gemm_q"]["ms"] + fa_ms
                      + kernels[layer.w2.shape.name]["gemm_o_final"]["ms"])
     fa_flops = w0.attention_flops()
-    traffic, traffic_state = traffic_from_profile()
+    traffic, traffic_state = traffic_from_profile("decoded list")
+    run_traffic, run_traffic_state = traffic_from_profile("rows from symbols")
     roofline = {
-        "kernel": "sparse_fa_kernel<bf16> (config 0, FLUX shape)", "bound": "mfma",
+        "kernel": "sparse_fa_kernel<bf16> (config 0, FLUX shape, decoded list)", "bound": "mfma",
         "achieved": round(fa_flops / (fa_ms * 1e-3) / 1e12, 2), "peak": PEAK_BF16, "unit": "TFLOP/s",
         "frac": round(fa_flops / (fa_ms * 1e-3) / 1e12 / PEAK_BF16, 4),
         # HBM bytes per launch: read from the committed summary of two rocprofv3 --pmc runs of this
@@ -682,6 +689,11 @@ def main():
         "traffic": traffic, "traffic_state": traffic_state, "traffic_unit": "bytes/launch",
         "traffic_source": "profiles/" + os.path.basename(TRAFFIC_PROFILE),
         "launch_ms": round(fa_ms, 5), "algorithmic_flop_per_launch": fa_flops,
+        # the same attention as a plain run() launches it (timed with the call's host side, as a user calls it)
+        "rows_from_symbols": {
+            "achieved": round(fa_flops / (run_ms * 1e-3) / 1e12, 2),
+            "frac": round(fa_flops / (run_ms * 1e-3) / 1e12 / PEAK_BF16, 4),
+            "traffic": run_traffic, "traffic_state": run_traffic_state, "launch_ms": round(run_ms, 5)},
     }
     cpu = None
     if not args.no_cpu:
@@ -698,7 +710,8 @@ def main():
         "dropin_call_sequence": {
             "ms_per_step": round(dropin_ms, 5), "tflops": round(chain_flops / (dropin_ms * 1e-3) / 1e12, 2),
             "note": "flashomni_gemm -> wrapper.run(q, k, v, symbols) -> flashomni_gemm_reduction on one stream, "
-                    "the decode inside run(); `value` overlaps the decode with GEMM-Q on a second stream"},
+                    "whose run() takes its rows from the symbols without a decode; `value` decodes a list beside GEMM-Q "
+                    "on a second stream and runs that"},
         "captured_graph": {"error": graph_error} if graph_ms is None else {
             "ms_per_step": round(graph_ms, 5), "tflops": round(chain_flops / (graph_ms * 1e-3) / 1e12, 2),
             "note": "the same two-stream step replayed as one HIP graph; `value` is the eager step"},
