@@ -159,12 +159,12 @@ struct FaParams {
   const int32_t* blk_qb;
   int32_t n_blk, batch, symbol_heads, is_full;
   int32_t zero_skipped;  // `o` is fresh: the rows of q blocks that are not computed are cleared
-  // copy of the symbols for a later decode of the same rows (or null): bytes, and the two indptrs
+  // copy of the symbols for a later decode of the same rows (or null): bytes, and the two indptrs; keep_indptr
+  // also where every bit counts as set (no copy): the launch marks sched[kSchedKept]
   uint8_t* keep_info;
   uint8_t* keep_kv_info;
   int32_t* keep_indptr;
   int32_t info_bytes, kv_info_bytes;
-  int32_t mark;  // value for sched[kSchedKept], or 0: the word stays
 };
 
 template <typename T>
@@ -870,7 +870,7 @@ sparse_fa_kernel(const FaParams p) {
         p.keep_indptr[p.batch + 1 + i] = p.kv_info_indptr[i];
       }
     }
-    if (p.mark != 0 && blockIdx.x == 0 && tid == 0) p.sched[kSchedKept] = p.mark;
+    if (p.keep_indptr != nullptr && blockIdx.x == 0 && tid == 0) p.sched[kSchedKept] = p.is_full ? 2 : 1;
     direct_schedule();
     if (wv == 0) {
       if (lane == 0) s_share[0] = 0;
@@ -2222,10 +2222,10 @@ extern "C" int fo_sparse_attention_direct(const void* args) {
   p.zero_skipped = a.zero_skipped && !a.is_full;
   if (!a.is_full && (a.keep_info || a.keep_kv_info || a.keep_indptr)) {
     FO_REQUIRE(a.keep_info && a.keep_kv_info && a.keep_indptr, "sparse_attention: null pointer");
-    p.keep_info = a.keep_info; p.keep_kv_info = a.keep_kv_info; p.keep_indptr = a.keep_indptr;
+    p.keep_info = a.keep_info; p.keep_kv_info = a.keep_kv_info;
     p.info_bytes = a.info_bytes; p.kv_info_bytes = a.kv_info_bytes;
   }
-  p.mark = a.keep_indptr == nullptr ? 0 : a.is_full ? 2 : 1;
+  p.keep_indptr = a.keep_indptr;
   hipStream_t s = static_cast<hipStream_t>(a.stream);
   const bool bf16 = a.dtype == FO_BF16;
   if (a.logits_soft_cap > 0.f) {
