@@ -156,6 +156,9 @@ class PlannedBatch:
         return self.tables.narrow(0, self._table_at[(0, 1, 4, 5, 6, 7, 2, 3)[i]],
                                   self.batch_size + 1 if i < 6 else max(self.n_q_blk, 1))
 
+    def _address(self, i: int) -> int:
+        return self.tables.data_ptr() + 4 * self._table_at[(0, 1, 4, 5, 6, 7, 2, 3)[i]]
+
     blk_req = property(lambda self: self.table(6))
     blk_qb = property(lambda self: self.table(7))
     q_blk_base = property(lambda self: self.table(2))
@@ -202,22 +205,22 @@ class PlannedBatch:
         with _lib.device_guard(self.device):
             _lib.check(_lib.lib().fo_decode_sparse(
                 _lib.ptr(tensors[0]), _lib.ptr(tensors[1]), _lib.ptr(tensors[2]), _lib.ptr(tensors[3]),
-                _lib.ptr(self.blk_req), _lib.ptr(self.blk_qb), _lib.ptr(self.kv_indptr),
+                self._address(6), self._address(7), _lib.ptr(self.kv_indptr),
                 self.n_q_blk, self.symbol_heads, self.block_kv, int(bool(is_full)),
                 _lib.ptr(wl.row_req), _lib.ptr(wl.row_qb), _lib.ptr(wl.row_head), _lib.ptr(wl.kv_row_ptr),
                 _lib.ptr(wl.kv_idx), _lib.ptr(wl.counts), _lib.ptr(wl.order), _lib.ptr(wl.sched),
                 _lib.ptr(wl.scratch), _lib.ptr(wl.shares if self.split_ok else None),
                 stream.cuda_stream))
-        self._note_list(is_full)
+        self._note_list(is_full, stream)
         return wl
 
-    def _note_list(self, is_full):
-        """A list has been decoded on the current stream."""
+    def _note_list(self, is_full, stream):
+        """A list has been decoded on the (current) stream."""
         _lib.native().note_list(self.native, is_full)
-        if not torch.cuda.is_current_stream_capturing():
+        if not self.native.recording:
             # remembered for reuse_decoded: which stream the list was decoded on (a run on another stream must be
             # ordered after it)
-            self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
+            self.decoded = (bool(is_full), stream, [])
 
     def attention(self, q, k, v, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full,
                   out, lse, return_lse, sm_scale, logits_soft_cap, hnd, qo_indptr=None, kv_indptr=None):
@@ -234,7 +237,7 @@ class PlannedBatch:
                 qo_indptr, kv_indptr)
             if r is False:
                 wl = self.worklist
-        if r is not None and self.native.state == 0 and not torch.cuda.is_current_stream_capturing():
+        if r is not None and self.native.state == 0 and not self.native.recording:
             self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
         return r
 
@@ -254,16 +257,16 @@ class PlannedBatch:
             if source == 1:
                 self.decode(info, kv_info, info_ip, kv_ip, full)
             else:
-                wl = self.worklist
+                wl, stream = self.worklist, torch.cuda.current_stream(self.device)
                 with _lib.device_guard(self.device):
                     _lib.check(_lib.lib().fo_decode_sparse_kept(
-                        _lib.ptr(info), _lib.ptr(kv_info), _lib.ptr(info_ip), _lib.ptr(kv_ip), _lib.ptr(self.blk_req),
-                        _lib.ptr(self.blk_qb), _lib.ptr(self.kv_indptr), self.n_q_blk, self.symbol_heads, self.block_kv,
+                        _lib.ptr(info), _lib.ptr(kv_info), _lib.ptr(info_ip), _lib.ptr(kv_ip), self._address(6),
+                        self._address(7), _lib.ptr(self.kv_indptr), self.n_q_blk, self.symbol_heads, self.block_kv,
                         _lib.ptr(wl.row_req), _lib.ptr(wl.row_qb), _lib.ptr(wl.row_head), _lib.ptr(wl.kv_row_ptr),
                         _lib.ptr(wl.kv_idx), _lib.ptr(wl.counts), _lib.ptr(wl.order), _lib.ptr(wl.sched),
                         _lib.ptr(wl.scratch), _lib.ptr(wl.shares if self.split_ok else None),
-                        _lib.current_stream(self.device)))
-                self._note_list(full)
+                        stream.cuda_stream))
+                self._note_list(full, stream)
         elif self.decoded is not None:
             self._follow_list()
         return self.worklist
@@ -362,8 +365,8 @@ class PlannedBatch:
                 _lib.dtype_code(q.dtype), _lib.ptr(q_lo), _lib.ptr(k_lo), _lib.ptr(q_scale if fp8 else None),
                 _lib.ptr(k_scale if fp8 else None),
                 q.stride(0), q.stride(1), k_sn, k_sh, v_sn, v_sh, out.stride(0), out.stride(1),
-                _lib.ptr(self.qo_indptr), _lib.ptr(self.kv_indptr), _lib.ptr(self.q_blk_base),
-                _lib.ptr(self.kv_blk_base), self.n_q_blk, self.n_kv_blk, _lib.ptr(wl.row_req),
+                _lib.ptr(self.qo_indptr), _lib.ptr(self.kv_indptr), self._address(2),
+                self._address(3), self.n_q_blk, self.n_kv_blk, _lib.ptr(wl.row_req),
                 _lib.ptr(wl.row_qb), _lib.ptr(wl.row_head), _lib.ptr(wl.kv_row_ptr), _lib.ptr(wl.kv_idx),
                 _lib.ptr(wl.order), _lib.ptr(wl.sched), self.max_rows, q.size(1), self.num_kv_heads,
                 int(self.gqa_packed), q.size(2), self.block_q, self.block_kv, float(sm_scale),

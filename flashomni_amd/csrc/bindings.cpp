@@ -304,7 +304,8 @@ struct Plan {
   // (`captured`), whether the list or the kept symbols are newer is read on the device (sched[33]).
   // listed_in: the capture whose last launch on this plan was a decode; recorded_in, recorded_full: the last
   // capture that recorded a decode or run, and its is_full.
-  int captured, recorded_full;
+  // recording: the last launch was recorded.
+  int captured, recorded_full, recording;
   unsigned long long listed_in, recorded_in;
   // The copy lies behind the tables, in one place for as long as the plan lives (a graph writes it at every
   // replay): room for the symbols that such a run takes, at keep_at[0] info, [1] kv_info, [2] the indptrs (bytes
@@ -345,7 +346,9 @@ unsigned long long capture_of(hipStream_t stream) {
 
 // A launch that leaves a list (state 0) or takes rows without one (1, 2) has been queued on the stream.
 void note(Plan* p, hipStream_t stream, int state, bool full) {
-  if (const unsigned long long id = capture_of(stream)) {
+  const unsigned long long id = capture_of(stream);
+  p->recording = id != 0;
+  if (id) {
     p->captured = 1;
     p->recorded_in = id;
     p->recorded_full = full;
@@ -1002,6 +1005,7 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods
 
 PyMemberDef g_plan_members[] = {{"state", T_INT, offsetof(Plan, state), 0, nullptr},
                                 {"recorded_in", T_ULONGLONG, offsetof(Plan, recorded_in), 0, nullptr},
+                                {"recording", T_INT, offsetof(Plan, recording), READONLY, nullptr},
                                 {"recorded_full", T_INT, offsetof(Plan, recorded_full), READONLY, nullptr},
                                 {"sched_at", T_LONGLONG, offsetof(Plan, z.sched), READONLY, nullptr},
                                 {nullptr, 0, 0, 0, nullptr}};

@@ -125,7 +125,8 @@ extern "C" int fo_plan_batch(const int32_t* qo, const int32_t* kv, int32_t batch
   }
   z.blk_req = at;
   z.blk_qb = at + std::max<int64_t>(z.n_q_blocks, 1);
-  z.sched = z.blk_qb + std::max<int64_t>(z.n_q_blocks, 1);
+  // (lines of its own: the launches' device-wide atomics on it would drop the tables from the caches)
+  z.sched = (z.blk_qb + std::max<int64_t>(z.n_q_blocks, 1) + 63) / 64 * 64;
   z.table_ints = z.sched + kSchedInts;
   std::memcpy(sizes, &z, sizeof(z));
   return FO_OK;
