@@ -17,6 +17,7 @@
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
+#include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -488,6 +489,7 @@ hipError_t enter(Plan* p) {
     p->complete = wait_word(p->word);
     return p->complete ? hipSuccess : hipErrorNotReady;
   }
+  const c10::hip::HIPGuard device(static_cast<c10::DeviceIndex>(p->dev));  // (whose default stream is meant)
   c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);  // (this thread or another is capturing)
   if (!p->behind) {
     hipError_t e = hipEventCreateWithFlags(&p->behind, hipEventDisableTiming);
@@ -685,6 +687,7 @@ PyObject* follow_run(PyObject*, PyObject* arg) {
     PyErr_SetString(PyExc_RuntimeError, "the stream of the last run() is being captured: its list cannot be reused on another");
     return nullptr;
   }
+  const c10::hip::HIPGuard device(static_cast<c10::DeviceIndex>(p->dev));  // (whose default stream is meant)
   hipEvent_t ev;
   hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
   if (e != hipSuccess) return raise_hip(e);
