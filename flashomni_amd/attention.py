@@ -4,12 +4,15 @@ The public surface (constructor, ``plan``, ``run``, ``run_return_lse``, the depr
 ``forward*`` aliases, defaults and error types) is that of the reference
 (flashomni/attention.py:194-869).  Behind it:
 
-* ``plan()`` runs the host planner (fo_prefill_plan) into the wrapper's integer workspace, builds
-  the q-block table and sizes the work-list buffers;
-* ``run()`` first decodes the bit-packed symbols into a compacted work list on the GPU
-  (fo_decode_sparse, every call: the symbol buffers may have been rewritten in place by writers
-  torch does not see; ``reuse_decoded=True`` skips it on the caller's word) and then launches the
-  sparse FlashAttention kernel over that list (fo_sparse_fa_run).
+* ``plan()`` runs the host planner (fo_prefill_plan) into the wrapper's integer workspace, queues
+  the launch that builds the batch's tables, and sizes the work list.  It does not wait: the first
+  use on another stream does;
+* ``run()`` reads the bit-packed symbols on every call (the buffers may have been rewritten in place
+  by writers torch does not see).  Up to 1024 (q block, head) pairs the attention launch takes its
+  rows straight from them (fo_sparse_attention_direct) and keeps a copy; above, and for fp8, they
+  are decoded into a compacted work list (fo_decode_sparse) that the sparse FlashAttention kernel
+  runs over (fo_sparse_fa_run).  ``reuse_decoded=True`` runs the last list on the caller's word,
+  decoding the kept symbols first where that is still to do.
 
 Of the options the reference's shipped build supports (setup.py:30-38, :98-111) head_dim 128 and the
 logits soft cap are implemented: no causal / custom mask, no positional encoding, fp32 logits.
@@ -391,6 +394,11 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
     are left untouched), ``sparse_kv_info`` one bit per (q-block, head, kv-block) (1 = keep), both
     packed little-endian per request; the two indptr tensors are the byte offsets returned by
     ``segment_packbits``.
+
+    The float workspace receives the partial results of rows that are cut for several workgroups
+    (lists of up to 1024 (q block, head) pairs, and decoded ones of up to two rows per CU), so runs
+    that share one, of one wrapper or of several, must not overlap in time: give wrappers that run on
+    different streams a workspace each, or order the streams.
     """
 
     def __init__(
@@ -498,7 +506,8 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         counterpart in the reference).  The host planner tiles the batch into the
         integer workspace; in addition the q-block table of the symbol decoder is built and the
         work-list buffers are sized for the worst case (every bit set).  Cannot be captured in a
-        graph (it copies the indptrs to the host)."""
+        graph (it copies the indptrs to the host), and ends the use of graphs that hold runs of the
+        earlier plan, whose tables go with it."""
         q_data_type = canonicalize_torch_dtype(q_data_type)
         if kv_data_type is None:
             kv_data_type = q_data_type

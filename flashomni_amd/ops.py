@@ -11,7 +11,8 @@ The attention pair needs state the reference's signatures have no slot for (the 
 table and the work-list buffers).  ``batch_sparseFA_with_kv_plan`` builds it and files it under the
 address of the integer workspace it was given; ``batch_sparseFA_with_ragged_kv_run`` finds it there,
 as the reference's run finds its tile arrays inside that workspace.  plan() allocates (it is not
-part of a captured graph in the reference either, flashomni/attention.py:140-141); run() does not.
+part of a captured graph in the reference either, flashomni/attention.py:140-141); run() allocates the
+work list when a plan first needs one (more than 1024 (q block, head) pairs).
 """
 import collections
 import weakref
