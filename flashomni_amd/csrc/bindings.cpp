@@ -213,11 +213,10 @@ PyObject* gemm_o(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ---- attention -----------------------------------------------------------------------------------
-// What plan() derives from a batch: sizes, and one int32 tensor on the device that holds every table
-// (see fo_plan_tables).
-// A word of pinned memory that a plan's launch leaves its ticket in (not on the default stream, see Plan).  Tickets ascend and a word is handed out
-// again only when its ticket is there, so that a word and a ticket stay comparable after that.  There are as many
-// as plans have ever been alive or under way at a time, in pages of 512 (guarded by the interpreter's lock).
+// A word of pinned memory that a plan's launch leaves its ticket in (not on the default stream, see Plan).
+// Tickets ascend and a word is handed out again only when its ticket is there, so that a word and a ticket stay
+// comparable after that.  There are as many as plans have ever been alive or under way at a time, in pages of
+// 512 (guarded by the interpreter's lock).
 struct Word {
   uint64_t* at;
   uint32_t ticket;
@@ -247,6 +246,11 @@ bool take_word(Word* w) {
   w->ticket = ++g_plan_ticket;
   __atomic_store_n(w->at, static_cast<uint64_t>(w->ticket - 1) << 32, __ATOMIC_RELEASE);
   return true;
+}
+
+// no launch will write it
+void settle_word(const Word& w) {
+  if (w.at) __atomic_store_n(w.at, static_cast<uint64_t>(w.ticket) << 32, __ATOMIC_RELEASE);
 }
 
 void give_word(const Word& w) {
@@ -280,6 +284,8 @@ hipError_t host_wait(hipEvent_t event) {
   return e;
 }
 
+// What plan() derives from a batch: sizes, and one int32 tensor on the device that holds every table
+// (see fo_plan_tables).
 struct Plan {
   PyObject_HEAD
   Tensor tables;
@@ -546,7 +552,8 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   int64_t hq, hkv, dev, sent;
   if (!(n == 12 && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
         whole(args[3], &hkv) && whole(args[5], &dev) && whole(args[8], &sent) && opt_tensor(args[9], &iws) &&
-        opt_tensor(args[10], &pin) && (sent == 0 || (iws && pin && Py_TYPE(args[11]) == g_ring_type)) && opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
+        opt_tensor(args[10], &pin) && (sent == 0 || (iws && pin && Py_TYPE(args[11]) == g_ring_type)) &&
+        opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
         qo->scalar_type() == at::kInt && kv->scalar_type() == at::kInt && qo->is_contiguous() && kv->is_contiguous() &&
         qo->is_cpu() && kv->is_cpu() && qo->numel() == kv->numel() && qo->numel() >= 1)) {
     PyErr_SetString(PyExc_RuntimeError, "plan: bad argument");
@@ -605,6 +612,7 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
         e = hipMemcpyAsync(iws->data_ptr(), host, sent, hipMemcpyHostToDevice, home);
       }
       if (e != hipSuccess) {
+        settle_word(p->word);
         Py_DECREF(self);
         PyErr_Format(PyExc_RuntimeError, "the copy into the integer workspace failed: %s", hipGetErrorString(e));
         return nullptr;
@@ -612,8 +620,12 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     rc = fo_plan_tables_signal(qo->data_ptr<int32_t>(), kv->data_ptr<int32_t>(), batch, hq, hkv, packed,
                                p->tables.data_ptr<int32_t>(), p->word.at, p->word.ticket, p->home);
-    if (rc) (void)hipStreamSynchronize(home);  // (no word to wait for)
-    else if (ring) ring_note(ring, static_cast<size_t>(sent) > mirror / 2, home, p->word);
+    if (rc) {
+      (void)hipStreamSynchronize(home);  // (the copy has no word to be waited for by)
+      settle_word(p->word);
+    } else if (ring) {
+      ring_note(ring, static_cast<size_t>(sent) > mirror / 2, home, p->word);
+    }
   } catch (...) {
     Py_DECREF(self);
     throw;

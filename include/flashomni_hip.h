@@ -303,7 +303,8 @@ int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float
  * candidates, more than 2^20 keep bits, no split workspace of fo_sparse_fa_split_workspace_bytes() bytes.
  * Arguments as in fo_decode_sparse (symbols, blk_req, blk_qb, is_full; n_blk symbol rows of symbol_heads
  * heads) and fo_sparse_fa_run.  sched: 1024 int32, its words [64, 576) zero before the first launch and left
- * zero by every one (it may be the sched of a decoded list).  A workgroup lists at most 4096 kv blocks of a row, as in fo_sparse_fa_run.
+ * zero by every one (it may be the sched of a decoded list).  A workgroup lists at most 4096 kv blocks of a
+ * row, as in fo_sparse_fa_run.
  * zero_skipped: the rows of q blocks that are not computed are cleared in o.  keep_info,
  * keep_kv_info, keep_indptr (optional): receive the info_bytes / kv_info_bytes of symbols and the two
  * indptrs ([2 * (batch + 1)]) that this launch read, for a decode of the same list later; with keep_indptr (also

@@ -212,3 +212,39 @@ def test_plans_beyond_the_pinned_mirror(dev, stream, capturing):
     for i, (info, got) in enumerate(zip(seen, copies.cpu())):
         assert info == exp[i % 3][0]
         assert arrays(info, got, batches[i % 3]) == exp[i % 3][1], i
+
+
+@pytest.mark.parametrize("lens", [[5] * 401, [128 * 3000 - 7, 1], [700]])   # copied; several workgroups; one
+@pytest.mark.parametrize("capturing", [False, True])
+def test_tables_read_from_another_stream(dev, lens, capturing):
+    """The tables of a plan queued on a busy side stream, read from another stream, also while the planning stream
+    is being captured (then the host waits for the launch's word)."""
+    import flashomni_amd as fo
+    qo = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    kv = torch.arange(len(lens) + 1, dtype=torch.int32) * 64
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(256 << 20, dtype=torch.uint8, device=dev))
+    side = torch.cuda.Stream(device=dev)
+    torch.cuda.synchronize(dev)
+    with torch.cuda.stream(side):
+        busy = torch.empty(1 << 30, dtype=torch.uint8, device=dev)
+        for i in range(20):
+            busy.fill_(i)
+        w.plan(qo, kv, 2, 2, 128, q_data_type=torch.bfloat16)
+    got = [torch.empty_like(w._planned.tables) for _ in range(2)]
+    graph = torch.cuda.CUDAGraph()
+    if capturing:
+        with torch.cuda.stream(side):
+            graph.capture_begin(capture_error_mode="relaxed")
+    w._planned.table(0)
+    got[0].copy_(w._planned.tables)
+    if capturing:
+        with torch.cuda.stream(side):
+            got[1].copy_(w._planned.tables)
+            graph.capture_end()
+    torch.cuda.synchronize(dev)
+    rows = -(-np.asarray(lens) // 128)
+    at = w._planned._table_at
+    exp = {0: qo.numpy(), 1: kv.numpy(), 2: np.repeat(np.arange(len(lens)), rows),
+           3: np.concatenate([np.arange(r) for r in rows])}
+    for i, e in exp.items():
+        np.testing.assert_array_equal(got[0][at[i]:at[i] + len(e)].cpu().numpy(), e, err_msg=str(i))
