@@ -27,9 +27,9 @@
 // makes both the row-wise 128-bit K reads (16 consecutive rows, one chunk column) and the 4-row
 // transpose reads of V (4 rows x 4 chunks) hit every bank exactly once.
 //
-// Work distribution: workgroups are persistent and pop rows from 8 queues (one per XCD, chosen by
-// blockIdx % 8) that the decoder filled head by head, so one XCD's L2 serves a few heads' K/V; an
-// idle XCD steals from its neighbours.  The last workgroup to finish resets the queue cursors.
+// Work distribution: workgroups are persistent and take rows from 8 queues (one per XCD, chosen by
+// blockIdx % 8) that the decoder filled head by head, so one XCD's L2 serves a few heads' K/V; the
+// first row by their index, further ones from the queue's cursor; an idle XCD steals from its neighbours.  The last workgroup to finish resets the queue cursors.
 // When a queue is so short that half of its XCD's workgroups would stay idle, its positions stand
 // for parts of rows (ranges of a row's kv blocks): parts publish unnormalised partial results to
 // the caller's workspace and the last one to arrive combines them (see the end of the row loop).
@@ -269,21 +269,46 @@ __device__ __forceinline__ void load_pair_device(const float* p, float& a, float
   b = __uint_as_float(static_cast<uint32_t>(v >> 32));
 }
 
-// Pop the next row for this workgroup from the queues: own XCD queue first, then the neighbours'.
-// `first` is the first queue that may still hold rows: a queue found empty stays empty for the rest
-// of the launch, so it is not asked again.  `q` is the launch's copy of the queue bounds: the pop
-// itself is one atomic.  Returns the entry's position in `order` or -1.
-__device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q, int* first) {
-  for (int a = *first; a < kXcds; ++a) {
-    const int x = (xcd + a) & (kXcds - 1);
-    const int beg = q[x], end = q[x + 1];
-    if (beg < end) {
-      const int pos = beg + atomicAdd(&p.sched[16 + x], 1);
-      if (pos < end) {
-        *first = a;
-        return pos;
+// Pop the next row for this workgroup from the queues, by one whole wavefront: own XCD queue first, then the
+// neighbours'.  A queue's first rows belong to the workgroups of its XCD by their index and are taken without an
+// atomic (see fetch_next); the cursor counts the positions behind them.  `first` is the queue that this
+// workgroup took its last row from.  When that one is empty all eight cursors are looked at with one load, and
+// only a queue that still holds rows is asked: the cursors share a cache line, whose atomics are carried out one
+// after the other (512 workgroups asking the other seven queues in turn took some 40 us at the end of a launch
+// whose workgroups end together: 512 rows of 8 kv blocks 89 -> 41 us, 1536 rows 153 -> 131; 256 workgroups, 512
+// rows 53 -> 46).  `q` is the launch's copy of the queue bounds.  Returns the entry's position in `order` or -1.
+__device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q, int* first, int lane) {
+  // (rows of queue x that belong to its workgroups from the start)
+  auto dealt = [&](int x) { return static_cast<int>(gridDim.x + kXcds - 1 - x) / kXcds; };
+  int a = __builtin_amdgcn_readfirstlane(*first);
+  unsigned left = a < kXcds ? 1u << a : 0u;  // queues to ask, by distance from the own one
+  for (bool looked = false;;) {
+    while (left) {
+      a = __ffs(left) - 1;
+      left &= left - 1;
+      const int x = (xcd + a) & (kXcds - 1);
+      const int beg = __builtin_amdgcn_readfirstlane(q[x]) + dealt(x), end = __builtin_amdgcn_readfirstlane(q[x + 1]);
+      if (beg < end) {
+        int pos = 0;
+        if (lane == 0) pos = atomicAdd(&p.sched[16 + x], 1);
+        pos = beg + __builtin_amdgcn_readfirstlane(pos);
+        if (pos < end) {
+          *first = a;
+          return pos;
+        }
       }
     }
+    if (looked || a >= kXcds) break;
+    looked = true;
+    bool some = false;
+    if (lane < kXcds) {
+      const int x = (xcd + lane) & (kXcds - 1);
+      const int beg = q[x] + dealt(x), end = q[x + 1];
+      // (a cursor only grows: a queue seen empty stays empty)
+      if (beg < end)
+        some = beg + __hip_atomic_load(&p.sched[16 + x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < end;
+    }
+    left = static_cast<unsigned>(__ballot(some));
   }
   *first = kXcds;
   return -1;
@@ -449,7 +474,6 @@ sparse_fa_kernel(const FaParams p) {
   if constexpr (!kDirect) {
     if (tid < 9) s_queue[tid] = p.sched[tid];
     if (tid >= 64 && tid < 64 + 6) s_queue[9 + tid - 64] = p.sched[kSchedEven + tid - 64];
-    if (tid == 128) s_guess = 0;
     __syncthreads();
   }
   // Even shares: the decoder has laid the rows out head by head and given every row a cost
@@ -509,11 +533,11 @@ sparse_fa_kernel(const FaParams p) {
     }
   };
   const bool have_records = queue_word(14) != 0 && p.shares != nullptr;
-  int first_queue = 0;  // kept by the popping lane (the first pop is lane 0's, the others lane 256's)
+  int first_queue = 0;  // kept by the popping wavefront
   // One wavefront: lane 0 takes the next item (even shares: from the gathered records; otherwise it
   // pops a row and gathers its metadata, two rounds of loads), then all lanes copy the row's kv
   // block list; both go to LDS for the whole workgroup.
-  auto fetch_next = [&](int slot_idx) {
+  auto fetch_next = [&](int slot_idx, bool dealt) {
     slot_idx = __builtin_amdgcn_readfirstlane(slot_idx);
     const int lane = fresh_lane();
     RowInfo ri;
@@ -529,20 +553,23 @@ sparse_fa_kernel(const FaParams p) {
         s_next_row[slot_idx] = ri;
       }
     } else {
-      // Queues.  The trips to memory are kept to two: the pop's atomic travels together with loads of
-      // the 64 records that follow this workgroup's last position in the queue (the 32 workgroups of an
-      // XCD pop about once per row each, so the answer is nearly always one of them; otherwise the
-      // record is read after the pop), and the row's bounds and its kv block list are asked for
-      // together once the record is known.
+      // Queues.  A workgroup's first row is the one of its XCD's queue at its own index (its record is asked
+      // for straight away), the others are popped.  The trips to memory are kept to two: the pop's atomic
+      // travels together with loads of the 64 records that follow this workgroup's last position in the
+      // queue (the 32 workgroups of an XCD pop about once per row each, so the answer is nearly always one
+      // of them; otherwise the record is read after the pop), and the row's bounds and its kv block list
+      // are asked for together once the record is known.
       typedef __attribute__((ext_vector_type(4))) int i32x4;
       const int xcd = blockIdx.x & (kXcds - 1);
+      const int own = queue_word(xcd) + static_cast<int>(blockIdx.x / kXcds);
+      dealt = dealt && own < queue_word(xcd + 1);
       i32x4 w0 = {0, 0, 0, 0}, w1 = w0;  // lane i: the record at queue position win_lo + i
       int win_lo = 0, win_hi = 0;
       if (have_records) {
         const int fq = __builtin_amdgcn_readfirstlane(first_queue);
         if (fq < kXcds) {
           const int x = (xcd + fq) & (kXcds - 1);
-          win_lo = max(queue_word(x), __builtin_amdgcn_readfirstlane(s_guess));
+          win_lo = dealt ? own : max(queue_word(x), __builtin_amdgcn_readfirstlane(s_guess));
           win_hi = min(queue_word(x + 1), win_lo + 64);
           if (win_lo + lane < win_hi) {
             const i32x4* rec = reinterpret_cast<const i32x4*>(p.shares + kMaxShares + kRecordInts * static_cast<int64_t>(win_lo + lane));
@@ -551,9 +578,7 @@ sparse_fa_kernel(const FaParams p) {
           }
         }
       }
-      int at_lane = -1;
-      if (lane == 0) at_lane = pop_row(p, xcd, s_queue, &first_queue);
-      const int at = __builtin_amdgcn_readfirstlane(at_lane);
+      const int at = dealt ? own : pop_row(p, xcd, s_queue, &first_queue, lane);
       ri.part = 0;
       ri.parts = 1;
       ri.slot = 0;
@@ -614,7 +639,7 @@ sparse_fa_kernel(const FaParams p) {
       }
       if (lane == 0) {
         s_next_row[slot_idx] = ri;
-        if (at >= 0) s_guess = at + 1;
+        s_guess = at + 1;
       }
     }
     if (even && __builtin_amdgcn_readfirstlane(ri.row) >= 0) {
@@ -886,7 +911,7 @@ sparse_fa_kernel(const FaParams p) {
         if (lane == 0) s_share[0] = 0;
         fill_items(0);
       }
-      fetch_next(0);
+      fetch_next(0, true);
     }
   }
   for (int row_it = 0;; ++row_it) {
@@ -949,7 +974,7 @@ sparse_fa_kernel(const FaParams p) {
         if (p.lse && g_p == 0) p.lse[q_tok * p.num_heads + my_head] = kNegInf;
       }
       if (wv == kFetchWave) {
-        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1);
+        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1, false);
       }
       continue;
     }
@@ -1780,7 +1805,7 @@ sparse_fa_kernel(const FaParams p) {
       __syncthreads();
     }
     if (wv == kFetchWave) {
-        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1);
+        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1, false);
       }
     float m_all = 0.f, d_all = 0.f;  // kv group 0: row maximum and row sum over both groups
     // A lane owns one q row and runs of four d: stored from here, a row would leave as 32 scattered
@@ -2001,8 +2026,9 @@ sparse_fa_kernel(const FaParams p) {
     return;
   }
   // the last workgroup to leave rewinds the queues for the next launch
+  // (every pop's answer has come back by now, so no fence is needed between the atomics; one writes the XCD's L2
+  // back, once per workgroup)
   if (tid == 0) {
-    __threadfence();
     const int done = atomicAdd(&p.sched[24], 1);
     if (done == static_cast<int>(gridDim.x) - 1) {
       for (int x = 0; x < kXcds; ++x) p.sched[16 + x] = 0;

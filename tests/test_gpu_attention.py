@@ -795,3 +795,26 @@ def test_random_batches_all_options(dev, seed):
         if float(exp[touched].float().norm()) > 0:
             assert rel_l2(got[touched], exp[touched]) <= REL_L2
         assert float((lse.cpu()[touched] - exp_lse[touched]).abs().max()) < 2e-2
+
+
+@pytest.mark.parametrize("case", [(1, 1100, 0.9), (1, 1100, 0.05), (3, 400, 0.5), (9, 130, 0.95), (13, 100, 0.002)])
+def test_queues_of_uneven_length(dev, case):
+    """Queues that hold less than their XCD's workgroups take at the start, queues that hold nothing and ones that
+    the other XCDs empty: every row once, and again after the cursors were rewound."""
+    import flashomni_amd as fo
+    heads, blocks, pa = case
+    ql, kl = [blocks * 128 - 5], [200]
+    m = make_ragged_masks(ql, kl, heads, pa, 0.7, seed=heads)
+    g = torch.Generator().manual_seed(heads)
+    q, k, v = (torch.randn(n, heads, 128, generator=g).to(torch.bfloat16) for n in (ql[0], kl[0], kl[0]))
+    t = lambda n: torch.from_numpy(m[n]).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(1 << 20, dtype=torch.uint8, device=dev))   # no room for parts
+    w.plan(t("qo_indptr"), t("kv_indptr"), heads, heads, 128, q_data_type=torch.bfloat16)
+    args = (q.to(dev), k.to(dev), v.to(dev), *(t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")))
+    out0 = sentinel_like(q.shape, torch.bfloat16)
+    exp = oracle.sparse_attention(q, k, v, m["packed_info"], m["packed_keep"], m["info_indptr"], m["keep_indptr"],
+                                  m["qo_indptr"], m["kv_indptr"], out=out0.clone())
+    for reuse in (False, True, True):
+        out = out0.clone().to(dev)
+        w.run(*args, out=out, reuse_decoded=reuse)
+        _check(out.cpu(), exp, out0, m, heads)
