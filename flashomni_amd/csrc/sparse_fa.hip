@@ -108,6 +108,7 @@ constexpr int kXcds = 8;
 constexpr int kMaxRowBlocks = 4096;  // kv blocks of one row held in LDS (512 Ki tokens per request)
 constexpr int kMaxRowBlocksKLo = 2048;  // the same for the two-term k, whose tiles leave less LDS
 constexpr int kMaxRowBlocksOneGroup = 3072;  // and for the one-group form (two workgroups share a CU's LDS)
+constexpr int kMaxRowBlocksOneGroupDirect = 1024;  // where the rows' table is in LDS as well
 constexpr float kLazyLog2 = 8.0f;  // the running max is raised only past a 2^8 overshoot
 // merge area (reuses the tile buffers): O^T of kv group 1, then its (m, d)
 static_assert(kOutTileOff + kOutTileBytes <= Geom<true>::kSmemBytes, "merge area must fit");
@@ -245,7 +246,7 @@ __device__ __forceinline__ float max_across_halves(float x) {
 // sched[33]: 0, or this launch's rows (1: kept symbols, 2: every row) are newer than the decoded list
 constexpr int kSchedEven = 26, kSchedKept = 33, kSchedArrived = 64;
 constexpr int kRecordInts = 8;  // queue entry record: row, request, q block, head, first kv slot, kv count
-constexpr int kMaxShares = 512, kMaxSplitParts = 4, kRowOverhead = 3;
+constexpr int kMaxShares = 512, kRowOverhead = 3, kRowOverheadPipe = 2;
 constexpr int kItemBatch = 16;  // item records of a share gathered at a time
 constexpr int kSplitPartFloats = 128 * 128 + 2 * 256;  // O (fp32) + (max, sum) per lane of kv group 0
 // Partial results live in 2 * kMaxShares areas of the workspace: share j writes the part of a row
@@ -344,6 +345,9 @@ struct DirectMask {
 struct NoMask {};
 constexpr int kDirectMaxCand = 1024;  // candidates (symbol row, head): two per thread of a workgroup
 constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
+constexpr int kDirectMapBytes = (1 << 16) - 16;  // keep bits that are staged in the tile buffers (both forms have as much)
+constexpr int kOlderGain = 10;  // see cut_at
+constexpr int kPartExtra = 2, kEvenExtra = 5;  // what cutting rows costs a workgroup, in kv blocks (see direct_schedule)
 constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologue, epilogue and exchange cost about as many
 
 // T: element type of V, P and O (and of Q, K unless kFp8).  kFp8: Q and K are e4m3fn bytes with one
@@ -373,6 +377,7 @@ sparse_fa_kernel(const FaParams p) {
   static_assert(kQLo || !kKLo, "the two-term k is built on the two-term q");
   static_assert(!kCap || (!kFp8 && !kPipe), "the logits soft cap is built into the two-phase loop for 16-bit operands");
   constexpr int kWaves = 4 * kGroups;
+  constexpr int kShareRowCost = kPipe ? kRowOverheadPipe : kRowOverhead;  // kDirect: what a row costs beside its kv blocks
   constexpr int kFetchWave = kGroups == 2 ? 4 : 0;  // the wavefront that fetches the next item
   using TT = Types<T>;
   using x8 = typename TT::x8;
@@ -400,8 +405,8 @@ sparse_fa_kernel(const FaParams p) {
     }
   };
   // q_begin: first token of the item's q rows; q_rows: how many of its 128 rows exist
-  auto set_q_range = [&](RowInfo& it) {
-    const int q0 = p.qo_indptr[it.req], q1 = p.qo_indptr[it.req + 1];
+  auto set_q_range = [&](RowInfo& it, const int32_t* ends) {
+    const int q0 = ends[0], q1 = ends[1];
     if (kGqaPack) {  // (rows are (token, q head) pairs counted from the request's first token)
       it.q_begin = q0;
       it.q_rows = min(kBlockQ, (q1 - q0) * p.gqa_pack - it.qb * kBlockQ);
@@ -416,7 +421,9 @@ sparse_fa_kernel(const FaParams p) {
   __shared__ int s_share[1];   // even shares: items of this workgroup's share handed out so far
   __shared__ int s_guess;      // queues: one past the position this workgroup popped last
   __shared__ RowInfo s_items[kItemBatch];  // even shares: records of the share's next items
-  constexpr int kRowBlocks = kGroups == 1 ? kMaxRowBlocksOneGroup : kKLo ? kMaxRowBlocksKLo : kMaxRowBlocks;
+  constexpr int kRowBlocks = kGroups == 1 ? (kDirect ? kMaxRowBlocksOneGroupDirect : kMaxRowBlocksOneGroup)
+                             : kKLo       ? kMaxRowBlocksKLo
+                                          : kMaxRowBlocks;
   __shared__ uint16_t s_blk2[2][kRowBlocks];  // kv block list of this row / the next one
   // fp8: the k dequantisation scales of the listed blocks (read per tile: from global memory the
   // compiler would wait for every tile copy in flight along with them)
@@ -519,7 +526,7 @@ sparse_fa_kernel(const FaParams p) {
           it.req = p.row_req[w];
           it.qb = p.row_qb[w];
           it.head = p.row_head[w];
-          set_q_range(it);
+          set_q_range(it, p.qo_indptr + it.req);
           it.kv_begin = p.kv_indptr[it.req];
           it.kv_len = p.kv_indptr[it.req + 1] - it.kv_begin;
           // this share's range of the row's kv blocks
@@ -623,7 +630,7 @@ sparse_fa_kernel(const FaParams p) {
         const int n = ri.nb, list0 = ri.ptr0;
         int blk_first = 0;
         if (lane < n) blk_first = p.kv_idx[list0 + lane];
-        set_q_range(ri);
+        set_q_range(ri, p.qo_indptr + ri.req);
         ri.kv_begin = p.kv_indptr[ri.req];
         ri.kv_len = p.kv_indptr[ri.req + 1] - ri.kv_begin;
         fill_scales(ri);
@@ -657,43 +664,81 @@ sparse_fa_kernel(const FaParams p) {
     __builtin_amdgcn_s_waitcnt(0x0f70);
   };
   // ---- kDirect: rows straight from the packed symbols (short lists) ----
-  // Every workgroup reads all flags and keep bits itself, two candidates (symbol row, head) per thread in
-  // head-major order, and works out with two or three workgroup scans which rows or parts of rows are its
-  // own.  A decode launch in front of this one costs 8-15 us and a launch gap at these sizes, most of it
-  // latency of a single workgroup; here the same trips to memory (two, for a batch of one request) replace
+  // Every workgroup reads all flags and keep bits itself, two or four candidates (symbol row, head) per
+  // thread in head-major order, and works out with two or three workgroup scans which rows or parts of rows
+  // are its own.  A decode launch in front of this one costs 8-15 us and a launch gap at these sizes, most of
+  // it latency of a single workgroup; here the same trips to memory (two, for a batch of one request) replace
   // the three that fetching the decoded schedule costs.
-  //   * No more rows than workgroups: one workgroup per row, or per part of it where workgroups are left
-  //     over and a part still has kDirectMinPart kv blocks.  (Even shares would cut short rows at share
-  //     boundaries here and give workgroups two pieces.)
-  //   * More: even shares as the decoder lays them out (a row costs kRowOverhead + its kv blocks, share j
-  //     is the cost range [j * share, (j + 1) * share)), with the table of rows in LDS.
-  __shared__ int s_wave[4][8];
+  //   * Whole parts: one workgroup per row, or per part of it where workgroups are left over and a part still
+  //     has kDirectMinPart kv blocks.  Where there are no more rows than workgroups and the longest part is
+  //     no longer than an even share and what its cuts cost.
+  //   * Even shares as the decoder lays them out (a row costs kShareRowCost + its kv blocks, a share is a range
+  //     of that cost), with the table of rows in LDS.  (154 rows of 260 kv blocks on 256 workgroups: 517 us as
+  //     whole rows, 338 in shares; 160 rows of 64 blocks 139 -> 92.)
+  // In the pipelined form the next item is fetched beside a row's first copies instead of at its end, where the
+  // trips to memory are 2.4 us that nothing hides.
+  __shared__ int s_wave[4 + kDirectMaxParts / 2][8];
   __shared__ uint16_t s_row_cand[kDirect ? kDirectMaxCand : 1];  // even shares: candidate of every active row ...
   __shared__ int s_row_u[kDirect ? kDirectMaxCand + 1 : 1];      // ... and the cost at which its kv blocks begin
   __shared__ uint16_t s_zero[kDirect ? 64 : 1];                  // candidates this workgroup clears
-  __shared__ int s_dir[4];                         // first row of the share, candidates to clear
-  int dir_rows = 0, dir_share = 0, dir_total = 0;                // even shares; rows = 0: one item at most
-  // (a constant where it is not used: worked out there as well, it made the compiler spill 15 more scalar and 3
-  // more vector registers in the form for decoded lists, 40 bytes of scratch per lane in place of 28)
-  const int dir_g = !kDirect                          ? 0
-                    : (gridDim.x & (kXcds - 1)) == 0 ? (blockIdx.x & (kXcds - 1)) * (gridDim.x / kXcds) + blockIdx.x / kXcds
-                                                     : static_cast<int>(blockIdx.x);
+  // first row of the share, candidates to clear; even shares: rows (0: one item at most), shares, cost of all
+  // (in LDS and not in registers, where they would live through the main loop)
+  __shared__ int s_dir[5];
+  __shared__ int s_ends[5];  // a batch of one request: its q and kv tokens, where its keep bits begin
+  constexpr int kCands = kDirectMaxCand / (64 * kWaves);         // candidates of a thread
+  // this workgroup's share: neighbouring ones on one XCD
+  auto dir_index = [&]() {
+    return (gridDim.x & (kXcds - 1)) == 0 ? (blockIdx.x & (kXcds - 1)) * (gridDim.x / kXcds) + blockIdx.x / kXcds
+                                          : static_cast<int>(blockIdx.x);
+  };
+  // floor(a / d) for a < 2^20: with half a unit added the quotient is further from a whole number than the
+  // reciprocal's error
+  auto part_of = [](int a, int d) {
+    return static_cast<int>((static_cast<float>(a) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(d)));
+  };
+  // Share j of `shares` begins at cost cut_at(j) (products below 2^30: at most 2^20 keep bits, 512 shares);
+  // share_of is the share that holds a unit of cost.  Where two workgroups share a CU the one that was launched
+  // first is ahead of the other throughout (its wavefronts are older and go first: 126 against 146 us with equal
+  // shares, and the younger one then runs alone on its CU, at two thirds of the pair's rate), so the shares of an
+  // XCD's first half are longer by kOlderGain / 128 and those of the second half shorter.
+  auto cut_at = [&](int j, int total, int shares) {
+    if constexpr (kPipe) {
+      const int per = shares / kXcds;
+      if (shares == static_cast<int>(gridDim.x) && per * kXcds == shares && (per & 1) == 0) {
+        const int i = j - part_of(j, per) * per;
+        // 2^16 times the part of all cost that lies in front of share j
+        const uint32_t in_front = static_cast<uint32_t>(j * 128 + min(i, per - i) * kOlderGain) * 512u / shares;
+        return static_cast<int>((static_cast<uint64_t>(total) * in_front) >> 16);
+      }
+    }
+    return static_cast<int>(static_cast<uint32_t>(j) * total / shares);
+  };
+  auto share_of = [&](int at, int total, int shares) {
+    int j = static_cast<int>((static_cast<uint32_t>(at + 1) * shares - 1) / total);
+    if constexpr (kPipe) {
+      while (cut_at(j, total, shares) > at) --j;
+      while (j + 1 < shares && cut_at(j + 1, total, shares) <= at) ++j;
+    }
+    return j;
+  };
   // everything about candidate `cand` but its part
   auto direct_row = [&](int cand, RowInfo& it) {
-    const int h = cand / p.n_blk, t = cand - h * p.n_blk;
+    const int h = part_of(cand, p.n_blk), t = cand - h * p.n_blk;
     it.row = cand;
     it.req = p.batch == 1 ? 0 : p.blk_req[t];
     it.qb = p.batch == 1 ? t : p.blk_qb[t];
     it.head = h;
-    set_q_range(it);
-    it.kv_begin = p.kv_indptr[it.req];
-    it.kv_len = p.kv_indptr[it.req + 1] - it.kv_begin;
+    // (one request: its bounds are in LDS)
+    const bool one = p.batch == 1;
+    set_q_range(it, one ? s_ends : p.qo_indptr + it.req);
+    it.kv_begin = one ? s_ends[2] : p.kv_indptr[it.req];
+    it.kv_len = (one ? s_ends[3] : p.kv_indptr[it.req + 1]) - it.kv_begin;
     if constexpr (kDirect) {
       it.nkv = (it.kv_len + kBlockKV - 1) / kBlockKV;
       it.mask = nullptr;
       it.mask_first = 0;
       if (!p.is_full) {
-        const BitRange r(p.kv_info + p.kv_info_indptr[it.req],
+        const BitRange r(p.kv_info + (one ? s_ends[4] : p.kv_info_indptr[it.req]),
                          (static_cast<int64_t>(it.qb) * p.symbol_heads + h) * it.nkv, it.nkv);
         it.mask = r.words;
         it.mask_first = r.first;
@@ -703,36 +748,120 @@ sparse_fa_kernel(const FaParams p) {
     it.k_scale0 = 0;
   };
   auto direct_schedule = [&]() {
-    const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads;
-    bool act[2];
-    int n[2];
+    const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads, dir_g = dir_index();
+    bool act[kCands];
+    int n[kCands], nkv[kCands];
+    {
+      // All of a thread's candidates make their trips to memory together.  Where the keep bits are more than two
+      // words to a candidate they come as one piece into the tile buffers, which nothing uses yet.  (Candidate
+      // after candidate and word after word, 864 candidates took 14 us until the first row began; now 8.)
+      int req[kCands], bit[kCands];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int cand = 2 * tid + u;
-      act[u] = false;
-      n[u] = 0;
-      if (cand < n_cand) {
-        const int h = cand / p.n_blk, t = cand - h * p.n_blk;
-        const int req = p.batch == 1 ? 0 : p.blk_req[t], qb = p.batch == 1 ? t : p.blk_qb[t];
-        const int nkv = (p.kv_indptr[req + 1] - p.kv_indptr[req] + kBlockKV - 1) / kBlockKV;
-        act[u] = true;
-        n[u] = nkv;
-        if (!p.is_full) {
-          const int64_t bit = static_cast<int64_t>(qb) * p.symbol_heads + h;
-          const uint8_t flags = p.info[p.info_indptr[req] + (bit >> 3)];
-          const BitRange r(p.kv_info + p.kv_info_indptr[req], bit * nkv, nkv);
-          int kept = 0;
-          const int words = r.count();
-          for (int i = 0; i < words; ++i) kept += __popc(r.trim(r.words[i], i));
-          act[u] = (flags >> (bit & 7)) & 1;
-          n[u] = act[u] ? kept : 0;
+      for (int u = 0; u < kCands; ++u) {
+        const int cand = min(kCands * tid + u, n_cand - 1);
+        const int h = part_of(cand, p.n_blk), t = cand - h * p.n_blk;
+        req[u] = p.batch == 1 ? 0 : p.blk_req[t];
+        bit[u] = (p.batch == 1 ? t : p.blk_qb[t]) * p.symbol_heads + h;
+      }
+      if (p.batch == 1 && tid == 0) {
+        s_ends[0] = p.qo_indptr[0];
+        s_ends[1] = p.qo_indptr[1];
+        s_ends[2] = p.kv_indptr[0];
+        s_ends[3] = p.kv_indptr[1];
+        s_ends[4] = p.is_full ? 0 : p.kv_info_indptr[0];
+      }
+#pragma unroll
+      for (int u = 0; u < kCands; ++u) {
+        nkv[u] = (p.kv_indptr[req[u] + 1] - p.kv_indptr[req[u]] + kBlockKV - 1) / kBlockKV;
+        act[u] = kCands * tid + u < n_cand;
+        n[u] = act[u] ? nkv[u] : 0;
+      }
+      if (!p.is_full) {
+        int keep_at[kCands];
+        uint8_t flags[kCands];
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) {
+          keep_at[u] = p.kv_info_indptr[req[u]];
+          flags[u] = p.info[p.info_indptr[req[u]] + (bit[u] >> 3)];
+        }
+        const int map_lo = p.kv_info_indptr[0], map_hi = p.kv_info_indptr[p.batch], map_bytes = map_hi - map_lo;
+        if (map_bytes > 8 * n_cand && map_bytes <= kDirectMapBytes) {
+          const uintptr_t at = reinterpret_cast<uintptr_t>(p.kv_info) + map_lo;
+          const int skew = static_cast<int>(at & 3);
+          const uint32_t* src = reinterpret_cast<const uint32_t*>(at & ~uintptr_t(3));
+          const int n_words = (skew + map_bytes + 3) >> 2;
+          uint32_t* dst = reinterpret_cast<uint32_t*>(smem);
+          for (int i = tid; i < n_words; i += 4 * 64 * kWaves) {
+            uint32_t v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = src[min(i + j * 64 * kWaves, n_words - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (i + j * 64 * kWaves < n_words) dst[i + j * 64 * kWaves] = v[j];
+          }
+          __syncthreads();
+          const uint32_t* words[kCands];
+          int first[kCands], left = 0;
+#pragma unroll
+          for (int u = 0; u < kCands; ++u) {
+            act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
+            n[u] = first[u] = 0;
+            words[u] = reinterpret_cast<const uint32_t*>(smem);
+            if (act[u]) {
+              const int64_t at_bit = static_cast<int64_t>(bit[u]) * nkv[u];
+              // (a caller's segments may lie in any order: one outside of the piece is read where it is)
+              if (keep_at[u] >= map_lo && keep_at[u] + ((at_bit + nkv[u] + 7) >> 3) <= map_hi) {
+                const int byte = skew + keep_at[u] - map_lo + static_cast<int>(at_bit >> 3);
+                words[u] += byte >> 2;
+                first[u] = (byte & 3) * 8 + static_cast<int>(at_bit & 7);
+                left = max(left, (first[u] + nkv[u] + 31) >> 5);
+              } else {
+                const BitRange r(p.kv_info + keep_at[u], at_bit, nkv[u]);
+                for (int i = 0; i < r.count(); ++i) n[u] += __popc(r.trim(r.words[i], i));
+                nkv[u] = 0;
+              }
+            }
+          }
+          for (int i = 0; i < left; ++i)
+#pragma unroll
+            for (int u = 0; u < kCands; ++u) {
+              BitRange r(nullptr, 0, nkv[u]);
+              r.first = first[u];
+              if (act[u] && i < r.count()) n[u] += __popc(r.trim(words[u][i], i));
+            }
+        } else {
+          constexpr int kAhead = 3;
+          uint32_t v[kCands][kAhead];
+#pragma unroll
+          for (int u = 0; u < kCands; ++u) {
+            const BitRange r(p.kv_info + keep_at[u], static_cast<int64_t>(bit[u]) * nkv[u], nkv[u]);
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) v[u][i] = i < r.count() && nkv[u] > 0 ? r.words[i] : 0u;
+          }
+#pragma unroll
+          for (int u = 0; u < kCands; ++u) {
+            const BitRange r(p.kv_info + keep_at[u], static_cast<int64_t>(bit[u]) * nkv[u], nkv[u]);
+            act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
+            n[u] = 0;
+            if (act[u] && nkv[u] > 0) {
+#pragma unroll
+              for (int i = 0; i < kAhead; ++i)
+                if (i < r.count()) n[u] += __popc(r.trim(v[u][i], i));
+              for (int i = kAhead; i < r.count(); ++i) n[u] += __popc(r.trim(r.words[i], i));
+            }
+          }
         }
       }
     }
-    if (tid < 4) s_dir[tid] = tid == 0 ? 0x7fffffff : 0;
-    const int rows_mine = act[0] + act[1], n_mine = n[0] + n[1];
+    if (tid < 3) s_dir[tid] = 0;
+    int rows_mine = 0, n_mine = 0, mx = 0;
+#pragma unroll
+    for (int u = 0; u < kCands; ++u) {
+      rows_mine += act[u];
+      n_mine += n[u];
+      mx = max(mx, n[u]);
+    }
     const int rows_incl = wave_scan(rows_mine), n_incl = wave_scan(n_mine);
-    int mx = max(n[0], n[1]);
     for (int off = 32; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off, 64));
     if (lane == 63) {
       s_wave[0][wv] = rows_incl;
@@ -742,7 +871,7 @@ sparse_fa_kernel(const FaParams p) {
     __syncthreads();
     int rows = 0, blocks = 0, max_n = 0, row = rows_incl - rows_mine, before = n_incl - n_mine;
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
       if (w < wv) {
         row += s_wave[0][w];
         before += s_wave[1][w];
@@ -753,67 +882,104 @@ sparse_fa_kernel(const FaParams p) {
     }
     // q blocks that are not computed are cleared by turns
     if (p.zero_skipped) {
-      int skipped = 2 * tid - row;
+      int skipped = kCands * tid - row;
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-        if (2 * tid + u < n_cand && !act[u]) {
-          if (skipped % n_wg == dir_g) {
-            s_zero[skipped / n_wg] = static_cast<uint16_t>(2 * tid + u);
-            atomicAdd(&s_dir[1], 1);
-          }
+      for (int u = 0; u < kCands; ++u)
+        if (kCands * tid + u < n_cand && !act[u]) {
+          const int turn = part_of(skipped, n_wg);
+          if (skipped - turn * n_wg == dir_g) s_zero[turn] = static_cast<uint16_t>(kCands * tid + u);
           ++skipped;
         }
+      if (tid == 0) s_dir[1] = max(n_cand - rows - dir_g + n_wg - 1, 0) / n_wg;
     }
+    const int total = kShareRowCost * rows + blocks;
+    // (a row in at most four parts: no share is shorter than a third of the longest row)
+    const int shares = max(min(min(n_wg, total), max_n > 0 ? 3 * total / max_n : 1), 1);
     if (rows <= n_wg) {
-      const int spare = n_wg - rows;
-      const int want = max(max(spare > 0 ? (blocks + spare - 1) / spare : max_n, (max_n + kDirectMaxParts - 1) / kDirectMaxParts),
-                           kDirectMinPart);
-      int parts[2];
+      // parts of at most ceil(max_n / k) kv blocks: how many there are for every k
+      int longest = max(max_n, kDirectMinPart);
+      if (max_n > kDirectMinPart) {
+        uint32_t counts[kDirectMaxParts / 2];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) parts[u] = act[u] ? max((n[u] + want - 1) / want, 1) : 0;
-      const int parts_mine = parts[0] + parts[1], parts_incl = wave_scan(parts_mine);
-      if (lane == 63) s_wave[3][wv] = parts_incl;
-      if (tid < kItemBatch) s_items[tid].row = -1;
-      __syncthreads();
-      int first = parts_incl - parts_mine;
-      for (int w = 0; w < wv; ++w) first += s_wave[3][w];
+        for (int k = 1; k <= kDirectMaxParts; ++k) {
+          const int w = max((max_n + k - 1) / k, kDirectMinPart);
+          int parts_mine = 0;
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        if (first <= dir_g && dir_g < first + parts[u]) {
-          RowInfo it;
-          direct_row(2 * tid + u, it);
-          const int per = (n[u] + parts[u] - 1) / parts[u];
-          it.part = dir_g - first;
-          it.parts = parts[u];
-          it.slot = first;
-          it.ptr0 = it.part * per;
-          // (no part is empty but that of a row without kv blocks: per <= want, so parts - 1 of them are fewer
-          // than n blocks.  Longer than the LDS list, a part is cut, as the other forms cut a row: callers that plan a
-          // batch send requests of more than kRowBlocks kv blocks to the decoder)
-          it.nb = min(max(min(n[u] - it.ptr0, per), 0), kRowBlocks);
-          s_items[0] = it;
+          for (int u = 0; u < kCands; ++u) parts_mine += act[u] ? part_of(max(n[u], 1) - 1, w) + 1 : 0;
+          if (k & 1) counts[k >> 1] = parts_mine; else counts[(k >> 1) - 1] |= static_cast<uint32_t>(parts_mine) << 16;
         }
-        first += parts[u];
-      }
-      __syncthreads();
-      return;
-    }
-    dir_rows = rows;
-    dir_total = kRowOverhead * rows + blocks;
-    dir_share = max(max((dir_total + n_wg - 1) / n_wg, (max_n + 2) / 3), 1);
-    const int a = dir_g * dir_share;
-    int cost = kRowOverhead * row + before;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+        for (int k = 0; k < kDirectMaxParts / 2; ++k) {
+          const int sum = wave_scan(static_cast<int>(counts[k]));
+          if (lane == 63) s_wave[4 + k][wv] = sum;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kDirectMaxParts / 2; ++k) {
+          uint32_t all = 0;
+#pragma unroll
+          for (int w = 0; w < kWaves; ++w) all += static_cast<uint32_t>(s_wave[4 + k][w]);
+          if (static_cast<int>(all & 0xffff) <= n_wg) longest = max((max_n + 2 * k) / (2 * k + 1), kDirectMinPart);
+          if (static_cast<int>(all >> 16) <= n_wg) longest = max((max_n + 2 * k + 1) / (2 * k + 2), kDirectMinPart);
+        }
+      }
+      // Whole parts or even shares: whichever has the least on its slowest workgroup.  A share is as good as never
+      // made of one piece only: a second prologue, epilogue and exchange are worth kEvenExtra blocks.
+      if (longest + (longest < max_n ? kPartExtra : 0) <= total / shares + kEvenExtra) {
+        int parts[kCands], parts_mine = 0;
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) {
+          parts[u] = act[u] ? part_of(max(n[u], 1) - 1, longest) + 1 : 0;
+          parts_mine += parts[u];
+        }
+        const int parts_incl = wave_scan(parts_mine);
+        if (lane == 63) s_wave[3][wv] = parts_incl;
+        if (tid < kItemBatch) s_items[tid].row = -1;
+        __syncthreads();
+        int first = parts_incl - parts_mine;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w)
+          if (w < wv) first += s_wave[3][w];
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) {
+          if (first <= dir_g && dir_g < first + parts[u]) {
+            RowInfo it;
+            direct_row(kCands * tid + u, it);
+            const int per = (n[u] + parts[u] - 1) / parts[u];
+            it.part = dir_g - first;
+            it.parts = parts[u];
+            it.slot = first;
+            it.ptr0 = it.part * per;
+            // (no part is empty but that of a row without kv blocks: per <= longest, so parts - 1 of them are fewer
+            // than n blocks.  Longer than the LDS list, a part is cut, as the other forms cut a row: callers that
+            // plan a batch send requests of more than kRowBlocks kv blocks to the decoder)
+            it.nb = min(max(min(n[u] - it.ptr0, per), 0), kRowBlocks);
+            s_items[0] = it;
+          }
+          first += parts[u];
+        }
+        __syncthreads();
+        return;
+      }
+    }
+    const int a = cut_at(dir_g, total, shares);
+    int cost = kShareRowCost * row + before;
+#pragma unroll
+    for (int u = 0; u < kCands; ++u)
       if (act[u]) {
-        s_row_cand[row] = static_cast<uint16_t>(2 * tid + u);
-        s_row_u[row] = cost + kRowOverhead;
-        cost += kRowOverhead + n[u];
-        // first row of the share: the first one that ends behind the share's lower bound
-        if (cost > a) atomicMin(&s_dir[0], row);
+        s_row_cand[row] = static_cast<uint16_t>(kCands * tid + u);
+        s_row_u[row] = cost + kShareRowCost;
+        // first row of the share: the one that holds the share's lower bound
+        if (cost <= a && a < cost + kShareRowCost + n[u]) s_dir[0] = row;
+        cost += kShareRowCost + n[u];
         ++row;
       }
-    if (tid == 0) s_row_u[rows] = dir_total + kRowOverhead;
+    if (tid == 0) {
+      s_row_u[rows] = total + kShareRowCost;
+      s_dir[2] = rows;
+      s_dir[3] = shares;
+      s_dir[4] = total;
+    }
     __syncthreads();
   };
   // sixteen items of the share from `batch_base` on
@@ -822,9 +988,10 @@ sparse_fa_kernel(const FaParams p) {
     if (lane < kItemBatch) {
       RowInfo it;
       it.row = -1;
-      const int a = dir_g * dir_share, b = min(a + dir_share, dir_total), i = s_dir[0] + batch_base + lane;
-      if (a < dir_total && i >= 0 && i < dir_rows) {
-        const int u = s_row_u[i], e = s_row_u[i + 1] - kRowOverhead;  // kv blocks cost [u, e)
+      const int dir_g = dir_index(), rows = s_dir[2], shares = s_dir[3], total = s_dir[4];
+      const int a = cut_at(dir_g, total, shares), b = cut_at(dir_g + 1, total, shares), i = s_dir[0] + batch_base + lane;
+      if (dir_g < shares && i >= 0 && i < rows) {
+        const int u = s_row_u[i], e = s_row_u[i + 1] - kShareRowCost;  // kv blocks cost [u, e)
         // (a row without kv blocks stands for the last unit of its own overhead)
         if ((e > u ? u : u - 1) < b) {
           direct_row(s_row_cand[i], it);
@@ -832,7 +999,7 @@ sparse_fa_kernel(const FaParams p) {
           it.parts = 1;
           it.slot = 0;
           if (e > u) {
-            const int j_lo = u / dir_share, j_hi = (e - 1) / dir_share;
+            const int j_lo = share_of(u, total, shares), j_hi = share_of(e - 1, total, shares);
             it.part = dir_g - j_lo;
             it.parts = j_hi - j_lo + 1;
             it.slot = j_lo;
@@ -866,19 +1033,22 @@ sparse_fa_kernel(const FaParams p) {
         r.words = reinterpret_cast<const uint32_t*>(
             static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m >> 32)))) << 32 |
             static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m))));
-        int seen = 0;
-        for (int w0 = 0; w0 < r.count(); w0 += 64) {
-          const int w = w0 + lane;
-          uint32_t bits = w < r.count() ? r.trim(r.words[w], w) : 0u;
-          const int incl = wave_scan(__popc(bits));
-          int at_bit = seen + incl - __popc(bits) - lo;
-          while (bits) {
-            const int b = __ffs(bits) - 1;
-            bits &= bits - 1;
-            if (at_bit >= 0 && at_bit < n) s_blk2[slot_idx][at_bit] = static_cast<uint16_t>(32 * w + b - r.first);
-            ++at_bit;
+        // a kv block per lane, its place in the list from the bits below it; four rounds' words requested together
+        int seen = -lo;
+        for (int b0 = 0; b0 < r.n && seen < n; b0 += 4 * 64) {
+          uint32_t v[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = r.words[(r.first + min(b0 + 64 * j + lane, r.n - 1)) >> 5];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int b = b0 + 64 * j + lane;
+            const bool kept = b < r.n && (v[j] >> ((r.first + b) & 31)) & 1;
+            const uint64_t all = __ballot(kept);
+            const int at_bit = seen + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(all >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(all), 0u)));
+            if (kept && at_bit >= 0 && at_bit < n) s_blk2[slot_idx][at_bit] = static_cast<uint16_t>(b);
+            seen += __popcll(all);
           }
-          seen += __builtin_amdgcn_readlane(incl, 63);
         }
       }
     }
@@ -887,7 +1057,7 @@ sparse_fa_kernel(const FaParams p) {
   if constexpr (kDirect) {
     // (the copy of the symbols for a later decode: requested first, so that it passes beside the scans)
     if (p.keep_info != nullptr) {
-      const int step = gridDim.x * kThreads, at = blockIdx.x * kThreads + tid;
+      const int step = gridDim.x * (64 * kWaves), at = blockIdx.x * (64 * kWaves) + tid;
       for (int i = at; i < p.kv_info_bytes; i += step) p.keep_kv_info[i] = p.kv_info[i];
       for (int i = at; i < p.info_bytes; i += step) p.keep_info[i] = p.info[i];
       for (int i = at; i <= p.batch; i += step) {
@@ -901,7 +1071,7 @@ sparse_fa_kernel(const FaParams p) {
     direct_schedule();
     if (wv == 0) {
       if (lane == 0) s_share[0] = 0;
-      if (dir_rows > 0) direct_items(0);
+      if (__builtin_amdgcn_readfirstlane(s_dir[2]) > 0) direct_items(0);
       direct_next(0);
     }
   }
@@ -1062,6 +1232,9 @@ sparse_fa_kernel(const FaParams p) {
       if (n_steps > 1) copy_k(1);
       if (n_steps > 2) copy_k(2);
       copy_v(0);
+      // (shares are known from the start: the next item and its kv block list are fetched beside these copies)
+      if constexpr (kDirect)
+        if (wv == 0) direct_next((row_it + 1) & 1);
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __builtin_amdgcn_s_barrier();
       x8 qreg[8], kop[4], vop[4];
@@ -1805,8 +1978,9 @@ sparse_fa_kernel(const FaParams p) {
       __syncthreads();
     }
     if (wv == kFetchWave) {
-        if constexpr (kDirect) direct_next((row_it + 1) & 1); else fetch_next((row_it + 1) & 1, false);
-      }
+      if constexpr (!kDirect) fetch_next((row_it + 1) & 1, false);
+      else if constexpr (!kPipe) direct_next((row_it + 1) & 1);
+    }
     float m_all = 0.f, d_all = 0.f;  // kv group 0: row maximum and row sum over both groups
     // A lane owns one q row and runs of four d: stored from here, a row would leave as 32 scattered
     // 8-byte pieces per instruction (measured: ~12 k cycles per row).  The finished row goes through
@@ -1818,17 +1992,22 @@ sparse_fa_kernel(const FaParams p) {
     if constexpr (kGroups == 1) {
       // one kv group: the accumulators hold the whole row
       const float d_tot = d_part + __shfl_xor(d_part, 32, 64);
-      const float inv = __builtin_amdgcn_rcpf(d_tot);
+      if (!kDirect || parts == 1) {
+        const float inv = __builtin_amdgcn_rcpf(d_tot);
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          x4 out;
+          for (int i4 = 0; i4 < 4; ++i4) {
+            x4 out;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(o_acc[dt][i4 * 4 + j] * inv);
-          *reinterpret_cast<x4*>(out_row + (dt * 32 + i4 * 8 + g_e * 4) * sizeof(T)) = out;
-        }
-      if (row_ok_e && p.lse && g_e == 0) p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(d_tot) + m_run;
+            for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(o_acc[dt][i4 * 4 + j] * inv);
+            *reinterpret_cast<x4*>(out_row + (dt * 32 + i4 * 8 + g_e * 4) * sizeof(T)) = out;
+          }
+        if (row_ok_e && p.lse && g_e == 0) p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(d_tot) + m_run;
+      } else {
+        m_all = m_run;
+        d_all = d_tot;
+      }
     }
     if (kGroups == 2 && kg == 0) {
       const float m1 = md[(qs * 64 + lane_m) * 2 + 0], d1 = md[(qs * 64 + lane_m) * 2 + 1];
@@ -1874,7 +2053,7 @@ sparse_fa_kernel(const FaParams p) {
         d_all = d_tot;
       }
     }
-    if (kGroups == 2 && parts > 1) {
+    if ((kGroups == 2 || kDirect) && parts > 1) {
       // Whoever comes last combines the parts and writes the row.  A workgroup that finds every
       // other part arrived already need not publish its own; otherwise it publishes, then counts
       // itself in, and may still turn out to be the last.
@@ -1911,18 +2090,18 @@ sparse_fa_kernel(const FaParams p) {
           auto part_base = [&](int i) {
             return p.split_ws + static_cast<int64_t>(part_area(split_slot, i)) * kSplitPartFloats;
           };
-          constexpr int kParts = kDirect ? kDirectMaxParts : kMaxSplitParts;
-          float m_p[kParts], d_p[kParts];
+          // (a part's maximum and sum are read twice: held in an array, they would be in scratch memory)
           const float m_own = m_all, d_own = d_all;
+          auto part_stats = [&](int i, float& m, float& d) {
+            m = m_own;
+            d = d_own;
+            if (i != part) load_pair_device(part_base(i) + 128 * 128 + (qs * 64 + lane_m) * 2, m, d);
+          };
           m_all = kNegInf;
           for (int i = 0; i < parts; ++i) {
-            if (i == part) {
-              m_p[i] = m_own;
-              d_p[i] = d_own;
-            } else {
-              load_pair_device(part_base(i) + 128 * 128 + (qs * 64 + lane_m) * 2, m_p[i], d_p[i]);
-            }
-            m_all = fmaxf(m_all, m_p[i]);
+            float m, d;
+            part_stats(i, m, d);
+            m_all = fmaxf(m_all, m);
           }
           d_all = 0.f;
           f32x16 acc[4];
@@ -1932,9 +2111,11 @@ sparse_fa_kernel(const FaParams p) {
             for (int e = 0; e < 16; ++e) acc[dt][e] = 0.f;
           const int ln = fresh_lane();
           for (int i = 0; i < parts; ++i) {
-            const float a = __builtin_amdgcn_exp2f(m_p[i] - m_all);
-            d_all = __builtin_fmaf(d_p[i], a, d_all);
+            float m, d;
+            part_stats(i, m, d);
             if (i == part) {
+              const float a = __builtin_amdgcn_exp2f(m - m_all);
+              d_all = __builtin_fmaf(d, a, d_all);
 #pragma unroll
               for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -1949,6 +2130,8 @@ sparse_fa_kernel(const FaParams p) {
                 load_pair_device(lane_ws + e * 256 + 128, u[e][2], u[e][3]);
               }
               __builtin_amdgcn_sched_barrier(0);
+              const float a = __builtin_amdgcn_exp2f(m - m_all);
+              d_all = __builtin_fmaf(d, a, d_all);
 #pragma unroll
               for (int e = 0; e < 16; ++e)
 #pragma unroll
@@ -2009,7 +2192,7 @@ sparse_fa_kernel(const FaParams p) {
       direct_row(s_zero[z], it);
       const int gq = kGqaPack ? p.gqa_pack : 0;
       T* dst = op + static_cast<int64_t>(it.q_begin) * p.o_sn + static_cast<int64_t>(gq ? it.head * gq : it.head) * p.o_sh;
-      for (int i = tid; i < it.q_rows * 16; i += kThreads) {
+      for (int i = tid; i < it.q_rows * 16; i += 64 * kWaves) {
         const int r = i >> 4;
         int64_t off;
         if constexpr (kGqaPack) {
@@ -2264,6 +2447,24 @@ extern "C" int fo_sparse_attention_direct(const void* args) {
                   : launch<_Float16, false, false, false, 2, false, true, true, true>(p, n_cand, s);
     return bf16 ? launch<__bf16, false, false, false, 2, false, false, true, true>(p, n_cand, s)
                 : launch<_Float16, false, false, false, 2, false, false, true, true>(p, n_cand, s);
+  }
+  // From 2.5 candidates per CU on: two workgroups of four wavefronts per CU and the software-pipelined loop, whose
+  // row boundaries pass beside the other workgroup's main loop; below, the two-phase loop with twice the wavefronts
+  // per row.  Pipelined against two-phase, with (active rows, kept blocks): 864 candidates of 36 blocks 155 / 165 us
+  // (100 %, 50 %), 273 / 295 (100 %, 100 %), 119 / 127 (75 %, 50 %), 62 / 59 (30 %, 50 %); 1000 of 25 blocks 106 / 113
+  // (75 %, 50 %), 56 / 54 (30 %, 50 %); 512 of 32 blocks 76 / 72 (75 %, 50 %), 44 / 41 (30 %, 50 %); 216 of 9 blocks
+  // 31 / 27.  What it needs besides: partial results of two shares per CU, room in LDS for a row's list (the
+  // longest row is bounded by all keep bits where there are several requests), 32-bit copy offsets.
+  const int64_t nkv = a.max_nnz / (a.batch == 1 ? n_cand : a.symbol_heads), span = (nkv + 1) * kBlockKV * 2;
+  const bool pipe = 2 * n_cand >= int64_t(5) * fo_num_cu() && nkv <= kMaxRowBlocksOneGroupDirect &&
+                    2 * fo_num_cu() <= kMaxShares && a.split_ws_bytes >= 2 * fo_sparse_fa_split_workspace_bytes() &&
+                    span * a.k_stride_n < (int64_t(1) << 32) && span * a.v_stride_n < (int64_t(1) << 32);
+  if (pipe) {
+    if (packed)
+      return bf16 ? launch<__bf16, false, false, false, 1, true, true, false, true>(p, n_cand, s)
+                  : launch<_Float16, false, false, false, 1, true, true, false, true>(p, n_cand, s);
+    return bf16 ? launch<__bf16, false, false, false, 1, true, false, false, true>(p, n_cand, s)
+                : launch<_Float16, false, false, false, 1, true, false, false, true>(p, n_cand, s);
   }
   if (packed)
     return bf16 ? launch<__bf16, false, false, false, 2, false, true, false, true>(p, n_cand, s)
