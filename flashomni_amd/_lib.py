@@ -42,6 +42,10 @@ SIGNATURES = {
     "fo_sparse_fa_run": ([c_vp] * 5 + [c_int, c_vp, c_vp, c_vp, c_vp] + [c_i64] * 8 + [c_vp] * 4 + [c_i32, c_i32]
                          + [c_vp] * 7 + [c_i64, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_f32, c_f32, c_vp, c_vp, c_i64, c_vp],
                          c_int),
+    "fo_sparse_fa_wide_bytes": ([c_i64, c_i32, c_i32], c_i64),
+    "fo_sparse_fa_run_wide": ([c_vp] * 5 + [c_int, c_vp, c_vp, c_vp, c_vp] + [c_i64] * 8 + [c_vp] * 4 + [c_i32, c_i32]
+                              + [c_vp] * 7 + [c_i64, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_f32, c_f32, c_vp, c_vp,
+                                              c_i64, c_vp, c_i64, c_i32, c_vp], c_int),
     "fo_sparse_attention_direct_serves": ([c_vp], c_int),
     "fo_sparse_attention_direct": ([c_vp], c_int),
     "fo_gemm_workspace_bytes": ([c_i32, c_i32, c_i32], c_i64),

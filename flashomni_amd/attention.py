@@ -362,8 +362,17 @@ class PlannedBatch:
                 raise ValueError("q_scale / k_scale must be [H, number of 128-token blocks] "
                                  "(k_scale: one row per kv head)")
         wl = self.worklist
+        wide = None
+        if k_lo is not None:
+            # two-term fp8 q and k of a long list: room for the widened k (see fo_sparse_fa_run_wide)
+            n = _lib.lib().fo_sparse_fa_wide_bytes(self.max_rows, self.num_kv_heads, self.n_kv_blk)
+            if n:
+                try:
+                    wide = torch.empty(n, dtype=torch.uint8, device=self.device)
+                except torch.cuda.OutOfMemoryError:
+                    pass  # (the fp8 operands are multiplied as they are)
         with _lib.device_guard(self.device):
-            _lib.check(_lib.lib().fo_sparse_fa_run(
+            _lib.check(_lib.lib().fo_sparse_fa_run_wide(
                 _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse),
                 _lib.dtype_code(q.dtype), _lib.ptr(q_lo), _lib.ptr(k_lo), _lib.ptr(q_scale if fp8 else None),
                 _lib.ptr(k_scale if fp8 else None),
@@ -376,7 +385,8 @@ class PlannedBatch:
                 float(logits_soft_cap or 0.0),
                 _lib.ptr(wl.shares if self.split_ok else None),
                 _lib.ptr(self.float_ws) if self.split_ok else None,
-                self.float_ws_bytes(), _lib.current_stream(self.device)))
+                self.float_ws_bytes(), _lib.ptr(wide), 0 if wide is None else wide.numel(), self.batch_size,
+                _lib.current_stream(self.device)))
 
 
 class BatchFlashOmniFAWithRaggedKVWrapper:

@@ -166,6 +166,10 @@ struct FaParams {
   uint8_t* keep_kv_info;
   int32_t* keep_indptr;
   int32_t info_bytes, kv_info_bytes;
+  // widened fp8 operands (see widen_k_kernel; null: none): the factor of q per kv head, and a word that the
+  // widened form sets when it has left rows to the fp8 form of the same call
+  const float* wide_factor;
+  int32_t* wide_left;
 };
 
 template <typename T>
@@ -201,6 +205,23 @@ struct Types<_Float16> {
     return acc;
   }
 };
+
+// Whether a row's q, scale times the kv head's factor, can be widened: no single product of a logit above 2^8.
+// (464 = the largest sum of two e4m3 terms, 2 = the bound of a widened k; not for a scale that is not a number)
+__device__ __forceinline__ bool wide_holds(float q_scale, float c) { return 464.f * 2.f * q_scale * fabsf(c) <= 256.f && q_scale > 0.f; }
+
+// eight e4m3 pairs (hi + lo) * f, rounded once to fp16
+__device__ __forceinline__ void widen8(u32x2 hi, u32x2 lo, float f, f16x8& out) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const f32x2 h0 = __builtin_amdgcn_cvt_pk_f32_fp8(hi[j], false), h1 = __builtin_amdgcn_cvt_pk_f32_fp8(hi[j], true);
+    const f32x2 l0 = __builtin_amdgcn_cvt_pk_f32_fp8(lo[j], false), l1 = __builtin_amdgcn_cvt_pk_f32_fp8(lo[j], true);
+    out[4 * j + 0] = static_cast<_Float16>((h0[0] + l0[0]) * f);
+    out[4 * j + 1] = static_cast<_Float16>((h0[1] + l0[1]) * f);
+    out[4 * j + 2] = static_cast<_Float16>((h1[0] + l1[0]) * f);
+    out[4 * j + 3] = static_cast<_Float16>((h1[1] + l1[1]) * f);
+  }
+}
 
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(3))) void lds_void;
@@ -368,9 +389,10 @@ constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologu
 // their phases together, there is no merge, and one's row prologue / epilogue overlaps the other's
 // main loop.  A row takes twice as long, so this is the form for long lists (many rows per CU).
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false, bool kDirect = false>
+          bool kCap = false, bool kDirect = false, bool kWide = false>
 __global__ void __launch_bounds__(kGroups * kGroupThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 sparse_fa_kernel(const FaParams p) {
+  static_assert(!kWide || (kPipe && !kGqaPack && !kDirect), "widened operands are a variant of the pipelined loop");
   static_assert(kPipe == (kGroups == 1), "one kv group runs the software-pipelined loop, two the two-phase loop");
   static_assert(!kPipe || !kFp8, "the software-pipelined loop is built for 16-bit operands");
   static_assert(kFp8 || !kQLo, "the two-term q is an fp8 form");
@@ -380,6 +402,8 @@ sparse_fa_kernel(const FaParams p) {
   constexpr int kShareRowCost = kPipe ? kRowOverheadPipe : kRowOverhead;  // kDirect: what a row costs beside its kv blocks
   constexpr int kFetchWave = kGroups == 2 ? 4 : 0;  // the wavefront that fetches the next item
   using TT = Types<T>;
+  using TS = Types<typename std::conditional<kWide, _Float16, T>::type>;  // Q and K
+  using q8 = typename TS::x8;
   using x8 = typename TT::x8;
   using x4 = typename TT::x4;
   using G = Geom<kFp8, kKLo, kGroups>;
@@ -399,8 +423,10 @@ sparse_fa_kernel(const FaParams p) {
   auto fill_scales = [&](RowInfo& it) {
     it.q_scale = 1.f;
     it.k_scale0 = 0;
-    if constexpr (kFp8) {
+    if constexpr (kFp8 || kWide)
       it.q_scale = p.q_scale[static_cast<int64_t>(it.head) * p.n_q_blocks + p.q_blk_base[it.req] + it.qb];
+    if constexpr (kWide) it.q_scale *= p.wide_factor[it.head / p.kv_group];
+    if constexpr (kFp8) {
       it.k_scale0 = (it.head / p.kv_group) * p.n_kv_blocks + p.kv_blk_base[it.req];
     }
   };
@@ -476,6 +502,9 @@ sparse_fa_kernel(const FaParams p) {
       }
   }
 
+  // (what the widened form has left, most often nothing)
+  if constexpr (kKLo)
+    if (p.wide_left != nullptr && *p.wide_left == 0) return;
   // The next row is popped by kv group 1 while kv group 0 combines and stores the current one
   // (group 1 has nothing else to do then), so the queue atomics are off the critical path.
   if constexpr (!kDirect) {
@@ -1134,9 +1163,17 @@ sparse_fa_kernel(const FaParams p) {
     const int64_t q_tok = q_begin + my_tok;
     const int my_head = head_q0 + my_hq;
 
-    if (nb == 0) {
+    // one of the two forms of a call with widened operands takes this row
+    bool other_form = false;
+    if constexpr (kWide) {
+      other_form = !wide_holds(ri.q_scale, c);
+      if (other_form && tid == 0) *p.wide_left = 1;
+    } else if constexpr (kKLo) {
+      if (p.wide_left != nullptr) other_form = wide_holds(ri.q_scale * p.wide_factor[head / p.kv_group], c);
+    }
+    if (nb == 0 || other_form) {
       // listed row without kv blocks: zeros, lse = -5e4
-      if (row_ok && kg == 0) {
+      if (row_ok && kg == 0 && !other_form) {
         T* dst = op + q_tok * p.o_sn + static_cast<int64_t>(my_head) * p.o_sh + g_p * 64;
         const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -1215,7 +1252,19 @@ sparse_fa_kernel(const FaParams p) {
       };
 
       // prologue: Q, K(0..2), V(0) requested together
-      {
+      if constexpr (kWide) {
+        // (two tiles of 128-byte rows: q, then q_lo)
+        const int ln_q = fresh_lane();
+        const int q_row = ln_q >> 3, q_chunk = ((ln_q & 7) ^ ((4 * (qs & 1) + (ln_q >> 4)) & 7)) * 16;
+        const int64_t q_off = static_cast<int64_t>(q_begin) * p.q_sn + static_cast<int64_t>(head_q0) * p.q_sh;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+          int r = 8 * (4 * (n & 3) + qs) + q_row;
+          r = r < q_rows ? r : q_rows - 1;
+          copy16_to_lds(static_cast<const uint8_t*>(n < 4 ? p.q : p.q_lo) + q_off,
+                        static_cast<uint32_t>(r * p.q_sn + q_chunk), lds0 + 4 * kBuf + qs * 1024 + n * 4096);
+        }
+      } else {
         const uint8_t* q_head = reinterpret_cast<const uint8_t*>(
             qp + static_cast<int64_t>(q_begin) * p.q_sn + static_cast<int64_t>(head_q0) * p.q_sh);
         const int ln_q = fresh_lane();
@@ -1237,15 +1286,27 @@ sparse_fa_kernel(const FaParams p) {
         if (wv == 0) direct_next((row_it + 1) & 1);
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __builtin_amdgcn_s_barrier();
-      x8 qreg[8], kop[4], vop[4];
+      q8 qreg[8], kop[4];
+      x8 vop[4];
       u32x4 pA[2], pB[2];  // P of a step: 2 x 8 rounded values, as 32-bit pairs
       f32x16 sA, sB;
-      {
+      if constexpr (kWide) {
+        // q + q_lo under the q block's scale, the softmax scale and the kv head's factor, in fp16
+        const int ln_r = fresh_lane(), row = qs * 32 + (ln_r & 31);
+        const uint8_t* qt = smem + 4 * kBuf + row * kRowBytes8 + (ln_r >> 5) * 8;
+        const float f = c * __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, ri.q_scale)));
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+          const uint8_t* at = qt + ((ks ^ swz8(row)) << 4);
+          const u32x2 hi = *reinterpret_cast<const u32x2*>(at), lo = *reinterpret_cast<const u32x2*>(at + 128 * kRowBytes8);
+          widen8(hi, lo, f, qreg[ks]);
+        }
+      } else {
         const int ln_r = fresh_lane();
         const int q_rd_base = (ln_r & 31) * kRowBytes, q_rd_x = ((ln_r >> 5) ^ swz(ln_r & 31)) << 4;
         const uint8_t* qt = smem + 4 * kBuf + qs * 32 * kRowBytes + q_rd_base;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) qreg[ks] = *reinterpret_cast<const x8*>(qt + (q_rd_x ^ (ks << 5)));
+        for (int ks = 0; ks < 8; ++ks) qreg[ks] = *reinterpret_cast<const q8*>(qt + (q_rd_x ^ (ks << 5)));
         // the softmax scale (log2 domain) is folded into Q, so S^T needs no multiply
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks)
@@ -1255,7 +1316,7 @@ sparse_fa_kernel(const FaParams p) {
       // LDS address of the K operand reads of a step, without the buffer's offset (an immediate of the
       // read): read i is at kx0 ^ (i << 5) (row bits, chunk bits and the 256-byte aligned base of
       // the array do not overlap)
-      typedef __attribute__((address_space(3))) const x8 lds_x8;
+      typedef __attribute__((address_space(3))) const q8 lds_x8;
       uint32_t kx0 = lds0 + static_cast<uint32_t>(k_rd_base | k_rd_x);
       asm volatile("" : "+v"(kx0));
       // K operand slice i (16 d) of the step whose K is in buffer `buf`
@@ -1285,11 +1346,11 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) sA[i] = 0.f;
       {
-        x8 k0[8];
+        q8 k0[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) k0[i] = read_k(kx0, 0, i);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sA = TT::mfma(k0[i], qreg[i], sA);
+        for (int i = 0; i < 8; ++i) sA = TS::mfma(k0[i], qreg[i], sA);
       }
       __builtin_amdgcn_sched_barrier(0);
       // (a row of one step reads a buffer nobody filled: the result is never used)
@@ -1394,7 +1455,7 @@ sparse_fa_kernel(const FaParams p) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          s_next = TT::mfma(kop[i & 3], qreg[i], s_next);
+          s_next = TS::mfma(kop[i & 3], qreg[i], s_next);
           // the operand of the S MFMA four slots on: second half of K(t+1), then first half of K(t+2)
           kop[i & 3] = i < 4 ? read_k(kx, (kB + 1) & 3, i + 4) : read_k(kx, (kB + 2) & 3, i - 4);
           o_acc[i & 3] = TT::mfma(vop[i & 3], __builtin_bit_cast(x8, p_prev[i >> 2]), o_acc[i & 3]);
@@ -2220,8 +2281,77 @@ sparse_fa_kernel(const FaParams p) {
   }
 }
 
+// The two-term fp8 k of a long list, widened once per call: k16 = (k + k_lo) * k_scale * 2^-e in fp16, kv head by
+// kv head ([num_kv_heads][n_kv_blocks * 128][128], tokens as numbered by kv_indptr), e per kv head such that its
+// largest value lies in [1, 2); q's factor, applied where a row is begun, carries 2^e back.  The fp8 form multiplies
+// three times (k.q, k.q_lo, k_lo.q) in the two-phase loop; fp16 operands take one product in the pipelined loop and
+// leave nothing out.  A sum of two e4m3 terms has at most 8 significant bits and an error of 2^-9 of its own, fp16
+// keeps 11, so the logits are closer to the products of the four terms than the fp8 form's, which leaves k_lo.q_lo out.
+// What fp16 cannot hold is left to the fp8 form, row by row: k scales of a head that are not positive and finite,
+// and q blocks with which single products of a logit may exceed 2^8 (below that a q is far from fp16's largest value, and
+// what k loses under fp16's smallest step of 2^-24, in blocks far below the head's largest, moves a logit by less
+// than 128 * 2^8 * 2^-25 = 2^-10).
+// 2 bytes read and 2 written per element: 0.3 ms for 76112 tokens x 40 heads, where attention went from 11.1 to
+// 8.0 ms.
+__global__ void __launch_bounds__(256) widen_k_kernel(
+    const uint8_t* __restrict__ k, const uint8_t* __restrict__ k_lo, int64_t k_sn, int64_t k_sh,
+    const float* __restrict__ k_scale, const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_blk_base,
+    int32_t batch, int32_t n_kv_blocks, _Float16* __restrict__ k16, float* __restrict__ factor, int32_t* __restrict__ left) {
+  __shared__ float s_max[4];
+  __shared__ int s_req;
+  const int blk = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  if (tid == 0) s_req = -1;
+  __syncthreads();
+  // the request of this block, and the head's largest scale (a scale that is not positive and finite counts as infinite)
+  for (int r = tid; r < batch; r += 256)
+    if (kv_blk_base[r] <= blk && blk < kv_blk_base[r + 1]) s_req = r;
+  float mx = 0.f;
+  for (int i = tid; i < n_kv_blocks; i += 256) {
+    const float v = k_scale[static_cast<int64_t>(head) * n_kv_blocks + i];
+    mx = fmaxf(mx, v > 0.f ? v : __builtin_inff());
+  }
+  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  if (lane == 0) s_max[wv] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+  // (in this range 2^e and 2^-e are ordinary numbers; the k16 of a head outside of it is never read)
+  const bool held = mx * 448.f >= 0x1p-100f && mx * 448.f < 0x1p100f;
+  const float two_e = held ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, mx * 448.f) & 0x7f800000u) : __builtin_inff();
+  if (blk == 0 && tid == 0) {
+    factor[head] = two_e;
+    if (head == 0) *left = 0;
+  }
+  const int req = s_req;
+  if (!held || req < 0) return;
+  const int tok0 = kv_indptr[req] + (blk - kv_blk_base[req]) * kBlockKV;
+  const int len = min(kBlockKV, kv_indptr[req + 1] - tok0);
+  const float f = k_scale[static_cast<int64_t>(head) * n_kv_blocks + blk] * (1.f / two_e);
+  const int col = (tid & 7) * 16;
+  _Float16* out = k16 + (static_cast<int64_t>(head) * n_kv_blocks * kBlockKV + tok0) * kHeadDim + col;
+  const int64_t in = static_cast<int64_t>(tok0) * k_sn + static_cast<int64_t>(head) * k_sh + col;
+  u32x4 hi[4], lo[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = min((tid >> 3) + 32 * i, len - 1);
+    hi[i] = *reinterpret_cast<const u32x4*>(k + in + r * k_sn);
+    lo[i] = *reinterpret_cast<const u32x4*>(k_lo + in + r * k_sn);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (tid >> 3) + 32 * i;
+    if (r < len) {
+      f16x8 a, b;
+      widen8(u32x2{hi[i][0], hi[i][1]}, u32x2{lo[i][0], lo[i][1]}, f, a);
+      widen8(u32x2{hi[i][2], hi[i][3]}, u32x2{lo[i][2], lo[i][3]}, f, b);
+      f16x8* dst = reinterpret_cast<f16x8*>(out + r * kHeadDim);
+      dst[0] = a;
+      dst[1] = b;
+    }
+  }
+}
+
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups = 2, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false, bool kDirect = false>
+          bool kCap = false, bool kDirect = false, bool kWide = false>
 int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   constexpr int kSmemBytes = Geom<kFp8, kKLo, kGroups>::kSmemBytes;
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
@@ -2230,7 +2360,7 @@ int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
-    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect>),
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect, kWide>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes));
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
@@ -2239,7 +2369,7 @@ int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   int64_t grid = num_cu * (3 - kGroups);  // persistent workgroups: one per CU, or two of one kv group each (LDS bound)
   // (with even shares every workgroup may hold a part of a row; otherwise at most one row each)
   if (!kDirect && !(p.split_ws && p.shares) && grid > max_rows) grid = max_rows;
-  sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect><<<static_cast<unsigned>(grid), kGroups * kGroupThreads, kSmemBytes, stream>>>(p);
+  sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect, kWide><<<static_cast<unsigned>(grid), kGroups * kGroupThreads, kSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
 }
@@ -2256,12 +2386,25 @@ extern "C" int fo_sparse_fa_set_variant(int variant) {
   return FO_OK;
 }
 
+extern "C" int64_t fo_sparse_fa_wide_bytes(int64_t max_rows, int32_t num_kv_heads, int32_t n_kv_blocks);
+
 extern "C" int64_t fo_sparse_fa_split_workspace_bytes(void) {
   // two areas per share, one share per workgroup = per CU
   return static_cast<int64_t>(2) * fo_num_cu() * kSplitPartFloats * sizeof(float);
 }
 
-extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float* lse,
+namespace {
+// widened fp8 operands: the head of the workspace (factors of the kv heads and a word), then k16
+int64_t wide_head_bytes(int32_t num_kv_heads) { return (static_cast<int64_t>(num_kv_heads) * 4 + 4 + 255) / 256 * 256; }
+// the pipelined form is taken from this many rows on
+bool long_list(int64_t max_rows) { return max_rows >= static_cast<int64_t>(8) * fo_num_cu(); }
+bool wide_serves(int64_t max_rows, int32_t num_kv_heads, int32_t n_kv_blocks) {
+  const int variant = g_variant.load(std::memory_order_relaxed);
+  return (variant == 1 || (variant == 0 && long_list(max_rows))) && max_rows > 0 && num_kv_heads > 0 && num_kv_heads <= 65535 &&
+         n_kv_blocks > 0 && n_kv_blocks <= kMaxRowBlocksOneGroup;
+}
+
+int run_decoded(const void* q, const void* k, const void* v, void* o, float* lse,
                                 int dtype, const void* q_lo, const void* k_lo, const float* q_scale,
                                 const float* k_scale,
                                 int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
@@ -2276,7 +2419,7 @@ extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, voi
                                 int32_t num_heads, int32_t num_kv_heads, int32_t gqa_packed, int32_t head_dim,
                                 int32_t block_q, int32_t block_kv, float sm_scale, float logits_soft_cap,
                                 const int32_t* shares, void* split_workspace, int64_t split_workspace_bytes,
-                                void* stream) {
+                                void* wide, int64_t wide_bytes, int32_t batch, void* stream) {
   FO_REQUIRE(head_dim == kHeadDim, "sparse_fa: head_dim %d is not supported (only 128)", head_dim);
   FO_REQUIRE(block_q == kBlockQ && block_kv == kBlockKV,
              "sparse_fa: sparse block sizes (%d, %d) are not supported (only 128, 128)", block_q,
@@ -2314,7 +2457,7 @@ extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, voi
     FO_REQUIRE((reinterpret_cast<uintptr_t>(ptr) & 15) == 0,
                "sparse_fa: q/k/v/o must be 16-byte aligned");
 
-  FaParams p;
+  FaParams p{};
   p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
   p.q_lo = q_lo; p.k_lo = k_lo; p.q_scale = q_scale; p.k_scale = k_scale;
   p.q_sn = q_stride_n; p.q_sh = q_stride_h; p.k_sn = k_stride_n; p.k_sh = k_stride_h;
@@ -2365,7 +2508,7 @@ extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, voi
                             n_kv_blocks <= kMaxRowBlocksOneGroup && span * k_stride_n < (int64_t(1) << 32) &&
                             span * v_stride_n < (int64_t(1) << 32);
   const int variant = g_variant.load(std::memory_order_relaxed);
-  const bool one_group = one_group_ok && (variant == 1 || (variant == 0 && max_rows >= static_cast<int64_t>(8) * fo_num_cu()));
+  const bool one_group = one_group_ok && (variant == 1 || (variant == 0 && long_list(max_rows)));
   if (p.gqa_pack) {  // packed tiles of several q heads: the row mapping is compiled in
     if (dtype == FO_BF16)
       return one_group ? launch<__bf16, false, false, false, 1, true, true>(p, max_rows, s)
@@ -2379,9 +2522,85 @@ extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, voi
   if (dtype == FO_F16)
     return one_group ? launch<_Float16, false, false, false, 1, true>(p, max_rows, s)
                      : launch<_Float16, false, false, false, 2>(p, max_rows, s);
-  if (k_lo != nullptr) return launch<__bf16, true, true, true>(p, max_rows, s);
+  if (k_lo != nullptr) {
+    if (wide != nullptr && wide_serves(max_rows, num_kv_heads, n_kv_blocks) && span * v_stride_n < (int64_t(1) << 32)) {
+      FO_REQUIRE(batch > 0 && wide_bytes >= fo_sparse_fa_wide_bytes(max_rows, num_kv_heads, n_kv_blocks) &&
+                     (reinterpret_cast<uintptr_t>(wide) & 255) == 0,
+                 "sparse_fa: the workspace for widened operands must be 256-byte aligned and hold "
+                 "fo_sparse_fa_wide_bytes() bytes");
+      float* factor = static_cast<float*>(wide);
+      int32_t* left = reinterpret_cast<int32_t*>(factor + num_kv_heads);
+      _Float16* k16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(wide) + wide_head_bytes(num_kv_heads));
+      widen_k_kernel<<<dim3(n_kv_blocks, num_kv_heads), 256, 0, s>>>(
+          static_cast<const uint8_t*>(k), static_cast<const uint8_t*>(k_lo), k_stride_n, k_stride_h, k_scale, kv_indptr,
+          kv_blk_base, batch, n_kv_blocks, k16, factor, left);
+      FO_CHECK_LAUNCH();
+      p.wide_factor = factor;
+      p.wide_left = left;
+      FaParams w = p;
+      w.k = k16;
+      w.k_sn = kHeadDim;
+      w.k_sh = static_cast<int64_t>(n_kv_blocks) * kBlockKV * kHeadDim;
+      const int rc = launch<__bf16, false, false, false, 1, true, false, false, false, true>(w, max_rows, s);
+      if (rc != FO_OK) return rc;
+    }
+    return launch<__bf16, true, true, true>(p, max_rows, s);
+  }
   if (q_lo != nullptr) return launch<__bf16, true, true, false>(p, max_rows, s);
   return launch<__bf16, true, false, false>(p, max_rows, s);
+}
+
+}  // namespace
+
+extern "C" int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float* lse,
+                                int dtype, const void* q_lo, const void* k_lo, const float* q_scale,
+                                const float* k_scale,
+                                int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
+                                int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h,
+                                int64_t o_stride_n, int64_t o_stride_h, const int32_t* qo_indptr,
+                                const int32_t* kv_indptr, const int32_t* q_blk_base,
+                                const int32_t* kv_blk_base, int32_t n_q_blocks,
+                                int32_t n_kv_blocks, const int32_t* row_req,
+                                const int32_t* row_qb, const int32_t* row_head,
+                                const int32_t* kv_row_ptr, const int32_t* kv_idx,
+                                const int32_t* order, int32_t* sched, int64_t max_rows,
+                                int32_t num_heads, int32_t num_kv_heads, int32_t gqa_packed, int32_t head_dim,
+                                int32_t block_q, int32_t block_kv, float sm_scale, float logits_soft_cap,
+                                const int32_t* shares, void* split_workspace, int64_t split_workspace_bytes,
+                                void* stream) {
+  return run_decoded(q, k, v, o, lse, dtype, q_lo, k_lo, q_scale, k_scale, q_stride_n, q_stride_h, k_stride_n, k_stride_h,
+                     v_stride_n, v_stride_h, o_stride_n, o_stride_h, qo_indptr, kv_indptr, q_blk_base, kv_blk_base, n_q_blocks,
+                     n_kv_blocks, row_req, row_qb, row_head, kv_row_ptr, kv_idx, order, sched, max_rows, num_heads,
+                     num_kv_heads, gqa_packed, head_dim, block_q, block_kv, sm_scale, logits_soft_cap, shares,
+                     split_workspace, split_workspace_bytes, nullptr, 0, 0, stream);
+}
+
+extern "C" int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, float* lse,
+                                int dtype, const void* q_lo, const void* k_lo, const float* q_scale,
+                                const float* k_scale,
+                                int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
+                                int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h,
+                                int64_t o_stride_n, int64_t o_stride_h, const int32_t* qo_indptr,
+                                const int32_t* kv_indptr, const int32_t* q_blk_base,
+                                const int32_t* kv_blk_base, int32_t n_q_blocks,
+                                int32_t n_kv_blocks, const int32_t* row_req,
+                                const int32_t* row_qb, const int32_t* row_head,
+                                const int32_t* kv_row_ptr, const int32_t* kv_idx,
+                                const int32_t* order, int32_t* sched, int64_t max_rows,
+                                int32_t num_heads, int32_t num_kv_heads, int32_t gqa_packed, int32_t head_dim,
+                                int32_t block_q, int32_t block_kv, float sm_scale, float logits_soft_cap,
+                                const int32_t* shares, void* split_workspace, int64_t split_workspace_bytes,
+                                void* wide, int64_t wide_bytes, int32_t batch, void* stream) {
+  return run_decoded(q, k, v, o, lse, dtype, q_lo, k_lo, q_scale, k_scale, q_stride_n, q_stride_h, k_stride_n, k_stride_h,
+                     v_stride_n, v_stride_h, o_stride_n, o_stride_h, qo_indptr, kv_indptr, q_blk_base, kv_blk_base, n_q_blocks,
+                     n_kv_blocks, row_req, row_qb, row_head, kv_row_ptr, kv_idx, order, sched, max_rows, num_heads,
+                     num_kv_heads, gqa_packed, head_dim, block_q, block_kv, sm_scale, logits_soft_cap, shares,
+                     split_workspace, split_workspace_bytes, wide, wide_bytes, batch, stream);
+}
+
+extern "C" int64_t fo_sparse_fa_wide_bytes(int64_t max_rows, int32_t num_kv_heads, int32_t n_kv_blocks) {
+  if (!wide_serves(max_rows, num_kv_heads, n_kv_blocks)) return 0;
+  return wide_head_bytes(num_kv_heads) + static_cast<int64_t>(num_kv_heads) * n_kv_blocks * kBlockKV * kHeadDim * 2;
 }
 
 extern "C" int fo_sparse_attention_direct_serves(const void* args) {

@@ -297,6 +297,32 @@ int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float
                      const int32_t* shares, void* split_workspace, int64_t split_workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * fo_sparse_fa_run with a workspace for widened fp8 operands (no counterpart in the reference).  With the
+ * two-term q and k of a long list, k is widened once per call to fp16, (k + k_lo) times its scale, and the list
+ * runs in the software-pipelined form with one fp16 product per logit, in place of three fp8 products in the
+ * 8-wavefront form: closer to the products of the four terms, which the latter takes without k_lo.q_lo.  Rows
+ * whose scales are not positive and finite, or admit a single product of a logit above 2^8 (times log2(e)), are
+ * found on the device and run in the fp8 form, in a second launch of the same call.
+ * wide: fo_sparse_fa_wide_bytes() bytes of device memory, 256-byte aligned, used by this call only (null, or a
+ * call that does not use it: as fo_sparse_fa_run); batch: number of requests, kv_blk_base[batch] = n_kv_blocks.
+ * fo_sparse_fa_wide_bytes: 0 where the list is too short (max_rows below 8 per CU) or the batch has more than
+ * 3072 kv blocks.
+ * ------------------------------------------------------------------------------------------- */
+int64_t fo_sparse_fa_wide_bytes(int64_t max_rows, int32_t num_kv_heads, int32_t n_kv_blocks);
+int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, float* lse, int dtype,
+                          const void* q_lo, const void* k_lo, const float* q_scale, const float* k_scale,
+                          int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
+                          int64_t v_stride_n, int64_t v_stride_h, int64_t o_stride_n, int64_t o_stride_h,
+                          const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* q_blk_base,
+                          const int32_t* kv_blk_base, int32_t n_q_blocks, int32_t n_kv_blocks,
+                          const int32_t* row_req, const int32_t* row_qb, const int32_t* row_head,
+                          const int32_t* kv_row_ptr, const int32_t* kv_idx, const int32_t* order, int32_t* sched,
+                          int64_t max_rows, int32_t num_heads, int32_t num_kv_heads, int32_t gqa_packed,
+                          int32_t head_dim, int32_t block_q, int32_t block_kv, float sm_scale,
+                          float logits_soft_cap, const int32_t* shares, void* split_workspace,
+                          int64_t split_workspace_bytes, void* wide, int64_t wide_bytes, int32_t batch, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * The same attention straight from the packed symbols, without a decoded list: short lists whose rows
  * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)

@@ -289,6 +289,42 @@ def test_fp8_attention(dev, case, two_term):
         assert err <= 4.5e-2       # not the contract: the level two e4m3 operands explain
 
 
+@pytest.mark.parametrize("n", [640, 300])
+def test_fp8_rows_that_cannot_be_widened(dev, n):
+    """Two-term q and k whose scales fp16 cannot hold, beside ones that it can: an outlier block and a scale that
+    is not a number in k, both not kept by any row, a q block of huge scale that is cached (its scale is whatever
+    the buffer held), a head of tiny values and an ordinary one."""
+    import flashomni_amd as fo
+    heads = 4
+    m = make_ragged_masks([n], [n], heads, 0.8, 0.7, seed=31)
+    info, keep = m["info"][0], m["keep"][0]
+    keep[:, 0, 0] = keep[:, 1, 1] = False
+    info[1, 3] = False
+    m["packed_info"], m["packed_keep"] = (np.packbits(x.reshape(-1).astype(np.uint8), bitorder="little") for x in (info, keep))
+    g = torch.Generator().manual_seed(31)
+    q, k, v = (torch.randn(n, heads, 128, generator=g) for _ in range(3))
+    k[:128, 0] *= 300
+    q[:, 2] *= 2.0 ** -40
+    k[:, 2] *= 2.0 ** 40
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    t = lambda a: torch.from_numpy(a).to(dev)
+    ip = torch.tensor([0, n], dtype=torch.int32)
+    q8, qs, q_lo = fo.quant_fp8_block(q.to(dev), ip, residual=True)
+    k8, ks, k_lo = fo.quant_fp8_block(k.to(dev), ip, residual=True)
+    ks[1, 1] = float("nan")
+    qs[3, 1] = 1e30
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(ip, ip, heads, heads, 128, q_data_type=torch.float8_e4m3fn)
+    out0 = sentinel_like((n, heads, 128), torch.bfloat16)
+    sym = [m[x] for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    exp = oracle.sparse_attention(q8.cpu(), k8.cpu(), v, *sym, m["qo_indptr"], m["kv_indptr"], out=out0.clone(),
+                                  q_scale=qs.cpu(), k_scale=ks.cpu().nan_to_num(1.0), q_lo=q_lo.cpu(), k_lo=k_lo.cpu())
+    for _ in range(2):
+        out = out0.clone().to(dev)
+        w.run(q8, k8, v.to(dev), *(t(x) for x in sym), out=out, q_scale=qs, k_scale=ks, q_lo=q_lo, k_lo=k_lo)
+        _check(out.cpu(), exp, out0, m, heads)
+
+
 @pytest.mark.parametrize("config", [4])
 def test_fp8_attention_video_shape_sampled_rows(dev, config):
     """fp8 attention (two-term q) at config 4's full size on unit-variance q, k, v: sampled rows within the
