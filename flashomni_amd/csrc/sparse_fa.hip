@@ -257,7 +257,12 @@ __device__ __forceinline__ s16x4 lds_read_tr16(const uint8_t* p) {
 __device__ __forceinline__ float max_across_halves(float x) {
   const unsigned u = __builtin_bit_cast(unsigned, x);
   const u32x2 r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+  // (Each element in a scalar first: a bit cast of a vector's element reads element 0 whichever is named, and
+  // then this was the maximum of the lower half.  And the instruction itself: fmaxf quiets both operands first.)
+  const unsigned lo = r[0], hi = r[1];
+  float m;
+  asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(lo), "v"(hi));
+  return m;
 }
 
 // words of `sched` (written by the decoder): [0..8] queue bounds inside `order`, [16..23] queue

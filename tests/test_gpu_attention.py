@@ -415,6 +415,39 @@ def test_logits_that_move_the_running_max(dev, sign):
     assert float(((lse.cpu() - exp_lse).abs() / (1.0 + exp_lse.abs())).max()) < 2e-3
 
 
+@pytest.mark.parametrize("dtype,fp8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("nk", [32, 129, 1000])
+def test_logits_far_apart(dev, dtype, fp8, nk):
+    """Logits hundreds apart in the log2 domain, the largest of a tile anywhere in it: every value of p is at most
+    2^8 of the row's reference point, in the half of a wavefront that holds the largest and in the other."""
+    import flashomni_amd as fo
+    heads, nq = 2, 200
+    m = make_ragged_masks([nq], [nk], heads, 1.0, 1.0, seed=5)
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(n, heads, 128, generator=g) for n in (nq, nk, nk))
+    q, k, v = (8 * q).to(dtype), (8 * k).to(dtype), v.to(dtype)
+    extra = {}
+    if fp8:
+        qi, ki = torch.tensor([0, nq], dtype=torch.int32), torch.tensor([0, nk], dtype=torch.int32)
+        q8, qs, q_lo = fo.quant_fp8_block(q.to(dev), qi, residual=True)
+        k8, ks, k_lo = fo.quant_fp8_block(k.to(dev), ki, residual=True)
+        extra = dict(q_scale=qs, k_scale=ks, q_lo=q_lo, k_lo=k_lo)
+        q, k = q8.cpu(), k8.cpu()
+    t = lambda a: torch.from_numpy(a).to(dev)
+    sym = [m[x] for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t(m["qo_indptr"]), t(m["kv_indptr"]), heads, heads, 128, q_data_type=q.dtype)
+    out, lse = w.run(q.to(dev), k.to(dev), v.to(dev), *(t(x) for x in sym), return_lse=True, **extra)
+    exp_lse = torch.full((nq, heads), float("nan"))
+    oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=torch.zeros(nq, heads, 128, dtype=dtype),
+                            lse=exp_lse, **{n: x.cpu() for n, x in extra.items()})
+    # A logit is off by up to 2^-9 of each of its 128 products (bf16, once more for fp8's left-out term), whose root mean
+    # square is 8 * 8 * 0.1275: 8.2 * sqrt(128) * 2^-9 / sqrt(3) = 0.1, six times that; weights that close to a tie
+    # follow it, so the output is checked as a convex combination of v only.
+    assert bool(torch.isfinite(out).all()) and float((lse.cpu() - exp_lse).abs().max()) < 0.7
+    assert float(out.abs().max()) <= float(v.abs().max()) * 1.02
+
+
 def _split_case(dev, ql, kl, heads, seed, share, dtype=torch.bfloat16, pk=0.6):
     """Run one launch (twice, to see the arrival counters re-armed) with or without rows shared
     between workgroups; returns (out, lse, sched words, expectations)."""
