@@ -58,6 +58,9 @@
 // where a cached partial is added, the request follows the stores, because the partial's pieces need
 // the staging registers).
 //
+// Launches of few units, launches whose quads would leave CUs idle and GEMM-O passes that select few heads run a
+// workgroup per unit instead (gemm_unit_kernel, gemm_packed_kernel, and the rule in launch_half).
+//
 // Work order.  Workgroups are persistent (one per CU).  The quad list is ordered by token window,
 // then column pair, then row pair, and XCD x (= blockIdx % 8) owns the x-th contiguous eighth of it.
 // The ~32 workgroups of an XCD therefore work at the same time on one token window and four
@@ -129,6 +132,9 @@ struct GemmParams {
                          // quads are enumerated arithmetically (GEMM-O, GEMM-Q with is_full)
   const int32_t* qoff;   // qoff[0..8] queue boundaries inside `quads`
   int32_t* cursor;       // GEMM-O, long launches: one work-item cursor per XCD (zero at launch), or null
+  // GEMM-O launched in both forms, as quads and as packed units: the latter run where this word (cursor[8]) is not
+  // zero, the former where it is; null: packed units only
+  const int32_t* sparse_word;
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
   int32_t n_win;         // windows of 16 token blocks per batch
   int32_t inline_cells;  // > 0: GEMM-Q builds its quad list itself from the flags of this many cells
@@ -359,9 +365,28 @@ __global__ void __launch_bounds__(kListThreads) gemm_quads_kernel(ListArgs a, Li
   }
 }
 
-// (the cursors of a launch that hands out its work items dynamically; a kernel, not a memset, so that
-// a captured graph replays it faithfully)
-__global__ void gemm_cursor_clear_kernel(int32_t* cursor) { cursor[threadIdx.x] = 0; }
+// Clears the cursors of a launch that hands out its work items dynamically (a kernel, not a memset, so that
+// a captured graph replays it faithfully), and sets cursor[8] where fewer than limit / 256 of the head slices are
+// selected, judged by up to 32768 flags of the first request from `first_byte` on.
+__global__ void __launch_bounds__(kThreads) gemm_choose_kernel(int32_t* cursor, const uint8_t* __restrict__ sparse_info,
+                                                               const int32_t* __restrict__ sparse_info_indptr,
+                                                               int32_t first_byte, int32_t n_bytes, int32_t pick, int32_t limit) {
+  __shared__ int32_t s_ones[kThreads / 64];
+  int ones = 0;
+  if (n_bytes > 0) {
+    const uint8_t* info = sparse_info + sparse_info_indptr[0] + first_byte;
+    for (int i = threadIdx.x; i < n_bytes; i += kThreads) ones += __popc(info[i]);
+  }
+  for (int off = 32; off > 0; off >>= 1) ones += __shfl_xor(ones, off, 64);
+  if ((threadIdx.x & 63) == 0) s_ones[threadIdx.x >> 6] = ones;
+  __syncthreads();
+  if (threadIdx.x < 8) cursor[threadIdx.x] = 0;
+  if (threadIdx.x == 8) {
+    for (int w = 1; w < kThreads / 64; ++w) s_ones[0] += s_ones[w];
+    const int selected = pick ? s_ones[0] : 8 * n_bytes - s_ones[0];
+    cursor[8] = 32 * selected < limit * n_bytes;
+  }
+}
 
 // ---------------------------------------------------------------------------------------------
 // Main kernel.  kReduce = false: GEMM-Q.  kReduce = true: GEMM-O.  kAux: GEMM-Q with fused
@@ -761,6 +786,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   // (the value is needed at the top of the next item and waits in a register until then).
   bool popping = false;
   if constexpr (kReduce) popping = p.cursor != nullptr;
+  if (popping && p.cursor[8] != 0) return;  // (launched in both forms, and the flags are for the other one)
   int popped = 0;
   auto pop = [&]() {
     if (tid == 0) popped = per_xcd + atomicAdd(p.cursor + xcd, 1);  // (the first per_xcd items are dealt by slot)
@@ -1666,6 +1692,269 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_unit_kernel(const GemmParams
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Launches whose quads leave a part of the chip idle: a workgroup per unit, four of them on a CU.  260 quads on
+// 256 CUs are two rounds, the second nearly empty, and 138 are one that half of the CUs sit out; GEMM-O's
+// quads walk the union of two token blocks' heads besides.  A unit per workgroup needs no list, walks its own
+// heads, and the hardware hands the next one to whichever CU is free.  What a workgroup lacks, a second slab
+// buffer and staging registers, the other three on the CU make up for: a slab is copied straight to LDS (32 KB,
+// one buffer), waited for, read and multiplied, and meanwhile the others are somewhere else in that cycle.
+// What bounds it is LDS: 96 KB written and read per unit and slab, 750 cycles at 128 B per clock beside 512 of
+// matrix core; about 920 are measured with four workgroups on every CU, against 605 per unit of a full quad.
+// (Wavefronts of 64 x 128, two per workgroup, with all operands of a slab in registers need 80 KB: 710 cycles
+// with four workgroups per CU, but a third slower where there are two or three; not kept.)
+// us, quads -> this: 2900 x 3072 (552 units) cache pass with a quarter cached 35 -> 26, final pass 66 -> 56, dense
+// 64 -> 61; 3200 x 5120 (1000 units) 112 -> 85, 197 -> 147, 212 -> 167; 8192 x 3072 (1536 units) 89 -> 75, 142 -> 135,
+// 144 -> 139; 4608 x 3072 (864 units, 216 quads in one round) 44 -> 43, 76 -> 87, 77 -> 94.
+// ---------------------------------------------------------------------------------------------
+constexpr int kPackedSmemBytes = 2 * kUnitBytes;  // one slab: X, W
+
+template <typename T, bool kReduce, bool kPartial>
+__global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmParams p) {
+  if constexpr (kReduce)
+    if (p.sparse_word != nullptr && *p.sparse_word == 0) return;
+  using TT = Types<T>;
+  using x8 = typename TT::x8;
+  using x4 = typename TT::x4;
+  constexpr int NT = 2, MT = 2;  // wavefront tile: 64 columns (W rows) x 64 token rows (X rows)
+  constexpr int kCopies = 4;     // of X and of W each, per wavefront and slab
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+  __shared__ uint16_t s_heads[kReduce ? kMaxHeads + 1 : 1];
+  __shared__ int32_t s_nsel;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, g = lane >> 5;
+  const int wr = wv >> 1, wc = wv & 1;  // half of the unit's rows, of its columns
+
+  // ---- which unit (order as in gemm_unit_kernel) ----
+  const int units_per_batch = p.n_row_tiles * p.n_col_tiles;
+  const int64_t total = static_cast<int64_t>(units_per_batch) * p.batch;
+  const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
+  const int u_lo = static_cast<int>(total * xcd / kXcds);
+  const int u = u_lo + slot;
+  if (u >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
+  const int bz = u / units_per_batch;
+  const int rem = u - bz * units_per_batch;
+  const int win = rem / (kUnitWindow * p.n_col_tiles);
+  const int in_win = rem - win * kUnitWindow * p.n_col_tiles;
+  const int win_rows = min(kUnitWindow, p.n_row_tiles - win * kUnitWindow);
+  const int col = in_win / win_rows;
+  const int row = win * kUnitWindow + in_win - col * win_rows;
+  const int m0 = row * kTile, n0 = col * kTile;
+  const uint32_t flag_row =
+      static_cast<uint32_t>(p.num_text_tokens + m0) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
+  if constexpr (!kReduce) {
+    if (p.flag == 0) {
+      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+      if (!flag_bit(info, flag_row + static_cast<uint32_t>(n0) / p.head_dim)) return;
+    }
+  }
+  int n_iter, iph = 1;
+  if constexpr (kReduce) {
+    if (wv == 0) {
+      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+      const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
+      const int n_slices = p.k / p.head_dim;
+      int count = 0;
+      for (int h0 = 0; h0 < n_slices; h0 += 64) {
+        const int h = h0 + lane;
+        const bool sel = h < n_slices && flag_bit(info, flag_row + h) == pick;
+        const unsigned long long mask = __ballot(sel);
+        if (sel) s_heads[count + __popcll(mask & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(h);
+        count += __popcll(mask);
+      }
+      if (lane == 0) s_nsel = count;
+    }
+    __syncthreads();
+    iph = p.head_dim / kBK;
+    n_iter = __builtin_amdgcn_readfirstlane(s_nsel) * iph;
+  } else {
+    n_iter = p.k / kBK;
+  }
+
+  // ---- operand tiles (rows past M read as zeros through the descriptor's range check) ----
+  const T* __restrict__ xg = static_cast<const T*>(p.x);
+  const T* __restrict__ wg = static_cast<const T*>(p.w);
+  const int rows_here = min(p.m - m0, kTile);
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(xg + (static_cast<int64_t>(bz) * p.m + m0) * p.k), 0, rows_here * p.k * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(wg + static_cast<int64_t>(n0) * p.k), 0, kTile * p.k * 2, 0x00020000);
+  // A copy is 64 lanes x 16 bytes, global -> LDS: eight rows, lane i at row i / 8 and chunk position i % 8, where
+  // logical chunk (i % 8) ^ (row / 2 % 8) belongs; row / 2 % 8 = 4 * (copy % 2) + i / 16.
+  uint32_t voff[2];
+#pragma unroll
+  for (int par = 0; par < 2; ++par)
+    voff[par] = static_cast<uint32_t>((lane >> 3) * p.k * 2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4));
+  typedef __attribute__((address_space(3))) void lds_void;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem)) + wv * kCopies * 8 * kRowBytes;
+  const uint32_t row_bytes8 = 8u * static_cast<uint32_t>(p.k) * 2u, wave_off = static_cast<uint32_t>(kCopies * wv) * row_bytes8;
+  auto copy = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(vo), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+  };
+  f32x16 acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
+
+  const int rd_x = (g ^ ((l32 >> 1) & 7)) << 4;
+  const uint8_t* const a_base = smem + kUnitBytes + (wc * 64 + l32) * kRowBytes;  // W rows
+  const uint8_t* const b_base = smem + (wr * 64 + l32) * kRowBytes;               // X rows
+  // copy j of a slab: eight rows of X (the first kCopies) or of W
+  auto slab_copy = [&](int j, uint32_t so) __attribute__((always_inline)) {
+    const int i = j % kCopies;
+    copy(j < kCopies ? rsrc_x : rsrc_w, voff[j & 1], so + i * row_bytes8, lds0 + (j < kCopies ? 0 : kUnitBytes) + i * 8 * kRowBytes);
+  };
+  uint32_t k0 = 0;
+  int head = 0, sub = 0;
+  if constexpr (kReduce) {
+    if (n_iter > 0) k0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(s_heads[0])) * p.head_dim;
+  }
+  if (n_iter > 0) {
+#pragma unroll
+    for (int j = 0; j < 2 * kCopies; ++j) slab_copy(j, k0 * 2u + wave_off);
+  }
+  for (int it = 0; it < n_iter; ++it) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    x8 a[2][NT], b[2][MT];
+    auto lread = [&](int ks) __attribute__((always_inline)) {
+      const int x = rd_x ^ (ks << 5);
+#pragma unroll
+      for (int i = 0; i < NT; ++i) a[ks & 1][i] = *reinterpret_cast<const x8*>(a_base + i * 32 * kRowBytes + x);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) b[ks & 1][i] = *reinterpret_cast<const x8*>(b_base + i * 32 * kRowBytes + x);
+    };
+    lread(0);
+    if constexpr (kReduce) {
+      if (++sub < iph) {
+        k0 += kBK;
+      } else {
+        sub = 0;
+        ++head;
+        k0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(s_heads[min(head, kMaxHeads - 1)])) * p.head_dim;
+      }
+    } else {
+      k0 += kBK;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) {
+        lread(ks + 1);
+      } else {
+        // every operand is in registers: the slab's place is free once that holds for every wavefront
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NT * MT; ++i) acc[i / MT][i % MT] = TT::mfma(a[ks & 1][i / MT], b[ks & 1][i % MT], acc[i / MT][i % MT]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (it + 1 < n_iter) {
+#pragma unroll
+      for (int j = 0; j < 2 * kCopies; ++j) slab_copy(j, k0 * 2u + wave_off);
+    }
+  }
+
+  // ---- epilogue: as in gemm_unit_kernel, 32 rows at a time through a wavefront's quarter of the slab ----
+  uint8_t* const region = smem + wv * (kPackedSmemBytes / 4);
+  const int col4 = lane & 15, rsub = lane >> 4;
+  const int el_off = n0 + wc * 64 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 4*i
+  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
+  auto out_rsrc = [&](const void* base, int elem_bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
+        rows_here * p.n * elem_bytes, 0x00020000);
+  };
+  auto turn = [&](auto bias_tag, auto f32_tag) {
+    using BiasT = decltype(bias_tag);
+    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
+    constexpr bool kOutF32 = decltype(f32_tag)::value;
+    constexpr int kBytes = sizeof(BiasT);
+    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!kPartial) {
+      if (p.bias_kind == FO_BIAS_VECTOR) {
+        const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + wc * 64 + col4 * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+      }
+    }
+    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      BiasVec bm[8];
+      if constexpr (kPartial) {
+        const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int r = 4 * (8 * mt + i) * p.n;
+          if constexpr (kBytes == 4) {
+            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, r * 4, 0));
+          } else {
+            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, r * 2, 0));
+          }
+        }
+      }
+      // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 256 bytes = 16 chunks)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          f32x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = acc[nt][mt][i4 * 4 + j];
+          const int chunk = nt * 8 + i4 * 2 + g;
+          *reinterpret_cast<f32x4*>(region + l32 * 256 + ((chunk ^ (l32 & 15)) << 4)) = v;
+        }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int rk = i * 4 + rsub;
+        f32x4 v = *reinterpret_cast<const f32x4*>(region + rk * 256 + ((col4 ^ (rk & 15)) << 4));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (kPartial) {
+            v[j] += static_cast<float>(bm[i][j]);
+          } else {
+            v[j] += bvec[j];
+          }
+        }
+        const int r = 4 * (8 * mt + i) * p.n;
+        if constexpr (kOutF32) {
+          // (no scalar offset: see the quads' store)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + r) * 4, 0, 2);
+        } else {
+          x4 out;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+          typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, r * 2, 2);
+        }
+      }
+    }
+  };
+  using std::false_type;
+  using std::true_type;
+  if constexpr (!kReduce) {
+    turn(T{}, false_type{});
+  } else if constexpr (kPartial) {
+    if (p.bias_f32) {
+      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
+    } else {
+      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+    }
+  } else {
+    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+  }
+}
+
 ListGeom make_geom(int32_t batch, int32_t m, int32_t n) {
   ListGeom gm;
   gm.batch = batch;
@@ -1703,6 +1992,18 @@ int launch_units(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   return FO_OK;
 }
 
+// the same, four on a CU
+template <typename T, bool kReduce, bool kAux>
+int launch_packed(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
+  p.n_row_tiles = gm.n_row_tiles;
+  p.n_col_tiles = gm.n_col_tiles;
+  const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
+  const int64_t grid = (units + kXcds - 1) / kXcds * kXcds;
+  gemm_packed_kernel<T, kReduce, kAux><<<static_cast<unsigned>(grid), kThreads, kPackedSmemBytes, stream>>>(p);
+  FO_CHECK_LAUNCH();
+  return FO_OK;
+}
+
 template <typename T, bool kReduce, bool kHalf, bool kAux>
 int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace, hipStream_t stream) {
   const int num_cu = fo_num_cu();
@@ -1715,6 +2016,37 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
   if constexpr (kReduce || !kAux) {
     if (static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles <= 2 * num_cu)
       return launch_units<T, kReduce, kHalf, kAux>(p, gm, stream);
+  }
+  // Packed units or quads, both timed with every unit computed: a CU takes ~920 cycles per unit and slab of the
+  // former (four at a time) and 2420 per quad and slab, and quads come in rounds of one per CU.
+  //   * Quads that fill little of their rounds: packed units, up to 21 / 32 where every unit is computed in full
+  //     (0.64, 1320 units of K = 3072: 136 -> 130 us; 0.66, 1360 of K = 5120: 216 -> 222; 0.66, 680: 105 -> 115), up to
+  //     49 / 64 for GEMM-O, whose quads walk more heads (680 units, a quarter cached: cache pass 59 -> 50, final pass
+  //     102 -> 97; 0.77, 2352 units of K = 3072: 116 -> 81 and 215 -> 215; 0.78, 3192 units: 163 -> 115 and 282 -> 317).
+  //   * GEMM-O's longer launches depend on the flags: a quad walks 2 p - p^2 of the head slices where p of them are
+  //     selected, a unit p, so units are ahead while p < 2 - the ratio of the two dense times (17000 x 3072, 3192
+  //     units: p = 0.25 163 -> 115, 0.75 281 -> 298).  The host does not see the flags: both forms are launched
+  //     and one of them ends at once, as a kernel of a few microseconds in front has decided.
+  // GEMM-Q with flags keeps its lists, which pack units whatever their number (at 552 units, a quarter of them
+  // flagged, 42 us against 47).
+  if constexpr (!kHalf && (kReduce || !kAux)) {
+    const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
+    const int64_t quads = static_cast<int64_t>(gm.batch) * gm.n_cp *
+                          (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
+    const int64_t rounds = (quads + num_cu - 1) / num_cu;
+    if (!use_flags && 64 * units <= (kReduce ? 49 : 42) * 4 * num_cu * rounds) return launch_packed<T, kReduce, kAux>(p, gm, stream);
+    if constexpr (kReduce) {
+      const int limit = 473 - static_cast<int>(256 * 920 * ((units + num_cu - 1) / num_cu) / (2420 * rounds));  // of 256
+      if (p.cursor != nullptr && units > 4 * num_cu && limit >= 32) {
+        const int64_t first = static_cast<int64_t>(p.num_text_tokens) / p.sparse_q_size * p.num_heads / 8;
+        const int64_t bits = static_cast<int64_t>(p.m) / p.sparse_q_size * p.num_heads;
+        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, static_cast<int32_t>(first),
+                                                       static_cast<int32_t>(bits / 8 < 4096 ? bits / 8 : 4096), p.flag == 0, limit);
+        FO_CHECK_LAUNCH();
+        p.sparse_word = p.cursor + 8;
+        if (int rc = launch_packed<T, kReduce, kAux>(p, gm, stream)) return rc;
+      }
+    }
   }
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
   // are atomic because host threads may launch concurrently, and setting it twice is harmless)
@@ -1745,9 +2077,11 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
     // save the extra launch)
     const int64_t items = static_cast<int64_t>(gm.batch) * gm.n_cp *
                           (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
-    if (kReduce && p.cursor != nullptr && items >= 4 * grid) {
-      gemm_cursor_clear_kernel<<<1, 16, 0, stream>>>(p.cursor);
-      FO_CHECK_LAUNCH();
+    if (kReduce && p.cursor != nullptr && (items >= 4 * grid || p.sparse_word != nullptr)) {
+      if (p.sparse_word == nullptr) {
+        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, 0, 0, 0, 0);
+        FO_CHECK_LAUNCH();
+      }
     } else {
       p.cursor = nullptr;
     }

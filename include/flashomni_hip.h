@@ -393,7 +393,9 @@ int fo_gemm_q(const void* x, const void* w, const void* bias, void* y, int dtype
  * order is computed arithmetically), so `workspace` may be NULL; fo_gemm_q with is_full != 0
  * likewise.  Given 64 bytes or more of 4-byte-aligned device scratch, a launch with several work
  * items per CU hands them out through cursors kept there (work items of unequal length then stay
- * neighbours in L2); launches that share the scratch must not overlap in time.
+ * neighbours in L2), and a launch of more than four tiles per CU is computed tile by tile or four tiles at
+ * a time as the density of the flags, judged on the device, makes faster (the same results, bit for bit);
+ * launches that share the scratch must not overlap in time.
  * ------------------------------------------------------------------------------------------- */
 int fo_gemm_o(const void* x, const void* w, const void* bias, void* y, int dtype, int bias_kind,
               int bias_dtype, int y_dtype, int32_t batch, int32_t m, int32_t n, int32_t k,

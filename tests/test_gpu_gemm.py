@@ -486,6 +486,68 @@ def test_workgroup_per_unit_equals_quads(dev, case, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [(1100, 128, 8, 8, 25), (130, 64, 16, 33, 128), (1025, 256, 5, 6, 20)])
+def test_packed_units_equal_quads(dev, case, dtype):
+    """Launches whose quads would fill their rounds badly run four workgroups of one unit each on a CU, better
+    filled ones quads: the same inputs as a few batch entries and as one of many give the same bits.  One and two
+    token rows past a block, an odd number of row and column blocks, heads of 64 to 256 columns."""
+    import flashomni_amd as fo
+    m, hd, heads, few, many = case
+    n = heads * hd
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    rows, cols = -(-m // 128), n // 128
+    fill = lambda batch: batch * rows * cols / (4 * cus * -(-batch * ((cols + 1) // 2) * ((rows + 1) // 2) // cus))
+    if cus == 256:
+        assert few * rows * cols > 2 * cus and fill(few) <= 42 / 64 and fill(many) > 49 / 64
+    info, packed, indptr = _flags(many, rows + 1, heads, 0.6, seed=m + hd)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(many, m, n, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+
+    def chain(x, ip):
+        full = fo.flashomni_gemm(x, w, heads, num_text_tokens=0, bias=b, is_full=True)
+        part = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=b, is_for_cache=True)
+        part32 = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, is_for_cache=True, out_dtype=torch.float32)
+        return [full, part, part32, fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part),
+                fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part32)]
+
+    everything = chain(x, ip)
+    for k, (one, all_) in enumerate(zip(chain(x[:few].contiguous(), ip[:few + 1].contiguous()), everything)):
+        assert torch.equal(one, all_[:few]), k
+    ref = torch.nn.functional.linear(x[:few].float(), w.float(), b.float())
+    assert rel_l2(everything[0][:few], ref) <= REL_L2
+
+
+@pytest.mark.parametrize("p_active", [0.0, 0.05, 0.35, 0.65, 0.95, 1.0])
+@pytest.mark.parametrize("text", [0, 256])
+def test_gemm_o_form_chosen_on_the_device(dev, p_active, text):
+    """Long GEMM-O launches are queued in two forms, of which the flags' density lets one run: both passes at
+    densities on either side of the line, none and all selected, against the same call without scratch memory, which
+    is always computed as quads."""
+    from flashomni_amd import _lib
+    L = _lib.lib()
+    m, n, heads = 16384 - 5, 1024, 8          # 1024 units
+    batch = 3                                 # 3072: quads fill their rounds
+    info, packed, indptr = _flags(batch, (text + m + 127) // 128, heads, p_active, seed=int(100 * p_active) + text)
+    g = torch.Generator(device=dev).manual_seed(text)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    ws = torch.full((64,), 7, dtype=torch.int32, device=dev)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    for cache in (1, 0):
+        outs = []
+        for scratch, size in ((ws.data_ptr(), 256), (None, 0), (ws.data_ptr(), 256)):
+            y = torch.full((batch, m, n), 7.0, dtype=torch.bfloat16, device=dev)
+            _lib.check(L.fo_gemm_o(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), 0, 0, 0, 0, batch, m, n, n, 128, heads,
+                                   pk.data_ptr(), ip.data_ptr(), text, cache, scratch, size, stream))
+            outs.append(y)
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch", [1, 2, 5])
 def test_fp32_output_rounds_to_the_16_bit_one(dev, batch, dtype):
     """GEMM-O forms the same fp32 value whatever it stores: the fp32 result rounded is the 16-bit result,
