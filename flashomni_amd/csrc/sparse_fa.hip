@@ -931,8 +931,11 @@ sparse_fa_kernel(const FaParams p) {
     const int shares = max(min(min(n_wg, total), max_n > 0 ? 3 * total / max_n : 1), 1);
     if (rows <= n_wg) {
       // parts of at most ceil(max_n / k) kv blocks: how many there are for every k
-      int longest = max(max_n, kDirectMinPart);
-      if (max_n > kDirectMinPart) {
+      // (the finest cut fits where even a row of the most parts in place of every row would)
+      const int finest = max((max_n + kDirectMaxParts - 1) / kDirectMaxParts, kDirectMinPart);
+      const bool fits = rows * (part_of(max(max_n, 1) - 1, finest) + 1) <= n_wg;
+      int longest = fits ? finest : max(max_n, kDirectMinPart);
+      if (!fits) {
         uint32_t counts[kDirectMaxParts / 2];
 #pragma unroll
         for (int k = 1; k <= kDirectMaxParts; ++k) {
