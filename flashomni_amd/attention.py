@@ -176,9 +176,17 @@ class PlannedBatch:
         return (self.share_rows and self.float_ws.data_ptr() % 16 == 0
                 and self.float_ws_bytes() >= _lib.lib().fo_sparse_fa_split_workspace_bytes())
 
+    def clears(self, q, dtype) -> bool:
+        """Whether a decode can clear the rows of a fresh output like ``q`` that nothing computes: 16-bit, the
+        planned batch's own rows and heads, and a list long enough for the decoder's launches that do so."""
+        return (dtype.itemsize == 2 and self.native.from_zero and q.device == self.device
+                and tuple(q.shape) == (self.total_q_rows, self.num_qo_heads, 128)
+                and self.n_q_blk * self.symbol_heads >= _lib.lib().fo_decode_sparse_clear_min_pairs())
+
     def decode(self, sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr,
-               is_full: bool = False) -> DecodedWorkList:
-        """fo_decode_sparse on the current stream into the work-list buffers."""
+               is_full: bool = False, clear=None) -> DecodedWorkList:
+        """fo_decode_sparse on the current stream into the work-list buffers; ``clear``: a fresh output (see
+        ``clears``)."""
         wl = self.worklist
         if not is_full:
             if sparse_info is None or sparse_kv_info is None or sparse_info_indptr is None \
@@ -205,15 +213,19 @@ class PlannedBatch:
         else:
             tensors = [None] * 4
         stream = torch.cuda.current_stream(self.device)
-        with _lib.device_guard(self.device):
-            _lib.check(_lib.lib().fo_decode_sparse(
-                _lib.ptr(tensors[0]), _lib.ptr(tensors[1]), _lib.ptr(tensors[2]), _lib.ptr(tensors[3]),
+        args = [_lib.ptr(tensors[0]), _lib.ptr(tensors[1]), _lib.ptr(tensors[2]), _lib.ptr(tensors[3]),
                 self._address(6), self._address(7), _lib.ptr(self.kv_indptr),
                 self.n_q_blk, self.symbol_heads, self.block_kv, int(bool(is_full)),
                 _lib.ptr(wl.row_req), _lib.ptr(wl.row_qb), _lib.ptr(wl.row_head), _lib.ptr(wl.kv_row_ptr),
                 _lib.ptr(wl.kv_idx), _lib.ptr(wl.counts), _lib.ptr(wl.order), _lib.ptr(wl.sched),
-                _lib.ptr(wl.scratch), _lib.ptr(wl.shares if self.split_ok else None),
-                stream.cuda_stream))
+                _lib.ptr(wl.scratch), _lib.ptr(wl.shares if self.split_ok else None)]
+        with _lib.device_guard(self.device):
+            if clear is None:
+                _lib.check(_lib.lib().fo_decode_sparse(*args, stream.cuda_stream))
+            else:
+                _lib.check(_lib.lib().fo_decode_sparse_clear(
+                    *args, _lib.ptr(clear), clear.stride(0), clear.stride(1), _lib.ptr(self.qo_indptr),
+                    self.num_qo_heads // self.num_kv_heads if self.gqa_packed else 1, stream.cuda_stream))
         self._note_list(is_full, stream)
         return wl
 
@@ -703,14 +715,18 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
                 lse = torch.empty((q.size(0), q.size(1)), dtype=torch.float32, device=q.device)
             else:
                 _check_shape_dtype_device(lse, (q.size(0), q.size(1)), torch.float32, q.device, "lse")
+        clear = None
         if out is None:
-            out = torch.zeros(q.shape[:-1] + v.shape[-1:], dtype=out_dtype, device=q.device)
+            # (long lists: the decoder's launches clear what the attention leaves, in place of a fill of all of it)
+            fresh = not reuse_decoded and v.size(-1) == 128 and pb.clears(q, out_dtype)
+            out = (torch.empty if fresh else torch.zeros)(q.shape[:-1] + v.shape[-1:], dtype=out_dtype, device=q.device)
+            clear = out if fresh else None
         else:
             _check_shape_dtype_device(out, q.shape[:-1] + v.shape[-1:], out_dtype, q.device, "out")
         if reuse_decoded:
             pb.reuse_decoded(is_full)
         else:
-            pb.decode(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full)
+            pb.decode(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full, clear=clear)
         pb.launch(q, k, v, out, lse if return_lse else None, self._kv_layout, sm_scale, q_scale, k_scale, q_lo,
                   k_lo, logits_soft_cap=self._logits_soft_cap or 0.0)
         return (out, lse) if return_lse else out

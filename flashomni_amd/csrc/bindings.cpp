@@ -1022,6 +1022,7 @@ PyMemberDef g_plan_members[] = {{"state", T_INT, offsetof(Plan, state), 0, nullp
                                 {"recorded_in", T_ULONGLONG, offsetof(Plan, recorded_in), 0, nullptr},
                                 {"recording", T_INT, offsetof(Plan, recording), READONLY, nullptr},
                                 {"recorded_full", T_INT, offsetof(Plan, recorded_full), READONLY, nullptr},
+                                {"from_zero", T_BOOL, offsetof(Plan, from_zero), READONLY, nullptr},
                                 {"sched_at", T_LONGLONG, offsetof(Plan, z.sched), READONLY, nullptr},
                                 {nullptr, 0, 0, 0, nullptr}};
 PyType_Slot g_ring_slots[] = {{Py_tp_dealloc, reinterpret_cast<void*>(ring_dealloc)}, {0, nullptr}};

@@ -116,6 +116,28 @@ def test_fresh_output_of_decoded_lists(dev, case, layout):
         assert torch.equal(w.run(q, k, v, *sym), exp)
 
 
+def test_fresh_output_of_a_decoded_fp8_list(dev):
+    """The same for fp8 q and k, whose lists are always decoded; q of other heads than planned is still refused."""
+    import flashomni_amd as fo
+    ql, kl, heads = [5000, 77], [300, 640], 30
+    m = make_ragged_masks(ql, kl, heads, 0.4, 0.5, seed=8)
+    g = torch.Generator(device=dev).manual_seed(8)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for n in (sum(ql), sum(kl), sum(kl)))
+    t = lambda n: torch.from_numpy(m[n]).to(dev)
+    q8, qs = fo.quant_fp8_block(q, torch.from_numpy(m["qo_indptr"]))
+    k8, ks = fo.quant_fp8_block(k, torch.from_numpy(m["kv_indptr"]))
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t("qo_indptr"), t("kv_indptr"), heads, heads, 128, q_data_type=torch.float8_e4m3fn)
+    sym = [t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    exp = w.run(q8, k8, v, *sym, out=torch.zeros_like(q), q_scale=qs, k_scale=ks)
+    for _ in range(3):
+        junk = torch.full((256 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
+        del junk
+        assert torch.equal(w.run(q8, k8, v, *sym, q_scale=qs, k_scale=ks), exp)
+    with pytest.raises(ValueError, match="head count"):
+        w.run(q8[:, :20].contiguous(), k8, v, *sym, q_scale=qs, k_scale=ks)
+
+
 @pytest.mark.parametrize("run_on_default", [True, False])
 def test_list_of_a_run_reused_on_another_stream(dev, run_on_default):
     """A run that took its rows from the symbols is still to come on its (busy) stream when another stream
