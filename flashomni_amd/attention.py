@@ -438,7 +438,8 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         self._kv_layout = kv_layout
         self._float_workspace_buffer = float_workspace_buffer
         # give the decoder a share table (queue-entry records; even shares for short lists); needs a
-        # float workspace of fo_sparse_fa_split_workspace_bytes().  Read at plan() time.
+        # float workspace of fo_sparse_fa_split_workspace_bytes() (33 MiB on 256 CUs; from twice that on,
+        # runs straight from the symbols may put two workgroups on a CU).  Read at plan() time.
         self._share_rows = True
         self.device = float_workspace_buffer.device
         if self.device.type != "cuda":

@@ -29,10 +29,11 @@
 //
 // Work distribution: workgroups are persistent and take rows from 8 queues (one per XCD, chosen by
 // blockIdx % 8) that the decoder filled head by head, so one XCD's L2 serves a few heads' K/V; the
-// first row by their index, further ones from the queue's cursor; an idle XCD steals from its neighbours.  The last workgroup to finish resets the queue cursors.
-// When a queue is so short that half of its XCD's workgroups would stay idle, its positions stand
-// for parts of rows (ranges of a row's kv blocks): parts publish unnormalised partial results to
-// the caller's workspace and the last one to arrive combines them (see the end of the row loop).
+// first row by their index, further ones from the queue's cursor; an idle XCD steals from its neighbours.
+// The last workgroup to finish resets the queue cursors.  A list of at most two rows per CU is instead cut
+// into one share of equal cost per workgroup, rows at the borders in parts (ranges of their kv blocks): parts
+// publish unnormalised partial results to the caller's workspace and the last one to arrive combines them
+// (see the end of the row loop).
 //
 // Between rows: while kv group 0 combines the two groups' states, one wavefront of group 1 pops the
 // next item, gathers its row's metadata and copies its kv block list into LDS, so the next row
@@ -46,7 +47,10 @@
 // pipelined in steps of 32 keys: the MFMAs of S(t+1) and P(t-1).V(t-1) are interleaved, instruction
 // by instruction, with the softmax of S(t), the operand reads four slots ahead and the copies two
 // steps ahead (see the kPipe branch of the kernel).  Measured on the video-sized lists it is ~5 %
-// faster than the two-phase form; on short lists a row's doubled latency costs more than that.
+// faster than the two-phase form; on short decoded lists, whose rows are taken whole, a row's doubled latency
+// costs more than that.  Short lists read straight from the symbols are cut in parts as fine as it takes and run
+// in it from 2.5 candidates per CU on (fo_sparse_attention_direct below); long lists of two-term fp8 q and k do
+// once their k has been widened to fp16 (kWide, wide_serves).
 //
 // Numerics follow the reference kernel (include/flashomni/attention/prefill.cuh:759-962): base-2
 // softmax p = exp2(s*c - m*c) with c = sm_scale*log2(e), P rounded to the activation type before

@@ -280,7 +280,8 @@ int64_t fo_sparse_fa_split_workspace_bytes(void);
  * independent 4-wavefront workgroups per CU, one row each, with a software-pipelined loop; shorter
  * ones as one 8-wavefront workgroup per CU whose two halves share a row.  1 / 2 force the first /
  * second form where it applies (the first needs 16-bit q, k, v, at most 3072 kv blocks in the batch
- * and kv strides that keep a request's keys within 4 GiB).  Results agree within the stated
+ * and kv strides that keep a request's keys within 4 GiB; two-term fp8 q and k take it through
+ * fo_sparse_fa_run_wide; with 1 fo_sparse_attention_direct serves no batch).  Results agree within the stated
  * tolerances, not bit for bit.  For tests and measurements. */
 int fo_sparse_fa_set_variant(int variant);
 int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float* lse, int dtype,
@@ -327,6 +328,9 @@ int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, 
  * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
  * candidates, more than 2^20 keep bits, no split workspace of fo_sparse_fa_split_workspace_bytes() bytes.
+ * With twice that many bytes, from 2.5 candidates per CU on and where a row has at most 1024 kv blocks (of one
+ * request: the share of keep bits of a candidate; of several: all kv blocks), the launch runs in the
+ * software-pipelined form, two workgroups per CU.
  * Arguments as in fo_decode_sparse (symbols, blk_req, blk_qb, is_full; n_blk symbol rows of symbol_heads
  * heads) and fo_sparse_fa_run.  sched: 1024 int32, its words [64, 576) zero before the first launch and left
  * zero by every one (it may be the sched of a decoded list).  A workgroup lists at most 4096 kv blocks of a
