@@ -1742,16 +1742,10 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
   const int col = in_win / win_rows;
   const int row = win * kUnitWindow + in_win - col * win_rows;
   const int m0 = row * kTile, n0 = col * kTile;
-  const uint32_t flag_row =
-      static_cast<uint32_t>(p.num_text_tokens + m0) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
-  if constexpr (!kReduce) {
-    if (p.flag == 0) {
-      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
-      if (!flag_bit(info, flag_row + static_cast<uint32_t>(n0) / p.head_dim)) return;
-    }
-  }
   int n_iter, iph = 1;
   if constexpr (kReduce) {
+    const uint32_t flag_row =
+        static_cast<uint32_t>(p.num_text_tokens + m0) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
     if (wv == 0) {
       const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
       const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
