@@ -300,25 +300,31 @@ __device__ __forceinline__ void load_pair_device(const float* p, float& a, float
   b = __uint_as_float(static_cast<uint32_t>(v >> 32));
 }
 
+constexpr int kQueueUneven = 15;  // word of a launch's copy of the queue bounds: their lengths differ by a round or more
+
 // Pop the next row for this workgroup from the queues, by one whole wavefront: own XCD queue first, then the
 // neighbours'.  A queue's first rows belong to the workgroups of its XCD by their index and are taken without an
-// atomic (see fetch_next); the cursor counts the positions behind them.  `first` is the queue that this
-// workgroup took its last row from.  When that one is empty all eight cursors are looked at with one load, and
-// only a queue that still holds rows is asked: the cursors share a cache line, whose atomics are carried out one
-// after the other (512 workgroups asking the other seven queues in turn took some 40 us at the end of a launch
-// whose workgroups end together: 512 rows of 8 kv blocks 89 -> 41 us, 1536 rows 153 -> 131; 256 workgroups, 512
-// rows 53 -> 46).  `q` is the launch's copy of the queue bounds.  Returns the entry's position in `order` or -1.
-__device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q, int* first, int lane) {
-  // (rows of queue x that belong to its workgroups from the start)
-  auto dealt = [&](int x) { return static_cast<int>(gridDim.x + kXcds - 1 - x) / kXcds; };
+// atomic (see fetch_next); the cursor counts the positions behind them, which begin at `behind`.  `first` is the
+// queue that this workgroup took its last row from.  When that one is empty:
+//   * Queues of about one length end together, and then there is little to find: all eight cursors are looked at
+//     with one load, and only a queue that still holds rows is asked.  The cursors share a cache line, whose atomics
+//     are carried out one after the other (512 workgroups asking the other seven queues in turn took some 40 us at
+//     the end of a launch: 512 rows of 8 kv blocks 89 -> 41 us, 1536 rows 153 -> 131; 256 workgroups: 768 rows
+//     87 -> 78, 640 rows of 15 to 26 blocks 120 -> 117).
+//   * Queues that differ by a round of rows or more (heads that do not divide by eight) have to be shared out in
+//     any case, and the others are asked in turn, without the look: 1130 rows of 12 heads 103 -> 96 us, 1050 of 10
+//     heads 78 -> 75, 790 of 6 heads 72 -> 66, 1510 rows of 12 heads on 512 workgroups 192 -> 182.
+// `q` is the launch's copy of the queue bounds.  (What the workgroups of an XCD are dealt is in `behind`, in LDS, and
+// not worked out from the grid's size, which is a scalar load from the launch's packet in front of every pop.)  Returns the entry's position in `order` or -1.
+__device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q, const int* behind, int* first, int lane) {
   int a = __builtin_amdgcn_readfirstlane(*first);
   unsigned left = a < kXcds ? 1u << a : 0u;  // queues to ask, by distance from the own one
-  for (bool looked = false;;) {
+  for (bool others = false;;) {
     while (left) {
       a = __ffs(left) - 1;
       left &= left - 1;
       const int x = (xcd + a) & (kXcds - 1);
-      const int beg = __builtin_amdgcn_readfirstlane(q[x]) + dealt(x), end = __builtin_amdgcn_readfirstlane(q[x + 1]);
+      const int beg = __builtin_amdgcn_readfirstlane(behind[x]), end = __builtin_amdgcn_readfirstlane(q[x + 1]);
       if (beg < end) {
         int pos = 0;
         if (lane == 0) pos = atomicAdd(&p.sched[16 + x], 1);
@@ -329,17 +335,21 @@ __device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q,
         }
       }
     }
-    if (looked || a >= kXcds) break;
-    looked = true;
-    bool some = false;
-    if (lane < kXcds) {
-      const int x = (xcd + lane) & (kXcds - 1);
-      const int beg = q[x] + dealt(x), end = q[x + 1];
-      // (a cursor only grows: a queue seen empty stays empty)
-      if (beg < end)
-        some = beg + __hip_atomic_load(&p.sched[16 + x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < end;
+    if (others || a >= kXcds) break;
+    others = true;
+    if (__builtin_amdgcn_readfirstlane(q[kQueueUneven])) {
+      left = 0xffu & ~((2u << a) - 1u);
+    } else {
+      bool some = false;
+      if (lane < kXcds) {
+        const int x = (xcd + lane) & (kXcds - 1);
+        const int beg = behind[x], end = q[x + 1];
+        // (a cursor only grows: a queue seen empty stays empty)
+        if (beg < end)
+          some = beg + __hip_atomic_load(&p.sched[16 + x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < end;
+      }
+      left = static_cast<unsigned>(__ballot(some));
     }
-    left = static_cast<unsigned>(__ballot(some));
   }
   *first = kXcds;
   return -1;
@@ -452,6 +462,7 @@ sparse_fa_kernel(const FaParams p) {
   };
   __shared__ RowInfo s_next_row[2];
   __shared__ int s_arrived;
+  __shared__ int s_behind[kXcds];  // the position of every queue behind the rows that are dealt
   __shared__ int s_queue[16];  // queue bounds and even-share words of `sched`, read once
   __shared__ int s_share[1];   // even shares: items of this workgroup's share handed out so far
   __shared__ int s_guess;      // queues: one past the position this workgroup popped last
@@ -517,7 +528,21 @@ sparse_fa_kernel(const FaParams p) {
   // The next row is popped by kv group 1 while kv group 0 combines and stores the current one
   // (group 1 has nothing else to do then), so the queue atomics are off the critical path.
   if constexpr (!kDirect) {
-    if (tid < 9) s_queue[tid] = p.sched[tid];
+    if (tid < kXcds) {
+      const int lo = p.sched[tid], hi = p.sched[tid + 1];
+      s_queue[tid] = lo;
+      if (tid == kXcds - 1) s_queue[kXcds] = hi;
+      s_behind[tid] = lo + static_cast<int>(gridDim.x + kXcds - 1 - tid) / kXcds;
+      // (longest and shortest of eight lanes)
+      int longest = hi - lo, shortest = longest;
+      longest = max(longest, __builtin_amdgcn_update_dpp(longest, longest, 0xb1, 0xf, 0xf, false));  // quad_perm 1 0 3 2
+      shortest = min(shortest, __builtin_amdgcn_update_dpp(shortest, shortest, 0xb1, 0xf, 0xf, false));
+      longest = max(longest, __builtin_amdgcn_update_dpp(longest, longest, 0x4e, 0xf, 0xf, false));  // quad_perm 2 3 0 1
+      shortest = min(shortest, __builtin_amdgcn_update_dpp(shortest, shortest, 0x4e, 0xf, 0xf, false));
+      longest = max(longest, __builtin_amdgcn_update_dpp(longest, longest, 0x141, 0xf, 0xf, false));  // row_half_mirror
+      shortest = min(shortest, __builtin_amdgcn_update_dpp(shortest, shortest, 0x141, 0xf, 0xf, false));
+      if (tid == 0) s_queue[kQueueUneven] = longest - shortest >= static_cast<int>(gridDim.x + kXcds - 1) / kXcds;
+    }
     if (tid >= 64 && tid < 64 + 6) s_queue[9 + tid - 64] = p.sched[kSchedEven + tid - 64];
     __syncthreads();
   }
@@ -623,7 +648,7 @@ sparse_fa_kernel(const FaParams p) {
           }
         }
       }
-      const int at = dealt ? own : pop_row(p, xcd, s_queue, &first_queue, lane);
+      const int at = dealt ? own : pop_row(p, xcd, s_queue, s_behind, &first_queue, lane);
       ri.part = 0;
       ri.parts = 1;
       ri.slot = 0;

@@ -866,10 +866,12 @@ def test_random_batches_all_options(dev, seed):
         assert float((lse.cpu()[touched] - exp_lse[touched]).abs().max()) < 2e-2
 
 
-@pytest.mark.parametrize("case", [(1, 1100, 0.9), (1, 1100, 0.05), (3, 400, 0.5), (9, 130, 0.95), (13, 100, 0.002)])
+@pytest.mark.parametrize("case", [(1, 1100, 0.9), (1, 1100, 0.05), (3, 400, 0.5), (9, 130, 0.95), (13, 100, 0.002),
+                                  (8, 140, 0.8), (16, 70, 0.95)])
 def test_queues_of_uneven_length(dev, case):
     """Queues that hold less than their XCD's workgroups take at the start, queues that hold nothing and ones that
-    the other XCDs empty: every row once, and again after the cursors were rewound."""
+    the other XCDs empty, asked in turn; queues that differ by less than a round, which are looked at first: every
+    row once, and again after the cursors were rewound."""
     import flashomni_amd as fo
     heads, blocks, pa = case
     ql, kl = [blocks * 128 - 5], [200]
