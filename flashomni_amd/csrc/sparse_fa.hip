@@ -67,6 +67,7 @@
 
 namespace {
 
+using fo::wave_max;
 using fo::wave_scan;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -925,7 +926,7 @@ sparse_fa_kernel(const FaParams p) {
       mx = max(mx, n[u]);
     }
     const int rows_incl = wave_scan(rows_mine), n_incl = wave_scan(n_mine);
-    for (int off = 32; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off, 64));
+    mx = wave_max(mx);
     if (lane == 63) {
       s_wave[0][wv] = rows_incl;
       s_wave[1][wv] = n_incl;
