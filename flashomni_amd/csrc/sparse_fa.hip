@@ -436,7 +436,7 @@ sparse_fa_kernel(const FaParams p) {
   struct RowInfo : std::conditional<kDirect, DirectMask, NoMask>::type {
     int row, part, parts, slot, req, qb, head, q_begin, q_rows, kv_begin, kv_len, ptr0, nb;
     float q_scale;  // fp8: dequantisation scale of the row's q block
-    int k_scale0;   // fp8: position of the request's first kv block in k_scale (the kv head's row)
+    int k_scale0;   // fp8: position of the request's first kv block in k_scale (the kv head's row); kWide: in k16
   };
   // (fetched with the rest of the record: read in the row's prologue, they would wait behind every
   // tile copy in flight)
@@ -446,9 +446,7 @@ sparse_fa_kernel(const FaParams p) {
     if constexpr (kFp8 || kWide)
       it.q_scale = p.q_scale[static_cast<int64_t>(it.head) * p.n_q_blocks + p.q_blk_base[it.req] + it.qb];
     if constexpr (kWide) it.q_scale *= p.wide_factor[it.head / p.kv_group];
-    if constexpr (kFp8) {
-      it.k_scale0 = (it.head / p.kv_group) * p.n_kv_blocks + p.kv_blk_base[it.req];
-    }
+    if constexpr (kFp8 || kWide) it.k_scale0 = (it.head / p.kv_group) * p.n_kv_blocks + p.kv_blk_base[it.req];
   };
   // q_begin: first token of the item's q rows; q_rows: how many of its 128 rows exist
   auto set_q_range = [&](RowInfo& it, const int32_t* ends) {
@@ -1250,8 +1248,10 @@ sparse_fa_kernel(const FaParams p) {
       const int last_valid = min(kBlockKV, kv_len - s_blk[nb - 1] * kBlockKV);
       const int n_steps = 4 * (nb - 1) + ((last_valid + kStep - 1) / kStep);
       const int kv_head = head / p.kv_group;
+      // (a widened k is laid out block by block, wherever the batch's tokens begin)
       const uint8_t* k_head = reinterpret_cast<const uint8_t*>(
-          kp + static_cast<int64_t>(kv_begin) * p.k_sn + static_cast<int64_t>(kv_head) * p.k_sh);
+          kp + (kWide ? static_cast<int64_t>(__builtin_amdgcn_readfirstlane(ri.k_scale0)) * (kBlockKV * kHeadDim)
+                      : static_cast<int64_t>(kv_begin) * p.k_sn + static_cast<int64_t>(kv_head) * p.k_sh));
       const uint8_t* v_head = reinterpret_cast<const uint8_t*>(
           vp + static_cast<int64_t>(kv_begin) * p.v_sn + static_cast<int64_t>(kv_head) * p.v_sh);
       // K and V copies go through buffer descriptors that end with the request's last key: a copy
@@ -2320,8 +2320,8 @@ sparse_fa_kernel(const FaParams p) {
 }
 
 // The two-term fp8 k of a long list, widened once per call: k16 = (k + k_lo) * k_scale * 2^-e in fp16, kv head by
-// kv head ([num_kv_heads][n_kv_blocks * 128][128], tokens as numbered by kv_indptr), e per kv head such that its
-// largest value lies in [1, 2); q's factor, applied where a row is begun, carries 2^e back.  The fp8 form multiplies
+// kv head ([num_kv_heads][n_kv_blocks][128][128], blocks numbered as in k_scale, so that the room does not depend on where
+// the batch's tokens begin; a request's last block is filled as far as the request goes), e per kv head such that its largest value lies in [1, 2); q's factor, applied where a row is begun, carries 2^e back.  The fp8 form multiplies
 // three times (k.q, k.q_lo, k_lo.q) in the two-phase loop; fp16 operands take one product in the pipelined loop and
 // leave nothing out.  A sum of two e4m3 terms has at most 8 significant bits and an error of 2^-9 of its own, fp16
 // keeps 11, so the logits are closer to the products of the four terms than the fp8 form's, which leaves k_lo.q_lo out.
@@ -2365,7 +2365,7 @@ __global__ void __launch_bounds__(256) widen_k_kernel(
   const int len = min(kBlockKV, kv_indptr[req + 1] - tok0);
   const float f = k_scale[static_cast<int64_t>(head) * n_kv_blocks + blk] * (1.f / two_e);
   const int col = (tid & 7) * 16;
-  _Float16* out = k16 + (static_cast<int64_t>(head) * n_kv_blocks * kBlockKV + tok0) * kHeadDim + col;
+  _Float16* out = k16 + (static_cast<int64_t>(head) * n_kv_blocks + blk) * (kBlockKV * kHeadDim) + col;
   const int64_t in = static_cast<int64_t>(tok0) * k_sn + static_cast<int64_t>(head) * k_sh + col;
   u32x4 hi[4], lo[4];
 #pragma unroll
@@ -2578,7 +2578,6 @@ int run_decoded(const void* q, const void* k, const void* v, void* o, float* lse
       FaParams w = p;
       w.k = k16;
       w.k_sn = kHeadDim;
-      w.k_sh = static_cast<int64_t>(n_kv_blocks) * kBlockKV * kHeadDim;
       const int rc = launch<__bf16, false, false, false, 1, true, false, false, false, true>(w, max_rows, s);
       if (rc != FO_OK) return rc;
     }

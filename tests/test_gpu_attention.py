@@ -289,6 +289,60 @@ def test_fp8_attention(dev, case, two_term):
         assert err <= 4.5e-2       # not the contract: the level two e4m3 operands explain
 
 
+@pytest.mark.parametrize("heads,terms", [(3, None), (24, None), (40, None)] + [(h, n) for h in (3, 40) for n in (0, 1, 2)])
+def test_batch_that_does_not_begin_at_token_0(dev, kernel_variant, heads, terms, monkeypatch):
+    """qo_indptr and kv_indptr that begin behind the first token of q / k and v (a part of a larger batch), in every
+    form: 3 heads are a short list, 24 a short one in the pipelined form, 40 are decoded.  terms: 16-bit, or fp8 with
+    that many second terms (of q, of q and k).  Nothing outside of the batch's rows changes, and the room for a widened
+    k (two second terms, long form) is not left: 4 KB of a pattern behind it stay."""
+    import flashomni_amd as fo
+    from flashomni_amd import _lib
+    q_from, k_from = 512, 640
+    m = make_ragged_masks([1300, 2300], [600, 333], heads, 0.75, 0.5, seed=heads)
+    m["qo_indptr"] = m["qo_indptr"] + np.int32(q_from)
+    m["kv_indptr"] = m["kv_indptr"] + np.int32(k_from)
+    g = torch.Generator().manual_seed(heads)
+    nq, nk = int(m["qo_indptr"][-1]) + 77, int(m["kv_indptr"][-1]) + 33
+    q = torch.randn(nq, heads, 128, generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(nk, heads, 128, generator=g).to(torch.bfloat16) for _ in range(2))
+    t = lambda a: torch.from_numpy(a).to(dev)
+    qo_ip, kv_ip = torch.from_numpy(m["qo_indptr"]), torch.from_numpy(m["kv_indptr"])
+    qd, kd, given = q.to(dev), k.to(dev), {}
+    if terms is not None:
+        qd, qs, q_lo = fo.quant_fp8_block(qd, qo_ip, residual=True)
+        kd, ks, k_lo = fo.quant_fp8_block(kd, kv_ip, residual=True)
+        given = dict(q_scale=qs, k_scale=ks)
+        if terms >= 1:
+            given["q_lo"] = q_lo
+        if terms == 2:
+            given["k_lo"] = k_lo
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(qo_ip, kv_ip, heads, heads, 128, q_data_type=qd.dtype)
+    sym = [m[x] for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    out0 = sentinel_like((nq, heads, 128), torch.bfloat16)
+    exp = oracle.sparse_attention(qd.cpu(), kd.cpu(), v, *sym, m["qo_indptr"], m["kv_indptr"], out=out0.clone(),
+                                  **{x: y.cpu() for x, y in given.items()})
+    room = _lib.lib().fo_sparse_fa_wide_bytes(w._planned.max_rows, heads, w._planned.n_kv_blk) if terms == 2 else 0
+    assert (room > 0) == (terms == 2 and kernel_variant == "one_group")
+    behind, empty = [], torch.empty
+
+    def empty_and_more(*size, **kw):
+        if room and size == (room,) and kw.get("dtype") is torch.uint8:
+            buf = torch.full((room + 4096,), 0xA5, dtype=torch.uint8, device=dev)
+            behind.append(buf[room:])
+            return buf[:room]
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty_and_more)
+    out = w.run(qd, kd, v.to(dev), *(t(x) for x in sym), out=out0.clone().to(dev), **given)
+    fresh = w.run(qd, kd, v.to(dev), *(t(x) for x in sym), **given)
+    monkeypatch.undo()
+    assert len(behind) == (2 if room else 0) and all(bool((b == 0xA5).all()) for b in behind)
+    _check(out.cpu(), exp, out0, m, heads)
+    _check(fresh.cpu(), torch.where(_touched(m, heads, exp.shape)[..., None], exp, torch.zeros_like(exp)),
+           torch.zeros_like(out0), m, heads)
+
+
 @pytest.mark.parametrize("n", [640, 300])
 def test_fp8_rows_that_cannot_be_widened(dev, n):
     """Two-term q and k whose scales fp16 cannot hold, beside ones that it can: an outlier block and a scale that
