@@ -540,7 +540,10 @@ sparse_fa_kernel(const FaParams p) {
       shortest = min(shortest, __builtin_amdgcn_update_dpp(shortest, shortest, 0x4e, 0xf, 0xf, false));
       longest = max(longest, __builtin_amdgcn_update_dpp(longest, longest, 0x141, 0xf, 0xf, false));  // row_half_mirror
       shortest = min(shortest, __builtin_amdgcn_update_dpp(shortest, shortest, 0x141, 0xf, 0xf, false));
-      if (tid == 0) s_queue[kQueueUneven] = longest - shortest >= static_cast<int>(gridDim.x + kXcds - 1) / kXcds;
+      if (tid == 0) {
+        s_queue[kQueueUneven] = longest - shortest >= static_cast<int>(gridDim.x + kXcds - 1) / kXcds;
+        s_guess = 0;  // (read first by a workgroup that is dealt no row)
+      }
     }
     if (tid >= 64 && tid < 64 + 6) s_queue[9 + tid - 64] = p.sched[kSchedEven + tid - 64];
     __syncthreads();

@@ -343,6 +343,31 @@ def test_batch_that_does_not_begin_at_token_0(dev, kernel_variant, heads, terms,
            torch.zeros_like(out0), m, heads)
 
 
+@pytest.mark.parametrize("heads,p_active", [(1, 1.0), (2, 0.7), (7, 0.9), (8, 0.0)])
+def test_workgroups_that_are_dealt_no_row(dev, heads, p_active):
+    """Queues with one record per entry where whole XCDs hold none (fewer than eight heads) or no queue does (every q
+    block cached): the workgroups there begin with a neighbour's queue, or leave."""
+    import flashomni_amd as fo
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    blocks = max(int(2.2 * n_cu / (heads * max(p_active, 0.5))), 1100 // heads)
+    m = make_ragged_masks([blocks * 128 - 5], [300], heads, p_active, 0.6, seed=heads)
+    g = torch.Generator().manual_seed(heads)
+    nq = int(m["qo_indptr"][-1])
+    q = torch.randn(nq, heads, 128, generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(300, heads, 128, generator=g).to(torch.bfloat16) for _ in range(2))
+    t = lambda a: torch.from_numpy(a).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t(m["qo_indptr"]), t(m["kv_indptr"]), heads, heads, 128, q_data_type=torch.bfloat16)
+    sym = [m[x] for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    out0 = sentinel_like((nq, heads, 128), torch.bfloat16)
+    exp = oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=out0.clone())
+    for _ in range(2):
+        out = out0.clone().to(dev)
+        w.run(q.to(dev), k.to(dev), v.to(dev), *(t(x) for x in sym), out=out)
+        assert int(w._worklist.sched[31]) == 1
+        _check(out.cpu(), exp, out0, m, heads)
+
+
 @pytest.mark.parametrize("n", [640, 300])
 def test_fp8_rows_that_cannot_be_widened(dev, n):
     """Two-term q and k whose scales fp16 cannot hold, beside ones that it can: an outlier block and a scale that
