@@ -685,9 +685,13 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         return): the logits are computed from ``q + q_lo``, which leaves only the rounding of ``k``
         in them and brings the output within relative L2 3e-2 of the unquantised result for
         unit-variance q (two e4m3 operands alone give ~3.9e-2).  ``k_lo`` (needs ``q_lo``): the
-        same for ``k`` (``quant_fp8_block(k, ..., residual=True)``); the logits then are
-        ``k.q + k.q_lo + k_lo.q`` under the same scales, as accurate as 16-bit logits, for data
-        on which one e4m3 byte per element of ``k`` is too coarse (q with rms well above 1).
+        same for ``k`` (``quant_fp8_block(k, ..., residual=True)``); the logits are then as accurate
+        as 16-bit ones, for data on which one e4m3 byte per element of ``k`` is too coarse (q with
+        rms well above 1).  They are ``k.q + k.q_lo + k_lo.q`` under the same scales, or, on lists
+        of at least eight (q block, head) pairs per CU and up to 3072 kv blocks, the one product of
+        ``k + k_lo`` and ``q + q_lo``, each rounded to fp16 (11 bits, which hold the sum but for
+        residuals below 2^-7 of their value's binade; nothing is left out): closer to the four
+        terms' products unless a second term is zero throughout.
 
         ``reuse_decoded`` (keyword-only extension): the symbols are decoded on every call, because
         a buffer rewritten in place (by a kernel of the caller's, through the C ABI, ...) looks the

@@ -171,9 +171,9 @@ struct FaParams {
   uint8_t* keep_kv_info;
   int32_t* keep_indptr;
   int32_t info_bytes, kv_info_bytes;
-  // widened fp8 operands (see widen_k_kernel; null: none): the factor of q per kv head, and a word that the
-  // widened form sets when it has left rows to the fp8 form of the same call
-  const float* wide_factor;
+  // widened fp8 operands (see widen_k_kernel; null: none): smallest and largest k scale of every kv head, and a word
+  // that the widened form sets when it has left rows to the fp8 form of the same call
+  const f32x2* wide_range;
   int32_t* wide_left;
 };
 
@@ -211,20 +211,24 @@ struct Types<_Float16> {
   }
 };
 
-// Whether a row's q, scale times the kv head's factor, can be widened: no single product of a logit above 2^8.
-// (464 = the largest sum of two e4m3 terms, 2 = the bound of a widened k; not for a scale that is not a number)
-__device__ __forceinline__ bool wide_holds(float q_scale, float c) { return 464.f * 2.f * q_scale * fabsf(c) <= 256.f && q_scale > 0.f; }
+// Whether a row runs with widened operands: the factors of its products (softmax scale c, q's scale, the k scales of its
+// kv head, between range[0] and range[1]) are positive and ordinary numbers.  (False for what is not a number.)
+__device__ __forceinline__ bool wide_holds(float q_scale, f32x2 range, float c) {
+  const float f = c * q_scale;
+  return f > 0.f && f * range[0] >= 0x1p-100f && f * range[1] <= 0x1p+90f;
+}
 
-// eight e4m3 pairs (hi + lo) * f, rounded once to fp16
-__device__ __forceinline__ void widen8(u32x2 hi, u32x2 lo, float f, f16x8& out) {
+// eight e4m3 pairs, hi + lo rounded once to fp16: both terms are multiples of 2^-9 of at most 448, so the sum is an ordinary
+// fp16 number, and exact unless it takes more than 11 bits
+__device__ __forceinline__ void widen8(u32x2 hi, u32x2 lo, f16x8& out) {
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const f32x2 h0 = __builtin_amdgcn_cvt_pk_f32_fp8(hi[j], false), h1 = __builtin_amdgcn_cvt_pk_f32_fp8(hi[j], true);
     const f32x2 l0 = __builtin_amdgcn_cvt_pk_f32_fp8(lo[j], false), l1 = __builtin_amdgcn_cvt_pk_f32_fp8(lo[j], true);
-    out[4 * j + 0] = static_cast<_Float16>((h0[0] + l0[0]) * f);
-    out[4 * j + 1] = static_cast<_Float16>((h0[1] + l0[1]) * f);
-    out[4 * j + 2] = static_cast<_Float16>((h1[0] + l1[0]) * f);
-    out[4 * j + 3] = static_cast<_Float16>((h1[1] + l1[1]) * f);
+    out[4 * j + 0] = static_cast<_Float16>(h0[0] + l0[0]);
+    out[4 * j + 1] = static_cast<_Float16>(h0[1] + l0[1]);
+    out[4 * j + 2] = static_cast<_Float16>(h1[0] + l1[0]);
+    out[4 * j + 3] = static_cast<_Float16>(h1[1] + l1[1]);
   }
 }
 
@@ -401,7 +405,8 @@ constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologu
 // fp8 matrix cores run at twice the 16-bit rate, so the two terms cost what a 16-bit S^T costs.
 // kKLo: k comes as two e4m3 terms as well, k + k_lo; S^T = k.q^T + k.q_lo^T + k_lo.q^T (the product
 // of the two residuals, 2^-8 of the logit, is left out): both operands then carry ~7 significant
-// bits and the logits are as accurate as 16-bit ones.  This is the accuracy form, not a fast one.
+// bits and the logits are as accurate as 16-bit ones.  This is the accuracy form, not a fast one.  Long lists of
+// such operands run with both widened to fp16 where there is room for it (kWide, see widen_k_kernel): one product.
 //
 // kGroups: kv groups of a workgroup.  2: the form described at the top of this file (8 wavefronts).
 // 1: a workgroup is 4 wavefronts (q sub-tiles 0..3) that walk all tiles of the row, two such
@@ -445,7 +450,6 @@ sparse_fa_kernel(const FaParams p) {
     it.k_scale0 = 0;
     if constexpr (kFp8 || kWide)
       it.q_scale = p.q_scale[static_cast<int64_t>(it.head) * p.n_q_blocks + p.q_blk_base[it.req] + it.qb];
-    if constexpr (kWide) it.q_scale *= p.wide_factor[it.head / p.kv_group];
     if constexpr (kFp8 || kWide) it.k_scale0 = (it.head / p.kv_group) * p.n_kv_blocks + p.kv_blk_base[it.req];
   };
   // q_begin: first token of the item's q rows; q_rows: how many of its 128 rows exist
@@ -1205,10 +1209,10 @@ sparse_fa_kernel(const FaParams p) {
     // one of the two forms of a call with widened operands takes this row
     bool other_form = false;
     if constexpr (kWide) {
-      other_form = !wide_holds(ri.q_scale, c);
+      other_form = !wide_holds(ri.q_scale, p.wide_range[head / p.kv_group], c);
       if (other_form && tid == 0) *p.wide_left = 1;
     } else if constexpr (kKLo) {
-      if (p.wide_left != nullptr) other_form = wide_holds(ri.q_scale * p.wide_factor[head / p.kv_group], c);
+      if (p.wide_left != nullptr) other_form = wide_holds(ri.q_scale, p.wide_range[head / p.kv_group], c);
     }
     if (nb == 0 || other_form) {
       // listed row without kv blocks: zeros, lse = -5e4
@@ -1322,6 +1326,21 @@ sparse_fa_kernel(const FaParams p) {
       if (n_steps > 1) copy_k(1);
       if (n_steps > 2) copy_k(2);
       copy_v(0);
+      // Block numbers of the row's list as scalars: blk0 = the block of the current four steps, blk1
+      // the one after it.  They come from a register that holds 64 consecutive entries of the list,
+      // one per lane, refilled every 64 blocks: the loop itself reads no list from LDS (the wait
+      // for such a read would also wait for the operand reads in flight).
+      int blk_win = 0, blk0 = 0, blk1 = 0;
+      // kWide: the factor that makes a logit of S, per kv block: softmax scale, q block's scale, k block's scale, in fp32
+      // as in the fp8 form.  Kept like the block numbers; the first 64 are asked for beside the copies.
+      float f_win = 0.f, f_blk = 1.f;
+      auto k_factor = [&]() __attribute__((always_inline)) {
+        return p.k_scale[__builtin_amdgcn_readfirstlane(ri.k_scale0) + blk_win];
+      };
+      if constexpr (kWide) {
+        blk_win = s_blk[min(lane, nb - 1)];
+        f_win = k_factor();
+      }
       // (shares are known from the start: the next item and its kv block list are fetched beside these copies)
       if constexpr (kDirect)
         if (wv == 0) direct_next((row_it + 1) & 1);
@@ -1332,15 +1351,15 @@ sparse_fa_kernel(const FaParams p) {
       u32x4 pA[2], pB[2];  // P of a step: 2 x 8 rounded values, as 32-bit pairs
       f32x16 sA, sB;
       if constexpr (kWide) {
-        // q + q_lo under the q block's scale, the softmax scale and the kv head's factor, in fp16
+        // q + q_lo in fp16 (the scales are applied to S)
+        f_win *= c * ri.q_scale;
         const int ln_r = fresh_lane(), row = qs * 32 + (ln_r & 31);
         const uint8_t* qt = smem + 4 * kBuf + row * kRowBytes8 + (ln_r >> 5) * 8;
-        const float f = c * __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, ri.q_scale)));
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
           const uint8_t* at = qt + ((ks ^ swz8(row)) << 4);
           const u32x2 hi = *reinterpret_cast<const u32x2*>(at), lo = *reinterpret_cast<const u32x2*>(at + 128 * kRowBytes8);
-          widen8(hi, lo, f, qreg[ks]);
+          widen8(hi, lo, qreg[ks]);
         }
       } else {
         const int ln_r = fresh_lane();
@@ -1424,12 +1443,7 @@ sparse_fa_kernel(const FaParams p) {
 
 #pragma unroll
       for (int i = 0; i < 16; ++i) sB[i] = 0.f;  // S(1) accumulates from the reference point 0, moved by the first step
-      // Block numbers of the row's list as scalars: blk0 = the block of the current four steps, blk1
-      // the one after it.  They come from a register that holds 64 consecutive entries of the list,
-      // one per lane, refilled every 64 blocks: the loop itself reads no list from LDS (the wait
-      // for such a read would also wait for the operand reads in flight).
-      int blk_win = s_blk[min(lane, nb - 1)];
-      int blk0 = 0, blk1 = 0;
+      if constexpr (!kWide) blk_win = s_blk[min(lane, nb - 1)];
       typedef __attribute__((ext_vector_type(2))) T x2;
       const x2 ones2 = {static_cast<T>(1.0f), static_cast<T>(1.0f)};
       // One step (kB = t % 4 picks the LDS buffers).  Straight-line code apart from small
@@ -1468,6 +1482,8 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s_cur[i]);
         mx = max_across_halves(mx);  // row max relative to m_run
+        // (kWide: S is the plain product, its factor positive: the largest logit is the one of the largest S)
+        if constexpr (kWide) mx = __builtin_fmaf(mx, f_blk, -m_run);
         const bool first = t == 0;
         // The reference point moves always on a row's first step, afterwards only past a 2^8
         // overshoot (a rare, wavefront-uniform branch that changes registers in place): S(t), the
@@ -1482,10 +1498,12 @@ sparse_fa_kernel(const FaParams p) {
             d_part *= o_scale;
           }
           m_run += delta;
+          if constexpr (!kWide) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s_cur[i] -= delta;
+            for (int i = 0; i < 16; ++i) s_cur[i] -= delta;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s_next[i] -= delta;
+            for (int i = 0; i < 16; ++i) s_next[i] -= delta;
+          }
         }
         const f32x2 neg_m2 = {-m_run, -m_run};
         // (made opaque once per step: otherwise the eight read offsets are worked out once per
@@ -1493,10 +1511,13 @@ sparse_fa_kernel(const FaParams p) {
         uint32_t kx = kx0;
         asm volatile("" : "+v"(kx));
         float psum = 0.f;
+        f32x16 s_zero16;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_zero16[i] = 0.f;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          s_next = TS::mfma(kop[i & 3], qreg[i], s_next);
+          s_next = TS::mfma(kop[i & 3], qreg[i], kWide && i == 0 ? s_zero16 : s_next);
           // the operand of the S MFMA four slots on: second half of K(t+1), then first half of K(t+2)
           kop[i & 3] = i < 4 ? read_k(kx, (kB + 1) & 3, i + 4) : read_k(kx, (kB + 2) & 3, i - 4);
           o_acc[i & 3] = TT::mfma(vop[i & 3], __builtin_bit_cast(x8, p_prev[i >> 2]), o_acc[i & 3]);
@@ -1505,7 +1526,13 @@ sparse_fa_kernel(const FaParams p) {
           // (the two values are pinned to this slot: without the empty statements the compiler
           // gathers all exponentials of a step in front of its MFMAs)
           float e0 = s_cur[2 * i], e1 = s_cur[2 * i + 1];
-          asm volatile("" : "+v"(e0), "+v"(e1));
+          if constexpr (kWide) {
+            asm volatile("v_fma_f32 %0, %2, %4, -%5\n\tv_fma_f32 %1, %3, %4, -%5"
+                         : "=&v"(e0), "=v"(e1)
+                         : "v"(s_cur[2 * i]), "v"(s_cur[2 * i + 1]), "s"(f_blk), "v"(m_run));
+          } else {
+            asm volatile("" : "+v"(e0), "+v"(e1));
+          }
           const x2 pk = {static_cast<T>(__builtin_amdgcn_exp2f(e0)), static_cast<T>(__builtin_amdgcn_exp2f(e1))};
           uint32_t pu = __builtin_bit_cast(uint32_t, pk);
           // the row sum is taken over the rounded p, as the reference does
@@ -1514,12 +1541,16 @@ sparse_fa_kernel(const FaParams p) {
           } else {
             psum = __builtin_amdgcn_fdot2(pk, ones2, psum, false);
           }
-          // (the accumulator that held the two values is set to the reference point for its next use)
-          f32x2 r01 = neg_m2;
-          asm volatile("" : "+v"(pu), "+v"(psum), "+v"(r01));
+          if constexpr (kWide) {
+            asm volatile("" : "+v"(pu), "+v"(psum));
+          } else {
+            // (the accumulator that held the two values is set to the reference point for its next use)
+            f32x2 r01 = neg_m2;
+            asm volatile("" : "+v"(pu), "+v"(psum), "+v"(r01));
+            s_cur[2 * i] = r01[0];
+            s_cur[2 * i + 1] = r01[1];
+          }
           p_cur[i >> 2][i & 3] = pu;
-          s_cur[2 * i] = r01[0];
-          s_cur[2 * i + 1] = r01[1];
           if (i == 1 || i == 3) {
             copy_desc(v_rsrc, v_voff, v_soff + (i >> 1) * 16 * v_sn2, m0_base + vbuf((kB + 2) & 3) + (i >> 1) * 4096);
           } else if (i == 5 || i == 7) {
@@ -1542,7 +1573,12 @@ sparse_fa_kernel(const FaParams p) {
       for (int t = 0; t < n_steps; t += 4) {
         const int bi = t >> 2;
         blk0 = __builtin_amdgcn_readlane(blk_win, bi & 63);
-        if (((bi + 1) & 63) == 0) blk_win = s_blk[min(bi + 1 + lane, nb - 1)];
+        if constexpr (kWide)
+          f_blk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f_win), bi & 63));
+        if (((bi + 1) & 63) == 0) {
+          blk_win = s_blk[min(bi + 1 + lane, nb - 1)];
+          if constexpr (kWide) f_win = c * ri.q_scale * k_factor();
+        }
         blk1 = __builtin_amdgcn_readlane(blk_win, (bi + 1) & 63);
         do_step(t, B0{}, sA, sB, pB, pA);
         do_step(t + 1, B1{}, sB, sA, pA, pB);
@@ -2322,51 +2358,63 @@ sparse_fa_kernel(const FaParams p) {
   }
 }
 
-// The two-term fp8 k of a long list, widened once per call: k16 = (k + k_lo) * k_scale * 2^-e in fp16, kv head by
-// kv head ([num_kv_heads][n_kv_blocks][128][128], blocks numbered as in k_scale, so that the room does not depend on where
-// the batch's tokens begin; a request's last block is filled as far as the request goes), e per kv head such that its largest value lies in [1, 2); q's factor, applied where a row is begun, carries 2^e back.  The fp8 form multiplies
-// three times (k.q, k.q_lo, k_lo.q) in the two-phase loop; fp16 operands take one product in the pipelined loop and
-// leave nothing out.  A sum of two e4m3 terms has at most 8 significant bits and an error of 2^-9 of its own, fp16
-// keeps 11, so the logits are closer to the products of the four terms than the fp8 form's, which leaves k_lo.q_lo out.
-// What fp16 cannot hold is left to the fp8 form, row by row: k scales of a head that are not positive and finite,
-// and q blocks with which single products of a logit may exceed 2^8 (below that a q is far from fp16's largest value, and
-// what k loses under fp16's smallest step of 2^-24, in blocks far below the head's largest, moves a logit by less
-// than 128 * 2^8 * 2^-25 = 2^-10).
-// 2 bytes read and 2 written per element: 0.3 ms for 76112 tokens x 40 heads, where attention went from 11.1 to
-// 8.0 ms.
+// The two-term fp8 k of a long list, widened once per call: k16 = k + k_lo in fp16, kv head by kv head
+// ([num_kv_heads][n_kv_blocks][128][128], blocks numbered as in k_scale, so that the room does not depend on where the
+// batch's tokens begin; a request's last block is filled as far as the request goes).  The fp8 form multiplies three
+// times (k.q, k.q_lo, k_lo.q) in the two-phase loop; fp16 operands take one product in the pipelined loop.  All scales
+// stay out of the operands: they are multiplied into S in fp32, block by block, as the fp8 form does.
+// Precision: where a residual's bits lie within 11 of its value's first one the widened operand is the exact sum (it
+// always is for values that e4m3 holds by themselves); a smaller residual (|lo| < 2^-7 of the binade: one value in
+// eight) is rounded with an error of at most 2^-11 of the value, and the pair's own distance from the number it stands
+// for is up to four times as much.  The fp8 form keeps every residual, and leaves k_lo.q_lo out of every logit.  Logits
+// of 128 products against 64 bits, rms over the sum of the products' sizes, fp8 form and this: 9.4e-5 and 1.5e-5
+// (normal data, whatever the blocks' scales), 4.4e-5 and 2.8e-8 (both on the e4m3 grid, a 448 among small values),
+// 4.3e-6 and 1.2e-5 (q_lo all zero and k normal: here the fp8 form leaves nothing out; to the numbers that the pairs
+// stand for both are equally far).
+// What is left to the fp8 form, row by row: k scales of a head that are not positive and finite, and products of the
+// scales outside of 2^-100 .. 2^90.
+// 2 bytes read and 2 written per element: 0.3 ms for 76112 tokens x 40 heads, where the layer's call went from 17.3 to
+// 14.8 ms.  (With the scales rounded into the operands, and the accumulators of S beginning at the softmax's reference
+// point, 14.7.)
 __global__ void __launch_bounds__(256) widen_k_kernel(
     const uint8_t* __restrict__ k, const uint8_t* __restrict__ k_lo, int64_t k_sn, int64_t k_sh,
     const float* __restrict__ k_scale, const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_blk_base,
-    int32_t batch, int32_t n_kv_blocks, _Float16* __restrict__ k16, float* __restrict__ factor, int32_t* __restrict__ left) {
-  __shared__ float s_max[4];
+    int32_t batch, int32_t n_kv_blocks, _Float16* __restrict__ k16, f32x2* __restrict__ range, int32_t* __restrict__ left) {
+  __shared__ float s_max[4], s_min[4];
   __shared__ int s_req;
   const int blk = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (tid == 0) s_req = -1;
   __syncthreads();
-  // the request of this block, and the head's largest scale (a scale that is not positive and finite counts as infinite)
+  // the request of this block
   for (int r = tid; r < batch; r += 256)
     if (kv_blk_base[r] <= blk && blk < kv_blk_base[r + 1]) s_req = r;
-  float mx = 0.f;
-  for (int i = tid; i < n_kv_blocks; i += 256) {
-    const float v = k_scale[static_cast<int64_t>(head) * n_kv_blocks + i];
-    mx = fmaxf(mx, v > 0.f ? v : __builtin_inff());
+  // a head's smallest and largest scale, by its first workgroup (one that is not positive and finite counts as infinite)
+  if (blk == 0) {
+    float mx = 0.f, mn = __builtin_inff();
+    for (int i = tid; i < n_kv_blocks; i += 256) {
+      const float v = k_scale[static_cast<int64_t>(head) * n_kv_blocks + i];
+      mx = fmaxf(mx, v > 0.f ? v : __builtin_inff());
+      mn = fminf(mn, v);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      mn = fminf(mn, __shfl_xor(mn, off, 64));
+    }
+    if (lane == 0) {
+      s_max[wv] = mx;
+      s_min[wv] = mn;
+    }
   }
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  if (lane == 0) s_max[wv] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-  // (in this range 2^e and 2^-e are ordinary numbers; the k16 of a head outside of it is never read)
-  const bool held = mx * 448.f >= 0x1p-100f && mx * 448.f < 0x1p100f;
-  const float two_e = held ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, mx * 448.f) & 0x7f800000u) : __builtin_inff();
   if (blk == 0 && tid == 0) {
-    factor[head] = two_e;
+    range[head] = f32x2{fminf(fminf(s_min[0], s_min[1]), fminf(s_min[2], s_min[3])),
+                        fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]))};
     if (head == 0) *left = 0;
   }
   const int req = s_req;
-  if (!held || req < 0) return;
+  if (req < 0) return;
   const int tok0 = kv_indptr[req] + (blk - kv_blk_base[req]) * kBlockKV;
   const int len = min(kBlockKV, kv_indptr[req + 1] - tok0);
-  const float f = k_scale[static_cast<int64_t>(head) * n_kv_blocks + blk] * (1.f / two_e);
   const int col = (tid & 7) * 16;
   _Float16* out = k16 + (static_cast<int64_t>(head) * n_kv_blocks + blk) * (kBlockKV * kHeadDim) + col;
   const int64_t in = static_cast<int64_t>(tok0) * k_sn + static_cast<int64_t>(head) * k_sh + col;
@@ -2382,8 +2430,8 @@ __global__ void __launch_bounds__(256) widen_k_kernel(
     const int r = (tid >> 3) + 32 * i;
     if (r < len) {
       f16x8 a, b;
-      widen8(u32x2{hi[i][0], hi[i][1]}, u32x2{lo[i][0], lo[i][1]}, f, a);
-      widen8(u32x2{hi[i][2], hi[i][3]}, u32x2{lo[i][2], lo[i][3]}, f, b);
+      widen8(u32x2{hi[i][0], hi[i][1]}, u32x2{lo[i][0], lo[i][1]}, a);
+      widen8(u32x2{hi[i][2], hi[i][3]}, u32x2{lo[i][2], lo[i][3]}, b);
       f16x8* dst = reinterpret_cast<f16x8*>(out + r * kHeadDim);
       dst[0] = a;
       dst[1] = b;
@@ -2435,8 +2483,8 @@ extern "C" int64_t fo_sparse_fa_split_workspace_bytes(void) {
 }
 
 namespace {
-// widened fp8 operands: the head of the workspace (factors of the kv heads and a word), then k16
-int64_t wide_head_bytes(int32_t num_kv_heads) { return (static_cast<int64_t>(num_kv_heads) * 4 + 4 + 255) / 256 * 256; }
+// widened fp8 operands: the head of the workspace (the kv heads' ranges of scales and a word), then k16
+int64_t wide_head_bytes(int32_t num_kv_heads) { return (static_cast<int64_t>(num_kv_heads) * 8 + 4 + 255) / 256 * 256; }
 // the pipelined form is taken from this many rows on
 bool long_list(int64_t max_rows) { return max_rows >= static_cast<int64_t>(8) * fo_num_cu(); }
 bool wide_serves(int64_t max_rows, int32_t num_kv_heads, int32_t n_kv_blocks) {
@@ -2569,14 +2617,14 @@ int run_decoded(const void* q, const void* k, const void* v, void* o, float* lse
                      (reinterpret_cast<uintptr_t>(wide) & 255) == 0,
                  "sparse_fa: the workspace for widened operands must be 256-byte aligned and hold "
                  "fo_sparse_fa_wide_bytes() bytes");
-      float* factor = static_cast<float*>(wide);
-      int32_t* left = reinterpret_cast<int32_t*>(factor + num_kv_heads);
+      f32x2* range = static_cast<f32x2*>(wide);
+      int32_t* left = reinterpret_cast<int32_t*>(range + num_kv_heads);
       _Float16* k16 = reinterpret_cast<_Float16*>(static_cast<uint8_t*>(wide) + wide_head_bytes(num_kv_heads));
       widen_k_kernel<<<dim3(n_kv_blocks, num_kv_heads), 256, 0, s>>>(
           static_cast<const uint8_t*>(k), static_cast<const uint8_t*>(k_lo), k_stride_n, k_stride_h, k_scale, kv_indptr,
-          kv_blk_base, batch, n_kv_blocks, k16, factor, left);
+          kv_blk_base, batch, n_kv_blocks, k16, range, left);
       FO_CHECK_LAUNCH();
-      p.wide_factor = factor;
+      p.wide_range = range;
       p.wide_left = left;
       FaParams w = p;
       w.k = k16;

@@ -250,7 +250,8 @@ int fo_decode_sparse_static(const uint8_t* sparse_info, const uint8_t* sparse_kv
  * rounding error is left in them.  k_lo (optional, else NULL; needs q_lo): the same for k, laid out
  * like k under k's scales; the logits are then k.q^T + k.q_lo^T + k_lo.q^T (the product of the two
  * residuals is left out), as accurate as 16-bit logits at three fp8 products per tile: the
- * accuracy form for data on which one e4m3 byte per element of k is too coarse, not a fast one.
+ * accuracy form for data on which one e4m3 byte per element of k is too coarse, not a fast one
+ * (long lists: see fo_sparse_fa_run_wide).
  * A request may hold at most 524 288 kv tokens (4096 kv blocks, the list of one row is staged in
  * LDS), with k_lo 262 144: the caller checks that (the lengths live on the device).
  * (The fp8 form has no counterpart in the reference.)
@@ -299,11 +300,15 @@ int fo_sparse_fa_run(const void* q, const void* k, const void* v, void* o, float
 
 /* ---------------------------------------------------------------------------------------------
  * fo_sparse_fa_run with a workspace for widened fp8 operands (no counterpart in the reference).  With the
- * two-term q and k of a long list, k is widened once per call to fp16, (k + k_lo) times its scale, and the list
- * runs in the software-pipelined form with one fp16 product per logit, in place of three fp8 products in the
- * 8-wavefront form: closer to the products of the four terms, which the latter takes without k_lo.q_lo.  Rows
- * whose scales are not positive and finite, or admit a single product of a logit above 2^8 (times log2(e)), are
- * found on the device and run in the fp8 form, in a second launch of the same call.
+ * two-term q and k of a long list, k + k_lo is widened once per call to fp16, and the list runs in the
+ * software-pipelined form with one fp16 product per logit, in place of three fp8 products in the 8-wavefront
+ * form; the scales are multiplied into the logits in fp32, in either form.  Precision: a sum of two terms is
+ * rounded to 11 bits (which hold it but for residuals below 2^-7 of their value's binade: an error of at most
+ * 2^-11 of the value), and nothing is left out; the fp8 form rounds no operand and leaves k_lo.q_lo out.  The
+ * widened logits are closer to the products of the four terms unless q_lo or k_lo is (next to) zero throughout;
+ * a caller that wants the e4m3 products as they are passes no workspace.  Rows whose scales are not positive and
+ * finite, or whose products with the softmax scale lie outside of 2^-100 .. 2^90, are found on the device and
+ * run in the fp8 form, in a second launch of the same call.
  * wide: fo_sparse_fa_wide_bytes() bytes of device memory, 256-byte aligned, used by this call only (null, or a
  * call that does not use it: as fo_sparse_fa_run); batch: number of requests, kv_blk_base[batch] = n_kv_blocks.
  * fo_sparse_fa_wide_bytes: 0 where the list is too short (max_rows below 8 per CU) or the batch has more than

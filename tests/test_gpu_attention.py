@@ -404,6 +404,62 @@ def test_fp8_rows_that_cannot_be_widened(dev, n):
         _check(out.cpu(), exp, out0, m, heads)
 
 
+@pytest.mark.parametrize("data", ["normal", "large q", "plus or minus one", "on the grid", "blocks of mixed scale", "q on the grid"])
+def test_widened_logits_against_64_bits(dev, data):
+    """Two-term fp8 q and k: the logits of the widened form (one fp16 product, scales in fp32) are no further from the
+    products of the four terms in 64 bits than those of the fp8 form, which leaves k_lo.q_lo out.  Requests of one key,
+    whose lse is the logit itself.  Where q_lo is zero the fp8 form leaves nothing out, and what the widened k rounds
+    shows: at most 2^-11 of a value, and nothing beside the pair's own distance from the number it stands for."""
+    import flashomni_amd as fo
+    from flashomni_amd import _lib
+    heads, n = 4, 48
+    g = torch.Generator(device=dev).manual_seed(len(data))
+    rand = lambda *shape: torch.randn(*shape, generator=g, device=dev)
+    on_grid = lambda x: x.clamp(-3.9, 3.9).to(torch.float8_e4m3fn).float()
+    q, k = rand(128 * n, heads, 128), rand(n, heads, 128)
+    if data == "large q":
+        q *= 8
+    elif data == "plus or minus one":
+        q, k = q.sign(), k.sign()
+    elif data in ("on the grid", "q on the grid"):
+        # (a power of two as scale: 448 in every block)
+        q, k = on_grid(q), on_grid(k) if data == "on the grid" else k
+        q[::128, :, 0] = 448.0
+        if data == "on the grid":
+            k[:, :, 0] = 448.0
+    elif data == "blocks of mixed scale":
+        q *= torch.exp2(torch.randint(-14, 1, (n, heads, 1), generator=g, device=dev).float()).repeat_interleave(128, 0)
+        k *= torch.exp2(torch.randint(-14, 1, (n, heads, 1), generator=g, device=dev).float())
+    q, k = q.to(torch.bfloat16), k.to(torch.bfloat16)
+    v = rand(n, heads, 128).to(torch.bfloat16)
+    qo_ip, kv_ip = torch.arange(0, 128 * n + 1, 128, dtype=torch.int32), torch.arange(0, n + 1, dtype=torch.int32)
+    q8, qs, q_lo = fo.quant_fp8_block(q, qo_ip, residual=True)
+    k8, ks, k_lo = fo.quant_fp8_block(k, kv_ip, residual=True)
+    c = 1.4426950408889634 / 128 ** 0.5
+    wide_q = ((q8.double() + q_lo.double()) * qs.double().t().repeat_interleave(128, 0)[:, :, None]).view(n, 128, heads, 128)
+    wide_k = (k8.double() + k_lo.double()) * ks.double().t()[:, :, None]
+    logits = lambda a, b: (a * b[:, None]).sum(-1).mul(c).reshape(128 * n, heads)
+    exact, size = logits(wide_q, wide_k), logits(wide_q.abs(), wide_k.abs())
+    got = []
+    for variant in (2, 1):
+        _lib.check(_lib.lib().fo_sparse_fa_set_variant(variant))
+        w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+        w.plan(qo_ip, kv_ip, heads, heads, 128, q_data_type=torch.float8_e4m3fn)
+        assert (_lib.lib().fo_sparse_fa_wide_bytes(w._planned.max_rows, heads, w._planned.n_kv_blk) > 0) == (variant == 1)
+        got.append(w.run(q8, k8, v, is_full=True, q_scale=qs, k_scale=ks, q_lo=q_lo, k_lo=k_lo, return_lse=True)[1].double())
+    rms = lambda x: float((x / size).pow(2).mean().sqrt())
+    fp8, wide = rms(got[0] - exact), rms(got[1] - exact)
+    print("%s: rms error over the sum of the products' sizes: fp8 form %.2e, widened %.2e" % (data, fp8, wide))
+    # (both forms add 128 exact products in fp32 and round the scaled sum: a few 2^-24 of the sum of their sizes)
+    if data == "q on the grid":
+        assert not bool(q_lo.float().any()) and bool(k_lo.float().any())
+        assert float(((got[1] - exact).abs() / size).max()) <= 2.0 ** -11 + 2.0 ** -21
+        true = logits(q.double().view(n, 128, heads, 128), k.double())
+        assert rms(got[1] - true) <= 1.02 * rms(got[0] - true)
+    else:
+        assert wide <= max(fp8, 2.0 ** -22)
+
+
 @pytest.mark.parametrize("config", [4])
 def test_fp8_attention_video_shape_sampled_rows(dev, config):
     """fp8 attention (two-term q) at config 4's full size on unit-variance q, k, v: sampled rows within the
