@@ -135,6 +135,7 @@ class PlannedBatch:
             self._list.use_sched(self._sched())
         self.share_rows = share_rows
         self.split_ok = self._split_ws_ok()
+        self.no_room = False  # the allocator has refused the scratch of a widened k
         # [is_full, stream, streams already ordered after it] of the list the work-list buffers hold
         self.decoded = None
 
@@ -317,7 +318,7 @@ class PlannedBatch:
         return self.listed()
 
     def launch(self, q, k, v, out, lse, kv_layout, sm_scale, q_scale=None, k_scale=None, q_lo=None,
-               k_lo=None, logits_soft_cap=0.0) -> None:
+               k_lo=None, logits_soft_cap=0.0, widen_k=True) -> None:
         """Shape checks against the planned batch, then fo_sparse_fa_run over the decoded list."""
         if logits_soft_cap and logits_soft_cap > 0 and is_float8(q):
             raise NotImplementedError("the logits soft cap takes 16-bit q and k")
@@ -375,14 +376,16 @@ class PlannedBatch:
                                  "(k_scale: one row per kv head)")
         wl = self.worklist
         wide = None
-        if k_lo is not None:
+        if k_lo is not None and widen_k and not self.no_room:
             # two-term fp8 q and k of a long list: room for the widened k (see fo_sparse_fa_run_wide)
             n = _lib.lib().fo_sparse_fa_wide_bytes(self.max_rows, self.num_kv_heads, self.n_kv_blk)
             if n:
                 try:
                     wide = torch.empty(n, dtype=torch.uint8, device=self.device)
                 except torch.cuda.OutOfMemoryError:
-                    pass  # (the fp8 operands are multiplied as they are)
+                    # The fp8 operands are multiplied as they are, and no later run of this plan asks again: a
+                    # request that fails has the allocator give all its cached blocks back first, which waits.
+                    self.no_room = True
         with _lib.device_guard(self.device):
             _lib.check(_lib.lib().fo_sparse_fa_run_wide(
                 _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse),
@@ -670,6 +673,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         q_lo: Optional[torch.Tensor] = None,
         k_lo: Optional[torch.Tensor] = None,
         reuse_decoded: bool = False,
+        widen_k: bool = True,
     ) -> Union[torch.Tensor, Tuple[torch.Tensor, torch.Tensor]]:
         r"""Compute block-sparse prefill attention.
 
@@ -691,7 +695,11 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         of at least eight (q block, head) pairs per CU and up to 3072 kv blocks, the one product of
         ``k + k_lo`` and ``q + q_lo``, each rounded to fp16 (11 bits, which hold the sum but for
         residuals below 2^-7 of their value's binade; nothing is left out): closer to the four
-        terms' products unless a second term is zero throughout.
+        terms' products unless a second term is zero throughout.  That takes two bytes of scratch per
+        element of ``k``, from the caching allocator for the duration of the call (0.78 GB for 76112
+        tokens x 40 heads); where it is refused, this run and later ones of the plan multiply the fp8
+        terms.  ``widen_k=False`` (keyword-only extension) asks for neither: no scratch, the three
+        fp8 products.
 
         ``reuse_decoded`` (keyword-only extension): the symbols are decoded on every call, because
         a buffer rewritten in place (by a kernel of the caller's, through the C ABI, ...) looks the
@@ -733,7 +741,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         else:
             pb.decode(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full, clear=clear)
         pb.launch(q, k, v, out, lse if return_lse else None, self._kv_layout, sm_scale, q_scale, k_scale, q_lo,
-                  k_lo, logits_soft_cap=self._logits_soft_cap or 0.0)
+                  k_lo, logits_soft_cap=self._logits_soft_cap or 0.0, widen_k=widen_k)
         return (out, lse) if return_lse else out
 
     run_return_lse = functools.partialmethod(run, return_lse=True)

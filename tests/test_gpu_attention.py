@@ -460,6 +460,45 @@ def test_widened_logits_against_64_bits(dev, data):
         assert wide <= max(fp8, 2.0 ** -22)
 
 
+def test_widened_k_without_room(dev, kernel_variant, monkeypatch):
+    """The scratch of a widened k is asked for once per plan where it is refused, and not at all with widen_k=False;
+    either way the run is the three fp8 products, bit for bit."""
+    import flashomni_amd as fo
+    from flashomni_amd import _lib
+    heads, n = 3, 700
+    g = torch.Generator(device=dev).manual_seed(5)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    ip = torch.tensor([0, n], dtype=torch.int32)
+    q8, qs, q_lo = fo.quant_fp8_block(q, ip, residual=True)
+    k8, ks, k_lo = fo.quant_fp8_block(k, ip, residual=True)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    plan = lambda: w.plan(ip, ip, heads, heads, 128, q_data_type=torch.float8_e4m3fn)
+    run = lambda **kw: w.run(q8, k8, v, is_full=True, q_scale=qs, k_scale=ks, q_lo=q_lo, k_lo=k_lo, **kw)
+    plan()
+    room = _lib.lib().fo_sparse_fa_wide_bytes(w._planned.max_rows, heads, w._planned.n_kv_blk)
+    assert (room > 0) == (kernel_variant == "one_group")
+    _lib.check(_lib.lib().fo_sparse_fa_set_variant(2))
+    fp8 = run()
+    _lib.check(_lib.lib().fo_sparse_fa_set_variant(1 if kernel_variant == "one_group" else 0))
+    asked, empty = [], torch.empty
+
+    def refuse(*size, **kw):
+        if room and size == (room,):
+            asked.append(size)
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", refuse)
+    assert torch.equal(run(widen_k=False), fp8) and not asked
+    for _ in range(2):
+        assert torch.equal(run(), fp8) and len(asked) == (1 if room else 0)
+    plan()
+    assert torch.equal(run(), fp8) and len(asked) == (2 if room else 0)
+    monkeypatch.undo()
+    plan()
+    assert torch.equal(run(), fp8) == (room == 0)
+
+
 @pytest.mark.parametrize("config", [4])
 def test_fp8_attention_video_shape_sampled_rows(dev, config):
     """fp8 attention (two-term q) at config 4's full size on unit-variance q, k, v: sampled rows within the
