@@ -60,6 +60,11 @@ SIGNATURES = {
     "fo_symbols_from_scores": ([c_vp, c_int] + [c_i32] * 6 + [c_vp] * 7, c_int),
 }
 
+# Entry points whose several launches hand something on in scratch memory that belongs to a stream (GEMM-Q's list,
+# GEMM-O's cursors and choice of form): called with the interpreter lock held, as the native call path does, so that the
+# launches of two threads' calls on one stream do not come to lie between each other.
+ONE_CALL_AT_A_TIME = ("fo_gemm_q", "fo_gemm_q_quant", "fo_gemm_o")
+
 FO_BF16, FO_F16, FO_FP8_E4M3, FO_F32 = 0, 1, 2, 3
 FO_BIAS_NONE, FO_BIAS_VECTOR, FO_BIAS_MATRIX = 0, 1, 2
 
@@ -74,6 +79,9 @@ def lib():
                 "(there is no fallback path)" % LIB_PATH)
         handle = ctypes.CDLL(LIB_PATH)
         for name, (argtypes, restype) in SIGNATURES.items():
+            if name in ONE_CALL_AT_A_TIME:
+                setattr(handle, name, ctypes.PYFUNCTYPE(restype, *argtypes)((name, handle)))
+                continue
             fn = getattr(handle, name)
             fn.argtypes = argtypes
             fn.restype = restype
