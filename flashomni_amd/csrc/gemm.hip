@@ -366,25 +366,53 @@ __global__ void __launch_bounds__(kListThreads) gemm_quads_kernel(ListArgs a, Li
 }
 
 // Clears the cursors of a launch that hands out its work items dynamically (a kernel, not a memset, so that
-// a captured graph replays it faithfully), and sets cursor[8] where fewer than limit / 256 of the head slices are
-// selected, judged by up to 32768 flags of the first request from `first_byte` on.
+// a captured graph replays it faithfully), and sets cursor[8] where packed units are faster than quads (see launch_half):
+// with p of a request's head slices selected its units take a time of p, its quads one of 2 p - p^2, and packed units
+// 2 - limit / 256 times a quad's time for the same work, so they are ahead where the sum of p (limit / 256 - p) over the
+// requests is not negative.  (A batch is judged as a whole: by its first request alone, one of 5 % selected in front of two
+// of 95 %, 8192 x 3072 each, ran as packed units, 422 us in place of 382.)  Judged by up to 4096 bytes of flags in all, of up to 64 requests spread over the
+// batch, from each one's `first_byte` on (n_bytes: how many a request has); all of them are in flight together.
+constexpr int kJudged = 64, kJudgedBytes = 4096;
 __global__ void __launch_bounds__(kThreads) gemm_choose_kernel(int32_t* cursor, const uint8_t* __restrict__ sparse_info,
-                                                               const int32_t* __restrict__ sparse_info_indptr,
+                                                               const int32_t* __restrict__ sparse_info_indptr, int32_t batch,
                                                                int32_t first_byte, int32_t n_bytes, int32_t pick, int32_t limit) {
-  __shared__ int32_t s_ones[kThreads / 64];
-  int ones = 0;
-  if (n_bytes > 0) {
-    const uint8_t* info = sparse_info + sparse_info_indptr[0] + first_byte;
-    for (int i = threadIdx.x; i < n_bytes; i += kThreads) ones += __popc(info[i]);
+  __shared__ int32_t s_ones[kThreads / 4];
+  const int tid = threadIdx.x;
+  if (tid < 8) cursor[tid] = 0;
+  if (n_bytes == 0) {
+    if (tid == 8) cursor[8] = 0;
+    return;
   }
-  for (int off = 32; off > 0; off >>= 1) ones += __shfl_xor(ones, off, 64);
-  if ((threadIdx.x & 63) == 0) s_ones[threadIdx.x >> 6] = ones;
+  const int judged = min(batch, kJudged);
+  int threads = kThreads;  // of a request: a power of two, at least kThreads / kJudged
+  while (threads * judged > kThreads) threads >>= 1;
+  constexpr int kPer = kJudgedBytes / kThreads;
+  const int n = min(n_bytes, kPer * threads);
+  const int j = tid / threads, at = tid - j * threads;
+  int ones = 0;
+  if (j < judged) {
+    const uint8_t* info = sparse_info + sparse_info_indptr[static_cast<int64_t>(j) * batch / judged] + first_byte;
+    uint8_t v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = at + i * threads < n ? info[at + i * threads] : 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) ones += __popc(v[i]);
+  }
+  const int width = min(threads, 64);
+  for (int off = width >> 1; off > 0; off >>= 1) ones += __shfl_xor(ones, off, 64);
+  if (tid % width == 0) s_ones[tid / width] = ones;
   __syncthreads();
-  if (threadIdx.x < 8) cursor[threadIdx.x] = 0;
-  if (threadIdx.x == 8) {
-    for (int w = 1; w < kThreads / 64; ++w) s_ones[0] += s_ones[w];
-    const int selected = pick ? s_ones[0] : 8 * n_bytes - s_ones[0];
-    cursor[8] = 32 * selected < limit * n_bytes;
+  if (tid < 64) {
+    // (up to 2^15 selected times 2^21: 64 bits)
+    long long ahead = 0;
+    if (tid < judged) {
+      int selected = 0;
+      for (int w = 0; w < threads / width; ++w) selected += s_ones[tid * (threads / width) + w];
+      if (!pick) selected = 8 * n - selected;
+      ahead = static_cast<long long>(selected) * (limit * n - 32 * selected);
+    }
+    for (int off = 32; off > 0; off >>= 1) ahead += __shfl_xor(ahead, off, 64);
+    if (tid == 0) cursor[8] = ahead >= 0;
   }
 }
 
@@ -2034,8 +2062,8 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
       if (p.cursor != nullptr && units > 4 * num_cu && limit >= 32) {
         const int64_t first = static_cast<int64_t>(p.num_text_tokens) / p.sparse_q_size * p.num_heads / 8;
         const int64_t bits = static_cast<int64_t>(p.m) / p.sparse_q_size * p.num_heads;
-        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, static_cast<int32_t>(first),
-                                                       static_cast<int32_t>(bits / 8 < 4096 ? bits / 8 : 4096), p.flag == 0, limit);
+        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, gm.batch, static_cast<int32_t>(first),
+                                                       static_cast<int32_t>(bits / 8 < kJudgedBytes ? bits / 8 : kJudgedBytes), p.flag == 0, limit);
         FO_CHECK_LAUNCH();
         p.sparse_word = p.cursor + 8;
         if (int rc = launch_packed<T, kReduce, kAux>(p, gm, stream)) return rc;
@@ -2073,7 +2101,7 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
                           (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
     if (kReduce && p.cursor != nullptr && (items >= 4 * grid || p.sparse_word != nullptr)) {
       if (p.sparse_word == nullptr) {
-        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, 0, 0, 0, 0);
+        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, 0, 0, 0, 0, 0);
         FO_CHECK_LAUNCH();
       }
     } else {

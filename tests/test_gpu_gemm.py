@@ -547,6 +547,46 @@ def test_gemm_o_form_chosen_on_the_device(dev, p_active, text):
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("p_active", [(0.05, 0.95, 0.95), (0.95, 0.05, 0.05), (0.1, 0.25, 0.15), (0.9, 0.6, 0.8),
+                                      (0.0, 0.0, 0.0), (0.05,) * 70 + (0.9,) * 70])
+def test_gemm_o_form_of_a_mixed_batch(dev, p_active):
+    """The form of a long GEMM-O call is chosen by all requests (up to 64 of them, spread over the batch): the choice in
+    the scratch's ninth word is the rule's, and the results are those of the quads, bit for bit."""
+    from flashomni_amd import _lib
+    L = _lib.lib()
+    batch = len(p_active)
+    n, heads, text = 1024, 8, 128
+    m = 16384 if batch == 3 else 512
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    blocks = -(-m // 128)
+    flags = np.concatenate([_flags(1, blocks + 1, heads, p, seed=7 + i)[0] for i, p in enumerate(p_active)])
+    segs = [np.packbits(f.reshape(-1).astype(np.uint8), bitorder="little") for f in flags]
+    packed, indptr = np.concatenate(segs), np.cumsum([0] + [len(s) for s in segs]).astype(np.int32)
+    g = torch.Generator(device=dev).manual_seed(batch)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    ws = torch.full((64,), 7, dtype=torch.int32, device=dev)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    units, quads = batch * blocks * 8, batch * 4 * (blocks // 2)
+    rounds = -(-quads // n_cu)
+    limit = 473 - 256 * 920 * -(-units // n_cu) // (2420 * rounds)
+    assert units > 4 * n_cu and limit >= 32 and 64 * units > 49 * 4 * n_cu * rounds, "not a shape of both forms"
+    judged = [j * batch // min(batch, 64) for j in range(min(batch, 64))]
+    for cache in (1, 0):
+        outs = []
+        for scratch, size in ((ws.data_ptr(), 256), (None, 0)):
+            y = torch.full((batch, m, n), 7.0, dtype=torch.bfloat16, device=dev)
+            _lib.check(L.fo_gemm_o(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), 0, 0, 0, 0, batch, m, n, n, 128, heads,
+                                   pk.data_ptr(), ip.data_ptr(), text, cache, scratch, size, stream))
+            outs.append(y)
+        assert torch.equal(outs[0], outs[1])
+        n_bytes = blocks * heads // 8
+        selected = [int((flags[j, 1:] != bool(cache)).sum()) for j in judged]
+        ahead = sum(s * (limit * n_bytes - 32 * s) for s in selected)
+        assert int(ws[8]) == int(ahead >= 0)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch", [1, 2, 5])
 def test_fp32_output_rounds_to_the_16_bit_one(dev, batch, dtype):
