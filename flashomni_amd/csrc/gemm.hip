@@ -366,12 +366,12 @@ __global__ void __launch_bounds__(kListThreads) gemm_quads_kernel(ListArgs a, Li
 }
 
 // Clears the cursors of a launch that hands out its work items dynamically (a kernel, not a memset, so that
-// a captured graph replays it faithfully), and sets cursor[8] where packed units are faster than quads (see launch_half):
-// with p of a request's head slices selected its units take a time of p, its quads one of 2 p - p^2, and packed units
-// 2 - limit / 256 times a quad's time for the same work, so they are ahead where the sum of p (limit / 256 - p) over the
-// requests is not negative.  (A batch is judged as a whole: by its first request alone, one of 5 % selected in front of two
-// of 95 %, 8192 x 3072 each, ran as packed units, 422 us in place of 382.)  Judged by up to 4096 bytes of flags in all, of up to 64 requests spread over the
-// batch, from each one's `first_byte` on (n_bytes: how many a request has); all of them are in flight together.
+// a captured graph replays it faithfully), and sets cursor[8] where packed units are faster than quads: with p of a
+// request's head slices selected its quads take a time of 2 p - p^2, its units (2 - limit / 256) p, so units are ahead where the
+// sum of p (limit / 256 - p) over the requests is not negative; limit: see launch_half.  (A batch is judged as a whole:
+// by its first request alone, one of 5 % selected in front of two of 95 %, 8192 x 3072 each, ran as packed units, 422 us in
+// place of 382.)  Judged by up to 4096 bytes of flags in all, of up to 64 requests spread over the batch, from each one's
+// `first_byte` on (n_bytes: how many a request has); all of them are in flight together.
 constexpr int kJudged = 64, kJudgedBytes = 4096;
 __global__ void __launch_bounds__(kThreads) gemm_choose_kernel(int32_t* cursor, const uint8_t* __restrict__ sparse_info,
                                                                const int32_t* __restrict__ sparse_info_indptr, int32_t batch,
@@ -2039,27 +2039,41 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
     if (static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles <= 2 * num_cu)
       return launch_units<T, kReduce, kHalf, kAux>(p, gm, stream);
   }
-  // Packed units or quads, both timed with every unit computed: a CU takes ~920 cycles per unit and slab of the
-  // former (four at a time) and 2420 per quad and slab, and quads come in rounds of one per CU.
-  //   * Quads that fill little of their rounds: packed units, up to 21 / 32 where every unit is computed in full
-  //     (0.64, 1320 units of K = 3072: 136 -> 130 us; 0.66, 1360 of K = 5120: 216 -> 222; 0.66, 680: 105 -> 115), up to
-  //     49 / 64 for GEMM-O, whose quads walk more heads (680 units, a quarter cached: cache pass 59 -> 50, final pass
-  //     102 -> 97; 0.77, 2352 units of K = 3072: 116 -> 81 and 215 -> 215; 0.78, 3192 units: 163 -> 115 and 282 -> 317).
-  //   * GEMM-O's longer launches depend on the flags: a quad walks 2 p - p^2 of the head slices where p of them are
-  //     selected, a unit p, so units are ahead while p < 2 - the ratio of the two dense times (17000 x 3072, 3192
-  //     units: p = 0.25 163 -> 115, 0.75 281 -> 298).  The host does not see the flags: both forms are launched
-  //     and one of them ends at once, as a kernel of a few microseconds in front has decided.
+  // Packed units or quads.  Quads come in rounds of one per CU, so packed units are ahead where the last round is
+  // nearly empty, and in GEMM-O, whose quads walk the union of two token blocks' heads; they fall behind with the
+  // width: more of W than an XCD's L2 holds, and, where the flags differ from block to block, workgroups of
+  // neighbouring units that drift apart in it.  Measured over 2.1 to 32 units per CU, heads of 128, square W; times of
+  // packed units over quads' with 2, 25, 50, 80, 100 % of the heads selected, at 20 to 24 units per CU in full rounds:
+  //    8 heads 0.66 0.66 0.76 0.90 1.00      16  0.62 0.70 0.83 0.99 1.05      24  0.61 0.83 1.05 1.28 1.15
+  //   40 heads 0.65 0.99 1.24 1.53 1.34      64  0.70 1.12 1.56 1.91 1.31
+  //   * GEMM-O of one round: up to three units per CU (0.5 .. 1.02 with up to 80 % selected, at most 1.14 with all; four
+  //     units: 0.65 .. 1.35).
+  //   * GEMM-O of more: always up to K = 2048 (at worst 1.09, all heads selected; a choice by the flags costs 7 us, 2 to
+  //     10 % of these launches), wider up to 21 / 32 of the rounds filled (at worst 1.0) or as far as the width times
+  //     the fill is at most 18 heads' (24 heads, rounds filled to 3/4: at worst 1.05).
+  //   * Beyond that it depends on the flags, which the host does not see: both forms are launched, and one of them
+  //     ends at once, as a kernel of a few microseconds in front has decided (5 to 8 us in all where quads are
+  //     chosen, up to 3 % of these launches).  Packed units run where the selected share is below 13 heads over
+  //     (width times fill), 10 from sixteen units per CU on: the line where the two were measured equal, to 0.06 (24
+  //     heads: 0.67 at 7 units per CU and a fill of 0.88, 0.57 at 12 and 1.0, 0.41 at 24 and 1.0; 40 heads: 0.47 at 12
+  //     and 0.75, 0.32 at 10 and 0.87, 0.26 at 20 and 1.0; 64 heads: 0.23 at 10 and 0.88, 0.16 at 20 and 1.0).
+  //   * Dense GEMM-Q: up to 21 / 32 of the rounds filled (0.75 .. 1.02; at 0.75 0.85 with 8 heads, 1.14 with 40), in a single
+  //     round only up to K = 2048 (0.88 .. 1.01; 24 heads 1.05, 40 heads 1.07 .. 1.11).
   // GEMM-Q with flags keeps its lists, which pack units whatever their number (at 552 units, a quarter of them
   // flagged, 42 us against 47).
   if constexpr (!kHalf && (kReduce || !kAux)) {
     const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
     const int64_t quads = static_cast<int64_t>(gm.batch) * gm.n_cp *
                           (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
-    const int64_t rounds = (quads + num_cu - 1) / num_cu;
-    if (!use_flags && 64 * units <= (kReduce ? 49 : 42) * 4 * num_cu * rounds) return launch_packed<T, kReduce, kAux>(p, gm, stream);
+    const int64_t rounds = (quads + num_cu - 1) / num_cu, slots = 4 * num_cu * rounds;
+    const bool narrow = p.k <= 2048, few = 32 * units <= 21 * slots;
+    if (!use_flags && (rounds == 1 ? (kReduce ? units <= 3 * num_cu : narrow && few)
+                                   : few || (kReduce && (narrow || p.k * units <= 18 * 128 * slots))))
+      return launch_packed<T, kReduce, kAux>(p, gm, stream);
     if constexpr (kReduce) {
-      const int limit = 473 - static_cast<int>(256 * 920 * ((units + num_cu - 1) / num_cu) / (2420 * rounds));  // of 256
-      if (p.cursor != nullptr && units > 4 * num_cu && limit >= 32) {
+      const int64_t line = (units > 15 * num_cu ? 10 : 13) * 128 * 256 * slots / (p.k * units);
+      const int limit = static_cast<int>(line < 256 ? line : 256);  // of 256
+      if (p.cursor != nullptr && rounds > 1 && limit >= 32) {
         const int64_t first = static_cast<int64_t>(p.num_text_tokens) / p.sparse_q_size * p.num_heads / 8;
         const int64_t bits = static_cast<int64_t>(p.m) / p.sparse_q_size * p.num_heads;
         gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, gm.batch, static_cast<int32_t>(first),

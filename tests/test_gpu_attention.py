@@ -21,7 +21,8 @@ def kernel_variant(request):
     """Every test of this module runs twice: with the kernel form chosen from the list's size (short
     lists: one 8-wavefront workgroup per CU shares a row) and with the form for long lists forced
     (two 4-wavefront workgroups per CU, software-pipelined loop), which these small cases would not
-    reach on their own.  Inputs the second form does not take (fp8) run the first one either way."""
+    reach on their own.  Inputs the second form does not take (the soft cap, fp8 but for two-term q and k, whose k
+    is widened for it) run the first one either way."""
     from flashomni_amd import _lib
     _lib.check(_lib.lib().fo_sparse_fa_set_variant(1 if request.param == "one_group" else 0))
     yield request.param
@@ -370,11 +371,12 @@ def test_workgroups_that_are_dealt_no_row(dev, heads, p_active):
 
 @pytest.mark.parametrize("n", [640, 300])
 def test_fp8_rows_that_cannot_be_widened(dev, n):
-    """Two-term q and k whose scales fp16 cannot hold, beside ones that it can: an outlier block and a scale that
-    is not a number in k, both not kept by any row, a q block of huge scale that is cached (its scale is whatever
-    the buffer held), a head of tiny values and an ordinary one."""
+    """Two-term q and k whose scales the widened form leaves to the fp8 form, beside ones that it takes: a scale that is not
+    a number in a k head (in a block no row keeps), a head of k that is negative throughout one block, a q block whose
+    factors end below 2^-100 and one of negative scale between ordinary ones, a cached q block of huge scale (its scale
+    is whatever the buffer held); taken: an outlier block, tiny q against huge k."""
     import flashomni_amd as fo
-    heads = 4
+    heads = 5
     m = make_ragged_masks([n], [n], heads, 0.8, 0.7, seed=31)
     info, keep = m["info"][0], m["keep"][0]
     keep[:, 0, 0] = keep[:, 1, 1] = False
@@ -391,7 +393,10 @@ def test_fp8_rows_that_cannot_be_widened(dev, n):
     q8, qs, q_lo = fo.quant_fp8_block(q.to(dev), ip, residual=True)
     k8, ks, k_lo = fo.quant_fp8_block(k.to(dev), ip, residual=True)
     ks[1, 1] = float("nan")
+    ks[4, 0] *= -1
     qs[3, 1] = 1e30
+    qs[3, 0] *= 2.0 ** -100
+    qs[0, 2] *= -1
     w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
     w.plan(ip, ip, heads, heads, 128, q_data_type=torch.float8_e4m3fn)
     out0 = sentinel_like((n, heads, 128), torch.bfloat16)

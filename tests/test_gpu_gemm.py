@@ -547,32 +547,47 @@ def test_gemm_o_form_chosen_on_the_device(dev, p_active, text):
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
-@pytest.mark.parametrize("p_active", [(0.05, 0.95, 0.95), (0.95, 0.05, 0.05), (0.1, 0.25, 0.15), (0.9, 0.6, 0.8),
-                                      (0.0, 0.0, 0.0), (0.05,) * 70 + (0.9,) * 70])
-def test_gemm_o_form_of_a_mixed_batch(dev, p_active):
-    """The form of a long GEMM-O call is chosen by all requests (up to 64 of them, spread over the batch): the choice in
-    the scratch's ninth word is the rule's, and the results are those of the quads, bit for bit."""
+def _gemm_o_rule(n_cu, batch, m, n):
+    """launch_half's rule for heads of 128: (packed whatever the flags, quads whatever the flags, line between them)."""
+    rows, cols = -(-m // 128), n // 128
+    units, quads = batch * rows * cols, batch * (cols // 2) * (rows // 16 * 8 + (rows % 16 + 1) // 2)
+    rounds = -(-quads // n_cu)
+    slots = 4 * n_cu * rounds
+    if rounds == 1:
+        return units <= 3 * n_cu, units > 3 * n_cu, 0
+    limit = min(256, (10 if units > 15 * n_cu else 13) * 128 * 256 * slots // (n * units))
+    packed = n <= 2048 or 32 * units <= 21 * slots or n * units <= 18 * 128 * slots
+    return packed, not packed and limit < 32, limit
+
+
+@pytest.mark.parametrize("shape,p_active", [
+    ((8192, 2560), (0.05, 0.95, 0.95)), ((8192, 2560), (0.95, 0.05, 0.05)), ((8192, 2560), (0.1, 0.3, 0.2)),
+    ((8192, 2560), (0.9, 0.7, 0.8)), ((8192, 2560), (0.0, 0.0, 0.0)), ((8192, 2560), (1.0, 1.0, 1.0)),
+    ((512, 2560), (0.05,) * 35 + (0.9,) * 35),   # more requests than are judged
+    ((9609, 3072), (0.5,)), ((9609, 3072), (0.8,)),
+])
+def test_gemm_o_form_of_a_mixed_batch(dev, shape, p_active):
+    """Where the flags choose the form of a long GEMM-O call they do so for all requests (up to 64 of them, spread over
+    the batch): the choice in the scratch's ninth word is the rule's, and the results are those of the quads (the form
+    of a call without scratch), bit for bit, in either pass."""
     from flashomni_amd import _lib
     L = _lib.lib()
-    batch = len(p_active)
-    n, heads, text = 1024, 8, 128
-    m = 16384 if batch == 3 else 512
-    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
-    blocks = -(-m // 128)
+    batch, (m, n), text = len(p_active), shape, 128
+    heads, blocks = n // 128, -(-m // 128)
+    packed, quads, limit = _gemm_o_rule(torch.cuda.get_device_properties(dev).multi_processor_count, batch, m, n)
+    assert not packed and not quads, "not a shape of both forms"
     flags = np.concatenate([_flags(1, blocks + 1, heads, p, seed=7 + i)[0] for i, p in enumerate(p_active)])
     segs = [np.packbits(f.reshape(-1).astype(np.uint8), bitorder="little") for f in flags]
-    packed, indptr = np.concatenate(segs), np.cumsum([0] + [len(s) for s in segs]).astype(np.int32)
+    info, indptr = np.concatenate(segs), np.cumsum([0] + [len(s) for s in segs]).astype(np.int32)
     g = torch.Generator(device=dev).manual_seed(batch)
     x = torch.randn(batch, m, n, generator=g, device=dev).to(torch.bfloat16)
     w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
-    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    pk, ip = torch.from_numpy(info).to(dev), torch.from_numpy(indptr).to(dev)
     ws = torch.full((64,), 7, dtype=torch.int32, device=dev)
     stream = torch.cuda.current_stream(dev).cuda_stream
-    units, quads = batch * blocks * 8, batch * 4 * (blocks // 2)
-    rounds = -(-quads // n_cu)
-    limit = 473 - 256 * 920 * -(-units // n_cu) // (2420 * rounds)
-    assert units > 4 * n_cu and limit >= 32 and 64 * units > 49 * 4 * n_cu * rounds, "not a shape of both forms"
     judged = [j * batch // min(batch, 64) for j in range(min(batch, 64))]
+    first = heads // 8                                     # byte that the text block's flags end in
+    n_bytes = min(m // 128 * heads // 8, 4096, 16 * (256 // (1 << (len(judged) - 1).bit_length())))
     for cache in (1, 0):
         outs = []
         for scratch, size in ((ws.data_ptr(), 256), (None, 0)):
@@ -581,10 +596,32 @@ def test_gemm_o_form_of_a_mixed_batch(dev, p_active):
                                    pk.data_ptr(), ip.data_ptr(), text, cache, scratch, size, stream))
             outs.append(y)
         assert torch.equal(outs[0], outs[1])
-        n_bytes = blocks * heads // 8
-        selected = [int((flags[j, 1:] != bool(cache)).sum()) for j in judged]
-        ahead = sum(s * (limit * n_bytes - 32 * s) for s in selected)
-        assert int(ws[8]) == int(ahead >= 0)
+        ones = [int(np.unpackbits(segs[j][first:first + n_bytes]).sum()) for j in judged]
+        selected = [8 * n_bytes - o if cache else o for o in ones]
+        assert int(ws[8]) == int(sum(s * (limit * n_bytes - 32 * s) for s in selected) >= 0)
+
+
+@pytest.mark.parametrize("shape", [(1, 6200, 1536), (1, 6300, 1536), (1, 16100, 2048), (1, 8185, 3072), (2, 3300, 2560),
+                                   (1, 4090, 5120), (1, 2553, 5120)])
+def test_gemm_o_forms_without_scratch(dev, shape):
+    """Shapes on both sides of the lines at which packed units or quads are taken whatever the flags (one round of quads
+    and more of them, narrow and wide): sampled rows of both passes against the fp32 product of the selected heads."""
+    import flashomni_amd as fo
+    batch, m, n = shape
+    heads, blocks = n // 128, -(-m // 128)
+    info, packed, indptr = _flags(batch, blocks, heads, 0.6, seed=m)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    part = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 0, is_for_cache=True, out_dtype=torch.float32)
+    y = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 0, bias=part)
+    rows = sorted({0, 1, 127, 128, m // 2, m - 1} | set(range(5, m, 977)))
+    for b in range(batch):
+        a = x[b, rows].float()
+        on = torch.from_numpy(info[b, np.array(rows) // 128]).to(dev).repeat_interleave(128, 1)
+        for got, exp in ((part, (a * ~on) @ w.float().t()), (y, a @ w.float().t())):
+            assert max_abs(got[b, rows], exp) <= MAX_ABS * max(1.0, float(exp.abs().max()) / 2) and rel_l2(got[b, rows], exp) <= REL_L2
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
