@@ -25,10 +25,9 @@
 // strips of one token block x three column blocks for the rest: 91 % of the slots, but a strip's
 // three columns lie far apart and few concurrent items share its W tiles, 9.4 GB fetched per launch
 // against 6.8 GB, and the launch was 1.3 % shorter.  Either way the time per round of work items
-// rises with the fill.)  GEMM-O (and GEMM-Q with is_full) computes every unit: no list
-// then, the kernel derives its quads from the shape.  GEMM-O walks the union of the two token
-// blocks' selected heads; a token block that does not select a head reads that k step's X operand
-// as zeros.
+// rises with the fill.)  GEMM-Q with is_full computes every unit: no list then, the
+// kernel derives its quads from the shape.  GEMM-O, whose token blocks differ in length, runs as strips
+// (gemm_strip_kernel).
 //
 // Data path.  Operands are staged in slabs of 64 k: a tile row is then 128 B, one whole memory line.
 // A wavefront fetches its sixteen 8-row pieces of a slab with buffer loads (a resource descriptor
@@ -42,7 +41,7 @@
 // per copy and wavefront, cost a quarter of the loop.)  One barrier per slab.  Rows are XOR-swizzled
 // instead of padded: row r keeps logical 16-byte chunk c at position c ^ ((r >> 1) & 7), applied to
 // the LDS write address; the 128-bit operand reads of 16 consecutive rows then cover all 64 banks.
-// A k range that is not a multiple of 64 (K or the head width of GEMM-O = 32 mod 64) ends in a slab
+// A k range that is not a multiple of 64 (K = 32 mod 64) ends in a slab
 // that reaches 32 back into its neighbour; that half of its X operand is cleared on the way to LDS
 // (a separate instantiation, so that the common case carries no masking).
 //
@@ -53,13 +52,10 @@
 // 32 rows at a time in fp32, into a layout where 32 consecutive lanes cover one row; there the bias
 // vector or the cached partial is added in fp32 and the result is rounded once and stored through a
 // buffer descriptor that ends with the matrix (no per-row tests).  The first slab of the next work
-// item is requested before the epilogue, so that its latency hides behind the stores (GEMM-O: the
-// item's flags are fetched a whole item ahead and its k-step list is built just before that request;
-// where a cached partial is added, the request follows the stores, because the partial's pieces need
-// the staging registers).
+// item is requested before the epilogue, so that its latency hides behind the stores.
 //
-// Launches of few units, launches whose quads would leave CUs idle and GEMM-O passes that select few heads run a
-// workgroup per unit instead (gemm_unit_kernel, gemm_packed_kernel, and the rule in launch_half).
+// Launches of few units and launches whose quads would leave CUs idle run a workgroup per unit or per strip instead
+// (gemm_unit_kernel, gemm_packed_kernel, gemm_strip_kernel, and the rules in launch_o and launch_q).
 //
 // Work order.  Workgroups are persistent (one per CU).  The quad list is ordered by token window,
 // then column pair, then row pair, and XCD x (= blockIdx % 8) owns the x-th contiguous eighth of it.
@@ -68,6 +64,7 @@
 // that XCD's L2; work items of equal length keep them in step in k, which is what makes the tiles
 // hit (measured at the Wan size: 6.8 GB fetched per launch against 28 GB of operand loads).
 #include "fo_common.h"
+#include "fo_device.h"
 
 #include <type_traits>
 
@@ -131,11 +128,11 @@ struct GemmParams {
   const int32_t* quads;  // kQuadInts per quad, queue by queue; null: every unit is computed and the
                          // quads are enumerated arithmetically (GEMM-O, GEMM-Q with is_full)
   const int32_t* qoff;   // qoff[0..8] queue boundaries inside `quads`
-  int32_t* cursor;       // GEMM-O, long launches: one work-item cursor per XCD (zero at launch), or null
-  // GEMM-O launched in both forms, as quads and as packed units: the latter run where this word (cursor[8]) is not
-  // zero, the former where it is; null: packed units only
-  const int32_t* sparse_word;
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
+  int32_t strip_cols;    // strips: column groups of XCDs
+  int32_t strip_sorted;  // strips: token blocks with the most selected heads first
+  int32_t* judgement;    // strips: where judge_flags leaves its word, or null
+  int32_t judge_first, judge_bytes, judge_limit;
   int32_t n_win;         // windows of 16 token blocks per batch
   int32_t inline_cells;  // > 0: GEMM-Q builds its quad list itself from the flags of this many cells
   int32_t batch, m, n, k;
@@ -365,79 +362,20 @@ __global__ void __launch_bounds__(kListThreads) gemm_quads_kernel(ListArgs a, Li
   }
 }
 
-// Clears the cursors of a launch that hands out its work items dynamically (a kernel, not a memset, so that
-// a captured graph replays it faithfully), and sets cursor[8] where packed units are faster than quads: with p of a
-// request's head slices selected its quads take a time of 2 p - p^2, its units (2 - limit / 256) p, so units are ahead where the
-// sum of p (limit / 256 - p) over the requests is not negative; limit: see launch_half.  (A batch is judged as a whole:
-// by its first request alone, one of 5 % selected in front of two of 95 %, 8192 x 3072 each, ran as packed units, 422 us in
-// place of 382.)  Judged by up to 4096 bytes of flags in all, of up to 64 requests spread over the batch, from each one's
-// `first_byte` on (n_bytes: how many a request has); all of them are in flight together.
-constexpr int kJudged = 64, kJudgedBytes = 4096;
-__global__ void __launch_bounds__(kThreads) gemm_choose_kernel(int32_t* cursor, const uint8_t* __restrict__ sparse_info,
-                                                               const int32_t* __restrict__ sparse_info_indptr, int32_t batch,
-                                                               int32_t first_byte, int32_t n_bytes, int32_t pick, int32_t limit) {
-  __shared__ int32_t s_ones[kThreads / 4];
-  const int tid = threadIdx.x;
-  if (tid < 8) cursor[tid] = 0;
-  if (n_bytes == 0) {
-    if (tid == 8) cursor[8] = 0;
-    return;
-  }
-  const int judged = min(batch, kJudged);
-  int threads = kThreads;  // of a request: a power of two, at least kThreads / kJudged
-  while (threads * judged > kThreads) threads >>= 1;
-  constexpr int kPer = kJudgedBytes / kThreads;
-  const int n = min(n_bytes, kPer * threads);
-  const int j = tid / threads, at = tid - j * threads;
-  int ones = 0;
-  if (j < judged) {
-    const uint8_t* info = sparse_info + sparse_info_indptr[static_cast<int64_t>(j) * batch / judged] + first_byte;
-    uint8_t v[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) v[i] = at + i * threads < n ? info[at + i * threads] : 0;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) ones += __popc(v[i]);
-  }
-  const int width = min(threads, 64);
-  for (int off = width >> 1; off > 0; off >>= 1) ones += __shfl_xor(ones, off, 64);
-  if (tid % width == 0) s_ones[tid / width] = ones;
-  __syncthreads();
-  if (tid < 64) {
-    // (up to 2^15 selected times 2^21: 64 bits)
-    long long ahead = 0;
-    if (tid < judged) {
-      int selected = 0;
-      for (int w = 0; w < threads / width; ++w) selected += s_ones[tid * (threads / width) + w];
-      if (!pick) selected = 8 * n - selected;
-      ahead = static_cast<long long>(selected) * (limit * n - 32 * selected);
-    }
-    for (int off = 32; off > 0; off >>= 1) ahead += __shfl_xor(ahead, off, 64);
-    if (tid == 0) cursor[8] = ahead >= 0;
-  }
-}
-
 // ---------------------------------------------------------------------------------------------
-// Main kernel.  kReduce = false: GEMM-Q.  kReduce = true: GEMM-O.  kAux: GEMM-Q with fused
-// quantisation / GEMM-O that adds a cached partial (epilogues with register needs of their own).
+// GEMM-Q as quads.  kQuant: with fused quantisation (an epilogue with register needs of its own).
 // ---------------------------------------------------------------------------------------------
-template <typename T, bool kReduce, bool kHalf, bool kAux>
+template <typename T, bool kHalf, bool kQuant>
 __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
-  constexpr bool kQuant = !kReduce && kAux, kPartial = kReduce && kAux;
   using TT = Types<T>;
   using x8 = typename TT::x8;
   using x4 = typename TT::x4;
   constexpr int NT = 4, MT = 4;  // wavefront tile = one unit: 128 columns (W rows) x 128 token rows (X rows)
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  __shared__ int32_t s_popped;
-  __shared__ int32_t s_heads[kMaxHeads + 1];  // GEMM-O: head | (row0 selects) << 16 | (row1 selects) << 17
-  __shared__ int32_t s_nsel;
-  // GEMM-O: per k step, k offset | (row0 selects) << 16 | (row1 selects) << 17; four entries past
-  // the end repeat the last step
-  __shared__ int32_t s_step[kReduce ? kMaxSteps + 4 : 1];
   // GEMM-Q listing its own quads (short launches: saves the list kernel's launch): quad count
   // prefix and flagged-row masks of every cell, and the entry picked for the current work item
-  __shared__ int32_t s_cell_pref[kReduce ? 1 : kInlineCells + 1];
-  __shared__ uint32_t s_cell_mask[kReduce ? 1 : 2 * kInlineCells];
+  __shared__ int32_t s_cell_pref[kInlineCells + 1];
+  __shared__ uint32_t s_cell_mask[2 * kInlineCells];
   __shared__ int32_t s_cell_wave[kThreads / 64];
   __shared__ int32_t s_entry[8];
 
@@ -473,65 +411,62 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   const int last_q = (last_rows + 1) / 2;
   const int quads_per_batch = (full_w * per_win + last_q) * p.n_cp;
   int q_lo, q_len;
-  bool inline_list = false;
-  if constexpr (!kReduce) inline_list = p.inline_cells > 0;
+  const bool inline_list = p.inline_cells > 0;
   // Few flagged units (GEMM-Q that lists its own work): a quad would keep one CU busy for four units' time
   // while others idle.  If items of at most two units are no more than the workgroups, the list is made of
   // those, and two wavefronts share a unit: each takes two of a slab's four substeps (half of k), and the
   // halves are added through LDS at the end.  Measured with K = 3072 (us, quads -> pairs): 16 k tokens x 24
   // heads with one unit in ten flagged 60 -> 45, 4.6 k tokens with a quarter flagged 60 -> 43.  The error
   // against 64-bit sums is the same (bf16 1.66e-3, fp16 2.08e-4: the rounding of the result).
-  constexpr bool kPairs = !kReduce && !kAux;
+  constexpr bool kPairs = !kQuant;
   bool pairs = false;
   if (inline_list) {
-    if constexpr (!kReduce) {
-      // thread = cell: masks, quad count, workgroup-wide inclusive scan of the counts
-      ListGeom gm;
-      gm.batch = p.batch;
-      gm.n_row_tiles = p.n_row_tiles;
-      gm.n_col_tiles = p.n_col_tiles;
-      gm.n_win = p.n_win;
-      gm.n_cp = p.n_cp;
-      int32_t cnt = 0;
-      if (tid < p.inline_cells) {
-        int b, row0, cp;
-        uint32_t m0, m1;
-        cell_masks(gm, tid, true, p.sparse_info, p.sparse_info_indptr, p.sparse_q_size, p.num_heads,
-                   p.head_dim, p.num_text_tokens, &b, &row0, &cp, &m0, &m1);
-        for_each_quad(m0, m1, true, [&](int, int, int, int) { ++cnt; });
-        if constexpr (kPairs) {  // (both counts in one scan: at most 16 per cell and kInlineCells cells)
-          cnt += count_pairs(m0, m1) << 16;
-        }
-        s_cell_mask[2 * tid] = m0;
-        s_cell_mask[2 * tid + 1] = m1;
+    // thread = cell: masks, quad count, workgroup-wide inclusive scan of the counts
+    ListGeom gm;
+    gm.batch = p.batch;
+    gm.n_row_tiles = p.n_row_tiles;
+    gm.n_col_tiles = p.n_col_tiles;
+    gm.n_win = p.n_win;
+    gm.n_cp = p.n_cp;
+    int32_t cnt = 0;
+    if (tid < p.inline_cells) {
+      int b, row0, cp;
+      uint32_t m0, m1;
+      cell_masks(gm, tid, true, p.sparse_info, p.sparse_info_indptr, p.sparse_q_size, p.num_heads,
+                 p.head_dim, p.num_text_tokens, &b, &row0, &cp, &m0, &m1);
+      for_each_quad(m0, m1, true, [&](int, int, int, int) { ++cnt; });
+      if constexpr (kPairs) {  // (both counts in one scan: at most 16 per cell and kInlineCells cells)
+        cnt += count_pairs(m0, m1) << 16;
       }
-      int32_t incl = cnt;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int32_t up = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += up;
-      }
-      if (lane == 63) s_cell_wave[wv] = incl;
-      __syncthreads();
-      int32_t base = 0, total = 0;
-#pragma unroll
-      for (int w = 0; w < kThreads / 64; ++w) {
-        const int32_t t = s_cell_wave[w];
-        if (w < wv) base += t;
-        total += t;
-      }
-      incl += base;
-      if constexpr (kPairs) {
-        pairs = (total >> 16) <= static_cast<int>(gridDim.x);
-        total = pairs ? total >> 16 : total & 0xFFFF;
-        incl = pairs ? incl >> 16 : incl & 0xFFFF;
-      }
-      if (tid < kInlineCells) s_cell_pref[tid + 1] = incl;
-      if (tid == 0) s_cell_pref[0] = 0;
-      q_lo = static_cast<int>(static_cast<int64_t>(total) * xcd / kXcds);
-      q_len = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / kXcds) - q_lo;
-      __syncthreads();
+      s_cell_mask[2 * tid] = m0;
+      s_cell_mask[2 * tid + 1] = m1;
     }
+    int32_t incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t up = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += up;
+    }
+    if (lane == 63) s_cell_wave[wv] = incl;
+    __syncthreads();
+    int32_t base = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) {
+      const int32_t t = s_cell_wave[w];
+      if (w < wv) base += t;
+      total += t;
+    }
+    incl += base;
+    if constexpr (kPairs) {
+      pairs = (total >> 16) <= static_cast<int>(gridDim.x);
+      total = pairs ? total >> 16 : total & 0xFFFF;
+      incl = pairs ? incl >> 16 : incl & 0xFFFF;
+    }
+    if (tid < kInlineCells) s_cell_pref[tid + 1] = incl;
+    if (tid == 0) s_cell_pref[0] = 0;
+    q_lo = static_cast<int>(static_cast<int64_t>(total) * xcd / kXcds);
+    q_len = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / kXcds) - q_lo;
+    __syncthreads();
   } else if (p.quads) {
     q_lo = p.qoff[xcd];
     q_len = p.qoff[xcd + 1] - q_lo;
@@ -559,44 +494,42 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   auto decode_item = [&](int work) -> Item {
     int bz, valid, r[2], c[2], r2 = 0;
     if (inline_list) {
-      if constexpr (!kReduce) {
-        // the thread whose cell holds quad q_lo + work walks the cell's quads up to it
-        const int q = q_lo + work;
-        if (tid < p.inline_cells && s_cell_pref[tid] <= q && q < s_cell_pref[tid + 1]) {
-          const int cp = tid % p.n_cp, t = tid / p.n_cp;
-          const int w = t % p.n_win, b = t / p.n_win;
-          int k = q - s_cell_pref[tid];
-          auto entry = [&](int r0, int r1, int v, int r2) {
-            if (k == 0) {
-              s_entry[0] = b;
-              s_entry[1] = w * kWindow + r0;
-              s_entry[2] = w * kWindow + (r1 < 0 ? r0 : r1);
-              if (v & kColStrip) {
-                s_entry[3] = s_entry[4] = (v & kColStripSecond) ? 2 * cp + 1 : 2 * cp;
-              } else {
-                s_entry[3] = (v & 0x5) ? 2 * cp : 2 * cp + 1;
-                s_entry[4] = (v & 0xA) ? 2 * cp + 1 : 2 * cp;
-              }
-              s_entry[5] = v;
-              s_entry[6] = w * kWindow + r2;
+      // the thread whose cell holds quad q_lo + work walks the cell's quads up to it
+      const int q = q_lo + work;
+      if (tid < p.inline_cells && s_cell_pref[tid] <= q && q < s_cell_pref[tid + 1]) {
+        const int cp = tid % p.n_cp, t = tid / p.n_cp;
+        const int w = t % p.n_win, b = t / p.n_win;
+        int k = q - s_cell_pref[tid];
+        auto entry = [&](int r0, int r1, int v, int r2) {
+          if (k == 0) {
+            s_entry[0] = b;
+            s_entry[1] = w * kWindow + r0;
+            s_entry[2] = w * kWindow + (r1 < 0 ? r0 : r1);
+            if (v & kColStrip) {
+              s_entry[3] = s_entry[4] = (v & kColStripSecond) ? 2 * cp + 1 : 2 * cp;
+            } else {
+              s_entry[3] = (v & 0x5) ? 2 * cp : 2 * cp + 1;
+              s_entry[4] = (v & 0xA) ? 2 * cp + 1 : 2 * cp;
             }
-            --k;
-          };
-          if (kPairs && pairs) {
-            for_each_pair(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], entry);
-          } else {
-            for_each_quad(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], true, entry);
+            s_entry[5] = v;
+            s_entry[6] = w * kWindow + r2;
           }
+          --k;
+        };
+        if (kPairs && pairs) {
+          for_each_pair(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], entry);
+        } else {
+          for_each_quad(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], true, entry);
         }
-        __syncthreads();
-        bz = s_entry[0];
-        r[0] = s_entry[1];
-        r[1] = s_entry[2];
-        c[0] = s_entry[3];
-        c[1] = s_entry[4];
-        valid = s_entry[5];
-        r2 = s_entry[6];
       }
+      __syncthreads();
+      bz = s_entry[0];
+      r[0] = s_entry[1];
+      r[1] = s_entry[2];
+      c[0] = s_entry[3];
+      c[1] = s_entry[4];
+      valid = s_entry[5];
+      r2 = s_entry[6];
     } else if (p.quads) {
       const int32_t* e = p.quads + kQuadInts * static_cast<int64_t>(q_lo + work);
       bz = e[0];
@@ -642,123 +575,15 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
     }
     return it;
   };
-  // k-step list of an item (GEMM-O: the union of the two token blocks' selected heads); returns the
-  // number of slabs.  Called by all threads together, when nobody reads the previous list any more.
-  // GEMM-O: the flags of an item's two token blocks, fetched by the first wavefront (lane = head, two
-  // bits per group of 64 heads; up to 128 heads travel this way, more are read when the list is built).
-  // Asked for at the top of the item before, so that the two dependent memory latencies (segment
-  // offset, flag byte) pass behind that item's main loop.
-  constexpr int kFetchedHeads = 128;
-  int seg_bz = -1, seg_off = 0;
-  auto fetch_flags = [&](const Item& item) -> uint32_t {
-    uint32_t f = 0;
-    if constexpr (kReduce) {
-      const int n_slices = p.k / p.head_dim;
-      if (wv == 0 && n_slices <= kFetchedHeads) {
-        // (the segment offset of the batch entry is kept: one memory latency less on the way to the flags)
-        if (item.bz != seg_bz) {
-          seg_bz = item.bz;
-          seg_off = p.sparse_info_indptr[item.bz];
-        }
-        const uint8_t* info = p.sparse_info + seg_off;
-        const uint32_t base0 =
-            static_cast<uint32_t>(p.num_text_tokens + item.r[0] * kTile) / p.sparse_q_size * p.num_heads;
-        const uint32_t base1 =
-            static_cast<uint32_t>(p.num_text_tokens + item.r[1] * kTile) / p.sparse_q_size * p.num_heads;
-        const bool want1 = (item.valid & 0xC) != 0;
-        const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
-#pragma unroll
-        for (int g = 0; g < kFetchedHeads / 64; ++g) {
-          const int h = g * 64 + lane;
-          if (h < n_slices) {
-            const uint32_t s0 = flag_bit(info, base0 + h) == pick ? 1u : 0u;
-            const uint32_t s1 = want1 && (flag_bit(info, base1 + h) == pick) ? 2u : 0u;
-            f |= (s0 | s1) << (2 * g);
-          }
-        }
-      }
-    }
-    return f;
-  };
-  auto build_steps = [&](const Item& item, uint32_t fetched) -> int {
-    const int bz = item.bz, valid = item.valid;
-    const int r[2] = {item.r[0], item.r[1]};
-    int n_iter;
-    if constexpr (kReduce) {
-      if (wv == 0) {
-        const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
-        const uint32_t base0 =
-            static_cast<uint32_t>(p.num_text_tokens + r[0] * kTile) / p.sparse_q_size * p.num_heads;
-        const uint32_t base1 =
-            static_cast<uint32_t>(p.num_text_tokens + r[1] * kTile) / p.sparse_q_size * p.num_heads;
-        const bool want1 = (valid & 0xC) != 0;
-        const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
-        int count = 0;
-        const int n_slices = p.k / p.head_dim;
-        const bool have_fetched = n_slices <= kFetchedHeads;
-        for (int h0 = 0; h0 < n_slices; h0 += 64) {
-          const int h = h0 + lane;
-          bool s0 = false, s1 = false;
-          if (have_fetched) {
-            const uint32_t two = fetched >> (2 * (h0 >> 6));
-            s0 = (two & 1) != 0;
-            s1 = (two & 2) != 0;
-          } else if (h < n_slices) {
-            s0 = flag_bit(info, base0 + h) == pick;
-            s1 = want1 && (flag_bit(info, base1 + h) == pick);
-          }
-          const unsigned long long mask = __ballot(s0 || s1);
-          if (s0 || s1)
-            s_heads[count + __popcll(mask & ((1ull << lane) - 1ull))] = h | (s0 << 16) | (s1 << 17);
-          count += __popcll(mask);
-        }
-        if (lane == 0) s_nsel = count;
-      }
-      __syncthreads();
-      // slabs of a head slice: full 64-wide ones, then (head_dim % 64 == 32) one that reaches 32 back
-      // into the slab before it and counts for its second half only (the first slice of the matrix
-      // instead reaches forward and counts for its first half)
-      const int iph = (p.head_dim + kBK - 1) / kBK;
-      n_iter = __builtin_amdgcn_readfirstlane(s_nsel) * iph;
-      if (n_iter > 0) {
-        for (int i = tid; i < n_iter + 4; i += kThreads) {
-          const int ii = i < n_iter ? i : n_iter - 1;
-          const int hv = s_heads[ii / iph];
-          const int k0 = (hv & 0xFFFF) * p.head_dim + (ii % iph) * kBK;
-          int e = k0;
-          if ((ii % iph) * kBK + kBK > p.head_dim) e = k0 >= 32 ? (k0 - 32) | kZeroFirst : k0 | kZeroSecond;
-          s_step[i] = e | (hv & 0x30000);
-        }
-      }
-      __syncthreads();
-    } else {
-      n_iter = (p.k + kBK - 1) / kBK;
-    }
-
-    return n_iter;
-  };
-  int n_iter = 0;
-  // k offset of step it (steps past the end repeat the last one); GEMM-O: plus the select bits
+  const int n_iter = (p.k + kBK - 1) / kBK;
+  // k offset of step it (steps past the end repeat the last one)
   auto step_entry = [&](int it) -> int {
-    if constexpr (kReduce) {
-      return __builtin_amdgcn_readfirstlane(s_step[it]);  // uniform: the descriptor choice below stays scalar
-    } else {
-      // (K % 64 == 32: the last slab reaches 32 back and counts for its second half only)
-      const int i = it < n_iter ? it : n_iter - 1;
-      return (i + 1) * kBK <= p.k ? i * kBK | 0x30000 : (p.k - kBK) | kZeroFirst | 0x30000;
-    }
-  };
-  // the same without making the list's value scalar (that needs the LDS read to have returned)
-  auto step_entry_raw = [&](int it) -> int {
-    if constexpr (kReduce) {
-      return s_step[it];
-    } else {
-      return step_entry(it);
-    }
+    // (K % 64 == 32: the last slab reaches 32 back and counts for its second half only)
+    const int i = it < n_iter ? it : n_iter - 1;
+    return (i + 1) * kBK <= p.k ? i * kBK : (p.k - kBK) | kZeroFirst;
   };
   // ---- operand tiles: buffer resource descriptors in scalar registers ----
-  // The X descriptors end with the matrix, so rows past M read as zeros; a token block that does
-  // not select a slab's head (GEMM-O) loads through an empty descriptor: zeros, no memory access.
+  // The X descriptors end with the matrix, so rows past M read as zeros.
   const __amdgpu_buffer_rsrc_t rsrc_none = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(xg), 0, 0, 0x00020000);
   __amdgpu_buffer_rsrc_t rsrc[4] = {rsrc_none, rsrc_none, rsrc_none, rsrc_none};
   auto make_rsrc = [&](const Item& item) {
@@ -771,13 +596,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
       rsrc[2 + u] = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<T*>(wg + static_cast<int64_t>(item.c[u]) * kTile * p.k), 0, kTile * p.k * 2, 0x00020000);
     }
-    if constexpr (!kReduce) {
-      if (item.valid & kColStrip) {  // a column strip's fourth tile is its third X tile
-        const int rows_left = min(p.m - item.r2 * kTile, kTile);
-        rsrc[3] = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T*>(xg + (static_cast<int64_t>(item.bz) * p.m + static_cast<int64_t>(item.r2) * kTile) * p.k), 0,
-            rows_left * p.k * 2, 0x00020000);
-      }
+    if (item.valid & kColStrip) {  // a column strip's fourth tile is its third X tile
+      const int rows_left = min(p.m - item.r2 * kTile, kTile);
+      rsrc[3] = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(xg + (static_cast<int64_t>(item.bz) * p.m + static_cast<int64_t>(item.r2) * kTile) * p.k), 0,
+          rows_left * p.k * 2, 0x00020000);
     }
   };
   int ld_off[4];
@@ -786,9 +609,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   // Staging registers: piece j of a slab waits here between its global load and its LDS write.
   u32x4 stg[P];
   auto gload = [&](int j, int entry) {
-    const int t = j >> 2;  // tiles 0, 1: X of token block 0, 1 (select bits 16, 17 of the entry); 2, 3: W
-    const bool sel = t >= 2 || ((entry >> (16 + t)) & 1) != 0;
-    stg[j] = __builtin_amdgcn_raw_buffer_load_b128(sel ? rsrc[t] : rsrc_none, ld_off[j & 3], (entry & 0xFFFF) * 2, 0);
+    stg[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc[j >> 2], ld_off[j & 3], (entry & 0xFFFF) * 2, 0);
   };
   // kHalf: only one half of a slab that reaches into its neighbour counts; the other half of the X
   // pieces is cleared on the way to LDS
@@ -805,26 +626,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
     *reinterpret_cast<u32x4*>(dst) = v;
   };
 
-  // The first slab of an item is requested before the epilogue of the item before it, so that its
-  // latency (and the list work above) hides behind the stores.
-  // Work items of unequal length (GEMM-O: every item walks its own head list) let the workgroups of an
-  // XCD drift apart when each strides through the queue in fixed steps, and items that run together
-  // then no longer share tiles in L2.  Long GEMM-O launches therefore take their items from a cursor
-  // per XCD: the items in flight are always neighbours in the queue.  One thread pops, an item ahead
-  // (the value is needed at the top of the next item and waits in a register until then).
-  bool popping = false;
-  if constexpr (kReduce) popping = p.cursor != nullptr;
-  if (popping && p.cursor[8] != 0) return;  // (launched in both forms, and the flags are for the other one)
-  int popped = 0;
-  auto pop = [&]() {
-    if (tid == 0) popped = per_xcd + atomicAdd(p.cursor + xcd, 1);  // (the first per_xcd items are dealt by slot)
-  };
   if constexpr (kPairs) {
     if (pairs) {
       // One item of at most two units (no more items than workgroups), two wavefronts each.
       if (slot >= q_len) return;
       const Item item = decode_item(slot);
-      n_iter = build_steps(item, 0);
       // Three tiles at most: X r0, X r1, W of a column pair; X, W c0, W c1 of a row's two units; X, none, W.
       // (What the loop waits for is the vector memory path: a CU takes ~37 bytes per clock through it, and
       // loads that fetch nothing hold it up as well: with four tiles, one or two of them empty, 51 and 47 us.
@@ -1012,19 +818,19 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
       return;
     }
   }
-  if (popping) pop();
   int work = slot;
   bool have = work < q_len;
   Item cur{};
+  // (the first slab of an item is requested before the epilogue of the item before it: its latency hides behind the stores)
+  auto request_first = [&](const Item& item) {
+    make_rsrc(item);
+    const int e0 = step_entry(0);
+#pragma unroll
+    for (int j = 0; j < P; ++j) gload(j, e0);
+  };
   if (have) {
     cur = decode_item(work);
-    n_iter = build_steps(cur, fetch_flags(cur));
-    make_rsrc(cur);
-    if (n_iter > 0) {
-      const int e0 = step_entry(0);
-#pragma unroll
-      for (int j = 0; j < P; ++j) gload(j, e0);
-    }
+    request_first(cur);
   }
   while (have) {
     const int bz = cur.bz, valid = cur.valid;
@@ -1032,31 +838,18 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
     int out_r = wr ? cur.r[1] : cur.r[0], out_c = wc ? cur.c[1] : cur.c[0];
     bool my_valid = (valid >> (wr * 2 + wc)) & 1;
     int a_tile = 2 + wc, b_tile = wr;  // LDS tiles of this wavefront's W and X operands
-    if constexpr (!kReduce) {
-      if (valid & kColStrip) {
-        out_r = wv == 0 ? cur.r[0] : wv == 1 ? cur.r[1] : cur.r2;
-        out_c = cur.c[0];
-        my_valid = wv < 3 && ((valid >> wv) & 1);
-        a_tile = 2;
-        b_tile = wv == 2 ? 3 : wv;
-      }
+    if (valid & kColStrip) {
+      out_r = wv == 0 ? cur.r[0] : wv == 1 ? cur.r[1] : cur.r2;
+      out_c = cur.c[0];
+      my_valid = wv < 3 && ((valid >> wv) & 1);
+      a_tile = 2;
+      b_tile = wv == 2 ? 3 : wv;
     }
     // (the next item is looked up here, while no accumulator is live)
-    int next_work = work + per_xcd;
-    if (popping) {
-      if (tid == 0) s_popped = popped;
-      __builtin_amdgcn_s_waitcnt(0xc07f);
-      __builtin_amdgcn_s_barrier();
-      next_work = __builtin_amdgcn_readfirstlane(s_popped);
-      if (next_work < q_len) pop();  // for the item after the next
-    }
+    const int next_work = work + per_xcd;
     const bool have_next = next_work < q_len;
     Item nxt{};
-    uint32_t nxt_flags = 0;
-    if (have_next) {
-      nxt = decode_item(next_work);
-      nxt_flags = fetch_flags(nxt);
-    }
+    if (have_next) nxt = decode_item(next_work);
     // every wavefront is done with the ring (the previous item's epilogue turned through it)
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
@@ -1070,7 +863,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
     // slab it+2 goes into stage it % 2 and that of slab it+3 is requested.  Every substep issues the
     // same mix (sixteen MFMAs, eight operand reads, four LDS writes, four global loads), so the memory
     // path sees an even stream and a load has a whole slab period to arrive.
-    if (n_iter > 0) {
+    {
       const int e0 = step_entry(0), e1 = step_entry(1), e2 = step_entry(2);
       {
         const unsigned keep = keep_of(e0);
@@ -1090,29 +883,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
       __builtin_amdgcn_s_barrier();
     }
 
-    // ---- next item: list work and the request for its first slab (every wavefront, once per item,
-    // after its last use of the ring and of the step list, before the epilogue: the slab's latency
-    // hides behind the stores). ----
-    int next_iter = 0;
     auto ring_free = [&]() {
       __builtin_amdgcn_s_waitcnt(0xc07f);
-      __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring and with the step list
+      __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring
     };
-    auto prefetch_next = [&]() {
-      if (have_next) {
-        next_iter = build_steps(nxt, nxt_flags);
-        make_rsrc(nxt);
-        if (next_iter > 0) {
-          const int saved = n_iter;
-          n_iter = next_iter;  // (step_entry of the listless form clamps against it)
-          const int e0 = step_entry(0);
-          n_iter = saved;
-#pragma unroll
-          for (int j = 0; j < P; ++j) gload(j, e0);
-        }
-      }
-    };
-    // ---- accumulators (bias / cached partial are added in the epilogue) ----
+    // ---- accumulators (the bias is added in the epilogue) ----
     // acc[nt][mt][i]: n = n0 + nt*32 + (i/4)*8 + g*4 + i%4, m = m0 + mt*32 + l32
     const int m0 = out_r * kTile;
     const int n0 = out_c * kTile;
@@ -1138,7 +913,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         }
       }
       ring_free();
-      prefetch_next();
+      if (have_next) request_first(nxt);
     } else {
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
@@ -1146,7 +921,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
-      if (n_iter > 0) {
+      {
         // LDS byte offsets of this wavefront's operand rows inside a stage
         const int a_base = a_tile * kUnitBytes + l32 * kRowBytes;  // W rows nt*32 + l32
         const int b_base = b_tile * kUnitBytes + l32 * kRowBytes;  // X rows mt*32 + l32
@@ -1180,31 +955,23 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         };
 #pragma unroll
         for (int idx = 0; idx < NT + MT; ++idx) lread(0, 0, idx);
-        // (the step entries of the next three slabs ride along in scalar registers; the fourth is
-        // read from the list a slab ahead and becomes scalar after the wait the barrier needs anyway,
-        // so the list costs no wait of its own)
         int en1 = step_entry(1), en2 = step_entry(2), en3 = step_entry(3);
         for (int it = 0; it < n_iter; ++it) {
           const int st = it & 1;
-          const int en4_raw = step_entry_raw(it + 4);
           const unsigned keep1 = keep_of(en1), keep2 = keep_of(en2);
           substep(0, st, 1, st ^ 1, PS, keep1, en2);
           substep(1, st, 2, st ^ 1, 2 * PS, keep1, en2);
           substep(0, st, 3, st ^ 1, 3 * PS, keep1, en2);
           __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): my reads of slab it and my writes of slab it+1 are done
           __builtin_amdgcn_s_barrier();        // ... for every wavefront
-          const int en4 = __builtin_amdgcn_readfirstlane(en4_raw);
           substep(1, st ^ 1, 0, st, 0, keep2, en3);
           en1 = en2;
           en2 = en3;
-          en3 = en4;
+          en3 = step_entry(it + 4);
         }
       }
       ring_free();
-      // The request for the next item's first slab goes out before the epilogue and its data waits in
-      // the staging registers, except where the epilogue adds a cached partial: its pieces need those
-      // registers, so there the request follows the stores.
-      if constexpr (!kPartial) prefetch_next();
+      if (have_next) request_first(nxt);
 
     // ---- epilogue ----
     // In the accumulator layout a lane owns one output row and runs of four columns: written from
@@ -1275,9 +1042,8 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
       }
-      // Output (and the cached partial, if there is one) go through buffer descriptors that end with the
-      // matrix: rows past M are dropped (read as zeros) by the address unit, no lane is masked and no
-      // row is tested.  A null output gets an empty descriptor.
+      // Output goes through buffer descriptors that end with the matrix: rows past M are dropped by the address
+      // unit, no lane is masked and no row is tested.  A null output gets an empty descriptor.
       const int rows_out = min(p.m - m0, kTile);
       const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
       auto out_rsrc = [&](const void* base, int elem_bytes) {
@@ -1285,29 +1051,8 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
             const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
             base ? rows_out * p.n * elem_bytes : 0, 0x00020000);
       };
-      // 32 rows of the block.  kMatrix: a cached partial [B, M, N] of element type BiasT is added;
-      // kOutF32: the output is fp32
-      // (the cached partial of 32 rows: sixteen pieces, the four values this lane adds to each of its
-      // rows, all in flight together while the rows turn through LDS.  Requesting the next 32 rows'
-      // pieces earlier, in a second register set or piece by piece as the first set is consumed, was
-      // measured: the compiler then spills 100-300 registers, some of them inside the main loop.)
-      auto load_partial = [&](int mt, auto* bm) {
-        using BiasVec = typename std::remove_reference<decltype(bm[0])>::type;
-        constexpr int kBytes = sizeof(BiasVec) / 4;  // of one element
-        const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
-        const int el_off = n0 + col4 * 4 + rsub * p.n;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int row_off = (mt * 32 + 2 * i) * p.n * kBytes;
-          if constexpr (kBytes == 4) {
-            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, row_off, 0));
-          } else {
-            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, row_off, 0));
-          }
-        }
-      };
-      auto turn_half = [&](int mt, auto matrix_tag, auto* bm, auto f32_tag) {
-        constexpr bool kMatrix = decltype(matrix_tag)::value, kOutF32 = decltype(f32_tag)::value;
+      // 32 rows of the block
+      auto turn_half = [&](int mt) {
         uint8_t* const region = region0 + (mt & 1) * (kSmemBytes / 8);
         // 16-byte chunk c of row r sits at chunk position c ^ r (rows are 512 bytes = 32 chunks)
 #pragma unroll
@@ -1324,8 +1069,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         // scalar offset per row
         const int el_off = n0 + col4 * 4 + rsub * p.n;  // in elements, row mt*32 + rsub
         auto row_off = [&](int i, int elem_bytes) { return (mt * 32 + 2 * i) * p.n * elem_bytes; };
-        if constexpr (kMatrix) load_partial(mt, bm);
-        const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
+        const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, 2);
         // eight rows at a time are read back (two LDS latencies per turn) and biased, then stored
         f32x4 vals[8];
 #pragma unroll
@@ -1339,27 +1083,15 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
             __builtin_amdgcn_sched_barrier(0);
           }
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            if constexpr (kMatrix) {
-              vals[i & 7][j] += static_cast<float>(bm[i][j]);
-            } else {
-              vals[i & 7][j] += bvec[j];
-            }
-          }
+          for (int j = 0; j < 4; ++j) vals[i & 7][j] += bvec[j];
           const f32x4 v = vals[i & 7];
           // (stored with the streaming hint, cache policy 2: the output is not read again by this launch
           // and should not push operand tiles out of the L2; 0.5-1.5 % at both sizes)
-          if constexpr (kOutF32) {
-            // (the row offset travels in the lane's: with one in a scalar register the compiler may write the
-            // first data register in the very next instruction, and the last lanes then store that value)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, el_off * 4 + row_off(i, 4), 0, 2);
-          } else {
-            x4 out;
+          x4 out;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
-            typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, row_off(i, 2), 2);
-          }
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+          typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, row_off(i, 2), 2);
           if constexpr (kQuant) {
             float f[4];
 #pragma unroll
@@ -1378,31 +1110,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
           }
         }
       };
-      auto turn_all = [&](auto matrix_tag, auto bias_tag, auto f32_tag) {
-        using BiasT = decltype(bias_tag);
-        using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
-        BiasVec bm[16];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) turn_half(mt, matrix_tag, bm, f32_tag);
-      };
-      using std::false_type;
-      using std::true_type;
-      if constexpr (!kReduce) {
-        turn_all(false_type{}, T{}, false_type{});  // GEMM-Q: bias vector or none, output in the activation type
-      } else if constexpr (kPartial) {
-        if (p.bias_f32) {
-          if (p.y_f32) turn_all(true_type{}, 0.f, true_type{}); else turn_all(true_type{}, 0.f, false_type{});
-        } else {
-          if (p.y_f32) turn_all(true_type{}, T{}, true_type{}); else turn_all(true_type{}, T{}, false_type{});
-        }
-      } else {
-        if (p.y_f32) turn_all(false_type{}, T{}, true_type{}); else turn_all(false_type{}, T{}, false_type{});
-      }
+      for (int mt = 0; mt < MT; ++mt) turn_half(mt);
     }
-      if constexpr (kPartial) prefetch_next();
     }
     cur = nxt;
-    n_iter = next_iter;
     work = next_work;
     have = have_next;
   }
@@ -1721,26 +1433,22 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_unit_kernel(const GemmParams
 }
 
 // ---------------------------------------------------------------------------------------------
-// Launches whose quads leave a part of the chip idle: a workgroup per unit, four of them on a CU.  260 quads on
-// 256 CUs are two rounds, the second nearly empty, and 138 are one that half of the CUs sit out; GEMM-O's
-// quads walk the union of two token blocks' heads besides.  A unit per workgroup needs no list, walks its own
-// heads, and the hardware hands the next one to whichever CU is free.  What a workgroup lacks, a second slab
-// buffer and staging registers, the other three on the CU make up for: a slab is copied straight to LDS (32 KB,
+// Dense GEMM-Q whose quads leave a part of the chip idle, and narrow GEMM-O: a workgroup per unit, four of them on a CU.
+// 260 quads on 256 CUs are two rounds, the second nearly empty, and 138 are one that half of the CUs sit out.  A unit per
+// workgroup needs no list, and the hardware hands the next one to whichever CU is free.  What a workgroup lacks, a second
+// slab buffer and staging registers, the other three on the CU make up for: a slab is copied straight to LDS (32 KB,
 // one buffer), waited for, read and multiplied, and meanwhile the others are somewhere else in that cycle.
 // What bounds it is LDS: 96 KB written and read per unit and slab, 750 cycles at 128 B per clock beside 512 of
 // matrix core; about 920 are measured with four workgroups on every CU, against 605 per unit of a full quad.
 // (Wavefronts of 64 x 128, two per workgroup, with all operands of a slab in registers need 80 KB: 710 cycles
 // with four workgroups per CU, but a third slower where there are two or three; not kept.)
-// us, quads -> this: 2900 x 3072 (552 units) cache pass with a quarter cached 35 -> 26, final pass 66 -> 56, dense
-// 64 -> 61; 3200 x 5120 (1000 units) 112 -> 85, 197 -> 147, 212 -> 167; 8192 x 3072 (1536 units) 89 -> 75, 142 -> 135,
-// 144 -> 139; 4608 x 3072 (864 units, 216 quads in one round) 44 -> 43, 76 -> 87, 77 -> 94.
+// us, quads -> this, dense: 2900 x 3072 (552 units) 64 -> 61; 3200 x 5120 (1000 units) 212 -> 167; 4608 x 3072 (864 units, 216 quads
+// in one round) 77 -> 94.
 // ---------------------------------------------------------------------------------------------
 constexpr int kPackedSmemBytes = 2 * kUnitBytes;  // one slab: X, W
 
 template <typename T, bool kReduce, bool kPartial>
 __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmParams p) {
-  if constexpr (kReduce)
-    if (p.sparse_word != nullptr && *p.sparse_word == 0) return;
   using TT = Types<T>;
   using x8 = typename TT::x8;
   using x4 = typename TT::x4;
@@ -1977,6 +1685,479 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// GEMM-O: a workgroup per strip, one token block x two column blocks, two workgroups on a CU.  A strip walks its own
+// block's heads (a quad walks the union of two blocks': 22.5 of 24 where each has 18, 10.5 where each has 6), and
+// 864 units are 432 strips that the hardware hands out, not one round of 216 quads that lasts as long as the longest.
+// A wavefront computes 64 rows x 128 columns: 128 accumulators, a slab's X operands in 32 registers, two sets of W
+// operands of 32 columns; 206 registers, so two wavefronts share a SIMD and one's first touches, waits and epilogue lie
+// beside the other's MFMAs.
+//
+// Data path.  Copies go straight to LDS, whole 128-byte lines.  A slab of W (two tiles, 32 KB) would leave no room for
+// the next one beside a second workgroup, so a slab is multiplied 32 columns at a time, over all of its k, and W lives in
+// a ring of six pieces of 2 x 32 rows (8 KB) of which three to five are on their way; X (16 KB) has two places: 80 KB.
+// Step nt of slab t multiplies piece 4t + nt and reads piece 4t + nt + 1 (and, in its last step, X of slab t + 1, each
+// register as its last MFMA is issued).  Two steps lie between barriers.  Behind the barrier in front of steps 0 and 1:
+// pieces 4t + 5 and 4t + 6 are asked for, into the places of 4t - 1 and 4t, which every wavefront has read by then (of
+// its operand reads only the last four, of X, may be outstanding); in front of steps 2 and 3: pieces 4t + 7 and 4t + 8 and X of slab
+// t + 2.  What a pair of steps reads was asked for at least one pair earlier, so that pair's copies may be outstanding:
+// eight in front of step 0, four in front of step 2.  Copies past the last slab go through empty descriptors (zeros, no
+// memory access).
+//
+// Order.  XCD x owns column pairs of one group and every so many-th token block (strip_cols, see launch_strips), so that
+// its part of W stays in its L2; token blocks with the most selected heads come first (strip_sorted): the long ones do not end
+// the launch, and those that run together walk lists of one length and stay in step, which is what keeps W in L2.  Every
+// workgroup works the order out for itself (a byte or two of flags per block, one pass; ~1 us beside the other
+// workgroup's loop).
+//
+// us, the form it replaces (quads, packed units, or both queued and one chosen on the device) -> strips, bf16: 4608 x 3072
+// (24 heads), flags per head, a quarter selected 46.8 -> 31.5, three quarters 73.5 -> 66.1; a quarter of the blocks with all
+// heads 59.9 -> 42.1, three quarters 72.8 -> 75.1; 33 000 x 3072 with 30 % 250 -> 192; 20 000 x 5120 with 60 % 744 -> 581;
+// 76 112 x 5120 with 80 % 3105 -> 2818, with 20 % 1101 -> 871; 13 000 x 1024 with 60 % 31.4 -> 25.1.  Without the order: 36.2 (4608,
+// a quarter), 670 (20 000 x 5120) and 3321 (76 112 x 5120).
+//
+// What bounds it: LDS and the matrix cores together (96 KB read, 48 KB written per slab of two units beside 1024 cycles of
+// MFMA) and, over long launches, power: dense it takes the time of full quads to 5 % (GEMM-Q's rule in launch_q).
+// ---------------------------------------------------------------------------------------------
+constexpr int kStripPiece = 2 * 32 * kRowBytes;  // 32 rows of W of both column blocks
+constexpr int kStripRing = 6;
+constexpr int kStripSorted = 4096;  // token blocks that are put in order
+constexpr int kStripSmemBytes = 2 * kUnitBytes + kStripRing * kStripPiece;  // 80 KB: two X tiles, the ring of W
+
+// Whether a long launch selects few of its heads, for the ninth word of a caller's scratch: with p of a request's head
+// slices selected, the sum of p (limit / 256 - p) over the requests is not negative.  Judged by up to 4096 bytes of flags in
+// all, of up to 64 requests spread over the batch, from each one's `first_byte` on (n_bytes: how many a request has), by
+// one workgroup; all of them are in flight together.
+constexpr int kJudged = 64, kJudgedBytes = 4096;
+__device__ __forceinline__ void judge_flags(const GemmParams& p, int32_t* s_ones) {
+  const int tid = threadIdx.x, judged = min(p.batch, kJudged);
+  int threads = kThreads;  // of a request: a power of two, at least kThreads / kJudged
+  while (threads * judged > kThreads) threads >>= 1;
+  constexpr int kPer = kJudgedBytes / kThreads;
+  const int n = min(p.judge_bytes, kPer * threads);
+  const int j = tid / threads, at = tid - j * threads;
+  int ones = 0;
+  if (j < judged) {
+    const uint8_t* info = p.sparse_info + p.sparse_info_indptr[static_cast<int64_t>(j) * p.batch / judged] + p.judge_first;
+    uint8_t v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = at + i * threads < n ? info[at + i * threads] : 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) ones += __popc(v[i]);
+  }
+  const int width = min(threads, 64);
+  for (int off = width >> 1; off > 0; off >>= 1) ones += __shfl_xor(ones, off, 64);
+  if (tid % width == 0) s_ones[tid / width] = ones;
+  __syncthreads();
+  if (tid < 64) {
+    // (up to 2^15 selected times 2^21: 64 bits)
+    long long few = 0;
+    if (tid < judged) {
+      int selected = 0;
+      for (int w = 0; w < threads / width; ++w) selected += s_ones[tid * (threads / width) + w];
+      if (p.flag) selected = 8 * n - selected;
+      few = static_cast<long long>(selected) * (p.judge_limit * n - 32 * selected);
+    }
+    for (int off = 32; off > 0; off >>= 1) few += __shfl_xor(few, off, 64);
+    if (tid == 0) *p.judgement = few >= 0;
+  }
+  __syncthreads();
+}
+
+template <typename T, bool kReduce, bool kHalf, bool kPartial>
+__global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParams p) {
+  using TT = Types<T>;
+  using x8 = typename TT::x8;
+  using x4 = typename TT::x4;
+  constexpr int NT = 4, MT = 2;  // wavefront tile: 128 columns (W rows) x 64 token rows (X rows)
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, g = lane >> 5;
+  const int wr = wv >> 1, wc = wv & 1;  // half of the rows; column block
+
+  // ---- which strip ----
+  const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
+  const int cols = p.strip_cols;                 // column groups of XCDs
+  const int xr = xcd / cols, xc = xcd - xr * cols;
+  const int per = p.n_cp / cols;                 // column pairs of an XCD
+  const int rank = xr + (kXcds / cols) * (slot / per);
+  const int cp = xc * per + slot % per;
+  const int n_blocks = p.batch * p.n_row_tiles;
+  if (rank >= n_blocks) return;
+  auto flag_row_of = [&](int row) -> uint32_t {
+    return static_cast<uint32_t>(p.num_text_tokens + row * kTile) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
+  };
+  int block = rank;
+  if constexpr (kReduce) {
+    if (p.judgement != nullptr && blockIdx.x == 0) judge_flags(p, reinterpret_cast<int32_t*>(smem));
+    if (p.strip_sorted) {
+      // token blocks with the most selected heads first
+      uint8_t* const s_key = smem;
+      int32_t* const s_hist = reinterpret_cast<int32_t*>(smem + kStripSorted);
+      const int n_slices = p.k / p.head_dim;
+      if (tid < 64) s_hist[tid] = 0;
+      __syncthreads();
+      for (int i = tid; i < n_blocks; i += kThreads) {
+        const int b = i / p.n_row_tiles;
+        const uint8_t* info = p.sparse_info + p.sparse_info_indptr[b];
+        const uint32_t lo = flag_row_of(i - b * p.n_row_tiles), hi = lo + n_slices;
+        int ones = 0;
+        for (uint32_t at = lo >> 3; at <= (hi - 1) >> 3; ++at) {
+          uint32_t v = info[at];
+          if (at == lo >> 3) v &= 0xFFu << (lo & 7);
+          if (at == hi >> 3) v &= (1u << (hi & 7)) - 1u;
+          ones += __popc(v);
+        }
+        if (p.flag) ones = n_slices - ones;
+        const int key = n_slices < 64 ? ones : ones * 63 / n_slices;
+        s_key[i] = static_cast<uint8_t>(key);
+        atomicAdd(&s_hist[key], 1);
+      }
+      __syncthreads();
+      const int here = s_hist[63 - lane], upto = fo::wave_scan(here);
+      const unsigned long long past = __ballot(rank < upto);
+      const int at = __builtin_ctzll(past), want = 63 - at;
+      int skip = rank - __builtin_amdgcn_readlane(upto - here, at);
+      for (int i0 = 0; i0 < n_blocks; i0 += 64) {
+        unsigned long long same = __ballot(i0 + lane < n_blocks && s_key[i0 + lane] == want);
+        const int n = __popcll(same);
+        if (skip < n) {
+          for (; skip > 0; --skip) same &= same - 1;
+          block = i0 + __builtin_ctzll(same);
+          break;
+        }
+        skip -= n;
+      }
+      __syncthreads();
+    }
+  }
+  const int bz = block / p.n_row_tiles, row = block - bz * p.n_row_tiles;
+  const int m0 = row * kTile;
+  const uint32_t flag_row = flag_row_of(row);
+
+  const int c0 = 2 * cp, c1 = 2 * cp + 1 < p.n_col_tiles ? 2 * cp + 1 : -1;  // (the last pair may lack its second)
+  // ---- the slabs: heads of this token block (GEMM-O), or all of k ----
+  unsigned long long mask[4] = {0, 0, 0, 0};
+  int n_iter, iph = 1, word = 0, sub = 0, k0 = 0;
+  if constexpr (kReduce) {
+    const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+    const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
+    const int n_slices = p.k / p.head_dim;
+    bool sel[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sel[i] = 64 * i + lane < n_slices && flag_bit(info, flag_row + 64 * i + lane) == pick;
+    int count = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      mask[i] = __ballot(sel[i]);
+      count += __popcll(mask[i]);
+    }
+    iph = (p.head_dim + kBK - 1) / kBK;
+    n_iter = count * iph;
+  } else {
+    n_iter = (p.k + kBK - 1) / kBK;
+  }
+  // The next slab: its k offset, and (kHalf: heads or K of 32 mod 64) which half of it counts.  The last slab of a slice
+  // reaches 32 back; where the matrix begins, forward.
+  struct Slab {
+    uint32_t k;             // in bytes
+    uint32_t first, second;  // masks of its halves
+  };
+  auto next_slab = [&]() __attribute__((always_inline)) -> Slab {
+    Slab s{0, ~0u, ~0u};
+    if constexpr (kReduce) {
+      if (sub == 0) {
+        unsigned long long m = mask[0];
+#pragma unroll
+        for (int i = 1; i < 4; ++i) {
+          if (m == 0 && word < i) {
+            word = i;
+            mask[0] = m = mask[i];
+          }
+        }
+        k0 = (64 * word + __builtin_ctzll(m | (1ull << 63))) * p.head_dim;
+        mask[0] = m & (m - 1);
+      } else {
+        k0 += kBK;
+      }
+      if (++sub == iph) sub = 0;
+      s.k = static_cast<uint32_t>(k0) * 2u;
+      if constexpr (kHalf) {
+        if (sub == 0) {
+          if (k0 >= 32) s.k -= 64u;
+          (k0 >= 32 ? s.first : s.second) = 0u;
+        }
+      }
+    } else {
+      s.k = static_cast<uint32_t>(k0) * 2u;
+      k0 += kBK;
+      if constexpr (kHalf) {
+        if (k0 > p.k) {
+          s.k -= 64u;
+          s.first = 0u;
+        }
+      }
+    }
+    return s;
+  };
+
+  const T* __restrict__ xg = static_cast<const T*>(p.x);
+  const T* __restrict__ wg = static_cast<const T*>(p.w);
+  const int rows_here = min(p.m - m0, kTile);
+  const uint32_t k2 = static_cast<uint32_t>(p.k) * 2u;
+  const T* const x_base = xg + (static_cast<int64_t>(bz) * p.m + m0) * p.k;
+  const uint32_t x_bytes = static_cast<uint32_t>(rows_here) * k2;
+  // (a wavefront copies for column block wv / 2 and computes column block wv % 2)
+  const int c_copy = wv >> 1 ? c1 : c0, c_mine = wc ? c1 : c0;
+  const T* const w_base = wg + static_cast<int64_t>(max(c_copy, 0)) * kTile * p.k;
+  const uint32_t w_bytes = c_copy < 0 ? 0u : kTile * k2;
+  auto rsrc = [&](const T* base, uint32_t bytes) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, bytes, 0x00020000);
+  };
+  uint32_t voff[2];
+#pragma unroll
+  for (int par = 0; par < 2; ++par)
+    voff[par] = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4);
+  typedef __attribute__((address_space(3))) void lds_void;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
+  const uint32_t ldsw = lds0 + 2 * kUnitBytes;  // the ring
+  const uint32_t row8 = 8u * k2;
+  auto copy = [&](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(vo), "s"(r), "s"(soff)
+                 : "memory", "m0");
+  };
+  const uint32_t x_soff = 4u * wv * row8, w_soff = 2u * (wv & 1) * row8;
+  const uint32_t x_dst = lds0 + wv * 32 * kRowBytes, w_dst = ldsw + (wv >> 1) * 32 * kRowBytes + (wv & 1) * 16 * kRowBytes;
+  auto copy_x = [&](__amdgpu_buffer_rsrc_t r, int i, uint32_t koff, uint32_t buf) __attribute__((always_inline)) {
+    copy(r, voff[i & 1], koff + x_soff + i * row8, x_dst + buf + i * 8 * kRowBytes);
+  };
+  auto copy_w = [&](__amdgpu_buffer_rsrc_t r, int nt, int i, uint32_t koff, uint32_t at) __attribute__((always_inline)) {
+    copy(r, voff[i & 1], koff + w_soff + (4 * nt + i) * row8, w_dst + at + i * 8 * kRowBytes);
+  };
+
+  // acc[nt][mt][i]: column nt*32 + (i/4)*8 + g*4 + i%4 of the block, row wr*64 + mt*32 + l32
+  f32x16 acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
+
+  if (n_iter > 0) {
+    typedef __attribute__((address_space(3))) const x8 lds_x8;
+    const int rd_x = (g ^ ((l32 >> 1) & 7)) << 4;
+    uint32_t lane_off[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) lane_off[ks] = static_cast<uint32_t>(l32 * kRowBytes + (rd_x ^ (ks << 5)));
+    const uint32_t x_src = lds0 + wr * 64 * kRowBytes, w_src = ldsw + wc * 32 * kRowBytes;
+    x8 xr_[MT][4], wreg[2][4];
+    auto read_x = [&](int mt, int ks, uint32_t buf) __attribute__((always_inline)) {
+      xr_[mt][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (x_src + buf) + mt * 32 * kRowBytes));
+    };
+    auto read_w = [&](int set, int ks, uint32_t at) __attribute__((always_inline)) {
+      wreg[set][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (w_src + at)));
+    };
+    // prologue: X of slab 0, pieces 0 to 2 | pieces 3 and 4, X of slab 1
+    Slab sa = next_slab(), sb = sa;  // slabs it, it + 1
+    if (n_iter > 1) sb = next_slab();
+    {
+      const __amdgpu_buffer_rsrc_t rx = rsrc(x_base, x_bytes), rw = rsrc(w_base, w_bytes);
+      const __amdgpu_buffer_rsrc_t rx1 = rsrc(x_base, n_iter > 1 ? x_bytes : 0u), rw1 = rsrc(w_base, n_iter > 1 ? w_bytes : 0u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) copy_x(rx, i, sa.k, 0);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) copy_w(rw, q, i, sa.k, q * kStripPiece);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) copy_w(rw, 3, i, sa.k, 3 * kStripPiece);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) copy_w(rw1, 0, i, sb.k, 4 * kStripPiece);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) copy_x(rx1, i, sb.k, kUnitBytes);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) read_w(0, ks, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      read_x(0, ks, 0);
+      read_x(1, ks, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t ring = 0;  // place of the slab's first piece
+    uint32_t xbuf = 0;
+    auto place = [&](int j) __attribute__((always_inline)) -> uint32_t {  // of the j-th piece from the slab's first on
+      uint32_t at = ring + j * kStripPiece;
+      at = at >= 2 * kStripRing * kStripPiece ? at - 2 * kStripRing * kStripPiece : at;
+      return at >= kStripRing * kStripPiece ? at - kStripRing * kStripPiece : at;
+    };
+    for (int it = 0; it < n_iter; ++it) {
+      const bool live1 = it + 1 < n_iter, live2 = it + 2 < n_iter;
+      Slab sc = sb;
+      if (live2) sc = next_slab();
+      const __amdgpu_buffer_rsrc_t rw1 = rsrc(w_base, live1 ? w_bytes : 0u);
+      const __amdgpu_buffer_rsrc_t rw2 = rsrc(w_base, live2 ? w_bytes : 0u), rx2 = rsrc(x_base, live2 ? x_bytes : 0u);
+      auto step = [&](auto nt_tag) __attribute__((always_inline)) {
+        constexpr int nt = decltype(nt_tag)::value, set = nt & 1;
+        const uint32_t rd = place(nt + 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int ks = j >> 1, mt = j & 1;
+          if constexpr (kHalf && nt == 0) {
+            u32x4 v = __builtin_bit_cast(u32x4, xr_[mt][ks]);
+            v &= ks < 2 ? sa.first : sa.second;
+            xr_[mt][ks] = __builtin_bit_cast(x8, v);
+          }
+          acc[nt][mt] = TT::mfma(wreg[set][ks], xr_[mt][ks], acc[nt][mt]);
+          if (j < 4) read_w(set ^ 1, j, rd);
+          if constexpr (nt == 3) {
+            if (j & 1) {
+              read_x(0, ks, xbuf ^ kUnitBytes);
+              read_x(1, ks, xbuf ^ kUnitBytes);
+            }
+          }
+          if constexpr (nt < 2) {
+            if (j == 2 || j == 5) copy_w(rw1, nt + 1, j == 5, sb.k, place(5 + nt));
+          } else {
+            if (j == 1 || j == 3) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, j == 3, nt == 2 ? sb.k : sc.k, place(5 + nt));
+            if (j == 5 || j == 7) copy_x(rx2, 2 * (nt - 2) + (j == 7), sc.k, xbuf);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
+      __builtin_amdgcn_s_waitcnt(0xc47f);      // lgkmcnt(4)
+      __builtin_amdgcn_s_barrier();
+      step(std::integral_constant<int, 0>{});
+      step(std::integral_constant<int, 1>{});
+      __builtin_amdgcn_s_waitcnt(0x0f70 | 4);  // vmcnt(4)
+      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      step(std::integral_constant<int, 2>{});
+      step(std::integral_constant<int, 3>{});
+      ring = place(4);
+      xbuf ^= kUnitBytes;
+      sa = sb;
+      sb = sc;
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): copies past the end and operand reads
+  __builtin_amdgcn_s_barrier();
+  if (c_mine < 0) return;
+
+  // ---- epilogue: 32 rows at a time through a wavefront's quarter of the memory ----
+  uint8_t* const region = smem + wv * (kStripSmemBytes / 4);
+  const int col4 = lane & 31, rsub = lane >> 5;
+  const int n0 = c_mine * kTile;
+  const int el_off = n0 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 2*i
+  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
+  auto out_rsrc = [&](const void* base, int elem_bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
+        rows_here * p.n * elem_bytes, 0x00020000);
+  };
+  auto turn = [&](auto bias_tag, auto f32_tag) {
+    using BiasT = decltype(bias_tag);
+    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
+    constexpr bool kOutF32 = decltype(f32_tag)::value;
+    constexpr int kBytes = sizeof(BiasT);
+    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!kPartial) {
+      if (p.bias_kind == FO_BIAS_VECTOR) {
+        const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + col4 * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+      }
+    }
+    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      // (rows whose partial is in flight together: sixteen of fp32 do not fit beside the accumulators)
+      constexpr int kAhead = kBytes == 4 ? 8 : 16;
+      BiasVec bm[kAhead];
+      auto load_partial = [&](int i0) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const int r = (32 * mt + 2 * (i0 + i)) * p.n;
+          if constexpr (kBytes == 4) {
+            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, r * 4, 0));
+          } else {
+            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, r * 2, 0));
+          }
+        }
+      };
+      if constexpr (kPartial) load_partial(0);
+      // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 512 bytes = 32 chunks)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          f32x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = acc[nt][mt][i4 * 4 + j];
+          const int chunk = nt * 8 + i4 * 2 + g;
+          *reinterpret_cast<f32x4*>(region + l32 * 512 + ((chunk ^ (l32 & 15)) << 4)) = v;
+        }
+      f32x4 vals[8];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if ((i & 7) == 0) {
+          if constexpr (kPartial)
+            if (i > 0 && i % kAhead == 0) load_partial(i);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const int rk = (i + k) * 2 + rsub;
+            vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 512 + ((col4 ^ (rk & 15)) << 4));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x4 v = vals[i & 7];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (kPartial) {
+            v[j] += static_cast<float>(bm[i % kAhead][j]);
+          } else {
+            v[j] += bvec[j];
+          }
+        }
+        const int r = (32 * mt + 2 * i) * p.n;
+        if constexpr (kOutF32) {
+          // (no scalar offset: see the quads' store)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + r) * 4, 0, 2);
+        } else {
+          x4 out;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+          typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, r * 2, 2);
+        }
+      }
+    }
+  };
+  using std::false_type;
+  using std::true_type;
+  if constexpr (!kReduce) {
+    turn(T{}, false_type{});
+  } else if constexpr (kPartial) {
+    if (p.bias_f32) {
+      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
+    } else {
+      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+    }
+  } else {
+    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+  }
+}
+
 ListGeom make_geom(int32_t batch, int32_t m, int32_t n) {
   ListGeom gm;
   gm.batch = batch;
@@ -1994,6 +2175,15 @@ int64_t workspace_ints(const ListGeom& gm, int64_t* max_quads_out) {
   return 16 + kQuadInts * max_quads;
 }
 
+int64_t unit_count(const ListGeom& gm) { return static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles; }
+
+// units that the rounds of quads have room for, a quad per CU and round
+int64_t quad_slots(const ListGeom& gm, int num_cu) {
+  const int64_t quads = static_cast<int64_t>(gm.batch) * gm.n_cp *
+                        (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
+  return (quads + num_cu - 1) / num_cu * 4 * num_cu;
+}
+
 // a workgroup per unit
 template <typename T, bool kReduce, bool kHalf, bool kAux>
 int launch_units(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
@@ -2007,7 +2197,7 @@ int launch_units(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   }
   p.n_row_tiles = gm.n_row_tiles;
   p.n_col_tiles = gm.n_col_tiles;
-  const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
+  const int64_t units = unit_count(gm);
   const int64_t grid = (units + kXcds - 1) / kXcds * kXcds;
   gemm_unit_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kUnitSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
@@ -2019,7 +2209,7 @@ template <typename T, bool kReduce, bool kAux>
 int launch_packed(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   p.n_row_tiles = gm.n_row_tiles;
   p.n_col_tiles = gm.n_col_tiles;
-  const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
+  const int64_t units = unit_count(gm);
   const int64_t grid = (units + kXcds - 1) / kXcds * kXcds;
   gemm_packed_kernel<T, kReduce, kAux><<<static_cast<unsigned>(grid), kThreads, kPackedSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
@@ -2027,61 +2217,85 @@ int launch_packed(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 }
 
 template <typename T, bool kReduce, bool kHalf, bool kAux>
-int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace, hipStream_t stream) {
+int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
+  static std::atomic<bool> attr_set[64] = {};
+  int dev = 0;
+  FO_HIP_CALL(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_strip_kernel<T, kReduce, kHalf, kAux>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kStripSmemBytes));
+    if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
+  }
+  p.n_row_tiles = gm.n_row_tiles;
+  p.n_col_tiles = gm.n_col_tiles;
+  p.n_cp = gm.n_cp;
+  // Column groups of XCDs: four, two or one that divide the column pairs and leave each at least three (20 000 x 5120, 60 % of
+  // the heads: one group 734 us, two 619, four 574; 33 000 x 3072 dense 514, 499, 500).  Narrower ones are bound by memory, and
+  // there a token block should be read by one XCD (60 000 x 512 dense: one group 36.8 us, two 39.4).
+  int cols = 1;
+  while (cols < 4 && gm.n_cp % (2 * cols) == 0 && gm.n_cp >= 6 * cols) cols *= 2;
+  p.strip_cols = cols;
+  const int64_t rows = static_cast<int64_t>(gm.batch) * gm.n_row_tiles;
+  p.strip_sorted = rows <= kStripSorted;
+  const int rx = kXcds / cols;
+  const int64_t grid = (rows + rx - 1) / rx * (gm.n_cp / cols) * kXcds;
+  gemm_strip_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kStripSmemBytes, stream>>>(p);
+  FO_CHECK_LAUNCH();
+  return FO_OK;
+}
+
+// GEMM-O.
+//   * A workgroup per unit while all of them fit the chip at once, two per CU (144 units of K = 1024: quads 28 us, units
+//     12; strips over units up to one per CU 1.3 .. 1.6, of one to two 0.91 .. 1.3, about equal from K = 1024 on).
+//   * Narrow matrices, up to K = 512, are bound by memory and want the most loads in flight: packed units (strips over them,
+//     three to ten units per CU: 256 columns 1.0 .. 1.3, 384 1.1 .. 1.4, 512 1.0 .. 1.1).
+//   * Everything else: strips.  Over the better of quads and packed units, 2.3 to 9.7 units per CU, with 10, 50, 90 % of
+//     the heads selected:
+//        8 heads 0.69 .. 1.06, 0.84 .. 1.03, 0.91 .. 1.06     12  0.65 .. 0.94, 0.79 .. 0.97, 0.87 .. 1.02
+//       16       0.68 .. 0.93, 0.78 .. 0.97, 0.88 .. 1.02     24  0.63 .. 0.90, 0.69 .. 1.01, 0.84 .. 1.04
+//       40       0.64 .. 0.85, 0.60 .. 0.89, 0.80 .. 1.06
+template <typename T, bool kHalf, bool kPartial>
+int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   const int num_cu = fo_num_cu();
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
-  // A workgroup per unit while all of them fit the chip at once, two per CU: quads would leave most CUs
-  // idle or without their fourth unit.  Measured (us, quads -> units): 144 units of K = 1024 28 -> 12,
-  // 256 of K = 2048 46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged.  Above
-  // that it depends on the flags, which the host does not see: 864 units of K = 3072 83 -> 98 dense,
-  // 59 -> 43 with a quarter flagged.  (The fused quantiser needs a unit's absmax: quads only.)
-  if constexpr (kReduce || !kAux) {
-    if (static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles <= 2 * num_cu)
-      return launch_units<T, kReduce, kHalf, kAux>(p, gm, stream);
-  }
-  // Packed units or quads.  Quads come in rounds of one per CU, so packed units are ahead where the last round is
-  // nearly empty, and in GEMM-O, whose quads walk the union of two token blocks' heads; they fall behind with the
-  // width: more of W than an XCD's L2 holds, and, where the flags differ from block to block, workgroups of
-  // neighbouring units that drift apart in it.  Measured over 2.1 to 32 units per CU, heads of 128, square W; times of
-  // packed units over quads' with 2, 25, 50, 80, 100 % of the heads selected, at 20 to 24 units per CU in full rounds:
-  //    8 heads 0.66 0.66 0.76 0.90 1.00      16  0.62 0.70 0.83 0.99 1.05      24  0.61 0.83 1.05 1.28 1.15
-  //   40 heads 0.65 0.99 1.24 1.53 1.34      64  0.70 1.12 1.56 1.91 1.31
-  //   * GEMM-O of one round: up to three units per CU (0.5 .. 1.02 with up to 80 % selected, at most 1.14 with all; four
-  //     units: 0.65 .. 1.35).
-  //   * GEMM-O of more: always up to K = 2048 (at worst 1.09, all heads selected; a choice by the flags costs 7 us, 2 to
-  //     10 % of these launches), wider up to 21 / 32 of the rounds filled (at worst 1.0) or as far as the width times
-  //     the fill is at most 18 heads' (24 heads, rounds filled to 3/4: at worst 1.05).
-  //   * Beyond that it depends on the flags, which the host does not see: both forms are launched, and one of them
-  //     ends at once, as a kernel of a few microseconds in front has decided (5 to 8 us in all where quads are
-  //     chosen, up to 3 % of these launches).  Packed units run where the selected share is below 13 heads over
-  //     (width times fill), 10 from sixteen units per CU on: the line where the two were measured equal, to 0.06 (24
-  //     heads: 0.67 at 7 units per CU and a fill of 0.88, 0.57 at 12 and 1.0, 0.41 at 24 and 1.0; 40 heads: 0.47 at 12
-  //     and 0.75, 0.32 at 10 and 0.87, 0.26 at 20 and 1.0; 64 heads: 0.23 at 10 and 0.88, 0.16 at 20 and 1.0).
-  //   * Dense GEMM-Q: up to 21 / 32 of the rounds filled (0.75 .. 1.02; at 0.75 0.85 with 8 heads, 1.14 with 40), in a single
-  //     round only up to K = 2048 (0.88 .. 1.01; 24 heads 1.05, 40 heads 1.07 .. 1.11).
-  // GEMM-Q with flags keeps its lists, which pack units whatever their number (at 552 units, a quarter of them
-  // flagged, 42 us against 47).
-  if constexpr (!kHalf && (kReduce || !kAux)) {
-    const int64_t units = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_col_tiles;
-    const int64_t quads = static_cast<int64_t>(gm.batch) * gm.n_cp *
-                          (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
-    const int64_t rounds = (quads + num_cu - 1) / num_cu, slots = 4 * num_cu * rounds;
-    const bool narrow = p.k <= 2048, few = 32 * units <= 21 * slots;
-    if (!use_flags && (rounds == 1 ? (kReduce ? units <= 3 * num_cu : narrow && few)
-                                   : few || (kReduce && (narrow || p.k * units <= 18 * 128 * slots))))
-      return launch_packed<T, kReduce, kAux>(p, gm, stream);
-    if constexpr (kReduce) {
-      const int64_t line = (units > 15 * num_cu ? 10 : 13) * 128 * 256 * slots / (p.k * units);
-      const int limit = static_cast<int>(line < 256 ? line : 256);  // of 256
-      if (p.cursor != nullptr && rounds > 1 && limit >= 32) {
-        const int64_t first = static_cast<int64_t>(p.num_text_tokens) / p.sparse_q_size * p.num_heads / 8;
-        const int64_t bits = static_cast<int64_t>(p.m) / p.sparse_q_size * p.num_heads;
-        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, gm.batch, static_cast<int32_t>(first),
-                                                       static_cast<int32_t>(bits / 8 < kJudgedBytes ? bits / 8 : kJudgedBytes), p.flag == 0, limit);
-        FO_CHECK_LAUNCH();
-        p.sparse_word = p.cursor + 8;
-        if (int rc = launch_packed<T, kReduce, kAux>(p, gm, stream)) return rc;
-      }
+  if (unit_count(gm) <= 2 * num_cu) return launch_units<T, true, kHalf, kPartial>(p, gm, stream);
+  if constexpr (!kHalf)
+    if (p.k <= 512) return launch_packed<T, true, kPartial>(p, gm, stream);
+  // (launches that could be judged both ways: more than one round of quads, 13 heads over the width times the rounds' fill,
+  // 10 from sixteen units per CU on)
+  const int64_t slots = quad_slots(gm, num_cu), units = unit_count(gm);
+  const int64_t line = (units > 15 * num_cu ? 10 : 13) * 128 * 256 * slots / (p.k * units);
+  p.judge_limit = static_cast<int32_t>(line < 256 ? line : 256);  // of 256
+  if (kHalf || slots == 4 * num_cu || p.judge_limit < 32) p.judgement = nullptr;
+  p.judge_first = p.num_text_tokens / p.sparse_q_size * p.num_heads / 8;
+  const int64_t bytes = static_cast<int64_t>(p.m) / p.sparse_q_size * p.num_heads / 8;
+  p.judge_bytes = static_cast<int32_t>(bytes < kJudgedBytes ? bytes : kJudgedBytes);
+  return launch_strips<T, true, kHalf, kPartial>(p, gm, stream);
+}
+
+// GEMM-Q.
+//   * A workgroup per unit while all of them fit the chip at once, two per CU (us, quads -> units: 256 units of K = 2048
+//     46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged).
+//   * With flags: quads, column strips and pairs by the kernel's own list.
+//   * Dense: a quad per CU and round, so it depends on how full the rounds are.  Packed units up to 21 / 32 of them (over
+//     quads 0.75 .. 1.02), in a single round only up to K = 2048 (0.88 .. 1.01; 24 heads 1.05, 40 heads 1.07 .. 1.11).  Strips
+//     up to K = 512 (0.87 .. 0.95 over 2.9 to 23 units per CU) and where two quads' units per CU would be empty in the last
+//     of several rounds (8 heads 0.80 .. 0.87, 16 0.85 .. 0.92, 24 0.87 .. 0.95, 40 0.88 .. 0.98; fuller rounds 0.95 .. 1.09;
+//     where packed units are taken they take 1.0 .. 1.2 of those' time).
+//   (The fused quantiser needs a unit's absmax in one wavefront: quads only.)
+template <typename T, bool kHalf, bool kQuant>
+int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace, hipStream_t stream) {
+  const int num_cu = fo_num_cu();
+  if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
+  if constexpr (!kQuant) {
+    const int64_t units = unit_count(gm);
+    if (units <= 2 * num_cu) return launch_units<T, false, kHalf, false>(p, gm, stream);
+    if (!use_flags) {
+      const int64_t slots = quad_slots(gm, num_cu);
+      const bool one_round = slots == 4 * num_cu;
+      if constexpr (!kHalf)
+        if (32 * units <= 21 * slots && (!one_round || p.k <= 2048)) return launch_packed<T, false, false>(p, gm, stream);
+      if (p.k <= 512 || (!one_round && slots - units >= 2 * num_cu)) return launch_strips<T, false, kHalf, false>(p, gm, stream);
     }
   }
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
@@ -2090,7 +2304,7 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
-    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<T, kReduce, kHalf, kAux>),
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<T, kHalf, kQuant>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes));
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
@@ -2109,29 +2323,17 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
     // every unit is computed: no list, the kernel enumerates the quads itself
     p.quads = nullptr;
     p.qoff = nullptr;
-    // (cursors pay off when a workgroup sees several items; short launches keep the fixed stride and
-    // save the extra launch)
-    const int64_t items = static_cast<int64_t>(gm.batch) * gm.n_cp *
-                          (gm.n_row_tiles / kWindow * (kWindow / 2) + (gm.n_row_tiles % kWindow + 1) / 2);
-    if (kReduce && p.cursor != nullptr && (items >= 4 * grid || p.sparse_word != nullptr)) {
-      if (p.sparse_word == nullptr) {
-        gemm_choose_kernel<<<1, kThreads, 0, stream>>>(p.cursor, p.sparse_info, p.sparse_info_indptr, 0, 0, 0, 0, 0);
-        FO_CHECK_LAUNCH();
-      }
-    } else {
-      p.cursor = nullptr;
-    }
-    gemm_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
+    gemm_kernel<T, kHalf, kQuant><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
     FO_CHECK_LAUNCH();
     return FO_OK;
   }
   const int64_t n_cells = static_cast<int64_t>(gm.batch) * gm.n_win * gm.n_cp;
-  if (!kReduce && n_cells <= kInlineCells) {
+  if (n_cells <= kInlineCells) {
     // short launch: the kernel lists its quads itself (one launch less)
     p.quads = nullptr;
     p.qoff = nullptr;
     p.inline_cells = static_cast<int32_t>(n_cells);
-    gemm_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
+    gemm_kernel<T, kHalf, kQuant><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
     FO_CHECK_LAUNCH();
     return FO_OK;
   }
@@ -2149,7 +2351,7 @@ int launch_half(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspa
   FO_CHECK_LAUNCH();
   p.quads = quads;
   p.qoff = qoff;
-  gemm_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
+  gemm_kernel<T, kHalf, kQuant><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
 }
@@ -2161,11 +2363,17 @@ int launch(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace, h
   const bool half = (kReduce ? p.head_dim : p.k) % kBK != 0;
   // fused quantisation (GEMM-Q) and the cached partial (GEMM-O) get instantiations of their own, so
   // that the plain kernels do not carry their registers
-  if (kReduce ? p.bias_kind == FO_BIAS_MATRIX : p.y8 != nullptr)
-    return half ? launch_half<T, kReduce, true, true>(p, gm, use_flags, workspace, stream)
-                : launch_half<T, kReduce, false, true>(p, gm, use_flags, workspace, stream);
-  return half ? launch_half<T, kReduce, true, false>(p, gm, use_flags, workspace, stream)
-              : launch_half<T, kReduce, false, false>(p, gm, use_flags, workspace, stream);
+  if constexpr (kReduce) {
+    if (p.bias_kind == FO_BIAS_MATRIX)
+      return half ? launch_o<T, true, true>(p, gm, stream) : launch_o<T, false, true>(p, gm, stream);
+    return half ? launch_o<T, true, false>(p, gm, stream) : launch_o<T, false, false>(p, gm, stream);
+  } else {
+    if (p.y8 != nullptr)
+      return half ? launch_q<T, true, true>(p, gm, use_flags, workspace, stream)
+                  : launch_q<T, false, true>(p, gm, use_flags, workspace, stream);
+    return half ? launch_q<T, true, false>(p, gm, use_flags, workspace, stream)
+                : launch_q<T, false, false>(p, gm, use_flags, workspace, stream);
+  }
 }
 
 int check_common(const void* x, const void* w, void* y, int dtype, int32_t batch, int32_t m,
@@ -2298,10 +2506,9 @@ extern "C" int fo_gemm_o(const void* x, const void* w, const void* bias, void* y
   p.bias_kind = bias_kind;
   p.bias_f32 = bias_dtype == FO_F32;
   p.y_f32 = y_dtype == FO_F32;
-  // (optional workspace: room for the work-item cursors of a long launch)
-  p.cursor = workspace != nullptr && workspace_bytes >= 64 && (reinterpret_cast<uintptr_t>(workspace) & 3) == 0
-                 ? static_cast<int32_t*>(workspace)
-                 : nullptr;
+  p.judgement = workspace != nullptr && workspace_bytes >= 64 && (reinterpret_cast<uintptr_t>(workspace) & 3) == 0
+                    ? static_cast<int32_t*>(workspace) + 8
+                    : nullptr;
   const ListGeom gm = make_geom(batch, m, n);
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == FO_BF16 ? launch<__bf16, true>(p, gm, false, workspace, s)

@@ -49,7 +49,7 @@ def _symbols(sparse_info, sparse_info_indptr, device, name, batch, m, num_qo_hea
     return info, indptr
 
 
-# Scratch of the GEMMs (GEMM-Q's tile list, GEMM-O's work-item cursors).  Eager calls share one
+# Scratch of the GEMMs (GEMM-Q's tile list, GEMM-O's word on the flags' density).  Eager calls share one
 # buffer per (device, stream): calls on one stream run in order, calls on different streams may
 # overlap and get their own.  A call made while its stream is being captured into a graph gets a
 # buffer of its own from the allocator (the graph's memory pool then owns it for as long as the
@@ -229,8 +229,8 @@ def flashomni_gemm_reduction(
     info, indptr = _symbols(sparse_info, sparse_info_indptr, A.device, "flashomni_gemm_reduction",
                             Bsz, M, num_qo_heads, num_text_tokens, sparse_q_size)
     L = _lib.lib()
-    # (the reduction visits every token block and needs no tile list; long launches keep their
-    # work-item cursors in the first bytes of the stream's scratch buffer)
+    # (the reduction visits every token block and needs no tile list; long launches leave a word on the flags'
+    # density in the stream's scratch buffer)
     stream = _lib.current_stream(A.device)
     ws_bytes = 256
     workspace = _gemm_workspace(A.device, stream, ws_bytes)

@@ -400,13 +400,10 @@ int fo_gemm_q(const void* x, const void* w, const void* bias, void* y, int dtype
  * y_dtype: the activation dtype or FO_F32 (so a cached partial can stay in fp32).
  * hd must be a multiple of 32.  No tile list is needed (every token block is visited, the tile
  * order is computed arithmetically), so `workspace` may be NULL; fo_gemm_q with is_full != 0
- * likewise.  Given 64 bytes or more of 4-byte-aligned device scratch, a call of more than four tiles (128 x 128)
- * per CU may hand its work items out through cursors kept there (work items of unequal length then stay
- * neighbours in L2), and be computed tile by tile or four tiles at a time as the density of the flags, judged on the
- * device, makes faster (the same results, bit for bit).  Such a call is several launches, which hand cursors and
- * choice on in the scratch.  Calls that share the scratch must not overlap in time, and none of their launches
- * may come to lie between another one's: on one stream that means that host threads make them one at a time
- * (two calls whose launches mix can leave an output unwritten).  fo_gemm_q's workspace likewise.
+ * likewise.  Given 64 bytes or more of 4-byte-aligned device scratch, a call of more than one round of four tiles (128 x
+ * 128) per CU leaves in its ninth word whether the flags select few of the heads (1) or many (0), which chooses nothing.
+ * fo_gemm_q's workspace holds a call's tile list: calls that share it must not overlap in time, and none of their launches
+ * may come to lie between another one's: on one stream that means that host threads make them one at a time.
  * ------------------------------------------------------------------------------------------- */
 int fo_gemm_o(const void* x, const void* w, const void* bias, void* y, int dtype, int bias_kind,
               int bias_dtype, int y_dtype, int32_t batch, int32_t m, int32_t n, int32_t k,

@@ -520,6 +520,65 @@ def test_packed_units_equal_quads(dev, case, dtype):
     assert rel_l2(everything[0][:few], ref) <= REL_L2
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [(1025, 128, 5, 14), (130, 96, 8, 48), (257, 64, 70, 5), (384, 32, 132, 6), (1, 32, 256, 9),
+                                  (2177, 320, 4, 4), (3, 128, 5, 4100)])
+def test_strips_equal_units(dev, case, dtype):
+    """GEMM-O of many units computes strips of one token block x two column blocks, few units one at a time: a batch
+    entry alone and among many gives the same bits, in both passes, with either output and partial type.  Requests with
+    no head selected anywhere, with one head (a list of one slab), with all of them; one, two, three and more token rows
+    past a block; an odd number of column blocks; heads of 32 to 320 columns, so slabs of which one half counts, at the
+    beginning of the matrix too; 5 to 256 heads (one to four words of flags); more token blocks than are put in order."""
+    import flashomni_amd as fo
+    m, hd, heads, batch = case
+    n, rows = heads * hd, -(-m // 128)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert n > 512 and rows * (n // 128) <= 2 * 256 and (cus != 256 or batch * rows * (n // 128) > 2 * cus)
+    rng = np.random.default_rng(m + heads)
+    info = rng.random((batch, rows + 1, heads)) < rng.random((batch, rows + 1, 1))
+    info[0], info[-1] = True, False
+    info[1] = np.arange(heads) == rng.integers(heads, size=(rows + 1, 1))
+    segs = [np.packbits(f.reshape(-1).astype(np.uint8), bitorder="little") for f in info]
+    pk = torch.from_numpy(np.concatenate(segs)).to(dev)
+    ip = torch.from_numpy(np.cumsum([0] + [len(f) for f in segs]).astype(np.int32)).to(dev)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+
+    def chain(x, ip):
+        part = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=b, is_for_cache=True)
+        part32 = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=b, is_for_cache=True, out_dtype=torch.float32)
+        return [part, part32, fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part),
+                fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part32, out_dtype=torch.float32)]
+
+    many = chain(x, ip)
+    for i in sorted({0, 1, batch // 2, batch - 1}):
+        for k, (one, all_) in enumerate(zip(chain(x[i:i + 1].contiguous(), ip[i:i + 2].contiguous()), many)):
+            assert torch.equal(one[0], all_[i]), (i, k)
+    dense = torch.nn.functional.linear(x.float(), w.float(), b.float())
+    assert rel_l2(many[3], dense) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 26003, 512, 512), (3, 10497, 384, 96), (1, 7289, 3072, 3072), (2, 3650, 2944, 2976)])
+def test_dense_gemm_q_as_strips(dev, shape, dtype):
+    """Full GEMM-Q of narrow matrices and of rounds of quads that end half empty: strips.  Ragged last rows, an odd number
+    of column blocks, K of 32 mod 64; against the fp32 product (the result is rounded once: half a unit of its last place)."""
+    import flashomni_amd as fo
+    batch, m, n, k = shape
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(batch, m, k, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, k, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+    y = fo.flashomni_gemm(x, w, n // 128, num_text_tokens=0, bias=b, is_full=True)
+    ref = torch.nn.functional.linear(x.float(), w.float(), b.float())
+    half_ulp = 2.0 ** (-9 if dtype == torch.bfloat16 else -11)
+    # (sums of k products in another order: k * 2^-24 of the sum of their sizes, below 16 standard deviations of one)
+    assert bool(((y.float() - ref).abs() <= 2 * half_ulp * ref.abs() + k * 2.0 ** -24 * 16 * 0.02).all())
+    assert rel_l2(y, ref) <= half_ulp
+
+
 @pytest.mark.parametrize("p_active", [0.0, 0.05, 0.35, 0.65, 0.95, 1.0])
 @pytest.mark.parametrize("text", [0, 256])
 def test_gemm_o_form_chosen_on_the_device(dev, p_active, text):
