@@ -366,7 +366,8 @@ __device__ __forceinline__ int pop_row(const FaParams& p, int xcd, const int* q,
 struct BitRange {
   const uint32_t* words;
   int first, n;
-  __device__ __forceinline__ BitRange(const uint8_t* seg, int64_t bit, int n_) : n(n_) {
+  // (at most 2^20 keep bits: 32-bit positions)
+  __device__ __forceinline__ BitRange(const uint8_t* seg, uint32_t bit, int n_) : n(n_) {
     const uintptr_t a = reinterpret_cast<uintptr_t>(seg) + (bit >> 3);
     words = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
     first = static_cast<int>(a & 3) * 8 + static_cast<int>(bit & 7);
@@ -753,8 +754,8 @@ sparse_fa_kernel(const FaParams p) {
   // first row of the share, candidates to clear; even shares: rows (0: one item at most), shares, cost of all
   // (in LDS and not in registers, where they would live through the main loop)
   __shared__ int s_dir[5];
+  __shared__ int s_list_at;  // whole parts: where the item's keep bits are in LDS (words from smem on), or -1
   __shared__ int s_ends[5];  // a batch of one request: its q and kv tokens, where its keep bits begin
-  constexpr int kCands = kDirectMaxCand / (64 * kWaves);         // candidates of a thread
   // this workgroup's share: neighbouring ones on one XCD
   auto dir_index = [&]() {
     return (gridDim.x & (kXcds - 1)) == 0 ? (blockIdx.x & (kXcds - 1)) * (gridDim.x / kXcds) + blockIdx.x / kXcds
@@ -808,7 +809,7 @@ sparse_fa_kernel(const FaParams p) {
       it.mask_first = 0;
       if (!p.is_full) {
         const BitRange r(p.kv_info + (one ? s_ends[4] : p.kv_info_indptr[it.req]),
-                         (static_cast<int64_t>(it.qb) * p.symbol_heads + h) * it.nkv, it.nkv);
+                         static_cast<uint32_t>(it.qb * p.symbol_heads + h) * it.nkv, it.nkv);
         it.mask = r.words;
         it.mask_first = r.first;
       }
@@ -816,10 +817,22 @@ sparse_fa_kernel(const FaParams p) {
     it.q_scale = 1.f;
     it.k_scale0 = 0;
   };
+  constexpr int kCands = kDirectMaxCand / (64 * kWaves);         // candidates of a thread, at most
   auto direct_schedule = [&]() {
     const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads, dir_g = dir_index();
+    // (No more of them than it takes: the schedule is bound by the instructions of its two wavefronts per SIMD, not by
+    // its trips to memory.  With this, the symbols' copy below off the critical path and a whole part's list made from keep
+    // bits that are at hand: 384 tokens x 2 heads 15.8 -> 15.1 us a call, 13 711 x 226 tokens x 3 heads 14.1 -> 13.5,
+    // 2764 x 3 heads 26.8 -> 26.3.)
+    const int per_thread = part_of(n_cand - 1, 64 * kWaves) + 1;
+    const int first_cand = per_thread * tid;
+    if (tid < kItemBatch) s_items[tid].row = -1;
+    if (tid == 0) s_next_row[0].row = -1;
+    int list_at[kCands];  // where a candidate's keep bits are in LDS (words from smem on), or -1
     bool act[kCands];
     int n[kCands], nkv[kCands];
+    constexpr int kAhead = 3, kOwnWords = 0x10000;  // words that a thread asks for itself
+    uint32_t own[kCands][kAhead];
     {
       // All of a thread's candidates make their trips to memory together.  Where the keep bits are more than two
       // words to a candidate they come as one piece into the tile buffers, which nothing uses yet.  (Candidate
@@ -827,7 +840,11 @@ sparse_fa_kernel(const FaParams p) {
       int req[kCands], bit[kCands];
 #pragma unroll
       for (int u = 0; u < kCands; ++u) {
-        const int cand = min(kCands * tid + u, n_cand - 1);
+        if (u >= per_thread) {
+          req[u] = bit[u] = 0;
+          continue;
+        }
+        const int cand = min(first_cand + u, n_cand - 1);
         const int h = part_of(cand, p.n_blk), t = cand - h * p.n_blk;
         req[u] = p.batch == 1 ? 0 : p.blk_req[t];
         bit[u] = (p.batch == 1 ? t : p.blk_qb[t]) * p.symbol_heads + h;
@@ -841,8 +858,11 @@ sparse_fa_kernel(const FaParams p) {
       }
 #pragma unroll
       for (int u = 0; u < kCands; ++u) {
+        act[u] = false;
+        n[u] = nkv[u] = 0;
+        if (u >= per_thread) continue;
         nkv[u] = (p.kv_indptr[req[u] + 1] - p.kv_indptr[req[u]] + kBlockKV - 1) / kBlockKV;
-        act[u] = kCands * tid + u < n_cand;
+        act[u] = first_cand + u < n_cand;
         n[u] = act[u] ? nkv[u] : 0;
       }
       if (!p.is_full) {
@@ -850,6 +870,8 @@ sparse_fa_kernel(const FaParams p) {
         uint8_t flags[kCands];
 #pragma unroll
         for (int u = 0; u < kCands; ++u) {
+          keep_at[u] = flags[u] = 0;
+          if (u >= per_thread) continue;
           keep_at[u] = p.kv_info_indptr[req[u]];
           flags[u] = p.info[p.info_indptr[req[u]] + (bit[u] >> 3)];
         }
@@ -877,11 +899,12 @@ sparse_fa_kernel(const FaParams p) {
             n[u] = first[u] = 0;
             words[u] = reinterpret_cast<const uint32_t*>(smem);
             if (act[u]) {
-              const int64_t at_bit = static_cast<int64_t>(bit[u]) * nkv[u];
+              list_at[u] = -1;
+              const uint32_t at_bit = static_cast<uint32_t>(bit[u]) * nkv[u];
               // (a caller's segments may lie in any order: one outside of the piece is read where it is)
-              if (keep_at[u] >= map_lo && keep_at[u] + ((at_bit + nkv[u] + 7) >> 3) <= map_hi) {
+              if (keep_at[u] >= map_lo && keep_at[u] + static_cast<int>((at_bit + nkv[u] + 7) >> 3) <= map_hi) {
                 const int byte = skew + keep_at[u] - map_lo + static_cast<int>(at_bit >> 3);
-                words[u] += byte >> 2;
+                words[u] += list_at[u] = byte >> 2;
                 first[u] = (byte & 3) * 8 + static_cast<int>(at_bit & 7);
                 left = max(left, (first[u] + nkv[u] + 31) >> 5);
               } else {
@@ -899,19 +922,28 @@ sparse_fa_kernel(const FaParams p) {
               if (act[u] && i < r.count()) n[u] += __popc(r.trim(words[u][i], i));
             }
         } else {
-          constexpr int kAhead = 3;
           uint32_t v[kCands][kAhead];
 #pragma unroll
           for (int u = 0; u < kCands; ++u) {
-            const BitRange r(p.kv_info + keep_at[u], static_cast<int64_t>(bit[u]) * nkv[u], nkv[u]);
+            if (u >= per_thread) {
+#pragma unroll
+              for (int i = 0; i < kAhead; ++i) v[u][i] = 0u;
+              continue;
+            }
+            const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
 #pragma unroll
             for (int i = 0; i < kAhead; ++i) v[u][i] = i < r.count() && nkv[u] > 0 ? r.words[i] : 0u;
           }
 #pragma unroll
           for (int u = 0; u < kCands; ++u) {
-            const BitRange r(p.kv_info + keep_at[u], static_cast<int64_t>(bit[u]) * nkv[u], nkv[u]);
+            list_at[u] = -1;
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) own[u][i] = v[u][i];
+            if (u >= per_thread) continue;
+            const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
             act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
             n[u] = 0;
+            list_at[u] = r.count() <= kAhead ? kOwnWords : -1;
             if (act[u] && nkv[u] > 0) {
 #pragma unroll
               for (int i = 0; i < kAhead; ++i)
@@ -951,12 +983,12 @@ sparse_fa_kernel(const FaParams p) {
     }
     // q blocks that are not computed are cleared by turns
     if (p.zero_skipped) {
-      int skipped = kCands * tid - row;
+      int skipped = first_cand - row;
 #pragma unroll
       for (int u = 0; u < kCands; ++u)
-        if (kCands * tid + u < n_cand && !act[u]) {
+        if (u < per_thread && first_cand + u < n_cand && !act[u]) {
           const int turn = part_of(skipped, n_wg);
-          if (skipped - turn * n_wg == dir_g) s_zero[turn] = static_cast<uint16_t>(kCands * tid + u);
+          if (skipped - turn * n_wg == dir_g) s_zero[turn] = static_cast<uint16_t>(first_cand + u);
           ++skipped;
         }
       if (tid == 0) s_dir[1] = max(n_cand - rows - dir_g + n_wg - 1, 0) / n_wg;
@@ -998,25 +1030,29 @@ sparse_fa_kernel(const FaParams p) {
       // Whole parts or even shares: whichever has the least on its slowest workgroup.  A share is as good as never
       // made of one piece only: a second prologue, epilogue and exchange are worth kEvenExtra blocks.
       if (longest + (longest < max_n ? kPartExtra : 0) <= total / shares + kEvenExtra) {
-        int parts[kCands], parts_mine = 0;
+        int parts[kCands], first = row;
 #pragma unroll
-        for (int u = 0; u < kCands; ++u) {
-          parts[u] = act[u] ? part_of(max(n[u], 1) - 1, longest) + 1 : 0;
-          parts_mine += parts[u];
+        for (int u = 0; u < kCands; ++u) parts[u] = act[u];
+        if (longest < max_n) {
+          int parts_mine = 0;
+#pragma unroll
+          for (int u = 0; u < kCands; ++u) {
+            parts[u] = act[u] ? part_of(max(n[u], 1) - 1, longest) + 1 : 0;
+            parts_mine += parts[u];
+          }
+          const int parts_incl = wave_scan(parts_mine);
+          if (lane == 63) s_wave[3][wv] = parts_incl;
+          __syncthreads();
+          first = parts_incl - parts_mine;
+#pragma unroll
+          for (int w = 0; w < kWaves; ++w)
+            if (w < wv) first += s_wave[3][w];
         }
-        const int parts_incl = wave_scan(parts_mine);
-        if (lane == 63) s_wave[3][wv] = parts_incl;
-        if (tid < kItemBatch) s_items[tid].row = -1;
-        __syncthreads();
-        int first = parts_incl - parts_mine;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w)
-          if (w < wv) first += s_wave[3][w];
 #pragma unroll
         for (int u = 0; u < kCands; ++u) {
           if (first <= dir_g && dir_g < first + parts[u]) {
             RowInfo it;
-            direct_row(kCands * tid + u, it);
+            direct_row(first_cand + u, it);
             const int per = (n[u] + parts[u] - 1) / parts[u];
             it.part = dir_g - first;
             it.parts = parts[u];
@@ -1026,7 +1062,13 @@ sparse_fa_kernel(const FaParams p) {
             // than n blocks.  Longer than the LDS list, a part is cut, as the other forms cut a row: callers that
             // plan a batch send requests of more than kRowBlocks kv blocks to the decoder)
             it.nb = min(max(min(n[u] - it.ptr0, per), 0), kRowBlocks);
-            s_items[0] = it;
+            s_next_row[0] = it;
+            // its keep bits: in LDS already, or this thread's own
+            s_list_at = p.is_full || list_at[u] == kOwnWords ? 0 : list_at[u];
+            if (!p.is_full && list_at[u] == kOwnWords) {
+#pragma unroll
+              for (int i = 0; i < kAhead; ++i) reinterpret_cast<uint32_t*>(smem)[i] = own[u][i];
+            }
           }
           first += parts[u];
         }
@@ -1039,7 +1081,7 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
     for (int u = 0; u < kCands; ++u)
       if (act[u]) {
-        s_row_cand[row] = static_cast<uint16_t>(kCands * tid + u);
+        s_row_cand[row] = static_cast<uint16_t>(first_cand + u);
         s_row_u[row] = cost + kShareRowCost;
         // first row of the share: the one that holds the share's lower bound
         if (cost <= a && a < cost + kShareRowCost + n[u]) s_dir[0] = row;
@@ -1083,7 +1125,47 @@ sparse_fa_kernel(const FaParams p) {
       s_items[lane] = it;
     }
   };
-  // One wavefront: the next item and its kv block list, from the row's keep bits
+  // One wavefront: the kv block list of the item in s_next_row[slot_idx], from the row's keep bits (words_at: in LDS from
+  // there on, -1: in memory)
+  auto direct_list = [&](int slot_idx, const RowInfo& it, int words_at) __attribute__((always_inline)) {
+    const int lane = fresh_lane();
+    const int lo = __builtin_amdgcn_readfirstlane(it.ptr0), n = __builtin_amdgcn_readfirstlane(it.nb);
+    if (p.is_full) {
+      for (int i = lane; i < n; i += 64) s_blk2[slot_idx][i] = static_cast<uint16_t>(lo + i);
+    } else if constexpr (kDirect) {
+      BitRange r(nullptr, 0, __builtin_amdgcn_readfirstlane(it.nkv));
+      r.first = __builtin_amdgcn_readfirstlane(it.mask_first);
+      // a kv block per lane, its place in the list from the bits below it
+      int seen = -lo;
+      auto keep_bits = [&](int b, uint32_t word) __attribute__((always_inline)) {
+        const bool kept = b < r.n && (word >> ((r.first + b) & 31)) & 1;
+        const uint64_t all = __ballot(kept);
+        const int at_bit = seen + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(all >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(all), 0u)));
+        if (kept && at_bit >= 0 && at_bit < n) s_blk2[slot_idx][at_bit] = static_cast<uint16_t>(b);
+        seen += __popcll(all);
+      };
+      if (words_at >= 0) {
+        const uint32_t* const words = reinterpret_cast<const uint32_t*>(smem) + words_at;
+        for (int b0 = 0; b0 < r.n && seen < n; b0 += 64) keep_bits(b0 + lane, words[(r.first + min(b0 + lane, r.n - 1)) >> 5]);
+      } else {
+        const uint64_t m = reinterpret_cast<uint64_t>(it.mask);
+        r.words = reinterpret_cast<const uint32_t*>(
+            static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m >> 32)))) << 32 |
+            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m))));
+        // four rounds' words requested together
+        for (int b0 = 0; b0 < r.n && seen < n; b0 += 4 * 64) {
+          uint32_t v[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = r.words[(r.first + min(b0 + 64 * j + lane, r.n - 1)) >> 5];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) keep_bits(b0 + 64 * j + lane, v[j]);
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // (see fetch_next)
+  };
+  // One wavefront: the next item and its list
   auto direct_next = [&](int slot_idx) {
     slot_idx = __builtin_amdgcn_readfirstlane(slot_idx);
     const int lane = fresh_lane();
@@ -1094,57 +1176,66 @@ sparse_fa_kernel(const FaParams p) {
       s_next_row[slot_idx] = it;
       s_share[0] = at + 1;
     }
-    if (__builtin_amdgcn_readfirstlane(it.row) >= 0) {
-      const int lo = __builtin_amdgcn_readfirstlane(it.ptr0), n = __builtin_amdgcn_readfirstlane(it.nb);
-      if (p.is_full) {
-        for (int i = lane; i < n; i += 64) s_blk2[slot_idx][i] = static_cast<uint16_t>(lo + i);
-      } else if constexpr (kDirect) {
-        BitRange r(nullptr, 0, __builtin_amdgcn_readfirstlane(it.nkv));
-        r.first = __builtin_amdgcn_readfirstlane(it.mask_first);
-        const uint64_t m = reinterpret_cast<uint64_t>(it.mask);
-        r.words = reinterpret_cast<const uint32_t*>(
-            static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m >> 32)))) << 32 |
-            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m))));
-        // a kv block per lane, its place in the list from the bits below it; four rounds' words requested together
-        int seen = -lo;
-        for (int b0 = 0; b0 < r.n && seen < n; b0 += 4 * 64) {
-          uint32_t v[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = r.words[(r.first + min(b0 + 64 * j + lane, r.n - 1)) >> 5];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int b = b0 + 64 * j + lane;
-            const bool kept = b < r.n && (v[j] >> ((r.first + b) & 31)) & 1;
-            const uint64_t all = __ballot(kept);
-            const int at_bit = seen + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(all >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(all), 0u)));
-            if (kept && at_bit >= 0 && at_bit < n) s_blk2[slot_idx][at_bit] = static_cast<uint16_t>(b);
-            seen += __popcll(all);
-          }
-        }
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // (see fetch_next)
+    if (__builtin_amdgcn_readfirstlane(it.row) >= 0) direct_list(slot_idx, it, -1);
   };
   if constexpr (kDirect) {
-    // (the copy of the symbols for a later decode: requested first, so that it passes beside the scans)
-    if (p.keep_info != nullptr) {
-      const int step = gridDim.x * (64 * kWaves), at = blockIdx.x * (64 * kWaves) + tid;
-      for (int i = at; i < p.kv_info_bytes; i += step) p.keep_kv_info[i] = p.kv_info[i];
-      for (int i = at; i < p.info_bytes; i += step) p.keep_info[i] = p.info[i];
-      for (int i = at; i <= p.batch; i += step) {
-        p.keep_indptr[i] = p.info_indptr[i];
-        p.keep_indptr[p.batch + 1 + i] = p.kv_info_indptr[i];
+    // The copy of the symbols for a later decode: 2 KB or so by each of the last workgroups, asked for in front of the
+    // schedule and stored behind it.  (By all of them, with nothing between load and store, it was 0.6 us that every workgroup
+    // waited; at the launch's end the last ones were 0.3 us late for it.)
+    constexpr int kKeep = 4, kAll = 64 * kWaves;
+    const int back = static_cast<int>(gridDim.x - 1 - blockIdx.x), keep_at = back * kKeep * kAll + tid, keep_ip = back * kAll + tid;
+    const bool keeps = p.keep_info != nullptr && (back * kKeep * kAll < max(p.kv_info_bytes, p.info_bytes) || back * kAll <= p.batch);
+    uint8_t kept_kv[kKeep], kept[kKeep];
+    int32_t kept_ip[2];
+    if (keeps) {
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j) {
+        const int i = keep_at + j * kAll;
+        if (i < p.kv_info_bytes) kept_kv[j] = p.kv_info[i];
+        if (i < p.info_bytes) kept[j] = p.info[i];
+      }
+      if (keep_ip <= p.batch) {
+        kept_ip[0] = p.info_indptr[keep_ip];
+        kept_ip[1] = p.kv_info_indptr[keep_ip];
       }
     }
     // (by the workgroup with the last share, which has the least to do: the first one is 0.4 us late for it, 1 % of
     // a launch of 33 us)
     if (p.keep_indptr != nullptr && blockIdx.x == gridDim.x - 1 && tid == 0) p.sched[kSchedKept] = p.is_full ? 2 : 1;
     direct_schedule();
+    if (keeps) {
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j) {
+        const int i = keep_at + j * kAll;
+        if (i < p.kv_info_bytes) p.keep_kv_info[i] = kept_kv[j];
+        if (i < p.info_bytes) p.keep_info[i] = kept[j];
+      }
+      if (keep_ip <= p.batch) {
+        p.keep_indptr[keep_ip] = kept_ip[0];
+        p.keep_indptr[p.batch + 1 + keep_ip] = kept_ip[1];
+      }
+      // (more than the workgroups take at a time)
+      const int all = static_cast<int>(gridDim.x) * kAll;
+      for (int i = kKeep * all + back * kAll + tid; i < max(p.kv_info_bytes, p.info_bytes); i += all) {
+        if (i < p.kv_info_bytes) p.keep_kv_info[i] = p.kv_info[i];
+        if (i < p.info_bytes) p.keep_info[i] = p.info[i];
+      }
+      for (int i = all + keep_ip; i <= p.batch; i += all) {
+        p.keep_indptr[i] = p.info_indptr[i];
+        p.keep_indptr[p.batch + 1 + i] = p.kv_info_indptr[i];
+      }
+    }
     if (wv == 0) {
       if (lane == 0) s_share[0] = 0;
-      if (__builtin_amdgcn_readfirstlane(s_dir[2]) > 0) direct_items(0);
-      direct_next(0);
+      if (__builtin_amdgcn_readfirstlane(s_dir[2]) > 0) {
+        direct_items(0);
+        direct_next(0);
+      } else {
+        // whole parts: the item is there, and the only one
+        if (lane == 0) s_share[0] = 1;
+        if (__builtin_amdgcn_readfirstlane(s_next_row[0].row) >= 0)
+          direct_list(0, s_next_row[0], __builtin_amdgcn_readfirstlane(s_list_at));
+      }
     }
   }
   if constexpr (!kDirect) {

@@ -71,6 +71,21 @@ def test_rows_from_the_symbols(dev, case, is_full, dtype):
     assert max_abs(listed.cpu(), got) <= 8e-3
 
 
+@pytest.mark.parametrize("case", [
+    ([2048], [300], 32, 0.4),                              # 512 candidates, one per thread
+    ([2048], [300], 33, 0.4),                              # 528, two per thread
+    ([128] + [100] * 40, [26000] + [64] * 40, 2, 0.8),     # a row of 204 keep bits among short ones: read where they are
+    ([640], [12200], 3, 0.8),                              # 96 bits: three words of a thread, or four by their alignment
+    ([2048], [20000], 8, 0.6),                             # kept symbols copied by two workgroups
+    ([1] * 700, [1, 300] * 350, 1, 0.7),                   # offsets of 700 requests, by two workgroups
+])
+@pytest.mark.parametrize("is_full", [False, True])
+def test_schedule_of_short_lists(dev, case, is_full):
+    """The lines inside the schedule of a short list: candidates per thread, where a row's keep bits are found, what a
+    workgroup copies of the symbols that a later decode reads."""
+    test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
+
+
 @pytest.mark.parametrize("group", [2, 7])
 def test_fresh_output_of_packed_tiles(dev, group):
     """Skipped tiles of grouped-query attention: the rows of a tile are spread over the group's q heads."""
