@@ -1780,17 +1780,135 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
   // ---- which strip ----
   const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
   const int cols = p.strip_cols;                 // column groups of XCDs
-  const int xr = xcd / cols, xc = xcd - xr * cols;
-  const int per = p.n_cp / cols;                 // column pairs of an XCD
-  const int rank = xr + (kXcds / cols) * (slot / per);
-  const int cp = xc * per + slot % per;
   const int n_blocks = p.batch * p.n_row_tiles;
-  if (rank >= n_blocks) return;
   auto flag_row_of = [&](int row) -> uint32_t {
     return static_cast<uint32_t>(p.num_text_tokens + row * kTile) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
   };
-  int block = rank;
+  int block, c0, c1;  // token block, column blocks (c1 < 0: only one)
+  if (!kReduce && p.sparse_info != nullptr) {
+    // ---- GEMM-Q with flags: a token block's flagged column blocks two at a time, group of columns by group ----
+    auto group_begin = [&](int g) { return g * p.n_col_tiles / cols; };
+    auto flags_of = [&](int i, uint32_t* row0) -> const uint8_t* {
+      const int b = i / p.n_row_tiles;
+      *row0 = flag_row_of(i - b * p.n_row_tiles);
+      return p.sparse_info + p.sparse_info_indptr[b];
+    };
+    // strips of cells first .. first + 3 (those before `end`): their flags' loads are in flight together
+    constexpr int kTogether = 4;
+    auto strips_of = [&](int first, int end, int (&n)[kTogether]) {
+      const uint8_t* info[kTogether];
+      uint32_t lo[kTogether], hi[kTogether];
+#pragma unroll
+      for (int q = 0; q < kTogether; ++q) {
+        const int cell = min(first + q, end - 1), grp = cell / n_blocks;
+        info[q] = flags_of(cell - grp * n_blocks, &lo[q]);
+        hi[q] = lo[q] + group_begin(grp + 1);
+        lo[q] += group_begin(grp);
+        n[q] = 0;
+      }
+      if (p.head_dim == kTile) {  // (a flag per column block: four bytes of them at a time)
+        for (uint32_t at0 = 0;; at0 += 4) {
+          uint32_t v[kTogether][4];
+          bool more = false;
+#pragma unroll
+          for (int q = 0; q < kTogether; ++q) {
+            const uint32_t last = (hi[q] - 1) >> 3;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[q][u] = info[q][min((lo[q] >> 3) + at0 + u, last)];
+            more |= (lo[q] >> 3) + at0 + 4 <= last;
+          }
+#pragma unroll
+          for (int q = 0; q < kTogether; ++q) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const uint32_t at = (lo[q] >> 3) + at0 + u;
+              if (at == lo[q] >> 3) v[q][u] &= 0xFFu << (lo[q] & 7);
+              if (at == hi[q] >> 3) v[q][u] &= (1u << (hi[q] & 7)) - 1u;
+              if (at <= (hi[q] - 1) >> 3) n[q] += __popc(v[q][u]);
+            }
+          }
+          if (!more) break;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < kTogether; ++q) {
+          const uint32_t c_lo = group_begin(min(first + q, end - 1) / n_blocks), row0 = lo[q] - c_lo;
+          for (uint32_t c = c_lo; c < hi[q] - row0; ++c) n[q] += flag_bit(info[q], row0 + c * kTile / p.head_dim);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kTogether; ++q) n[q] = first + q < end ? (n[q] + 1) >> 1 : 0;
+    };
+    int32_t* const s_tot = reinterpret_cast<int32_t*>(smem);
+    const int n_cells = cols * n_blocks;
+    const int run = (n_cells + kThreads - 1) / kThreads;
+    const int lo = min(tid * run, n_cells), hi = min(lo + run, n_cells);
+    int here = 0, n[kTogether];
+    for (int i = lo; i < hi; i += kTogether) {
+      strips_of(i, hi, n);
+#pragma unroll
+      for (int q = 0; q < kTogether; ++q) here += n[q];
+    }
+    int upto = fo::wave_scan(here);
+    if (lane == 63) s_tot[wv] = upto;
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) {
+      const int t = s_tot[w];
+      if (w < wv) upto += t;
+      total += __builtin_amdgcn_readfirstlane(t);
+    }
+    const int s_lo = static_cast<int>(static_cast<int64_t>(total) * xcd / kXcds);
+    if (s_lo + slot >= static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / kXcds)) return;
+    if (const int mine = s_lo + slot - (upto - here); mine >= 0 && mine < here) {  // (one thread)
+      int skip = mine;
+      for (int i = lo; i < hi; i += kTogether) {
+        if (run > kTogether) strips_of(i, hi, n);  // (else they are at hand)
+#pragma unroll
+        for (int q = 0; q < kTogether; ++q) {
+          if (skip >= 0 && skip < n[q]) {
+            s_tot[8] = i + q;
+            s_tot[9] = skip;
+          }
+          skip -= n[q];
+        }
+      }
+    }
+    __syncthreads();
+    const int cell = __builtin_amdgcn_readfirstlane(s_tot[8]);
+    int skip = 2 * __builtin_amdgcn_readfirstlane(s_tot[9]);
+    __syncthreads();
+    const int grp = cell / n_blocks, c_end = group_begin(grp + 1);
+    block = cell - grp * n_blocks;
+    uint32_t row0;
+    const uint8_t* info = flags_of(block, &row0);
+    c0 = c1 = -1;
+    for (int cw = group_begin(grp); cw < c_end && c1 < 0; cw += 64) {
+      const int c = min(cw + lane, c_end - 1);
+      unsigned long long m = __ballot(cw + lane < c_end && flag_bit(info, row0 + static_cast<uint32_t>(c * kTile) / p.head_dim));
+      if (c0 < 0 && skip >= __popcll(m)) {
+        skip -= __popcll(m);
+        continue;
+      }
+      if (c0 < 0) {
+        for (; skip > 0; --skip) m &= m - 1;
+        c0 = cw + __builtin_ctzll(m);
+        m &= m - 1;
+      }
+      if (m) c1 = cw + __builtin_ctzll(m);
+    }
+  } else {
+    const int xr = xcd / cols, xc = xcd - xr * cols;
+    const int per = p.n_cp / cols;                 // column pairs of an XCD
+    const int cp = xc * per + slot % per;
+    block = xr + (kXcds / cols) * (slot / per);
+    if (block >= n_blocks) return;
+    c0 = 2 * cp;
+    c1 = 2 * cp + 1 < p.n_col_tiles ? 2 * cp + 1 : -1;  // (the last pair may lack its second)
+  }
   if constexpr (kReduce) {
+    const int rank = block;
     if (p.judgement != nullptr && blockIdx.x == 0) judge_flags(p, reinterpret_cast<int32_t*>(smem));
     if (p.strip_sorted) {
       // token blocks with the most selected heads first
@@ -1833,11 +1951,14 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       __syncthreads();
     }
   }
-  const int bz = block / p.n_row_tiles, row = block - bz * p.n_row_tiles;
+  // (a descriptor has to be in scalar registers, and divisions are not)
+  block = __builtin_amdgcn_readfirstlane(block);
+  c0 = __builtin_amdgcn_readfirstlane(c0);
+  c1 = __builtin_amdgcn_readfirstlane(c1);
+  const int bz = __builtin_amdgcn_readfirstlane(block / p.n_row_tiles), row = block - bz * p.n_row_tiles;
   const int m0 = row * kTile;
   const uint32_t flag_row = flag_row_of(row);
 
-  const int c0 = 2 * cp, c1 = 2 * cp + 1 < p.n_col_tiles ? 2 * cp + 1 : -1;  // (the last pair may lack its second)
   // ---- the slabs: heads of this token block (GEMM-O), or all of k ----
   unsigned long long mask[4] = {0, 0, 0, 0};
   int n_iter, iph = 1, word = 0, sub = 0, k0 = 0;
@@ -2232,13 +2353,25 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   // Column groups of XCDs: four, two or one that divide the column pairs and leave each at least three (20 000 x 5120, 60 % of
   // the heads: one group 734 us, two 619, four 574; 33 000 x 3072 dense 514, 499, 500).  Narrower ones are bound by memory, and
   // there a token block should be read by one XCD (60 000 x 512 dense: one group 36.8 us, two 39.4).
-  int cols = 1;
-  while (cols < 4 && gm.n_cp % (2 * cols) == 0 && gm.n_cp >= 6 * cols) cols *= 2;
-  p.strip_cols = cols;
+  // Of flagged units the strips themselves are dealt to the XCDs, an eighth each, group by group; two groups where one would
+  // have more than 32 column blocks (12 000 x 5120, 20 / 50 % flagged: one group 140 / 275 us, two 130 / 267; 16 columns and
+  // fewer lose up to a quarter with two).
+  const bool flagged = !kReduce && p.sparse_info != nullptr;
   const int64_t rows = static_cast<int64_t>(gm.batch) * gm.n_row_tiles;
+  int cols = 1;
+  int64_t grid;
+  if (flagged) {
+    if (gm.n_col_tiles > 32) cols = 2;
+    int64_t per = 0;  // strips of a token block, at most
+    for (int g = 0; g < cols; ++g) per += ((g + 1) * gm.n_col_tiles / cols - g * gm.n_col_tiles / cols + 1) / 2;
+    grid = (rows * per + kXcds - 1) / kXcds * kXcds;
+  } else {
+    while (cols < 4 && gm.n_cp % (2 * cols) == 0 && gm.n_cp >= 6 * cols) cols *= 2;
+    const int rx = kXcds / cols;
+    grid = (rows + rx - 1) / rx * (gm.n_cp / cols) * kXcds;
+  }
+  p.strip_cols = cols;
   p.strip_sorted = rows <= kStripSorted;
-  const int rx = kXcds / cols;
-  const int64_t grid = (rows + rx - 1) / rx * (gm.n_cp / cols) * kXcds;
   gemm_strip_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kStripSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
@@ -2276,7 +2409,12 @@ int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 // GEMM-Q.
 //   * A workgroup per unit while all of them fit the chip at once, two per CU (us, quads -> units: 256 units of K = 2048
 //     46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged).
-//   * With flags: quads, column strips and pairs by the kernel's own list.
+//   * With flags: strips from 4.5 to 32 units per CU (16 beyond 32 column blocks, whose W the strips, which drift apart,
+//     read again and again; six column blocks at least, of which pairs can be made), otherwise quads, column strips and pairs
+//     by the kernel's own list, whose rounds last as long however few units they hold.  Strips over those, 10 .. 95 % flagged:
+//        8 heads, 4.4 to 15 units per CU  0.71 .. 1.18     16, 4.6 to 29  0.65 .. 1.05     24, 5.2 to 30  0.64 .. 1.06
+//       40, 5.6 to 16                     0.66 .. 1.02         to 24      0.71 .. 1.03         to 94      1.0 .. 1.36
+//     (above one where strips begin to share CUs, 257 to 300 of them; 3.4 to 4.4 units per CU 0.84 .. 1.13; 4 heads 1.1 .. 1.2).
 //   * Dense: a quad per CU and round, so it depends on how full the rounds are.  Packed units up to 21 / 32 of them (over
 //     quads 0.75 .. 1.02), in a single round only up to K = 2048 (0.88 .. 1.01; 24 heads 1.05, 40 heads 1.07 .. 1.11).  Strips
 //     up to K = 512 (0.87 .. 0.95 over 2.9 to 23 units per CU) and where two quads' units per CU would be empty in the last
@@ -2290,6 +2428,8 @@ int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace,
   if constexpr (!kQuant) {
     const int64_t units = unit_count(gm);
     if (units <= 2 * num_cu) return launch_units<T, false, kHalf, false>(p, gm, stream);
+    if (use_flags && 2 * units > 9 * num_cu && units <= (gm.n_col_tiles <= 32 ? 32 : 16) * num_cu && gm.n_col_tiles >= 6)
+      return launch_strips<T, false, kHalf, false>(p, gm, stream);
     if (!use_flags) {
       const int64_t slots = quad_slots(gm, num_cu);
       const bool one_round = slots == 4 * num_cu;

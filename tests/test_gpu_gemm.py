@@ -735,6 +735,39 @@ def test_gemm_q_few_flagged_units(dev, shape, flagged, dtype):
         assert rel_l2(out[kept], exp[kept]) <= REL_L2
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [(1, 25000, 768, 64, 6, 0, 0.5), (1, 170000, 768, 96, 6, 0, 0.3), (2, 9050, 2432, 160, 19, 256, 0.6),
+                                  (1, 8100, 2560, 128, 40, 128, 0.5), (1, 19200, 1280, 64, 5, 0, 0.4), (3, 1409, 5248, 96, 41, 0, 0.2),
+                                  (2, 1500, 8960, 64, 70, 0, 0.05), (1, 20000, 1024, 64, 8, 0, 0.0), (1, 20000, 1024, 64, 8, 0, 1.0)])
+def test_gemm_q_flagged_strips(dev, case, dtype):
+    """GEMM-Q with flags of 4.5 to 32 units per CU: strips of one token block x two of its flagged column blocks, which need not
+    be neighbours.  One token block to six (more than are counted together) per thread that counts; one and two groups of columns, of
+    more than 64 columns in all; odd numbers of flagged and of column blocks; heads of 64 columns (a column block reads the
+    flag of its first head) and of 256; a batch, text tokens, ragged last rows, K of 32 mod 64; none and all flagged.  Skipped
+    tiles keep their bytes."""
+    import flashomni_amd as fo
+    batch, m, n, k, heads, text, flagged = case
+    rows = -(-m // 128)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert cus != 256 or 4.5 * cus < batch * rows * (n // 128) <= (32 if n <= 4096 else 16) * cus
+    info, packed, indptr = _flags(batch, (text + m + 127) // 128, heads, flagged, seed=m)
+    x, w, b = _operands(batch, m, n, k, dtype, seed=k)
+    out = sentinel_like((batch, m, n), dtype).to(dev)
+    out0 = out.clone()
+    x, w, b = x.to(dev), w.to(dev), b.to(dev)
+    fo.flashomni_gemm(x, w, heads, torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev), text, b, out=out)
+    tile_head = (np.arange(n // 128) * 128) // (n // heads)
+    kept = torch.from_numpy(info[:, text // 128:][:, :rows, tile_head]).to(dev)
+    half_ulp = 2.0 ** (-9 if dtype == torch.bfloat16 else -11)
+    for i in range(batch):
+        mask = kept[i].repeat_interleave(128, 0)[:m].repeat_interleave(128, 1)
+        assert torch.equal(out[i].view(torch.int16)[~mask], out0[i].view(torch.int16)[~mask])
+        ref = torch.nn.functional.linear(x[i].float(), w.float(), b.float())[mask]
+        got = out[i].float()[mask]
+        # one rounding; sums of k products in another order: k * 2^-24 of the sum of their sizes, below 16 standard deviations of one
+        assert bool(((got - ref).abs() <= 2 * half_ulp * ref.abs() + k * 2.0 ** -24 * 16 * 0.02).all())
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_random_gemm_shapes(dev, seed):
     """Seeded random shapes through GEMM-Q (flags or is_full) and the two passes of GEMM-O (the cached
