@@ -1697,12 +1697,14 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
 // the next one beside a second workgroup, so a slab is multiplied 32 columns at a time, over all of its k, and W lives in
 // a ring of six pieces of 2 x 32 rows (8 KB) of which three to five are on their way; X (16 KB) has two places: 80 KB.
 // Step nt of slab t multiplies piece 4t + nt and reads piece 4t + nt + 1 (and, in its last step, X of slab t + 1, each
-// register as its last MFMA is issued).  Two steps lie between barriers.  Behind the barrier in front of steps 0 and 1:
-// pieces 4t + 5 and 4t + 6 are asked for, into the places of 4t - 1 and 4t, which every wavefront has read by then (of
-// its operand reads only the last four, of X, may be outstanding); in front of steps 2 and 3: pieces 4t + 7 and 4t + 8 and X of slab
-// t + 2.  What a pair of steps reads was asked for at least one pair earlier, so that pair's copies may be outstanding:
-// eight in front of step 0, four in front of step 2.  Copies past the last slab go through empty descriptors (zeros, no
-// memory access).
+// register as its last MFMA is issued).  Two steps lie between barriers.  Behind the barrier in front of steps 0 and 1, when
+// every wavefront has X of slab t and piece 4t in registers: pieces 4t + 5 and 4t + 6, into the places of 4t - 1 and 4t, and
+// then X of slab t + 2 into that of t; in front of steps 2 and 3: pieces 4t + 7 and 4t + 8.  A piece is waited for one pair of
+// steps after the pair that asked for it, X one pair later still, so eight copies may be outstanding at either barrier: X and
+// two pieces behind the pieces that steps 0 and 1 read, two pieces and X behind what steps 2 and 3 do.  (X comes from memory
+// when inputs are new and W from an XCD's L2: asked for half a slab later and waited for at the same barrier, X cost GEMM-Q of
+// 16 384 x 3072 with a tenth flagged 56.9 us in place of 49.5, a full step of 4608 x 3072 503 in place of 494.)
+// Copies past the last slab go through empty descriptors (zeros, no memory access).
 //
 // Order.  XCD x owns column pairs of one group and every so many-th token block (strip_cols, see launch_strips), so that
 // its part of W stays in its L2; token blocks with the most selected heads come first (strip_sorted): the long ones do not end
@@ -2096,11 +2098,11 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
 #pragma unroll
         for (int i = 0; i < 2; ++i) copy_w(rw, q, i, sa.k, q * kStripPiece);
 #pragma unroll
+      for (int i = 0; i < 4; ++i) copy_x(rx1, i, sb.k, kUnitBytes);
+#pragma unroll
       for (int i = 0; i < 2; ++i) copy_w(rw, 3, i, sa.k, 3 * kStripPiece);
 #pragma unroll
       for (int i = 0; i < 2; ++i) copy_w(rw1, 0, i, sb.k, 4 * kStripPiece);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) copy_x(rx1, i, sb.k, kUnitBytes);
     }
     __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
     __builtin_amdgcn_s_barrier();
@@ -2145,21 +2147,22 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
               read_x(1, ks, xbuf ^ kUnitBytes);
             }
           }
-          if constexpr (nt < 2) {
-            if (j == 2 || j == 5) copy_w(rw1, nt + 1, j == 5, sb.k, place(5 + nt));
+          if constexpr (nt == 0) {
+            if (j & 1) copy_w(rw1, 1 + (j >> 2), (j >> 1) & 1, sb.k, place(5 + (j >> 2)));
+          } else if constexpr (nt == 1) {
+            if (j & 1) copy_x(rx2, j >> 1, sc.k, xbuf);
           } else {
-            if (j == 1 || j == 3) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, j == 3, nt == 2 ? sb.k : sc.k, place(5 + nt));
-            if (j == 5 || j == 7) copy_x(rx2, 2 * (nt - 2) + (j == 7), sc.k, xbuf);
+            if (j == 2 || j == 5) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, j == 5, nt == 2 ? sb.k : sc.k, place(5 + nt));
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       };
       __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
-      __builtin_amdgcn_s_waitcnt(0xc47f);      // lgkmcnt(4)
+      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
       step(std::integral_constant<int, 0>{});
       step(std::integral_constant<int, 1>{});
-      __builtin_amdgcn_s_waitcnt(0x0f70 | 4);  // vmcnt(4)
+      __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
       __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
       step(std::integral_constant<int, 2>{});
