@@ -58,6 +58,7 @@ SIGNATURES = {
     "fo_quant_fp8_block": ([c_vp, c_int, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32,
                             c_vp], c_int),
     "fo_symbols_from_scores": ([c_vp, c_int] + [c_i32] * 6 + [c_vp] * 7, c_int),
+    "fo_symbols_from_scores_uniform": ([c_vp, c_int] + [c_i32] * 6 + [c_vp, c_f32] * 2 + [c_vp] * 5, c_int),
 }
 
 # Entry points whose several launches hand something on in scratch memory that belongs to a stream (GEMM-Q's list,

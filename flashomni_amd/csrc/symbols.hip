@@ -21,9 +21,10 @@
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
 constexpr int kRowsPerGroup = 8;
+constexpr unsigned kShortLaunch = 512;  // workgroups; from two per CU on the vector ALUs are busy throughout
 constexpr int kMaxBlocks = 4096;
 constexpr float kFixedOne = 1073741824.0f;  // 2^30
 
@@ -80,7 +81,7 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 // whether entry (e * 64 + lane) gets symbol 0.  `threshold` is the admitted cumulative probability.
 template <int E>
 __device__ __forceinline__ void select_low_mass(const float (&score)[E], int n, float threshold,
-                                                int lane, bool (&drop)[E]) {
+                                                int lane, bool short_launch, bool (&drop)[E]) {
   uint32_t key[E], w[E];
   float m = -INFINITY;
 #pragma unroll
@@ -102,17 +103,33 @@ __device__ __forceinline__ void select_low_mass(const float (&score)[E], int n, 
   const float t = fminf(fmaxf(threshold, 0.f), 1.5f);
   const uint32_t budget = static_cast<uint32_t>(t * kFixedOne);
 
-  // largest bound x with  sum{ w : key < x } <= budget
+  // largest bound x with  sum{ w : key < x } <= budget.  Rows of few entries per lane wait for one sum after the other: where
+  // few rows run beside each other they try three candidates, two bits of x, at a time (24 heads of 36 x 36 blocks 9.4 -> 8.8 us;
+  // 80 of 300 x 65, whose vector ALUs are busy, would take 42 in place of 35).
   uint32_t x = 0, below = 0;
-  for (int bit = 31; bit >= 0; --bit) {
-    const uint32_t c = x | (1u << bit);
+  auto mass_below = [&](uint32_t c) __attribute__((always_inline)) {
     uint32_t part = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) part += key[e] < c ? w[e] : 0u;
-    const uint32_t g = wave_sum_u32(part);
-    if (g <= budget) {
-      x = c;
-      below = g;
+    return wave_sum_u32(part);
+  };
+  if (E <= 4 && short_launch) {
+    for (int bit = 30; bit >= 0; bit -= 2) {
+      const uint32_t c1 = x | (1u << bit), c2 = x | (2u << bit), c3 = x | (3u << bit);
+      const uint32_t g1 = mass_below(c1), g2 = mass_below(c2), g3 = mass_below(c3);
+      if (g1 <= budget) {  // (g1 <= g2 <= g3)
+        x = g3 <= budget ? c3 : g2 <= budget ? c2 : c1;
+        below = g3 <= budget ? g3 : g2 <= budget ? g2 : g1;
+      }
+    }
+  } else {
+    for (int bit = 31; bit >= 0; --bit) {
+      const uint32_t c = x | (1u << bit);
+      const uint32_t g = mass_below(c);
+      if (g <= budget) {
+        x = c;
+        below = g;
+      }
     }
   }
   // entries whose key equals x straddle the cut: admit them in index order while they fit
@@ -136,8 +153,9 @@ __device__ __forceinline__ void select_low_mass(const float (&score)[E], int n, 
 
 struct ProducerArgs {
   const void* scores;           // [batch, H, NQ, NK]
-  const float* q_threshold;     // [batch]
-  const float* kv_threshold;    // [H]
+  const float* q_threshold;     // [batch], or null: q_value for every request
+  const float* kv_threshold;    // [H], or null: kv_value for every head
+  float q_value, kv_value;
   uint8_t* sparse_info;         // batch * ceil(NQ*H / 8) bytes
   uint8_t* sparse_kv_info;      // batch * ceil(NQ*H*NK / 8) bytes
   int32_t* sparse_info_indptr;     // [batch + 1] byte offsets (written)
@@ -152,8 +170,10 @@ __device__ __forceinline__ uint8_t gather8(uint64_t flags) {
 
 // ---- q symbols: one workgroup per request --------------------------------------------------------
 // The H * n_text_q contributing rows are split into `parts` interleaved subsets; a wavefront sums
-// one subset over one 64-column chunk (coalesced 256 B loads, eight in flight), and the partial sums
-// are added in subset order, so the result does not depend on which wavefront did what.
+// one subset over one 64-column chunk (coalesced 256 B loads), two such items at a time with eight
+// rows of each in flight, and the partial sums are added in subset order, so the result does not
+// depend on which wavefront did what.  (What bounds this job is trips to memory: with a trip per row, and four items one after
+// the other on each of four wavefronts, 36 x 36 blocks of 24 heads took the launch 14.7 us.)
 // LDS (carved from the launch's dynamic block): partial sums [parts][width], sums [width], keep
 // flags [n_q + 8].
 struct QJobLayout {
@@ -178,38 +198,63 @@ __device__ __forceinline__ void q_symbols_job(const ProducerArgs& a, int b, uint
   float* s_part = reinterpret_cast<float*>(lds);
   float* s_sum = s_part + parts * width;
   uint8_t* s_keep = reinterpret_cast<uint8_t*>(s_sum + width);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_img = a.n_k - a.text_kv;
   const int chunks = (n_img + 63) >> 6;
   const int n_rows = a.heads * a.text_q;
   const T* base = static_cast<const T*>(a.scores) + static_cast<int64_t>(b) * a.heads * a.n_q * a.n_k;
-  constexpr int kFlight = 8;
-  for (int item = wave; item < chunks * parts; item += kWaves) {
-    const int c = item / parts, part = item - c * parts;
-    const int j = c * 64 + lane;
-    float acc[kFlight];
+  constexpr int kFlight = 8, kItems = 2;
+  const int n_items = chunks * parts;
+  // one subset's rows lie `parts` apart; row = head * n_text_q + q
+  const int step_h = a.text_q ? parts / a.text_q : 0, step_q = a.text_q ? parts % a.text_q : 0;
+  for (int item0 = wave; item0 < n_items; item0 += kWaves * kItems) {
+    float acc[kItems][kFlight];
+    const T* col[kItems];
+    int rows[kItems], h[kItems], q[kItems];
+    int most = 0;
 #pragma unroll
-    for (int u = 0; u < kFlight; ++u) acc[u] = 0.f;
-    if (j < n_img) {
-      const T* col = base + a.text_kv + j;
-      int r = part;
-      for (; r + (kFlight - 1) * parts < n_rows; r += kFlight * parts) {
+    for (int t = 0; t < kItems; ++t) {
+      const int item = min(item0 + t * kWaves, n_items - 1), c = item / parts, part = item - c * parts;
+      col[t] = base + a.text_kv + min(c * 64 + lane, n_img - 1);
+      rows[t] = part < n_rows ? (n_rows - part + parts - 1) / parts : 0;
+      h[t] = rows[t] ? part / a.text_q : 0;
+      q[t] = rows[t] ? part - h[t] * a.text_q : 0;
+      most = max(most, rows[t]);
+#pragma unroll
+      for (int u = 0; u < kFlight; ++u) acc[t][u] = 0.f;
+    }
+    for (int i = 0; i < most; i += kFlight) {
+      float v[kItems][kFlight];
+#pragma unroll
+      for (int t = 0; t < kItems; ++t)
 #pragma unroll
         for (int u = 0; u < kFlight; ++u) {
-          const int row = r + u * parts;             // row = head * n_text_q + q
-          const int h = row / a.text_q, q = row - h * a.text_q;
-          acc[u] += to_f32(col[(static_cast<int64_t>(h) * a.n_q + q) * a.n_k]);
+          v[t][u] = i + u < rows[t] ? to_f32(col[t][(static_cast<int64_t>(h[t]) * a.n_q + q[t]) * a.n_k]) : 0.f;
+          h[t] += step_h;
+          q[t] += step_q;
+          if (q[t] >= a.text_q) {
+            q[t] -= a.text_q;
+            ++h[t];
+          }
+        }
+#pragma unroll
+      for (int t = 0; t < kItems; ++t) {
+        const bool whole = i + kFlight <= rows[t];  // (what is left of a subset is added to the first sum, row by row)
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) {
+          if (whole) acc[t][u] += v[t][u]; else acc[t][0] += v[t][u];
         }
       }
-      for (; r < n_rows; r += parts) {
-        const int h = r / a.text_q, q = r - h * a.text_q;
-        acc[0] += to_f32(col[(static_cast<int64_t>(h) * a.n_q + q) * a.n_k]);
-      }
     }
-    float total = 0.f;
 #pragma unroll
-    for (int u = 0; u < kFlight; ++u) total += acc[u];
-    s_part[part * width + j] = total;
+    for (int t = 0; t < kItems; ++t) {
+      const int item = item0 + t * kWaves, c = item / parts, part = item - c * parts;
+      if (item >= n_items) break;
+      float total = 0.f;
+#pragma unroll
+      for (int u = 0; u < kFlight; ++u) total += acc[t][u];
+      s_part[part * width + c * 64 + lane] = total;
+    }
   }
   for (int q = tid; q < a.n_q + 8; q += kThreads) s_keep[q] = q < a.n_q ? 1 : 0;
   __syncthreads();
@@ -224,7 +269,7 @@ __device__ __forceinline__ void q_symbols_job(const ProducerArgs& a, int b, uint
     bool drop[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) score[e] = e * 64 + lane < n_img ? s_sum[e * 64 + lane] : 0.f;
-    select_low_mass<E>(score, n_img, a.q_threshold[b], lane, drop);
+    select_low_mass<E>(score, n_img, a.q_threshold ? a.q_threshold[b] : a.q_value, lane, true, drop);
 #pragma unroll
     for (int e = 0; e < E; ++e)
       if (e * 64 + lane < n_img && drop[e]) s_keep[a.text_q + e * 64 + lane] = 0;
@@ -259,6 +304,7 @@ __global__ void __launch_bounds__(kThreads) symbols_kernel(ProducerArgs a, int g
     return;
   }
   const int block = blockIdx.x - a.batch;
+  const bool short_launch = gridDim.x <= kShortLaunch;
   const int b = block / groups_per_request;
   const int g = block - b * groups_per_request;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -282,7 +328,7 @@ __global__ void __launch_bounds__(kThreads) symbols_kernel(ProducerArgs a, int g
     bool drop[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) score[e] = e * 64 + lane < a.n_k ? to_f32(src[e * 64 + lane]) : 0.f;
-    select_low_mass<E>(score, a.n_k, a.kv_threshold[h], lane, drop);
+    select_low_mass<E>(score, a.n_k, a.kv_threshold ? a.kv_threshold[h] : a.kv_value, lane, short_launch, drop);
 #pragma unroll
     for (int e = 0; e < E; ++e)
       if (e * 64 + lane < a.n_k) flags[e * 64 + lane] = drop[e] ? 0 : 1;
@@ -328,12 +374,11 @@ int dispatch_slots(const ProducerArgs& a, int need, hipStream_t stream) {
 
 }  // namespace
 
-extern "C" int fo_symbols_from_scores(const void* scores, int dtype, int32_t batch, int32_t num_heads,
-                                      int32_t n_q_blocks, int32_t n_kv_blocks, int32_t n_text_q,
-                                      int32_t n_text_kv, const float* q_threshold,
-                                      const float* kv_threshold, uint8_t* sparse_info,
-                                      int32_t* sparse_info_indptr, uint8_t* sparse_kv_info,
-                                      int32_t* sparse_kv_info_indptr, void* stream) {
+namespace {
+int symbols_impl(const void* scores, int dtype, int32_t batch, int32_t num_heads, int32_t n_q_blocks, int32_t n_kv_blocks,
+                 int32_t n_text_q, int32_t n_text_kv, const float* q_threshold, float q_value, const float* kv_threshold,
+                 float kv_value, uint8_t* sparse_info, int32_t* sparse_info_indptr, uint8_t* sparse_kv_info,
+                 int32_t* sparse_kv_info_indptr, void* stream) {
   FO_REQUIRE(dtype == FO_F32 || dtype == FO_BF16 || dtype == FO_F16,
              "symbols_from_scores: scores must be float32, bfloat16 or float16");
   FO_REQUIRE(batch >= 0 && num_heads > 0 && n_q_blocks > 0 && n_kv_blocks > 0,
@@ -353,14 +398,35 @@ extern "C" int fo_symbols_from_scores(const void* scores, int dtype, int32_t bat
   FO_REQUIRE(kv_bytes * (batch > 0 ? batch : 1) <= INT32_MAX,
              "symbols_from_scores: packed sparse_kv_info exceeds int32 byte offsets");
   if (batch == 0) return FO_OK;
-  FO_REQUIRE(scores && q_threshold && kv_threshold && sparse_info && sparse_info_indptr &&
-                 sparse_kv_info && sparse_kv_info_indptr,
+  FO_REQUIRE(scores && sparse_info && sparse_info_indptr && sparse_kv_info && sparse_kv_info_indptr,
              "symbols_from_scores: null pointer");
-  ProducerArgs a{scores, q_threshold, kv_threshold, sparse_info, sparse_kv_info, sparse_info_indptr,
+  ProducerArgs a{scores, q_threshold, kv_threshold, q_value, kv_value, sparse_info, sparse_kv_info, sparse_info_indptr,
                  sparse_kv_info_indptr, batch, num_heads, n_q_blocks, n_kv_blocks, n_text_q, n_text_kv};
   const int need = (n_kv_blocks + 63) / 64;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == FO_F32) return dispatch_slots<float>(a, need, s);
   if (dtype == FO_BF16) return dispatch_slots<__hip_bfloat16>(a, need, s);
   return dispatch_slots<__half>(a, need, s);
+}
+}  // namespace
+
+extern "C" int fo_symbols_from_scores(const void* scores, int dtype, int32_t batch, int32_t num_heads,
+                                      int32_t n_q_blocks, int32_t n_kv_blocks, int32_t n_text_q,
+                                      int32_t n_text_kv, const float* q_threshold,
+                                      const float* kv_threshold, uint8_t* sparse_info,
+                                      int32_t* sparse_info_indptr, uint8_t* sparse_kv_info,
+                                      int32_t* sparse_kv_info_indptr, void* stream) {
+  FO_REQUIRE(batch <= 0 || (q_threshold && kv_threshold), "symbols_from_scores: null pointer");
+  return symbols_impl(scores, dtype, batch, num_heads, n_q_blocks, n_kv_blocks, n_text_q, n_text_kv, q_threshold, 0.f,
+                      kv_threshold, 0.f, sparse_info, sparse_info_indptr, sparse_kv_info, sparse_kv_info_indptr, stream);
+}
+
+extern "C" int fo_symbols_from_scores_uniform(const void* scores, int dtype, int32_t batch, int32_t num_heads,
+                                              int32_t n_q_blocks, int32_t n_kv_blocks, int32_t n_text_q,
+                                              int32_t n_text_kv, const float* q_threshold, float q_value,
+                                              const float* kv_threshold, float kv_value, uint8_t* sparse_info,
+                                              int32_t* sparse_info_indptr, uint8_t* sparse_kv_info,
+                                              int32_t* sparse_kv_info_indptr, void* stream) {
+  return symbols_impl(scores, dtype, batch, num_heads, n_q_blocks, n_kv_blocks, n_text_q, n_text_kv, q_threshold, q_value,
+                      kv_threshold, kv_value, sparse_info, sparse_info_indptr, sparse_kv_info, sparse_kv_info_indptr, stream);
 }

@@ -5,6 +5,7 @@ cumsum and searchsorted, then Triton kernels that clear the selected entries of 
 benchmark/test_flashomni_attention.py:254-257 transposes and packs).  Here one HIP launch goes
 from the scores to the packed bits.
 """
+import math
 from typing import Optional, Tuple, Union
 
 import torch
@@ -13,13 +14,17 @@ from . import _lib
 from .utils import _require_gpu_tensor
 
 
-def _threshold_vector(value, count: int, device, name: str) -> torch.Tensor:
+def _threshold(value, count: int, device, name: str):
+    """(vector, 0) of a tensor, (None, value) of one threshold for all."""
     if isinstance(value, torch.Tensor):
         t = value.to(device=device, dtype=torch.float32).reshape(-1).contiguous()
         if t.numel() != count:
             raise ValueError("%s must have %d entries, got %d" % (name, count, t.numel()))
-        return t
-    return torch.full((count,), float(value), dtype=torch.float32, device=device)
+        return t, 0.0
+    value = float(value)
+    if math.isfinite(value) and abs(value) > torch.finfo(torch.float32).max:
+        raise RuntimeError("%s = %g cannot be represented in float32" % (name, value))
+    return None, value
 
 
 def sparse_symbols_from_scores(
@@ -50,8 +55,8 @@ def sparse_symbols_from_scores(
     t2t = int(num_text_q_blocks)
     t2t_kv = t2t if num_text_kv_blocks is None else int(num_text_kv_blocks)
     dev = scores.device
-    q_thr = _threshold_vector(q_threshold, B, dev, "q_threshold")
-    kv_thr = _threshold_vector(kv_threshold, H, dev, "kv_threshold")
+    q_thr, q_value = _threshold(q_threshold, B, dev, "q_threshold")
+    kv_thr, kv_value = _threshold(kv_threshold, H, dev, "kv_threshold")
     info_bytes = (NQ * H + 7) // 8
     kv_bytes = (NQ * H * NK + 7) // 8
     sparse_info = torch.empty(B * info_bytes, dtype=torch.uint8, device=dev)
@@ -59,8 +64,8 @@ def sparse_symbols_from_scores(
     info_indptr = torch.empty(B + 1, dtype=torch.int32, device=dev)
     kv_indptr = torch.empty(B + 1, dtype=torch.int32, device=dev)
     with _lib.device_guard(dev):
-        _lib.check(_lib.lib().fo_symbols_from_scores(
+        _lib.check(_lib.lib().fo_symbols_from_scores_uniform(
             _lib.ptr(scores), _lib.dtype_code(scores.dtype), B, H, NQ, NK, t2t, t2t_kv,
-            _lib.ptr(q_thr), _lib.ptr(kv_thr), _lib.ptr(sparse_info), _lib.ptr(info_indptr),
+            _lib.ptr(q_thr), q_value, _lib.ptr(kv_thr), kv_value, _lib.ptr(sparse_info), _lib.ptr(info_indptr),
             _lib.ptr(sparse_kv_info), _lib.ptr(kv_indptr), _lib.current_stream(dev)))
     return sparse_info, info_indptr, sparse_kv_info, kv_indptr

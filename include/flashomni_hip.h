@@ -463,6 +463,13 @@ int fo_symbols_from_scores(const void* scores, int dtype, int32_t batch, int32_t
                            int32_t n_text_kv, const float* q_threshold, const float* kv_threshold,
                            uint8_t* sparse_info, int32_t* sparse_info_indptr,
                            uint8_t* sparse_kv_info, int32_t* sparse_kv_info_indptr, void* stream);
+/* The same with one threshold for all requests (q_threshold null: q_value) or all heads (kv_threshold null: kv_value). */
+int fo_symbols_from_scores_uniform(const void* scores, int dtype, int32_t batch, int32_t num_heads,
+                                   int32_t n_q_blocks, int32_t n_kv_blocks, int32_t n_text_q,
+                                   int32_t n_text_kv, const float* q_threshold, float q_value,
+                                   const float* kv_threshold, float kv_value, uint8_t* sparse_info,
+                                   int32_t* sparse_info_indptr, uint8_t* sparse_kv_info,
+                                   int32_t* sparse_kv_info_indptr, void* stream);
 
 #ifdef __cplusplus
 }

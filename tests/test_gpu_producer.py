@@ -133,6 +133,28 @@ def test_no_text_blocks(dev):
     np.testing.assert_array_equal(got_kv, exp_kv)
 
 
+@pytest.mark.parametrize("shape", [(1, 24, 36, 36, 4), (2, 3, 9, 9, 1), (1, 40, 70, 66, 3), (1, 7, 130, 130, 5), (3, 2, 260, 260, 2)])
+def test_one_threshold_for_all(dev, shape):
+    """A float stands for a vector of it, byte for byte, each threshold by itself; text rows of fewer than eight, of several
+    and of a ragged number of rows per partial sum.  The summed score of the q symbols: the fp64 sum decides them wherever it
+    is not within 1e-5 of the cut."""
+    import flashomni_amd as fo
+    B, H, NQ, NK, t2t = shape
+    pooled = torch.randn(B, H, NQ, NK, generator=torch.Generator().manual_seed(NQ), dtype=torch.float32)
+    x = pooled.to(dev)
+    q, kv = torch.full((B,), 0.2, device=dev), torch.full((H,), 0.3, device=dev)
+    expect = fo.sparse_symbols_from_scores(x, t2t, q, kv)
+    for args in ((0.2, 0.3), (0.2, kv), (q, 0.3)):
+        for got, want in zip(fo.sparse_symbols_from_scores(x, t2t, *args), expect):
+            assert torch.equal(got, want)
+    got_q, _ = _unpack(expect, B, H, NQ, NK)
+    sums = pooled[:, :, :t2t, t2t:].double().sum(dim=(1, 2)).float().numpy()
+    exp_q = producer.q_symbols(pooled.numpy(), t2t, t2t, np.full(B, 0.2, dtype=np.float32))
+    _check_rows(sums, np.full(B, 0.2, dtype=np.float32), got_q[:, 0, t2t:t2t + NK - t2t] == 0, exp_q[:, 0, t2t:t2t + NK - t2t] == 0)
+    with pytest.raises(RuntimeError):
+        fo.sparse_symbols_from_scores(x, t2t, 1e60, 0.3)
+
+
 def test_symbols_feed_the_decoder(dev):
     """The packed output is what run()/decode() read: decoding it lists the kept blocks."""
     import flashomni_amd as fo
