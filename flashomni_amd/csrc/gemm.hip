@@ -87,6 +87,8 @@ constexpr int kStageBytes = 4 * kUnitBytes;        // X0, X1, W0, W1
 constexpr int kStages = 2;
 constexpr int kSmemBytes = kStages * kStageBytes;  // 128 KB
 constexpr int kUnitSmemBytes = kStages * 2 * kUnitBytes;  // workgroup per unit: 64 KB, two workgroups per CU
+constexpr int kDeepCopiers = 8, kDeepThreads = 256 + 64 * kDeepCopiers, kDeepRing = 5;  // ... one per CU: four wavefronts compute, eight copy
+constexpr int kDeepSmemBytes = kDeepRing * 2 * kUnitBytes;  // 160 KB
 constexpr int kUnitWindow = 8;  // ... token blocks per scheduling window
 constexpr int kZeroFirst = 1 << 18, kZeroSecond = 1 << 19;  // slab entry: half of the slab does not count
 constexpr int kMaxHeads = 256;
@@ -129,7 +131,7 @@ struct GemmParams {
                          // quads are enumerated arithmetically (GEMM-O, GEMM-Q with is_full)
   const int32_t* qoff;   // qoff[0..8] queue boundaries inside `quads`
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
-  int32_t strip_cols;    // strips: column groups of XCDs
+  int32_t strip_cols;    // strips: column groups of XCDs; 0: an eighth of the strips each
   int32_t strip_sorted;  // strips: token blocks with the most selected heads first
   int32_t* judgement;    // strips: where judge_flags leaves its word, or null
   int32_t judge_first, judge_bytes, judge_limit;
@@ -1120,6 +1122,179 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   }
 }
 
+// The slabs of a token block in the order of k: the selected heads' slices (GEMM-O), or all of k.  kHalf (heads or K of 32
+// mod 64): the last slab of a slice reaches 32 back, where the matrix begins, forward, and counts for one half.
+struct Slab {
+  uint32_t k;              // offset in bytes
+  uint32_t first, second;  // masks of its halves
+};
+template <bool kReduce, bool kHalf>
+struct SlabWalk {
+  unsigned long long mask[4] = {0, 0, 0, 0};  // selected heads that are still to come
+  int n_iter, iph = 1, word = 0, sub = 0, k0 = 0;
+
+  __device__ __forceinline__ void begin(const GemmParams& p, int bz, uint32_t flag_row, int lane) {
+    if constexpr (kReduce) {
+      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+      const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
+      const int n_slices = p.k / p.head_dim;
+      bool sel[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sel[i] = 64 * i + lane < n_slices && flag_bit(info, flag_row + 64 * i + lane) == pick;
+      int count = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        mask[i] = __ballot(sel[i]);
+        count += __popcll(mask[i]);
+      }
+      iph = (p.head_dim + kBK - 1) / kBK;
+      n_iter = count * iph;
+    } else {
+      n_iter = (p.k + kBK - 1) / kBK;
+    }
+  }
+
+  __device__ __forceinline__ Slab next(const GemmParams& p) {
+    Slab s{0, ~0u, ~0u};
+    if constexpr (kReduce) {
+      if (sub == 0) {
+        unsigned long long m = mask[0];
+#pragma unroll
+        for (int i = 1; i < 4; ++i) {
+          if (m == 0 && word < i) {
+            word = i;
+            mask[0] = m = mask[i];
+          }
+        }
+        k0 = (64 * word + __builtin_ctzll(m | (1ull << 63))) * p.head_dim;
+        mask[0] = m & (m - 1);
+      } else {
+        k0 += kBK;
+      }
+      if (++sub == iph) sub = 0;
+      s.k = static_cast<uint32_t>(k0) * 2u;
+      if constexpr (kHalf) {
+        if (sub == 0) {
+          if (k0 >= 32) s.k -= 64u;
+          (k0 >= 32 ? s.first : s.second) = 0u;
+        }
+      }
+    } else {
+      s.k = static_cast<uint32_t>(k0) * 2u;
+      k0 += kBK;
+      if constexpr (kHalf) {
+        if (k0 > p.k) {
+          s.k -= 64u;
+          s.first = 0u;
+        }
+      }
+    }
+    return s;
+  }
+};
+
+// Epilogue of a workgroup per unit: each wavefront turns its 64 x 64 block through 16 KB of its own (by then free) LDS in fp32,
+// into a layout in which 16 consecutive lanes cover a row; bias or partial is added there, the result
+// rounded once.  Output and partial go through descriptors that end with the matrix.
+template <typename T, bool kReduce, bool kPartial>
+__device__ __forceinline__ void unit_epilogue(const GemmParams& p, uint8_t* region, const f32x16 (&acc)[2][2], int bz, int m0,
+                                              int n0, int wr, int wc, int lane) {
+  using x4 = typename Types<T>::x4;
+  constexpr int NT = 2, MT = 2;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int rows_here = min(p.m - m0, kTile);
+  const int col4 = lane & 15, rsub = lane >> 4;
+  const int el_off = n0 + wc * 64 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 4*i
+  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
+  auto out_rsrc = [&](const void* base, int elem_bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
+        rows_here * p.n * elem_bytes, 0x00020000);
+  };
+  auto turn = [&](auto bias_tag, auto f32_tag) {
+    using BiasT = decltype(bias_tag);
+    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
+    constexpr bool kOutF32 = decltype(f32_tag)::value;
+    constexpr int kBytes = sizeof(BiasT);
+    BiasVec bm[16];
+    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (kPartial) {
+      // sixteen pieces in flight together while the rows turn through LDS
+      const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if constexpr (kBytes == 4) {
+          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, 4 * i * p.n * 4, 0));
+        } else {
+          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, 4 * i * p.n * 2, 0));
+        }
+      }
+    } else if (p.bias_kind == FO_BIAS_VECTOR) {
+      const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + wc * 64 + col4 * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+    }
+    // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 256 bytes = 16 chunks)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          f32x4 v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = acc[nt][mt][i4 * 4 + j];
+          const int chunk = nt * 8 + i4 * 2 + g;
+          *reinterpret_cast<f32x4*>(region + (mt * 32 + l32) * 256 + ((chunk ^ (l32 & 15)) << 4)) = v;
+        }
+    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
+    f32x4 vals[8];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if ((i & 7) == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int rk = (i + k) * 4 + rsub;
+          vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 256 + ((col4 ^ (rk & 15)) << 4));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      f32x4 v = vals[i & 7];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (kPartial) {
+          v[j] += static_cast<float>(bm[i][j]);
+        } else {
+          v[j] += bvec[j];
+        }
+      }
+      if constexpr (kOutF32) {
+        // (no scalar offset: see the quads' store)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + 4 * i * p.n) * 4, 0, 2);
+      } else {
+        x4 out;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+        typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, 4 * i * p.n * 2, 2);
+      }
+    }
+  };
+  using std::false_type;
+  using std::true_type;
+  if constexpr (!kReduce) {
+    turn(T{}, false_type{});
+  } else if constexpr (kPartial) {
+    if (p.bias_f32) {
+      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
+    } else {
+      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+    }
+  } else {
+    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Short launches: a workgroup per unit.  Quads keep a CU busy with one work item of four units for
 // its whole k range, so a launch lasts whole rounds of quads however few units are in them: nine
@@ -1336,100 +1511,210 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_unit_kernel(const GemmParams
   __builtin_amdgcn_s_waitcnt(0xc07f);
   __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring
 
-  // ---- epilogue: each wavefront turns its 64 x 64 block through its quarter of the ring in fp32, into
-  // a layout in which 16 consecutive lanes cover a row; bias or partial is added there, the result
-  // rounded once.  Output and partial go through descriptors that end with the matrix. ----
-  uint8_t* const region = smem + wv * (kUnitSmemBytes / 4);
-  const int col4 = lane & 15, rsub = lane >> 4;
-  const int el_off = n0 + wc * 64 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 4*i
-  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
-  auto out_rsrc = [&](const void* base, int elem_bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
-        rows_here * p.n * elem_bytes, 0x00020000);
-  };
-  auto turn = [&](auto bias_tag, auto f32_tag) {
-    using BiasT = decltype(bias_tag);
-    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
-    constexpr bool kOutF32 = decltype(f32_tag)::value;
-    constexpr int kBytes = sizeof(BiasT);
-    BiasVec bm[16];
-    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (kPartial) {
-      // sixteen pieces in flight together while the rows turn through LDS
-      const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        if constexpr (kBytes == 4) {
-          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, 4 * i * p.n * 4, 0));
-        } else {
-          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, 4 * i * p.n * 2, 0));
-        }
-      }
-    } else if (p.bias_kind == FO_BIAS_VECTOR) {
-      const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + wc * 64 + col4 * 4);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+  unit_epilogue<T, kReduce, kPartial>(p, smem + wv * (kUnitSmemBytes / 4), acc, bz, m0, n0, wr, wc, lane);
+}
+
+// ---------------------------------------------------------------------------------------------
+// At most a unit per CU.  Nothing but the depth of a unit's own pipeline hides its trips to L2 and memory then (staged through
+// registers a slab ahead, as above, a slab takes ~1050 cycles even on 84 of 256 CUs, 512 of them matrix core).  So a
+// workgroup has the whole CU: four wavefronts compute 64 x 64 each and eight more only copy, straight to LDS, through a ring of
+// five slabs of 32 KB; a copy's issue stalls then hold up nobody's MFMAs.  One barrier per slab, in the middle of the
+// computation of slab t: behind it slab t + 1, which every copying wavefront has waited for, may be read, and slab t + 5 is asked
+// for, into the place of slab t, whose operands are all in registers by then (four of the copying wavefronts ask for slab t + 4
+// instead).  Two to four slabs are on their way at any time.
+// What bounds it: the copies.  Where K is a multiple of 256, the lines of a slab's rows collide somewhere on their way to the
+// CU: 120 units of K = 5056 / 5120 / 5184 take 30.3 / 40.6 / 30.8 us with four copying wavefronts, 5120 33.0 with eight and 32.3
+// with four of these a slab behind (eight computing wavefronts of 64 x 32: as long; other orders of k per column: as long).
+// us, two workgroups to a CU -> this, inputs of four kinds in turn, GEMM-Q flagged, dense, GEMM-O cache and final pass:
+//   2 x 1100 x 1024 (144 units, 75 % flagged) 12.1 11.5 8.7 12.6 -> 10.5 10.1 8.1 10.6
+//   1200 x 3072 (240, 70 %)                   26.9 28.0 17.0 25.8 -> 22.8 25.0 15.2 21.9
+//   300 x 5120 (120, 70 %)                    39.7 38.8 20.9 31.9 -> 32.0 31.1 16.4 24.9
+// From 257 units on it would be two rounds: 384 units of K = 3072 39.6 -> 49.7.
+// ---------------------------------------------------------------------------------------------
+template <typename T, bool kReduce, bool kHalf, bool kPartial>
+__global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const GemmParams p) {
+  using TT = Types<T>;
+  using x8 = typename TT::x8;
+  using x4 = typename TT::x4;
+  constexpr int NT = 2, MT = 2;  // wavefront tile: 64 columns (W rows) x 64 token rows (X rows)
+  constexpr uint32_t kStage = 2 * kUnitBytes;  // X, W
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wv = wave & 3;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int wr = wv >> 1, wc = wv & 1;  // half of the unit's rows, of its columns
+
+  // ---- which unit: XCD x owns the x-th eighth of the units, ordered batch, window of eight token
+  // blocks, column, row: the units an XCD works on at a time share 8 + 4 operand tiles in its L2 ----
+  const int units_per_batch = p.n_row_tiles * p.n_col_tiles;
+  const int64_t total = static_cast<int64_t>(units_per_batch) * p.batch;
+  const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
+  const int u_lo = static_cast<int>(total * xcd / kXcds);
+  const int u = u_lo + slot;
+  if (u >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
+  const int bz = __builtin_amdgcn_readfirstlane(u / units_per_batch);
+  const int rem = u - bz * units_per_batch;
+  const int win = rem / (kUnitWindow * p.n_col_tiles);
+  const int in_win = rem - win * kUnitWindow * p.n_col_tiles;
+  const int win_rows = min(kUnitWindow, p.n_row_tiles - win * kUnitWindow);
+  const int col = __builtin_amdgcn_readfirstlane(in_win / win_rows);
+  const int row = __builtin_amdgcn_readfirstlane(win * kUnitWindow + in_win - col * win_rows);
+  const int m0 = row * kTile, n0 = col * kTile;
+  const uint32_t flag_row =
+      static_cast<uint32_t>(p.num_text_tokens + m0) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
+  if constexpr (!kReduce) {
+    if (p.flag == 0) {
+      const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
+      if (!flag_bit(info, flag_row + static_cast<uint32_t>(n0) / p.head_dim)) return;
     }
-    // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 256 bytes = 16 chunks)
+  }
+  SlabWalk<kReduce, kHalf> walk;
+  walk.begin(p, bz, flag_row, lane);
+  const int n_iter = walk.n_iter;
+  const int rows_here = min(p.m - m0, kTile);
+
+  if (wave >= 4) {
+    // ---- copies: 128 / kDeepCopiers rows of both tiles (rows past M read as zeros through the descriptor's range check; slabs past the
+    // last one go through empty descriptors: zeros, no memory access) ----
+    if (n_iter > 0) {
+      const uint32_t k2 = static_cast<uint32_t>(p.k) * 2u;
+      const T* const x_base = static_cast<const T*>(p.x) + (static_cast<int64_t>(bz) * p.m + m0) * p.k;
+      const T* const w_base = static_cast<const T*>(p.w) + static_cast<int64_t>(n0) * p.k;
+      uint32_t voff[2];
+#pragma unroll
+      for (int par = 0; par < 2; ++par)
+        voff[par] = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4);
+      typedef __attribute__((address_space(3))) void lds_void;
+      const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
+      auto copy = [&](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     :
+                     : "s"(lds_addr), "v"(vo), "s"(r), "s"(soff)
+                     : "memory", "m0");
+      };
+      constexpr uint32_t kPieces = 16 / kDeepCopiers;  // of eight rows, of either tile
+      const uint32_t cw = wave - 4;
+      int asked = 0;
+      uint32_t at = lds0 + cw * kPieces * 8 * kRowBytes;  // where the next slab goes
+      auto ask = [&]() __attribute__((always_inline)) {
+        const bool live = asked < n_iter;
+        const uint32_t koff = live ? walk.next(p).k + cw * kPieces * 8u * k2 : 0u;
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T*>(x_base), 0, live ? static_cast<uint32_t>(rows_here) * k2 : 0u, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(w_base), 0, live ? kTile * k2 : 0u, 0x00020000);
+#pragma unroll
+        for (uint32_t i = 0; i < kPieces; ++i) {
+          copy(rx, voff[i & 1], koff + i * 8u * k2, at + i * 8 * kRowBytes);
+          copy(rw, voff[i & 1], koff + i * 8u * k2, at + kUnitBytes + i * 8 * kRowBytes);
+        }
+        ++asked;
+        at = at >= lds0 + (kDeepRing - 1) * kStage ? at - (kDeepRing - 1) * kStage : at + kStage;
+      };
+      auto wait_copies = [&](auto n_tag) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_tag)::value;
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | ((n >> 4) << 14));  // vmcnt(n)
+      };
+      // kLag: how many slabs this wavefront's copies are behind
+      auto go = [&](auto lag_tag) __attribute__((always_inline)) {
+        constexpr int kLag = decltype(lag_tag)::value;
+        for (int i = 0; i < kDeepRing - kLag; ++i) ask();
+        wait_copies(std::integral_constant<int, 2 * kPieces * (kDeepRing - 1 - kLag)>{});
+        __builtin_amdgcn_s_barrier();
+        for (int it = 0; it < n_iter; ++it) {
+          wait_copies(std::integral_constant<int, 2 * kPieces * (kDeepRing - 2 - kLag)>{});
+          __builtin_amdgcn_s_barrier();
+          ask();
+        }
+      };
+      if (cw < kDeepCopiers / 2) go(std::integral_constant<int, 0>{}); else go(std::integral_constant<int, 1>{});
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): copies past the end
+    __builtin_amdgcn_s_barrier();
+    return;
+  }
+
+  // acc[nt][mt][i]: column wc*64 + nt*32 + (i/4)*8 + g*4 + i%4, row wr*64 + mt*32 + l32 of the unit
+  f32x16 acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+      for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
+
+  if (n_iter > 0) {
+    typedef __attribute__((address_space(3))) const x8 lds_x8;
+    typedef __attribute__((address_space(3))) void lds_void;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
+    const int rd_x = (g ^ ((l32 >> 1) & 7)) << 4;
+    const uint32_t a_base = lds0 + kUnitBytes + (wc * 64 + l32) * kRowBytes;  // W rows
+    const uint32_t b_base = lds0 + (wr * 64 + l32) * kRowBytes;               // X rows
+    // Operands are read two substeps ahead of their MFMAs (register set = substep): one ahead is 128 cycles
+    // of MFMAs, less than the LDS pipe's queue of four wavefronts.
+    x8 a[4][NT], b[4][MT];
+    auto lread = [&](uint32_t stage, int sub, int idx) __attribute__((always_inline)) {  // W rows 0, both X row groups, W rows 1
+      const uint32_t x = stage + (rd_x ^ (sub << 5));
+      if (idx == 0) {
+        a[sub][0] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(a_base + x));
+      } else if (idx <= MT) {
+        b[sub][idx - 1] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(b_base + (idx - 1) * 32 * kRowBytes + x));
+      } else {
+        a[sub][idx - MT] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(a_base + (idx - MT) * 32 * kRowBytes + x));
+      }
+    };
+    Slab now{0, ~0u, ~0u};
+    auto mma = [&](int sub, int i) __attribute__((always_inline)) {
+      if constexpr (kHalf) {
+        if (i == 0) {
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          f32x4 v;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = acc[nt][mt][i4 * 4 + j];
-          const int chunk = nt * 8 + i4 * 2 + g;
-          *reinterpret_cast<f32x4*>(region + (mt * 32 + l32) * 256 + ((chunk ^ (l32 & 15)) << 4)) = v;
+          for (int mt = 0; mt < MT; ++mt)
+            b[sub][mt] = __builtin_bit_cast(x8, __builtin_bit_cast(u32x4, b[sub][mt]) & (sub < 2 ? now.first : now.second));
         }
-    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
-    f32x4 vals[8];
+      }
+      acc[i / MT][i % MT] = TT::mfma(a[sub][i / MT], b[sub][i % MT], acc[i / MT][i % MT]);
+    };
+    __builtin_amdgcn_s_barrier();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if ((i & 7) == 0) {
+    for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int rk = (i + k) * 4 + rsub;
-          vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 256 + ((col4 ^ (rk & 15)) << 4));
-        }
+      for (int idx = 0; idx < NT + MT; ++idx) lread(0, sub, idx);
+    uint32_t stage = 0;
+    for (int it = 0; it < n_iter; ++it) {
+      if constexpr (kHalf) now = walk.next(p);
+      const uint32_t ahead = stage == (kDeepRing - 1) * kStage ? 0u : stage + kStage;
+      // substeps 0 and 1; the slab's last operand reads are three MFMAs old at the barrier
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        mma(0, i);
+        lread(stage, 2, i);
+        if (i < 3) lread(stage, 3, i);
         __builtin_amdgcn_sched_barrier(0);
       }
-      f32x4 v = vals[i & 7];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (kPartial) {
-          v[j] += static_cast<float>(bm[i][j]);
-        } else {
-          v[j] += bvec[j];
+      for (int i = 0; i < 4; ++i) {
+        mma(1, i);
+        if (i == 0) lread(stage, 3, 3);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      // (behind the last slab these read what nobody uses: places of the ring that hold zeros or an older slab)
+#pragma unroll
+      for (int sub = 2; sub < 4; ++sub)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          mma(sub, i);
+          lread(ahead, sub - 2, i);
+          __builtin_amdgcn_sched_barrier(0);
         }
-      }
-      if constexpr (kOutF32) {
-        // (no scalar offset: see the quads' store)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + 4 * i * p.n) * 4, 0, 2);
-      } else {
-        x4 out;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
-        typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, 4 * i * p.n * 2, 2);
-      }
+      stage = ahead;
     }
-  };
-  using std::false_type;
-  using std::true_type;
-  if constexpr (!kReduce) {
-    turn(T{}, false_type{});
-  } else if constexpr (kPartial) {
-    if (p.bias_f32) {
-      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
-    } else {
-      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
-    }
-  } else {
-    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
   }
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring, and no copy is on its way
+
+  unit_epilogue<T, kReduce, kPartial>(p, smem + wv * kUnitBytes, acc, bz, m0, n0, wr, wc, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1901,11 +2186,20 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       if (m) c1 = cw + __builtin_ctzll(m);
     }
   } else {
-    const int xr = xcd / cols, xc = xcd - xr * cols;
-    const int per = p.n_cp / cols;                 // column pairs of an XCD
-    const int cp = xc * per + slot % per;
-    block = xr + (kXcds / cols) * (slot / per);
-    if (block >= n_blocks) return;
+    int cp;
+    if (!kReduce && cols == 0) {  // strips of one round: an eighth each
+      const int64_t total = static_cast<int64_t>(n_blocks) * p.n_cp;
+      const int s = static_cast<int>(total * xcd / kXcds) + slot;
+      if (s >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
+      block = s / p.n_cp;
+      cp = s - block * p.n_cp;
+    } else {
+      const int xr = xcd / cols, xc = xcd - xr * cols;
+      const int per = p.n_cp / cols;                 // column pairs of an XCD
+      cp = xc * per + slot % per;
+      block = xr + (kXcds / cols) * (slot / per);
+      if (block >= n_blocks) return;
+    }
     c0 = 2 * cp;
     c1 = 2 * cp + 1 < p.n_col_tiles ? 2 * cp + 1 : -1;  // (the last pair may lack its second)
   }
@@ -1962,69 +2256,10 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
   const uint32_t flag_row = flag_row_of(row);
 
   // ---- the slabs: heads of this token block (GEMM-O), or all of k ----
-  unsigned long long mask[4] = {0, 0, 0, 0};
-  int n_iter, iph = 1, word = 0, sub = 0, k0 = 0;
-  if constexpr (kReduce) {
-    const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
-    const bool pick = p.flag == 0;  // final pass picks bit 1, cache pass bit 0
-    const int n_slices = p.k / p.head_dim;
-    bool sel[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sel[i] = 64 * i + lane < n_slices && flag_bit(info, flag_row + 64 * i + lane) == pick;
-    int count = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      mask[i] = __ballot(sel[i]);
-      count += __popcll(mask[i]);
-    }
-    iph = (p.head_dim + kBK - 1) / kBK;
-    n_iter = count * iph;
-  } else {
-    n_iter = (p.k + kBK - 1) / kBK;
-  }
-  // The next slab: its k offset, and (kHalf: heads or K of 32 mod 64) which half of it counts.  The last slab of a slice
-  // reaches 32 back; where the matrix begins, forward.
-  struct Slab {
-    uint32_t k;             // in bytes
-    uint32_t first, second;  // masks of its halves
-  };
-  auto next_slab = [&]() __attribute__((always_inline)) -> Slab {
-    Slab s{0, ~0u, ~0u};
-    if constexpr (kReduce) {
-      if (sub == 0) {
-        unsigned long long m = mask[0];
-#pragma unroll
-        for (int i = 1; i < 4; ++i) {
-          if (m == 0 && word < i) {
-            word = i;
-            mask[0] = m = mask[i];
-          }
-        }
-        k0 = (64 * word + __builtin_ctzll(m | (1ull << 63))) * p.head_dim;
-        mask[0] = m & (m - 1);
-      } else {
-        k0 += kBK;
-      }
-      if (++sub == iph) sub = 0;
-      s.k = static_cast<uint32_t>(k0) * 2u;
-      if constexpr (kHalf) {
-        if (sub == 0) {
-          if (k0 >= 32) s.k -= 64u;
-          (k0 >= 32 ? s.first : s.second) = 0u;
-        }
-      }
-    } else {
-      s.k = static_cast<uint32_t>(k0) * 2u;
-      k0 += kBK;
-      if constexpr (kHalf) {
-        if (k0 > p.k) {
-          s.k -= 64u;
-          s.first = 0u;
-        }
-      }
-    }
-    return s;
-  };
+  SlabWalk<kReduce, kHalf> walk;
+  walk.begin(p, bz, flag_row, lane);
+  const int n_iter = walk.n_iter;
+  auto next_slab = [&]() __attribute__((always_inline)) -> Slab { return walk.next(p); };
 
   const T* __restrict__ xg = static_cast<const T*>(p.x);
   const T* __restrict__ wg = static_cast<const T*>(p.w);
@@ -2310,20 +2545,26 @@ int64_t quad_slots(const ListGeom& gm, int num_cu) {
 
 // a workgroup per unit
 template <typename T, bool kReduce, bool kHalf, bool kAux>
-int launch_units(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
+int launch_units(GemmParams& p, const ListGeom& gm, int num_cu, hipStream_t stream) {
   static std::atomic<bool> attr_set[64] = {};
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
     FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_unit_kernel<T, kReduce, kHalf, kAux>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kUnitSmemBytes));
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_unit_deep_kernel<T, kReduce, kHalf, kAux>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kDeepSmemBytes));
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
   p.n_row_tiles = gm.n_row_tiles;
   p.n_col_tiles = gm.n_col_tiles;
   const int64_t units = unit_count(gm);
-  const int64_t grid = (units + kXcds - 1) / kXcds * kXcds;
-  gemm_unit_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kUnitSmemBytes, stream>>>(p);
+  const unsigned grid = static_cast<unsigned>((units + kXcds - 1) / kXcds * kXcds);
+  if (units <= num_cu) {
+    gemm_unit_deep_kernel<T, kReduce, kHalf, kAux><<<grid, kDeepThreads, kDeepSmemBytes, stream>>>(p);
+  } else {
+    gemm_unit_kernel<T, kReduce, kHalf, kAux><<<grid, kThreads, kUnitSmemBytes, stream>>>(p);
+  }
   FO_CHECK_LAUNCH();
   return FO_OK;
 }
@@ -2341,7 +2582,7 @@ int launch_packed(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 }
 
 template <typename T, bool kReduce, bool kHalf, bool kAux>
-int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
+int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream, bool one_round = false) {
   static std::atomic<bool> attr_set[64] = {};
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
@@ -2368,6 +2609,9 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
     int64_t per = 0;  // strips of a token block, at most
     for (int g = 0; g < cols; ++g) per += ((g + 1) * gm.n_col_tiles / cols - g * gm.n_col_tiles / cols + 1) / 2;
     grid = (rows * per + kXcds - 1) / kXcds * kXcds;
+  } else if (one_round) {
+    cols = 0;
+    grid = (rows * gm.n_cp + kXcds - 1) / kXcds * kXcds;
   } else {
     while (cols < 4 && gm.n_cp % (2 * cols) == 0 && gm.n_cp >= 6 * cols) cols *= 2;
     const int rx = kXcds / cols;
@@ -2394,7 +2638,7 @@ template <typename T, bool kHalf, bool kPartial>
 int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   const int num_cu = fo_num_cu();
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
-  if (unit_count(gm) <= 2 * num_cu) return launch_units<T, true, kHalf, kPartial>(p, gm, stream);
+  if (unit_count(gm) <= 2 * num_cu) return launch_units<T, true, kHalf, kPartial>(p, gm, num_cu, stream);
   if constexpr (!kHalf)
     if (p.k <= 512) return launch_packed<T, true, kPartial>(p, gm, stream);
   // (launches that could be judged both ways: more than one round of quads, 13 heads over the width times the rounds' fill,
@@ -2411,7 +2655,9 @@ int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 
 // GEMM-Q.
 //   * A workgroup per unit while all of them fit the chip at once, two per CU (us, quads -> units: 256 units of K = 2048
-//     46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged).
+//     46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged).  Dense, from one per CU on, strips, an
+//     eighth on each XCD (units -> strips: 288 of K = 3072 41.5 -> 36.5, 504 51.3 -> 46.5, 480 of K = 5120 83.8 -> 78.3, 328
+//     of K = 1024 18.0 -> 15.7; with flags, whose strips have to be counted first, 0.95 .. 1.2).
 //   * With flags: strips from 4.5 to 32 units per CU (16 beyond 32 column blocks, whose W the strips, which drift apart,
 //     read again and again; six column blocks at least, of which pairs can be made), otherwise quads, column strips and pairs
 //     by the kernel's own list, whose rounds last as long however few units they hold.  Strips over those, 10 .. 95 % flagged:
@@ -2430,7 +2676,8 @@ int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace,
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
   if constexpr (!kQuant) {
     const int64_t units = unit_count(gm);
-    if (units <= 2 * num_cu) return launch_units<T, false, kHalf, false>(p, gm, stream);
+    if (units <= num_cu || (use_flags && units <= 2 * num_cu)) return launch_units<T, false, kHalf, false>(p, gm, num_cu, stream);
+    if (units <= 2 * num_cu) return launch_strips<T, false, kHalf, false>(p, gm, stream, gm.n_cp * gm.batch * gm.n_row_tiles <= num_cu);
     if (use_flags && 2 * units > 9 * num_cu && units <= (gm.n_col_tiles <= 32 ? 32 : 16) * num_cu && gm.n_col_tiles >= 6)
       return launch_strips<T, false, kHalf, false>(p, gm, stream);
     if (!use_flags) {

@@ -561,6 +561,28 @@ def test_strips_equal_units(dev, case, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 129, 384, k) for k in (64, 96, 128, 256, 288, 320, 384, 672, 704)] +
+                         [(1, 1, 128, 5120), (2, 16384, 128, 64), (1, 2603, 3072, 96), (3, 900, 2304, 128), (1, 130, 17664, 64),
+                          (1, 33000, 256, 64), (1, 32641, 256, 160)])
+def test_dense_gemm_q_of_one_and_two_units_per_cu(dev, shape, dtype):
+    """Up to 256 units: one per CU, through a ring of five slabs (one to eleven of them, of which the last may count for one
+    half).  Up to 512: strips of one round, as many on every XCD, odd numbers of column blocks, one strip too many for a round.
+    Against the fp32 product."""
+    import flashomni_amd as fo
+    batch, m, n, k = shape
+    g = torch.Generator(device=dev).manual_seed(m + k)
+    x = torch.randn(batch, m, k, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, k, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+    out = torch.full((batch, m, n), float("nan"), dtype=dtype, device=dev)
+    y = fo.flashomni_gemm(x, w, n // 128, num_text_tokens=0, bias=b, is_full=True, out=out)
+    ref = torch.nn.functional.linear(x.float(), w.float(), b.float())
+    half_ulp = 2.0 ** (-9 if dtype == torch.bfloat16 else -11)
+    # (one rounding; sums of k products in another order: k * 2^-24 of the sum of their sizes, below 16 standard deviations of one)
+    assert bool(((y.float() - ref).abs() <= 2 * half_ulp * ref.abs() + k * 2.0 ** -24 * 16 * 0.02).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(1, 26003, 512, 512), (3, 10497, 384, 96), (1, 7289, 3072, 3072), (2, 3650, 2944, 2976)])
 def test_dense_gemm_q_as_strips(dev, shape, dtype):
     """Full GEMM-Q of narrow matrices and of rounds of quads that end half empty: strips.  Ragged last rows, an odd number
