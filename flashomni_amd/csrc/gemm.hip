@@ -55,7 +55,7 @@
 // item is requested before the epilogue, so that its latency hides behind the stores.
 //
 // Launches of few units and launches whose quads would leave CUs idle run a workgroup per unit or per strip instead
-// (gemm_unit_kernel, gemm_packed_kernel, gemm_strip_kernel, and the rules in launch_o and launch_q).
+// (gemm_deep_kernel, gemm_unit_kernel, gemm_packed_kernel, gemm_strip_kernel, and the rules in launch_o and launch_q).
 //
 // Work order.  Workgroups are persistent (one per CU).  The quad list is ordered by token window,
 // then column pair, then row pair, and XCD x (= blockIdx % 8) owns the x-th contiguous eighth of it.
@@ -87,8 +87,9 @@ constexpr int kStageBytes = 4 * kUnitBytes;        // X0, X1, W0, W1
 constexpr int kStages = 2;
 constexpr int kSmemBytes = kStages * kStageBytes;  // 128 KB
 constexpr int kUnitSmemBytes = kStages * 2 * kUnitBytes;  // workgroup per unit: 64 KB, two workgroups per CU
-constexpr int kDeepCopiers = 8, kDeepThreads = 256 + 64 * kDeepCopiers, kDeepRing = 5;  // ... one per CU: four wavefronts compute, eight copy
-constexpr int kDeepSmemBytes = kDeepRing * 2 * kUnitBytes;  // 160 KB
+constexpr int kDeepThreads = 768;  // ... one per CU, or a strip of two units: W column blocks take four wavefronts each, the rest copy
+constexpr int deep_ring(int W) { return W == 1 ? 5 : 3; }
+constexpr int deep_smem_bytes(int W) { return deep_ring(W) * (1 + W) * kUnitBytes; }  // 160, 144 KB
 constexpr int kUnitWindow = 8;  // ... token blocks per scheduling window
 constexpr int kZeroFirst = 1 << 18, kZeroSecond = 1 << 19;  // slab entry: half of the slab does not count
 constexpr int kMaxHeads = 256;
@@ -131,7 +132,7 @@ struct GemmParams {
                          // quads are enumerated arithmetically (GEMM-O, GEMM-Q with is_full)
   const int32_t* qoff;   // qoff[0..8] queue boundaries inside `quads`
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
-  int32_t strip_cols;    // strips: column groups of XCDs; 0: an eighth of the strips each
+  int32_t strip_cols;    // strips: column groups of XCDs
   int32_t strip_sorted;  // strips: token blocks with the most selected heads first
   int32_t* judgement;    // strips: where judge_flags leaves its word, or null
   int32_t judge_first, judge_bytes, judge_limit;
@@ -1216,27 +1217,35 @@ __device__ __forceinline__ void unit_epilogue(const GemmParams& p, uint8_t* regi
     using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
     constexpr bool kOutF32 = decltype(f32_tag)::value;
     constexpr int kBytes = sizeof(BiasT);
-    BiasVec bm[16];
+    // (pieces of the partial in flight together: sixteen of fp32 do not fit beside the accumulators)
+    constexpr int kAhead = kBytes == 4 ? 8 : 16;
+    BiasVec bm[kAhead];
     float bvec[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (kPartial) {
-      // sixteen pieces in flight together while the rows turn through LDS
+    auto load_partial = [&](int i0) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
+      for (int k = 0; k < kAhead; ++k) {
+        const int i = i0 + k;
         if constexpr (kBytes == 4) {
-          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, 4 * i * p.n * 4, 0));
+          bm[k] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, 4 * i * p.n * 4, 0));
         } else {
-          bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, 4 * i * p.n * 2, 0));
+          bm[k] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, 4 * i * p.n * 2, 0));
         }
       }
+    };
+    if constexpr (kPartial) {
+      load_partial(0);
     } else if (p.bias_kind == FO_BIAS_VECTOR) {
       const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + wc * 64 + col4 * 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
     }
-    // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 256 bytes = 16 chunks)
+    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt) {
+      if constexpr (kPartial)
+        if (mt > 0 && 8 * mt % kAhead == 0) load_partial(8 * mt);
+      // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 256 bytes = 16 chunks)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -1247,36 +1256,35 @@ __device__ __forceinline__ void unit_epilogue(const GemmParams& p, uint8_t* regi
           const int chunk = nt * 8 + i4 * 2 + g;
           *reinterpret_cast<f32x4*>(region + (mt * 32 + l32) * 256 + ((chunk ^ (l32 & 15)) << 4)) = v;
         }
-    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
-    f32x4 vals[8];
+      f32x4 vals[8];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if ((i & 7) == 0) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int rk = (i + k) * 4 + rsub;
-          vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 256 + ((col4 ^ (rk & 15)) << 4));
-        }
-        __builtin_amdgcn_sched_barrier(0);
+      for (int k = 0; k < 8; ++k) {
+        const int rk = (8 * mt + k) * 4 + rsub;
+        vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 256 + ((col4 ^ (rk & 15)) << 4));
       }
-      f32x4 v = vals[i & 7];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (kPartial) {
-          v[j] += static_cast<float>(bm[i][j]);
+      for (int k = 0; k < 8; ++k) {
+        const int i = 8 * mt + k;
+        f32x4 v = vals[k];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (kPartial) {
+            v[j] += static_cast<float>(bm[i % kAhead][j]);
+          } else {
+            v[j] += bvec[j];
+          }
+        }
+        if constexpr (kOutF32) {
+          // (no scalar offset: see the quads' store)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + 4 * i * p.n) * 4, 0, 2);
         } else {
-          v[j] += bvec[j];
-        }
-      }
-      if constexpr (kOutF32) {
-        // (no scalar offset: see the quads' store)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + 4 * i * p.n) * 4, 0, 2);
-      } else {
-        x4 out;
+          x4 out;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
-        typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, 4 * i * p.n * 2, 2);
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+          typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, 4 * i * p.n * 2, 2);
+        }
       }
     }
   };
@@ -1515,126 +1523,161 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_unit_kernel(const GemmParams
 }
 
 // ---------------------------------------------------------------------------------------------
-// At most a unit per CU.  Nothing but the depth of a unit's own pipeline hides its trips to L2 and memory then (staged through
-// registers a slab ahead, as above, a slab takes ~1050 cycles even on 84 of 256 CUs, 512 of them matrix core).  So a
-// workgroup has the whole CU: four wavefronts compute 64 x 64 each and eight more only copy, straight to LDS, through a ring of
-// five slabs of 32 KB; a copy's issue stalls then hold up nobody's MFMAs.  One barrier per slab, in the middle of the
-// computation of slab t: behind it slab t + 1, which every copying wavefront has waited for, may be read, and slab t + 5 is asked
-// for, into the place of slab t, whose operands are all in registers by then (four of the copying wavefronts ask for slab t + 4
-// instead).  Two to four slabs are on their way at any time.
+// A CU for a work item: W = 1, a unit, where there is at most one per CU; W = 2, a strip of one token block x two column blocks,
+// where all strips fit one round.  Nothing but the depth of an item's own pipeline hides its trips to L2 and memory then (staged
+// through registers a slab ahead, as above, a unit's slab takes ~1050 cycles even on 84 of 256 CUs, 512 of them matrix core).  So
+// four wavefronts per column block compute 64 x 64 each, and the rest of twelve only copy, straight to LDS, through a ring of five
+// slabs of 32 KB or three of 48 KB; a copy's issue stalls (110 to 150 cycles of its wavefront) then hold up nobody's MFMAs.  With W = 2
+// four copying wavefronts would be what it waits for, so each computing one issues three of a slab's 48 copies too.
+// One barrier per slab, in the middle of the computation of slab t: behind it slab t + 1, which every wavefront has waited for, may
+// be read, and the slab a ring further on is asked for, into the place of slab t, whose operands are all in registers by
+// then (W = 1: four of the copying wavefronts are a slab behind).  Two to four (W = 2: one to two) slabs are on their way at
+// any time.  The k order is that of the other forms, and so are the results, bit for bit.
 // What bounds it: the copies.  Where K is a multiple of 256, the lines of a slab's rows collide somewhere on their way to the
 // CU: 120 units of K = 5056 / 5120 / 5184 take 30.3 / 40.6 / 30.8 us with four copying wavefronts, 5120 33.0 with eight and 32.3
 // with four of these a slab behind (eight computing wavefronts of 64 x 32: as long; other orders of k per column: as long).
-// us, two workgroups to a CU -> this, inputs of four kinds in turn, GEMM-Q flagged, dense, GEMM-O cache and final pass:
+// W = 1, us, two workgroups to a CU -> this, inputs of four kinds in turn, GEMM-Q flagged, dense, GEMM-O cache and final pass:
 //   2 x 1100 x 1024 (144 units, 75 % flagged) 12.1 11.5 8.7 12.6 -> 10.5 10.1 8.1 10.6
 //   1200 x 3072 (240, 70 %)                   26.9 28.0 17.0 25.8 -> 22.8 25.0 15.2 21.9
-//   300 x 5120 (120, 70 %)                    39.7 38.8 20.9 31.9 -> 32.0 31.1 16.4 24.9
-// From 257 units on it would be two rounds: 384 units of K = 3072 39.6 -> 49.7.
+//   700 x 5120 (240, 70 %)                    40.7 43.0 20.1 37.6 -> 34.3 36.5 17.4 31.9
+// From 257 units on it would be two rounds: 384 units of K = 3072 39.6 -> 49.7.  W = 2: see deep_strips.
 // ---------------------------------------------------------------------------------------------
-template <typename T, bool kReduce, bool kHalf, bool kPartial>
-__global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const GemmParams p) {
+template <typename T, bool kReduce, bool kHalf, bool kPartial, int W>
+__global__ void __launch_bounds__(kDeepThreads) gemm_deep_kernel(const GemmParams p) {
   using TT = Types<T>;
   using x8 = typename TT::x8;
   using x4 = typename TT::x4;
   constexpr int NT = 2, MT = 2;  // wavefront tile: 64 columns (W rows) x 64 token rows (X rows)
-  constexpr uint32_t kStage = 2 * kUnitBytes;  // X, W
+  constexpr int kCompute = 4 * W, kCopiers = kDeepThreads / 64 - kCompute, kRing = deep_ring(W);
+  constexpr uint32_t kStage = (1 + W) * kUnitBytes;  // X, W of every column block
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wv = wave & 3;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
-  const int wr = wv >> 1, wc = wv & 1;  // half of the unit's rows, of its columns
+  const int wr = wv / (2 * W), wc = wv % (2 * W);  // half of the rows, 64 columns
 
-  // ---- which unit: XCD x owns the x-th eighth of the units, ordered batch, window of eight token
-  // blocks, column, row: the units an XCD works on at a time share 8 + 4 operand tiles in its L2 ----
-  const int units_per_batch = p.n_row_tiles * p.n_col_tiles;
-  const int64_t total = static_cast<int64_t>(units_per_batch) * p.batch;
+  // ---- which work item ----
   const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
-  const int u_lo = static_cast<int>(total * xcd / kXcds);
-  const int u = u_lo + slot;
-  if (u >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
-  const int bz = __builtin_amdgcn_readfirstlane(u / units_per_batch);
-  const int rem = u - bz * units_per_batch;
-  const int win = rem / (kUnitWindow * p.n_col_tiles);
-  const int in_win = rem - win * kUnitWindow * p.n_col_tiles;
-  const int win_rows = min(kUnitWindow, p.n_row_tiles - win * kUnitWindow);
-  const int col = __builtin_amdgcn_readfirstlane(in_win / win_rows);
-  const int row = __builtin_amdgcn_readfirstlane(win * kUnitWindow + in_win - col * win_rows);
-  const int m0 = row * kTile, n0 = col * kTile;
+  int bz, row, c0, c1 = -1;
+  if constexpr (W == 1) {
+    // XCD x owns the x-th eighth of the units, ordered batch, window of eight token
+    // blocks, column, row: the units an XCD works on at a time share 8 + 4 operand tiles in its L2
+    const int units_per_batch = p.n_row_tiles * p.n_col_tiles;
+    const int64_t total = static_cast<int64_t>(units_per_batch) * p.batch;
+    const int u = static_cast<int>(total * xcd / kXcds) + slot;
+    if (u >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
+    bz = u / units_per_batch;
+    const int rem = u - bz * units_per_batch;
+    const int win = rem / (kUnitWindow * p.n_col_tiles);
+    const int in_win = rem - win * kUnitWindow * p.n_col_tiles;
+    const int win_rows = min(kUnitWindow, p.n_row_tiles - win * kUnitWindow);
+    c0 = in_win / win_rows;
+    row = win * kUnitWindow + in_win - c0 * win_rows;
+  } else {
+    // ... of the strips
+    const int64_t total = static_cast<int64_t>(p.batch) * p.n_row_tiles * p.n_cp;
+    const int u = static_cast<int>(total * xcd / kXcds) + slot;
+    if (u >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
+    const int block = u / p.n_cp, cp = u - block * p.n_cp;
+    bz = block / p.n_row_tiles;
+    row = block - bz * p.n_row_tiles;
+    c0 = 2 * cp;
+    c1 = c0 + 1 < p.n_col_tiles ? c0 + 1 : -1;
+  }
+  bz = __builtin_amdgcn_readfirstlane(bz);
+  row = __builtin_amdgcn_readfirstlane(row);
+  const int m0 = row * kTile;
   const uint32_t flag_row =
       static_cast<uint32_t>(p.num_text_tokens + m0) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
   if constexpr (!kReduce) {
     if (p.flag == 0) {
       const uint8_t* info = p.sparse_info + p.sparse_info_indptr[bz];
-      if (!flag_bit(info, flag_row + static_cast<uint32_t>(n0) / p.head_dim)) return;
+      auto flagged = [&](int c) { return flag_bit(info, flag_row + static_cast<uint32_t>(c * kTile) / p.head_dim); };
+      const bool f0 = flagged(c0), f1 = c1 >= 0 && flagged(max(c1, 0));
+      if (!f0) c0 = -1;
+      if (!f1) c1 = -1;
     }
   }
+  c0 = __builtin_amdgcn_readfirstlane(c0);
+  c1 = __builtin_amdgcn_readfirstlane(c1);
+  if (c0 < 0 && c1 < 0) return;
   SlabWalk<kReduce, kHalf> walk;
   walk.begin(p, bz, flag_row, lane);
   const int n_iter = walk.n_iter;
   const int rows_here = min(p.m - m0, kTile);
 
-  if (wave >= 4) {
-    // ---- copies: 128 / kDeepCopiers rows of both tiles (rows past M read as zeros through the descriptor's range check; slabs past the
-    // last one go through empty descriptors: zeros, no memory access) ----
-    if (n_iter > 0) {
-      const uint32_t k2 = static_cast<uint32_t>(p.k) * 2u;
-      const T* const x_base = static_cast<const T*>(p.x) + (static_cast<int64_t>(bz) * p.m + m0) * p.k;
-      const T* const w_base = static_cast<const T*>(p.w) + static_cast<int64_t>(n0) * p.k;
-      uint32_t voff[2];
+  // ---- copies: pieces of eight rows; rows past M read as zeros through the descriptor's range check; missing column blocks
+  // and slabs past the last one go through empty descriptors (zeros, no memory access) ----
+  const uint32_t k2 = static_cast<uint32_t>(p.k) * 2u;
+  const T* const x_base = static_cast<const T*>(p.x) + (static_cast<int64_t>(bz) * p.m + m0) * p.k;
+  uint32_t voff[2];
 #pragma unroll
-      for (int par = 0; par < 2; ++par)
-        voff[par] = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4);
-      typedef __attribute__((address_space(3))) void lds_void;
-      const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
-      auto copy = [&](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     :
-                     : "s"(lds_addr), "v"(vo), "s"(r), "s"(soff)
-                     : "memory", "m0");
-      };
-      constexpr uint32_t kPieces = 16 / kDeepCopiers;  // of eight rows, of either tile
-      const uint32_t cw = wave - 4;
-      int asked = 0;
-      uint32_t at = lds0 + cw * kPieces * 8 * kRowBytes;  // where the next slab goes
+  for (int par = 0; par < 2; ++par)
+    voff[par] = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4);
+  typedef __attribute__((address_space(3))) void lds_void;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
+  auto copy = [&](const T* base, uint32_t bytes, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, bytes, 0x00020000);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(vo), "s"(r), "s"(soff)
+                 : "memory", "m0");
+  };
+  // of piece q of the W tiles
+  auto w_base = [&](uint32_t q) __attribute__((always_inline)) -> const T* {
+    return static_cast<const T*>(p.w) + static_cast<int64_t>(max(q < 16 ? c0 : c1, 0)) * kTile * p.k;
+  };
+  auto w_bytes = [&](uint32_t q) __attribute__((always_inline)) -> uint32_t { return (q < 16 ? c0 : c1) < 0 ? 0u : kTile * k2; };
+  auto wait_copies = [&](auto n_tag) __attribute__((always_inline)) {
+    constexpr int n = decltype(n_tag)::value;
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | ((n >> 4) << 14));  // vmcnt(n)
+  };
+  int asked = 0;
+  uint32_t at = lds0;  // where the next slab goes
+  auto advance = [&]() __attribute__((always_inline)) {
+    ++asked;
+    at = at == lds0 + (kRing - 1) * kStage ? lds0 : at + kStage;
+  };
+
+  if (wv >= kCompute) {
+    if (n_iter > 0) {
+      const uint32_t cw = wv - kCompute;
+      // W == 1: an eighth of the rows of either tile.  W == 2: a quarter of the pieces 8 .. 31 of the two W tiles
+      constexpr int kPieces = W == 1 ? 16 / kCopiers : 24 / kCopiers, kCopies = W == 1 ? 2 * kPieces : kPieces;
+      const uint32_t q0 = W == 1 ? cw * kPieces : 8 + cw * kPieces;  // (even)
       auto ask = [&]() __attribute__((always_inline)) {
         const bool live = asked < n_iter;
-        const uint32_t koff = live ? walk.next(p).k + cw * kPieces * 8u * k2 : 0u;
-        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T*>(x_base), 0, live ? static_cast<uint32_t>(rows_here) * k2 : 0u, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(w_base), 0, live ? kTile * k2 : 0u, 0x00020000);
+        const uint32_t koff = live ? walk.next(p).k : 0u;
+        const uint32_t x_bytes = live ? static_cast<uint32_t>(rows_here) * k2 : 0u;
 #pragma unroll
-        for (uint32_t i = 0; i < kPieces; ++i) {
-          copy(rx, voff[i & 1], koff + i * 8u * k2, at + i * 8 * kRowBytes);
-          copy(rw, voff[i & 1], koff + i * 8u * k2, at + kUnitBytes + i * 8 * kRowBytes);
+        for (int i = 0; i < kPieces; ++i) {
+          const uint32_t q = q0 + i;
+          if constexpr (W == 1) copy(x_base, x_bytes, voff[i & 1], koff + q * 8u * k2, at + q * 8 * kRowBytes);
+          copy(w_base(q), live ? w_bytes(q) : 0u, voff[i & 1], koff + (q & 15) * 8u * k2, at + kUnitBytes + q * 8 * kRowBytes);
         }
-        ++asked;
-        at = at >= lds0 + (kDeepRing - 1) * kStage ? at - (kDeepRing - 1) * kStage : at + kStage;
-      };
-      auto wait_copies = [&](auto n_tag) __attribute__((always_inline)) {
-        constexpr int n = decltype(n_tag)::value;
-        __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | ((n >> 4) << 14));  // vmcnt(n)
+        advance();
       };
       // kLag: how many slabs this wavefront's copies are behind
       auto go = [&](auto lag_tag) __attribute__((always_inline)) {
         constexpr int kLag = decltype(lag_tag)::value;
-        for (int i = 0; i < kDeepRing - kLag; ++i) ask();
-        wait_copies(std::integral_constant<int, 2 * kPieces * (kDeepRing - 1 - kLag)>{});
+        for (int i = 0; i < kRing - kLag; ++i) ask();
+        wait_copies(std::integral_constant<int, kCopies * (kRing - 1 - kLag)>{});
         __builtin_amdgcn_s_barrier();
         for (int it = 0; it < n_iter; ++it) {
-          wait_copies(std::integral_constant<int, 2 * kPieces * (kDeepRing - 2 - kLag)>{});
+          wait_copies(std::integral_constant<int, kCopies * (kRing - 2 - kLag)>{});
           __builtin_amdgcn_s_barrier();
           ask();
         }
       };
-      if (cw < kDeepCopiers / 2) go(std::integral_constant<int, 0>{}); else go(std::integral_constant<int, 1>{});
+      if (W == 2 || cw < kCopiers / 2) go(std::integral_constant<int, 0>{}); else go(std::integral_constant<int, W == 1 ? 1 : 0>{});
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): copies past the end
     __builtin_amdgcn_s_barrier();
     return;
   }
 
-  // acc[nt][mt][i]: column wc*64 + nt*32 + (i/4)*8 + g*4 + i%4, row wr*64 + mt*32 + l32 of the unit
+  // acc[nt][mt][i]: column wc*64 + nt*32 + (i/4)*8 + g*4 + i%4, row wr*64 + mt*32 + l32 of the item
   f32x16 acc[NT][MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
@@ -1645,8 +1688,6 @@ __global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const Gemm
 
   if (n_iter > 0) {
     typedef __attribute__((address_space(3))) const x8 lds_x8;
-    typedef __attribute__((address_space(3))) void lds_void;
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
     const int rd_x = (g ^ ((l32 >> 1) & 7)) << 4;
     const uint32_t a_base = lds0 + kUnitBytes + (wc * 64 + l32) * kRowBytes;  // W rows
     const uint32_t b_base = lds0 + (wr * 64 + l32) * kRowBytes;               // X rows
@@ -1663,6 +1704,7 @@ __global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const Gemm
         a[sub][idx - MT] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(a_base + (idx - MT) * 32 * kRowBytes + x));
       }
     };
+    SlabWalk<kReduce, kHalf> mine = walk;
     Slab now{0, ~0u, ~0u};
     auto mma = [&](int sub, int i) __attribute__((always_inline)) {
       if constexpr (kHalf) {
@@ -1674,6 +1716,33 @@ __global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const Gemm
       }
       acc[i / MT][i % MT] = TT::mfma(a[sub][i / MT], b[sub][i % MT], acc[i / MT][i % MT]);
     };
+    // W == 2: two pieces of X and one of W are this wavefront's to copy
+    uint32_t koff = 0, x_bytes = 0, w0_bytes = 0;
+    const uint32_t voff_w = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * (wv & 1) + (lane >> 4)) & 7)) << 4);
+    auto ask_for = [&]() __attribute__((always_inline)) {
+      const bool live = asked < n_iter;
+      koff = live ? walk.next(p).k : 0u;
+      x_bytes = live ? static_cast<uint32_t>(rows_here) * k2 : 0u;
+      w0_bytes = live ? w_bytes(0) : 0u;
+    };
+    auto copy_mine = [&](int i) __attribute__((always_inline)) {
+      const uint32_t q = i < 2 ? 2 * wv + i : wv;
+      if (i < 2) {
+        copy(x_base, x_bytes, voff[i], koff + q * 8u * k2, at + q * 8 * kRowBytes);
+      } else {
+        copy(w_base(0), w0_bytes, voff_w, koff + q * 8u * k2, at + kUnitBytes + q * 8 * kRowBytes);
+      }
+    };
+    if constexpr (W == 2) {
+      for (int i = 0; i < kRing; ++i) {
+        ask_for();
+        copy_mine(0);
+        copy_mine(1);
+        copy_mine(2);
+        advance();
+      }
+      wait_copies(std::integral_constant<int, 3 * (kRing - 1)>{});
+    }
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub)
@@ -1681,8 +1750,8 @@ __global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const Gemm
       for (int idx = 0; idx < NT + MT; ++idx) lread(0, sub, idx);
     uint32_t stage = 0;
     for (int it = 0; it < n_iter; ++it) {
-      if constexpr (kHalf) now = walk.next(p);
-      const uint32_t ahead = stage == (kDeepRing - 1) * kStage ? 0u : stage + kStage;
+      if constexpr (kHalf) now = mine.next(p);
+      const uint32_t ahead = stage == (kRing - 1) * kStage ? 0u : stage + kStage;
       // substeps 0 and 1; the slab's last operand reads are three MFMAs old at the barrier
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1697,6 +1766,10 @@ __global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const Gemm
         if (i == 0) lread(stage, 3, 3);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (W == 2) {
+        wait_copies(std::integral_constant<int, 3 * (kRing - 2)>{});
+        ask_for();
+      }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
       // (behind the last slab these read what nobody uses: places of the ring that hold zeros or an older slab)
@@ -1706,15 +1779,19 @@ __global__ void __launch_bounds__(kDeepThreads) gemm_unit_deep_kernel(const Gemm
         for (int i = 0; i < 4; ++i) {
           mma(sub, i);
           lread(ahead, sub - 2, i);
+          if (W == 2 && (i == 1 || (sub == 2 && i == 3))) copy_mine(sub == 3 ? 2 : i >> 1);
           __builtin_amdgcn_sched_barrier(0);
         }
+      if constexpr (W == 2) advance();
       stage = ahead;
     }
   }
-  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0)
   __builtin_amdgcn_s_barrier();  // every wavefront is done with the ring, and no copy is on its way
 
-  unit_epilogue<T, kReduce, kPartial>(p, smem + wv * kUnitBytes, acc, bz, m0, n0, wr, wc, lane);
+  const int c_mine = W == 1 || wc < 2 ? c0 : c1;
+  if (c_mine < 0) return;
+  unit_epilogue<T, kReduce, kPartial>(p, smem + wv * kUnitBytes, acc, bz, m0, c_mine * kTile, wr, wc & 1, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2186,20 +2263,11 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       if (m) c1 = cw + __builtin_ctzll(m);
     }
   } else {
-    int cp;
-    if (!kReduce && cols == 0) {  // strips of one round: an eighth each
-      const int64_t total = static_cast<int64_t>(n_blocks) * p.n_cp;
-      const int s = static_cast<int>(total * xcd / kXcds) + slot;
-      if (s >= static_cast<int>(total * (xcd + 1) / kXcds)) return;
-      block = s / p.n_cp;
-      cp = s - block * p.n_cp;
-    } else {
-      const int xr = xcd / cols, xc = xcd - xr * cols;
-      const int per = p.n_cp / cols;                 // column pairs of an XCD
-      cp = xc * per + slot % per;
-      block = xr + (kXcds / cols) * (slot / per);
-      if (block >= n_blocks) return;
-    }
+    const int xr = xcd / cols, xc = xcd - xr * cols;
+    const int per = p.n_cp / cols;                 // column pairs of an XCD
+    const int cp = xc * per + slot % per;
+    block = xr + (kXcds / cols) * (slot / per);
+    if (block >= n_blocks) return;
     c0 = 2 * cp;
     c1 = 2 * cp + 1 < p.n_col_tiles ? 2 * cp + 1 : -1;  // (the last pair may lack its second)
   }
@@ -2543,30 +2611,59 @@ int64_t quad_slots(const ListGeom& gm, int num_cu) {
   return (quads + num_cu - 1) / num_cu * 4 * num_cu;
 }
 
-// a workgroup per unit
+// a workgroup per unit, two on a CU
 template <typename T, bool kReduce, bool kHalf, bool kAux>
-int launch_units(GemmParams& p, const ListGeom& gm, int num_cu, hipStream_t stream) {
+int launch_units(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   static std::atomic<bool> attr_set[64] = {};
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
     FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_unit_kernel<T, kReduce, kHalf, kAux>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kUnitSmemBytes));
-    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_unit_deep_kernel<T, kReduce, kHalf, kAux>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, kDeepSmemBytes));
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
   p.n_row_tiles = gm.n_row_tiles;
   p.n_col_tiles = gm.n_col_tiles;
   const int64_t units = unit_count(gm);
-  const unsigned grid = static_cast<unsigned>((units + kXcds - 1) / kXcds * kXcds);
-  if (units <= num_cu) {
-    gemm_unit_deep_kernel<T, kReduce, kHalf, kAux><<<grid, kDeepThreads, kDeepSmemBytes, stream>>>(p);
-  } else {
-    gemm_unit_kernel<T, kReduce, kHalf, kAux><<<grid, kThreads, kUnitSmemBytes, stream>>>(p);
-  }
+  const int64_t grid = (units + kXcds - 1) / kXcds * kXcds;
+  gemm_unit_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kUnitSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
+}
+
+// a workgroup per unit (W = 1) or per strip of two (W = 2), one on a CU
+template <typename T, bool kReduce, bool kHalf, bool kAux, int W>
+int launch_deep(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
+  static std::atomic<bool> attr_set[64] = {};
+  int dev = 0;
+  FO_HIP_CALL(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_deep_kernel<T, kReduce, kHalf, kAux, W>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, deep_smem_bytes(W)));
+    if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
+  }
+  p.n_row_tiles = gm.n_row_tiles;
+  p.n_col_tiles = gm.n_col_tiles;
+  p.n_cp = gm.n_cp;
+  const int64_t items = static_cast<int64_t>(gm.batch) * gm.n_row_tiles * (W == 1 ? gm.n_col_tiles : gm.n_cp);
+  const int64_t grid = (items + kXcds - 1) / kXcds * kXcds;
+  gemm_deep_kernel<T, kReduce, kHalf, kAux, W><<<static_cast<unsigned>(grid), kDeepThreads, deep_smem_bytes(W), stream>>>(p);
+  FO_CHECK_LAUNCH();
+  return FO_OK;
+}
+
+// Strips of two units with a CU each, where there is more than a unit per CU and all strips fit one round.  us, units two to a
+// CU -> this, inputs of four kinds in turn:
+//                       GEMM-Q flagged  dense          GEMM-O cache   final
+//   1500 x 3072 (288)   37.4 -> 31.9    40.7 -> 33.3   25.5 -> 22.9   31.1 -> 28.5    60 % of the heads
+//   2500 x 3072 (480)   44.4 -> 40.4    48.9 -> 42.4   22.6 -> 21.5   43.7 -> 41.5    75 %
+//   2 x 4000 x 1024     17.6 -> 16.1    20.7 -> 18.5   16.4 -> 15.1   19.0 -> 18.3    60 %
+//   1500 x 5120 (480)   74.1 -> 58.4    82.7 -> 77.8   62.6 -> 62.9   40.2 -> 43.4    30 %
+//   1000 x 5120 (320)   59.8 -> 53.4    66.1 -> 64.0   30.9 -> 29.4   55.1 -> 58.0    70 %
+//   30 000 x 256 (470)   9.1 -> 9.0      9.6 -> 9.6     9.4 -> 8.6    10.0 -> 10.2    50 %
+// so GEMM-Q, and GEMM-O (whose strips differ in length where units two to a CU even out) up to 4096 columns.
+bool deep_strips(const ListGeom& gm, int32_t k, bool reduce, int num_cu) {
+  return static_cast<int64_t>(gm.batch) * gm.n_row_tiles * gm.n_cp <= num_cu && (!reduce || k <= 4096);
 }
 
 // the same, four on a CU
@@ -2582,7 +2679,7 @@ int launch_packed(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 }
 
 template <typename T, bool kReduce, bool kHalf, bool kAux>
-int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream, bool one_round = false) {
+int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   static std::atomic<bool> attr_set[64] = {};
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
@@ -2609,9 +2706,6 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream, bool on
     int64_t per = 0;  // strips of a token block, at most
     for (int g = 0; g < cols; ++g) per += ((g + 1) * gm.n_col_tiles / cols - g * gm.n_col_tiles / cols + 1) / 2;
     grid = (rows * per + kXcds - 1) / kXcds * kXcds;
-  } else if (one_round) {
-    cols = 0;
-    grid = (rows * gm.n_cp + kXcds - 1) / kXcds * kXcds;
   } else {
     while (cols < 4 && gm.n_cp % (2 * cols) == 0 && gm.n_cp >= 6 * cols) cols *= 2;
     const int rx = kXcds / cols;
@@ -2625,8 +2719,8 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream, bool on
 }
 
 // GEMM-O.
-//   * A workgroup per unit while all of them fit the chip at once, two per CU (144 units of K = 1024: quads 28 us, units
-//     12; strips over units up to one per CU 1.3 .. 1.6, of one to two 0.91 .. 1.3, about equal from K = 1024 on).
+//   * A CU per unit or per strip (gemm_deep_kernel), then a workgroup per unit, while all of them fit the chip at once, two
+//     per CU (144 units of K = 1024: quads 28 us, units 12; strips, two workgroups to a CU, over units up to one per CU 1.3 .. 1.6, of one to two 0.91 .. 1.3, about equal from K = 1024 on).
 //   * Narrow matrices, up to K = 512, are bound by memory and want the most loads in flight: packed units (strips over them,
 //     three to ten units per CU: 256 columns 1.0 .. 1.3, 384 1.1 .. 1.4, 512 1.0 .. 1.1).
 //   * Everything else: strips.  Over the better of quads and packed units, 2.3 to 9.7 units per CU, with 10, 50, 90 % of
@@ -2638,7 +2732,9 @@ template <typename T, bool kHalf, bool kPartial>
 int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   const int num_cu = fo_num_cu();
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
-  if (unit_count(gm) <= 2 * num_cu) return launch_units<T, true, kHalf, kPartial>(p, gm, num_cu, stream);
+  if (unit_count(gm) <= num_cu) return launch_deep<T, true, kHalf, kPartial, 1>(p, gm, stream);
+  if (deep_strips(gm, p.k, true, num_cu)) return launch_deep<T, true, kHalf, kPartial, 2>(p, gm, stream);
+  if (unit_count(gm) <= 2 * num_cu) return launch_units<T, true, kHalf, kPartial>(p, gm, stream);
   if constexpr (!kHalf)
     if (p.k <= 512) return launch_packed<T, true, kPartial>(p, gm, stream);
   // (launches that could be judged both ways: more than one round of quads, 13 heads over the width times the rounds' fill,
@@ -2654,10 +2750,9 @@ int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 }
 
 // GEMM-Q.
-//   * A workgroup per unit while all of them fit the chip at once, two per CU (us, quads -> units: 256 units of K = 2048
-//     46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter flagged).  Dense, from one per CU on, strips, an
-//     eighth on each XCD (units -> strips: 288 of K = 3072 41.5 -> 36.5, 504 51.3 -> 46.5, 480 of K = 5120 83.8 -> 78.3, 328
-//     of K = 1024 18.0 -> 15.7; with flags, whose strips have to be counted first, 0.95 .. 1.2).
+//   * A CU per unit or per strip (gemm_deep_kernel), then a workgroup per unit, while all of them fit the chip at once, two
+//     per CU (us, quads -> units: 256 units of K = 2048 46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter
+//     flagged).
 //   * With flags: strips from 4.5 to 32 units per CU (16 beyond 32 column blocks, whose W the strips, which drift apart,
 //     read again and again; six column blocks at least, of which pairs can be made), otherwise quads, column strips and pairs
 //     by the kernel's own list, whose rounds last as long however few units they hold.  Strips over those, 10 .. 95 % flagged:
@@ -2676,8 +2771,9 @@ int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace,
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
   if constexpr (!kQuant) {
     const int64_t units = unit_count(gm);
-    if (units <= num_cu || (use_flags && units <= 2 * num_cu)) return launch_units<T, false, kHalf, false>(p, gm, num_cu, stream);
-    if (units <= 2 * num_cu) return launch_strips<T, false, kHalf, false>(p, gm, stream, gm.n_cp * gm.batch * gm.n_row_tiles <= num_cu);
+    if (units <= num_cu) return launch_deep<T, false, kHalf, false, 1>(p, gm, stream);
+    if (deep_strips(gm, p.k, false, num_cu)) return launch_deep<T, false, kHalf, false, 2>(p, gm, stream);
+    if (units <= 2 * num_cu) return launch_units<T, false, kHalf, false>(p, gm, stream);
     if (use_flags && 2 * units > 9 * num_cu && units <= (gm.n_col_tiles <= 32 ? 32 : 16) * num_cu && gm.n_col_tiles >= 6)
       return launch_strips<T, false, kHalf, false>(p, gm, stream);
     if (!use_flags) {

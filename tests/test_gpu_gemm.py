@@ -562,11 +562,11 @@ def test_strips_equal_units(dev, case, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(1, 129, 384, k) for k in (64, 96, 128, 256, 288, 320, 384, 672, 704)] +
-                         [(1, 1, 128, 5120), (2, 16384, 128, 64), (1, 2603, 3072, 96), (3, 900, 2304, 128), (1, 130, 17664, 64),
+                         [(1, 1, 128, 5120), (2, 16384, 128, 64), (1, 2603, 3072, 96), (3, 900, 2304, 128), (3, 900, 2304, 160), (1, 130, 17664, 64), (1, 300, 12672, 352),
                           (1, 33000, 256, 64), (1, 32641, 256, 160)])
 def test_dense_gemm_q_of_one_and_two_units_per_cu(dev, shape, dtype):
     """Up to 256 units: one per CU, through a ring of five slabs (one to eleven of them, of which the last may count for one
-    half).  Up to 512: strips of one round, as many on every XCD, odd numbers of column blocks, one strip too many for a round.
+    half).  Up to 512: strips with a CU each, through a ring of three, odd numbers of column blocks, one strip too many for a round.
     Against the fp32 product."""
     import flashomni_amd as fo
     batch, m, n, k = shape
