@@ -583,7 +583,7 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   p->state = 0;
   int rc = 0;
   int64_t ints = z.table_ints;
-  if (z.max_rows > 0 && z.max_rows < fo_decode_sparse_clear_min_pairs() && z.max_nnz <= (1 << 20) && z.max_kv_len <= kMaxListed) {
+  if (z.max_rows > 0 && z.max_rows <= fo_sparse_attention_direct_max_pairs() && z.max_nnz <= (1 << 20) && z.max_kv_len <= kMaxListed) {
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     // (symbol tensors much larger than the batch needs are not worth copying)
     p->keep_room[0] = z.min_info + 4096;

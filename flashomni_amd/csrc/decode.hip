@@ -44,7 +44,7 @@ constexpr int kXcds = 8;
 constexpr int kHistSlots = 8192;  // (head, length class) counters of the order layout
 // even shares (see the attention kernel): words of `sched` and limits
 constexpr int kSchedEven = 26, kSchedShare = 27, kSchedTotal = 28, kSchedShares = 29, kSchedRows = 30,
-              kSchedRecords = 31, kSchedOrdered = 32, kSchedKept = 33, kSchedArrived = 64;
+              kSchedRecords = 31, kSchedOrdered = 32, kSchedKept = 33, kSchedFill = 34, kSchedArrived = 64;
 constexpr int kSchedWords = 40;      // words [0, kSchedWords) are rewritten by every decode
 constexpr int kRecordInts = 8;  // queue entry: row, request, q block, head, first kv slot, kv count, pad, pad
 constexpr int kMaxShares = 512;      // arrival counters in `sched`, first-row entries in `shares`
@@ -114,9 +114,14 @@ __global__ void __launch_bounds__(kCountThreads) decode_count_kernel(
     const int32_t* __restrict__ sparse_info_indptr,
     const int32_t* __restrict__ sparse_kv_info_indptr, const int32_t* __restrict__ blk_req,
     const int32_t* __restrict__ blk_qb, const int32_t* __restrict__ kv_indptr, int64_t n_cand,
-    int32_t num_heads, int32_t block_kv, int is_full, int32_t* __restrict__ act,
+    int32_t num_heads, int32_t block_kv, int is_full, const int32_t* __restrict__ kept, int32_t* __restrict__ act,
     int32_t* __restrict__ cnt) {
   const int lane = threadIdx.x % kWave;
+  if (kept != nullptr) {  // (see fo_decode_sparse_kept)
+    const int32_t newer = kept[kSchedKept];
+    if (newer == 0) return;
+    is_full = newer == 2;
+  }
   const int64_t c = static_cast<int64_t>(blockIdx.x) * (kCountThreads / kWave) + threadIdx.x / kWave;
   if (c >= n_cand) return;
   const Candidate cd = load_candidate(c, num_heads, block_kv, is_full, sparse_info,
@@ -469,13 +474,25 @@ __global__ void __launch_bounds__(kScanThreads) decode_scan_kernel(
     int64_t n_cand, int32_t num_heads, int32_t* __restrict__ act, int32_t* __restrict__ cnt,
     int32_t* __restrict__ kv_row_ptr, int32_t* __restrict__ counts,
     int32_t* __restrict__ head_cursor, int32_t* __restrict__ sched, int32_t* __restrict__ order,
-    int32_t* __restrict__ shares, int32_t n_shares, int32_t n_wg) {
+    int32_t* __restrict__ shares, int32_t n_shares, int32_t n_wg, int kept) {
   __shared__ int32_t s_rows[kScanThreads];
   __shared__ int32_t s_kv[kScanThreads];
   __shared__ int32_t s_hist[kHistSlots];
   __shared__ int32_t s_max;
+  int32_t newer = 0;
+  if (kept) {  // what the fill is to do is left to it: the scan clears the word that says so
+    newer = sched[kSchedKept];
+    if (newer == 0) {
+      if (threadIdx.x == 0) sched[kSchedFill] = 0;
+      return;
+    }
+  }
   scan_body(n_cand, num_heads, act, cnt, kv_row_ptr, counts, head_cursor, sched, order, shares, n_shares, n_wg,
             s_rows, s_kv, s_hist, &s_max);
+  if (kept) {
+    __syncthreads();
+    if (threadIdx.x == 0) sched[kSchedFill] = newer;
+  }
 }
 
 // Short lists (at most one candidate per thread of one workgroup): count, scan and fill in one launch,
@@ -625,8 +642,13 @@ __global__ void __launch_bounds__(kCountThreads) decode_fill_kernel(
     int32_t* __restrict__ kv_row_ptr, int32_t* __restrict__ kv_idx,
     int32_t* __restrict__ head_cursor, int32_t* __restrict__ order,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ sched,
-    int32_t* __restrict__ shares, ClearRows clear) {
+    int32_t* __restrict__ shares, ClearRows clear, int kept) {
   const int lane = threadIdx.x % kWave;
+  if (kept) {
+    const int32_t newer = sched[kSchedFill];
+    if (newer == 0) return;
+    is_full = newer == 2;
+  }
   const int64_t c = static_cast<int64_t>(blockIdx.x) * (kCountThreads / kWave) + threadIdx.x / kWave;
   if (c >= n_cand) return;
   const int32_t pos = row_pos[c];
@@ -743,11 +765,11 @@ int decode_impl(const uint8_t* sparse_info, const uint8_t* sparse_kv_info, const
     const unsigned grid = static_cast<unsigned>((n_cand + per_wg - 1) / per_wg);
     decode_count_kernel<<<grid, kCountThreads, 0, s>>>(
         sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
-        kv_indptr, n_cand, num_heads, block_kv, is_full, act, cnt);
+        kv_indptr, n_cand, num_heads, block_kv, is_full, kept ? sched : nullptr, act, cnt);
     FO_CHECK_LAUNCH();
   }
   decode_scan_kernel<<<1, kScanThreads, 0, s>>>(n_cand, num_heads, act, cnt, kv_row_ptr, counts,
-                                                head_cursor, sched, order, shares, n_shares, n_wg);
+                                                head_cursor, sched, order, shares, n_shares, n_wg, kept);
   FO_CHECK_LAUNCH();
   if (n_cand > 0) {
     const int per_wg = kCountThreads / kWave;
@@ -755,7 +777,7 @@ int decode_impl(const uint8_t* sparse_info, const uint8_t* sparse_kv_info, const
     decode_fill_kernel<<<grid, kCountThreads, 0, s>>>(
         sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
         kv_indptr, n_cand, num_heads, block_kv, is_full, act, cnt, row_req, row_qb, row_head,
-        kv_row_ptr, kv_idx, head_cursor, order, counts, sched, shares, clear);
+        kv_row_ptr, kv_idx, head_cursor, order, counts, sched, shares, clear, kept);
     FO_CHECK_LAUNCH();
   }
   return FO_OK;
@@ -804,7 +826,8 @@ extern "C" int fo_decode_sparse_kept(const uint8_t* sparse_info, const uint8_t* 
                                      int32_t* counts, int32_t* order, int32_t* sched, int32_t* scratch, int32_t* shares,
                                      void* stream) {
   const int64_t n_cand = static_cast<int64_t>(n_blk) * num_heads;
-  FO_REQUIRE(n_cand > 0 && n_cand <= kScanThreads, "decode: lists of 1 to %d (q-block, head) pairs only", kScanThreads);
+  FO_REQUIRE(n_cand > 0 && n_cand <= fo_sparse_attention_direct_max_pairs(),
+             "decode: lists of 1 to %d (q-block, head) pairs only", fo_sparse_attention_direct_max_pairs());
   return decode_impl(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, blk_req, blk_qb,
                      kv_indptr, n_blk, num_heads, block_kv, 0, row_req, row_qb, row_head, kv_row_ptr, kv_idx, counts,
                      order, sched, scratch, shares, stream, ClearRows{}, 1);

@@ -389,7 +389,11 @@ struct DirectMask {
   int mask_first, nkv;
 };
 struct NoMask {};
-constexpr int kDirectMaxCand = 1024;  // candidates (symbol row, head): two per thread of a workgroup
+// candidates (symbol row, head): two per thread of a workgroup, four in the pipelined form, of which there is a kernel for
+// more (kMany: seven per thread; with the steps for them 1000 candidates would take 61.4 us in place of 59.7)
+constexpr int direct_max_cand(bool many) { return many ? 1792 : 1024; }
+constexpr int kDirectMaxFull = 1408;    // ... where every row is computed whole (is_full), see fo_sparse_attention_direct_serves
+constexpr int kDirectShareRows = 1024;  // rows of a share that the table of them holds (see direct_table_holds)
 constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
 constexpr int kDirectMapBytes = (1 << 16) - 16;  // keep bits that are staged in the tile buffers (both forms have as much)
 constexpr int kOlderGain = 10;  // see cut_at
@@ -415,7 +419,7 @@ constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologu
 // their phases together, there is no merge, and one's row prologue / epilogue overlaps the other's
 // main loop.  A row takes twice as long, so this is the form for long lists (many rows per CU).
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false, bool kDirect = false, bool kWide = false>
+          bool kCap = false, bool kDirect = false, bool kWide = false, bool kMany = false>
 __global__ void __launch_bounds__(kGroups * kGroupThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 sparse_fa_kernel(const FaParams p) {
   static_assert(!kWide || (kPipe && !kGqaPack && !kDirect), "widened operands are a variant of the pipelined loop");
@@ -748,10 +752,13 @@ sparse_fa_kernel(const FaParams p) {
   // In the pipelined form the next item is fetched beside a row's first copies instead of at its end, where the
   // trips to memory are 2.4 us that nothing hides.
   __shared__ int s_wave[4 + kDirectMaxParts / 2][8];
-  __shared__ uint16_t s_row_cand[kDirect ? kDirectMaxCand : 1];  // even shares: candidate of every active row ...
-  __shared__ int s_row_u[kDirect ? kDirectMaxCand + 1 : 1];      // ... and the cost at which its kv blocks begin
-  __shared__ uint16_t s_zero[kDirect ? 64 : 1];                  // candidates this workgroup clears
-  // first row of the share, candidates to clear; even shares: rows (0: one item at most), shares, cost of all
+  // even shares: the rows of this workgroup's share, where there may be more than the table holds row i at i % kDirectShareRows
+  __shared__ uint16_t s_row_cand[kDirect ? kDirectShareRows : 1];  // a row's candidate ...
+  __shared__ int s_row_u[kDirect ? kDirectShareRows + 1 : 1];      // ... and the cost at which its kv blocks begin
+  auto row_at = [](int i) { return kMany ? i & (kDirectShareRows - 1) : i; };
+  constexpr int kMaxCand = direct_max_cand(kMany);
+  __shared__ uint16_t s_zero[kDirect ? kMaxCand / 16 : 1];         // candidates this workgroup clears (of 16 or more)
+  // first row of the share, candidates to clear; even shares: the row behind its last one (0: one item at most), shares, cost of all
   // (in LDS and not in registers, where they would live through the main loop)
   __shared__ int s_dir[5];
   __shared__ int s_list_at;  // whole parts: where the item's keep bits are in LDS (words from smem on), or -1
@@ -817,7 +824,7 @@ sparse_fa_kernel(const FaParams p) {
     it.q_scale = 1.f;
     it.k_scale0 = 0;
   };
-  constexpr int kCands = kDirectMaxCand / (64 * kWaves);         // candidates of a thread, at most
+  constexpr int kCands = kMaxCand / (64 * kWaves);  // candidates of a thread, at most
   auto direct_schedule = [&]() {
     const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads, dir_g = dir_index();
     // (No more of them than it takes: the schedule is bound by the instructions of its two wavefronts per SIMD, not by
@@ -995,7 +1002,7 @@ sparse_fa_kernel(const FaParams p) {
     }
     const int total = kShareRowCost * rows + blocks;
     // (a row in at most four parts: no share is shorter than a third of the longest row)
-    const int shares = max(min(min(n_wg, total), max_n > 0 ? 3 * total / max_n : 1), 1);
+    const int shares = max(min(min(n_wg, total), max_n > 0 ? 3 * total / max_n : total), 1);
     if (rows <= n_wg) {
       // parts of at most ceil(max_n / k) kv blocks: how many there are for every k
       // (the finest cut fits where even a row of the most parts in place of every row would)
@@ -1076,21 +1083,28 @@ sparse_fa_kernel(const FaParams p) {
         return;
       }
     }
-    const int a = cut_at(dir_g, total, shares);
+    // Rows of the share alone: there are no more than the table holds (direct_table_holds).
+    const int a = cut_at(dir_g, total, shares), b = cut_at(dir_g + 1, total, shares);
     int cost = kShareRowCost * row + before;
 #pragma unroll
     for (int u = 0; u < kCands; ++u)
       if (act[u]) {
-        s_row_cand[row] = static_cast<uint16_t>(first_cand + u);
-        s_row_u[row] = cost + kShareRowCost;
-        // first row of the share: the one that holds the share's lower bound
-        if (cost <= a && a < cost + kShareRowCost + n[u]) s_dir[0] = row;
-        cost += kShareRowCost + n[u];
+        const int after = cost + kShareRowCost + n[u];
+        if (cost < b && a < after) {
+          s_row_cand[row_at(row)] = static_cast<uint16_t>(first_cand + u);
+          s_row_u[row_at(row)] = cost + kShareRowCost;
+          // first row of the share: the one that holds the share's lower bound; its last one holds the upper bound's unit in front
+          if (cost <= a) s_dir[0] = row;
+          if (b <= after) {
+            s_row_u[row_at(row + 1)] = after + kShareRowCost;
+            s_dir[2] = row + 1;
+          }
+        }
+        cost = after;
         ++row;
       }
     if (tid == 0) {
-      s_row_u[rows] = total + kShareRowCost;
-      s_dir[2] = rows;
+      if (dir_g >= shares) s_dir[2] = 1;  // (no row: see direct_items)
       s_dir[3] = shares;
       s_dir[4] = total;
     }
@@ -1105,10 +1119,11 @@ sparse_fa_kernel(const FaParams p) {
       const int dir_g = dir_index(), rows = s_dir[2], shares = s_dir[3], total = s_dir[4];
       const int a = cut_at(dir_g, total, shares), b = cut_at(dir_g + 1, total, shares), i = s_dir[0] + batch_base + lane;
       if (dir_g < shares && i >= 0 && i < rows) {
-        const int u = s_row_u[i], e = s_row_u[i + 1] - kShareRowCost;  // kv blocks cost [u, e)
+        // kv blocks cost [u, e)
+        const int u = s_row_u[row_at(i)], e = s_row_u[row_at(i + 1)] - kShareRowCost;
         // (a row without kv blocks stands for the last unit of its own overhead)
         if ((e > u ? u : u - 1) < b) {
-          direct_row(s_row_cand[i], it);
+          direct_row(s_row_cand[row_at(i)], it);
           it.part = 0;
           it.parts = 1;
           it.slot = 0;
@@ -2531,7 +2546,7 @@ __global__ void __launch_bounds__(256) widen_k_kernel(
 }
 
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups = 2, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false, bool kDirect = false, bool kWide = false>
+          bool kCap = false, bool kDirect = false, bool kWide = false, bool kMany = false>
 int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   constexpr int kSmemBytes = Geom<kFp8, kKLo, kGroups>::kSmemBytes;
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
@@ -2540,7 +2555,7 @@ int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   int dev = 0;
   FO_HIP_CALL(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
-    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect, kWide>),
+    FO_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect, kWide, kMany>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes));
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
@@ -2549,7 +2564,7 @@ int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   int64_t grid = num_cu * (3 - kGroups);  // persistent workgroups: one per CU, or two of one kv group each (LDS bound)
   // (with even shares every workgroup may hold a part of a row; otherwise at most one row each)
   if (!kDirect && !(p.split_ws && p.shares) && grid > max_rows) grid = max_rows;
-  sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect, kWide><<<static_cast<unsigned>(grid), kGroups * kGroupThreads, kSmemBytes, stream>>>(p);
+  sparse_fa_kernel<T, kFp8, kQLo, kKLo, kGroups, kPipe, kGqaPack, kCap, kDirect, kWide, kMany><<<static_cast<unsigned>(grid), kGroups * kGroupThreads, kSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
 }
@@ -2782,17 +2797,54 @@ extern "C" int64_t fo_sparse_fa_wide_bytes(int64_t max_rows, int32_t num_kv_head
   return wide_head_bytes(num_kv_heads) + static_cast<int64_t>(num_kv_heads) * n_kv_blocks * kBlockKV * kHeadDim * 2;
 }
 
+namespace {
+
+// From 2.5 candidates per CU on: two workgroups of four wavefronts per CU and the software-pipelined loop, whose
+// row boundaries pass beside the other workgroup's main loop; below, the two-phase loop with twice the wavefronts
+// per row.  Pipelined against two-phase, with (active rows, kept blocks): 864 candidates of 36 blocks 155 / 165 us
+// (100 %, 50 %), 273 / 295 (100 %, 100 %), 119 / 127 (75 %, 50 %), 62 / 59 (30 %, 50 %); 1000 of 25 blocks 106 / 113
+// (75 %, 50 %), 56 / 54 (30 %, 50 %); 512 of 32 blocks 76 / 72 (75 %, 50 %), 44 / 41 (30 %, 50 %); 216 of 9 blocks
+// 31 / 27.  What it needs besides: partial results of two shares per CU, room in LDS for a row's list (the
+// longest row is bounded by all keep bits where there are several requests), 32-bit copy offsets.
+bool direct_pipe(const fo_attention_args& a, int num_cu) {
+  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  const int64_t nkv = a.max_nnz / (a.batch == 1 ? n_cand : a.symbol_heads), span = (nkv + 1) * kBlockKV * 2;
+  return a.logits_soft_cap <= 0.f && 2 * n_cand >= int64_t(5) * num_cu && nkv <= kMaxRowBlocksOneGroupDirect &&
+         2 * num_cu <= kMaxShares && a.split_ws_bytes >= 2 * fo_sparse_fa_split_workspace_bytes() &&
+         span * a.k_stride_n < (int64_t(1) << 32) && span * a.v_stride_n < (int64_t(1) << 32);
+}
+
+// Whether a share of the pipelined form has fewer rows than its table: a row costs kRowOverheadPipe at least, and a share
+// is no longer than an even part of all cost, kOlderGain / 128 more, or four ninths of the longest row (of 3 and
+// a part thirds 3 are made).
+bool direct_table_holds(int64_t n_cand, int64_t max_nnz, int num_cu) {
+  const int64_t even = (max_nnz + kRowOverheadPipe * n_cand) / (2 * num_cu), longest = kMaxRowBlocksOneGroupDirect;
+  return ((even + 2) * (128 + kOlderGain) / 128 / kRowOverheadPipe + 3 < kDirectShareRows &&
+          (4 * longest / 9 + 2) / kRowOverheadPipe + 3 < kDirectShareRows);
+}
+
+}  // namespace
+
 extern "C" int fo_sparse_attention_direct_serves(const void* args) {
   const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
   const int num_cu = fo_num_cu();
   const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
-  // Two candidates per thread at most, and keep bits that every workgroup can afford to read (2^20 bits =
-  // 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also sorts
-  // their rows.
+  // Candidates that a workgroup's threads can go through at the top of a launch, and keep bits that every workgroup can
+  // afford to read (2^20 bits = 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also
+  // sorts their rows by head, so that one head's K and V at a time are in an XCD's L2: the more of a row's blocks are kept, the
+  // earlier.  The lists that only the pipelined form takes, decoded -> straight from the symbols, us per call (rows, blocks kept):
+  //   1032 candidates of 43 blocks  72 -> 62 (50, 10 %)  189 -> 170 (75, 50)  446 -> 383 (all)     1040 of 26  53 -> 44 (30, 5)
+  //   1320 of 55                    71 -> 65 (20, 20)    273 -> 260 (75, 50)  654 -> 593 (all)     1040 of 65  101 -> 89 (70, 10)
+  //   1536 of 64 to 192             256 -> 235 (70, 10)  759 -> 773 (100, 30) 779 -> 817, 1152 -> 1200 (all)
+  //   1704 of 71                    210 -> 194 (50, 30)  427 -> 421 (75, 50)  971 -> 1008 (all)
+  //   2040 of 85                    256 -> 246 (100, 10) 560 -> 573 (75, 50)  1356 -> 1420 (all)
   return (a.dtype == FO_BF16 || a.dtype == FO_F16) && g_variant.load(std::memory_order_relaxed) != 1 && n_cand >= 1 &&
-         n_cand <= kDirectMaxCand && a.max_nnz <= (1 << 20) && num_cu >= 16 && num_cu <= kMaxShares && a.split_ws &&
-         a.split_ws_bytes >= fo_sparse_fa_split_workspace_bytes() && (reinterpret_cast<uintptr_t>(a.split_ws) & 15) == 0;
+         (n_cand <= direct_max_cand(false) ||
+          (n_cand <= (a.is_full ? kDirectMaxFull : direct_max_cand(true)) && g_variant.load(std::memory_order_relaxed) == 0 && direct_pipe(a, num_cu) && direct_table_holds(n_cand, a.max_nnz, num_cu))) &&
+         a.max_nnz <= (1 << 20) && num_cu >= 16 && num_cu <= kMaxShares && a.split_ws && a.split_ws_bytes >= fo_sparse_fa_split_workspace_bytes() && (reinterpret_cast<uintptr_t>(a.split_ws) & 15) == 0;
 }
+
+extern "C" int32_t fo_sparse_attention_direct_max_pairs(void) { return direct_max_cand(true); }
 
 extern "C" int fo_sparse_attention_direct(const void* args) {
   FO_REQUIRE(args, "sparse_attention: null pointer");
@@ -2846,18 +2898,14 @@ extern "C" int fo_sparse_attention_direct(const void* args) {
     return bf16 ? launch<__bf16, false, false, false, 2, false, false, true, true>(p, n_cand, s)
                 : launch<_Float16, false, false, false, 2, false, false, true, true>(p, n_cand, s);
   }
-  // From 2.5 candidates per CU on: two workgroups of four wavefronts per CU and the software-pipelined loop, whose
-  // row boundaries pass beside the other workgroup's main loop; below, the two-phase loop with twice the wavefronts
-  // per row.  Pipelined against two-phase, with (active rows, kept blocks): 864 candidates of 36 blocks 155 / 165 us
-  // (100 %, 50 %), 273 / 295 (100 %, 100 %), 119 / 127 (75 %, 50 %), 62 / 59 (30 %, 50 %); 1000 of 25 blocks 106 / 113
-  // (75 %, 50 %), 56 / 54 (30 %, 50 %); 512 of 32 blocks 76 / 72 (75 %, 50 %), 44 / 41 (30 %, 50 %); 216 of 9 blocks
-  // 31 / 27.  What it needs besides: partial results of two shares per CU, room in LDS for a row's list (the
-  // longest row is bounded by all keep bits where there are several requests), 32-bit copy offsets.
-  const int64_t nkv = a.max_nnz / (a.batch == 1 ? n_cand : a.symbol_heads), span = (nkv + 1) * kBlockKV * 2;
-  const bool pipe = 2 * n_cand >= int64_t(5) * fo_num_cu() && nkv <= kMaxRowBlocksOneGroupDirect &&
-                    2 * fo_num_cu() <= kMaxShares && a.split_ws_bytes >= 2 * fo_sparse_fa_split_workspace_bytes() &&
-                    span * a.k_stride_n < (int64_t(1) << 32) && span * a.v_stride_n < (int64_t(1) << 32);
-  if (pipe) {
+  if (n_cand > direct_max_cand(false)) {
+    if (packed)
+      return bf16 ? launch<__bf16, false, false, false, 1, true, true, false, true, false, true>(p, n_cand, s)
+                  : launch<_Float16, false, false, false, 1, true, true, false, true, false, true>(p, n_cand, s);
+    return bf16 ? launch<__bf16, false, false, false, 1, true, false, false, true, false, true>(p, n_cand, s)
+                : launch<_Float16, false, false, false, 1, true, false, false, true, false, true>(p, n_cand, s);
+  }
+  if (direct_pipe(a, fo_num_cu())) {
     if (packed)
       return bf16 ? launch<__bf16, false, false, false, 1, true, true, false, true>(p, n_cand, s)
                   : launch<_Float16, false, false, false, 1, true, true, false, true>(p, n_cand, s);

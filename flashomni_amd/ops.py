@@ -12,7 +12,7 @@ table and the work-list buffers).  ``batch_sparseFA_with_kv_plan`` builds it and
 address of the integer workspace it was given; ``batch_sparseFA_with_ragged_kv_run`` finds it there,
 as the reference's run finds its tile arrays inside that workspace.  plan() allocates (it is not
 part of a captured graph in the reference either, flashomni/attention.py:140-141); run() allocates the
-work list when a plan first needs one (more than 1024 (q block, head) pairs).
+work list when a plan first needs one (a list that the attention launch does not take from the symbols).
 """
 import collections
 import weakref

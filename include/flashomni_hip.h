@@ -175,7 +175,7 @@ int fo_decode_sparse(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
  * fo_decode_sparse of what the last fo_sparse_attention_direct on the same `sched` computed, if that is newer
  * than the list: sched[33] is 0 (every decode leaves it so) and the list stays, or 1 and the symbols given here
  * are decoded (the ones that launch kept), or 2 and every bit counts as set.  For callers that cannot know which
- * of two launches came last, because graphs hold them.  1 to 1024 (q block, head) pairs.
+ * of two launches came last, because graphs hold them.  1 to fo_sparse_attention_direct_max_pairs() (q block, head) pairs.
  * ------------------------------------------------------------------------------------------- */
 int fo_decode_sparse_kept(const uint8_t* sparse_info, const uint8_t* sparse_kv_info,
                           const int32_t* sparse_info_indptr, const int32_t* sparse_kv_info_indptr,
@@ -332,7 +332,8 @@ int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, 
  * The same attention straight from the packed symbols, without a decoded list: short lists whose rows
  * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
- * candidates, more than 2^20 keep bits, no split workspace of fo_sparse_fa_split_workspace_bytes() bytes.
+ * candidates (1792 in the software-pipelined form, 1408 where is_full), more than 2^20 keep bits, no split workspace of
+ * fo_sparse_fa_split_workspace_bytes() bytes.
  * With twice that many bytes, from 2.5 candidates per CU on and where a row has at most 1024 kv blocks (of one
  * request: the share of keep bits of a candidate; of several: all kv blocks), the launch runs in the
  * software-pipelined form, two workgroups per CU.
@@ -365,6 +366,7 @@ typedef struct fo_attention_args {
 } fo_attention_args;
 enum { FO_NOT_DIRECT = 1 };
 int fo_sparse_attention_direct_serves(const void* args);  /* 1: fo_sparse_attention_direct takes the batch */
+int32_t fo_sparse_attention_direct_max_pairs(void);       /* ... and never one of more (symbol row, head) pairs */
 int fo_sparse_attention_direct(const void* args);
 
 /* ---------------------------------------------------------------------------------------------

@@ -15,7 +15,7 @@ CASES = [
     ([640], [20000], 1, 1.0),                 # 5 rows of ~80 kept blocks: eight parts each
     ([300, 1, 128, 1000, 129], [77, 513, 128, 1100, 64], 3, 0.6),
     ([2048], [300], 64, 0.7),                 # 1024 candidates, ~720 rows: even shares
-    ([2049], [300], 64, 0.7),                 # 1088 candidates: decoded
+    ([2049], [300], 64, 0.7),                 # 1088 candidates
     ([1200, 900], [1300, 2500], 24, 0.95),    # more rows than workgroups, rows cut at share boundaries
     ([512], [512], 2, 0.0),                   # nothing to compute
     # 640 candidates and more: two workgroups per CU
@@ -86,6 +86,51 @@ def test_schedule_of_short_lists(dev, case, is_full):
     test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
 
 
+@pytest.mark.parametrize("case", [
+    ([2049], [300], 64, 0.7),                  # 1088 candidates: five per thread
+    ([3584], [300], 64, 0.9),                  # 1792, seven per thread, ~1610 rows (every row: decoded)
+    ([3585], [300], 64, 0.9),                  # 1856: decoded
+    ([2816], [300], 64, 0.9),                  # 1408 (every row, too)
+    ([3000, 1, 2300], [1200, 770, 1000], 40, 0.8),   # 1720 of three requests
+    ([5500], [300], 24, 0.5),                  # 1032
+    ([8200], [300], 16, 0.0),                  # 1040, nothing to compute
+    ([4000], [9000], 33, 0.05),                # 1056 of 71 blocks, fewer rows than workgroups
+])
+@pytest.mark.parametrize("is_full", [False, True])
+def test_longer_lists_from_the_symbols(dev, case, is_full):
+    """1025 to 1792 candidates: seven to a thread at most, and only the rows of a workgroup's own share are in its table.
+    (Keys enough that no result reaches 2: the list's is compared to one bf16 step of what is smaller.)"""
+    test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
+
+
+@pytest.mark.parametrize("empty", ["all", "half", "most"])
+@pytest.mark.parametrize("tokens, heads", [(3584, 64), (5500, 24), (2048, 64), (2000, 64)])
+def test_shares_of_rows_without_blocks(dev, tokens, heads, empty):
+    """Rows that keep no kv block, which cost a share least: all of them, half of the heads, all but one: as the decoded list."""
+    import flashomni_amd as fo
+    kv, rows = 640, -(-tokens // 128)
+    keep = torch.zeros(rows, heads, 5, dtype=torch.bool)
+    if empty == "half":
+        keep[:, heads // 2:] = True
+    elif empty == "most":
+        keep[rows // 2, heads // 3] = True
+    ip = lambda n: torch.tensor([0, n], dtype=torch.int32, device=dev)
+    flags = torch.ones(rows * heads, dtype=torch.bool, device=dev)
+    info, info_ip = fo.segment_packbits(flags, ip(rows * heads), "little")
+    kv_info, kv_ip = fo.segment_packbits(keep.view(-1).to(dev), ip(keep.numel()), "little")
+    g = torch.Generator(device=dev).manual_seed(7)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for n in (tokens, kv, kv))
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(ip(tokens).cpu(), ip(kv).cpu(), heads, heads, 128, q_data_type=torch.bfloat16)
+    sym = (info, kv_info, info_ip, kv_ip)
+    out, lse = w.run(q, k, v, *sym, out=torch.full_like(q, 3.0), lse=torch.full((tokens, heads), 7.0, device=dev), return_lse=True)
+    w.decode(*sym)
+    exp, exp_lse = w.run(q, k, v, *sym, out=torch.full_like(q, 3.0), lse=torch.full((tokens, heads), 7.0, device=dev),
+                         return_lse=True, reuse_decoded=True)
+    assert max_abs(out.cpu(), exp.cpu()) <= 8e-3
+    assert torch.allclose(lse, exp_lse, atol=2e-3, rtol=1e-3)
+
+
 @pytest.mark.parametrize("group", [2, 7])
 def test_fresh_output_of_packed_tiles(dev, group):
     """Skipped tiles of grouped-query attention: the rows of a tile are spread over the group's q heads."""
@@ -110,7 +155,7 @@ def test_fresh_output_of_packed_tiles(dev, group):
                                   ([5000, 129, 1], [640, 300, 77], 8, 4, 0.3), ([9000], [300], 16, 1, 0.0)])
 @pytest.mark.parametrize("layout", ["NHD", "HND"])
 def test_fresh_output_of_decoded_lists(dev, case, layout):
-    """Lists above 1024 pairs: the decoder's launches clear the skipped rows of a fresh output (ragged last
+    """Lists above 1024 pairs: the launch, or above 1792 the decoder's launches, clear the skipped rows of a fresh output (ragged last
     tiles, tiles of grouped-query rows, nothing to compute); the same bits as over a cleared output."""
     import flashomni_amd as fo
     ql, kl, hkv, group, pa = case

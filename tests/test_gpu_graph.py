@@ -210,10 +210,12 @@ def test_captured_short_run_keeps_its_symbols_in_place(dev):
 class _ShortList:
     """Two short requests, a wrapper, and the result of every symbol set by the oracle."""
 
+    heads = 2
+
     def __init__(self, dev, seed):
         import flashomni_amd as fo
         import oracle
-        self.dev, heads, lens = dev, 2, [384, 130]
+        self.dev, heads, lens = dev, self.heads, [384, 130]
         g = torch.Generator().manual_seed(seed)
         q, k, v = (torch.randn(sum(lens), heads, 128, generator=g).to(torch.bfloat16) for _ in range(3))
         names = ("packed_info", "packed_keep", "info_indptr", "keep_indptr")
@@ -278,6 +280,17 @@ def test_captured_reuse_runs_the_list_of_the_moment(dev):
     s.run([None] * 4, is_full=True)
     s.check(s.full, reuse.replay)
     s.check(s.full, s.run, [None] * 4, reuse=True, is_full=True)
+
+
+class _LongerList(_ShortList):
+    heads = 206    # 1030 candidates: decoded, where a list is asked for, by three launches
+
+
+def test_captured_lists_of_three_launches(dev, monkeypatch):
+    """The same where what a run left behind is decoded by more than one launch, of which the device decides each."""
+    import sys
+    monkeypatch.setattr(sys.modules[__name__], "_ShortList", _LongerList)
+    test_captured_reuse_runs_the_list_of_the_moment(dev)
 
 
 def test_captured_decode_and_reuse(dev):
