@@ -738,7 +738,7 @@ sparse_fa_kernel(const FaParams p) {
     __builtin_amdgcn_s_waitcnt(0x0f70);
   };
   // ---- kDirect: rows straight from the packed symbols (short lists) ----
-  // Every workgroup reads all flags and keep bits itself, two or four candidates (symbol row, head) per
+  // Every workgroup reads all flags and keep bits itself, two, four or seven candidates (symbol row, head) per
   // thread in head-major order, and works out with two or three workgroup scans which rows or parts of rows
   // are its own.  A decode launch in front of this one costs 8-15 us and a launch gap at these sizes, most of
   // it latency of a single workgroup; here the same trips to memory (two, for a batch of one request) replace
@@ -747,7 +747,7 @@ sparse_fa_kernel(const FaParams p) {
   //     has kDirectMinPart kv blocks.  Where there are no more rows than workgroups and the longest part is
   //     no longer than an even share and what its cuts cost.
   //   * Even shares as the decoder lays them out (a row costs kShareRowCost + its kv blocks, a share is a range
-  //     of that cost), with the table of rows in LDS.  (154 rows of 260 kv blocks on 256 workgroups: 517 us as
+  //     of that cost), with the table of the share's rows in LDS.  (154 rows of 260 kv blocks on 256 workgroups: 517 us as
   //     whole rows, 338 in shares; 160 rows of 64 blocks 139 -> 92.)
   // In the pipelined form the next item is fetched beside a row's first copies instead of at its end, where the
   // trips to memory are 2.4 us that nothing hides.
