@@ -134,7 +134,7 @@ struct GemmParams {
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
   int32_t strip_cols;    // strips: column groups of XCDs
   int32_t strip_sorted;  // strips: token blocks with the most selected heads first
-  int32_t* judgement;    // strips: where judge_flags leaves its word, or null
+  int32_t* judgement;    // strips: where judge_flags leaves its word (GEMM-O) or quads whether they ran (GEMM-Q), or null
   int32_t judge_first, judge_bytes, judge_limit;
   int32_t n_win;         // windows of 16 token blocks per batch
   int32_t inline_cells;  // > 0: GEMM-Q builds its quad list itself from the flags of this many cells
@@ -464,6 +464,19 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
       pairs = (total >> 16) <= static_cast<int>(gridDim.x);
       total = pairs ? total >> 16 : total & 0xFFFF;
       incl = pairs ? incl >> 16 : incl & 0xFFFF;
+      if (p.judgement != nullptr) {  // (a launch of strips follows, which reads whose turn it is: launch_q)
+        int units = tid < p.inline_cells ? __popc(s_cell_mask[2 * tid]) + __popc(s_cell_mask[2 * tid + 1]) : 0;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) units += __shfl_xor(units, off, 64);
+        if (lane == 0) s_entry[wv] = units;
+        __syncthreads();
+        units = s_entry[0] + s_entry[1] + s_entry[2] + s_entry[3];
+        // (strips: half of a token block's two groups of columns will hold an odd number)
+        const int cus = gridDim.x, strips = (units + p.batch * p.n_row_tiles) / 2;
+        const bool mine = !pairs && total <= cus && strips > cus;
+        if (blockIdx.x == 0 && tid == 0) *p.judgement = mine;
+        if (!mine) return;
+      }
     }
     if (tid < kInlineCells) s_cell_pref[tid + 1] = incl;
     if (tid == 0) s_cell_pref[0] = 0;
@@ -2141,6 +2154,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
   const int l32 = lane & 31, g = lane >> 5;
   const int wr = wv >> 1, wc = wv & 1;  // half of the rows; column block
 
+  if (!kReduce && p.judgement != nullptr && *p.judgement != 0) return;  // (computed as quads)
   // ---- which strip ----
   const int xcd = blockIdx.x & (kXcds - 1), slot = blockIdx.x >> 3;
   const int cols = p.strip_cols;                 // column groups of XCDs
@@ -2758,7 +2772,15 @@ int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 //     by the kernel's own list, whose rounds last as long however few units they hold.  Strips over those, 10 .. 95 % flagged:
 //        8 heads, 4.4 to 15 units per CU  0.71 .. 1.18     16, 4.6 to 29  0.65 .. 1.05     24, 5.2 to 30  0.64 .. 1.06
 //       40, 5.6 to 16                     0.66 .. 1.02         to 24      0.71 .. 1.03         to 94      1.0 .. 1.36
-//     (above one where strips begin to share CUs, 257 to 300 of them; 3.4 to 4.4 units per CU 0.84 .. 1.13; 4 heads 1.1 .. 1.2).
+//     (3.4 to 4.4 units per CU 0.84 .. 1.13; 4 heads 1.1 .. 1.2).  With new inputs in every call strips are slower where they
+//     begin to share CUs and one round of quads still holds the units, 250 to 350 strips: 9000 x 3072 60 -> 67 us, 16 384 x 2048
+//     46 -> 52, 20 000 x 1024 up to 270 strips 23 -> 28.
+//   * Beyond 32 column blocks that is a wide range (8000 x 5120 from 19 to 29 % flagged, 5200 x 5120 from 30 to 47 %) and a large
+//     loss, so the quads are launched first: they count, run if one round holds them, but not items of two units nor strips
+//     a CU each, and leave in the scratch's first word whether they did; the strips behind them return if so.  us, strips alone ->
+//     this (quads alone): 8000 x 5120, 230 strips 81 -> 84 (80), 260 121 -> 105 (103), 300 134 -> 111 (113), 345 131 -> 122 (121), 400 138 ->
+//     142 (199); 5200 x 5120 80 -> 82 (81), 114 -> 100 (99), 122 -> 108 (107), 125 -> 115 (114), 133 -> 136 (204).  At 24 columns and
+//     fewer the two launches cost what they give (3 us of every call; 9000 x 3072, 230 / 260 / 400 strips 50 -> 52, 71 -> 64, 82 -> 86).
 //   * Dense: a quad per CU and round, so it depends on how full the rounds are.  Packed units up to 21 / 32 of them (over
 //     quads 0.75 .. 1.02), in a single round only up to K = 2048 (0.88 .. 1.01; 24 heads 1.05, 40 heads 1.07 .. 1.11).  Strips
 //     up to K = 512 (0.87 .. 0.95 over 2.9 to 23 units per CU) and where two quads' units per CU would be empty in the last
@@ -2769,13 +2791,18 @@ template <typename T, bool kHalf, bool kQuant>
 int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace, hipStream_t stream) {
   const int num_cu = fo_num_cu();
   if (num_cu <= 0) return fo::fail(FO_ERR_HIP, "gemm: no device");
+  bool strips = false;  // behind the quads, unless those run
   if constexpr (!kQuant) {
     const int64_t units = unit_count(gm);
     if (units <= num_cu) return launch_deep<T, false, kHalf, false, 1>(p, gm, stream);
     if (deep_strips(gm, p.k, false, num_cu)) return launch_deep<T, false, kHalf, false, 2>(p, gm, stream);
     if (units <= 2 * num_cu) return launch_units<T, false, kHalf, false>(p, gm, stream);
-    if (use_flags && 2 * units > 9 * num_cu && units <= (gm.n_col_tiles <= 32 ? 32 : 16) * num_cu && gm.n_col_tiles >= 6)
-      return launch_strips<T, false, kHalf, false>(p, gm, stream);
+    if (use_flags && 2 * units > 9 * num_cu && units <= (gm.n_col_tiles <= 32 ? 32 : 16) * num_cu && gm.n_col_tiles >= 6) {
+      if (static_cast<int64_t>(gm.batch) * gm.n_win * gm.n_cp > kInlineCells || gm.n_col_tiles <= 32)
+        return launch_strips<T, false, kHalf, false>(p, gm, stream);
+      strips = true;
+      p.judgement = static_cast<int32_t*>(workspace);  // (its first word: no list is made here)
+    }
     if (!use_flags) {
       const int64_t slots = quad_slots(gm, num_cu);
       const bool one_round = slots == 4 * num_cu;
@@ -2821,6 +2848,8 @@ int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace,
     p.inline_cells = static_cast<int32_t>(n_cells);
     gemm_kernel<T, kHalf, kQuant><<<static_cast<unsigned>(grid), kThreads, kSmemBytes, stream>>>(p);
     FO_CHECK_LAUNCH();
+    if constexpr (!kQuant)
+      if (strips) return launch_strips<T, false, kHalf, false>(p, gm, stream);
     return FO_OK;
   }
   int32_t* qoff = static_cast<int32_t*>(workspace);

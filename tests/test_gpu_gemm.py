@@ -92,6 +92,42 @@ def test_gemm_q_large_lists_with_column_strips(dev, case):
     assert rel_l2(out[active], exp[active]) <= REL_L2
 
 
+@pytest.mark.parametrize("shape", [(1, 4400, 4352, 34, 64), (1, 4401, 5248, 41, 96), (2, 2200, 4608, 36, 160)])
+@pytest.mark.parametrize("p", [0.0, 0.1, 0.45, 0.55, 0.9, 1.0])
+def test_flagged_gemm_q_as_quads_or_strips(dev, shape, p):
+    """Flagged GEMM-Q of 4.5 units per CU and more, wide: quads if one round holds them and items of two units would be more than
+    one, strips if not; the first launch leaves in the scratch's first word whether it ran.  Either way each wanted tile is
+    the fp32 product's, rounded once, and the others stay; the word, whatever it held, is written by every call."""
+    from flashomni_amd import _lib
+    batch, m, n, heads, k = shape
+    L, blocks = _lib.lib(), -(-m // 128)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    info, packed, indptr = _flags(batch, blocks, heads, p, seed=m)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(batch, m, k, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    need = L.fo_gemm_workspace_bytes(batch, m, n)
+    exp = (x.float() @ w.float().t())
+    on = torch.from_numpy(info).to(dev).bool().repeat_interleave(128, 1)[:, :m].repeat_interleave(128, 2)
+    units = int(info.astype(np.int64).sum())
+    for before in (0, 1):
+        ws = torch.full((need // 4,), before, dtype=torch.int32, device=dev)
+        y = torch.full((batch, m, n), -7.0, dtype=torch.bfloat16, device=dev)
+        _lib.check(L.fo_gemm_q(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), 0, batch, m, n, k, 128, heads, pk.data_ptr(),
+                               ip.data_ptr(), 0, 0, ws.data_ptr(), need, torch.cuda.current_stream(dev).cuda_stream))
+        assert bool((y[~on] == -7.0).all())
+        err = (y.float() - exp).abs() - 2.0 ** -8 * exp.abs() - k * 2.0 ** -24 * 16 * 0.05
+        assert not bool(on.any()) or float(err[on].max()) <= 0
+        if cus == 256:
+            if units > 4 * cus:   # more than a round of quads
+                assert int(ws[0]) == 0
+            elif units <= cus:    # items of at most two units fit a round
+                assert int(ws[0]) == 0
+            elif p == 0.45 and m == 4400:
+                assert int(ws[0]) == 1
+
+
 def test_gemm_q_is_full_equals_linear(dev):
     import flashomni_amd as fo
     x, w, b = _operands(1, 384, 256, 192, torch.bfloat16, seed=9)
