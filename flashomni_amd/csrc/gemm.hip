@@ -65,6 +65,7 @@
 // hit (measured at the Wan size: 6.8 GB fetched per launch against 28 GB of operand loads).
 #include "fo_common.h"
 #include "fo_device.h"
+#include "fo_flags.h"
 
 #include <type_traits>
 
@@ -2175,13 +2176,13 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
     constexpr int kTogether = 4;
     auto strips_of = [&](int first, int end, int (&n)[kTogether]) {
       const uint8_t* info[kTogether];
-      uint32_t lo[kTogether], hi[kTogether];
+      fo::FlagRange r[kTogether];
 #pragma unroll
       for (int q = 0; q < kTogether; ++q) {
         const int cell = min(first + q, end - 1), grp = cell / n_blocks;
-        info[q] = flags_of(cell - grp * n_blocks, &lo[q]);
-        hi[q] = lo[q] + group_begin(grp + 1);
-        lo[q] += group_begin(grp);
+        info[q] = flags_of(cell - grp * n_blocks, &r[q].lo);
+        r[q].hi = r[q].lo + group_begin(grp + 1);
+        r[q].lo += group_begin(grp);
         n[q] = 0;
       }
       if (p.head_dim == kTile) {  // (a flag per column block: four bytes of them at a time)
@@ -2190,28 +2191,21 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
           bool more = false;
 #pragma unroll
           for (int q = 0; q < kTogether; ++q) {
-            const uint32_t last = (hi[q] - 1) >> 3;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[q][u] = info[q][min((lo[q] >> 3) + at0 + u, last)];
-            more |= (lo[q] >> 3) + at0 + 4 <= last;
+            for (int u = 0; u < 4; ++u) v[q][u] = info[q][min(r[q].first() + at0 + u, r[q].last())];
+            more |= r[q].first() + at0 + 4 <= r[q].last();
           }
 #pragma unroll
-          for (int q = 0; q < kTogether; ++q) {
+          for (int q = 0; q < kTogether; ++q)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const uint32_t at = (lo[q] >> 3) + at0 + u;
-              if (at == lo[q] >> 3) v[q][u] &= 0xFFu << (lo[q] & 7);
-              if (at == hi[q] >> 3) v[q][u] &= (1u << (hi[q] & 7)) - 1u;
-              if (at <= (hi[q] - 1) >> 3) n[q] += __popc(v[q][u]);
-            }
-          }
+            for (int u = 0; u < 4; ++u) n[q] += __popc(r[q].trim(r[q].first() + at0 + u, v[q][u]));
           if (!more) break;
         }
       } else {
 #pragma unroll
         for (int q = 0; q < kTogether; ++q) {
-          const uint32_t c_lo = group_begin(min(first + q, end - 1) / n_blocks), row0 = lo[q] - c_lo;
-          for (uint32_t c = c_lo; c < hi[q] - row0; ++c) n[q] += flag_bit(info[q], row0 + c * kTile / p.head_dim);
+          const uint32_t c_lo = group_begin(min(first + q, end - 1) / n_blocks), row0 = r[q].lo - c_lo;
+          for (uint32_t c = c_lo; c < r[q].hi - row0; ++c) n[q] += flag_bit(info[q], row0 + c * kTile / p.head_dim);
         }
       }
 #pragma unroll
@@ -2298,14 +2292,10 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       for (int i = tid; i < n_blocks; i += kThreads) {
         const int b = i / p.n_row_tiles;
         const uint8_t* info = p.sparse_info + p.sparse_info_indptr[b];
-        const uint32_t lo = flag_row_of(i - b * p.n_row_tiles), hi = lo + n_slices;
+        const uint32_t row0 = flag_row_of(i - b * p.n_row_tiles);
+        const fo::FlagRange r{row0, row0 + n_slices};
         int ones = 0;
-        for (uint32_t at = lo >> 3; at <= (hi - 1) >> 3; ++at) {
-          uint32_t v = info[at];
-          if (at == lo >> 3) v &= 0xFFu << (lo & 7);
-          if (at == hi >> 3) v &= (1u << (hi & 7)) - 1u;
-          ones += __popc(v);
-        }
+        for (uint32_t at = r.first(); at <= r.last(); ++at) ones += __popc(r.trim(at, info[at]));
         if (p.flag) ones = n_slices - ones;
         const int key = n_slices < 64 ? ones : ones * 63 / n_slices;
         s_key[i] = static_cast<uint8_t>(key);

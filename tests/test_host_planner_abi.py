@@ -4,6 +4,7 @@ closed forms; workload generators hit the stated mask densities."""
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -206,6 +207,29 @@ def test_ops_fail_loudly_without_a_gpu_or_library(monkeypatch):
     monkeypatch.setattr(L, "LIB_PATH", "/nonexistent/libflashomni_hip.so")
     with pytest.raises(RuntimeError, match="no fallback"):
         L.lib()
+
+
+def test_flag_ranges(tmp_path):
+    """The bytes that the kernels read for a run of flags hold its bits and no others, and lie where they are: empty runs
+    too, at the beginning of the flags as well, where the byte of the last bit would be half a gigabyte behind them."""
+    src, so = tmp_path / "flags.cpp", tmp_path / "flags.so"
+    src.write_text('#include "fo_flags.h"\n'
+                   'extern "C" uint32_t first(uint32_t lo, uint32_t hi) { return fo::FlagRange{lo, hi}.first(); }\n'
+                   'extern "C" uint32_t last(uint32_t lo, uint32_t hi) { return fo::FlagRange{lo, hi}.last(); }\n'
+                   'extern "C" uint32_t trim(uint32_t lo, uint32_t hi, uint32_t at, uint32_t v) {\n'
+                   '  return fo::FlagRange{lo, hi}.trim(at, v);\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "flashomni_amd", "csrc"), str(src),
+                    "-o", str(so)], check=True)
+    h = ctypes.CDLL(str(so))
+    bits = np.random.default_rng(0).random(48) < 0.5
+    packed = np.packbits(bits, bitorder="little")
+    for lo in range(41):
+        for hi in range(lo, 41):
+            first, last = h.first(lo, hi), h.last(lo, hi)
+            assert (first, last) == (lo // 8, max(lo, hi - 1) // 8)
+            # (read a few at a time: the last byte again behind it)
+            ones = sum(bin(h.trim(lo, hi, at, int(packed[min(at, last)]))).count("1") for at in range(first, first + 8))
+            assert ones == bits[lo:hi].sum(), (lo, hi)
 
 
 def test_workload_mask_densities():
