@@ -62,10 +62,10 @@ SIGNATURES = {
     "fo_symbols_from_scores_uniform": ([c_vp, c_int] + [c_i32] * 6 + [c_vp, c_f32] * 2 + [c_vp] * 5, c_int),
 }
 
-# Entry points whose several launches hand something on in scratch memory that belongs to a stream (GEMM-Q's list,
-# GEMM-O's cursors and choice of form): called with the interpreter lock held, as the native call path does, so that the
-# launches of two threads' calls on one stream do not come to lie between each other.
-ONE_CALL_AT_A_TIME = ("fo_gemm_q", "fo_gemm_q_quant", "fo_gemm_o")
+# Entry points whose several launches hand something on in scratch memory that belongs to a stream (GEMM-Q's list, or the
+# word that says which of two forms computes the call): called with the interpreter lock held, as the native call path does,
+# so that the launches of two threads' calls on one stream do not come to lie between each other.
+ONE_CALL_AT_A_TIME = ("fo_gemm_q", "fo_gemm_q_quant")
 
 FO_BF16, FO_F16, FO_FP8_E4M3, FO_F32 = 0, 1, 2, 3
 FO_BIAS_NONE, FO_BIAS_VECTOR, FO_BIAS_MATRIX = 0, 1, 2

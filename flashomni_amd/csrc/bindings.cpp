@@ -201,12 +201,10 @@ PyObject* gemm_o(PyObject*, PyObject* const* args, Py_ssize_t n) {
     kind = FO_BIAS_MATRIX;
     if (bias->scalar_type() == at::kFloat) bias_code = FO_F32;
   }
-  Tensor y = new_tensor({batch, m, cols}, f32 ? at::kFloat : a->scalar_type(), dev), scratch;
-  void* stream = stream_of(dev);
-  if (!gemm_scratch(dev, stream, 256, &scratch)) return nullptr;
+  Tensor y = new_tensor({batch, m, cols}, f32 ? at::kFloat : a->scalar_type(), dev);
   if (fo_gemm_o(a->data_ptr(), b->data_ptr(), data(bias), y.data_ptr(), code, kind, bias_code, f32 ? FO_F32 : code, batch,
                 m, cols, k, q_size, heads, static_cast<const uint8_t*>(data(info)),
-                static_cast<const int32_t*>(data(indptr)), text, cache, scratch.data_ptr(), 256, stream))
+                static_cast<const int32_t*>(data(indptr)), text, cache, nullptr, 0, stream_of(dev)))
     return raise_last();
   return THPVariable_Wrap(std::move(y));
   TORCH_GUARD_END

@@ -135,8 +135,7 @@ struct GemmParams {
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
   int32_t strip_cols;    // strips: column groups of XCDs
   int32_t strip_sorted;  // strips: token blocks with the most selected heads first
-  int32_t* judgement;    // strips: where judge_flags leaves its word (GEMM-O) or quads whether they ran (GEMM-Q), or null
-  int32_t judge_first, judge_bytes, judge_limit;
+  int32_t* judgement;    // GEMM-Q: the word in which quads leave to the strips behind them whether they ran, or null
   int32_t n_win;         // windows of 16 token blocks per batch
   int32_t inline_cells;  // > 0: GEMM-Q builds its quad list itself from the flags of this many cells
   int32_t batch, m, n, k;
@@ -2102,46 +2101,6 @@ constexpr int kStripRing = 6;
 constexpr int kStripSorted = 4096;  // token blocks that are put in order
 constexpr int kStripSmemBytes = 2 * kUnitBytes + kStripRing * kStripPiece;  // 80 KB: two X tiles, the ring of W
 
-// Whether a long launch selects few of its heads, for the ninth word of a caller's scratch: with p of a request's head
-// slices selected, the sum of p (limit / 256 - p) over the requests is not negative.  Judged by up to 4096 bytes of flags in
-// all, of up to 64 requests spread over the batch, from each one's `first_byte` on (n_bytes: how many a request has), by
-// one workgroup; all of them are in flight together.
-constexpr int kJudged = 64, kJudgedBytes = 4096;
-__device__ __forceinline__ void judge_flags(const GemmParams& p, int32_t* s_ones) {
-  const int tid = threadIdx.x, judged = min(p.batch, kJudged);
-  int threads = kThreads;  // of a request: a power of two, at least kThreads / kJudged
-  while (threads * judged > kThreads) threads >>= 1;
-  constexpr int kPer = kJudgedBytes / kThreads;
-  const int n = min(p.judge_bytes, kPer * threads);
-  const int j = tid / threads, at = tid - j * threads;
-  int ones = 0;
-  if (j < judged) {
-    const uint8_t* info = p.sparse_info + p.sparse_info_indptr[static_cast<int64_t>(j) * p.batch / judged] + p.judge_first;
-    uint8_t v[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) v[i] = at + i * threads < n ? info[at + i * threads] : 0;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) ones += __popc(v[i]);
-  }
-  const int width = min(threads, 64);
-  for (int off = width >> 1; off > 0; off >>= 1) ones += __shfl_xor(ones, off, 64);
-  if (tid % width == 0) s_ones[tid / width] = ones;
-  __syncthreads();
-  if (tid < 64) {
-    // (up to 2^15 selected times 2^21: 64 bits)
-    long long few = 0;
-    if (tid < judged) {
-      int selected = 0;
-      for (int w = 0; w < threads / width; ++w) selected += s_ones[tid * (threads / width) + w];
-      if (p.flag) selected = 8 * n - selected;
-      few = static_cast<long long>(selected) * (p.judge_limit * n - 32 * selected);
-    }
-    for (int off = 32; off > 0; off >>= 1) few += __shfl_xor(few, off, 64);
-    if (tid == 0) *p.judgement = few >= 0;
-  }
-  __syncthreads();
-}
-
 template <typename T, bool kReduce, bool kHalf, bool kPartial>
 __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParams p) {
   using TT = Types<T>;
@@ -2281,7 +2240,6 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
   }
   if constexpr (kReduce) {
     const int rank = block;
-    if (p.judgement != nullptr && blockIdx.x == 0) judge_flags(p, reinterpret_cast<int32_t*>(smem));
     if (p.strip_sorted) {
       // token blocks with the most selected heads first
       uint8_t* const s_key = smem;
@@ -2741,15 +2699,6 @@ int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   if (unit_count(gm) <= 2 * num_cu) return launch_units<T, true, kHalf, kPartial>(p, gm, stream);
   if constexpr (!kHalf)
     if (p.k <= 512) return launch_packed<T, true, kPartial>(p, gm, stream);
-  // (launches that could be judged both ways: more than one round of quads, 13 heads over the width times the rounds' fill,
-  // 10 from sixteen units per CU on)
-  const int64_t slots = quad_slots(gm, num_cu), units = unit_count(gm);
-  const int64_t line = (units > 15 * num_cu ? 10 : 13) * 128 * 256 * slots / (p.k * units);
-  p.judge_limit = static_cast<int32_t>(line < 256 ? line : 256);  // of 256
-  if (kHalf || slots == 4 * num_cu || p.judge_limit < 32) p.judgement = nullptr;
-  p.judge_first = p.num_text_tokens / p.sparse_q_size * p.num_heads / 8;
-  const int64_t bytes = static_cast<int64_t>(p.m) / p.sparse_q_size * p.num_heads / 8;
-  p.judge_bytes = static_cast<int32_t>(bytes < kJudgedBytes ? bytes : kJudgedBytes);
   return launch_strips<T, true, kHalf, kPartial>(p, gm, stream);
 }
 
@@ -3011,9 +2960,6 @@ extern "C" int fo_gemm_o(const void* x, const void* w, const void* bias, void* y
   p.bias_kind = bias_kind;
   p.bias_f32 = bias_dtype == FO_F32;
   p.y_f32 = y_dtype == FO_F32;
-  p.judgement = workspace != nullptr && workspace_bytes >= 64 && (reinterpret_cast<uintptr_t>(workspace) & 3) == 0
-                    ? static_cast<int32_t*>(workspace) + 8
-                    : nullptr;
   const ListGeom gm = make_geom(batch, m, n);
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == FO_BF16 ? launch<__bf16, true>(p, gm, false, workspace, s)

@@ -49,7 +49,7 @@ def _symbols(sparse_info, sparse_info_indptr, device, name, batch, m, num_qo_hea
     return info, indptr
 
 
-# Scratch of the GEMMs (GEMM-Q's tile list, GEMM-O's word on the flags' density).  Eager calls share one
+# Scratch of GEMM-Q (its tile list, or the word by which two launches agree on the form).  Eager calls share one
 # buffer per (device, stream): calls on one stream run in order, calls on different streams may
 # overlap and get their own.  A call made while its stream is being captured into a graph gets a
 # buffer of its own from the allocator (the graph's memory pool then owns it for as long as the
@@ -229,15 +229,11 @@ def flashomni_gemm_reduction(
     info, indptr = _symbols(sparse_info, sparse_info_indptr, A.device, "flashomni_gemm_reduction",
                             Bsz, M, num_qo_heads, num_text_tokens, sparse_q_size)
     L = _lib.lib()
-    # (the reduction visits every token block and needs no tile list; long launches leave a word on the flags'
-    # density in the stream's scratch buffer)
-    stream = _lib.current_stream(A.device)
-    ws_bytes = 256
-    workspace = _gemm_workspace(A.device, stream, ws_bytes)
+    # (the reduction visits every token block: no tile list, no scratch)
     with _lib.device_guard(A.device):
         _lib.check(L.fo_gemm_o(
             _lib.ptr(A), _lib.ptr(B), _lib.ptr(bias), _lib.ptr(out), _lib.dtype_code(A.dtype), kind,
             bias_code, _lib.dtype_code(out_dtype), Bsz, M, N, A.shape[2], sparse_q_size, num_qo_heads,
             _lib.ptr(info), _lib.ptr(indptr), num_text_tokens, int(bool(is_for_cache)),
-            _lib.ptr(workspace), ws_bytes, stream))
+            None, 0, _lib.current_stream(A.device)))
     return out

@@ -401,9 +401,8 @@ int fo_gemm_q(const void* x, const void* w, const void* bias, void* y, int dtype
  * bias_dtype: the activation dtype (as in the reference) or FO_F32 for the matrix form;
  * y_dtype: the activation dtype or FO_F32 (so a cached partial can stay in fp32).
  * hd must be a multiple of 32.  No tile list is needed (every token block is visited, the tile
- * order is computed arithmetically), so `workspace` may be NULL; fo_gemm_q with is_full != 0
- * likewise.  Given 64 bytes or more of 4-byte-aligned device scratch, a call of more than one round of four tiles (128 x
- * 128) per CU leaves in its ninth word whether the flags select few of the heads (1) or many (0), which chooses nothing.
+ * order is computed arithmetically): `workspace` may be NULL and is neither read nor written; fo_gemm_q with
+ * is_full != 0 likewise.
  * fo_gemm_q's workspace holds a call's tile list: calls that share it must not overlap in time, and none of their launches
  * may come to lie between another one's: on one stream that means that host threads make them one at a time.
  * ------------------------------------------------------------------------------------------- */

@@ -445,13 +445,28 @@ def test_video_gemms_sampled_token_blocks(dev):
         assert rel_l2(got_final, exp_final) <= REL_L2, iy
 
 
+def _check_gemm_o_rows(got, x, w, bias, info, text, cache, rows, hd):
+    """Rows of a pass over x [batch, m, k] against the fp32 product of the heads that it selects (info: [batch, blocks, heads])."""
+    for b in range(x.size(0)):
+        on = torch.from_numpy(info[b, (np.array(rows) + text) // 128]).to(x.device).repeat_interleave(hd, 1)
+        exp = (x[b, rows].float() * (~on if cache else on)) @ w.float().t()
+        if bias is not None:
+            exp = exp + (bias.float() if bias.dim() == 1 else bias[b, rows].float())
+        scale = max(1.0, float(exp.abs().max()) / 2)
+        assert max_abs(got[b, rows].cpu(), exp.cpu()) <= MAX_ABS * scale, b
+        assert rel_l2(got[b, rows].cpu(), exp.cpu()) <= REL_L2, b
+
+
+def _some_rows(m, step):
+    return sorted({0, 1, 127, 128, m // 2, m - 1} | set(range(5, m, step)))
+
+
 @pytest.mark.parametrize("shape", [(1, 22016, 3072, 24), (2, 43800, 768, 8)])
-def test_gemm_o_cursors_and_fixed_stride_agree(dev, shape):
-    """A long GEMM-O launch hands out its work items through cursors when it is given scratch memory and
-    in fixed strides when it is not: the order of the work items changes, no result may.  (M = 22016:
-    86 row pairs x 12 column pairs, four work items per CU; the second shape has two batch entries, a
-    ragged last token block and heads of width 96, i.e. slabs that count for one half only.  The
-    wrapper passes scratch, the bare entry point here gets none.)"""
+def test_long_gemm_o_leaves_scratch_alone(dev, shape):
+    """Long launches, both passes: rows of every part of the output against the selected heads' fp32 product, and the
+    same bits whether the entry point is given scratch memory, which it neither reads nor writes, or none.  (22016 x 3072: 172
+    token blocks, 2064 strips; the second shape has two batch entries, a ragged last token block and heads of width 96,
+    i.e. slabs that count for one half only.)"""
     import flashomni_amd as fo
     from flashomni_amd import _lib
     batch, m, n, heads = shape
@@ -462,17 +477,22 @@ def test_gemm_o_cursors_and_fixed_stride_agree(dev, shape):
     b = (torch.randn(n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
     pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
     code = _lib.dtype_code(torch.bfloat16)
+    rows = _some_rows(m, 997)
     for is_for_cache, bias, kind in ((True, b, _lib.FO_BIAS_VECTOR), (False, None, _lib.FO_BIAS_MATRIX)):
         if bias is None:
             bias = got_cache
         got = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 0, bias=bias, is_for_cache=is_for_cache)
-        bare = torch.full_like(got, -3.0)
-        with _lib.device_guard(dev):
-            _lib.check(_lib.lib().fo_gemm_o(
-                _lib.ptr(x), _lib.ptr(w), _lib.ptr(bias), _lib.ptr(bare), code, kind, code, code, batch, m, n, n,
-                128, heads, _lib.ptr(pk), _lib.ptr(ip), 0, int(is_for_cache), None, 0, _lib.current_stream(dev)))
-        torch.cuda.synchronize()
-        assert torch.equal(got.view(torch.int16), bare.view(torch.int16))
+        for word in (7, 0):
+            scratch = torch.full((64,), word, dtype=torch.int32, device=dev)
+            bare = torch.full_like(got, -3.0)
+            with _lib.device_guard(dev):
+                _lib.check(_lib.lib().fo_gemm_o(
+                    _lib.ptr(x), _lib.ptr(w), _lib.ptr(bias), _lib.ptr(bare), code, kind, code, code, batch, m, n, n,
+                    128, heads, _lib.ptr(pk), _lib.ptr(ip), 0, int(is_for_cache), _lib.ptr(scratch), 256,
+                    _lib.current_stream(dev)))
+            assert torch.equal(got.view(torch.int16), bare.view(torch.int16))
+            assert bool((scratch == word).all())
+        _check_gemm_o_rows(got, x, w, bias, info, 0, is_for_cache, rows, n // heads)
         got_cache = got
     # and the end result is the dense layer
     dense = F.linear(x[0, :256].float(), w.float(), b.float()).cpu()
@@ -639,60 +659,34 @@ def test_dense_gemm_q_as_strips(dev, shape, dtype):
 
 @pytest.mark.parametrize("p_active", [0.0, 0.05, 0.35, 0.65, 0.95, 1.0])
 @pytest.mark.parametrize("text", [0, 256])
-def test_gemm_o_form_chosen_on_the_device(dev, p_active, text):
-    """Long GEMM-O launches are queued in two forms, of which the flags' density lets one run: both passes at
-    densities on either side of the line, none and all selected, against the same call without scratch memory, which
-    is always computed as quads."""
-    from flashomni_amd import _lib
-    L = _lib.lib()
-    m, n, heads = 16384 - 5, 1024, 8          # 1024 units
-    batch = 3                                 # 3072: quads fill their rounds
+def test_long_gemm_o_at_every_density(dev, p_active, text):
+    """Both passes of a long call of eight heads, none to all of them selected, flags from a text token on: rows of
+    every part against the selected heads' fp32 product."""
+    import flashomni_amd as fo
+    m, n, heads, batch = 16384 - 5, 1024, 8, 3
     info, packed, indptr = _flags(batch, (text + m + 127) // 128, heads, p_active, seed=int(100 * p_active) + text)
     g = torch.Generator(device=dev).manual_seed(text)
     x = torch.randn(batch, m, n, generator=g, device=dev).to(torch.bfloat16)
     w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
     pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
-    ws = torch.full((64,), 7, dtype=torch.int32, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    for cache in (1, 0):
-        outs = []
-        for scratch, size in ((ws.data_ptr(), 256), (None, 0), (ws.data_ptr(), 256)):
-            y = torch.full((batch, m, n), 7.0, dtype=torch.bfloat16, device=dev)
-            _lib.check(L.fo_gemm_o(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), 0, 0, 0, 0, batch, m, n, n, 128, heads,
-                                   pk.data_ptr(), ip.data_ptr(), text, cache, scratch, size, stream))
-            outs.append(y)
-        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
-
-
-def _gemm_o_rule(n_cu, batch, m, n):
-    """launch_half's rule for heads of 128: (packed whatever the flags, quads whatever the flags, line between them)."""
-    rows, cols = -(-m // 128), n // 128
-    units, quads = batch * rows * cols, batch * (cols // 2) * (rows // 16 * 8 + (rows % 16 + 1) // 2)
-    rounds = -(-quads // n_cu)
-    slots = 4 * n_cu * rounds
-    if rounds == 1:
-        return units <= 3 * n_cu, units > 3 * n_cu, 0
-    limit = min(256, (10 if units > 15 * n_cu else 13) * 128 * 256 * slots // (n * units))
-    packed = n <= 2048 or 32 * units <= 21 * slots or n * units <= 18 * 128 * slots
-    return packed, not packed and limit < 32, limit
+    for cache in (True, False):
+        y = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, text, is_for_cache=cache)
+        _check_gemm_o_rows(y, x, w, None, info, text, cache, _some_rows(m, 501), 128)
 
 
 @pytest.mark.parametrize("shape,p_active", [
     ((8192, 2560), (0.05, 0.95, 0.95)), ((8192, 2560), (0.95, 0.05, 0.05)), ((8192, 2560), (0.1, 0.3, 0.2)),
     ((8192, 2560), (0.9, 0.7, 0.8)), ((8192, 2560), (0.0, 0.0, 0.0)), ((8192, 2560), (1.0, 1.0, 1.0)),
-    ((512, 2560), (0.05,) * 35 + (0.9,) * 35),   # more requests than are judged
+    ((512, 2560), (0.05,) * 35 + (0.9,) * 35),
     ((9609, 3072), (0.5,)), ((9609, 3072), (0.8,)),
 ])
-def test_gemm_o_form_of_a_mixed_batch(dev, shape, p_active):
-    """Where the flags choose the form of a long GEMM-O call they do so for all requests (up to 64 of them, spread over
-    the batch): the choice in the scratch's ninth word is the rule's, and the results are those of the quads (the form
-    of a call without scratch), bit for bit, in either pass."""
-    from flashomni_amd import _lib
-    L = _lib.lib()
+def test_gemm_o_of_a_mixed_batch(dev, shape, p_active):
+    """Requests of unlike densities in one call, whose token blocks are put in order of their selected heads across the
+    batch: each request's rows against the selected heads' fp32 product, and the same bits as the request by itself (512
+    tokens: a workgroup per unit there), in either pass."""
+    import flashomni_amd as fo
     batch, (m, n), text = len(p_active), shape, 128
     heads, blocks = n // 128, -(-m // 128)
-    packed, quads, limit = _gemm_o_rule(torch.cuda.get_device_properties(dev).multi_processor_count, batch, m, n)
-    assert not packed and not quads, "not a shape of both forms"
     flags = np.concatenate([_flags(1, blocks + 1, heads, p, seed=7 + i)[0] for i, p in enumerate(p_active)])
     segs = [np.packbits(f.reshape(-1).astype(np.uint8), bitorder="little") for f in flags]
     info, indptr = np.concatenate(segs), np.cumsum([0] + [len(s) for s in segs]).astype(np.int32)
@@ -700,22 +694,13 @@ def test_gemm_o_form_of_a_mixed_batch(dev, shape, p_active):
     x = torch.randn(batch, m, n, generator=g, device=dev).to(torch.bfloat16)
     w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(torch.bfloat16)
     pk, ip = torch.from_numpy(info).to(dev), torch.from_numpy(indptr).to(dev)
-    ws = torch.full((64,), 7, dtype=torch.int32, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    judged = [j * batch // min(batch, 64) for j in range(min(batch, 64))]
-    first = heads // 8                                     # byte that the text block's flags end in
-    n_bytes = min(m // 128 * heads // 8, 4096, 16 * (256 // (1 << (len(judged) - 1).bit_length())))
-    for cache in (1, 0):
-        outs = []
-        for scratch, size in ((ws.data_ptr(), 256), (None, 0)):
-            y = torch.full((batch, m, n), 7.0, dtype=torch.bfloat16, device=dev)
-            _lib.check(L.fo_gemm_o(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), 0, 0, 0, 0, batch, m, n, n, 128, heads,
-                                   pk.data_ptr(), ip.data_ptr(), text, cache, scratch, size, stream))
-            outs.append(y)
-        assert torch.equal(outs[0], outs[1])
-        ones = [int(np.unpackbits(segs[j][first:first + n_bytes]).sum()) for j in judged]
-        selected = [8 * n_bytes - o if cache else o for o in ones]
-        assert int(ws[8]) == int(sum(s * (limit * n_bytes - 32 * s) for s in selected) >= 0)
+    for cache in (True, False):
+        y = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, text, is_for_cache=cache)
+        _check_gemm_o_rows(y, x, w, None, flags, text, cache, _some_rows(m, 701), 128)
+        for i in sorted({0, batch // 2, batch - 1}) if batch > 1 else ():
+            one = fo.flashomni_gemm_reduction(x[i:i + 1].contiguous(), w, heads, pk, ip[i:i + 2].contiguous(), text,
+                                              is_for_cache=cache)
+            assert torch.equal(one[0], y[i]), i
 
 
 @pytest.mark.parametrize("shape", [(1, 6200, 1536), (1, 6300, 1536), (1, 16100, 2048), (1, 8185, 3072), (2, 3300, 2560),

@@ -81,8 +81,7 @@ def test_captured_layer_pass_replays(dev):
 
 
 def test_captured_long_gemm_o_replays(dev):
-    """A GEMM-O launch long enough to hand out its work items through cursors (four items or more per CU):
-    the kernel that clears the cursors is captured with it, so every replay starts from zero.  Flags and
+    """A GEMM-O launch of many strips, whose order the kernel works out from the flags.  Flags and
     activations are rewritten in place between replays; each replay equals the eager call of that moment."""
     import flashomni_amd as fo
     m, n, heads = 22016, 3072, 24

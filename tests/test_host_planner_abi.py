@@ -34,16 +34,16 @@ def test_library_exports_every_declared_symbol():
 
 
 def test_gemm_calls_keep_the_interpreter_lock():
-    """GEMM-Q and GEMM-O hand lists, cursors and a choice of form from one launch to the next in scratch that belongs to
-    the stream: the launches of two host threads' calls must not mix, so ctypes may not let go of the lock."""
+    """GEMM-Q hands lists and a choice of form from one launch to the next in scratch that belongs to the stream: the
+    launches of two host threads' calls must not mix, so ctypes may not let go of the lock.  (GEMM-O is one launch.)"""
     from _ctypes import FUNCFLAG_PYTHONAPI
     L = _lib()
     for name, (argtypes, restype) in L.SIGNATURES.items():
         fn = getattr(L.lib(), name)
-        assert bool(fn._flags_ & FUNCFLAG_PYTHONAPI) == (name in ("fo_gemm_q", "fo_gemm_q_quant", "fo_gemm_o")), name
+        assert bool(fn._flags_ & FUNCFLAG_PYTHONAPI) == (name in ("fo_gemm_q", "fo_gemm_q_quant")), name
         assert list(fn.argtypes) == argtypes and fn.restype is restype
     with pytest.raises(RuntimeError):  # (and the error codes come back as from the others)
-        L.check(L.lib().fo_gemm_o(*[None if t is ctypes.c_void_p else 0 for t in L.SIGNATURES["fo_gemm_o"][0]]))
+        L.check(L.lib().fo_gemm_q(*[None if t is ctypes.c_void_p else 0 for t in L.SIGNATURES["fo_gemm_q"][0]]))
 
 
 _C_SCALARS = {"int": ctypes.c_int, "int32_t": ctypes.c_int32, "uint32_t": ctypes.c_uint32,
