@@ -102,7 +102,7 @@ class PlannedBatch:
 
     def __init__(self, float_workspace_buffer, qo_indptr_host, kv_indptr_host, qo_indptr_dev,
                  kv_indptr_dev, num_qo_heads, num_kv_heads, block_q, block_kv, share_rows=True,
-                 worklist=None, gqa_packed=False, send=(0, None, None, None)):
+                 worklist=None, gqa_packed=False, send=(0, None, None, None), q_dtype=None, logits_soft_cap=0.0):
         self.device = float_workspace_buffer.device
         self.float_ws = float_workspace_buffer
         self.num_qo_heads, self.num_kv_heads = num_qo_heads, num_kv_heads
@@ -120,9 +120,13 @@ class PlannedBatch:
         # tensors given to run() must have (checked there without reading the device): token counts,
         # and the packed bytes of the byte-aligned per-request segments.
         index = self.device.index if self.device.index is not None else torch.cuda.current_device()
+        self.share_rows = share_rows
+        self.split_ok = self._split_ws_ok()
+        # (the symbols of runs that never take their rows straight from them need no room)
+        direct_ws = self.float_ws_bytes() if self.split_ok and (q_dtype is None or q_dtype.itemsize == 2) else 0
         self.native, self.tables, sizes = _lib.native().plan(
             qo_indptr_host, kv_indptr_host, num_qo_heads, num_kv_heads, self.gqa_packed, index,
-            qo_indptr_dev, kv_indptr_dev, *send)
+            qo_indptr_dev, kv_indptr_dev, *send, direct_ws, float(logits_soft_cap))
         (self.n_q_blk, self.n_kv_blk, self.max_rows, self.max_nnz, self.total_q_rows, self.total_kv_rows,
          self.min_info_bytes, self.min_kv_info_bytes, self.max_kv_len, *self._table_at) = sizes
         self.qo_indptr = self._table(0) if qo_indptr_dev is None else qo_indptr_dev
@@ -134,8 +138,6 @@ class PlannedBatch:
             self._list = None
         if self._list is not None:
             self._list.use_sched(self._sched())
-        self.share_rows = share_rows
-        self.split_ok = self._split_ws_ok()
         self.no_room = False  # the allocator has refused the scratch of a widened k
         # [is_full, stream, streams already ordered after it] of the list the work-list buffers hold
         self.decoded = None
@@ -608,7 +610,8 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
                 num_kv_heads, sparse_block_size_for_q, sparse_block_size_for_kv, share_rows=self._share_rows,
                 worklist=self._planned._list if self._planned is not None else None,
                 gqa_packed=gqa_symbols != "per_q_head",
-                send=(sent, self._int_workspace_buffer, self._pin_memory_int_workspace_buffer, self._pin_ring))
+                send=(sent, self._int_workspace_buffer, self._pin_memory_int_workspace_buffer, self._pin_ring),
+                q_dtype=q_data_type, logits_soft_cap=logits_soft_cap)
             self._plan_info = plan_info
         if not graph:
             self._qo_indptr_buf, self._kv_indptr_buf = self._planned.qo_indptr, self._planned.kv_indptr

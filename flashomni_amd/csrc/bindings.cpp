@@ -310,7 +310,9 @@ struct Plan {
   // listed_in: the capture whose last launch on this plan was a decode; recorded_in, recorded_full: the last
   // capture that recorded a decode or run, and its is_full.
   // recording: the last launch was recorded.
-  int captured, recorded_full, recording;
+  // taken: rows have been taken straight from the symbols, or a graph holds a launch that does so.  Until then
+  // there is nothing that could be newer than the list.
+  int captured, recorded_full, recording, taken;
   unsigned long long listed_in, recorded_in;
   // The copy lies behind the tables, in one place for as long as the plan lives (a graph writes it at every
   // replay): room for the symbols that such a run takes, at keep_at[0] info, [1] kv_info, [2] the indptrs (bytes
@@ -353,6 +355,7 @@ unsigned long long capture_of(hipStream_t stream) {
 void note(Plan* p, hipStream_t stream, int state, bool full) {
   const unsigned long long id = capture_of(stream);
   p->recording = id != 0;
+  if (state) p->taken = 1;
   if (id) {
     p->captured = 1;
     p->recorded_in = id;
@@ -542,13 +545,15 @@ PyObject* enter_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // (qo_indptr, kv_indptr: int32 on the host; num_qo_heads, num_kv_heads, packed, device index,
-//  qo_indptr, kv_indptr of the device or None; and, to send host_plan()'s arrays: their bytes, the integer
-//  workspace, its pinned mirror and the mirror's Ring, or 0 and None) -> (Plan, tables, sizes)
+//  qo_indptr, kv_indptr of the device or None; to send host_plan()'s arrays: their bytes, the integer
+//  workspace, its pinned mirror and the mirror's Ring, or 0 and None; and bytes of the float workspace, 0: no room for
+//  parts of rows or operands that are always decoded, and the soft cap) -> (Plan, tables, sizes)
 PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_BEGIN
   const Tensor *qo, *kv, *qo_dev, *kv_dev, *iws, *pin;
-  int64_t hq, hkv, dev, sent;
-  if (!(n == 12 && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
+  int64_t hq, hkv, dev, sent, ws_bytes;
+  double cap;
+  if (!(n == 14 && whole(args[12], &ws_bytes) && real(args[13], &cap) && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
         whole(args[3], &hkv) && whole(args[5], &dev) && whole(args[8], &sent) && opt_tensor(args[9], &iws) &&
         opt_tensor(args[10], &pin) && (sent == 0 || (iws && pin && Py_TYPE(args[11]) == g_ring_type)) &&
         opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
@@ -581,7 +586,9 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   p->state = 0;
   int rc = 0;
   int64_t ints = z.table_ints;
-  if (z.max_rows > 0 && z.max_rows <= fo_sparse_attention_direct_max_pairs() && z.max_nnz <= (1 << 20) && z.max_kv_len <= kMaxListed) {
+  if (z.max_rows <= fo_sparse_attention_direct_max_pairs() && z.max_kv_len <= kMaxListed &&
+      fo_sparse_attention_direct_may_serve(static_cast<int32_t>(z.n_q_blocks), p->symbol_heads, batch, z.max_nnz, ws_bytes,
+                                           static_cast<float>(cap))) {
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     // (symbol tensors much larger than the batch needs are not worth copying)
     p->keep_room[0] = z.min_info + 4096;
@@ -734,7 +741,9 @@ PyObject* list_source(PyObject*, PyObject* arg) {
   Plan* p = reinterpret_cast<Plan*>(arg);
   const unsigned long long id = capture_of(static_cast<hipStream_t>(stream_of(p->dev)));
   if (id) p->captured = 1;
-  const int source = !p->keep_at[0] || (id && p->listed_in == id) ? 0 : p->captured ? 2 : p->state != 0;
+  // (a reuse that is recorded now may be replayed behind a run that takes its rows from the symbols later on)
+  const bool list = !p->keep_at[0] || (id ? p->listed_in == id : !p->taken);
+  const int source = list ? 0 : p->captured ? 2 : p->state != 0;
   return Py_BuildValue("(iK)", source, id);
   TORCH_GUARD_END
 }

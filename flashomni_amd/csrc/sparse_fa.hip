@@ -2823,25 +2823,46 @@ bool direct_table_holds(int64_t n_cand, int64_t max_nnz, int num_cu) {
           (4 * longest / 9 + 2) / kRowOverheadPipe + 3 < kDirectShareRows);
 }
 
+// Whether the launch takes its rows straight from the symbols.
+// Candidates that a workgroup's threads can go through at the top of a launch, and keep bits that every workgroup can
+// afford to read (2^20 bits = 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also
+// sorts their rows by head, so that one head's K and V at a time are in an XCD's L2: the more of a row's blocks are kept, the
+// earlier.  The lists that only the pipelined form takes, decoded -> straight from the symbols, us per call (rows, blocks kept):
+//   1032 candidates of 43 blocks  72 -> 62 (50, 10 %)  189 -> 170 (75, 50)  446 -> 383 (all)     1040 of 26  53 -> 44 (30, 5)
+//   1320 of 55                    71 -> 65 (20, 20)    273 -> 260 (75, 50)  654 -> 593 (all)     1040 of 65  101 -> 89 (70, 10)
+//   1536 of 64 to 192             256 -> 235 (70, 10)  759 -> 773 (100, 30) 779 -> 817, 1152 -> 1200 (all)
+//   1704 of 71                    210 -> 194 (50, 30)  427 -> 421 (75, 50)  971 -> 1008 (all)
+//   2040 of 85                    256 -> 246 (100, 10) 560 -> 573 (75, 50)  1356 -> 1420 (all)
+bool direct_takes(const fo_attention_args& a, int variant) {
+  const int num_cu = fo_num_cu();
+  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  return (a.dtype == FO_BF16 || a.dtype == FO_F16) && variant != 1 && n_cand >= 1 &&
+         (n_cand <= direct_max_cand(false) ||
+          (n_cand <= (a.is_full ? kDirectMaxFull : direct_max_cand(true)) && variant == 0 && direct_pipe(a, num_cu) &&
+           direct_table_holds(n_cand, a.max_nnz, num_cu))) &&
+         a.max_nnz <= (1 << 20) && num_cu >= 16 && num_cu <= kMaxShares &&
+         a.split_ws_bytes >= fo_sparse_fa_split_workspace_bytes();
+}
+
 }  // namespace
 
 extern "C" int fo_sparse_attention_direct_serves(const void* args) {
   const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
-  const int num_cu = fo_num_cu();
-  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
-  // Candidates that a workgroup's threads can go through at the top of a launch, and keep bits that every workgroup can
-  // afford to read (2^20 bits = 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also
-  // sorts their rows by head, so that one head's K and V at a time are in an XCD's L2: the more of a row's blocks are kept, the
-  // earlier.  The lists that only the pipelined form takes, decoded -> straight from the symbols, us per call (rows, blocks kept):
-  //   1032 candidates of 43 blocks  72 -> 62 (50, 10 %)  189 -> 170 (75, 50)  446 -> 383 (all)     1040 of 26  53 -> 44 (30, 5)
-  //   1320 of 55                    71 -> 65 (20, 20)    273 -> 260 (75, 50)  654 -> 593 (all)     1040 of 65  101 -> 89 (70, 10)
-  //   1536 of 64 to 192             256 -> 235 (70, 10)  759 -> 773 (100, 30) 779 -> 817, 1152 -> 1200 (all)
-  //   1704 of 71                    210 -> 194 (50, 30)  427 -> 421 (75, 50)  971 -> 1008 (all)
-  //   2040 of 85                    256 -> 246 (100, 10) 560 -> 573 (75, 50)  1356 -> 1420 (all)
-  return (a.dtype == FO_BF16 || a.dtype == FO_F16) && g_variant.load(std::memory_order_relaxed) != 1 && n_cand >= 1 &&
-         (n_cand <= direct_max_cand(false) ||
-          (n_cand <= (a.is_full ? kDirectMaxFull : direct_max_cand(true)) && g_variant.load(std::memory_order_relaxed) == 0 && direct_pipe(a, num_cu) && direct_table_holds(n_cand, a.max_nnz, num_cu))) &&
-         a.max_nnz <= (1 << 20) && num_cu >= 16 && num_cu <= kMaxShares && a.split_ws && a.split_ws_bytes >= fo_sparse_fa_split_workspace_bytes() && (reinterpret_cast<uintptr_t>(a.split_ws) & 15) == 0;
+  return direct_takes(a, g_variant.load(std::memory_order_relaxed)) && a.split_ws &&
+         (reinterpret_cast<uintptr_t>(a.split_ws) & 15) == 0;
+}
+
+extern "C" int fo_sparse_attention_direct_may_serve(int32_t n_blk, int32_t symbol_heads, int32_t batch, int64_t max_nnz,
+                                                    int64_t split_ws_bytes, float logits_soft_cap) {
+  fo_attention_args a{};  // (the rest at its most favourable)
+  a.dtype = FO_BF16;
+  a.n_blk = n_blk;
+  a.symbol_heads = symbol_heads;
+  a.batch = batch;
+  a.max_nnz = max_nnz;
+  a.split_ws_bytes = split_ws_bytes;
+  a.logits_soft_cap = logits_soft_cap;
+  return direct_takes(a, 0);
 }
 
 extern "C" int32_t fo_sparse_attention_direct_max_pairs(void) { return direct_max_cand(true); }

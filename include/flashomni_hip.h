@@ -367,6 +367,9 @@ typedef struct fo_attention_args {
 enum { FO_NOT_DIRECT = 1 };
 int fo_sparse_attention_direct_serves(const void* args);  /* 1: fo_sparse_attention_direct takes the batch */
 int32_t fo_sparse_attention_direct_max_pairs(void);       /* ... and never one of more (symbol row, head) pairs */
+/* 0: no 16-bit call over such a batch, with such a workspace and soft cap, is ever taken, whatever its strides and is_full */
+int fo_sparse_attention_direct_may_serve(int32_t n_blk, int32_t symbol_heads, int32_t batch, int64_t max_nnz,
+                                         int64_t split_ws_bytes, float logits_soft_cap);
 int fo_sparse_attention_direct(const void* args);
 
 /* ---------------------------------------------------------------------------------------------

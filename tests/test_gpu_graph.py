@@ -292,6 +292,81 @@ def test_captured_lists_of_three_launches(dev, monkeypatch):
     test_captured_reuse_runs_the_list_of_the_moment(dev)
 
 
+@pytest.mark.parametrize("why, heads", [("fp8", 2), ("fp8", 206), ("soft cap", 206), ("small workspace", 2),
+                                        ("small workspace", 206), ("no sharing", 2), ("no sharing", 206)])
+def test_reuse_behind_a_capture_of_lists_that_are_always_decoded(dev, why, heads, monkeypatch):
+    """A plan whose rows are never taken straight from the symbols (fp8, a soft cap on more than 1024 pairs, no room for parts
+    of rows) has nothing that could be newer than its list: a capture costs later reuses, eager and recorded ones, no launch."""
+    import flashomni_amd as fo
+    from flashomni_amd import _lib
+    n, soft = 514, why == "soft cap"
+    g = torch.Generator(device=dev).manual_seed(5)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    m = make_ragged_masks([384, 130], [384, 130], heads, 0.7, 0.6, seed=5)
+    sym = [torch.from_numpy(m[s]).to(dev) for s in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    indptr = torch.from_numpy(m["qo_indptr"])
+    kw = {}
+    if why == "fp8":
+        q, kw["q_scale"] = fo.quant_fp8_block(q, indptr)
+        k, kw["k_scale"] = fo.quant_fp8_block(k, indptr)
+    room = 128 << 20
+    if why == "small workspace":  # (from 1025 pairs on the launch needs twice as much)
+        room = (2 if heads > 2 else 1) * _lib.lib().fo_sparse_fa_split_workspace_bytes() - 16
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(room, dtype=torch.uint8, device=dev))
+    if why == "no sharing":
+        w._share_rows = False
+    w.plan(indptr, indptr, heads, heads, 128, q_data_type=q.dtype, logits_soft_cap=30.0 if soft else None)
+    kept = []
+    monkeypatch.setattr(_lib.lib(), "fo_decode_sparse_kept", lambda *a: kept.append(a) or 0)
+    run = lambda **more: w.run(q, k, v, *sym, out=torch.zeros_like(v), **kw, **more)
+    exp = run()
+    out = torch.zeros_like(v)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        w.run(q, k, v, *sym, out=out, **kw)
+        w.run(q, k, v, *sym, out=out, reuse_decoded=True, **kw)
+    again = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(again):
+        w.run(q, k, v, *sym, out=out, reuse_decoded=True, **kw)
+    assert torch.equal(run(reuse_decoded=True), exp)
+    for what in (graph, again):
+        out.zero_()
+        what.replay()
+        assert torch.equal(out, exp)
+    assert not kept
+
+
+def test_reuse_behind_a_capture_before_rows_came_from_the_symbols(dev, monkeypatch):
+    """Where they can be taken from them but have not been, eagerly or in a graph, an eager reuse makes no launch either; one
+    that a graph holds looks at every replay, since a run may come in between."""
+    from flashomni_amd import _lib
+    s = _ShortList(dev, 33)
+    lib, kept = _lib.lib(), []
+    launch = lib.fo_decode_sparse_kept
+    monkeypatch.setattr(lib, "fo_decode_sparse_kept", lambda *a: kept.append(a) or launch(*a))
+    a, b, c = s.sym
+    s.w.decode(*a)
+    torch.cuda.synchronize()
+    decode = s.capture(lambda: s.w.decode(*s.buf))
+    s.check(s.exp[0], s.run, a, reuse=True)
+    assert not kept
+    reuse = s.capture(lambda: s.run(a, reuse=True))
+    assert len(kept) == 1
+    s.check(s.exp[0], s.run, a, reuse=True)
+    assert len(kept) == 1
+    s.run(b)
+    s.check(s.exp[1], reuse.replay)
+    s.run(c)
+    s.check(s.exp[2], s.run, c, reuse=True)
+    assert len(kept) == 2
+    for dst, src in zip(s.buf, b):
+        dst.copy_(src)
+    decode.replay()
+    s.check(s.exp[1], s.run, b, reuse=True)
+    s.check(s.exp[1], reuse.replay)
+
+
 def test_captured_decode_and_reuse(dev):
     """decode() on a second stream and reuse of its list in one graph (no launch but those two), also on a plan that
     has not run before; a reuse made before the first replay computes nothing."""
