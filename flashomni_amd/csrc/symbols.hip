@@ -21,8 +21,11 @@
 
 namespace {
 
-constexpr int kThreads = 512;
-constexpr int kWaves = kThreads / 64;
+// Threads of a workgroup whose lanes hold E entries of a row each.  At 48 entries the registers leave room for three wavefronts
+// on a SIMD, of which workgroups of eight would use two (8 heads of 3000 x 3000 in fp32 357 us, of four 327; at 24, with room
+// for five: 198 and 210 the other way, 24 heads of 1500 x 1500).
+constexpr int kMaxThreads = 512;
+constexpr int threads_of(int E) { return E == 48 ? 256 : kMaxThreads; }
 constexpr int kRowsPerGroup = 8;
 constexpr unsigned kShortLaunch = 512;  // workgroups; from two per CU on the vector ALUs are busy throughout
 constexpr int kMaxBlocks = 4096;
@@ -193,6 +196,7 @@ __host__ __device__ inline QJobLayout q_job_layout(int n_q, int n_k, int text_kv
 
 template <typename T, int E>
 __device__ __forceinline__ void q_symbols_job(const ProducerArgs& a, int b, uint8_t* lds) {
+  constexpr int kThreads = threads_of(E), kWaves = kThreads / 64;
   const QJobLayout lay = q_job_layout(a.n_q, a.n_k, a.text_kv);
   const int width = lay.width, parts = lay.parts;
   float* s_part = reinterpret_cast<float*>(lds);
@@ -211,7 +215,7 @@ __device__ __forceinline__ void q_symbols_job(const ProducerArgs& a, int b, uint
     float acc[kItems][kFlight];
     const T* col[kItems];
     int rows[kItems], h[kItems], q[kItems];
-    int most = 0;
+    int most = 0, least = n_rows;
 #pragma unroll
     for (int t = 0; t < kItems; ++t) {
       const int item = min(item0 + t * kWaves, n_items - 1), c = item / parts, part = item - c * parts;
@@ -220,22 +224,43 @@ __device__ __forceinline__ void q_symbols_job(const ProducerArgs& a, int b, uint
       h[t] = rows[t] ? part / a.text_q : 0;
       q[t] = rows[t] ? part - h[t] * a.text_q : 0;
       most = max(most, rows[t]);
+      least = min(least, rows[t]);
 #pragma unroll
       for (int u = 0; u < kFlight; ++u) acc[t][u] = 0.f;
     }
-    for (int i = 0; i < most; i += kFlight) {
+    auto next_row = [&](int t) __attribute__((always_inline)) {
+      const T* at = col[t] + (static_cast<int64_t>(h[t]) * a.n_q + q[t]) * a.n_k;
+      h[t] += step_h;
+      q[t] += step_q;
+      if (q[t] >= a.text_q) {
+        q[t] -= a.text_q;
+        ++h[t];
+      }
+      return at;
+    };
+    // Eight rows of either subset, asked for without a condition: under one, a 16-bit value is waited for before the next is
+    // asked for (bf16, 40 heads of 595 x 595: 83 -> 71 us; and 66 with the rows of the kv symbols likewise, which take fp32's time
+    // then: 24 heads of 1500 x 1500 267 -> 198).
+    int i = 0;
+    for (; i + kFlight <= least; i += kFlight) {
+      T v[kItems][kFlight];
+#pragma unroll
+      for (int t = 0; t < kItems; ++t)
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) v[t][u] = *next_row(t);
+#pragma unroll
+      for (int t = 0; t < kItems; ++t)
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) acc[t][u] += to_f32(v[t][u]);
+    }
+    for (; i < most; i += kFlight) {
       float v[kItems][kFlight];
 #pragma unroll
       for (int t = 0; t < kItems; ++t)
 #pragma unroll
         for (int u = 0; u < kFlight; ++u) {
-          v[t][u] = i + u < rows[t] ? to_f32(col[t][(static_cast<int64_t>(h[t]) * a.n_q + q[t]) * a.n_k]) : 0.f;
-          h[t] += step_h;
-          q[t] += step_q;
-          if (q[t] >= a.text_q) {
-            q[t] -= a.text_q;
-            ++h[t];
-          }
+          const T* at = next_row(t);
+          v[t][u] = i + u < rows[t] ? to_f32(*at) : 0.f;
         }
 #pragma unroll
       for (int t = 0; t < kItems; ++t) {
@@ -297,7 +322,8 @@ __device__ __forceinline__ void q_symbols_job(const ProducerArgs& a, int b, uint
 // run beside the rest); every other workgroup makes the kv symbols of eight consecutive
 // (q_block, head) rows of a request ------------------------------------------------------------------
 template <typename T, int E>
-__global__ void __launch_bounds__(kThreads) symbols_kernel(ProducerArgs a, int groups_per_request) {
+__global__ void __launch_bounds__(kMaxThreads) symbols_kernel(ProducerArgs a, int groups_per_request) {
+  constexpr int kThreads = threads_of(E), kWaves = kThreads / 64;
   extern __shared__ __align__(16) uint8_t s_flags[];  // kv job: kRowsPerGroup * n_k (+8) keep flags
   if (static_cast<int>(blockIdx.x) < a.batch) {
     q_symbols_job<T, E>(a, blockIdx.x, s_flags);
@@ -324,10 +350,14 @@ __global__ void __launch_bounds__(kThreads) symbols_kernel(ProducerArgs a, int g
       continue;
     }
     const T* src = base + (static_cast<int64_t>(h) * a.n_q + qb) * a.n_k;
+    // (without a condition, see the q job; what lies behind the row's end is not looked at)
+    T from_mem[E];
     float score[E];
     bool drop[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) score[e] = e * 64 + lane < a.n_k ? to_f32(src[e * 64 + lane]) : 0.f;
+    for (int e = 0; e < E; ++e) from_mem[e] = src[min(e * 64 + lane, a.n_k - 1)];
+#pragma unroll
+    for (int e = 0; e < E; ++e) score[e] = to_f32(from_mem[e]);
     select_low_mass<E>(score, a.n_k, a.kv_threshold ? a.kv_threshold[h] : a.kv_value, lane, short_launch, drop);
 #pragma unroll
     for (int e = 0; e < E; ++e)
@@ -357,7 +387,7 @@ int launch_both(const ProducerArgs& a, hipStream_t stream) {
   size_t lds = static_cast<size_t>(kRowsPerGroup) * a.n_k + 8;
   const size_t lds_q = q_job_layout(a.n_q, a.n_k, a.text_kv).bytes;
   if (lds_q > lds) lds = lds_q;
-  symbols_kernel<T, E><<<a.batch * (groups + 1), kThreads, lds, stream>>>(a, groups);
+  symbols_kernel<T, E><<<a.batch * (groups + 1), threads_of(E), lds, stream>>>(a, groups);
   FO_CHECK_LAUNCH();
   return FO_OK;
 }

@@ -155,6 +155,28 @@ def test_one_threshold_for_all(dev, shape):
         fo.sparse_symbols_from_scores(x, t2t, 1e60, 0.3)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 24, 36, 36, 4), (2, 3, 9, 7, 1), (1, 40, 70, 66, 3), (1, 12, 595, 595, 4), (1, 5, 1030, 1030, 9),
+                                   (1, 3, 2049, 2049, 4), (1, 2, 3073, 3072, 5), (1, 1, 3100, 3074, 20), (1, 4, 64, 64, 0)])
+def test_16_bit_scores_are_their_fp32_values(dev, shape, dtype):
+    """Scores in 16 bits give the bytes of the same values in fp32, which the tests above hold against the oracle: subsets of
+    text rows of fewer than eight, of eight at a time and a rest, with and without text, rows whose last 64 are not all there,
+    of up to 64 entries per lane (at 48 of them workgroups are half as large)."""
+    import flashomni_amd as fo
+    B, H, NQ, NK, t2t = shape
+    x = torch.randn(B, H, NQ, NK, generator=torch.Generator().manual_seed(NK)).to(dtype).to(dev)
+    got = fo.sparse_symbols_from_scores(x, t2t, 0.3, 0.25)
+    expect = fo.sparse_symbols_from_scores(x.float(), t2t, 0.3, 0.25)
+    for g, e in zip(got, expect):
+        assert torch.equal(g, e)
+    _, got_kv = _unpack(got, B, H, NQ, NK)
+    scores = x.float().cpu().numpy()[:, :, t2t:].reshape(-1, NK)
+    thr = np.full(len(scores), 0.25, dtype=np.float32)
+    lo, hi = producer.selection_bounds(scores, thr, EPS)
+    n = (got_kv[:, :, t2t:] == 0).sum(axis=-1).reshape(-1)
+    assert ((lo <= n) & (n <= hi)).all()
+
+
 def test_symbols_feed_the_decoder(dev):
     """The packed output is what run()/decode() read: decoding it lists the kept blocks."""
     import flashomni_amd as fo
