@@ -827,12 +827,10 @@ sparse_fa_kernel(const FaParams p) {
   constexpr int kCands = kMaxCand / (64 * kWaves);  // candidates of a thread, at most
   auto direct_schedule = [&]() {
     const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads, dir_g = dir_index();
-    // (No more of them than it takes: the schedule is bound by the instructions of its two wavefronts per SIMD, not by
-    // its trips to memory.  With this, the symbols' copy below off the critical path and a whole part's list made from keep
-    // bits that are at hand: 384 tokens x 2 heads 15.8 -> 15.1 us a call, 13 711 x 226 tokens x 3 heads 14.1 -> 13.5,
-    // 2764 x 3 heads 26.8 -> 26.3.)
-    const int per_thread = part_of(n_cand - 1, 64 * kWaves) + 1;
-    const int first_cand = per_thread * tid;
+    // (All of a thread's candidates, also where it does not have as many: with a branch around each of those, their loads are
+    // waited for one after the other and their instructions do not mix.  9000 tokens x 8 heads over 500 29.6 -> 29.1 us, 808
+    // candidates of five requests 36.7 -> 35.7, 6600 x 24 53.6 -> 51.4; 6 candidates 14.9 either way.)
+    const int first_cand = kCands * tid;
     if (tid < kItemBatch) s_items[tid].row = -1;
     if (tid == 0) s_next_row[0].row = -1;
     int list_at[kCands];  // where a candidate's keep bits are in LDS (words from smem on), or -1
@@ -847,10 +845,6 @@ sparse_fa_kernel(const FaParams p) {
       int req[kCands], bit[kCands];
 #pragma unroll
       for (int u = 0; u < kCands; ++u) {
-        if (u >= per_thread) {
-          req[u] = bit[u] = 0;
-          continue;
-        }
         const int cand = min(first_cand + u, n_cand - 1);
         const int h = part_of(cand, p.n_blk), t = cand - h * p.n_blk;
         req[u] = p.batch == 1 ? 0 : p.blk_req[t];
@@ -865,9 +859,6 @@ sparse_fa_kernel(const FaParams p) {
       }
 #pragma unroll
       for (int u = 0; u < kCands; ++u) {
-        act[u] = false;
-        n[u] = nkv[u] = 0;
-        if (u >= per_thread) continue;
         nkv[u] = (p.kv_indptr[req[u] + 1] - p.kv_indptr[req[u]] + kBlockKV - 1) / kBlockKV;
         act[u] = first_cand + u < n_cand;
         n[u] = act[u] ? nkv[u] : 0;
@@ -877,8 +868,6 @@ sparse_fa_kernel(const FaParams p) {
         uint8_t flags[kCands];
 #pragma unroll
         for (int u = 0; u < kCands; ++u) {
-          keep_at[u] = flags[u] = 0;
-          if (u >= per_thread) continue;
           keep_at[u] = p.kv_info_indptr[req[u]];
           flags[u] = p.info[p.info_indptr[req[u]] + (bit[u] >> 3)];
         }
@@ -932,11 +921,6 @@ sparse_fa_kernel(const FaParams p) {
           uint32_t v[kCands][kAhead];
 #pragma unroll
           for (int u = 0; u < kCands; ++u) {
-            if (u >= per_thread) {
-#pragma unroll
-              for (int i = 0; i < kAhead; ++i) v[u][i] = 0u;
-              continue;
-            }
             const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
 #pragma unroll
             for (int i = 0; i < kAhead; ++i) v[u][i] = i < r.count() && nkv[u] > 0 ? r.words[i] : 0u;
@@ -946,7 +930,6 @@ sparse_fa_kernel(const FaParams p) {
             list_at[u] = -1;
 #pragma unroll
             for (int i = 0; i < kAhead; ++i) own[u][i] = v[u][i];
-            if (u >= per_thread) continue;
             const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
             act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
             n[u] = 0;
@@ -993,7 +976,7 @@ sparse_fa_kernel(const FaParams p) {
       int skipped = first_cand - row;
 #pragma unroll
       for (int u = 0; u < kCands; ++u)
-        if (u < per_thread && first_cand + u < n_cand && !act[u]) {
+        if (first_cand + u < n_cand && !act[u]) {
           const int turn = part_of(skipped, n_wg);
           if (skipped - turn * n_wg == dir_g) s_zero[turn] = static_cast<uint16_t>(first_cand + u);
           ++skipped;
@@ -1040,7 +1023,9 @@ sparse_fa_kernel(const FaParams p) {
         int parts[kCands], first = row;
 #pragma unroll
         for (int u = 0; u < kCands; ++u) parts[u] = act[u];
-        if (longest < max_n) {
+        // (where no row is cut a part is a row, and the scan is left out: 6 candidates 15.5 -> 15.2 us; in the pipelined form,
+        // whose four wavefronts are through with it sooner, the branch costs more than it saves: 808 candidates 36.4 -> 36.0 with it)
+        if (kPipe || longest < max_n) {
           int parts_mine = 0;
 #pragma unroll
           for (int u = 0; u < kCands; ++u) {

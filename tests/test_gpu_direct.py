@@ -72,8 +72,8 @@ def test_rows_from_the_symbols(dev, case, is_full, dtype):
 
 
 @pytest.mark.parametrize("case", [
-    ([2048], [300], 32, 0.4),                              # 512 candidates, one per thread
-    ([2048], [300], 33, 0.4),                              # 528, two per thread
+    ([2048], [300], 32, 0.4),                              # 512 candidates: half of the threads have two each
+    ([2048], [300], 33, 0.4),                              # 528
     ([128] + [100] * 40, [26000] + [64] * 40, 2, 0.8),     # a row of 204 keep bits among short ones: read where they are
     ([640], [12200], 3, 0.8),                              # 96 bits: three words of a thread, or four by their alignment
     ([2048], [20000], 8, 0.6),                             # kept symbols copied by two workgroups
@@ -81,14 +81,14 @@ def test_rows_from_the_symbols(dev, case, is_full, dtype):
 ])
 @pytest.mark.parametrize("is_full", [False, True])
 def test_schedule_of_short_lists(dev, case, is_full):
-    """The lines inside the schedule of a short list: candidates per thread, where a row's keep bits are found, what a
-    workgroup copies of the symbols that a later decode reads."""
+    """The lines inside the schedule of a short list: threads with and without candidates, where a row's keep bits are found,
+    what a workgroup copies of the symbols that a later decode reads."""
     test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
 
 
 @pytest.mark.parametrize("case", [
-    ([2049], [300], 64, 0.7),                  # 1088 candidates: five per thread
-    ([3584], [300], 64, 0.9),                  # 1792, seven per thread, ~1610 rows (every row: decoded)
+    ([2049], [300], 64, 0.7),                  # 1088 candidates, seven to a thread
+    ([3584], [300], 64, 0.9),                  # 1792, ~1610 rows (every row: decoded)
     ([3585], [300], 64, 0.9),                  # 1856: decoded
     ([2816], [300], 64, 0.9),                  # 1408 (every row, too)
     ([3000, 1, 2300], [1200, 770, 1000], 40, 0.8),   # 1720 of three requests
