@@ -151,15 +151,19 @@ def test_fresh_output_of_packed_tiles(dev, group):
     assert torch.equal(w.run(q, k, v, *sym), exp)
 
 
-@pytest.mark.parametrize("case", [([2000, 1, 130, 1500], [300, 77, 513, 640], 40, 1, 0.5),
-                                  ([5000, 129, 1], [640, 300, 77], 8, 4, 0.3), ([9000], [300], 16, 1, 0.0)])
+@pytest.mark.parametrize("case", [([2000, 1, 130, 1500], [300, 77, 513, 640], 40, 1, 0.5), ([2000, 1, 130, 1500], [300, 77, 513, 640], 64, 1, 0.5),
+                                  ([5000, 129, 1], [640, 300, 77], 8, 4, 0.3), ([5000, 129, 1], [640, 300, 77], 12, 4, 0.3),
+                                  ([9000], [300], 16, 1, 0.0), ([9000], [300], 26, 1, 0.0)])
 @pytest.mark.parametrize("layout", ["NHD", "HND"])
-def test_fresh_output_of_decoded_lists(dev, case, layout):
-    """Lists above 1024 pairs: the launch, or above 1792 the decoder's launches, clear the skipped rows of a fresh output (ragged last
-    tiles, tiles of grouped-query rows, nothing to compute); the same bits as over a cleared output."""
+def test_fresh_output_of_longer_lists(dev, case, layout):
+    """Lists above 1024 pairs, taken from the symbols, and above 1792, decoded: the launch, or the decoder's launches, clear
+    the skipped rows of a fresh output (ragged last tiles, tiles of grouped-query rows, nothing to compute); the same bits as
+    over a cleared output."""
     import flashomni_amd as fo
+    from flashomni_amd import _lib
     ql, kl, hkv, group, pa = case
     hq = hkv * group
+    pairs = sum(-(-n * group // 128) for n in ql) * hkv
     m = make_ragged_masks([n * group for n in ql], kl, hkv, pa, 0.5, seed=6)
     qo = torch.from_numpy(np.concatenate([[0], np.cumsum(ql)]).astype(np.int32))
     g = torch.Generator(device=dev).manual_seed(6)
@@ -170,6 +174,8 @@ def test_fresh_output_of_decoded_lists(dev, case, layout):
     w.plan(qo, t("kv_indptr"), hq, hkv, 128, q_data_type=torch.bfloat16)
     sym = [t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
     exp = w.run(q, k, v, *sym, out=torch.zeros_like(q))
+    decoded = w._planned.native.state == 0
+    assert decoded == (pairs > _lib.lib().fo_sparse_attention_direct_max_pairs())
     for _ in range(3):
         junk = torch.full((256 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
         del junk

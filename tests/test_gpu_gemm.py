@@ -263,11 +263,12 @@ def test_flux_gemm_o_full_config(dev):
     assert max_abs(final, dense) <= MAX_ABS and rel_l2(final, dense) <= REL_L2
 
 
-@pytest.mark.parametrize("shape", [(2, 2500, 384, 256), (1, 4224, 640, 128), (3, 130, 128, 64)])
+@pytest.mark.parametrize("shape", [(2, 2500, 384, 256), (1, 4224, 640, 128), (3, 130, 128, 64), (2, 10500, 1408, 576)])
 def test_dense_tile_enumeration_geometries(dev, shape):
     """Every unit computed (is_full GEMM-Q, GEMM-O): the kernel enumerates its tiles arithmetically.
     More than one 16-block window, a short last window, an odd number of column tiles, a token
-    tail and several batches; every output element must be written and right."""
+    tail and several batches; every output element must be written and right.  (Up to 256 units one to a CU; the last
+    shape as quads, GEMM-O as strips.)"""
     import flashomni_amd as fo
     batch, m, n, k = shape
     heads = n // 128
@@ -458,7 +459,7 @@ def _check_gemm_o_rows(got, x, w, bias, info, text, cache, rows, hd):
 
 
 def _some_rows(m, step):
-    return sorted({0, 1, 127, 128, m // 2, m - 1} | set(range(5, m, step)))
+    return sorted(r for r in {0, 1, 127, 128, m // 2, m - 1} | set(range(5, m, step)) if r < m)
 
 
 @pytest.mark.parametrize("shape", [(1, 22016, 3072, 24), (2, 43800, 768, 8)])
@@ -502,12 +503,11 @@ def test_long_gemm_o_leaves_scratch_alone(dev, shape):
 @pytest.mark.parametrize("case", [(1, 128, 1), (129, 128, 1), (1100, 64, 4), (1100, 128, 8), (2176, 96, 4), (3000, 256, 8),
                                   (130, 32, 12)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_workgroup_per_unit_equals_quads(dev, case, dtype):
-    """Launches of few units give each a workgroup of its own, longer ones compute quads: the same
-    inputs alone (few units) and as one of many batch entries (more than two units per CU) give the same
-    bits, because both add a unit's k steps in the same order.  One and two token rows past a block,
-    heads of 32 to 256 columns (slabs that count for one half only), every unit of the chip in use
-    (3000 x 2048: 384 units)."""
+def test_few_units_equal_many(dev, case, dtype):
+    """Launches of up to two units per CU give a unit or a pair of them a CU of its own, longer ones compute quads, strips or
+    (GEMM-O up to 512 columns) packed units: the same inputs alone and as one of many batch entries give the same bits,
+    because all add a unit's k steps in the same order.  One and two token rows past a block, heads of 32 to 256 columns (slabs
+    that count for one half only), every unit of the chip in use (3000 x 2048: 384 units, 192 pairs)."""
     import flashomni_amd as fo
     m, hd, heads = case
     n = heads * hd
@@ -542,38 +542,122 @@ def test_workgroup_per_unit_equals_quads(dev, case, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("case", [(1100, 128, 8, 8, 25), (130, 64, 16, 33, 128), (1025, 256, 5, 6, 20)])
+@pytest.mark.parametrize("case", [(1100, 8, 8, 25), (130, 8, 33, 128), (1025, 10, 6, 20)])
 def test_packed_units_equal_quads(dev, case, dtype):
-    """Launches whose quads would fill their rounds badly run four workgroups of one unit each on a CU, better
-    filled ones quads: the same inputs as a few batch entries and as one of many give the same bits.  One and two
-    token rows past a block, an odd number of row and column blocks, heads of 64 to 256 columns."""
+    """Dense GEMM-Q whose quads would fill their rounds badly runs four workgroups of one unit each on a CU, a better
+    filled one quads: the same inputs as a few batch entries and as one of many give the same bits.  One and two token rows
+    past a block, an odd number of row and column blocks."""
     import flashomni_amd as fo
-    m, hd, heads, few, many = case
-    n = heads * hd
+    m, cols, few, many = case
+    n = cols * 128
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    rows, cols = -(-m // 128), n // 128
+    rows = -(-m // 128)
     fill = lambda batch: batch * rows * cols / (4 * cus * -(-batch * ((cols + 1) // 2) * ((rows + 1) // 2) // cus))
     if cus == 256:
         assert few * rows * cols > 2 * cus and fill(few) <= 42 / 64 and fill(many) > 49 / 64
-    info, packed, indptr = _flags(many, rows + 1, heads, 0.6, seed=m + hd)
     g = torch.Generator(device=dev).manual_seed(m)
     x = torch.randn(many, m, n, generator=g, device=dev).to(dtype)
     w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(dtype)
     b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
-    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
-
-    def chain(x, ip):
-        full = fo.flashomni_gemm(x, w, heads, num_text_tokens=0, bias=b, is_full=True)
-        part = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=b, is_for_cache=True)
-        part32 = fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, is_for_cache=True, out_dtype=torch.float32)
-        return [full, part, part32, fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part),
-                fo.flashomni_gemm_reduction(x, w, heads, pk, ip, 128, bias=part32)]
-
-    everything = chain(x, ip)
-    for k, (one, all_) in enumerate(zip(chain(x[:few].contiguous(), ip[:few + 1].contiguous()), everything)):
-        assert torch.equal(one, all_[:few]), k
+    full = lambda x: fo.flashomni_gemm(x, w, cols, num_text_tokens=0, bias=b, is_full=True)
+    one, everything = full(x[:few].contiguous()), full(x)
+    assert torch.equal(one, everything[:few])
     ref = torch.nn.functional.linear(x[:few].float(), w.float(), b.float())
-    assert rel_l2(everything[0][:few], ref) <= REL_L2
+    assert rel_l2(one, ref) <= REL_L2
+
+
+def _chain_of_passes(x, w, b, heads, pk, ip, text):
+    """GEMM-O's cache pass with either output type and the final pass over either."""
+    import flashomni_amd as fo
+    o = lambda bias, cache, dtype=None: fo.flashomni_gemm_reduction(x, w, heads, pk, ip, text, bias=bias, is_for_cache=cache,
+                                                                    out_dtype=dtype)
+    part, part32 = o(b, True), o(b, True, torch.float32)
+    return [part, part32, o(part, False), o(part32, False, torch.float32)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [(8500, 128, 4, 2), (4000, 64, 6, 6), (9001, 128, 2, 4), (1, 128, 4, 140), (2100, 64, 6, 11)])
+def test_packed_gemm_o_equals_one_unit_per_cu(dev, case, dtype):
+    """GEMM-O up to 512 columns: more units than two per CU run four workgroups of one each on a CU.  A batch entry alone, of
+    at most a unit or a pair of them per CU, gives the same bits, in both passes, with either output and partial type; rows against
+    the selected heads' fp32 product."""
+    import flashomni_amd as fo
+    m, hd, heads, batch = case
+    n, rows = hd * heads, -(-m // 128)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert n <= 512 and (cus != 256 or (batch * rows * (n // 128) > 2 * cus >= 2 * rows * -(-n // 256)))
+    info, packed, indptr = _flags(batch, rows + 1, heads, 0.6, seed=m)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(batch, m, n, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.05).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.05).to(dtype)
+    pk, ip = torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev)
+    many = _chain_of_passes(x, w, b, heads, pk, ip, 128)
+    for i in sorted({0, batch // 2, batch - 1}):
+        alone = _chain_of_passes(x[i:i + 1].contiguous(), w, b, heads, pk, ip[i:i + 2].contiguous(), 128)
+        for one, all_ in zip(alone, many):
+            assert torch.equal(one[0], all_[i]), i
+    _check_gemm_o_rows(many[1], x, w, b, info, 128, True, _some_rows(m, 317), hd)
+    _check_gemm_o_rows(many[3], x, w, many[1], info, 128, False, _some_rows(m, 317), hd)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [(1025, 128, 40), (1407, 160, 32), (1500, 320, 16), (16513, 128, 3), (20001, 96, 4), (33000, 64, 2)])
+def test_gemm_o_units_two_to_a_cu(dev, case, dtype):
+    """One to two units per CU whose pairs are more than one per CU or whose width is above 4096: a workgroup per unit, two on a
+    CU.  Both passes, with either output and partial type, against the selected heads' fp32 product; the same bits as one of two batch
+    entries, which strips or packed units compute.  Heads of 160, 320 and 96 columns: slabs of which one half counts."""
+    m, hd, heads = case
+    n, rows = hd * heads, -(-m // 128)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    units, pairs = rows * (n // 128), rows * -(-n // 256)
+    if cus == 256:
+        assert cus < units <= 2 * cus < 2 * units and (pairs > cus or n > 4096)
+    info, packed, indptr = _flags(2, rows + 1, heads, 0.6, seed=m)
+    info[0, 0], info[0, 1] = False, True   # (the text block's flags; a block with every head)
+    segs = [np.packbits(f.reshape(-1).astype(np.uint8), bitorder="little") for f in info]
+    pk = torch.from_numpy(np.concatenate(segs)).to(dev)
+    ip = torch.from_numpy(np.cumsum([0] + [len(f) for f in segs]).astype(np.int32)).to(dev)
+    g = torch.Generator(device=dev).manual_seed(m)
+    x = torch.randn(2, m, n, generator=g, device=dev).to(dtype)
+    w = (torch.randn(n, n, generator=g, device=dev) * 0.02).to(dtype)
+    b = (torch.randn(n, generator=g, device=dev) * 0.02).to(dtype)
+    both = _chain_of_passes(x, w, b, heads, pk, ip, 128)
+    for i in range(2):
+        xi, ii = x[i:i + 1].contiguous(), info[i:i + 1]
+        alone = _chain_of_passes(xi, w, b, heads, pk, ip[i:i + 2].contiguous(), 128)
+        for one, all_ in zip(alone, both):
+            assert torch.equal(one[0], all_[i]), i
+        for out, cache in ((alone[0], True), (alone[1], True), (alone[2], False), (alone[3], False)):
+            bias = b if cache else alone[0] if out is alone[2] else alone[1]
+            _check_gemm_o_rows(out, xi, w, bias, ii, 128, cache, _some_rows(m, 131), hd)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [64, 96, 352, 384])
+@pytest.mark.parametrize("shape", [(1, 18001, 384, 0), (1, 33000, 128, 128), (2, 9100, 384, 0)])
+def test_gemm_q_units_two_to_a_cu(dev, shape, k, dtype):
+    """The same for GEMM-Q, dense and flagged (half, none, all): an odd number of column blocks, whose pairs are more than the
+    CUs.  Against the fp32 product, rounded once; tiles that are not flagged keep their bytes.  K of one slab, of 32 mod 64."""
+    import flashomni_amd as fo
+    batch, m, n, text = shape
+    rows, heads = -(-m // 128), n // 128
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert cus != 256 or (cus < batch * rows * heads <= 2 * cus and batch * rows * -(-n // 256) > cus)
+    x, w, b = (t.to(dev) for t in _operands(batch, m, n, k, dtype, seed=k))
+    ref = torch.nn.functional.linear(x.float(), w.float(), b.float())
+    half_ulp = 2.0 ** (-9 if dtype == torch.bfloat16 else -11)
+    # (one rounding; sums of k products in another order: k * 2^-24 of the sum of their sizes, below 16 standard deviations of one)
+    bound = 2 * half_ulp * ref.abs() + k * 2.0 ** -24 * 16 * 0.02
+    full = fo.flashomni_gemm(x, w, heads, num_text_tokens=0, bias=b, is_full=True)
+    assert bool(((full.float() - ref).abs() <= bound).all())
+    for p in (0.0, 0.5, 1.0):
+        info, packed, indptr = _flags(batch, text // 128 + rows, heads, p, seed=m)
+        out = torch.full((batch, m, n), -7.0, dtype=dtype, device=dev)
+        fo.flashomni_gemm(x, w, heads, torch.from_numpy(packed).to(dev), torch.from_numpy(indptr).to(dev), text, b, out=out)
+        on = torch.from_numpy(info[:, text // 128:]).to(dev).repeat_interleave(128, 1)[:, :m].repeat_interleave(128, 2)
+        assert bool((out[~on] == -7.0).all())
+        assert torch.equal(out[on], full[on])
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -705,9 +789,9 @@ def test_gemm_o_of_a_mixed_batch(dev, shape, p_active):
 
 @pytest.mark.parametrize("shape", [(1, 6200, 1536), (1, 6300, 1536), (1, 16100, 2048), (1, 8185, 3072), (2, 3300, 2560),
                                    (1, 4090, 5120), (1, 2553, 5120)])
-def test_gemm_o_forms_without_scratch(dev, shape):
-    """Shapes on both sides of the lines at which packed units or quads are taken whatever the flags (one round of quads
-    and more of them, narrow and wide): sampled rows of both passes against the fp32 product of the selected heads."""
+def test_gemm_o_sampled_rows(dev, shape):
+    """Shapes of 2.3 to 8 units per CU, narrow and wide, an odd number of token blocks among them: sampled rows of both passes
+    against the fp32 product of the selected heads."""
     import flashomni_amd as fo
     batch, m, n = shape
     heads, blocks = n // 128, -(-m // 128)
