@@ -383,8 +383,11 @@ int fo_sparse_attention_direct(const void* args);
  * Requires N % 128 == 0, K % 32 == 0 (csrc/gemm.cu:36) and 64 <= K <= 65536; M may have a tail (the
  * reference demands M % 128 == 0).
  * `workspace`: device scratch of at least fo_gemm_workspace_bytes(batch, m, n) bytes, 16-byte
- * aligned; it receives the list of tile quads that the GEMM kernel walks (short launches, up to
- * 256 windows x column pairs, build the list inside the GEMM kernel and leave it untouched).
+ * aligned.  Long calls leave the list of tile quads that the GEMM kernel walks there; of those that list their tiles
+ * inside the GEMM kernel (up to 256 windows x column pairs) the ones of more than 32 column blocks and 4.5 to 16 units per CU are
+ * two launches, the first of which leaves in the first word whether it has computed the call.  What the scratch held before
+ * is not read.  Calls that share it must not overlap in time, and none of their launches may come to lie between another one's:
+ * on one stream that means that host threads make them one at a time.
  * ------------------------------------------------------------------------------------------- */
 int64_t fo_gemm_workspace_bytes(int32_t batch, int32_t m, int32_t n);
 int fo_gemm_q(const void* x, const void* w, const void* bias, void* y, int dtype, int32_t batch,
@@ -406,8 +409,6 @@ int fo_gemm_q(const void* x, const void* w, const void* bias, void* y, int dtype
  * hd must be a multiple of 32.  No tile list is needed (every token block is visited, the tile
  * order is computed arithmetically): `workspace` may be NULL and is neither read nor written; fo_gemm_q with
  * is_full != 0 likewise.
- * fo_gemm_q's workspace holds a call's tile list: calls that share it must not overlap in time, and none of their launches
- * may come to lie between another one's: on one stream that means that host threads make them one at a time.
  * ------------------------------------------------------------------------------------------- */
 int fo_gemm_o(const void* x, const void* w, const void* bias, void* y, int dtype, int bias_kind,
               int bias_dtype, int y_dtype, int32_t batch, int32_t m, int32_t n, int32_t k,
