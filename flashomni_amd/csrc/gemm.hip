@@ -32,8 +32,7 @@
 // Data path.  Operands are staged in slabs of 64 k: a tile row is then 128 B, one whole memory line.
 // A wavefront fetches its sixteen 8-row pieces of a slab with buffer loads (a resource descriptor
 // per tile in scalar registers, 32-bit lane offsets, the k offset as the scalar offset: no vector
-// address arithmetic; rows past M and unselected heads read as zeros through the descriptor's range
-// check) into staging registers one slab ahead, and writes them to LDS (two slab buffers) a slab
+// address arithmetic; rows past M read as zeros through the descriptor's range check) into staging registers one slab ahead, and writes them to LDS (two slab buffers) a slab
 // later; loads, LDS writes and operand reads are spread evenly between the MFMAs (per sixteen MFMAs:
 // eight reads, four writes, four loads), so the memory path sees an even stream and nothing queues
 // behind a burst.  (Direct global -> LDS copies need no registers but can only be issued once a
@@ -129,8 +128,8 @@ struct GemmParams {
   void* y;           // [B, M, N]
   const uint8_t* sparse_info;
   const int32_t* sparse_info_indptr;
-  const int32_t* quads;  // kQuadInts per quad, queue by queue; null: every unit is computed and the
-                         // quads are enumerated arithmetically (GEMM-O, GEMM-Q with is_full)
+  const int32_t* quads;  // kQuadInts per quad, queue by queue; null: the kernel lists them itself (inline_cells), or every
+                         // unit is computed and the quads are enumerated arithmetically (is_full)
   const int32_t* qoff;   // qoff[0..8] queue boundaries inside `quads`
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
   int32_t strip_cols;    // strips: column groups of XCDs
@@ -166,7 +165,7 @@ struct ListGeom {
   int32_t batch, n_row_tiles, n_col_tiles, n_win, n_cp;  // windows per batch, column pairs
 };
 
-__device__ __forceinline__ void cell_masks(const ListGeom& gm, int cell, bool use_flags,
+__device__ __forceinline__ void cell_masks(const ListGeom& gm, int cell,
                                            const uint8_t* __restrict__ sparse_info,
                                            const int32_t* __restrict__ sparse_info_indptr,
                                            int32_t sparse_q_size, int32_t num_heads, int32_t head_dim,
@@ -181,11 +180,6 @@ __device__ __forceinline__ void cell_masks(const ListGeom& gm, int cell, bool us
   const int rows = min(kWindow, gm.n_row_tiles - w * kWindow);
   const uint32_t all = (1u << rows) - 1u;
   const bool has1 = 2 * cp + 1 < gm.n_col_tiles;
-  if (!use_flags) {
-    *m0 = all;
-    *m1 = has1 ? all : 0u;
-    return;
-  }
   const uint8_t* info = sparse_info + sparse_info_indptr[b];
   // All flag bytes of the cell are requested before the first is looked at (rows past the end repeat
   // the last one): one memory latency for the cell instead of one per row.
@@ -222,26 +216,23 @@ __device__ __forceinline__ int pop_lowest(uint32_t* m) {
 }
 
 // Packs a cell's flagged units into work items and calls f(r0, r1, valid, r2) for each; r1 < 0 = no
-// second row.  Quads: valid bits 1 = (r0,c0), 2 = (r0,c1), 4 = (r1,c0), 8 = (r1,c1).  Column strips
-// (col_strips: units come from flags): valid = kColStrip | 7 (| kColStripSecond for the cell's second
-// column), rows r0, r1, r2 of that column.
+// second row.  Quads: valid bits 1 = (r0,c0), 2 = (r0,c1), 4 = (r1,c0), 8 = (r1,c1).  Column strips:
+// valid = kColStrip | 7 (| kColStripSecond for the cell's second column), rows r0, r1, r2 of that column.
 template <typename F>
-__device__ __forceinline__ void for_each_quad(uint32_t m0, uint32_t m1, bool col_strips, F&& f) {
+__device__ __forceinline__ void for_each_quad(uint32_t m0, uint32_t m1, F&& f) {
   uint32_t both = m0 & m1, only0 = m0 & ~m1, only1 = m1 & ~m0;
   while (__popc(both) >= 2) {
     const int r0 = pop_lowest(&both), r1 = pop_lowest(&both);
     f(r0, r1, 0xF, 0);
   }
-  if (col_strips) {
-    // rows flagged in one column only: three at a time into a column strip (three X tiles, one W tile)
-    while (__popc(only0) >= 3) {
-      const int r0 = pop_lowest(&only0), r1 = pop_lowest(&only0), r2 = pop_lowest(&only0);
-      f(r0, r1, kColStrip | 0x7, r2);
-    }
-    while (__popc(only1) >= 3) {
-      const int r0 = pop_lowest(&only1), r1 = pop_lowest(&only1), r2 = pop_lowest(&only1);
-      f(r0, r1, kColStrip | kColStripSecond | 0x7, r2);
-    }
+  // rows flagged in one column only: three at a time into a column strip (three X tiles, one W tile)
+  while (__popc(only0) >= 3) {
+    const int r0 = pop_lowest(&only0), r1 = pop_lowest(&only0), r2 = pop_lowest(&only0);
+    f(r0, r1, kColStrip | 0x7, r2);
+  }
+  while (__popc(only1) >= 3) {
+    const int r0 = pop_lowest(&only1), r1 = pop_lowest(&only1), r2 = pop_lowest(&only1);
+    f(r0, r1, kColStrip | kColStripSecond | 0x7, r2);
   }
   while (__popc(only0) >= 2) {
     const int r0 = pop_lowest(&only0), r1 = pop_lowest(&only0);
@@ -301,7 +292,6 @@ __device__ __forceinline__ int count_pairs(uint32_t m0, uint32_t m1) {
 struct ListArgs {
   const uint8_t* sparse_info;
   const int32_t* sparse_info_indptr;
-  int32_t use_flags;  // GEMM-Q without is_full: units come from the flags
   int32_t sparse_q_size, num_heads, head_dim, num_text_tokens;
 };
 
@@ -318,9 +308,9 @@ __global__ void __launch_bounds__(kListThreads) gemm_quads_kernel(ListArgs a, Li
   const int lo = min(tid * per, n_cells), hi = min(lo + per, n_cells);
   int32_t my_cnt = 0;
   for (int cell = lo; cell < hi; ++cell) {
-    cell_masks(gm, cell, a.use_flags, a.sparse_info, a.sparse_info_indptr, a.sparse_q_size, a.num_heads,
+    cell_masks(gm, cell, a.sparse_info, a.sparse_info_indptr, a.sparse_q_size, a.num_heads,
                a.head_dim, a.num_text_tokens, &b, &row0, &cp, &m0, &m1);
-    for_each_quad(m0, m1, a.use_flags != 0, [&](int, int, int, int) { ++my_cnt; });
+    for_each_quad(m0, m1, [&](int, int, int, int) { ++my_cnt; });
   }
   // inclusive scan of the per-thread counts: inside a wavefront by lane shifts, then over the
   // sixteen wavefront totals
@@ -345,9 +335,9 @@ __global__ void __launch_bounds__(kListThreads) gemm_quads_kernel(ListArgs a, Li
   int32_t q = my_incl - my_cnt;
   for (int cell = lo; cell < hi; ++cell) {
     if (per > 1)  // with one cell per thread the masks of the counting pass are still at hand
-      cell_masks(gm, cell, a.use_flags, a.sparse_info, a.sparse_info_indptr, a.sparse_q_size, a.num_heads,
+      cell_masks(gm, cell, a.sparse_info, a.sparse_info_indptr, a.sparse_q_size, a.num_heads,
                  a.head_dim, a.num_text_tokens, &b, &row0, &cp, &m0, &m1);
-    for_each_quad(m0, m1, a.use_flags != 0, [&](int r0, int r1, int valid, int r2) {
+    for_each_quad(m0, m1, [&](int r0, int r1, int valid, int r2) {
       int32_t* e = quads + kQuadInts * static_cast<int64_t>(q);
       e[0] = b;
       e[1] = row0 + r0;
@@ -435,9 +425,9 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
     if (tid < p.inline_cells) {
       int b, row0, cp;
       uint32_t m0, m1;
-      cell_masks(gm, tid, true, p.sparse_info, p.sparse_info_indptr, p.sparse_q_size, p.num_heads,
+      cell_masks(gm, tid, p.sparse_info, p.sparse_info_indptr, p.sparse_q_size, p.num_heads,
                  p.head_dim, p.num_text_tokens, &b, &row0, &cp, &m0, &m1);
-      for_each_quad(m0, m1, true, [&](int, int, int, int) { ++cnt; });
+      for_each_quad(m0, m1, [&](int, int, int, int) { ++cnt; });
       if constexpr (kPairs) {  // (both counts in one scan: at most 16 per cell and kInlineCells cells)
         cnt += count_pairs(m0, m1) << 16;
       }
@@ -535,7 +525,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
         if (kPairs && pairs) {
           for_each_pair(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], entry);
         } else {
-          for_each_quad(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], true, entry);
+          for_each_quad(s_cell_mask[2 * tid], s_cell_mask[2 * tid + 1], entry);
         }
       }
       __syncthreads();
@@ -627,10 +617,10 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const GemmParams p) {
   auto gload = [&](int j, int entry) {
     stg[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc[j >> 2], ld_off[j & 3], (entry & 0xFFFF) * 2, 0);
   };
-  // kHalf: only one half of a slab that reaches into its neighbour counts; the other half of the X
+  // kHalf: only the second half of a slab that reaches into its neighbour counts; the first half of the X
   // pieces is cleared on the way to LDS
   auto keep_of = [&](int entry) -> unsigned {
-    return (entry & kZeroFirst) ? ~mask_first : ((entry & kZeroSecond) ? mask_first : 0xFFFFFFFFu);
+    return (entry & kZeroFirst) ? ~mask_first : 0xFFFFFFFFu;
   };
   auto lwrite = [&](int j, int stage, unsigned keep) {
     const int t = j >> 2;
@@ -1289,7 +1279,8 @@ __device__ __forceinline__ void unit_epilogue(const GemmParams& p, uint8_t* regi
           }
         }
         if constexpr (kOutF32) {
-          // (no scalar offset: see the quads' store)
+          // (the row offset travels in the lane's: with one in a scalar register the compiler may write the first data
+          // register in the very next instruction, and the last lanes then store that value)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + 4 * i * p.n) * 4, 0, 2);
         } else {
           x4 out;
@@ -1317,17 +1308,17 @@ __device__ __forceinline__ void unit_epilogue(const GemmParams& p, uint8_t* regi
 }
 
 // ---------------------------------------------------------------------------------------------
-// Short launches: a workgroup per unit.  Quads keep a CU busy with one work item of four units for
-// its whole k range, so a launch lasts whole rounds of quads however few units are in them: nine
-// token blocks x eight heads fill 36 of 256 CUs, and one unit in ten flagged over 16 k tokens is
-// ~200 items of one or two units that each take as long as four.  Here the four wavefronts share one
-// unit (64 x 64 each: 64 accumulators, 182 registers), two workgroups fit a CU (72 KB of LDS), one's
-// prologue and epilogue run beside the other's loop, and GEMM-O walks the heads of one token block
-// instead of the union of two.  The price is twice the operand bytes per flop over the L2 -> CU path
-// (32 KB per 128 x 128 x 64 step, ~550 cycles of it beside 512 of matrix core), so long launches keep
-// the quads.  The loop is the quads': staging registers a slab ahead, two LDS slab buffers, one
+// One to two units per CU that are not one round of pairs (an odd number of column blocks; GEMM-O above 4096 columns): a
+// workgroup per unit, two on a CU.  Quads would be one round that lasts as long however few units are in it (GEMM-Q of
+// 17 000 x 384, half of the units flagged: 16.3 us, as here 10.1).  The four wavefronts share one unit (64 x 64 each: 64
+// accumulators, 182 registers), two workgroups fit a CU (64 KB of LDS and GEMM-O's list), one's prologue and epilogue run
+// beside the other's loop, and GEMM-O walks the heads of one token block.  The price is twice the operand bytes per flop over
+// the L2 -> CU path (32 KB per 128 x 128 x 64 step, ~550 cycles of it beside 512 of matrix core), which is what bounds it.
+// The loop is the quads': staging registers a slab ahead, two LDS slab buffers, one
 // barrier per slab, the same mix of MFMAs, operand reads, LDS writes and loads in every substep; the
 // k order is the same, and so are the results, bit for bit.
+// (GEMM-O with new inputs in every call is no faster here than in the forms of longer launches: both passes of 17 000 x 384
+// 21.8 us, as packed units 21.4; 1500 x 5120 103.5, as strips 98.4.)
 // ---------------------------------------------------------------------------------------------
 template <typename T, bool kReduce, bool kHalf, bool kPartial>
 __global__ void __launch_bounds__(kThreads, 2) gemm_unit_kernel(const GemmParams p) {
@@ -2033,7 +2024,7 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
         }
         const int r = 4 * (8 * mt + i) * p.n;
         if constexpr (kOutF32) {
-          // (no scalar offset: see the quads' store)
+          // (no scalar offset: see unit_epilogue)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + r) * 4, 0, 2);
         } else {
           x4 out;
@@ -2520,7 +2511,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
         }
         const int r = (32 * mt + 2 * i) * p.n;
         if constexpr (kOutF32) {
-          // (no scalar offset: see the quads' store)
+          // (no scalar offset: see unit_epilogue)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + r) * 4, 0, 2);
         } else {
           x4 out;
@@ -2664,7 +2655,7 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   int cols = 1;
   int64_t grid;
   if (flagged) {
-    if (gm.n_col_tiles > 32) cols = 2;
+    if (gm.n_col_tiles > 32) cols = 2;  // (no group is without a column)
     int64_t per = 0;  // strips of a token block, at most
     for (int g = 0; g < cols; ++g) per += ((g + 1) * gm.n_col_tiles / cols - g * gm.n_col_tiles / cols + 1) / 2;
     grid = (rows * per + kXcds - 1) / kXcds * kXcds;
@@ -2681,7 +2672,7 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 }
 
 // GEMM-O.
-//   * A CU per unit or per strip (gemm_deep_kernel), then a workgroup per unit, while all of them fit the chip at once, two
+//   * A CU per unit or per strip (gemm_deep_kernel), then a workgroup per unit (gemm_unit_kernel), while all fit the chip at once, two
 //     per CU (144 units of K = 1024: quads 28 us, units 12; strips, two workgroups to a CU, over units up to one per CU 1.3 .. 1.6, of one to two 0.91 .. 1.3, about equal from K = 1024 on).
 //   * Narrow matrices, up to K = 512, are bound by memory and want the most loads in flight: packed units (strips over them,
 //     three to ten units per CU: 256 columns 1.0 .. 1.3, 384 1.1 .. 1.4, 512 1.0 .. 1.1).
@@ -2704,22 +2695,24 @@ int launch_o(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
 
 // GEMM-Q.
 //   * A CU per unit or per strip (gemm_deep_kernel), then a workgroup per unit, while all of them fit the chip at once, two
-//     per CU (us, quads -> units: 256 units of K = 2048 46 -> 23, 432 of K = 1536 39 -> 28 dense and 35 -> 23 with a quarter
-//     flagged).
+//     per CU (gemm_unit_kernel: us, quads -> units, 20 / 50 / 90 % flagged: 17 000 x 384 15.5 / 16.3 / 17.0 -> 9.6 / 10.1 / 10.8,
+//     40 000 x 128, 20 / 60 %, 12.5 / 13.2 -> 6.7 / 7.0).
 //   * With flags: strips from 4.5 to 32 units per CU (16 beyond 32 column blocks, whose W the strips, which drift apart,
 //     read again and again; six column blocks at least, of which pairs can be made), otherwise quads, column strips and pairs
 //     by the kernel's own list, whose rounds last as long however few units they hold.  Strips over those, 10 .. 95 % flagged:
 //        8 heads, 4.4 to 15 units per CU  0.71 .. 1.18     16, 4.6 to 29  0.65 .. 1.05     24, 5.2 to 30  0.64 .. 1.06
 //       40, 5.6 to 16                     0.66 .. 1.02         to 24      0.71 .. 1.03         to 94      1.0 .. 1.36
-//     (3.4 to 4.4 units per CU 0.84 .. 1.13; 4 heads 1.1 .. 1.2).  With new inputs in every call strips are slower where they
-//     begin to share CUs and one round of quads still holds the units, 250 to 350 strips: 9000 x 3072 60 -> 67 us, 16 384 x 2048
-//     46 -> 52, 20 000 x 1024 up to 270 strips 23 -> 28.
+//     (3.4 to 4.4 units per CU 0.84 .. 1.13; 4 heads 1.1 .. 1.2).  With new inputs in every call the same, 8 to 32 heads and
+//     4.9 to 29 units per CU: 0.60 .. 1.0 at most densities, but slower where the quads' last round is nearly full and strips begin
+//     to share CUs (250 to 350 strips: 9000 x 3072 with 30 % 61 -> 70 us, 16 384 x 3072 with 20 % 74 -> 87, 20 000 x 1024 with 35 %
+//     24 -> 28) or with most units flagged (90 %: 0.81 .. 1.12).
 //   * Beyond 32 column blocks that is a wide range (8000 x 5120 from 19 to 29 % flagged, 5200 x 5120 from 30 to 47 %) and a large
 //     loss, so the quads are launched first: they count, run if one round holds them, but not items of two units nor strips
 //     a CU each, and leave in the scratch's first word whether they did; the strips behind them return if so.  us, strips alone ->
 //     this (quads alone): 8000 x 5120, 230 strips 81 -> 84 (80), 260 121 -> 105 (103), 300 134 -> 111 (113), 345 131 -> 122 (121), 400 138 ->
 //     142 (199); 5200 x 5120 80 -> 82 (81), 114 -> 100 (99), 122 -> 108 (107), 125 -> 115 (114), 133 -> 136 (204).  At 24 columns and
-//     fewer the two launches cost what they give (3 us of every call; 9000 x 3072, 230 / 260 / 400 strips 50 -> 52, 71 -> 64, 82 -> 86).
+//     fewer the two launches cost what they give (3 us of every call; 9000 x 3072, 230 / 260 / 400 strips 50 -> 52, 71 -> 64, 82 -> 86;
+//     where the quads return on a count of the flags, before any cell is walked, 1 to 4 us of every call, 8 and 16 heads gain nothing).
 //   * Dense: a quad per CU and round, so it depends on how full the rounds are.  Packed units up to 21 / 32 of them (over
 //     quads 0.75 .. 1.02), in a single round only up to K = 2048 (0.88 .. 1.01; 24 heads 1.05, 40 heads 1.07 .. 1.11).  Strips
 //     up to K = 512 (0.87 .. 0.95 over 2.9 to 23 units per CU) and where two quads' units per CU would be empty in the last
@@ -2796,7 +2789,6 @@ int launch_q(GemmParams& p, const ListGeom& gm, bool use_flags, void* workspace,
   ListArgs la;
   la.sparse_info = p.sparse_info;
   la.sparse_info_indptr = p.sparse_info_indptr;
-  la.use_flags = use_flags ? 1 : 0;
   la.sparse_q_size = p.sparse_q_size;
   la.num_heads = p.num_heads;
   la.head_dim = p.head_dim;
