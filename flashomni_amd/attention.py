@@ -102,7 +102,7 @@ class PlannedBatch:
 
     def __init__(self, float_workspace_buffer, qo_indptr_host, kv_indptr_host, qo_indptr_dev,
                  kv_indptr_dev, num_qo_heads, num_kv_heads, block_q, block_kv, share_rows=True,
-                 worklist=None, gqa_packed=False, send=(0, None, None, None), q_dtype=None, logits_soft_cap=0.0):
+                 worklist=None, gqa_packed=False, send=(0, None, None, None), q_dtype=None):
         self.device = float_workspace_buffer.device
         self.float_ws = float_workspace_buffer
         self.num_qo_heads, self.num_kv_heads = num_qo_heads, num_kv_heads
@@ -122,11 +122,11 @@ class PlannedBatch:
         index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         self.share_rows = share_rows
         self.split_ok = self._split_ws_ok()
-        # (the symbols of runs that never take their rows straight from them need no room)
-        direct_ws = self.float_ws_bytes() if self.split_ok and (q_dtype is None or q_dtype.itemsize == 2) else 0
+        # (the symbols of runs that never take their rows straight from them, whatever the float workspace, need no room)
+        direct = share_rows and (q_dtype is None or q_dtype.itemsize == 2)
         self.native, self.tables, sizes = _lib.native().plan(
             qo_indptr_host, kv_indptr_host, num_qo_heads, num_kv_heads, self.gqa_packed, index,
-            qo_indptr_dev, kv_indptr_dev, *send, direct_ws, float(logits_soft_cap))
+            qo_indptr_dev, kv_indptr_dev, *send, direct)
         (self.n_q_blk, self.n_kv_blk, self.max_rows, self.max_nnz, self.total_q_rows, self.total_kv_rows,
          self.min_info_bytes, self.min_kv_info_bytes, self.max_kv_len, *self._table_at) = sizes
         self.qo_indptr = self._table(0) if qo_indptr_dev is None else qo_indptr_dev
@@ -260,12 +260,13 @@ class PlannedBatch:
             self.decoded = (bool(is_full), torch.cuda.current_stream(self.device), [])
         return r
 
-    def listed(self) -> DecodedWorkList:
+    def listed(self, logits_soft_cap=0.0) -> DecodedWorkList:
         """The work list of the last run or decode, ordered before the current stream's work.  A run that took
         its rows straight from the symbols has kept a copy of them: decoded here, behind that run.  Where graphs
         hold launches of this plan the device decides whether there is something to decode."""
         native = _lib.native()
-        source, _ = native.list_source(self.native)
+        source = native.list_source(self.native, self.float_ws_bytes() if self.split_ok else 0,
+                                    float(logits_soft_cap or 0.0))
         if source:
             full = self._was_full()
             if self.decoded is not None:
@@ -292,7 +293,7 @@ class PlannedBatch:
 
     def _was_full(self):
         """is_full of what the current list stands for, as far as the host knows; None: there is none."""
-        _, capture = _lib.native().list_source(self.native)
+        capture = _lib.native().capture(self.native)
         if self.native.recorded_in and (capture == self.native.recorded_in
                                         or (self.decoded is None and not self.native.state)):
             return bool(self.native.recorded_full)
@@ -311,14 +312,14 @@ class PlannedBatch:
             cur.wait_event(ev)
             ordered.append(cur)
 
-    def reuse_decoded(self, is_full: bool) -> DecodedWorkList:
+    def reuse_decoded(self, is_full: bool, logits_soft_cap=0.0) -> DecodedWorkList:
         """The work list of the last decode, ordered before the current stream's work."""
         was_full = self._was_full()
         if was_full is None:
             raise RuntimeError("reuse_decoded=True needs an earlier decode() or run() after plan()")
         if was_full != bool(is_full):
             raise RuntimeError("reuse_decoded=True: the last decode was made with is_full=%s" % was_full)
-        return self.listed()
+        return self.listed(logits_soft_cap)
 
     def launch(self, q, k, v, out, lse, kv_layout, sm_scale, q_scale=None, k_scale=None, q_lo=None,
                k_lo=None, logits_soft_cap=0.0, widen_k=True) -> None:
@@ -611,7 +612,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
                 worklist=self._planned._list if self._planned is not None else None,
                 gqa_packed=gqa_symbols != "per_q_head",
                 send=(sent, self._int_workspace_buffer, self._pin_memory_int_workspace_buffer, self._pin_ring),
-                q_dtype=q_data_type, logits_soft_cap=logits_soft_cap)
+                q_dtype=q_data_type)
             self._plan_info = plan_info
         if not graph:
             self._qo_indptr_buf, self._kv_indptr_buf = self._planned.qo_indptr, self._planned.kv_indptr
@@ -741,7 +742,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
         else:
             _check_shape_dtype_device(out, q.shape[:-1] + v.shape[-1:], out_dtype, q.device, "out")
         if reuse_decoded:
-            pb.reuse_decoded(is_full)
+            pb.reuse_decoded(is_full, self._logits_soft_cap)
         else:
             pb.decode(sparse_info, sparse_kv_info, sparse_info_indptr, sparse_kv_info_indptr, is_full, clear=clear)
         pb.launch(q, k, v, out, lse if return_lse else None, self._kv_layout, sm_scale, q_scale, k_scale, q_lo,

@@ -312,7 +312,9 @@ struct Plan {
   // recording: the last launch was recorded.
   // taken: rows have been taken straight from the symbols, or a graph holds a launch that does so.  Until then
   // there is nothing that could be newer than the list.
-  int captured, recorded_full, recording, taken;
+  // list_only: a graph holds a reuse that runs the list without looking for something newer, so that no run of the plan
+  // takes its rows from the symbols from then on.
+  int captured, recorded_full, recording, taken, list_only;
   unsigned long long listed_in, recorded_in;
   // The copy lies behind the tables, in one place for as long as the plan lives (a graph writes it at every
   // replay): room for the symbols that such a run takes, at keep_at[0] info, [1] kv_info, [2] the indptrs (bytes
@@ -349,6 +351,12 @@ unsigned long long capture_of(hipStream_t stream) {
   unsigned long long id = 0;
   if (!stream || hipStreamGetCaptureInfo(stream, &s, &id) != hipSuccess || s == hipStreamCaptureStatusNone) return 0;
   return id ? id : ~0ull;
+}
+
+// Whether a run of the plan with 16-bit operands may be taken straight from the symbols.
+bool may_take(const Plan* p, int64_t ws_bytes, double cap) {
+  return fo_sparse_attention_direct_may_serve(static_cast<int32_t>(p->z.n_q_blocks), p->symbol_heads, p->batch, p->z.max_nnz,
+                                              ws_bytes, static_cast<float>(cap));
 }
 
 // A launch that leaves a list (state 0) or takes rows without one (1, 2) has been queued on the stream.
@@ -546,14 +554,13 @@ PyObject* enter_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // (qo_indptr, kv_indptr: int32 on the host; num_qo_heads, num_kv_heads, packed, device index,
 //  qo_indptr, kv_indptr of the device or None; to send host_plan()'s arrays: their bytes, the integer
-//  workspace, its pinned mirror and the mirror's Ring, or 0 and None; and bytes of the float workspace, 0: no room for
-//  parts of rows or operands that are always decoded, and the soft cap) -> (Plan, tables, sizes)
+//  workspace, its pinned mirror and the mirror's Ring, or 0 and None; and whether runs may take their rows straight from
+//  the symbols, if the float workspace and the soft cap of the moment, which can change, let them) -> (Plan, tables, sizes)
 PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_BEGIN
   const Tensor *qo, *kv, *qo_dev, *kv_dev, *iws, *pin;
-  int64_t hq, hkv, dev, sent, ws_bytes;
-  double cap;
-  if (!(n == 14 && whole(args[12], &ws_bytes) && real(args[13], &cap) && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
+  int64_t hq, hkv, dev, sent;
+  if (!(n == 13 && opt_tensor(args[0], &qo) && qo && opt_tensor(args[1], &kv) && kv && whole(args[2], &hq) &&
         whole(args[3], &hkv) && whole(args[5], &dev) && whole(args[8], &sent) && opt_tensor(args[9], &iws) &&
         opt_tensor(args[10], &pin) && (sent == 0 || (iws && pin && Py_TYPE(args[11]) == g_ring_type)) &&
         opt_tensor(args[6], &qo_dev) && opt_tensor(args[7], &kv_dev) &&
@@ -586,9 +593,8 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   p->state = 0;
   int rc = 0;
   int64_t ints = z.table_ints;
-  if (z.max_rows <= fo_sparse_attention_direct_max_pairs() && z.max_kv_len <= kMaxListed &&
-      fo_sparse_attention_direct_may_serve(static_cast<int32_t>(z.n_q_blocks), p->symbol_heads, batch, z.max_nnz, ws_bytes,
-                                           static_cast<float>(cap))) {
+  if (truth(args[12]) && z.max_rows <= fo_sparse_attention_direct_max_pairs() && z.max_kv_len <= kMaxListed &&
+      may_take(p, INT64_MAX, 0.)) {
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     // (symbol tensors much larger than the batch needs are not worth copying)
     p->keep_room[0] = z.min_info + 4096;
@@ -730,21 +736,37 @@ PyObject* note_list(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_GUARD_END
 }
 
-// (Plan) -> how a reuse on the current stream gets its list: 0: as it is; 1: decoded from what the last run left
-// behind; 2: the device decides between the two (fo_decode_sparse_kept).  And the capture the stream is in.
-PyObject* list_source(PyObject*, PyObject* arg) {
+// (Plan, bytes of the float workspace that parts of rows may lie in, soft cap) -> how a reuse on the current stream gets
+// its list: 0: as it is; 1: decoded from what the last run left behind; 2: the device decides between the two
+// (fo_decode_sparse_kept).
+PyObject* list_source(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  TORCH_GUARD_BEGIN
+  int64_t ws_bytes;
+  double cap;
+  if (!(n == 3 && Py_TYPE(args[0]) == g_plan_type && whole(args[1], &ws_bytes) && real(args[2], &cap))) {
+    PyErr_SetString(PyExc_RuntimeError, "list_source: bad argument");
+    return nullptr;
+  }
+  Plan* p = reinterpret_cast<Plan*>(args[0]);
+  const unsigned long long id = capture_of(static_cast<hipStream_t>(stream_of(p->dev)));
+  if (id) p->captured = 1;
+  // A reuse that is recorded now may be replayed behind a run that takes its rows from the symbols later on.  Where runs like
+  // this one never do, there will be none: should workspace or cap change, such runs are decoded.
+  if (id && p->keep_at[0] && p->listed_in != id && !p->taken && !may_take(p, ws_bytes, cap)) p->list_only = 1;
+  const bool list = !p->keep_at[0] || p->list_only || (id ? p->listed_in == id : !p->taken);
+  const int source = list ? 0 : p->captured ? 2 : p->state != 0;
+  return PyLong_FromLong(source);
+  TORCH_GUARD_END
+}
+
+// (Plan) -> the capture that the current stream is in, 0: none
+PyObject* capture(PyObject*, PyObject* arg) {
   TORCH_GUARD_BEGIN
   if (Py_TYPE(arg) != g_plan_type) {
     PyErr_SetString(PyExc_RuntimeError, "not a plan");
     return nullptr;
   }
-  Plan* p = reinterpret_cast<Plan*>(arg);
-  const unsigned long long id = capture_of(static_cast<hipStream_t>(stream_of(p->dev)));
-  if (id) p->captured = 1;
-  // (a reuse that is recorded now may be replayed behind a run that takes its rows from the symbols later on)
-  const bool list = !p->keep_at[0] || (id ? p->listed_in == id : !p->taken);
-  const int source = list ? 0 : p->captured ? 2 : p->state != 0;
-  return Py_BuildValue("(iK)", source, id);
+  return PyLong_FromUnsignedLongLong(capture_of(static_cast<hipStream_t>(stream_of(reinterpret_cast<Plan*>(arg)->dev))));
   TORCH_GUARD_END
 }
 
@@ -848,7 +870,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor fresh;
   // the launch without a decoded list (it clears what it skips: every row of a fresh output is its own)
   const bool own = !out && p->from_zero && q->size(0) == p->z.total_q;
-  const bool small = p->keep_at[0] && (full || (sym[0]->numel() <= p->keep_room[0] && sym[1]->numel() <= p->keep_room[1]));
+  const bool small = p->keep_at[0] && !p->list_only && (full || (sym[0]->numel() <= p->keep_room[0] && sym[1]->numel() <= p->keep_room[1]));
   int rc = FO_NOT_DIRECT;
   if (small && fo_sparse_attention_direct_serves(&a)) {
     if (!out) fresh = own ? at::empty(q->sizes(), q->options()) : at::zeros(q->sizes(), q->options());
@@ -1015,7 +1037,8 @@ PyMethodDef g_methods[] = {
     {"enter_plan", FASTCALL(enter_plan), nullptr},
     {"follow_run", follow_run, METH_O, nullptr},
     {"note_list", FASTCALL(note_list), nullptr},
-    {"list_source", list_source, METH_O, nullptr},
+    {"list_source", FASTCALL(list_source), nullptr},
+    {"capture", capture, METH_O, nullptr},
     {"kept_symbols", kept_symbols, METH_O, nullptr},
     {"packbits", FASTCALL(packbits), nullptr},
     {"segment_packbits", FASTCALL(segment_packbits), nullptr},

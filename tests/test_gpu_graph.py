@@ -337,6 +337,55 @@ def test_reuse_behind_a_capture_of_lists_that_are_always_decoded(dev, why, heads
     assert not kept
 
 
+@pytest.mark.parametrize("why", ["soft cap", "small workspace"])
+@pytest.mark.parametrize("recorded", [False, True])
+def test_workspace_and_cap_of_the_moment(dev, why, recorded):
+    """Whether rows are taken straight from the symbols goes by the float workspace and the soft cap of the run, which may be
+    others than the plan's.  A graph that holds a reuse from before, which runs the list as it is, still runs the list of the
+    moment: the plan's runs are decoded then."""
+    import flashomni_amd as fo
+    from flashomni_amd import _lib
+    n, heads, cap = 514, 206, 30.0 if why == "soft cap" else None
+    g = torch.Generator(device=dev).manual_seed(6)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    masks = [make_ragged_masks([384, 130], [384, 130], heads, 0.7, 0.6, seed=s) for s in (5, 6)]
+    first, other = ([torch.from_numpy(m[s]).to(dev) for s in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+                    for m in masks)
+    indptr = torch.from_numpy(masks[0]["qo_indptr"])
+    room = lambda size: torch.empty(size, dtype=torch.uint8, device=dev)
+
+    def plain(sym, c):
+        w = fo.BatchFlashOmniFAWithRaggedKVWrapper(room(128 << 20))
+        w.plan(indptr, indptr, heads, heads, 128, q_data_type=q.dtype, logits_soft_cap=c)
+        return w.run(q, k, v, *sym)
+
+    small = room(2 * _lib.lib().fo_sparse_fa_split_workspace_bytes() - 16 if cap is None else 128 << 20)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(small)
+    w.plan(indptr, indptr, heads, heads, 128, q_data_type=q.dtype, logits_soft_cap=cap)
+    out = torch.zeros_like(v)
+    w.run(q, k, v, *first, out=out)
+    assert w._planned.native.state == 0
+    if recorded:
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            w.run(q, k, v, *first, out=out, reuse_decoded=True)
+    if cap is None:
+        w.reset_workspace_buffer(room(128 << 20), room(8 << 20))
+        got = w.run(q, k, v, *other)
+    else:
+        got = w.forward(q, k, v, *other)
+    assert (w._planned.native.state == 0) == recorded
+    exp = plain(other, None)
+    assert float((got.float() - exp.float()).abs().max()) <= 2e-2
+    if recorded:
+        exp = plain(other, cap)
+        for _ in range(2):
+            out.zero_()
+            graph.replay()
+            assert float((out.float() - exp.float()).abs().max()) <= 2e-2
+
+
 def test_reuse_behind_a_capture_before_rows_came_from_the_symbols(dev, monkeypatch):
     """Where they can be taken from them but have not been, eagerly or in a graph, an eager reuse makes no launch either; one
     that a graph holds looks at every replay, since a run may come in between."""
