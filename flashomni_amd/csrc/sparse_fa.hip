@@ -45,8 +45,8 @@
 // Long lists (eight rows per CU or more) run in a second form of the same kernel: a workgroup is
 // 4 wavefronts that own a whole row, two such workgroups share a CU, and the main loop is software-
 // pipelined in steps of 32 keys: the MFMAs of S(t+1) and P(t-1).V(t-1) are interleaved, instruction
-// by instruction, with the softmax of S(t), the operand reads four slots ahead and the copies two
-// steps ahead (see the kPipe branch of the kernel).  Measured on the video-sized lists it is ~5 %
+// by instruction, with the softmax of S(t), the operand reads eight MFMAs ahead and the copies two or three
+// steps ahead (see the kPipe branch of the kernel).  Measured on the video-sized lists it is ~12 %
 // faster than the two-phase form; on short decoded lists, whose rows are taken whole, a row's doubled latency
 // costs more than that.  Short lists read straight from the symbols are cut in parts as fine as it takes and run
 // in it from 2.5 candidates per CU on (fo_sparse_attention_direct below); long lists of two-term fp8 q and k do
@@ -95,6 +95,9 @@ constexpr int kMergeOBytes = 4 * 16 * 64 * 16;
 constexpr int kOutTileOff = kMergeOBytes + 4 * 64 * 8;  // behind the merge area
 constexpr int kOutRowBytes = 256 + 16;                  // one output row of 128 16-bit elements, padded
 constexpr int kOutTileBytes = 128 * kOutRowBytes;
+// The pipelined form's buffers of 32 keys.  K: every four rows (what one copy instruction fills) begin 16 bytes later
+// modulo the banks than the four before, so that rows a multiple of four apart need no swizzle against each other.
+constexpr int kPipeKRows4 = 4 * kRowBytes + 16, kPipeKBuf = 8 * kPipeKRows4, kPipeVBuf = 32 * kRowBytes;
 // LDS geometry of one kv group: two stages of (K tile, V tile); K is 16-bit or fp8
 template <bool kFp8, bool kKLo = false, int kGroups = 2>
 struct Geom {
@@ -102,7 +105,8 @@ struct Geom {
   static constexpr int kKBytes = kTileKV * (kFp8 ? (kKLo ? 2 : 1) * kRowBytes8 : kRowBytes);
   static constexpr int kStageBytes = kKBytes + kVBytes;
   static constexpr int kGroupBytes = 2 * kStageBytes;
-  static constexpr int kTilesBytes = kGroups * kGroupBytes;
+  // (one kv group: eight buffers of 32 keys, see kPipeKBuf)
+  static constexpr int kTilesBytes = kGroups == 1 ? 4 * (kPipeKBuf + kPipeVBuf) : kGroups * kGroupBytes;
   // the epilogue reuses the tile buffers: kv group 1's partial O (64 KB fp32) + its (max, sum)
   // pairs (2 KB), then the finished row as a padded tile for the coalesced store (one kv group:
   // no merge area, the output tile starts at 0)
@@ -518,7 +522,7 @@ sparse_fa_kernel(const FaParams p) {
   // V^T transpose read: this lane supplies row j = (lane%16)/4 of a 4-row patch that starts at kv
   // row 16*kk + 4*g (+8 for the second read), 8 bytes at element column 32*dt + 16*q2 + 4*(lane%4)
   int v_rd_off[4][2];
-  {
+  if constexpr (!kPipe) {
     const int j = (lane & 15) >> 2, q2 = (lane >> 4) & 1, i4 = lane & 3;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -1328,20 +1332,26 @@ sparse_fa_kernel(const FaParams p) {
     float m_run = 0.f, d_part = 0.f;
     if constexpr (kPipe) {
       // ---- software-pipelined row (one kv group) ----
-      // A step is 32 keys.  In step t a wavefront issues the MFMAs of S(t+1) = K(t+1).Q^T and of
-      // O^T += V(t-1)^T.P(t-1)^T, and between them, instruction by instruction, the softmax of S(t)
-      // (max, exp2, rounding, row sum -> P(t)), the operand reads of later MFMAs and the copies of
-      // later steps: the vector ALU work of a step runs in the shadow of its own MFMAs instead of in
-      // a phase of its own.  LDS holds four K and four V buffers of 32 keys (8 KB each).  The K
-      // operands of a step are read one step ahead (K(t) in step t-2), the V^T operands four slots
-      // ahead (V(t) in the second half of step t and the first half of step t+1); a copy is issued as
-      // soon as its buffer is dead: K three steps, V two steps before its first read.  One barrier
-      // per step.
-      constexpr int kStep = 32, kBuf = kStep * kRowBytes;
-      // K buffers 0..2 | V buffer 0 | K buffer 3 | V buffers 1..3; Q is staged in the upper 32 KB, so
+      // A step is 32 keys.  In step t a wavefront issues the eight MFMAs of S(t+1) = K(t+1).Q^T, then the eight of
+      // O^T += V(t-1)^T.P(t-1)^T, and between them, instruction by instruction, the softmax of S(t) (exp2, rounding, row
+      // sum -> P(t)), the largest value of S(t+1) as soon as it is complete, the operand reads and the copies of later
+      // steps: the vector ALU work of a step runs in the shadow of its own MFMAs instead of in a phase of its own.  Eight
+      // operands are in registers: each MFMA's is read eight MFMAs ahead, into the registers of the one just used, V(t-1)
+      // during the MFMAs of S and K(t+2) during those of P.V.  LDS holds four K and four V buffers of 32 keys; a copy is
+      // issued as soon as its buffer is dead: K two and a half steps, V three before its first read.  One barrier per step.
+      // What bounds it is the power limit (matrix cores 68 % busy at 1.7 GHz on long lists) and the vector ALU, 41
+      // instructions of a step beside the 16 MFMAs: 16 exp2, 8 roundings, 8 sums, 8 for the maximum and one more.  With S
+      // and P.V in turn instead of one after the other, the maximum in front of a step's first MFMA, 16 moves that set the
+      // accumulators of S to the reference point (now 16 registers that they accumulate from) and 7 address terms of K it
+      // was 73 of them besides the exp2: 33 k tokens x 24 heads with windows 1878 -> 1712 us, 16 896 x 24 with a fifth of the
+      // blocks in fp16 780 -> 714, 4608 x 24 from the symbols 126 -> 117.7.
+      constexpr int kStep = 32;
+      // K buffers 0..2 | V buffer 0 | K buffer 3 | V buffers 1..3; Q is staged from K buffer 3 on, so
       // that K(0..2) and V(0) can be requested together with it
-      auto kbuf = [&](int i) { return static_cast<uint32_t>(i * kBuf + (i == 3 ? kBuf : 0)); };
-      auto vbuf = [&](int i) { return static_cast<uint32_t>((4 + i) * kBuf - (i == 0 ? kBuf : 0)); };
+      constexpr int kQStage = 3 * kPipeKBuf + kPipeVBuf;
+      static_assert(kPipeKBuf + 3 * kPipeVBuf >= kBlockQ * kRowBytes, "Q must fit behind K(0..2) and V(0)");
+      auto kbuf = [&](int i) { return static_cast<uint32_t>(i * kPipeKBuf + (i == 3 ? kPipeVBuf : 0)); };
+      auto vbuf = [&](int i) { return static_cast<uint32_t>((i == 0 ? 3 : 4) * kPipeKBuf + i * kPipeVBuf); };
       const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
       const int last_valid = min(kBlockKV, kv_len - s_blk[nb - 1] * kBlockKV);
       const int n_steps = 4 * (nb - 1) + ((last_valid + kStep - 1) / kStep);
@@ -1361,11 +1371,16 @@ sparse_fa_kernel(const FaParams p) {
           const_cast<uint8_t*>(k_head), 0, static_cast<uint32_t>(kv_len - 1) * k_sn2 + kRowBytes, 0x00020000);
       const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<uint8_t*>(v_head), 0, static_cast<uint32_t>(kv_len - 1) * v_sn2 + kRowBytes, 0x00020000);
-      // a lane's part of a copy: row 4 * qs + lane / 16 of a 16-row group, swizzled 16-byte chunk
-      uint32_t k_voff = static_cast<uint32_t>(4 * qs + cp_row) * k_sn2 + cp_chunk * static_cast<uint32_t>(sizeof(T));
-      uint32_t v_voff = static_cast<uint32_t>(4 * qs + cp_row) * v_sn2 + cp_chunk * static_cast<uint32_t>(sizeof(T));
+      // A lane's part of a copy: row 4 * qs + lane / 16 of a 16-row group, 16-byte chunk swizzled by the row modulo four.
+      // (The operand reads of the loop then differ by immediate offsets but for two bits of the chunk: four addresses each
+      // for K and V.  With all four bits swizzled the reads of K took seven instructions a step.)
+      const int ln_c = fresh_lane();
+      const int cp_chunk = ((ln_c & 15) ^ ((ln_c >> 4) << 2)) * 16, cp_row = 4 * qs + (ln_c >> 4);
+      uint32_t k_voff = static_cast<uint32_t>(cp_row) * k_sn2 + cp_chunk;
+      uint32_t v_voff = static_cast<uint32_t>(cp_row) * v_sn2 + cp_chunk;
       asm volatile("" : "+v"(k_voff), "+v"(v_voff));
-      const uint32_t m0_base = lds0 + qs * 1024;  // LDS address of this wavefront's part of buffer offset 0
+      // LDS addresses of this wavefront's part of buffer offset 0
+      const uint32_t m0_k = lds0 + qs * kPipeKRows4, m0_v = lds0 + qs * 1024;
       // 64 lanes x 16 bytes of 4 rows, global -> LDS (see copy16_to_lds), addressed through a descriptor:
       // lane offset + scalar offset
       auto copy_desc = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
@@ -1379,12 +1394,12 @@ sparse_fa_kernel(const FaParams p) {
       auto copy_k = [&](int t) __attribute__((always_inline)) {
         const uint32_t soff = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(step_start(t))) * k_sn2;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) copy_desc(k_rsrc, k_voff, soff + j * 16 * k_sn2, m0_base + kbuf(t & 3) + j * 4096);
+        for (int j = 0; j < 2; ++j) copy_desc(k_rsrc, k_voff, soff + j * 16 * k_sn2, m0_k + kbuf(t & 3) + j * (4 * kPipeKRows4));
       };
       auto copy_v = [&](int t) __attribute__((always_inline)) {
         const uint32_t soff = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(step_start(t))) * v_sn2;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) copy_desc(v_rsrc, v_voff, soff + j * 16 * v_sn2, m0_base + vbuf(t & 3) + j * 4096);
+        for (int j = 0; j < 2; ++j) copy_desc(v_rsrc, v_voff, soff + j * 16 * v_sn2, m0_v + vbuf(t & 3) + j * 4096);
       };
 
       // prologue: Q, K(0..2), V(0) requested together
@@ -1398,7 +1413,7 @@ sparse_fa_kernel(const FaParams p) {
           int r = 8 * (4 * (n & 3) + qs) + q_row;
           r = r < q_rows ? r : q_rows - 1;
           copy16_to_lds(static_cast<const uint8_t*>(n < 4 ? p.q : p.q_lo) + q_off,
-                        static_cast<uint32_t>(r * p.q_sn + q_chunk), lds0 + 4 * kBuf + qs * 1024 + n * 4096);
+                        static_cast<uint32_t>(r * p.q_sn + q_chunk), lds0 + kQStage + qs * 1024 + n * 4096);
         }
       } else {
         const uint8_t* q_head = reinterpret_cast<const uint8_t*>(
@@ -1410,7 +1425,7 @@ sparse_fa_kernel(const FaParams p) {
           int r = 4 * (4 * n + qs) + cp_row;
           r = r < q_rows ? r : q_rows - 1;  // ragged last q block: re-read the last row
           copy16_to_lds(q_head, static_cast<uint32_t>((row_off(r, p.q_sn, p.q_sh) + cp_chunk) * sizeof(T)),
-                        lds0 + 4 * kBuf + qs * 1024 + n * 4096);
+                        lds0 + kQStage + qs * 1024 + n * 4096);
         }
       }
       copy_k(0);
@@ -1437,15 +1452,15 @@ sparse_fa_kernel(const FaParams p) {
         if (wv == 0) direct_next((row_it + 1) & 1);
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __builtin_amdgcn_s_barrier();
-      q8 qreg[8], kop[4];
-      x8 vop[4];
+      q8 qreg[8];
+      u32x4 op[8];  // operands of the next eight MFMAs: slices of K or of V^T
       u32x4 pA[2], pB[2];  // P of a step: 2 x 8 rounded values, as 32-bit pairs
       f32x16 sA, sB;
       if constexpr (kWide) {
         // q + q_lo in fp16 (the scales are applied to S)
         f_win *= c * ri.q_scale;
         const int ln_r = fresh_lane(), row = qs * 32 + (ln_r & 31);
-        const uint8_t* qt = smem + 4 * kBuf + row * kRowBytes8 + (ln_r >> 5) * 8;
+        const uint8_t* qt = smem + kQStage + row * kRowBytes8 + (ln_r >> 5) * 8;
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
           const uint8_t* at = qt + ((ks ^ swz8(row)) << 4);
@@ -1455,7 +1470,7 @@ sparse_fa_kernel(const FaParams p) {
       } else {
         const int ln_r = fresh_lane();
         const int q_rd_base = (ln_r & 31) * kRowBytes, q_rd_x = ((ln_r >> 5) ^ swz(ln_r & 31)) << 4;
-        const uint8_t* qt = smem + 4 * kBuf + qs * 32 * kRowBytes + q_rd_base;
+        const uint8_t* qt = smem + kQStage + qs * 32 * kRowBytes + q_rd_base;
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) qreg[ks] = *reinterpret_cast<const q8*>(qt + (q_rd_x ^ (ks << 5)));
         // the softmax scale (log2 domain) is folded into Q, so S^T needs no multiply
@@ -1464,25 +1479,24 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) qreg[ks][e] = static_cast<T>(static_cast<float>(qreg[ks][e]) * c);
       }
-      // LDS address of the K operand reads of a step, without the buffer's offset (an immediate of the
-      // read): read i is at kx0 ^ (i << 5) (row bits, chunk bits and the 256-byte aligned base of
-      // the array do not overlap)
+      // LDS addresses of the operand reads, without the buffer's offset and what else is an immediate of the read
       typedef __attribute__((address_space(3))) const q8 lds_x8;
-      uint32_t kx0 = lds0 + static_cast<uint32_t>(k_rd_base | k_rd_x);
-      asm volatile("" : "+v"(kx0));
-      // K operand slice i (16 d) of the step whose K is in buffer `buf`
-      auto read_k = [&](uint32_t kx, int buf, int i) __attribute__((always_inline)) {
-        return *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>((kx ^ (i << 5)) + kbuf(buf)));
-      };
-      // the same for the V^T operand reads: the eight lane offsets with the array's base added
-      uint32_t vrd[4][2];
+      uint32_t krd[4], vrd[4];
+      {
+        const int ln = fresh_lane();
+        const int r = ln & 31, j = (ln & 15) >> 2;
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int hi = 0; hi < 2; ++hi) {
-          vrd[dt][hi] = lds0 + static_cast<uint32_t>(v_rd_off[dt][hi]);
-          asm volatile("" : "+v"(vrd[dt][hi]));
+        for (int x = 0; x < 4; ++x) {
+          krd[x] = lds0 + (r >> 2) * kPipeKRows4 + (r & 3) * kRowBytes + ((x ^ (r & 3)) << 6) + (ln >> 5) * 16;
+          // (row 4 * (lane / 32) + j, columns 32 * x + 16 * (lane / 16 % 2) + 4 * (lane % 4): see lds_read_tr16)
+          vrd[x] = lds0 + ((ln >> 5) * 4 + j) * kRowBytes + ((x ^ j) << 6) + ((ln >> 4) & 1) * 32 + (ln & 3) * 8;
+          asm volatile("" : "+v"(krd[x]), "+v"(vrd[x]));
         }
+      }
+      // K operand slice i (16 d) of the step whose K is in buffer `buf`
+      auto read_k = [&](int buf, int i) __attribute__((always_inline)) {
+        return *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(krd[i >> 1] + kbuf(buf) + (i & 1) * 32));
+      };
       // V^T operand (kk, dt) of the step whose V is in buffer `buf`: 16 keys x 32 d, transposed
       auto read_v = [&](int buf, int kk, int dt) __attribute__((always_inline)) {
         union {
@@ -1490,8 +1504,8 @@ sparse_fa_kernel(const FaParams p) {
           x8 v;
         } a;
         const uint32_t off = vbuf(buf) + kk * 16 * kRowBytes;
-        a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(vrd[dt][0] + off)));
-        a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(vrd[dt][1] + off)));
+        a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(vrd[dt] + off)));
+        a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(vrd[dt] + off + 8 * kRowBytes)));
         return a.v;
       };
 #pragma unroll
@@ -1499,20 +1513,16 @@ sparse_fa_kernel(const FaParams p) {
       {
         q8 k0[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) k0[i] = read_k(kx0, 0, i);
+        for (int i = 0; i < 8; ++i) k0[i] = read_k(0, i);
 #pragma unroll
         for (int i = 0; i < 8; ++i) sA = TS::mfma(k0[i], qreg[i], sA);
       }
       __builtin_amdgcn_sched_barrier(0);
       // (a row of one step reads a buffer nobody filled: the result is never used)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) kop[i] = read_k(kx0, 1, i);
-      // (a row's first step multiplies P(-1) = 0 by what vop holds and by what its first half reads
-      // from V buffer 3, where Q was staged: both must be finite whatever Q holds)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) vop[i][e] = static_cast<T>(0.f);
+      for (int i = 0; i < 8; ++i) op[i] = __builtin_bit_cast(u32x4, read_k(1, i));
+      // (a row's first step multiplies P(-1) = 0 by what it reads from V buffer 3, where Q was staged: that must be
+      // finite whatever Q holds)
 #pragma unroll
       for (int e = 0; e < 4; ++e) pA[0][e] = pA[1][e] = pB[0][e] = pB[1][e] = 0u;
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): Q and K(0) are in registers
@@ -1527,130 +1537,171 @@ sparse_fa_kernel(const FaParams p) {
           vb[tid + kGroupThreads] = z;
         }
       }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the zeros are there, before the barrier of the first step
       if (n_steps > 1) {
-        copy_v(1);
         copy_k(min(3, n_steps - 1));  // (kept to four instructions per group: the loop's waits count them)
+        copy_v(1);
       }
-
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sB[i] = 0.f;  // S(1) accumulates from the reference point 0, moved by the first step
       if constexpr (!kWide) blk_win = s_blk[min(lane, nb - 1)];
       typedef __attribute__((ext_vector_type(2))) T x2;
       const x2 ones2 = {static_cast<T>(1.0f), static_cast<T>(1.0f)};
+      // keys of a step that a lane's half row does not have: p = 0
+      auto mask_tail = [&](f32x16& s, int valid) __attribute__((always_inline)) {
+        const int g4 = (fresh_lane() >> 5) * 4;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = (i >> 2) * 8 + (i & 3) + g4 < valid ? s[i] : -INFINITY;
+      };
+      auto row_max = [&](const f32x16& s) __attribute__((always_inline)) {
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        return max_across_halves(mx);
+      };
+      // What S accumulates from: the reference point, taken off (kWide: nothing, it comes off with the factor).
+      f32x16 s_init;
+      const int valid0 = kv_len - static_cast<int>(s_blk[0]) * kBlockKV;
+      if (valid0 < kStep) mask_tail(sA, valid0);
+      const float s_max0 = row_max(sA);
+      m_run = s_max0;
+      if constexpr (kWide) {
+        m_run *= __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f_win)));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_init[i] = 0.f;
+        asm volatile("" : "+v"(s_init));  // (held: as a constant it would be sixteen moves in every step)
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sA[i] -= m_run;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_init[i] = -m_run;
+      }
+      // The largest S of the lane's half row in the step at hand.  As an integer (kWide: not), which is right where any is
+      // positive, and the instruction does not quiet its operands first.
+      using over_t = typename std::conditional<kWide, float, int>::type;
+      over_t s_over = 0;
+      if constexpr (kWide) s_over = s_max0;
       // One step (kB = t % 4 picks the LDS buffers).  Straight-line code apart from small
-      // wavefront-uniform branches, so that the accumulators stay where they are.  Eight slots, each:
-      // one MFMA of S(t+1), one K operand read of step t+2, one MFMA of P(t-1).V(t-1), the V^T operand
-      // needed four slots later, and the softmax of two values of S(t): exp2, rounding, row sum; the
-      // accumulator that held them is set to the reference point for its next use (S(t+2)
-      // accumulates onto -m_run, so that p = exp2(S) with no subtraction).
+      // wavefront-uniform branches, so that the accumulators stay where they are.
       auto do_step = [&](int t, auto buf_tag, f32x16& s_cur, f32x16& s_next, u32x4 (&p_prev)[2], u32x4 (&p_cur)[2]) __attribute__((always_inline)) {
         constexpr int kB = decltype(buf_tag)::value;
-        // V(t) and K(t+2), first read in this step, were requested two barriers ago: they have landed
-        // once only the four copies of the last barrier are outstanding; after the barrier that holds
-        // for every wavefront
-        __builtin_amdgcn_s_waitcnt(0x0f70 | 4);  // vmcnt(4)
-        // (the buffers that this step's copies overwrite were last read in the first half of step t-1:
-        // the twelve operand reads of its second half may still be in flight)
-        __builtin_amdgcn_s_waitcnt(0xcc7f);  // lgkmcnt(12)
+        // V(t-1) and K(t+2), first read in this step, have landed once only what was asked for after them is outstanding:
+        // V(t) of step t-2 and the four copies of step t-1 (K goes first in every step); after the barrier that holds for
+        // every wavefront.  The buffers that this step's copies overwrite, K(t)'s and V(t-2)'s, were last read in steps
+        // t-2 and t-1, for MFMAs that every wavefront has issued by now.
+        __builtin_amdgcn_s_waitcnt(0x0f70 | 6);  // vmcnt(6)
         __builtin_amdgcn_s_barrier();
-        // this step's copies: V(t+2) into the buffer of V(t-2) and K(t+4) into the buffer of K(t), both
-        // last read in step t-1.  Their scalar offsets are worked out here from the block numbers held
-        // in scalar registers; the four instructions go out between the MFMAs below (V first, then
-        // K).  Steps past the row's end copy a block again or nothing (see the descriptors).
+        // This step's copies: K(t+4) and V(t+2).  Their scalar offsets are worked out here from the block numbers held
+        // in scalar registers.  Steps past the row's end copy a block again or nothing (see the descriptors).
         const uint32_t v_soff = static_cast<uint32_t>(((kB + 2) < 4 ? blk0 : blk1) * kBlockKV + ((kB + 2) & 3) * kStep) * v_sn2;
         const uint32_t k_soff = static_cast<uint32_t>(blk1 * kBlockKV + kB * kStep) * k_sn2;
         // (a row is padded to a multiple of four steps; a padded step has no keys: p = 0, against V
         // operands read from buffers that hold earlier steps of the same row)
         const int valid = t < n_steps ? min(kStep, kv_len - (blk0 * kBlockKV + kB * kStep)) : 0;
-        if (valid < kStep) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int kv = (i >> 2) * 8 + g * 4 + (i & 3);
-            if (kv >= valid) s_cur[i] = -INFINITY;  // p = 0
-          }
+        if (valid < kStep) mask_tail(s_cur, valid);
+        // The reference point moves only past a 2^8 overshoot (a rare, wavefront-uniform branch that changes registers in
+        // place): S(t), what S(t+1) accumulates from and the row sum move now; O, which still receives P(t-1).V(t-1) at
+        // the old point in this step, is rescaled at the step's end.
+        bool over;
+        if constexpr (kWide) {
+          over = __builtin_fmaf(s_over, f_blk, -m_run) > kLazyLog2;
+        } else {
+          over = s_over > __builtin_bit_cast(int, kLazyLog2);
         }
-        float mx = s_cur[0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s_cur[i]);
-        mx = max_across_halves(mx);  // row max relative to m_run
-        // (kWide: S is the plain product, its factor positive: the largest logit is the one of the largest S)
-        if constexpr (kWide) mx = __builtin_fmaf(mx, f_blk, -m_run);
-        const bool first = t == 0;
-        // The reference point moves always on a row's first step, afterwards only past a 2^8
-        // overshoot (a rare, wavefront-uniform branch that changes registers in place): S(t), the
-        // accumulator of S(t+1), which holds the old point, and the row sum move now; O, which still
-        // receives P(t-1).V(t-1) at the old point in this step, is rescaled at the step's end.
-        const bool moved = first || __builtin_expect(__any(mx > kLazyLog2), 0);
+        const bool moved = __builtin_expect(__any(over), 0);
         float o_scale = 1.f;
         if (moved) {
-          const float delta = first ? mx : fmaxf(mx, 0.f);
-          if (!first) {
-            o_scale = __builtin_amdgcn_exp2f(-delta);
-            d_part *= o_scale;
-          }
+          float mx = row_max(s_cur);  // row max relative to m_run
+          if constexpr (kWide) mx = __builtin_fmaf(mx, f_blk, -m_run);
+          const float delta = fmaxf(mx, 0.f);
+          o_scale = __builtin_amdgcn_exp2f(-delta);
+          d_part *= o_scale;
           m_run += delta;
           if constexpr (!kWide) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) s_cur[i] -= delta;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s_next[i] -= delta;
+            for (int i = 0; i < 16; ++i) s_init[i] -= delta;
           }
         }
-        const f32x2 neg_m2 = {-m_run, -m_run};
-        // (made opaque once per step: otherwise the eight read offsets are worked out once per
-        // kernel and live in eight registers, which the loop does not have)
-        uint32_t kx = kx0;
-        asm volatile("" : "+v"(kx));
+        // The softmax goes in pairs of values, a pair in every second slot: exp2 there, rounding a pair later, the row sum
+        // (over the rounded values, as the reference takes it) another one later, so that nothing waits for the instruction
+        // in front of it.  (The empty statements pin a pair to its slot: without them the compiler gathers all exponentials
+        // of a step in front of its MFMAs.)
         float psum = 0.f;
-        f32x16 s_zero16;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s_zero16[i] = 0.f;
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          s_next = TS::mfma(kop[i & 3], qreg[i], kWide && i == 0 ? s_zero16 : s_next);
-          // the operand of the S MFMA four slots on: second half of K(t+1), then first half of K(t+2)
-          kop[i & 3] = i < 4 ? read_k(kx, (kB + 1) & 3, i + 4) : read_k(kx, (kB + 2) & 3, i - 4);
-          o_acc[i & 3] = TT::mfma(vop[i & 3], __builtin_bit_cast(x8, p_prev[i >> 2]), o_acc[i & 3]);
-          // the operand of the P.V MFMA four slots on: second half of V(t-1), then first half of V(t)
-          vop[i & 3] = i < 4 ? read_v((kB + 3) & 3, 1, i) : read_v(kB, 0, i - 4);
-          // (the two values are pinned to this slot: without the empty statements the compiler
-          // gathers all exponentials of a step in front of its MFMAs)
-          float e0 = s_cur[2 * i], e1 = s_cur[2 * i + 1];
-          if constexpr (kWide) {
-            asm volatile("v_fma_f32 %0, %2, %4, -%5\n\tv_fma_f32 %1, %3, %4, -%5"
-                         : "=&v"(e0), "=v"(e1)
-                         : "v"(s_cur[2 * i]), "v"(s_cur[2 * i + 1]), "s"(f_blk), "v"(m_run));
-          } else {
-            asm volatile("" : "+v"(e0), "+v"(e1));
-          }
-          const x2 pk = {static_cast<T>(__builtin_amdgcn_exp2f(e0)), static_cast<T>(__builtin_amdgcn_exp2f(e1))};
-          uint32_t pu = __builtin_bit_cast(uint32_t, pk);
-          // the row sum is taken over the rounded p, as the reference does
+        float x0, x1;
+        uint32_t pu;
+        auto round_pair = [&]() __attribute__((always_inline)) {
+          const x2 pk = {static_cast<T>(x0), static_cast<T>(x1)};
+          pu = __builtin_bit_cast(uint32_t, pk);
+        };
+        auto add_pair = [&](int u) __attribute__((always_inline)) {
+          const x2 pk = __builtin_bit_cast(x2, pu);
           if constexpr (std::is_same<T, __bf16>::value) {
             psum = __builtin_amdgcn_fdot2_f32_bf16(pk, ones2, psum, false);
           } else {
             psum = __builtin_amdgcn_fdot2(pk, ones2, psum, false);
           }
-          if constexpr (kWide) {
-            asm volatile("" : "+v"(pu), "+v"(psum));
+          p_cur[u >> 2][u & 3] = pu;
+        };
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {
+          const int i = n & 7, u = n >> 1;
+          if (n < 8) {
+            s_next = TS::mfma(__builtin_bit_cast(q8, op[i]), qreg[i], n == 0 ? s_init : s_next);
+            op[i] = __builtin_bit_cast(u32x4, read_v((kB + 3) & 3, i >> 2, i & 3));
           } else {
-            // (the accumulator that held the two values is set to the reference point for its next use)
-            f32x2 r01 = neg_m2;
-            asm volatile("" : "+v"(pu), "+v"(psum), "+v"(r01));
-            s_cur[2 * i] = r01[0];
-            s_cur[2 * i + 1] = r01[1];
+            o_acc[i & 3] = TT::mfma(__builtin_bit_cast(x8, op[i]), __builtin_bit_cast(x8, p_prev[i >> 2]), o_acc[i & 3]);
+            op[i] = __builtin_bit_cast(u32x4, read_k((kB + 2) & 3, i));
           }
-          p_cur[i >> 2][i & 3] = pu;
-          if (i == 1 || i == 3) {
-            copy_desc(v_rsrc, v_voff, v_soff + (i >> 1) * 16 * v_sn2, m0_base + vbuf((kB + 2) & 3) + (i >> 1) * 4096);
-          } else if (i == 5 || i == 7) {
-            copy_desc(k_rsrc, k_voff, k_soff + ((i - 4) >> 1) * 16 * k_sn2, m0_base + kbuf(kB) + ((i - 4) >> 1) * 4096);
+          // softmax of two values of S(t)
+          if (n & 1) {
+            if (u == 0) {
+              asm volatile("" : "+v"(s_cur));
+            } else if (u == 1) {
+              asm volatile("" : "+v"(s_cur), "+v"(x0), "+v"(x1));
+            } else {
+              asm volatile("" : "+v"(s_cur), "+v"(x0), "+v"(x1), "+v"(pu), "+v"(psum));
+            }
+            float e0 = s_cur[2 * u], e1 = s_cur[2 * u + 1];
+            if (u >= 2) add_pair(u - 2);
+            if (u >= 1) round_pair();
+            if constexpr (kWide)
+              asm volatile("v_fma_f32 %0, %2, %4, -%5\n\tv_fma_f32 %1, %3, %4, -%5"
+                           : "=&v"(e0), "=v"(e1)
+                           : "v"(s_cur[2 * u]), "v"(s_cur[2 * u + 1]), "s"(f_blk), "v"(m_run));
+            x0 = __builtin_amdgcn_exp2f(e0);
+            x1 = __builtin_amdgcn_exp2f(e1);
+          }
+          if (n >= 12) {
+            auto bits = [&](int j) __attribute__((always_inline)) { return __builtin_bit_cast(over_t, static_cast<float>(s_next[j])); };
+            auto larger = [](over_t a, over_t b) __attribute__((always_inline)) {
+              if constexpr (kWide) return fmaxf(a, b);
+              else return max(a, b);
+            };
+            if (n == 12) s_over = larger(larger(bits(0), bits(1)), bits(2));
+            if (n == 13) s_over = larger(larger(larger(larger(s_over, bits(3)), bits(4)), bits(5)), bits(6));
+            if (n == 14) s_over = larger(larger(larger(larger(s_over, bits(7)), bits(8)), bits(9)), bits(10));
+            if (n == 15) s_over = larger(larger(larger(larger(larger(s_over, bits(11)), bits(12)), bits(13)), bits(14)), bits(15));
+          }
+          // The MFMAs of S go first where the other workgroup's wavefront on this SIMD has one of P.V or softmax work ready:
+          // 1733 -> 1712 us on the video-sized list (the other way round 1751; the line two or three slots earlier or later
+          // 1730 to 1738).
+          if (n == 7) __builtin_amdgcn_s_setprio(0);
+          if (n == 15) __builtin_amdgcn_s_setprio(1);
+          // (all four copies among the MFMAs of S 1747, all among those of P.V 1736, every fourth slot from 1 / 2 on 1724 / 1754)
+          if (n == 1 || n == 5) {
+            copy_desc(k_rsrc, k_voff, k_soff + (n >> 2) * 16 * k_sn2, m0_k + kbuf(kB) + (n >> 2) * (4 * kPipeKRows4));
+          } else if (n == 8 || n == 11) {
+            copy_desc(v_rsrc, v_voff, v_soff + (n > 8) * 16 * v_sn2, m0_v + vbuf((kB + 2) & 3) + (n > 8) * 4096);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
+        add_pair(6);
+        round_pair();
+        add_pair(7);
+        asm volatile("" : "+v"(psum), "+v"(p_cur[1][2]), "+v"(p_cur[1][3]), "+v"(s_over));
         d_part += psum;
-        if (moved && !first) {
+        if (moved) {
 #pragma unroll
           for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -1676,14 +1727,15 @@ sparse_fa_kernel(const FaParams p) {
         do_step(t + 2, B2{}, sA, sB, pB, pA);
         do_step(t + 3, B3{}, sB, sA, pA, pB);
       }
-      // P.V of the last step (real or padded; its V is in buffer 3, vop holds the first half)
+      __builtin_amdgcn_s_setprio(0);
+      // P.V of the last step (real or padded; its V is in buffer 3)
+      __builtin_amdgcn_s_waitcnt(0x0f70 | 6);  // vmcnt(6)
+      __builtin_amdgcn_s_barrier();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o_acc[i] = TT::mfma(vop[i], __builtin_bit_cast(x8, pB[0]), o_acc[i]);
-        vop[i] = read_v(3, 1, i);
-      }
+      for (int i = 0; i < 8; ++i) op[i] = __builtin_bit_cast(u32x4, read_v(3, i >> 2, i & 3));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o_acc[i] = TT::mfma(vop[i], __builtin_bit_cast(x8, pB[1]), o_acc[i]);
+      for (int i = 0; i < 8; ++i)
+        o_acc[i & 3] = TT::mfma(__builtin_bit_cast(x8, op[i]), __builtin_bit_cast(x8, pB[i >> 2]), o_acc[i & 3]);
       // The copies of the steps past the row's end (the loop asks for K four and V two steps ahead,
       // whatever is left of the row) are still in flight: they must have landed before the epilogue
       // lays the finished row out in the same LDS.  (Nothing else waits for them: the barrier below

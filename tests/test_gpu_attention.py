@@ -627,6 +627,51 @@ def test_logits_far_apart(dev, dtype, fp8, nk):
     assert float(out.abs().max()) <= float(v.abs().max()) * 1.02
 
 
+@pytest.mark.parametrize("terms", ["bf16", "fp16", "fp8"])
+def test_rows_of_few_steps(dev, terms):
+    """Rows of one to nine steps of 32 keys, at both sides of every border, whose logits grow from step to step in one
+    request and fall in the next; the row before q's end holds infinities (16-bit), which must not reach the other rows
+    through the buffers that q passes through on its way to registers."""
+    import flashomni_amd as fo
+    kl = [1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 255, 256, 257]
+    ql, heads = [130] * len(kl), 2
+    dtype = torch.float16 if terms == "fp16" else torch.bfloat16
+    m = make_ragged_masks(ql, kl, heads, 1.0, 1.0, seed=33)
+    g = torch.Generator().manual_seed(33)
+    nq, nk = sum(ql), sum(kl)
+    q = torch.randn(nq, heads, 128, generator=g) + 0.5
+    k = torch.randn(nk, heads, 128, generator=g) * 0.5
+    # a drift along q's mean of up to 34 in the log2 domain: 0.5 * 128 * 128^-0.5 * log2(e) = 8.2 per unit
+    k = k + torch.cat([torch.linspace(-2, 2, n) * (1 if i % 2 else -1) for i, n in enumerate(kl)]).view(-1, 1, 1)
+    q, k, v = q.to(dtype), k.to(dtype), torch.randn(nk, heads, 128, generator=g).to(dtype)
+    ok = torch.ones(nq, dtype=torch.bool)
+    extra = {}
+    if terms == "fp8":
+        q, qs, q_lo = fo.quant_fp8_block(q.to(dev), torch.from_numpy(m["qo_indptr"]), residual=True)
+        k, ks, k_lo = fo.quant_fp8_block(k.to(dev), torch.from_numpy(m["kv_indptr"]), residual=True)
+        q, k, extra = q.cpu(), k.cpu(), {n: x.cpu() for n, x in dict(q_scale=qs, k_scale=ks, q_lo=q_lo, k_lo=k_lo).items()}
+    else:
+        ok[torch.from_numpy(m["qo_indptr"][1:].copy()).long() - 2] = False
+        q[~ok] = float("inf")
+    t = lambda a: torch.from_numpy(a).to(dev)
+    sym = [m[x] for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t(m["qo_indptr"]), t(m["kv_indptr"]), heads, heads, 128, q_data_type=q.dtype)
+    out, lse = w.run(q.to(dev), k.to(dev), v.to(dev), *(t(x) for x in sym), return_lse=True,
+                     **{n: x.to(dev) for n, x in extra.items()})
+    exp_lse = torch.full((nq, heads), float("nan"))
+    exp = oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=torch.zeros(nq, heads, 128, dtype=dtype),
+                                  lse=exp_lse, **extra)
+    out, lse = out.cpu(), lse.cpu()
+    # per request: a short one must not hide behind the long ones.  (A logit of up to 20 in the log2 domain is off by 2^-9
+    # of its products' root sum of squares, about 20 * 2^-9 / sqrt(128) * 3: 1e-2, so an output of unit size by as much.)
+    for r in range(len(kl)):
+        a, b = int(m["qo_indptr"][r]), int(m["qo_indptr"][r + 1])
+        rows = ok[a:b]
+        assert rel_l2(out[a:b][rows], exp[a:b][rows]) <= 2 * REL_L2, kl[r]
+        assert float((lse[a:b][rows] - exp_lse[a:b][rows]).abs().max()) < 5e-2, kl[r]
+
+
 def _split_case(dev, ql, kl, heads, seed, share, dtype=torch.bfloat16, pk=0.6):
     """Run one launch (twice, to see the arrival counters re-armed) with or without rows shared
     between workgroups; returns (out, lse, sched words, expectations)."""
