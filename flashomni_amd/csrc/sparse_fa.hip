@@ -400,7 +400,7 @@ constexpr int kDirectMaxFull = 1408;    // ... where every row is computed whole
 constexpr int kDirectShareRows = 1024;  // rows of a share that the table of them holds (see direct_table_holds)
 constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
 constexpr int kDirectMapBytes = (1 << 16) - 16;  // keep bits that are staged in the tile buffers (both forms have as much)
-constexpr int kOlderGain = 10;  // see cut_at
+constexpr int kOlderGain = 4;  // see cut_at
 constexpr int kPartExtra = 2, kEvenExtra = 5;  // what cutting rows costs a workgroup, in kv blocks (see direct_schedule)
 constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologue, epilogue and exchange cost about as many
 
@@ -779,9 +779,10 @@ sparse_fa_kernel(const FaParams p) {
   };
   // Share j of `shares` begins at cost cut_at(j) (products below 2^30: at most 2^20 keep bits, 512 shares);
   // share_of is the share that holds a unit of cost.  Where two workgroups share a CU the one that was launched
-  // first is ahead of the other throughout (its wavefronts are older and go first: 126 against 146 us with equal
+  // first is ahead of the other throughout (its wavefronts are older and go first: 126.0 against 130.9 us with equal
   // shares, and the younger one then runs alone on its CU, at two thirds of the pair's rate), so the shares of an
-  // XCD's first half are longer by kOlderGain / 128 and those of the second half shorter.
+  // XCD's first half are longer by kOlderGain / 128 and those of the second half shorter: ends at 121.4 and 122.3 us.
+  // (Before the MFMAs of S had priority, whichever workgroup they are of, 126 and 146 us, and 10 / 128 was the best.)
   auto cut_at = [&](int j, int total, int shares) {
     if constexpr (kPipe) {
       const int per = shares / kXcds;
