@@ -111,6 +111,9 @@ struct Types<__bf16> {
   static __device__ __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f32x4 mfma16(x8 a, x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
 };
 template <>
 struct Types<_Float16> {
@@ -118,6 +121,9 @@ struct Types<_Float16> {
   using x4 = f16x4;
   static __device__ __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 mfma16(x8 a, x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
 };
 
@@ -2086,6 +2092,13 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
 //
 // What bounds it: LDS and the matrix cores together (96 KB read, 48 KB written per slab of two units beside 1024 cycles of
 // MFMA) and, over long launches, power: dense it takes the time of full quads to 5 % (GEMM-Q's rule in launch_q).
+//
+// Tiles of 16 x 16 over 32 of k: an accumulator is read and written once per 32 of k instead of once per 16, and the card
+// sustains 1.98 PFLOP/s of them on random operands against 1.76 of 32 x 32 x 16 (registers only, all CUs, both at the power limit;
+// with zeros both reach 2.42).  GEMM-O of 76 112 x 5120 with 80 % 2835 -> 2640 us, of 4608 x 3072, both passes, 97.5 -> 94.
+// They are worth it where two wavefronts share a SIMD and the vector ALU has nothing else to issue: quads, one wavefront to a
+// SIMD, wait for their own loads with 16 cycles of MFMA in flight instead of 32 (GEMM-Q of 76 112 x 5120 2940 -> 3230), and the
+// attention loop's exponentials want the issue slots that twice as many MFMAs take (33 k tokens x 24 heads 1709 -> 1785).
 // ---------------------------------------------------------------------------------------------
 constexpr int kStripPiece = 2 * 32 * kRowBytes;  // 32 rows of W of both column blocks
 constexpr int kStripRing = 6;
@@ -2097,12 +2110,12 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
   using TT = Types<T>;
   using x8 = typename TT::x8;
   using x4 = typename TT::x4;
-  constexpr int NT = 4, MT = 2;  // wavefront tile: 128 columns (W rows) x 64 token rows (X rows)
+  constexpr int NT = 8, MT = 4;  // wavefront tile: 128 columns (W rows) x 64 token rows (X rows), 16 x 16 each
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, g = lane >> 5;
+  const int l16 = lane & 15, g = lane >> 4;
   const int wr = wv >> 1, wc = wv & 1;  // half of the rows; column block
 
   if (!kReduce && p.judgement != nullptr && *p.judgement != 0) return;  // (computed as quads)
@@ -2318,28 +2331,28 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
     copy(r, voff[i & 1], koff + w_soff + (4 * nt + i) * row8, w_dst + at + i * 8 * kRowBytes);
   };
 
-  // acc[nt][mt][i]: column nt*32 + (i/4)*8 + g*4 + i%4 of the block, row wr*64 + mt*32 + l32
-  f32x16 acc[NT][MT];
+  // acc[ct][mt][i]: column ct*16 + g*4 + i of the block, row wr*64 + mt*16 + l16
+  f32x4 acc[NT][MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
+      for (int i = 0; i < 4; ++i) acc[nt][mt][i] = 0.f;
 
   if (n_iter > 0) {
     typedef __attribute__((address_space(3))) const x8 lds_x8;
-    const int rd_x = (g ^ ((l32 >> 1) & 7)) << 4;
-    uint32_t lane_off[4];
+    // an operand: 16 rows, 32 of k (ks); lane: row l16, 16-byte chunk 4*ks + g
+    uint32_t lane_off[2];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) lane_off[ks] = static_cast<uint32_t>(l32 * kRowBytes + (rd_x ^ (ks << 5)));
+    for (int ks = 0; ks < 2; ++ks) lane_off[ks] = static_cast<uint32_t>(l16 * kRowBytes + (((4 * ks + g) ^ (l16 >> 1)) << 4));
     const uint32_t x_src = lds0 + wr * 64 * kRowBytes, w_src = ldsw + wc * 32 * kRowBytes;
-    x8 xr_[MT][4], wreg[2][4];
+    x8 xr_[MT][2], wreg[2][2][2];
     auto read_x = [&](int mt, int ks, uint32_t buf) __attribute__((always_inline)) {
-      xr_[mt][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (x_src + buf) + mt * 32 * kRowBytes));
+      xr_[mt][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (x_src + buf) + mt * 16 * kRowBytes));
     };
-    auto read_w = [&](int set, int ks, uint32_t at) __attribute__((always_inline)) {
-      wreg[set][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (w_src + at)));
+    auto read_w = [&](int set, int ct, int ks, uint32_t at) __attribute__((always_inline)) {
+      wreg[set][ct][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (w_src + at) + ct * 16 * kRowBytes));
     };
     // prologue: X of slab 0, pieces 0 to 2 | pieces 3 and 4, X of slab 1
     Slab sa = next_slab(), sb = sa;  // slabs it, it + 1
@@ -2363,13 +2376,10 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
     __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
     __builtin_amdgcn_s_barrier();
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) read_w(0, ks, 0);
+    for (int j = 0; j < 4; ++j) read_w(0, j & 1, j >> 1, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      read_x(0, ks, 0);
-      read_x(1, ks, 0);
-    }
+    for (int j = 0; j < 8; ++j) read_x(j & 3, j >> 2, 0);
     __builtin_amdgcn_sched_barrier(0);
     uint32_t ring = 0;  // place of the slab's first piece
     uint32_t xbuf = 0;
@@ -2388,27 +2398,25 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
         constexpr int nt = decltype(nt_tag)::value, set = nt & 1;
         const uint32_t rd = place(nt + 1);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int ks = j >> 1, mt = j & 1;
+        for (int j = 0; j < 16; ++j) {
+          const int ks = j >> 3, ct = (j >> 2) & 1, mt = j & 3;
           if constexpr (kHalf && nt == 0) {
-            u32x4 v = __builtin_bit_cast(u32x4, xr_[mt][ks]);
-            v &= ks < 2 ? sa.first : sa.second;
-            xr_[mt][ks] = __builtin_bit_cast(x8, v);
-          }
-          acc[nt][mt] = TT::mfma(wreg[set][ks], xr_[mt][ks], acc[nt][mt]);
-          if (j < 4) read_w(set ^ 1, j, rd);
-          if constexpr (nt == 3) {
-            if (j & 1) {
-              read_x(0, ks, xbuf ^ kUnitBytes);
-              read_x(1, ks, xbuf ^ kUnitBytes);
+            if (ct == 0) {
+              u32x4 v = __builtin_bit_cast(u32x4, xr_[mt][ks]);
+              v &= ks == 0 ? sa.first : sa.second;
+              xr_[mt][ks] = __builtin_bit_cast(x8, v);
             }
           }
+          acc[2 * nt + ct][mt] = TT::mfma16(wreg[set][ct][ks], xr_[mt][ks], acc[2 * nt + ct][mt]);
+          if (j < 8 && !(j & 1)) read_w(set ^ 1, (j >> 1) & 1, j >> 2, rd);
+          if constexpr (nt == 3)
+            if (ct == 1) read_x(mt, ks, xbuf ^ kUnitBytes);
           if constexpr (nt == 0) {
-            if (j & 1) copy_w(rw1, 1 + (j >> 2), (j >> 1) & 1, sb.k, place(5 + (j >> 2)));
+            if ((j & 3) == 3) copy_w(rw1, 1 + (j >> 3), (j >> 2) & 1, sb.k, place(5 + (j >> 3)));
           } else if constexpr (nt == 1) {
-            if (j & 1) copy_x(rx2, j >> 1, sc.k, xbuf);
+            if ((j & 3) == 3) copy_x(rx2, j >> 2, sc.k, xbuf);
           } else {
-            if (j == 2 || j == 5) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, j == 5, nt == 2 ? sb.k : sc.k, place(5 + nt));
+            if (j == 5 || j == 11) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, j == 11, nt == 2 ? sb.k : sc.k, place(5 + nt));
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -2459,7 +2467,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
     }
     const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
+    for (int mt = 0; mt < MT / 2; ++mt) {  // (32 rows)
       // (rows whose partial is in flight together: sixteen of fp32 do not fit beside the accumulators)
       constexpr int kAhead = kBytes == 4 ? 8 : 16;
       BiasVec bm[kAhead];
@@ -2478,14 +2486,11 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       if constexpr (kPartial) load_partial(0);
       // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 512 bytes = 32 chunks)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+      for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          f32x4 v;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = acc[nt][mt][i4 * 4 + j];
-          const int chunk = nt * 8 + i4 * 2 + g;
-          *reinterpret_cast<f32x4*>(region + l32 * 512 + ((chunk ^ (l32 & 15)) << 4)) = v;
+        for (int half = 0; half < 2; ++half) {
+          const int r = half * 16 + l16, chunk = ct * 4 + g;
+          *reinterpret_cast<f32x4*>(region + r * 512 + ((chunk ^ (r & 15)) << 4)) = acc[ct][2 * mt + half];
         }
       f32x4 vals[8];
 #pragma unroll
