@@ -372,9 +372,11 @@ struct BitRange {
   int first, n;
   // (at most 2^20 keep bits: 32-bit positions)
   __device__ __forceinline__ BitRange(const uint8_t* seg, uint32_t bit, int n_) : n(n_) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(seg) + (bit >> 3);
-    words = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
-    first = static_cast<int>(a & 3) * 8 + static_cast<int>(bit & 7);
+    // (by steps from the pointer: one made from a number would be of an unknown address space, whose loads wait for LDS too)
+    const uint8_t* const a = seg + (bit >> 3);
+    const int skew = static_cast<int>(reinterpret_cast<uintptr_t>(a) & 3);
+    words = reinterpret_cast<const uint32_t*>(a - skew);
+    first = skew * 8 + static_cast<int>(bit & 7);
   }
   __device__ __forceinline__ int count() const { return (first + n + 31) >> 5; }
   __device__ __forceinline__ uint32_t trim(uint32_t v, int i) const {
@@ -389,7 +391,7 @@ struct BitRange {
 // launch at 76 k tokens x 40 heads 1 %): the row's keep bits (words, position of its first bit, kv blocks
 // of the request); ptr0 is then the first kept block of this part among the row's kept blocks
 struct DirectMask {
-  const uint32_t* mask;
+  int mask;  // in words from the first whole word at or in front of the keep bits' pointer
   int mask_first, nkv;
 };
 struct NoMask {};
@@ -755,35 +757,41 @@ sparse_fa_kernel(const FaParams p) {
   //     whole rows, 338 in shares; 160 rows of 64 blocks 139 -> 92.)
   // In the pipelined form the next item is fetched beside a row's first copies instead of at its end, where the
   // trips to memory are 2.4 us that nothing hides.
-  __shared__ int s_wave[4 + kDirectMaxParts / 2][8];
+  __shared__ int s_wave[6][8];
   // even shares: the rows of this workgroup's share, where there may be more than the table holds row i at i % kDirectShareRows
   __shared__ uint16_t s_row_cand[kDirect ? kDirectShareRows : 1];  // a row's candidate ...
   __shared__ int s_row_u[kDirect ? kDirectShareRows + 1 : 1];      // ... and the cost at which its kv blocks begin
   auto row_at = [](int i) { return kMany ? i & (kDirectShareRows - 1) : i; };
   constexpr int kMaxCand = direct_max_cand(kMany);
   __shared__ uint16_t s_zero[kDirect ? kMaxCand / 16 : 1];         // candidates this workgroup clears (of 16 or more)
-  // first row of the share, candidates to clear; even shares: the row behind its last one (0: one item at most), shares, cost of all
+  // first row of the share, candidates to clear; even shares: the row behind its last one (0: one item at most), shares, cost of all,
+  // the share's bounds
   // (in LDS and not in registers, where they would live through the main loop)
-  __shared__ int s_dir[5];
+  __shared__ int s_dir[7];
   __shared__ int s_list_at;  // whole parts: where the item's keep bits are in LDS (words from smem on), or -1
+  __shared__ int s_map[2];   // the piece of keep bits in the tile buffers until the first row: first word (as in DirectMask), words
+  // even shares, pipelined form: keep bits of the items at hand, where they are no more than this (fetched with the items: a list that is made
+  // beside a row's first copies must not wait for a load, which comes back behind them)
+  constexpr int kBitWords = 34;
+  __shared__ uint32_t s_bits[kDirect && kPipe ? kItemBatch : 1][kBitWords];
   __shared__ int s_ends[5];  // a batch of one request: its q and kv tokens, where its keep bits begin
+  const uint8_t* const kv_info_words = kDirect && p.kv_info ? p.kv_info - (reinterpret_cast<uintptr_t>(p.kv_info) & 3) : nullptr;
   // this workgroup's share: neighbouring ones on one XCD
   auto dir_index = [&]() {
     return (gridDim.x & (kXcds - 1)) == 0 ? (blockIdx.x & (kXcds - 1)) * (gridDim.x / kXcds) + blockIdx.x / kXcds
                                           : static_cast<int>(blockIdx.x);
   };
-  // floor(a / d) for a < 2^20: with half a unit added the quotient is further from a whole number than the
+  // floor(a / d) for a < 2^21: with half a unit added the quotient is further from a whole number than the
   // reciprocal's error
   auto part_of = [](int a, int d) {
     return static_cast<int>((static_cast<float>(a) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(d)));
   };
-  // Share j of `shares` begins at cost cut_at(j) (products below 2^30: at most 2^20 keep bits, 512 shares);
-  // share_of is the share that holds a unit of cost.  Where two workgroups share a CU the one that was launched
+  // Share j of `shares` begins at cost cut_at(j) (products below 2^30: at most 2^20 keep bits, 512 shares).  Where two workgroups share a CU the one that was launched
   // first is ahead of the other throughout (its wavefronts are older and go first: 126.0 against 130.9 us with equal
   // shares, and the younger one then runs alone on its CU, at two thirds of the pair's rate), so the shares of an
   // XCD's first half are longer by kOlderGain / 128 and those of the second half shorter: ends at 121.4 and 122.3 us.
   // (Before the MFMAs of S had priority, whichever workgroup they are of, 126 and 146 us, and 10 / 128 was the best.)
-  auto cut_at = [&](int j, int total, int shares) {
+  auto cut_at = [&](int j, int total, int shares) __attribute__((always_inline)) {
     if constexpr (kPipe) {
       const int per = shares / kXcds;
       if (shares == static_cast<int>(gridDim.x) && per * kXcds == shares && (per & 1) == 0) {
@@ -795,16 +803,8 @@ sparse_fa_kernel(const FaParams p) {
     }
     return static_cast<int>(static_cast<uint32_t>(j) * total / shares);
   };
-  auto share_of = [&](int at, int total, int shares) {
-    int j = static_cast<int>((static_cast<uint32_t>(at + 1) * shares - 1) / total);
-    if constexpr (kPipe) {
-      while (cut_at(j, total, shares) > at) --j;
-      while (j + 1 < shares && cut_at(j + 1, total, shares) <= at) ++j;
-    }
-    return j;
-  };
   // everything about candidate `cand` but its part
-  auto direct_row = [&](int cand, RowInfo& it) {
+  auto direct_row = [&](int cand, RowInfo& it) __attribute__((always_inline)) {
     const int h = part_of(cand, p.n_blk), t = cand - h * p.n_blk;
     it.row = cand;
     it.req = p.batch == 1 ? 0 : p.blk_req[t];
@@ -817,12 +817,12 @@ sparse_fa_kernel(const FaParams p) {
     it.kv_len = (one ? s_ends[3] : p.kv_indptr[it.req + 1]) - it.kv_begin;
     if constexpr (kDirect) {
       it.nkv = (it.kv_len + kBlockKV - 1) / kBlockKV;
-      it.mask = nullptr;
+      it.mask = 0;
       it.mask_first = 0;
       if (!p.is_full) {
         const BitRange r(p.kv_info + (one ? s_ends[4] : p.kv_info_indptr[it.req]),
                          static_cast<uint32_t>(it.qb * p.symbol_heads + h) * it.nkv, it.nkv);
-        it.mask = r.words;
+        it.mask = static_cast<int>(r.words - reinterpret_cast<const uint32_t*>(kv_info_words));
         it.mask_first = r.first;
       }
     }
@@ -838,50 +838,78 @@ sparse_fa_kernel(const FaParams p) {
     const int first_cand = kCands * tid;
     if (tid < kItemBatch) s_items[tid].row = -1;
     if (tid == 0) s_next_row[0].row = -1;
+    // What this costs is instructions: every wavefront goes through all of it, and 2300 of them are 5 us.
     int list_at[kCands];  // where a candidate's keep bits are in LDS (words from smem on), or -1
     bool act[kCands];
-    int n[kCands], nkv[kCands];
-    constexpr int kAhead = 3, kOwnWords = 0x10000;  // words that a thread asks for itself
-    uint32_t own[kCands][kAhead];
+    int n[kCands], map_word = 0, map_words = 0;
+    const bool one = p.batch == 1;
     {
-      // All of a thread's candidates make their trips to memory together.  Where the keep bits are more than two
-      // words to a candidate they come as one piece into the tile buffers, which nothing uses yet.  (Candidate
-      // after candidate and word after word, 864 candidates took 14 us until the first row began; now 8.)
-      int req[kCands], bit[kCands];
+      // All of a thread's candidates make their trips to memory together: request, where it begins, flags and keep bits.
+      // The keep bits come as one piece into the tile buffers, which nothing uses yet, where they fit.
+      int req[kCands], bit[kCands], nkv[kCands];
+      const int cand0 = min(first_cand, n_cand - 1);
+      int h = part_of(cand0, p.n_blk), t = cand0 - h * p.n_blk;
 #pragma unroll
       for (int u = 0; u < kCands; ++u) {
-        const int cand = min(first_cand + u, n_cand - 1);
-        const int h = part_of(cand, p.n_blk), t = cand - h * p.n_blk;
-        req[u] = p.batch == 1 ? 0 : p.blk_req[t];
-        bit[u] = (p.batch == 1 ? t : p.blk_qb[t]) * p.symbol_heads + h;
-      }
-      if (p.batch == 1 && tid == 0) {
-        s_ends[0] = p.qo_indptr[0];
-        s_ends[1] = p.qo_indptr[1];
-        s_ends[2] = p.kv_indptr[0];
-        s_ends[3] = p.kv_indptr[1];
-        s_ends[4] = p.is_full ? 0 : p.kv_info_indptr[0];
-      }
-#pragma unroll
-      for (int u = 0; u < kCands; ++u) {
-        nkv[u] = (p.kv_indptr[req[u] + 1] - p.kv_indptr[req[u]] + kBlockKV - 1) / kBlockKV;
+        req[u] = one ? 0 : p.blk_req[t];
+        bit[u] = (one ? t : p.blk_qb[t]) * p.symbol_heads + h;
         act[u] = first_cand + u < n_cand;
-        n[u] = act[u] ? nkv[u] : 0;
+        // (the next one, head by head; behind the last the last head again)
+        const bool wrap = ++t == p.n_blk;
+        t = wrap ? 0 : t;
+        h = wrap ? min(h + 1, p.symbol_heads - 1) : h;
       }
+      int ends[5] = {0, 0, 0, 0, 0}, map_lo = 0, map_hi = 0, info_at = 0;
       if (!p.is_full) {
+        map_lo = p.kv_info_indptr[0];
+        map_hi = p.kv_info_indptr[p.batch];
+        info_at = p.info_indptr[0];
+      }
+      if (one) {
+        ends[0] = p.qo_indptr[0];
+        ends[1] = p.qo_indptr[1];
+        ends[2] = p.kv_indptr[0];
+        ends[3] = p.kv_indptr[1];
+        ends[4] = map_lo;
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) nkv[u] = (ends[3] - ends[2] + kBlockKV - 1) / kBlockKV;
+      } else {
+#pragma unroll
+        for (int u = 0; u < kCands; ++u)
+          nkv[u] = (p.kv_indptr[req[u] + 1] - p.kv_indptr[req[u]] + kBlockKV - 1) / kBlockKV;
+      }
+      if (p.is_full) {
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) n[u] = act[u] ? nkv[u] : 0;
+        if (one && tid == 0)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) s_ends[i] = ends[i];
+      } else {
         int keep_at[kCands];
         uint8_t flags[kCands];
+        if (one) {
+          const uint8_t* const info = p.info + info_at;
 #pragma unroll
-        for (int u = 0; u < kCands; ++u) {
-          keep_at[u] = p.kv_info_indptr[req[u]];
-          flags[u] = p.info[p.info_indptr[req[u]] + (bit[u] >> 3)];
+          for (int u = 0; u < kCands; ++u) {
+            keep_at[u] = ends[4];
+            flags[u] = info[bit[u] >> 3];
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < kCands; ++u) {
+            keep_at[u] = p.kv_info_indptr[req[u]];
+            flags[u] = p.info[p.info_indptr[req[u]] + (bit[u] >> 3)];
+          }
         }
-        const int map_lo = p.kv_info_indptr[0], map_hi = p.kv_info_indptr[p.batch], map_bytes = map_hi - map_lo;
-        if (map_bytes > 8 * n_cand && map_bytes <= kDirectMapBytes) {
-          const uintptr_t at = reinterpret_cast<uintptr_t>(p.kv_info) + map_lo;
-          const int skew = static_cast<int>(at & 3);
-          const uint32_t* src = reinterpret_cast<const uint32_t*>(at & ~uintptr_t(3));
+        const int map_bytes = map_hi - map_lo;
+        const uint8_t* const at = p.kv_info + map_lo;
+        const int skew = static_cast<int>(reinterpret_cast<uintptr_t>(at) & 3);
+        const bool staged = map_bytes <= kDirectMapBytes;
+        if (staged) {
+          const uint32_t* src = reinterpret_cast<const uint32_t*>(at - skew);
           const int n_words = (skew + map_bytes + 3) >> 2;
+          map_word = static_cast<int>(src - reinterpret_cast<const uint32_t*>(kv_info_words));
+          map_words = n_words;
           uint32_t* dst = reinterpret_cast<uint32_t*>(smem);
           for (int i = tid; i < n_words; i += 4 * 64 * kWaves) {
             uint32_t v[4];
@@ -891,91 +919,87 @@ sparse_fa_kernel(const FaParams p) {
             for (int j = 0; j < 4; ++j)
               if (i + j * 64 * kWaves < n_words) dst[i + j * 64 * kWaves] = v[j];
           }
-          __syncthreads();
-          const uint32_t* words[kCands];
-          int first[kCands], left = 0;
-#pragma unroll
-          for (int u = 0; u < kCands; ++u) {
-            act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
-            n[u] = first[u] = 0;
-            words[u] = reinterpret_cast<const uint32_t*>(smem);
-            if (act[u]) {
-              list_at[u] = -1;
-              const uint32_t at_bit = static_cast<uint32_t>(bit[u]) * nkv[u];
-              // (a caller's segments may lie in any order: one outside of the piece is read where it is)
-              if (keep_at[u] >= map_lo && keep_at[u] + static_cast<int>((at_bit + nkv[u] + 7) >> 3) <= map_hi) {
-                const int byte = skew + keep_at[u] - map_lo + static_cast<int>(at_bit >> 3);
-                words[u] += list_at[u] = byte >> 2;
-                first[u] = (byte & 3) * 8 + static_cast<int>(at_bit & 7);
-                left = max(left, (first[u] + nkv[u] + 31) >> 5);
-              } else {
-                const BitRange r(p.kv_info + keep_at[u], at_bit, nkv[u]);
-                for (int i = 0; i < r.count(); ++i) n[u] += __popc(r.trim(r.words[i], i));
-                nkv[u] = 0;
-              }
-            }
-          }
-          for (int i = 0; i < left; ++i)
-#pragma unroll
-            for (int u = 0; u < kCands; ++u) {
-              BitRange r(nullptr, 0, nkv[u]);
-              r.first = first[u];
-              if (act[u] && i < r.count()) n[u] += __popc(r.trim(words[u][i], i));
-            }
-        } else {
-          uint32_t v[kCands][kAhead];
-#pragma unroll
-          for (int u = 0; u < kCands; ++u) {
-            const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
-#pragma unroll
-            for (int i = 0; i < kAhead; ++i) v[u][i] = i < r.count() && nkv[u] > 0 ? r.words[i] : 0u;
-          }
-#pragma unroll
-          for (int u = 0; u < kCands; ++u) {
-            list_at[u] = -1;
-#pragma unroll
-            for (int i = 0; i < kAhead; ++i) own[u][i] = v[u][i];
-            const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
-            act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
-            n[u] = 0;
-            list_at[u] = r.count() <= kAhead ? kOwnWords : -1;
-            if (act[u] && nkv[u] > 0) {
-#pragma unroll
-              for (int i = 0; i < kAhead; ++i)
-                if (i < r.count()) n[u] += __popc(r.trim(v[u][i], i));
-              for (int i = kAhead; i < r.count(); ++i) n[u] += __popc(r.trim(r.words[i], i));
-            }
-          }
         }
+        if (one && tid == 0)
+#pragma unroll
+          for (int i = 0; i < 5; ++i) s_ends[i] = ends[i];
+        __syncthreads();
+        int first[kCands], left = 0;
+        bool beside = false;
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) {
+          act[u] = act[u] && (flags[u] >> (bit[u] & 7)) & 1;
+          n[u] = 0;
+          const uint32_t at_bit = static_cast<uint32_t>(bit[u]) * nkv[u];
+          // (a caller's segments may lie in any order: one outside of the piece is read where it is)
+          const bool inside = staged && keep_at[u] >= map_lo && keep_at[u] + static_cast<int>((at_bit + nkv[u] + 7) >> 3) <= map_hi;
+          const int byte = skew + keep_at[u] - map_lo + static_cast<int>(at_bit >> 3);
+          list_at[u] = inside ? byte >> 2 : -1;
+          first[u] = (byte & 3) * 8 + static_cast<int>(at_bit & 7);
+          if (act[u] && !inside) beside = true;
+          if (act[u] && inside) left = max(left, nkv[u]);
+        }
+        if (beside) {
+#pragma unroll
+          for (int u = 0; u < kCands; ++u)
+            if (act[u] && list_at[u] < 0) {
+              const BitRange r(p.kv_info + keep_at[u], static_cast<uint32_t>(bit[u]) * nkv[u], nkv[u]);
+              for (int i = 0; i < r.count(); ++i) n[u] += __popc(r.trim(r.words[i], i));
+            }
+        }
+        // 32 kept blocks at a time (the word behind the last one is read as well: it is in the buffers, and masked)
+        const uint32_t* words[kCands];
+        uint32_t word[kCands];
+#pragma unroll
+        for (int u = 0; u < kCands; ++u) {
+          nkv[u] = act[u] && list_at[u] >= 0 ? nkv[u] : 0;
+          words[u] = reinterpret_cast<const uint32_t*>(smem) + max(list_at[u], 0);
+          word[u] = words[u][0];
+        }
+        for (int i = 0; i < left; i += 32)
+#pragma unroll
+          for (int u = 0; u < kCands; ++u) {
+            const uint32_t next = words[u][1];
+            ++words[u];
+            const int rest = max(nkv[u] - i, 0);
+            uint32_t v = __builtin_amdgcn_alignbit(next, word[u], first[u]);
+            v = rest >= 32 ? v : v & ~(~0u << rest);
+            n[u] += __popc(v);
+            word[u] = next;
+          }
       }
     }
     if (tid < 3) s_dir[tid] = 0;
-    int rows_mine = 0, n_mine = 0, mx = 0;
+    // rows and kv blocks in one scan: at most 1792 and 2^20 of them
+    constexpr int kBlockBits = 21;
+    static_assert(direct_max_cand(true) < (1 << (32 - kBlockBits)), "rows must fit above the kv blocks");
+    uint32_t mine = 0;
+    int mx = 0;
 #pragma unroll
     for (int u = 0; u < kCands; ++u) {
-      rows_mine += act[u];
-      n_mine += n[u];
+      mine += (static_cast<uint32_t>(act[u]) << kBlockBits) + n[u];
       mx = max(mx, n[u]);
     }
-    const int rows_incl = wave_scan(rows_mine), n_incl = wave_scan(n_mine);
+    const uint32_t incl = static_cast<uint32_t>(wave_scan(static_cast<int>(mine)));
     mx = wave_max(mx);
     if (lane == 63) {
-      s_wave[0][wv] = rows_incl;
-      s_wave[1][wv] = n_incl;
+      s_wave[0][wv] = static_cast<int>(incl);
       s_wave[2][wv] = mx;
     }
     __syncthreads();
-    int rows = 0, blocks = 0, max_n = 0, row = rows_incl - rows_mine, before = n_incl - n_mine;
+    uint32_t all = 0, in_front = incl - mine;
+    int max_n = 0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      if (w < wv) {
-        row += s_wave[0][w];
-        before += s_wave[1][w];
-      }
-      rows += s_wave[0][w];
-      blocks += s_wave[1][w];
+      const uint32_t t = static_cast<uint32_t>(s_wave[0][w]);
+      if (w < wv) in_front += t;
+      all += t;
       max_n = max(max_n, s_wave[2][w]);
     }
+    all = __builtin_amdgcn_readfirstlane(all);
+    max_n = __builtin_amdgcn_readfirstlane(max_n);
+    const int rows = static_cast<int>(all >> kBlockBits), blocks = static_cast<int>(all & ((1u << kBlockBits) - 1));
+    int row = static_cast<int>(in_front >> kBlockBits), before = static_cast<int>(in_front & ((1u << kBlockBits) - 1));
     // q blocks that are not computed are cleared by turns
     if (p.zero_skipped) {
       int skipped = first_cand - row;
@@ -990,36 +1014,42 @@ sparse_fa_kernel(const FaParams p) {
     }
     const int total = kShareRowCost * rows + blocks;
     // (a row in at most four parts: no share is shorter than a third of the longest row)
-    const int shares = max(min(min(n_wg, total), max_n > 0 ? 3 * total / max_n : total), 1);
+    int shares = max(min(n_wg, total), 1);
+    if (3 * total < shares * max_n) shares = max(3 * total / max_n, 1);
     if (rows <= n_wg) {
-      // parts of at most ceil(max_n / k) kv blocks: how many there are for every k
-      // (the finest cut fits where even a row of the most parts in place of every row would)
-      const int finest = max((max_n + kDirectMaxParts - 1) / kDirectMaxParts, kDirectMinPart);
-      const bool fits = rows * (part_of(max(max_n, 1) - 1, finest) + 1) <= n_wg;
-      int longest = fits ? finest : max(max_n, kDirectMinPart);
-      if (!fits) {
-        uint32_t counts[kDirectMaxParts / 2];
+      // Parts of at most `longest` kv blocks, as short as there are workgroups for.  Rows of n blocks make no more than n / longest
+      // + 1 parts each, nor than the longest row does, and at least n / longest: where the two bounds leave a choice, the parts
+      // are counted, two lengths at a time from the shortest on.  (Counted always, for every number of parts of the longest
+      // row, with four scans, 108 rows of two requests took 1.3 us more.)
+      const int finest = max(max((max_n + kDirectMaxParts - 1) / kDirectMaxParts, kDirectMinPart), part_of(blocks + n_wg - 1, n_wg));
+      int longest = finest;
+      if (rows * (part_of(max(max_n, 1) - 1, finest) + 1) > n_wg) {
+        const int spare = n_wg - rows, per_row = max(part_of(n_wg, max(rows, 1)), 1);
+        longest = max(finest, min(spare > 0 ? part_of(blocks + spare - 1, spare) : max_n, part_of(max_n + per_row - 1, per_row)));
+      }
+      for (int k = min(kDirectMaxParts, part_of(max_n + finest - 1, finest)), turn = 0; k > 0; k -= 2, turn ^= 1) {
+        const int w0 = max(part_of(max_n + k - 1, k), finest), w1 = k > 1 ? max(part_of(max_n + k - 2, k - 1), finest) : w0;
+        if (w0 >= longest) break;
+        uint32_t parts_mine = 0;
 #pragma unroll
-        for (int k = 1; k <= kDirectMaxParts; ++k) {
-          const int w = max((max_n + k - 1) / k, kDirectMinPart);
-          int parts_mine = 0;
-#pragma unroll
-          for (int u = 0; u < kCands; ++u) parts_mine += act[u] ? part_of(max(n[u], 1) - 1, w) + 1 : 0;
-          if (k & 1) counts[k >> 1] = parts_mine; else counts[(k >> 1) - 1] |= static_cast<uint32_t>(parts_mine) << 16;
+        for (int u = 0; u < kCands; ++u) {
+          const int last_block = max(n[u], 1) - 1;
+          if (act[u]) parts_mine += static_cast<uint32_t>((part_of(last_block, w0) + 1) | (part_of(last_block, w1) + 1) << 16);
         }
-#pragma unroll
-        for (int k = 0; k < kDirectMaxParts / 2; ++k) {
-          const int sum = wave_scan(static_cast<int>(counts[k]));
-          if (lane == 63) s_wave[4 + k][wv] = sum;
-        }
+        const int sum = wave_scan(static_cast<int>(parts_mine));
+        if (lane == 63) s_wave[4 + turn][wv] = sum;
         __syncthreads();
+        uint32_t parts_all = 0;
 #pragma unroll
-        for (int k = 0; k < kDirectMaxParts / 2; ++k) {
-          uint32_t all = 0;
-#pragma unroll
-          for (int w = 0; w < kWaves; ++w) all += static_cast<uint32_t>(s_wave[4 + k][w]);
-          if (static_cast<int>(all & 0xffff) <= n_wg) longest = max((max_n + 2 * k) / (2 * k + 1), kDirectMinPart);
-          if (static_cast<int>(all >> 16) <= n_wg) longest = max((max_n + 2 * k + 1) / (2 * k + 2), kDirectMinPart);
+        for (int w = 0; w < kWaves; ++w) parts_all += static_cast<uint32_t>(s_wave[4 + turn][w]);
+        parts_all = __builtin_amdgcn_readfirstlane(parts_all);
+        if (static_cast<int>(parts_all & 0xffff) <= n_wg) {
+          longest = w0;
+          break;
+        }
+        if (static_cast<int>(parts_all >> 16) <= n_wg) {
+          longest = min(longest, w1);
+          break;
         }
       }
       // Whole parts or even shares: whichever has the least on its slowest workgroup.  A share is as good as never
@@ -1061,11 +1091,7 @@ sparse_fa_kernel(const FaParams p) {
             it.nb = min(max(min(n[u] - it.ptr0, per), 0), kRowBlocks);
             s_next_row[0] = it;
             // its keep bits: in LDS already, or this thread's own
-            s_list_at = p.is_full || list_at[u] == kOwnWords ? 0 : list_at[u];
-            if (!p.is_full && list_at[u] == kOwnWords) {
-#pragma unroll
-              for (int i = 0; i < kAhead; ++i) reinterpret_cast<uint32_t*>(smem)[i] = own[u][i];
-            }
+            s_list_at = p.is_full ? 0 : list_at[u];
           }
           first += parts[u];
         }
@@ -1094,20 +1120,24 @@ sparse_fa_kernel(const FaParams p) {
         ++row;
       }
     if (tid == 0) {
+      s_map[0] = map_word;
+      s_map[1] = map_words;
       if (dir_g >= shares) s_dir[2] = 1;  // (no row: see direct_items)
       s_dir[3] = shares;
       s_dir[4] = total;
+      s_dir[5] = a;
+      s_dir[6] = b;
     }
     __syncthreads();
   };
   // sixteen items of the share from `batch_base` on
-  auto direct_items = [&](int batch_base) {
+  auto direct_items = [&](int batch_base) __attribute__((always_inline)) {
     const int lane = fresh_lane();
     if (lane < kItemBatch) {
       RowInfo it;
       it.row = -1;
       const int dir_g = dir_index(), rows = s_dir[2], shares = s_dir[3], total = s_dir[4];
-      const int a = cut_at(dir_g, total, shares), b = cut_at(dir_g + 1, total, shares), i = s_dir[0] + batch_base + lane;
+      const int a = s_dir[5], b = s_dir[6], i = s_dir[0] + batch_base + lane;
       if (dir_g < shares && i >= 0 && i < rows) {
         // kv blocks cost [u, e)
         const int u = s_row_u[row_at(i)], e = s_row_u[row_at(i + 1)] - kShareRowCost;
@@ -1118,7 +1148,12 @@ sparse_fa_kernel(const FaParams p) {
           it.parts = 1;
           it.slot = 0;
           if (e > u) {
-            const int j_lo = share_of(u, total, shares), j_hi = share_of(e - 1, total, shares);
+            // (the shares that hold its first and its last kv block: this one, or some next to it)
+            int j_lo = dir_g, j_hi = dir_g;
+            if (u < a)
+              do --j_lo; while (cut_at(j_lo, total, shares) > u);
+            if (e > b)
+              do ++j_hi; while (cut_at(j_hi + 1, total, shares) < e);
             it.part = dir_g - j_lo;
             it.parts = j_hi - j_lo + 1;
             it.slot = j_lo;
@@ -1129,10 +1164,27 @@ sparse_fa_kernel(const FaParams p) {
       }
       s_items[lane] = it;
     }
+    if constexpr (kDirect && kPipe) {
+      if (p.is_full) return;
+      // (four lanes to an item)
+      const int k = lane & (kItemBatch - 1);
+      const RowInfo& it = s_items[k];
+      const int words = (it.mask_first + it.nkv + 31) >> 5;
+      if (it.row >= 0 && words <= kBitWords) {
+        const int in_map = it.mask - s_map[0];
+        // (behind the first sixteen items the tile buffers are in use)
+        if (batch_base == 0 && in_map >= 0 && in_map + words <= s_map[1]) {
+          for (int i = lane >> 4; i < words; i += 4) s_bits[k][i] = reinterpret_cast<const uint32_t*>(smem)[in_map + i];
+        } else {
+          for (int i = lane >> 4; i < words; i += 4) s_bits[k][i] = reinterpret_cast<const uint32_t*>(kv_info_words)[it.mask + i];
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // (see fetch_next)
+    }
   };
   // One wavefront: the kv block list of the item in s_next_row[slot_idx], from the row's keep bits (words_at: in LDS from
-  // there on, -1: in memory)
-  auto direct_list = [&](int slot_idx, const RowInfo& it, int words_at) __attribute__((always_inline)) {
+  // there on, -1: in s_bits, row `bits_row`, or in memory)
+  auto direct_list = [&](int slot_idx, const RowInfo& it, int words_at, int bits_row) __attribute__((always_inline)) {
     const int lane = fresh_lane();
     const int lo = __builtin_amdgcn_readfirstlane(it.ptr0), n = __builtin_amdgcn_readfirstlane(it.nb);
     if (p.is_full) {
@@ -1153,11 +1205,11 @@ sparse_fa_kernel(const FaParams p) {
       if (words_at >= 0) {
         const uint32_t* const words = reinterpret_cast<const uint32_t*>(smem) + words_at;
         for (int b0 = 0; b0 < r.n && seen < n; b0 += 64) keep_bits(b0 + lane, words[(r.first + min(b0 + lane, r.n - 1)) >> 5]);
+      } else if (kPipe && bits_row >= 0 && r.count() <= kBitWords) {
+        const uint32_t* const words = s_bits[bits_row];
+        for (int b0 = 0; b0 < r.n && seen < n; b0 += 64) keep_bits(b0 + lane, words[(r.first + min(b0 + lane, r.n - 1)) >> 5]);
       } else {
-        const uint64_t m = reinterpret_cast<uint64_t>(it.mask);
-        r.words = reinterpret_cast<const uint32_t*>(
-            static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m >> 32)))) << 32 |
-            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m))));
+        r.words = reinterpret_cast<const uint32_t*>(kv_info_words) + __builtin_amdgcn_readfirstlane(it.mask);
         // four rounds' words requested together
         for (int b0 = 0; b0 < r.n && seen < n; b0 += 4 * 64) {
           uint32_t v[4];
@@ -1166,12 +1218,12 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) keep_bits(b0 + 64 * j + lane, v[j]);
         }
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // (see fetch_next)
       }
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // (see fetch_next)
   };
   // One wavefront: the next item and its list
-  auto direct_next = [&](int slot_idx) {
+  auto direct_next = [&](int slot_idx) __attribute__((always_inline)) {
     slot_idx = __builtin_amdgcn_readfirstlane(slot_idx);
     const int lane = fresh_lane();
     const int at = __builtin_amdgcn_readfirstlane(s_share[0]);  // items handed out so far
@@ -1181,7 +1233,7 @@ sparse_fa_kernel(const FaParams p) {
       s_next_row[slot_idx] = it;
       s_share[0] = at + 1;
     }
-    if (__builtin_amdgcn_readfirstlane(it.row) >= 0) direct_list(slot_idx, it, -1);
+    if (__builtin_amdgcn_readfirstlane(it.row) >= 0) direct_list(slot_idx, it, -1, at & (kItemBatch - 1));
   };
   if constexpr (kDirect) {
     // The copy of the symbols for a later decode: 2 KB or so by each of the last workgroups, asked for in front of the
@@ -1239,7 +1291,7 @@ sparse_fa_kernel(const FaParams p) {
         // whole parts: the item is there, and the only one
         if (lane == 0) s_share[0] = 1;
         if (__builtin_amdgcn_readfirstlane(s_next_row[0].row) >= 0)
-          direct_list(0, s_next_row[0], __builtin_amdgcn_readfirstlane(s_list_at));
+          direct_list(0, s_next_row[0], __builtin_amdgcn_readfirstlane(s_list_at), -1);
       }
     }
   }
@@ -2339,11 +2391,16 @@ sparse_fa_kernel(const FaParams p) {
       // Whoever comes last combines the parts and writes the row.  A workgroup that finds every
       // other part arrived already need not publish its own; otherwise it publishes, then counts
       // itself in, and may still turn out to be the last.
-      if (tid == 0)
-        s_arrived = __hip_atomic_load(&p.sched[kSchedArrived + split_slot], __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      bool last = s_arrived == parts - 1;
+      // (Even shares: the first item of a share is the end of a row that began in another share, whose last item its beginning
+      // is.  It is early, and does not ask.)
+      bool last = false;
+      if (!kDirect || row_it > 0 || part == 0) {
+        if (tid == 0)
+          s_arrived = __hip_atomic_load(&p.sched[kSchedArrived + split_slot], __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        last = s_arrived == parts - 1;
+      }
       if (!last) {
         if (kg == 0) {
           // same lane layout as the LDS merge area; two planes of 8-byte pairs, so that each store

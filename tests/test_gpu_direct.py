@@ -272,3 +272,37 @@ def test_routes_of_a_short_list_agree(dev, layout, group, ws_mib):
     assert torch.equal(got == 7.0, exp == 7.0)
     assert max_abs(got, exp) <= 2e-2 and rel_l2(got, exp) <= 6e-3
     assert torch.allclose(got_lse, exp_lse, atol=2e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("ql, kl, heads", [
+    ([300, 1, 700], [1100, 77, 513], 3),            # whole parts
+    ([3000, 1, 700], [1100, 77, 513], 24),          # 720 candidates, shares in the pipelined form
+    ([2600, 700, 500], [9000, 300, 4000], 24),      # keep bits of 70 and 31 blocks, read where they are or from LDS
+    ([1500, 128, 300], [40000, 40000, 700], 16),    # 313 blocks to a row
+])
+def test_symbols_in_any_order(dev, ql, kl, heads):
+    """Segments that lie in the buffer in another order than their requests, at odd bytes: what is outside of the piece from
+    the first segment to the end is read where it is, the rest from LDS.  The same bits as in order."""
+    import flashomni_amd as fo
+    m = make_ragged_masks(ql, kl, heads, 0.8, 0.4, seed=9)
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(n, heads, 128, generator=g).to(torch.bfloat16).to(dev) for n in (sum(ql), sum(kl), sum(kl)))
+    t = lambda a: torch.from_numpy(a).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t(m["qo_indptr"]), t(m["kv_indptr"]), heads, heads, 128, q_data_type=torch.bfloat16)
+
+    def moved(packed, indptr):
+        """The second request's segment in front, three bytes of ones before every segment."""
+        parts, at, starts = [], 0, {}
+        for r in (1, 0, 2):
+            seg = packed[indptr[r]:indptr[r + 1]]
+            parts += [np.full(3, 0xff, np.uint8), seg]
+            starts[r] = at + 3
+            at += 3 + len(seg)
+        return np.concatenate(parts), np.array([starts[0], starts[1], starts[2], at], np.int32)
+
+    want = w.run(q, k, v, t(m["packed_info"]), t(m["packed_keep"]), t(m["info_indptr"]), t(m["keep_indptr"]))
+    info, info_ip = moved(m["packed_info"], m["info_indptr"])
+    keep, keep_ip = moved(m["packed_keep"], m["keep_indptr"])
+    got = w.run(q, k, v, t(info), t(keep), t(info_ip), t(keep_ip))
+    assert torch.equal(got, want)
