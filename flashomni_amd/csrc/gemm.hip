@@ -140,6 +140,7 @@ struct GemmParams {
   int32_t n_row_tiles, n_col_tiles, n_cp;  // geometry for the arithmetic enumeration
   int32_t strip_cols;    // strips: column groups of XCDs
   int32_t strip_sorted;  // strips: token blocks with the most selected heads first
+  int32_t num_cu;        // strips of flagged units: up to as many have a CU each
   int32_t* judgement;    // GEMM-Q: the word in which quads leave to the strips behind them whether they ran, or null
   int32_t n_win;         // windows of 16 token blocks per batch
   int32_t inline_cells;  // > 0: GEMM-Q builds its quad list itself from the flags of this many cells
@@ -2097,26 +2098,313 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
 // sustains 1.98 PFLOP/s of them on random operands against 1.76 of 32 x 32 x 16 (registers only, all CUs, both at the power limit;
 // with zeros both reach 2.42).  GEMM-O of 76 112 x 5120 with 80 % 2835 -> 2640 us, of 4608 x 3072, both passes, 97.5 -> 94.
 // They are worth it where two wavefronts share a SIMD and the vector ALU has nothing else to issue: quads, one wavefront to a
-// SIMD, wait for their own loads with 16 cycles of MFMA in flight instead of 32 (GEMM-Q of 76 112 x 5120 2940 -> 3230), and the
-// attention loop's exponentials want the issue slots that twice as many MFMAs take (33 k tokens x 24 heads 1709 -> 1785).
+// SIMD, wait for their own loads with 16 cycles of MFMA in flight instead of 32 (GEMM-Q of 76 112 x 5120 2940 -> 3230), as do
+// strips of flagged units that have a CU each, which keep 32 x 32 (16 384 x 3072 with a tenth flagged, new inputs, 49.2 us, in 16 x 16
+// 50.3), and the attention loop's exponentials want the issue slots that twice as many MFMAs take (33 k tokens x 24 heads 1709 -> 1785).
 // ---------------------------------------------------------------------------------------------
 constexpr int kStripPiece = 2 * 32 * kRowBytes;  // 32 rows of W of both column blocks
 constexpr int kStripRing = 6;
 constexpr int kStripSorted = 4096;  // token blocks that are put in order
 constexpr int kStripSmemBytes = 2 * kUnitBytes + kStripRing * kStripPiece;  // 80 KB: two X tiles, the ring of W
 
-template <typename T, bool kReduce, bool kHalf, bool kPartial>
-__global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParams p) {
+// One strip: token block `block`, column blocks c0 and c1 (negative: none), MFMA tiles of kT x kT.
+template <typename T, bool kReduce, bool kHalf, bool kPartial, int kT>
+__device__ __forceinline__ void strip(const GemmParams& p, uint8_t* smem, int tid, int block, int c0, int c1) {
   using TT = Types<T>;
   using x8 = typename TT::x8;
   using x4 = typename TT::x4;
-  constexpr int NT = 8, MT = 4;  // wavefront tile: 128 columns (W rows) x 64 token rows (X rows), 16 x 16 each
+  // wavefront tile: 128 columns (W rows) x 64 token rows (X rows); a piece of W holds CT tiles of columns, a slab KS of k
+  constexpr int NT = 128 / kT, MT = 64 / kT, CT = 32 / kT, KS = kT / 8, kPieces = kT * kT / 256;
+  // (a descriptor has to be in scalar registers, and divisions are not)
+  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & (kT - 1), g = lane / kT;
+  const int wr = wv >> 1, wc = wv & 1;  // half of the rows; column block
+  block = __builtin_amdgcn_readfirstlane(block);
+  c0 = __builtin_amdgcn_readfirstlane(c0);
+  c1 = __builtin_amdgcn_readfirstlane(c1);
+  const int bz = __builtin_amdgcn_readfirstlane(block / p.n_row_tiles), row = block - bz * p.n_row_tiles;
+  const int m0 = row * kTile;
+  const uint32_t flag_row = static_cast<uint32_t>(p.num_text_tokens + row * kTile) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
+
+  // ---- the slabs: heads of this token block (GEMM-O), or all of k ----
+  SlabWalk<kReduce, kHalf> walk;
+  walk.begin(p, bz, flag_row, lane);
+  const int n_iter = walk.n_iter;
+  auto next_slab = [&]() __attribute__((always_inline)) -> Slab { return walk.next(p); };
+
+  const T* __restrict__ xg = static_cast<const T*>(p.x);
+  const T* __restrict__ wg = static_cast<const T*>(p.w);
+  const int rows_here = min(p.m - m0, kTile);
+  const uint32_t k2 = static_cast<uint32_t>(p.k) * 2u;
+  const T* const x_base = xg + (static_cast<int64_t>(bz) * p.m + m0) * p.k;
+  const uint32_t x_bytes = static_cast<uint32_t>(rows_here) * k2;
+  // (a wavefront copies for column block wv / 2 and computes column block wv % 2)
+  const int c_copy = wv >> 1 ? c1 : c0, c_mine = wc ? c1 : c0;
+  const T* const w_base = wg + static_cast<int64_t>(max(c_copy, 0)) * kTile * p.k;
+  const uint32_t w_bytes = c_copy < 0 ? 0u : kTile * k2;
+  auto rsrc = [&](const T* base, uint32_t bytes) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, bytes, 0x00020000);
+  };
+  uint32_t voff[2];
+#pragma unroll
+  for (int par = 0; par < 2; ++par)
+    voff[par] = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4);
+  typedef __attribute__((address_space(3))) void lds_void;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
+  const uint32_t ldsw = lds0 + 2 * kUnitBytes;  // the ring
+  const uint32_t row8 = 8u * k2;
+  auto copy = [&](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(vo), "s"(r), "s"(soff)
+                 : "memory", "m0");
+  };
+  const uint32_t x_soff = 4u * wv * row8, w_soff = 2u * (wv & 1) * row8;
+  const uint32_t x_dst = lds0 + wv * 32 * kRowBytes, w_dst = ldsw + (wv >> 1) * 32 * kRowBytes + (wv & 1) * 16 * kRowBytes;
+  auto copy_x = [&](__amdgpu_buffer_rsrc_t r, int i, uint32_t koff, uint32_t buf) __attribute__((always_inline)) {
+    copy(r, voff[i & 1], koff + x_soff + i * row8, x_dst + buf + i * 8 * kRowBytes);
+  };
+  auto copy_w = [&](__amdgpu_buffer_rsrc_t r, int nt, int i, uint32_t koff, uint32_t at) __attribute__((always_inline)) {
+    copy(r, voff[i & 1], koff + w_soff + (4 * nt + i) * row8, w_dst + at + i * 8 * kRowBytes);
+  };
+
+  // acc[ct][mt][i]: column ct*kT + (i/4)*8 + g*4 + i%4 of the block, row wr*64 + mt*kT + lr
+  typename std::conditional<kT == 16, f32x4, f32x16>::type acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4 * kPieces; ++i) acc[nt][mt][i] = 0.f;
+
+  if (n_iter > 0) {
+    typedef __attribute__((address_space(3))) const x8 lds_x8;
+    // an operand: kT rows, 512 / kT of k (ks); lane: row lr, 16-byte chunk ks*64/kT + g
+    uint32_t lane_off[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      lane_off[ks] = static_cast<uint32_t>(lr * kRowBytes + (((ks * (64 / kT) + g) ^ ((lr >> 1) & 7)) << 4));
+    const uint32_t x_src = lds0 + wr * 64 * kRowBytes, w_src = ldsw + wc * 32 * kRowBytes;
+    x8 xr_[MT][KS], wreg[2][CT][KS];
+    auto read_x = [&](int mt, int ks, uint32_t buf) __attribute__((always_inline)) {
+      xr_[mt][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (x_src + buf) + mt * kT * kRowBytes));
+    };
+    auto read_w = [&](int set, int ct, int ks, uint32_t at) __attribute__((always_inline)) {
+      wreg[set][ct][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (w_src + at) + ct * kT * kRowBytes));
+    };
+    // prologue: X of slab 0, pieces 0 to 2 | pieces 3 and 4, X of slab 1
+    Slab sa = next_slab(), sb = sa;  // slabs it, it + 1
+    if (n_iter > 1) sb = next_slab();
+    {
+      const __amdgpu_buffer_rsrc_t rx = rsrc(x_base, x_bytes), rw = rsrc(w_base, w_bytes);
+      const __amdgpu_buffer_rsrc_t rx1 = rsrc(x_base, n_iter > 1 ? x_bytes : 0u), rw1 = rsrc(w_base, n_iter > 1 ? w_bytes : 0u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) copy_x(rx, i, sa.k, 0);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) copy_w(rw, q, i, sa.k, q * kStripPiece);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) copy_x(rx1, i, sb.k, kUnitBytes);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) copy_w(rw, 3, i, sa.k, 3 * kStripPiece);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) copy_w(rw1, 0, i, sb.k, 4 * kStripPiece);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) read_w(0, j % CT, j / CT, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) read_x(j % MT, j / MT, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t ring = 0;  // place of the slab's first piece
+    uint32_t xbuf = 0;
+    auto place = [&](int j) __attribute__((always_inline)) -> uint32_t {  // of the j-th piece from the slab's first on
+      uint32_t at = ring + j * kStripPiece;
+      at = at >= 2 * kStripRing * kStripPiece ? at - 2 * kStripRing * kStripPiece : at;
+      return at >= kStripRing * kStripPiece ? at - kStripRing * kStripPiece : at;
+    };
+    for (int it = 0; it < n_iter; ++it) {
+      const bool live1 = it + 1 < n_iter, live2 = it + 2 < n_iter;
+      Slab sc = sb;
+      if (live2) sc = next_slab();
+      const __amdgpu_buffer_rsrc_t rw1 = rsrc(w_base, live1 ? w_bytes : 0u);
+      const __amdgpu_buffer_rsrc_t rw2 = rsrc(w_base, live2 ? w_bytes : 0u), rx2 = rsrc(x_base, live2 ? x_bytes : 0u);
+      auto step = [&](auto nt_tag) __attribute__((always_inline)) {
+        constexpr int nt = decltype(nt_tag)::value, set = nt & 1;
+        const uint32_t rd = place(nt + 1);
+        // (eighths of a step: the slots that reads and copies are dealt to)
+        constexpr int kPer = CT * MT * KS / 8;
+#pragma unroll
+        for (int j = 0; j < 8 * kPer; ++j) {
+          const int ks = j / (CT * MT), ct = j / MT % CT, mt = j % MT, slot = j / kPer;
+          const bool ends = j % kPer == kPer - 1;
+          if constexpr (kHalf && nt == 0) {
+            if (ct == 0) {
+              u32x4 v = __builtin_bit_cast(u32x4, xr_[mt][ks]);
+              v &= 2 * ks < KS ? sa.first : sa.second;
+              xr_[mt][ks] = __builtin_bit_cast(x8, v);
+            }
+          }
+          if constexpr (kT == 16) {
+            acc[CT * nt + ct][mt] = TT::mfma16(wreg[set][ct][ks], xr_[mt][ks], acc[CT * nt + ct][mt]);
+          } else {
+            acc[CT * nt + ct][mt] = TT::mfma(wreg[set][ct][ks], xr_[mt][ks], acc[CT * nt + ct][mt]);
+          }
+          if (slot < 4 && j % kPer == 0) read_w(set ^ 1, slot % CT, slot / CT, rd);
+          if constexpr (nt == 3) {
+            if constexpr (kT == 16) {
+              if (ct == CT - 1) read_x(mt, ks, xbuf ^ kUnitBytes);
+            } else if (mt == MT - 1) {
+              read_x(0, ks, xbuf ^ kUnitBytes);
+              read_x(1, ks, xbuf ^ kUnitBytes);
+            }
+          }
+          if constexpr (nt == 0) {
+            if ((slot & 1) && ends) copy_w(rw1, 1 + (slot >> 2), (slot >> 1) & 1, sb.k, place(5 + (slot >> 2)));
+          } else if constexpr (nt == 1) {
+            if ((slot & 1) && ends) copy_x(rx2, slot >> 1, sc.k, xbuf);
+          } else {
+            if ((slot == 2 || slot == 5) && ends) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, slot == 5, nt == 2 ? sb.k : sc.k, place(5 + nt));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
+      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      step(std::integral_constant<int, 0>{});
+      step(std::integral_constant<int, 1>{});
+      __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
+      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      step(std::integral_constant<int, 2>{});
+      step(std::integral_constant<int, 3>{});
+      ring = place(4);
+      xbuf ^= kUnitBytes;
+      sa = sb;
+      sb = sc;
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): copies past the end and operand reads
+  __builtin_amdgcn_s_barrier();
+  if (c_mine < 0) return;
+
+  // ---- epilogue: 32 rows at a time through a wavefront's quarter of the memory ----
+  uint8_t* const region = smem + wv * (kStripSmemBytes / 4);
+  const int col4 = lane & 31, rsub = lane >> 5;
+  const int n0 = c_mine * kTile;
+  const int el_off = n0 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 2*i
+  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
+  auto out_rsrc = [&](const void* base, int elem_bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
+        rows_here * p.n * elem_bytes, 0x00020000);
+  };
+  auto turn = [&](auto bias_tag, auto f32_tag) {
+    using BiasT = decltype(bias_tag);
+    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
+    constexpr bool kOutF32 = decltype(f32_tag)::value;
+    constexpr int kBytes = sizeof(BiasT);
+    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!kPartial) {
+      if (p.bias_kind == FO_BIAS_VECTOR) {
+        const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + col4 * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
+      }
+    }
+    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {  // (32 rows)
+      // (rows whose partial is in flight together: sixteen of fp32 do not fit beside the accumulators)
+      constexpr int kAhead = kBytes == 4 ? 8 : 16;
+      BiasVec bm[kAhead];
+      auto load_partial = [&](int i0) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const int r = (32 * mt + 2 * (i0 + i)) * p.n;
+          if constexpr (kBytes == 4) {
+            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, r * 4, 0));
+          } else {
+            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, r * 2, 0));
+          }
+        }
+      };
+      if constexpr (kPartial) load_partial(0);
+      // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 512 bytes = 32 chunks)
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+        for (int half = 0; half < 32 / kT; ++half)
+#pragma unroll
+          for (int i4 = 0; i4 < kPieces; ++i4) {
+            f32x4 v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = acc[ct][mt * (32 / kT) + half][i4 * 4 + j];
+            const int r = half * kT + lr, chunk = ct * (kT / 4) + i4 * 2 + g;
+            *reinterpret_cast<f32x4*>(region + r * 512 + ((chunk ^ (r & 15)) << 4)) = v;
+          }
+      f32x4 vals[8];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if ((i & 7) == 0) {
+          if constexpr (kPartial)
+            if (i > 0 && i % kAhead == 0) load_partial(i);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const int rk = (i + k) * 2 + rsub;
+            vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 512 + ((col4 ^ (rk & 15)) << 4));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x4 v = vals[i & 7];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (kPartial) {
+            v[j] += static_cast<float>(bm[i % kAhead][j]);
+          } else {
+            v[j] += bvec[j];
+          }
+        }
+        const int r = (32 * mt + 2 * i) * p.n;
+        if constexpr (kOutF32) {
+          // (no scalar offset: see unit_epilogue)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + r) * 4, 0, 2);
+        } else {
+          x4 out;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
+          typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, r * 2, 2);
+        }
+      }
+    }
+  };
+  using std::false_type;
+  using std::true_type;
+  if constexpr (!kReduce) {
+    turn(T{}, false_type{});
+  } else if constexpr (kPartial) {
+    if (p.bias_f32) {
+      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
+    } else {
+      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+    }
+  } else {
+    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+  }
+}
+
+template <typename T, bool kReduce, bool kHalf, bool kPartial>
+__global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l16 = lane & 15, g = lane >> 4;
-  const int wr = wv >> 1, wc = wv & 1;  // half of the rows; column block
 
   if (!kReduce && p.judgement != nullptr && *p.judgement != 0) return;  // (computed as quads)
   // ---- which strip ----
@@ -2127,6 +2415,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
     return static_cast<uint32_t>(p.num_text_tokens + row * kTile) / static_cast<uint32_t>(p.sparse_q_size) * p.num_heads;
   };
   int block, c0, c1;  // token block, column blocks (c1 < 0: only one)
+  bool alone = false;  // a CU each
   if (!kReduce && p.sparse_info != nullptr) {
     // ---- GEMM-Q with flags: a token block's flagged column blocks two at a time, group of columns by group ----
     auto group_begin = [&](int g) { return g * p.n_col_tiles / cols; };
@@ -2194,6 +2483,7 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       if (w < wv) upto += t;
       total += __builtin_amdgcn_readfirstlane(t);
     }
+    alone = total <= p.num_cu;
     const int s_lo = static_cast<int>(static_cast<int64_t>(total) * xcd / kXcds);
     if (s_lo + slot >= static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / kXcds)) return;
     if (const int mine = s_lo + slot - (upto - here); mine >= 0 && mine < here) {  // (one thread)
@@ -2281,266 +2571,13 @@ __global__ void __launch_bounds__(kThreads, 2) gemm_strip_kernel(const GemmParam
       __syncthreads();
     }
   }
-  // (a descriptor has to be in scalar registers, and divisions are not)
-  block = __builtin_amdgcn_readfirstlane(block);
-  c0 = __builtin_amdgcn_readfirstlane(c0);
-  c1 = __builtin_amdgcn_readfirstlane(c1);
-  const int bz = __builtin_amdgcn_readfirstlane(block / p.n_row_tiles), row = block - bz * p.n_row_tiles;
-  const int m0 = row * kTile;
-  const uint32_t flag_row = flag_row_of(row);
-
-  // ---- the slabs: heads of this token block (GEMM-O), or all of k ----
-  SlabWalk<kReduce, kHalf> walk;
-  walk.begin(p, bz, flag_row, lane);
-  const int n_iter = walk.n_iter;
-  auto next_slab = [&]() __attribute__((always_inline)) -> Slab { return walk.next(p); };
-
-  const T* __restrict__ xg = static_cast<const T*>(p.x);
-  const T* __restrict__ wg = static_cast<const T*>(p.w);
-  const int rows_here = min(p.m - m0, kTile);
-  const uint32_t k2 = static_cast<uint32_t>(p.k) * 2u;
-  const T* const x_base = xg + (static_cast<int64_t>(bz) * p.m + m0) * p.k;
-  const uint32_t x_bytes = static_cast<uint32_t>(rows_here) * k2;
-  // (a wavefront copies for column block wv / 2 and computes column block wv % 2)
-  const int c_copy = wv >> 1 ? c1 : c0, c_mine = wc ? c1 : c0;
-  const T* const w_base = wg + static_cast<int64_t>(max(c_copy, 0)) * kTile * p.k;
-  const uint32_t w_bytes = c_copy < 0 ? 0u : kTile * k2;
-  auto rsrc = [&](const T* base, uint32_t bytes) __attribute__((always_inline)) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, bytes, 0x00020000);
-  };
-  uint32_t voff[2];
-#pragma unroll
-  for (int par = 0; par < 2; ++par)
-    voff[par] = static_cast<uint32_t>(lane >> 3) * k2 + (((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4);
-  typedef __attribute__((address_space(3))) void lds_void;
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem));
-  const uint32_t ldsw = lds0 + 2 * kUnitBytes;  // the ring
-  const uint32_t row8 = 8u * k2;
-  auto copy = [&](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(lds_addr), "v"(vo), "s"(r), "s"(soff)
-                 : "memory", "m0");
-  };
-  const uint32_t x_soff = 4u * wv * row8, w_soff = 2u * (wv & 1) * row8;
-  const uint32_t x_dst = lds0 + wv * 32 * kRowBytes, w_dst = ldsw + (wv >> 1) * 32 * kRowBytes + (wv & 1) * 16 * kRowBytes;
-  auto copy_x = [&](__amdgpu_buffer_rsrc_t r, int i, uint32_t koff, uint32_t buf) __attribute__((always_inline)) {
-    copy(r, voff[i & 1], koff + x_soff + i * row8, x_dst + buf + i * 8 * kRowBytes);
-  };
-  auto copy_w = [&](__amdgpu_buffer_rsrc_t r, int nt, int i, uint32_t koff, uint32_t at) __attribute__((always_inline)) {
-    copy(r, voff[i & 1], koff + w_soff + (4 * nt + i) * row8, w_dst + at + i * 8 * kRowBytes);
-  };
-
-  // acc[ct][mt][i]: column ct*16 + g*4 + i of the block, row wr*64 + mt*16 + l16
-  f32x4 acc[NT][MT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[nt][mt][i] = 0.f;
-
-  if (n_iter > 0) {
-    typedef __attribute__((address_space(3))) const x8 lds_x8;
-    // an operand: 16 rows, 32 of k (ks); lane: row l16, 16-byte chunk 4*ks + g
-    uint32_t lane_off[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) lane_off[ks] = static_cast<uint32_t>(l16 * kRowBytes + (((4 * ks + g) ^ (l16 >> 1)) << 4));
-    const uint32_t x_src = lds0 + wr * 64 * kRowBytes, w_src = ldsw + wc * 32 * kRowBytes;
-    x8 xr_[MT][2], wreg[2][2][2];
-    auto read_x = [&](int mt, int ks, uint32_t buf) __attribute__((always_inline)) {
-      xr_[mt][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (x_src + buf) + mt * 16 * kRowBytes));
-    };
-    auto read_w = [&](int set, int ct, int ks, uint32_t at) __attribute__((always_inline)) {
-      wreg[set][ct][ks] = *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(lane_off[ks] + (w_src + at) + ct * 16 * kRowBytes));
-    };
-    // prologue: X of slab 0, pieces 0 to 2 | pieces 3 and 4, X of slab 1
-    Slab sa = next_slab(), sb = sa;  // slabs it, it + 1
-    if (n_iter > 1) sb = next_slab();
-    {
-      const __amdgpu_buffer_rsrc_t rx = rsrc(x_base, x_bytes), rw = rsrc(w_base, w_bytes);
-      const __amdgpu_buffer_rsrc_t rx1 = rsrc(x_base, n_iter > 1 ? x_bytes : 0u), rw1 = rsrc(w_base, n_iter > 1 ? w_bytes : 0u);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) copy_x(rx, i, sa.k, 0);
-#pragma unroll
-      for (int q = 0; q < 3; ++q)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) copy_w(rw, q, i, sa.k, q * kStripPiece);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) copy_x(rx1, i, sb.k, kUnitBytes);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) copy_w(rw, 3, i, sa.k, 3 * kStripPiece);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) copy_w(rw1, 0, i, sb.k, 4 * kStripPiece);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
-    __builtin_amdgcn_s_barrier();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) read_w(0, j & 1, j >> 1, 0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) read_x(j & 3, j >> 2, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    uint32_t ring = 0;  // place of the slab's first piece
-    uint32_t xbuf = 0;
-    auto place = [&](int j) __attribute__((always_inline)) -> uint32_t {  // of the j-th piece from the slab's first on
-      uint32_t at = ring + j * kStripPiece;
-      at = at >= 2 * kStripRing * kStripPiece ? at - 2 * kStripRing * kStripPiece : at;
-      return at >= kStripRing * kStripPiece ? at - kStripRing * kStripPiece : at;
-    };
-    for (int it = 0; it < n_iter; ++it) {
-      const bool live1 = it + 1 < n_iter, live2 = it + 2 < n_iter;
-      Slab sc = sb;
-      if (live2) sc = next_slab();
-      const __amdgpu_buffer_rsrc_t rw1 = rsrc(w_base, live1 ? w_bytes : 0u);
-      const __amdgpu_buffer_rsrc_t rw2 = rsrc(w_base, live2 ? w_bytes : 0u), rx2 = rsrc(x_base, live2 ? x_bytes : 0u);
-      auto step = [&](auto nt_tag) __attribute__((always_inline)) {
-        constexpr int nt = decltype(nt_tag)::value, set = nt & 1;
-        const uint32_t rd = place(nt + 1);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int ks = j >> 3, ct = (j >> 2) & 1, mt = j & 3;
-          if constexpr (kHalf && nt == 0) {
-            if (ct == 0) {
-              u32x4 v = __builtin_bit_cast(u32x4, xr_[mt][ks]);
-              v &= ks == 0 ? sa.first : sa.second;
-              xr_[mt][ks] = __builtin_bit_cast(x8, v);
-            }
-          }
-          acc[2 * nt + ct][mt] = TT::mfma16(wreg[set][ct][ks], xr_[mt][ks], acc[2 * nt + ct][mt]);
-          if (j < 8 && !(j & 1)) read_w(set ^ 1, (j >> 1) & 1, j >> 2, rd);
-          if constexpr (nt == 3)
-            if (ct == 1) read_x(mt, ks, xbuf ^ kUnitBytes);
-          if constexpr (nt == 0) {
-            if ((j & 3) == 3) copy_w(rw1, 1 + (j >> 3), (j >> 2) & 1, sb.k, place(5 + (j >> 3)));
-          } else if constexpr (nt == 1) {
-            if ((j & 3) == 3) copy_x(rx2, j >> 2, sc.k, xbuf);
-          } else {
-            if (j == 5 || j == 11) copy_w(nt == 2 ? rw1 : rw2, nt == 2 ? 3 : 0, j == 11, nt == 2 ? sb.k : sc.k, place(5 + nt));
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      };
-      __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
-      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
-      __builtin_amdgcn_s_barrier();
-      step(std::integral_constant<int, 0>{});
-      step(std::integral_constant<int, 1>{});
-      __builtin_amdgcn_s_waitcnt(0x0f70 | 8);  // vmcnt(8)
-      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
-      __builtin_amdgcn_s_barrier();
-      step(std::integral_constant<int, 2>{});
-      step(std::integral_constant<int, 3>{});
-      ring = place(4);
-      xbuf ^= kUnitBytes;
-      sa = sb;
-      sb = sc;
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): copies past the end and operand reads
-  __builtin_amdgcn_s_barrier();
-  if (c_mine < 0) return;
-
-  // ---- epilogue: 32 rows at a time through a wavefront's quarter of the memory ----
-  uint8_t* const region = smem + wv * (kStripSmemBytes / 4);
-  const int col4 = lane & 31, rsub = lane >> 5;
-  const int n0 = c_mine * kTile;
-  const int el_off = n0 + col4 * 4 + (wr * 64 + rsub) * p.n;  // rows wr*64 + rsub + 2*i
-  const int64_t row0 = static_cast<int64_t>(bz) * p.m + m0;
-  auto out_rsrc = [&](const void* base, int elem_bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(static_cast<const uint8_t*>(base) + row0 * p.n * elem_bytes), 0,
-        rows_here * p.n * elem_bytes, 0x00020000);
-  };
-  auto turn = [&](auto bias_tag, auto f32_tag) {
-    using BiasT = decltype(bias_tag);
-    using BiasVec = typename std::conditional<sizeof(BiasT) == 4, f32x4, x4>::type;
-    constexpr bool kOutF32 = decltype(f32_tag)::value;
-    constexpr int kBytes = sizeof(BiasT);
-    float bvec[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (!kPartial) {
-      if (p.bias_kind == FO_BIAS_VECTOR) {
-        const x4 bv = *reinterpret_cast<const x4*>(static_cast<const T*>(p.bias) + n0 + col4 * 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bvec[j] = static_cast<float>(bv[j]);
-      }
-    }
-    const __amdgpu_buffer_rsrc_t ry = out_rsrc(p.y, kOutF32 ? 4 : 2);
-#pragma unroll
-    for (int mt = 0; mt < MT / 2; ++mt) {  // (32 rows)
-      // (rows whose partial is in flight together: sixteen of fp32 do not fit beside the accumulators)
-      constexpr int kAhead = kBytes == 4 ? 8 : 16;
-      BiasVec bm[kAhead];
-      auto load_partial = [&](int i0) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t rb = out_rsrc(p.bias, kBytes);
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-          const int r = (32 * mt + 2 * (i0 + i)) * p.n;
-          if constexpr (kBytes == 4) {
-            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b128(rb, el_off * 4, r * 4, 0));
-          } else {
-            bm[i] = __builtin_bit_cast(BiasVec, __builtin_amdgcn_raw_buffer_load_b64(rb, el_off * 2, r * 2, 0));
-          }
-        }
-      };
-      if constexpr (kPartial) load_partial(0);
-      // 16-byte chunk c of row r sits at chunk position c ^ (r & 15) (rows are 512 bytes = 32 chunks)
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const int r = half * 16 + l16, chunk = ct * 4 + g;
-          *reinterpret_cast<f32x4*>(region + r * 512 + ((chunk ^ (r & 15)) << 4)) = acc[ct][2 * mt + half];
-        }
-      f32x4 vals[8];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        if ((i & 7) == 0) {
-          if constexpr (kPartial)
-            if (i > 0 && i % kAhead == 0) load_partial(i);
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const int rk = (i + k) * 2 + rsub;
-            vals[k] = *reinterpret_cast<const f32x4*>(region + rk * 512 + ((col4 ^ (rk & 15)) << 4));
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        f32x4 v = vals[i & 7];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if constexpr (kPartial) {
-            v[j] += static_cast<float>(bm[i % kAhead][j]);
-          } else {
-            v[j] += bvec[j];
-          }
-        }
-        const int r = (32 * mt + 2 * i) * p.n;
-        if constexpr (kOutF32) {
-          // (no scalar offset: see unit_epilogue)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, (el_off + r) * 4, 0, 2);
-        } else {
-          x4 out;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(v[j]);
-          typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, out), ry, el_off * 2, r * 2, 2);
-        }
-      }
-    }
-  };
-  using std::false_type;
-  using std::true_type;
   if constexpr (!kReduce) {
-    turn(T{}, false_type{});
-  } else if constexpr (kPartial) {
-    if (p.bias_f32) {
-      if (p.y_f32) turn(0.f, true_type{}); else turn(0.f, false_type{});
-    } else {
-      if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
+    if (alone) {
+      strip<T, kReduce, kHalf, kPartial, 32>(p, smem, tid, block, c0, c1);
+      return;
     }
-  } else {
-    if (p.y_f32) turn(T{}, true_type{}); else turn(T{}, false_type{});
   }
+  strip<T, kReduce, kHalf, kPartial, 16>(p, smem, tid, block, c0, c1);
 }
 
 ListGeom make_geom(int32_t batch, int32_t m, int32_t n) {
@@ -2671,6 +2708,7 @@ int launch_strips(GemmParams& p, const ListGeom& gm, hipStream_t stream) {
   }
   p.strip_cols = cols;
   p.strip_sorted = rows <= kStripSorted;
+  p.num_cu = fo_num_cu();
   gemm_strip_kernel<T, kReduce, kHalf, kAux><<<static_cast<unsigned>(grid), kThreads, kStripSmemBytes, stream>>>(p);
   FO_CHECK_LAUNCH();
   return FO_OK;
