@@ -95,9 +95,11 @@ constexpr int kMergeOBytes = 4 * 16 * 64 * 16;
 constexpr int kOutTileOff = kMergeOBytes + 4 * 64 * 8;  // behind the merge area
 constexpr int kOutRowBytes = 256 + 16;                  // one output row of 128 16-bit elements, padded
 constexpr int kOutTileBytes = 128 * kOutRowBytes;
-// The pipelined form's buffers of 32 keys.  K: every four rows (what one copy instruction fills) begin 16 bytes later
-// modulo the banks than the four before, so that rows a multiple of four apart need no swizzle against each other.
-constexpr int kPipeKRows4 = 4 * kRowBytes + 16, kPipeKBuf = 8 * kPipeKRows4, kPipeVBuf = 32 * kRowBytes;
+// The pipelined form's buffers of 32 keys.  K: row r keeps its 16-byte chunk c at c ^ (4 * (r % 4) + r / 4 % 4).
+constexpr int kPipeKBuf = 32 * kRowBytes;
+// V: every four rows (what one copy instruction fills) begin 32 bytes later modulo the banks than the four before, so that
+// two 16-lane groups of a transposed read, four rows apart, meet in no bank; chunks are swizzled by the row modulo four.
+constexpr int kPipeVRows4 = 4 * kRowBytes + 32, kPipeVBuf = 8 * kPipeVRows4;
 // LDS geometry of one kv group: two stages of (K tile, V tile); K is 16-bit or fp8
 template <bool kFp8, bool kKLo = false, int kGroups = 2>
 struct Geom {
@@ -190,6 +192,9 @@ struct Types<__bf16> {
   static __device__ __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f32x4 mfma16(x8 a, x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
   // acc + sum of the eight elements of v (v_dot2c_f32_bf16 against ones)
   static __device__ __forceinline__ float add_elems(x8 v, float acc) {
     typedef __attribute__((ext_vector_type(2))) __bf16 x2;
@@ -205,6 +210,9 @@ struct Types<_Float16> {
   using x4 = f16x4;
   static __device__ __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 mfma16(x8 a, x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ float add_elems(x8 v, float acc) {
     typedef __attribute__((ext_vector_type(2))) _Float16 x2;
@@ -272,6 +280,16 @@ __device__ __forceinline__ float max_across_halves(float x) {
   const u32x2 r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   // (Each element in a scalar first: a bit cast of a vector's element reads element 0 whichever is named, and
   // then this was the maximum of the lower half.  And the instruction itself: fmaxf quiets both operands first.)
+  const unsigned lo = r[0], hi = r[1];
+  float m;
+  asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(lo), "v"(hi));
+  return m;
+}
+
+// the same over lane and lane^16
+__device__ __forceinline__ float max_across_rows(float x) {
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const u32x2 r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
   const unsigned lo = r[0], hi = r[1];
   float m;
   asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(lo), "v"(hi));
@@ -1383,21 +1401,27 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) o_acc[dt][i] = 0.f;
     float m_run = 0.f, d_part = 0.f;
+    // kPipe: O^T as 16 x 16 tiles (16 d x 16 q rows), 2 * dt + qt: element j of a lane is d 16 * dt + 4 * (lane / 16) + j
+    // of q row 16 * qt + lane % 16; reference point and row sum per q row (the sum over the lane's own keys)
+    f32x4 o_tile[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o_tile[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_q[2] = {0.f, 0.f}, d_q[2] = {0.f, 0.f};
     if constexpr (kPipe) {
       // ---- software-pipelined row (one kv group) ----
-      // A step is 32 keys.  In step t a wavefront issues the eight MFMAs of S(t+1) = K(t+1).Q^T, then the eight of
-      // O^T += V(t-1)^T.P(t-1)^T, and between them, instruction by instruction, the softmax of S(t) (exp2, rounding, row
-      // sum -> P(t)), the largest value of S(t+1) as soon as it is complete, the operand reads and the copies of later
-      // steps: the vector ALU work of a step runs in the shadow of its own MFMAs instead of in a phase of its own.  Eight
-      // operands are in registers: each MFMA's is read eight MFMAs ahead, into the registers of the one just used, V(t-1)
-      // during the MFMAs of S and K(t+2) during those of P.V.  LDS holds four K and four V buffers of 32 keys; a copy is
-      // issued as soon as its buffer is dead: K two and a half steps, V three before its first read.  One barrier per step.
-      // What bounds it is the power limit (matrix cores 68 % busy at 1.7 GHz on long lists) and the vector ALU, 41
-      // instructions of a step beside the 16 MFMAs: 16 exp2, 8 roundings, 8 sums, 8 for the maximum and one more.  With S
-      // and P.V in turn instead of one after the other, the maximum in front of a step's first MFMA, 16 moves that set the
-      // accumulators of S to the reference point (now 16 registers that they accumulate from) and 7 address terms of K it
-      // was 73 of them besides the exp2: 33 k tokens x 24 heads with windows 1878 -> 1712 us, 16 896 x 24 with a fifth of the
-      // blocks in fp16 780 -> 714, 4608 x 24 from the symbols 126 -> 117.7.
+      // A step is 32 keys.  In step t a wavefront issues the MFMAs of S(t+1) = K(t+1).Q^T, sixteen tiles of 16 x 16 over 32 of
+      // k, then the sixteen of O^T += V(t-1)^T.P(t-1)^T, and behind either run a part of the softmax of S(t) (exp2, rounding,
+      // row sum -> P(t)); the largest value of S(t+1) is taken as soon as it is complete.  Eight operands are in registers,
+      // each of two MFMAs: read eight operands ahead, into the registers of the one just used, V(t-1) during the MFMAs of S
+      // and K(t+2) during those of P.V.  LDS holds four K and four V buffers of 32 keys; a copy is issued as soon as its
+      // buffer is dead: K two and a half steps, V three before its first read.  One barrier per step.
+      // What bounds it is the power limit and the vector ALU, which issues the MFMAs too: 32 of them, 16 exp2 and 26 other
+      // instructions a step.  MFMA tiles of 32 x 32 over 16, half as many, read and write each accumulator twice as often and
+      // held the clock at 1.55 GHz where these run at 1.8 (33 k tokens x 24 heads with windows, in 16 % fewer cycles at
+      // equal interleaving).  What then made them the faster ones: K's swizzle (see q_chunk_of), and runs of MFMAs in place of
+      // MFMAs and exponentials in turn, see the softmax's bursts.  33 k x 24 1713 -> 1664 us, 16 896 x 24 with a fifth of the
+      // blocks in fp16 712 -> 680, 4608 x 24 from the symbols 116.4 -> 113.1, the layer step of 76 112 x 5120 with two-term
+      // fp8 13 977 -> 13 678.
       constexpr int kStep = 32;
       // K buffers 0..2 | V buffer 0 | K buffer 3 | V buffers 1..3; Q is staged from K buffer 3 on, so
       // that K(0..2) and V(0) can be requested together with it
@@ -1424,16 +1448,15 @@ sparse_fa_kernel(const FaParams p) {
           const_cast<uint8_t*>(k_head), 0, static_cast<uint32_t>(kv_len - 1) * k_sn2 + kRowBytes, 0x00020000);
       const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<uint8_t*>(v_head), 0, static_cast<uint32_t>(kv_len - 1) * v_sn2 + kRowBytes, 0x00020000);
-      // A lane's part of a copy: row 4 * qs + lane / 16 of a 16-row group, 16-byte chunk swizzled by the row modulo four.
-      // (The operand reads of the loop then differ by immediate offsets but for two bits of the chunk: four addresses each
-      // for K and V.  With all four bits swizzled the reads of K took seven instructions a step.)
+      // A lane's part of a copy: row 4 * qs + lane / 16 of a 16-row group, 16-byte chunk swizzled.  (The operand reads of the
+      // loop then differ by immediate offsets but for two bits of the chunk: four addresses each for K and V.)
       const int ln_c = fresh_lane();
-      const int cp_chunk = ((ln_c & 15) ^ ((ln_c >> 4) << 2)) * 16, cp_row = 4 * qs + (ln_c >> 4);
-      uint32_t k_voff = static_cast<uint32_t>(cp_row) * k_sn2 + cp_chunk;
-      uint32_t v_voff = static_cast<uint32_t>(cp_row) * v_sn2 + cp_chunk;
+      const int cp_chunk = (ln_c & 15) ^ ((ln_c >> 4) << 2), cp_row = 4 * qs + (ln_c >> 4);
+      uint32_t k_voff = static_cast<uint32_t>(cp_row) * k_sn2 + (cp_chunk ^ qs) * 16;
+      uint32_t v_voff = static_cast<uint32_t>(cp_row) * v_sn2 + cp_chunk * 16;
       asm volatile("" : "+v"(k_voff), "+v"(v_voff));
       // LDS addresses of this wavefront's part of buffer offset 0
-      const uint32_t m0_k = lds0 + qs * kPipeKRows4, m0_v = lds0 + qs * 1024;
+      const uint32_t m0_k = lds0 + qs * 1024, m0_v = lds0 + qs * kPipeVRows4;
       // 64 lanes x 16 bytes of 4 rows, global -> LDS (see copy16_to_lds), addressed through a descriptor:
       // lane offset + scalar offset
       auto copy_desc = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) __attribute__((always_inline)) {
@@ -1447,12 +1470,12 @@ sparse_fa_kernel(const FaParams p) {
       auto copy_k = [&](int t) __attribute__((always_inline)) {
         const uint32_t soff = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(step_start(t))) * k_sn2;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) copy_desc(k_rsrc, k_voff, soff + j * 16 * k_sn2, m0_k + kbuf(t & 3) + j * (4 * kPipeKRows4));
+        for (int j = 0; j < 2; ++j) copy_desc(k_rsrc, k_voff, soff + j * 16 * k_sn2, m0_k + kbuf(t & 3) + j * 4096);
       };
       auto copy_v = [&](int t) __attribute__((always_inline)) {
         const uint32_t soff = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(step_start(t))) * v_sn2;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) copy_desc(v_rsrc, v_voff, soff + j * 16 * v_sn2, m0_v + vbuf(t & 3) + j * 4096);
+        for (int j = 0; j < 2; ++j) copy_desc(v_rsrc, v_voff, soff + j * 16 * v_sn2, m0_v + vbuf(t & 3) + j * (4 * kPipeVRows4));
       };
 
       // prologue: Q, K(0..2), V(0) requested together
@@ -1505,70 +1528,78 @@ sparse_fa_kernel(const FaParams p) {
         if (wv == 0) direct_next((row_it + 1) & 1);
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __builtin_amdgcn_s_barrier();
-      q8 qreg[8];
+      q8 qreg[8];  // 2 * ks + qt: 32 d of 16 q rows
       u32x4 op[8];  // operands of the next eight MFMAs: slices of K or of V^T
-      u32x4 pA[2], pB[2];  // P of a step: 2 x 8 rounded values, as 32-bit pairs
-      f32x16 sA, sB;
+      u32x4 pA[2], pB[2];  // P of a step, per q tile: 8 rounded values, as 32-bit pairs
+      f32x4 sA[4], sB[4];  // S of a step, 16 x 16 tiles 2 * kt + qt: keys 16 * kt + 4 * (lane / 16) + j of q row 16 * qt + lane % 16
+      // Which 8 of an operand's 32 d a group of 16 lanes holds, of Q and of K alike: 0, 3, 1, 2.  A ds_read_b128 serves lanes 0-3
+      // and 12-15 of a group together with lanes 4-11 of the next one; in this order, with K's swizzle, they meet in no bank
+      // (in ascending order, as the counters have it, every read took twice as long).
+      auto q_chunk_of = [](int ln) __attribute__((always_inline)) { return (0x9c >> (ln >> 4 << 1)) & 3; };
       if constexpr (kWide) {
         // q + q_lo in fp16 (the scales are applied to S)
         f_win *= c * ri.q_scale;
-        const int ln_r = fresh_lane(), row = qs * 32 + (ln_r & 31);
-        const uint8_t* qt = smem + kQStage + row * kRowBytes8 + (ln_r >> 5) * 8;
+        const int ln_r = fresh_lane(), gr = q_chunk_of(ln_r);
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-          const uint8_t* at = qt + ((ks ^ swz8(row)) << 4);
+        for (int i = 0; i < 8; ++i) {
+          const int row = qs * 32 + (i & 1) * 16 + (ln_r & 15);
+          const uint8_t* at = smem + kQStage + row * kRowBytes8 + (((i & ~1) + (gr >> 1)) ^ swz8(row)) * 16 + (gr & 1) * 8;
           const u32x2 hi = *reinterpret_cast<const u32x2*>(at), lo = *reinterpret_cast<const u32x2*>(at + 128 * kRowBytes8);
-          widen8(hi, lo, qreg[ks]);
+          widen8(hi, lo, qreg[i]);
         }
       } else {
         const int ln_r = fresh_lane();
-        const int q_rd_base = (ln_r & 31) * kRowBytes, q_rd_x = ((ln_r >> 5) ^ swz(ln_r & 31)) << 4;
+        const int q_rd_base = (ln_r & 15) * kRowBytes, q_rd_x = (q_chunk_of(ln_r) ^ swz(ln_r & 15)) << 4;
         const uint8_t* qt = smem + kQStage + qs * 32 * kRowBytes + q_rd_base;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) qreg[ks] = *reinterpret_cast<const q8*>(qt + (q_rd_x ^ (ks << 5)));
+        for (int i = 0; i < 8; ++i) qreg[i] = *reinterpret_cast<const q8*>(qt + (i & 1) * 16 * kRowBytes + (q_rd_x ^ ((i >> 1) << 6)));
         // the softmax scale (log2 domain) is folded into Q, so S^T needs no multiply
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
+        for (int i = 0; i < 8; ++i)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) qreg[ks][e] = static_cast<T>(static_cast<float>(qreg[ks][e]) * c);
+          for (int e = 0; e < 8; ++e) qreg[i][e] = static_cast<T>(static_cast<float>(qreg[i][e]) * c);
       }
       // LDS addresses of the operand reads, without the buffer's offset and what else is an immediate of the read
       typedef __attribute__((address_space(3))) const q8 lds_x8;
       uint32_t krd[4], vrd[4];
       {
         const int ln = fresh_lane();
-        const int r = ln & 31, j = (ln & 15) >> 2;
+        const int r = ln & 15, j = r >> 2;
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-          krd[x] = lds0 + (r >> 2) * kPipeKRows4 + (r & 3) * kRowBytes + ((x ^ (r & 3)) << 6) + (ln >> 5) * 16;
-          // (row 4 * (lane / 32) + j, columns 32 * x + 16 * (lane / 16 % 2) + 4 * (lane % 4): see lds_read_tr16)
-          vrd[x] = lds0 + ((ln >> 5) * 4 + j) * kRowBytes + ((x ^ j) << 6) + ((ln >> 4) & 1) * 32 + (ln & 3) * 8;
+          krd[x] = lds0 + r * kRowBytes + ((x ^ (r & 3)) << 6) + ((q_chunk_of(ln) ^ (r >> 2)) << 4);
+          // (row 4 * (lane / 16) + j, columns 32 * x + 4 * (lane % 4): see lds_read_tr16)
+          vrd[x] = lds0 + (ln >> 4) * kPipeVRows4 + j * kRowBytes + ((x ^ j) << 6) + (ln & 3) * 8;
           asm volatile("" : "+v"(krd[x]), "+v"(vrd[x]));
         }
       }
-      // K operand slice i (16 d) of the step whose K is in buffer `buf`
+      // K operand i = 2 * ks + kt (32 d of 16 keys) of the step whose K is in buffer `buf`
       auto read_k = [&](int buf, int i) __attribute__((always_inline)) {
-        return *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(krd[i >> 1] + kbuf(buf) + (i & 1) * 32));
+        return *reinterpret_cast<lds_x8*>(static_cast<uintptr_t>(krd[i >> 1] + kbuf(buf) + (i & 1) * 4096));
       };
-      // V^T operand (kk, dt) of the step whose V is in buffer `buf`: 16 keys x 32 d, transposed
-      auto read_v = [&](int buf, int kk, int dt) __attribute__((always_inline)) {
+      // V^T operand dt of the step whose V is in buffer `buf`: 16 d x 32 keys, transposed; a lane's keys are those that it
+      // has of S: 4 * (lane / 16) + 0..3, and 16 on
+      auto read_v = [&](int buf, int dt) __attribute__((always_inline)) {
         union {
           s16x4 h[2];
           x8 v;
         } a;
-        const uint32_t off = vbuf(buf) + kk * 16 * kRowBytes;
-        a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(vrd[dt] + off)));
-        a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(vrd[dt] + off + 8 * kRowBytes)));
+        const uint32_t at = vrd[dt >> 1] + vbuf(buf) + (dt & 1) * 32;
+        a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(at)));
+        a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(static_cast<uintptr_t>(at + 4 * kPipeVRows4)));
         return a.v;
       };
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sA[i] = 0.f;
+      for (int e = 0; e < 4; ++e) sA[e] = f32x4{0.f, 0.f, 0.f, 0.f};
       {
         q8 k0[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) k0[i] = read_k(0, i);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sA = TS::mfma(k0[i], qreg[i], sA);
+        for (int i = 0; i < 16; ++i) {
+          const int kt = (i >> 1) & 1, qt = i & 1, ks = i >> 2;
+          sA[2 * kt + qt] = TS::mfma16(k0[2 * ks + kt], qreg[2 * ks + qt], sA[2 * kt + qt]);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
       // (a row of one step reads a buffer nobody filled: the result is never used)
@@ -1585,9 +1616,9 @@ sparse_fa_kernel(const FaParams p) {
         // every V buffer it does not fill (read by its padded steps), must not hold Q any more
         const u32x4 z = {0u, 0u, 0u, 0u};
         for (int b = min(n_steps, 3); b < 4; ++b) {
-          u32x4* vb = reinterpret_cast<u32x4*>(smem + vbuf(b));
-          vb[tid] = z;
-          vb[tid + kGroupThreads] = z;
+          uint8_t* vb = smem + vbuf(b) + wv * kPipeVRows4 + lane * 16;
+          *reinterpret_cast<u32x4*>(vb) = z;
+          *reinterpret_cast<u32x4*>(vb + 4 * kPipeVRows4) = z;
         }
       }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the zeros are there, before the barrier of the first step
@@ -1599,42 +1630,49 @@ sparse_fa_kernel(const FaParams p) {
       typedef __attribute__((ext_vector_type(2))) T x2;
       const x2 ones2 = {static_cast<T>(1.0f), static_cast<T>(1.0f)};
       // keys of a step that a lane's half row does not have: p = 0
-      auto mask_tail = [&](f32x16& s, int valid) __attribute__((always_inline)) {
-        const int g4 = (fresh_lane() >> 5) * 4;
+      auto mask_tail = [&](f32x4 (&s)[4], int valid) __attribute__((always_inline)) {
+        const int g4 = (fresh_lane() >> 4) * 4;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = (i >> 2) * 8 + (i & 3) + g4 < valid ? s[i] : -INFINITY;
+        for (int i = 0; i < 16; ++i) s[i >> 2][i & 3] = (i >> 3) * 16 + (i & 3) + g4 < valid ? s[i >> 2][i & 3] : -INFINITY;
       };
-      auto row_max = [&](const f32x16& s) __attribute__((always_inline)) {
-        float mx = s[0];
+      auto row_max = [&](const f32x4 (&s)[4], int qt) __attribute__((always_inline)) {
+        float mx = s[qt][0];
 #pragma unroll
-        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        return max_across_halves(mx);
+        for (int i = 1; i < 8; ++i) mx = fmaxf(mx, s[qt + (i >> 2) * 2][i & 3]);
+        return max_across_rows(max_across_halves(mx));
       };
-      // What S accumulates from: the reference point, taken off (kWide: nothing, it comes off with the factor).
-      f32x16 s_init;
+      // What S accumulates from, per q tile: the reference point, taken off (kWide: nothing, it comes off with the factor).
+      f32x4 s_init[2];
       const int valid0 = kv_len - static_cast<int>(s_blk[0]) * kBlockKV;
       if (valid0 < kStep) mask_tail(sA, valid0);
-      const float s_max0 = row_max(sA);
-      m_run = s_max0;
-      if constexpr (kWide) {
-        m_run *= __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f_win)));
+      const float s_max0[2] = {row_max(sA, 0), row_max(sA, 1)};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s_init[i] = 0.f;
-        asm volatile("" : "+v"(s_init));  // (held: as a constant it would be sixteen moves in every step)
-      } else {
+      for (int qt = 0; qt < 2; ++qt) {
+        m_q[qt] = s_max0[qt];
+        if constexpr (kWide) {
+          m_q[qt] *= __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f_win)));
+          s_init[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+          asm volatile("" : "+v"(s_init[qt]));  // (held: as a constant it would be moves in every step)
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sA[i] -= m_run;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s_init[i] = -m_run;
+          for (int j = 0; j < 4; ++j) {
+            sA[qt][j] -= m_q[qt];
+            sA[2 + qt][j] -= m_q[qt];
+            s_init[qt][j] = -m_q[qt];
+          }
+        }
       }
-      // The largest S of the lane's half row in the step at hand.  As an integer (kWide: not), which is right where any is
-      // positive, and the instruction does not quiet its operands first.
+      // The largest S of the lane in the step at hand, of both its q rows.  As an integer (kWide: not, and per row), which is
+      // right where any is positive, and the instruction does not quiet its operands first.
       using over_t = typename std::conditional<kWide, float, int>::type;
-      over_t s_over = 0;
-      if constexpr (kWide) s_over = s_max0;
+      over_t s_over[kWide ? 2 : 1] = {};
+      if constexpr (kWide) {
+        s_over[0] = s_max0[0];
+        s_over[1] = s_max0[1];
+      }
       // One step (kB = t % 4 picks the LDS buffers).  Straight-line code apart from small
       // wavefront-uniform branches, so that the accumulators stay where they are.
-      auto do_step = [&](int t, auto buf_tag, f32x16& s_cur, f32x16& s_next, u32x4 (&p_prev)[2], u32x4 (&p_cur)[2]) __attribute__((always_inline)) {
+      auto do_step = [&](int t, auto buf_tag, f32x4 (&s_cur)[4], f32x4 (&s_next)[4], u32x4 (&p_prev)[2], u32x4 (&p_cur)[2]) __attribute__((always_inline)) {
         constexpr int kB = decltype(buf_tag)::value;
         // V(t-1) and K(t+2), first read in this step, have landed once only what was asked for after them is outstanding:
         // V(t) of step t-2 and the four copies of step t-1 (K goes first in every step); after the barrier that holds for
@@ -1655,110 +1693,132 @@ sparse_fa_kernel(const FaParams p) {
         // the old point in this step, is rescaled at the step's end.
         bool over;
         if constexpr (kWide) {
-          over = __builtin_fmaf(s_over, f_blk, -m_run) > kLazyLog2;
+          over = __builtin_fmaf(s_over[0], f_blk, -m_q[0]) > kLazyLog2 || __builtin_fmaf(s_over[1], f_blk, -m_q[1]) > kLazyLog2;
         } else {
-          over = s_over > __builtin_bit_cast(int, kLazyLog2);
+          over = s_over[0] > __builtin_bit_cast(int, kLazyLog2);
         }
         const bool moved = __builtin_expect(__any(over), 0);
-        float o_scale = 1.f;
+        float o_scale[2] = {1.f, 1.f};
         if (moved) {
-          float mx = row_max(s_cur);  // row max relative to m_run
-          if constexpr (kWide) mx = __builtin_fmaf(mx, f_blk, -m_run);
-          const float delta = fmaxf(mx, 0.f);
-          o_scale = __builtin_amdgcn_exp2f(-delta);
-          d_part *= o_scale;
-          m_run += delta;
-          if constexpr (!kWide) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s_cur[i] -= delta;
+          for (int qt = 0; qt < 2; ++qt) {
+            float mx = row_max(s_cur, qt);  // row max relative to m_q
+            if constexpr (kWide) mx = __builtin_fmaf(mx, f_blk, -m_q[qt]);
+            const float delta = fmaxf(mx, 0.f);
+            o_scale[qt] = __builtin_amdgcn_exp2f(-delta);
+            d_q[qt] *= o_scale[qt];
+            m_q[qt] += delta;
+            if constexpr (!kWide) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s_init[i] -= delta;
+              for (int j = 0; j < 4; ++j) {
+                s_cur[qt][j] -= delta;
+                s_cur[2 + qt][j] -= delta;
+                s_init[qt][j] -= delta;
+              }
+            }
           }
         }
-        // The softmax goes in pairs of values, a pair in every second slot: exp2 there, rounding a pair later, the row sum
-        // (over the rounded values, as the reference takes it) another one later, so that nothing waits for the instruction
-        // in front of it.  (The empty statements pin a pair to its slot: without them the compiler gathers all exponentials
-        // of a step in front of its MFMAs.)
-        float psum = 0.f;
-        float x0, x1;
-        uint32_t pu;
-        auto round_pair = [&]() __attribute__((always_inline)) {
-          const x2 pk = {static_cast<T>(x0), static_cast<T>(x1)};
-          pu = __builtin_bit_cast(uint32_t, pk);
-        };
-        auto add_pair = [&](int u) __attribute__((always_inline)) {
-          const x2 pk = __builtin_bit_cast(x2, pu);
-          if constexpr (std::is_same<T, __bf16>::value) {
-            psum = __builtin_amdgcn_fdot2_f32_bf16(pk, ones2, psum, false);
-          } else {
-            psum = __builtin_amdgcn_fdot2(pk, ones2, psum, false);
+        // The softmax of S(t) goes in two bursts, after the MFMAs of S(t+1) and after those of P.V: six exponentials and ten,
+        // the first six's rounding and row sum (over the rounded values, as the reference takes it) in the second one, so
+        // that nothing waits for the instruction in front of it.  An exponential takes the vector ALU as long as an MFMA the
+        // matrix core; between two MFMAs of the same wavefront it delays the second one, behind a run of them the other
+        // workgroup's wavefront has the matrix core.
+        float psum[2] = {0.f, 0.f};
+        float x[16];
+        // value m of the lane's P: eight of q tile 0, then of q tile 1; of either four of keys 0..15, then of 16..31
+        auto logit = [&](int m) __attribute__((always_inline)) {
+          float f = s_cur[((m >> 2) & 1) * 2 + (m >> 3)][m & 3];
+          if constexpr (kWide) {
+            const float e = f;
+            asm volatile("v_fma_f32 %0, %1, %2, -%3" : "=v"(f) : "v"(e), "s"(f_blk), "v"(m_q[m >> 3]));
           }
-          p_cur[u >> 2][u & 3] = pu;
+          return f;
         };
+        // (Volatile, so that they stay where they are: the compiler gathers all exponentials of a step in front of its MFMAs
+        // otherwise.  It does not see what they are, so the waits that they need are here: three states between an MFMA and a
+        // write of what may have been its third operand, one between an exponential and whoever reads it.)
+        auto exponentials = [&](int from, int to) __attribute__((always_inline)) {
+          float f[16];
+          asm volatile("s_nop 2");
+#pragma unroll
+          for (int m = from; m < to; ++m) f[m] = logit(m);
+#pragma unroll
+          for (int m = from; m < to; ++m) asm volatile("v_exp_f32 %0, %1" : "=v"(x[m]) : "v"(f[m]));
+        };
+        auto round_and_add = [&](int from, int to) __attribute__((always_inline)) {
+#pragma unroll
+          for (int u = from / 2; u < to / 2; ++u) {
+            const x2 pk = {static_cast<T>(x[2 * u]), static_cast<T>(x[2 * u + 1])};
+            p_cur[u >> 2][u & 3] = __builtin_bit_cast(uint32_t, pk);
+          }
+#pragma unroll
+          for (int u = from / 2; u < to / 2; ++u) {
+            const x2 pk = __builtin_bit_cast(x2, static_cast<uint32_t>(p_cur[u >> 2][u & 3]));
+            if constexpr (std::is_same<T, __bf16>::value) {
+              psum[u >> 2] = __builtin_amdgcn_fdot2_f32_bf16(pk, ones2, psum[u >> 2], false);
+            } else {
+              psum[u >> 2] = __builtin_amdgcn_fdot2(pk, ones2, psum[u >> 2], false);
+            }
+          }
+        };
+        auto largest = [&](int from, int to) __attribute__((always_inline)) {
+          auto bits = [&](int j) __attribute__((always_inline)) { return __builtin_bit_cast(over_t, static_cast<float>(s_next[j >> 2][j & 3])); };
+          auto larger = [](over_t a, over_t b) __attribute__((always_inline)) {
+            if constexpr (kWide) return fmaxf(a, b);
+            else return max(a, b);
+          };
+#pragma unroll
+          for (int j = from; j < to; ++j) {
+            over_t& most = s_over[kWide ? (j >> 2) & 1 : 0];
+            most = j == 0 || (kWide && j == 4) ? bits(j) : larger(most, bits(j));
+          }
+        };
+        constexpr int kFirst = 6;  // (4 and 8: 0.3 and 1 % longer, 2 of 16: 5 %; in bursts of two 3 %, all sixteen at once 5 %)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int n = 0; n < 16; ++n) {
-          const int i = n & 7, u = n >> 1;
-          if (n < 8) {
-            s_next = TS::mfma(__builtin_bit_cast(q8, op[i]), qreg[i], n == 0 ? s_init : s_next);
-            op[i] = __builtin_bit_cast(u32x4, read_v((kB + 3) & 3, i >> 2, i & 3));
-          } else {
-            o_acc[i & 3] = TT::mfma(__builtin_bit_cast(x8, op[i]), __builtin_bit_cast(x8, p_prev[i >> 2]), o_acc[i & 3]);
-            op[i] = __builtin_bit_cast(u32x4, read_k((kB + 2) & 3, i));
-          }
-          // softmax of two values of S(t)
-          if (n & 1) {
-            if (u == 0) {
-              asm volatile("" : "+v"(s_cur));
-            } else if (u == 1) {
-              asm volatile("" : "+v"(s_cur), "+v"(x0), "+v"(x1));
+          const int i = n & 7;
+#pragma unroll
+          for (int qt = 0; qt < 2; ++qt) {
+            if (n < 8) {
+              f32x4& to = s_next[2 * (i & 1) + qt];
+              to = TS::mfma16(__builtin_bit_cast(q8, op[i]), qreg[2 * (i >> 1) + qt], n < 2 ? s_init[qt] : to);
             } else {
-              asm volatile("" : "+v"(s_cur), "+v"(x0), "+v"(x1), "+v"(pu), "+v"(psum));
+              o_tile[2 * i + qt] = TT::mfma16(__builtin_bit_cast(x8, op[i]), __builtin_bit_cast(x8, p_prev[qt]), o_tile[2 * i + qt]);
             }
-            float e0 = s_cur[2 * u], e1 = s_cur[2 * u + 1];
-            if (u >= 2) add_pair(u - 2);
-            if (u >= 1) round_pair();
-            if constexpr (kWide)
-              asm volatile("v_fma_f32 %0, %2, %4, -%5\n\tv_fma_f32 %1, %3, %4, -%5"
-                           : "=&v"(e0), "=v"(e1)
-                           : "v"(s_cur[2 * u]), "v"(s_cur[2 * u + 1]), "s"(f_blk), "v"(m_run));
-            x0 = __builtin_amdgcn_exp2f(e0);
-            x1 = __builtin_amdgcn_exp2f(e1);
           }
-          if (n >= 12) {
-            auto bits = [&](int j) __attribute__((always_inline)) { return __builtin_bit_cast(over_t, static_cast<float>(s_next[j])); };
-            auto larger = [](over_t a, over_t b) __attribute__((always_inline)) {
-              if constexpr (kWide) return fmaxf(a, b);
-              else return max(a, b);
-            };
-            if (n == 12) s_over = larger(larger(bits(0), bits(1)), bits(2));
-            if (n == 13) s_over = larger(larger(larger(larger(s_over, bits(3)), bits(4)), bits(5)), bits(6));
-            if (n == 14) s_over = larger(larger(larger(larger(s_over, bits(7)), bits(8)), bits(9)), bits(10));
-            if (n == 15) s_over = larger(larger(larger(larger(larger(s_over, bits(11)), bits(12)), bits(13)), bits(14)), bits(15));
+          if (n < 8) op[i] = __builtin_bit_cast(u32x4, read_v((kB + 3) & 3, i));
+          else op[i] = __builtin_bit_cast(u32x4, read_k((kB + 2) & 3, i));
+          __builtin_amdgcn_sched_barrier(0);
+          if (n == 7) {
+            exponentials(0, kFirst);
+          } else if (n == 15) {
+            round_and_add(0, kFirst);
+            exponentials(kFirst, 16);
+            asm volatile("s_nop 0" : "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]),
+                                     "+v"(x[14]), "+v"(x[15]));
+            round_and_add(kFirst, 16);
           }
-          // The MFMAs of S go first where the other workgroup's wavefront on this SIMD has one of P.V or softmax work ready:
-          // 1733 -> 1712 us on the video-sized list (the other way round 1751; the line two or three slots earlier or later
-          // 1730 to 1738).
-          if (n == 7) __builtin_amdgcn_s_setprio(0);
-          if (n == 15) __builtin_amdgcn_s_setprio(1);
-          // (all four copies among the MFMAs of S 1747, all among those of P.V 1736, every fourth slot from 1 / 2 on 1724 / 1754)
-          if (n == 1 || n == 5) {
-            copy_desc(k_rsrc, k_voff, k_soff + (n >> 2) * 16 * k_sn2, m0_k + kbuf(kB) + (n >> 2) * (4 * kPipeKRows4));
-          } else if (n == 8 || n == 11) {
-            copy_desc(v_rsrc, v_voff, v_soff + (n > 8) * 16 * v_sn2, m0_v + vbuf((kB + 2) & 3) + (n > 8) * 4096);
-          }
+          // (kWide, with two maxima: all of it at the end, 0.6 % of the layer's time)
+          if (kWide && n == 15) largest(0, 16);
+          if (!kWide && n >= 12) largest(n == 12 ? 0 : 4 * n - 49, 4 * n - 45 + (n == 15));
+          // The MFMAs of P.V go first where the other workgroup's wavefront on this SIMD has some of S or softmax work ready:
+          // 1742 -> 1714 us on the video-sized list; both kinds first 1778, softmax work after S as well 1750, nobody 1760.
+          if (n == 7) __builtin_amdgcn_s_setprio(1);
+          if (n == 15) __builtin_amdgcn_s_setprio(0);
+          // (the copies of K among the MFMAs of S, those of V among P.V's: 1 % longer; all four at n = 7: 3 %)
+          if (n == 1) copy_desc(k_rsrc, k_voff, k_soff, m0_k + kbuf(kB));
+          if (n == 3) copy_desc(k_rsrc, k_voff, k_soff + 16 * k_sn2, m0_k + kbuf(kB) + 4096);
+          if (n == 4) copy_desc(v_rsrc, v_voff, v_soff, m0_v + vbuf((kB + 2) & 3));
+          if (n == 6) copy_desc(v_rsrc, v_voff, v_soff + 16 * v_sn2, m0_v + vbuf((kB + 2) & 3) + 4 * kPipeVRows4);
           __builtin_amdgcn_sched_barrier(0);
         }
-        add_pair(6);
-        round_pair();
-        add_pair(7);
-        asm volatile("" : "+v"(psum), "+v"(p_cur[1][2]), "+v"(p_cur[1][3]), "+v"(s_over));
-        d_part += psum;
+        asm volatile("" : "+v"(psum[0]), "+v"(psum[1]), "+v"(p_cur[1][2]), "+v"(p_cur[1][3]), "+v"(s_over[0]));
+        d_q[0] += psum[0];
+        d_q[1] += psum[1];
         if (moved) {
 #pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o_acc[dt][i] *= o_scale;
+          for (int e = 0; e < 16; ++e) o_tile[e] *= o_scale[e & 1];
         }
       };
       using B0 = std::integral_constant<int, 0>;
@@ -1782,13 +1842,17 @@ sparse_fa_kernel(const FaParams p) {
       }
       __builtin_amdgcn_s_setprio(0);
       // P.V of the last step (real or padded; its V is in buffer 3)
+      // (addresses that the compiler does not know to be the loop's: those that both use it would form ahead of the loop, in
+      // sixteen registers, in place of immediate offsets)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) asm volatile("" : "+v"(vrd[x]));
       __builtin_amdgcn_s_waitcnt(0x0f70 | 6);  // vmcnt(6)
       __builtin_amdgcn_s_barrier();
 #pragma unroll
-      for (int i = 0; i < 8; ++i) op[i] = __builtin_bit_cast(u32x4, read_v(3, i >> 2, i & 3));
+      for (int i = 0; i < 8; ++i) op[i] = __builtin_bit_cast(u32x4, read_v(3, i));
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        o_acc[i & 3] = TT::mfma(__builtin_bit_cast(x8, op[i]), __builtin_bit_cast(x8, pB[i >> 2]), o_acc[i & 3]);
+      for (int e = 0; e < 16; ++e)
+        o_tile[e] = TT::mfma16(__builtin_bit_cast(x8, op[e >> 1]), __builtin_bit_cast(x8, pB[e & 1]), o_tile[e]);
       // The copies of the steps past the row's end (the loop asks for K four and V two steps ahead,
       // whatever is left of the row) are still in flight: they must have landed before the epilogue
       // lays the finished row out in the same LDS.  (Nothing else waits for them: the barrier below
@@ -2315,32 +2379,51 @@ sparse_fa_kernel(const FaParams p) {
       if constexpr (!kDirect) fetch_next((row_it + 1) & 1, false);
       else if constexpr (!kPipe) direct_next((row_it + 1) & 1);
     }
-    float m_all = 0.f, d_all = 0.f;  // kv group 0: row maximum and row sum over both groups
-    // A lane owns one q row and runs of four d: stored from here, a row would leave as 32 scattered
+    // kv group 0: row maximum and row sum over both groups (kPipe: of the lane's two q rows)
+    constexpr int kQ = kPipe ? 2 : 1;
+    float m_all[kQ] = {}, d_all[kQ] = {};
+    // the accumulators as 16 vectors of four d of one q row, vector e of q row e % kQ of the lane
+    auto o_get = [&](int e, int j) __attribute__((always_inline)) {
+      if constexpr (kPipe) return static_cast<float>(o_tile[e][j]);
+      else return static_cast<float>(o_acc[e >> 2][(e & 3) * 4 + j]);
+    };
+    // (kPipe: lane l < 32 has the value of q row l)
+    auto of_lane = [&](const float (&x)[kQ]) __attribute__((always_inline)) { 
+      const float low = x[0], high = x[kQ - 1];
+      return kPipe && (lane_m & 16) ? high : low;
+    };
+    // A lane owns one q row (kPipe: two) and runs of four d: stored from here, a row would leave as scattered
     // 8-byte pieces per instruction (measured: ~12 k cycles per row).  The finished row goes through
     // a padded LDS tile instead and leaves in 16-byte pieces, 16 consecutive lanes per 256-byte row.
-    int ln_out = l32_e;
+    int ln_out = lane_m;
     asm volatile("" : "+v"(ln_out));  // (not hoisted out of the row loop and spilled)
-    uint8_t* const out_row = smem + G::kOutOff + (qs * 32 + ln_out) * kOutRowBytes;
+    constexpr int kTileRows = kPipe ? 16 : 32;
+    uint8_t* const out_row = smem + G::kOutOff + (qs * 32 + ln_out % kTileRows) * kOutRowBytes + ln_out / kTileRows * 8;
+    auto out_at = [&](int e) __attribute__((always_inline)) {
+      return reinterpret_cast<x4*>(kPipe ? out_row + (e & 1) * 16 * kOutRowBytes + (e >> 1) * 32 : out_row + e * 16);
+    };
     bool store_row = parts == 1;
     if constexpr (kGroups == 1) {
       // one kv group: the accumulators hold the whole row
-      const float d_tot = d_part + __shfl_xor(d_part, 32, 64);
+      float d_tot[kQ], inv[kQ];
+#pragma unroll
+      for (int i = 0; i < kQ; ++i) {
+        const float d_half = d_q[i] + __shfl_xor(d_q[i], 16, 64);
+        d_tot[i] = d_half + __shfl_xor(d_half, 32, 64);
+        inv[i] = __builtin_amdgcn_rcpf(d_tot[i]);
+        m_all[i] = m_q[i];
+        d_all[i] = d_tot[i];
+      }
       if (!kDirect || parts == 1) {
-        const float inv = __builtin_amdgcn_rcpf(d_tot);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int e = 0; e < 16; ++e) {
+          x4 out;
 #pragma unroll
-          for (int i4 = 0; i4 < 4; ++i4) {
-            x4 out;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(o_acc[dt][i4 * 4 + j] * inv);
-            *reinterpret_cast<x4*>(out_row + (dt * 32 + i4 * 8 + g_e * 4) * sizeof(T)) = out;
-          }
-        if (row_ok_e && p.lse && g_e == 0) p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(d_tot) + m_run;
-      } else {
-        m_all = m_run;
-        d_all = d_tot;
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(o_get(e, j) * inv[e % kQ]);
+          *out_at(e) = out;
+        }
+        if (row_ok_e && p.lse && g_e == 0)
+          p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(of_lane(d_all)) + of_lane(m_all);
       }
     }
     if (kGroups == 2 && kg == 0) {
@@ -2360,15 +2443,12 @@ sparse_fa_kernel(const FaParams p) {
         for (int e = 0; e < 16; ++e) t4[e] = mo[(qs * 16 + e) * 64 + lane_m];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int e = 0; e < 16; ++e) {
+          x4 out;
 #pragma unroll
-          for (int i4 = 0; i4 < 4; ++i4) {
-            x4 out;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              out[j] = static_cast<T>(o_acc[dt][i4 * 4 + j] * w0 + t4[dt * 4 + i4][j] * w1);
-            *reinterpret_cast<x4*>(out_row + (dt * 32 + i4 * 8 + g_e * 4) * sizeof(T)) = out;
-          }
+          for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(o_get(e, j) * w0 + t4[e][j] * w1);
+          *out_at(e) = out;
+        }
         if (row_ok_e && p.lse && g_e == 0)
           p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(d_tot) + m;
       } else {
@@ -2383,8 +2463,8 @@ sparse_fa_kernel(const FaParams p) {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             o_acc[e >> 2][(e & 3) * 4 + j] = o_acc[e >> 2][(e & 3) * 4 + j] * a0 + t4[e][j] * a1;
-        m_all = m;
-        d_all = d_tot;
+        m_all[0] = m;
+        d_all[0] = d_tot;
       }
     }
     if ((kGroups == 2 || kDirect) && parts > 1) {
@@ -2410,10 +2490,10 @@ sparse_fa_kernel(const FaParams p) {
           float* lane_ws = part_ws + (qs * 16 * 2 * 64 + ln) * 2;
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
-            store_pair_device(lane_ws + e * 256, o_acc[e >> 2][(e & 3) * 4 + 0], o_acc[e >> 2][(e & 3) * 4 + 1]);
-            store_pair_device(lane_ws + e * 256 + 128, o_acc[e >> 2][(e & 3) * 4 + 2], o_acc[e >> 2][(e & 3) * 4 + 3]);
+            store_pair_device(lane_ws + e * 256, o_get(e, 0), o_get(e, 1));
+            store_pair_device(lane_ws + e * 256 + 128, o_get(e, 2), o_get(e, 3));
           }
-          store_pair_device(part_ws + 128 * 128 + (qs * 64 + ln) * 2, m_all, d_all);
+          store_pair_device(part_ws + 128 * 128 + (qs * 64 + ln) * 2, of_lane(m_all), of_lane(d_all));
         }
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this lane's partial results have left
         __syncthreads();
@@ -2430,35 +2510,46 @@ sparse_fa_kernel(const FaParams p) {
             return p.split_ws + static_cast<int64_t>(part_area(split_slot, i)) * kSplitPartFloats;
           };
           // (a part's maximum and sum are read twice: held in an array, they would be in scratch memory)
-          const float m_own = m_all, d_own = d_all;
-          auto part_stats = [&](int i, float& m, float& d) {
-            m = m_own;
-            d = d_own;
-            if (i != part) load_pair_device(part_base(i) + 128 * 128 + (qs * 64 + lane_m) * 2, m, d);
-          };
-          m_all = kNegInf;
-          for (int i = 0; i < parts; ++i) {
-            float m, d;
-            part_stats(i, m, d);
-            m_all = fmaxf(m_all, m);
+          float m_own[kQ], d_own[kQ];
+#pragma unroll
+          for (int q = 0; q < kQ; ++q) {
+            m_own[q] = m_all[q];
+            d_own[q] = d_all[q];
+            m_all[q] = kNegInf;
+            d_all[q] = 0.f;
           }
-          d_all = 0.f;
-          f32x16 acc[4];
+          auto part_stats = [&](int i, float (&m)[kQ], float (&d)[kQ]) __attribute__((always_inline)) {
 #pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
+            for (int q = 0; q < kQ; ++q) {
+              m[q] = m_own[q];
+              d[q] = d_own[q];
+              if (i != part)
+                load_pair_device(part_base(i) + 128 * 128 + (qs * 64 + (kPipe ? 16 * q + (lane_m & 15) : lane_m)) * 2, m[q], d[q]);
+            }
+          };
+          for (int i = 0; i < parts; ++i) {
+            float m[kQ], d[kQ];
+            part_stats(i, m, d);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[dt][e] = 0.f;
+            for (int q = 0; q < kQ; ++q) m_all[q] = fmaxf(m_all[q], m[q]);
+          }
+          f32x4 acc[16];
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
           const int ln = fresh_lane();
           for (int i = 0; i < parts; ++i) {
-            float m, d;
+            float m[kQ], d[kQ], a[kQ];
             part_stats(i, m, d);
             if (i == part) {
-              const float a = __builtin_amdgcn_exp2f(m - m_all);
-              d_all = __builtin_fmaf(d, a, d_all);
 #pragma unroll
-              for (int dt = 0; dt < 4; ++dt)
+              for (int q = 0; q < kQ; ++q) {
+                a[q] = __builtin_amdgcn_exp2f(m[q] - m_all[q]);
+                d_all[q] = __builtin_fmaf(d[q], a[q], d_all[q]);
+              }
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[dt][e] = __builtin_fmaf(o_acc[dt][e], a, acc[dt][e]);
+              for (int e = 0; e < 16; ++e)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[e][j] = __builtin_fmaf(o_get(e, j), a[e % kQ], acc[e][j]);
             } else {
               const float* lane_ws = part_base(i) + (qs * 16 * 2 * 64 + ln) * 2;
               // all loads of the part in flight together
@@ -2469,27 +2560,29 @@ sparse_fa_kernel(const FaParams p) {
                 load_pair_device(lane_ws + e * 256 + 128, u[e][2], u[e][3]);
               }
               __builtin_amdgcn_sched_barrier(0);
-              const float a = __builtin_amdgcn_exp2f(m - m_all);
-              d_all = __builtin_fmaf(d, a, d_all);
+#pragma unroll
+              for (int q = 0; q < kQ; ++q) {
+                a[q] = __builtin_amdgcn_exp2f(m[q] - m_all[q]);
+                d_all[q] = __builtin_fmaf(d[q], a[q], d_all[q]);
+              }
 #pragma unroll
               for (int e = 0; e < 16; ++e)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                  acc[e >> 2][(e & 3) * 4 + j] = __builtin_fmaf(u[e][j], a, acc[e >> 2][(e & 3) * 4 + j]);
+                for (int j = 0; j < 4; ++j) acc[e][j] = __builtin_fmaf(u[e][j], a[e % kQ], acc[e][j]);
             }
           }
-          const float inv = __builtin_amdgcn_rcpf(d_all);
+          float inv[kQ];
 #pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
+          for (int q = 0; q < kQ; ++q) inv[q] = __builtin_amdgcn_rcpf(d_all[q]);
 #pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-              x4 out;
+          for (int e = 0; e < 16; ++e) {
+            x4 out;
 #pragma unroll
-              for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(acc[dt][i4 * 4 + j] * inv);
-              *reinterpret_cast<x4*>(out_row + (dt * 32 + i4 * 8 + g_e * 4) * sizeof(T)) = out;
-            }
+            for (int j = 0; j < 4; ++j) out[j] = static_cast<T>(acc[e][j] * inv[e % kQ]);
+            *out_at(e) = out;
+          }
           if (row_ok_e && p.lse && g_e == 0)
-            p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(d_all) + m_all;
+            p.lse[q_tok_e * p.num_heads + my_head_e] = __builtin_amdgcn_logf(of_lane(d_all)) + of_lane(m_all);
         }
         if (tid == 0) p.sched[kSchedArrived + split_slot] = 0;  // re-armed for the next launch
         store_row = true;

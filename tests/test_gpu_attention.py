@@ -627,6 +627,35 @@ def test_logits_far_apart(dev, dtype, fp8, nk):
     assert float(out.abs().max()) <= float(v.abs().max()) * 1.02
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_row_tiles(dev, dtype):
+    """Requests that end at either side of every border of 16 q rows; logits of odd tiles of 16 rows have another size and
+    grow along the keys where those of even ones fall, so that a tile's reference point and sum are nobody else's."""
+    import flashomni_amd as fo
+    ql, heads = [1, 15, 16, 17, 31, 32, 33, 48, 49, 113, 127, 128, 129], 2
+    kl = [200 + 16 * i for i in range(len(ql))]
+    m = make_ragged_masks(ql, kl, heads, 1.0, 1.0, seed=35)
+    g = torch.Generator().manual_seed(35)
+    nq, nk = sum(ql), sum(kl)
+    odd = torch.cat([torch.arange(n) // 16 % 2 for n in ql]).view(-1, 1, 1).float()
+    q = (torch.randn(nq, heads, 128, generator=g) * (0.3 + odd) + 0.5 * (2 * odd - 1)).to(dtype)
+    ramp = torch.cat([torch.linspace(-2, 2, n) for n in kl]).view(-1, 1, 1)
+    k, v = (torch.randn(nk, heads, 128, generator=g) * 0.5 + ramp).to(dtype), torch.randn(nk, heads, 128, generator=g).to(dtype)
+    sym = [m[x] for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    t = lambda a: torch.from_numpy(a).to(dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(t(m["qo_indptr"]), t(m["kv_indptr"]), heads, heads, 128, q_data_type=dtype)
+    out, lse = w.run(q.to(dev), k.to(dev), v.to(dev), *(t(x) for x in sym), return_lse=True)
+    exp_lse = torch.full((nq, heads), float("nan"))
+    exp = oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=torch.zeros(nq, heads, 128, dtype=dtype),
+                                  lse=exp_lse)
+    # (logits of up to 20 in the log2 domain: the bound of the test below)
+    for r in range(len(ql)):
+        a, b = int(m["qo_indptr"][r]), int(m["qo_indptr"][r + 1])
+        assert rel_l2(out[a:b].cpu(), exp[a:b]) <= 2 * REL_L2, ql[r]
+        assert float((lse[a:b].cpu() - exp_lse[a:b]).abs().max()) < 5e-2, ql[r]
+
+
 @pytest.mark.parametrize("terms", ["bf16", "fp16", "fp8"])
 def test_rows_of_few_steps(dev, terms):
     """Rows of one to nine steps of 32 keys, at both sides of every border, whose logits grow from step to step in one
