@@ -44,12 +44,12 @@
 //
 // Long lists (eight rows per CU or more) run in a second form of the same kernel: a workgroup is
 // 4 wavefronts that own a whole row, two such workgroups share a CU, and the main loop is software-
-// pipelined in steps of 32 keys: the MFMAs of S(t+1) and P(t-1).V(t-1) are interleaved, instruction
-// by instruction, with the softmax of S(t), the operand reads eight MFMAs ahead and the copies two or three
-// steps ahead (see the kPipe branch of the kernel).  Measured on the video-sized lists it is ~12 %
+// pipelined in steps of 32 keys: the MFMAs of S(t+1) and P(t-1).V(t-1) and a part of the softmax of S(t) behind
+// either, with the operand reads eight operands ahead and the copies two or three
+// steps ahead (see the kPipe branch of the kernel).  Measured on the video-sized lists it is a quarter
 // faster than the two-phase form; on short decoded lists, whose rows are taken whole, a row's doubled latency
 // costs more than that.  Short lists read straight from the symbols are cut in parts as fine as it takes and run
-// in it from 2.5 candidates per CU on (fo_sparse_attention_direct below); long lists of two-term fp8 q and k do
+// in it where there are enough rows (direct_pipe below); long lists of two-term fp8 q and k do
 // once their k has been widened to fp16 (kWide, wide_serves).
 //
 // Numerics follow the reference kernel (include/flashomni/attention/prefill.cuh:759-962): base-2
@@ -2987,17 +2987,21 @@ extern "C" int64_t fo_sparse_fa_wide_bytes(int64_t max_rows, int32_t num_kv_head
 
 namespace {
 
-// From 2.5 candidates per CU on: two workgroups of four wavefronts per CU and the software-pipelined loop, whose
-// row boundaries pass beside the other workgroup's main loop; below, the two-phase loop with twice the wavefronts
-// per row.  Pipelined against two-phase, with (active rows, kept blocks): 864 candidates of 36 blocks 155 / 165 us
-// (100 %, 50 %), 273 / 295 (100 %, 100 %), 119 / 127 (75 %, 50 %), 62 / 59 (30 %, 50 %); 1000 of 25 blocks 106 / 113
-// (75 %, 50 %), 56 / 54 (30 %, 50 %); 512 of 32 blocks 76 / 72 (75 %, 50 %), 44 / 41 (30 %, 50 %); 216 of 9 blocks
-// 31 / 27.  What it needs besides: partial results of two shares per CU, room in LDS for a row's list (the
+// Two workgroups of four wavefronts per CU and the software-pipelined loop, whose row boundaries pass beside the other
+// workgroup's main loop; where there are too few rows for that, the two-phase loop with twice the wavefronts per row.
+// Two-phase against pipelined, us per call.  Where every row is computed (is_full) from 13/8 of a candidate per CU on:
+//   416 candidates of 13 blocks 61.2 / 51.0    408 of 102 370 / 298    408 of 17 74.9 / 67.3    432 of 36 148 / 131
+//   384 of 24 85.5 / 86.5    384 of 32 109 / 101    384 of 16 62.8 / 61.0
+// With symbols the host does not know how many rows there are, and from 2.5 per CU on (with active rows, kept blocks):
+//   625 of 25 36.5 / 37.1 (20 %, 50 %)    576 of 24 65.0 / 59.5 (75, 50) 37.9 / 29.8 (75, 10) 31.6 / 35.6 (20, 50)
+//   500 of 125 213 / 182 (75, 50) 95.4 / 87.6 (30, 50)    480 of 40 83 / 76 (75, 50) 30.6 / 35.5 (10, 30)
+// What it needs besides: partial results of two shares per CU, room in LDS for a row's list (the
 // longest row is bounded by all keep bits where there are several requests), 32-bit copy offsets.
 bool direct_pipe(const fo_attention_args& a, int num_cu) {
   const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
   const int64_t nkv = a.max_nnz / (a.batch == 1 ? n_cand : a.symbol_heads), span = (nkv + 1) * kBlockKV * 2;
-  return a.logits_soft_cap <= 0.f && 2 * n_cand >= int64_t(5) * num_cu && nkv <= kMaxRowBlocksOneGroupDirect &&
+  const bool enough = a.is_full ? 8 * n_cand >= int64_t(13) * num_cu : 2 * n_cand >= int64_t(5) * num_cu;
+  return a.logits_soft_cap <= 0.f && enough && nkv <= kMaxRowBlocksOneGroupDirect &&
          2 * num_cu <= kMaxShares && a.split_ws_bytes >= 2 * fo_sparse_fa_split_workspace_bytes() &&
          span * a.k_stride_n < (int64_t(1) << 32) && span * a.v_stride_n < (int64_t(1) << 32);
 }

@@ -306,3 +306,22 @@ def test_symbols_in_any_order(dev, ql, kl, heads):
     keep, keep_ip = moved(m["packed_keep"], m["keep_indptr"])
     got = w.run(q, k, v, t(info), t(keep), t(info_ip), t(keep_ip))
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tokens, heads", [(1627, 32), (1627, 31), (5200, 10), (10500, 5)])
+def test_full_rows_around_the_choice_of_form(dev, tokens, heads):
+    """Every row computed, 403 to 416 candidates: the two loops meet there."""
+    import flashomni_amd as fo
+    g = torch.Generator().manual_seed(tokens)
+    q, k, v = (torch.randn(tokens, heads, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(3))
+    ip = torch.tensor([0, tokens], dtype=torch.int32)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(ip, ip, heads, heads, 128, q_data_type=torch.bfloat16)
+    out, lse = w.run(q, k, v, is_full=True, return_lse=True)
+    rows = torch.cat([torch.arange(0, 130), torch.arange(tokens - 130, tokens)]).to(dev)
+    for h in (0, heads // 2, heads - 1):
+        s = q[rows, h].float() @ k[:, h].float().t().contiguous() * 128 ** -0.5
+        exp = torch.softmax(s, -1) @ v[:, h].float()
+        # (p and the result are rounded to 8 bits, q * scale as well: 1e-2 of the result's size at most)
+        assert float((out[rows, h].float() - exp).norm() / exp.norm()) <= 1e-2
+        assert float((lse[rows, h] - torch.logsumexp(s, -1) * 1.4426950408889634).abs().max()) < 2e-2
