@@ -8,8 +8,8 @@ The public surface (constructor, ``plan``, ``run``, ``run_return_lse``, the depr
   the launch that builds the batch's tables, and sizes the work list.  It does not wait: the first
   use on another stream does;
 * ``run()`` reads the bit-packed symbols on every call (the buffers may have been rewritten in place
-  by writers torch does not see).  Up to 1024 (q block, head) pairs (1792 with a float workspace of
-  66 MiB on 256 CUs, 1408 of them where ``is_full``) the attention launch takes its
+  by writers torch does not see).  Up to 1024 (q block, head) pairs (2047 with a float workspace of
+  66 MiB on 256 CUs) the attention launch takes its
   rows straight from them (fo_sparse_attention_direct) and keeps a copy; above, and for fp8, they
   are decoded into a compacted work list (fo_decode_sparse) that the sparse FlashAttention kernel
   runs over (fo_sparse_fa_run).  ``reuse_decoded=True`` runs the last list on the caller's word,
@@ -425,7 +425,7 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
     ``segment_packbits``.
 
     The float workspace receives the partial results of rows that are cut for several workgroups
-    (lists of up to 1792 (q block, head) pairs, and decoded ones of up to two rows per CU), so runs
+    (lists of up to 2047 (q block, head) pairs, and decoded ones of up to two rows per CU), so runs
     that share one, of one wrapper or of several, must not overlap in time: give wrappers that run on
     different streams a workspace each, or order the streams.
     """

@@ -413,10 +413,12 @@ struct DirectMask {
   int mask_first, nkv;
 };
 struct NoMask {};
-// candidates (symbol row, head): two per thread of a workgroup, four in the pipelined form, of which there is a kernel for
-// more (kMany: seven per thread; with the steps for them 1000 candidates would take 61.4 us in place of 59.7)
-constexpr int direct_max_cand(bool many) { return many ? 1792 : 1024; }
-constexpr int kDirectMaxFull = 1408;    // ... where every row is computed whole (is_full), see fo_sparse_attention_direct_serves
+// candidates (symbol row, head): two per thread of a workgroup, four in the pipelined form, of which there are kernels for
+// more (kMany: seven or eight per thread; 1000 candidates would take 61.4 us in place of 59.7 with the steps for seven, 1032 37.9 in
+// place of 36.8 with those for eight; kernels for five and six of them gain nothing).  From kDirectMost + 1 on lists are long ones
+// (long_list below, 256 CUs).
+constexpr int kDirectMost = 2047;
+constexpr int direct_max_cand(int many) { return many == 0 ? 1024 : 256 * many < kDirectMost ? 256 * many : kDirectMost; }
 constexpr int kDirectShareRows = 1024;  // rows of a share that the table of them holds (see direct_table_holds)
 constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
 constexpr int kDirectMapBytes = (1 << 16) - 16;  // keep bits that are staged in the tile buffers (both forms have as much)
@@ -443,7 +445,7 @@ constexpr int kDirectMinPart = 4;     // kv blocks that a part is worth: prologu
 // their phases together, there is no merge, and one's row prologue / epilogue overlaps the other's
 // main loop.  A row takes twice as long, so this is the form for long lists (many rows per CU).
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false, bool kDirect = false, bool kWide = false, bool kMany = false>
+          bool kCap = false, bool kDirect = false, bool kWide = false, int kMany = 0>
 __global__ void __launch_bounds__(kGroups * kGroupThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 sparse_fa_kernel(const FaParams p) {
   static_assert(!kWide || (kPipe && !kGqaPack && !kDirect), "widened operands are a variant of the pipelined loop");
@@ -779,7 +781,7 @@ sparse_fa_kernel(const FaParams p) {
   // even shares: the rows of this workgroup's share, where there may be more than the table holds row i at i % kDirectShareRows
   __shared__ uint16_t s_row_cand[kDirect ? kDirectShareRows : 1];  // a row's candidate ...
   __shared__ int s_row_u[kDirect ? kDirectShareRows + 1 : 1];      // ... and the cost at which its kv blocks begin
-  auto row_at = [](int i) { return kMany ? i & (kDirectShareRows - 1) : i; };
+  auto row_at = [](int i) { return kMany != 0 ? i & (kDirectShareRows - 1) : i; };
   constexpr int kMaxCand = direct_max_cand(kMany);
   __shared__ uint16_t s_zero[kDirect ? kMaxCand / 16 : 1];         // candidates this workgroup clears (of 16 or more)
   // first row of the share, candidates to clear; even shares: the row behind its last one (0: one item at most), shares, cost of all,
@@ -847,7 +849,7 @@ sparse_fa_kernel(const FaParams p) {
     it.q_scale = 1.f;
     it.k_scale0 = 0;
   };
-  constexpr int kCands = kMaxCand / (64 * kWaves);  // candidates of a thread, at most
+  constexpr int kCands = (kMaxCand + 64 * kWaves - 1) / (64 * kWaves);  // candidates of a thread, at most
   auto direct_schedule = [&]() {
     const int n_wg = gridDim.x, n_cand = p.n_blk * p.symbol_heads, dir_g = dir_index();
     // (All of a thread's candidates, also where it does not have as many: with a branch around each of those, their loads are
@@ -988,9 +990,9 @@ sparse_fa_kernel(const FaParams p) {
       }
     }
     if (tid < 3) s_dir[tid] = 0;
-    // rows and kv blocks in one scan: at most 1792 and 2^20 of them
+    // rows and kv blocks in one scan: at most 2047 and 2^20 of them
     constexpr int kBlockBits = 21;
-    static_assert(direct_max_cand(true) < (1 << (32 - kBlockBits)), "rows must fit above the kv blocks");
+    static_assert(kDirectMost < (1 << (32 - kBlockBits)), "rows must fit above the kv blocks");
     uint32_t mine = 0;
     int mx = 0;
 #pragma unroll
@@ -2734,7 +2736,7 @@ __global__ void __launch_bounds__(256) widen_k_kernel(
 }
 
 template <typename T, bool kFp8, bool kQLo, bool kKLo, int kGroups = 2, bool kPipe = false, bool kGqaPack = false,
-          bool kCap = false, bool kDirect = false, bool kWide = false, bool kMany = false>
+          bool kCap = false, bool kDirect = false, bool kWide = false, int kMany = 0>
 int launch(const FaParams& p, int64_t max_rows, hipStream_t stream) {
   constexpr int kSmemBytes = Geom<kFp8, kKLo, kGroups>::kSmemBytes;
   // (the attribute belongs to the kernel's code object on one device: set once per device; the flags
@@ -3018,19 +3020,23 @@ bool direct_table_holds(int64_t n_cand, int64_t max_nnz, int num_cu) {
 // Whether the launch takes its rows straight from the symbols.
 // Candidates that a workgroup's threads can go through at the top of a launch, and keep bits that every workgroup can
 // afford to read (2^20 bits = 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also
-// sorts their rows by head, so that one head's K and V at a time are in an XCD's L2: the more of a row's blocks are kept, the
-// earlier.  The lists that only the pipelined form takes, decoded -> straight from the symbols, us per call (rows, blocks kept):
-//   1032 candidates of 43 blocks  72 -> 62 (50, 10 %)  189 -> 170 (75, 50)  446 -> 383 (all)     1040 of 26  53 -> 44 (30, 5)
-//   1320 of 55                    71 -> 65 (20, 20)    273 -> 260 (75, 50)  654 -> 593 (all)     1040 of 65  101 -> 89 (70, 10)
-//   1536 of 64 to 192             256 -> 235 (70, 10)  759 -> 773 (100, 30) 779 -> 817, 1152 -> 1200 (all)
-//   1704 of 71                    210 -> 194 (50, 30)  427 -> 421 (75, 50)  971 -> 1008 (all)
-//   2040 of 85                    256 -> 246 (100, 10) 560 -> 573 (75, 50)  1356 -> 1420 (all)
+// sorts their rows by head, so that one head's K and V at a time are in an XCD's L2, and where they are enough rows for whole ones on
+// two workgroups per CU (long_list) they run in the pipelined form as well.  The lists that only the pipelined form takes, decoded (and in
+// the two-phase form) -> straight from the symbols, us per call (rows, blocks kept):
+//   1440 of 60    736 -> 628 (all)
+//   1720 of 43    635 -> 544 (all)
+//   1840 of 46    750 -> 636 (all)  328 -> 276 (80, 50 %)  126 -> 93 (80, 10)  107 -> 90 (20, 50)  51.5 -> 39.6 (10, 20)
+//   1824 of 76    1200 -> 1008      496 -> 427             147 -> 125          154 -> 134          61.1 -> 49.9
+//   1920 of 128   2037 -> 1779      836 -> 731             221 -> 193          249 -> 215          78.0 -> 67.0
+//   2040 of 85    1415 -> 1260      620 -> 531             175 -> 150          182 -> 164          65.7 -> 53.7
+//   2040 of 170   2798 -> 2511      1188 -> 1032           289 -> 266          334 -> 299          94.7 -> 82.8
+// (Decoded and in the pipelined form, whose queues have whole rows only, 1800 of 90 with 10 % of the rows take 78.7 in place of 63.4.)
 bool direct_takes(const fo_attention_args& a, int variant) {
   const int num_cu = fo_num_cu();
   const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
   return (a.dtype == FO_BF16 || a.dtype == FO_F16) && variant != 1 && n_cand >= 1 &&
-         (n_cand <= direct_max_cand(false) ||
-          (n_cand <= (a.is_full ? kDirectMaxFull : direct_max_cand(true)) && variant == 0 && direct_pipe(a, num_cu) &&
+         (n_cand <= direct_max_cand(0) ||
+          (n_cand <= kDirectMost && variant == 0 && direct_pipe(a, num_cu) &&
            direct_table_holds(n_cand, a.max_nnz, num_cu))) &&
          a.max_nnz <= (1 << 20) && num_cu >= 16 && num_cu <= kMaxShares &&
          a.split_ws_bytes >= fo_sparse_fa_split_workspace_bytes();
@@ -3057,7 +3063,7 @@ extern "C" int fo_sparse_attention_direct_may_serve(int32_t n_blk, int32_t symbo
   return direct_takes(a, 0);
 }
 
-extern "C" int32_t fo_sparse_attention_direct_max_pairs(void) { return direct_max_cand(true); }
+extern "C" int32_t fo_sparse_attention_direct_max_pairs(void) { return kDirectMost; }
 
 extern "C" int fo_sparse_attention_direct(const void* args) {
   FO_REQUIRE(args, "sparse_attention: null pointer");
@@ -3111,12 +3117,16 @@ extern "C" int fo_sparse_attention_direct(const void* args) {
     return bf16 ? launch<__bf16, false, false, false, 2, false, false, true, true>(p, n_cand, s)
                 : launch<_Float16, false, false, false, 2, false, false, true, true>(p, n_cand, s);
   }
-  if (n_cand > direct_max_cand(false)) {
-    if (packed)
-      return bf16 ? launch<__bf16, false, false, false, 1, true, true, false, true, false, true>(p, n_cand, s)
-                  : launch<_Float16, false, false, false, 1, true, true, false, true, false, true>(p, n_cand, s);
-    return bf16 ? launch<__bf16, false, false, false, 1, true, false, false, true, false, true>(p, n_cand, s)
-                : launch<_Float16, false, false, false, 1, true, false, false, true, false, true>(p, n_cand, s);
+  if (n_cand > direct_max_cand(0)) {
+    auto many = [&](auto per) {
+      constexpr int kPer = decltype(per)::value;
+      if (packed)
+        return bf16 ? launch<__bf16, false, false, false, 1, true, true, false, true, false, kPer>(p, n_cand, s)
+                    : launch<_Float16, false, false, false, 1, true, true, false, true, false, kPer>(p, n_cand, s);
+      return bf16 ? launch<__bf16, false, false, false, 1, true, false, false, true, false, kPer>(p, n_cand, s)
+                  : launch<_Float16, false, false, false, 1, true, false, false, true, false, kPer>(p, n_cand, s);
+    };
+    return n_cand <= direct_max_cand(7) ? many(std::integral_constant<int, 7>{}) : many(std::integral_constant<int, 8>{});
   }
   if (direct_pipe(a, fo_num_cu())) {
     if (packed)

@@ -332,9 +332,9 @@ int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, 
  * The same attention straight from the packed symbols, without a decoded list: short lists whose rows
  * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
- * candidates (1792 in the software-pipelined form, 1408 where is_full), more than 2^20 keep bits, no split workspace of
+ * candidates (2047 in the software-pipelined form), more than 2^20 keep bits, no split workspace of
  * fo_sparse_fa_split_workspace_bytes() bytes.
- * With twice that many bytes, from 2.5 candidates per CU on and where a row has at most 1024 kv blocks (of one
+ * With twice that many bytes, from 2.5 candidates per CU on (1.625 where is_full) and where a row has at most 1024 kv blocks (of one
  * request: the share of keep bits of a candidate; of several: all kv blocks), the launch runs in the
  * software-pipelined form, two workgroups per CU.
  * Arguments as in fo_decode_sparse (symbols, blk_req, blk_qb, is_full; n_blk symbol rows of symbol_heads

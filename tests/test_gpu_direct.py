@@ -88,9 +88,9 @@ def test_schedule_of_short_lists(dev, case, is_full):
 
 @pytest.mark.parametrize("case", [
     ([2049], [300], 64, 0.7),                  # 1088 candidates, seven to a thread
-    ([3584], [300], 64, 0.9),                  # 1792, ~1610 rows (every row: decoded)
-    ([3585], [300], 64, 0.9),                  # 1856: decoded
-    ([2816], [300], 64, 0.9),                  # 1408 (every row, too)
+    ([3584], [300], 64, 0.9),                  # 1792, ~1610 rows
+    ([3585], [300], 64, 0.9),                  # 1856: eight to a thread
+    ([2816], [300], 64, 0.9),                  # 1408
     ([3000, 1, 2300], [1200, 770, 1000], 40, 0.8),   # 1720 of three requests
     ([5500], [300], 24, 0.5),                  # 1032
     ([8200], [300], 16, 0.0),                  # 1040, nothing to compute
@@ -98,9 +98,29 @@ def test_schedule_of_short_lists(dev, case, is_full):
 ])
 @pytest.mark.parametrize("is_full", [False, True])
 def test_longer_lists_from_the_symbols(dev, case, is_full):
-    """1025 to 1792 candidates: seven to a thread at most, and only the rows of a workgroup's own share are in its table.
+    """1025 candidates and more: seven to a thread up to 1792, and only the rows of a workgroup's own share are in its table.
     (Keys enough that no result reaches 2: the list's is compared to one bf16 step of what is smaller.)"""
     test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
+
+
+@pytest.mark.parametrize("case", [
+    ([2944], [300], 78, 0.9),                  # 1794 candidates, eight to a thread
+    ([2944], [300], 89, 0.7),                  # 2047, the most
+    ([2048], [300], 128, 0.7),                 # 2048: decoded
+    ([3000, 1, 2300], [1200, 770, 1000], 47, 0.8),   # 2021 of three requests
+    ([9000], [300], 28, 0.0),                  # 1988, nothing to compute
+    ([4000], [9000], 60, 0.05),                # 1920 of 71 blocks, fewer rows than workgroups
+])
+@pytest.mark.parametrize("is_full", [False, True])
+def test_lists_of_eight_candidates_per_thread(dev, case, is_full):
+    """1793 to 2047 candidates, with the bounds of the test above."""
+    test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
+
+
+def test_fresh_output_of_the_shortest_decoded_lists(dev):
+    """2059 pairs: the test of longer lists below, past the line."""
+    test_fresh_output_of_longer_lists(dev, ([9000], [300], 29, 1, 0.0), "NHD")
+    test_fresh_output_of_longer_lists(dev, ([2000, 1, 130, 1500], [300, 77, 513, 640], 72, 1, 0.5), "HND")
 
 
 @pytest.mark.parametrize("empty", ["all", "half", "most"])
@@ -156,7 +176,7 @@ def test_fresh_output_of_packed_tiles(dev, group):
                                   ([9000], [300], 16, 1, 0.0), ([9000], [300], 26, 1, 0.0)])
 @pytest.mark.parametrize("layout", ["NHD", "HND"])
 def test_fresh_output_of_longer_lists(dev, case, layout):
-    """Lists above 1024 pairs, taken from the symbols, and above 1792, decoded: the launch, or the decoder's launches, clear
+    """Lists above 1024 pairs, taken from the symbols, and above 2047, decoded: the launch, or the decoder's launches, clear
     the skipped rows of a fresh output (ragged last tiles, tiles of grouped-query rows, nothing to compute); the same bits as
     over a cleared output."""
     import flashomni_amd as fo
