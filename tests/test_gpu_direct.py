@@ -117,6 +117,27 @@ def test_lists_of_eight_candidates_per_thread(dev, case, is_full):
     test_rows_from_the_symbols(dev, case, is_full, torch.bfloat16)
 
 
+@pytest.mark.parametrize("is_full", [False, True])
+def test_packed_tiles_of_eight_candidates_per_thread(dev, is_full):
+    """1880 tiles of grouped-query attention in fp16: as the decoded list, whose rows other workgroups compute whole."""
+    import flashomni_amd as fo
+    n, hkv, group = 6000, 10, 4
+    m = make_ragged_masks([n * group], [900], hkv, 0.7, 0.5, seed=12)
+    g = torch.Generator(device=dev).manual_seed(12)
+    q, k, v = (torch.randn(t, h, 128, generator=g, device=dev).to(torch.float16) for t, h in ((n, hkv * group), (900, hkv), (900, hkv)))
+    sym = [torch.from_numpy(m[x]).to(dev) for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    ip = lambda t: torch.tensor([0, t], dtype=torch.int32)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    w.plan(ip(n), ip(900), hkv * group, hkv, 128, q_data_type=torch.float16)
+    out, lse = w.run(q, k, v, *sym, is_full, out=torch.zeros_like(q), lse=torch.zeros(n, hkv * group, device=dev), return_lse=True)
+    assert w._planned.native.state != 0
+    w.decode(*sym, is_full)
+    exp, exp_lse = w.run(q, k, v, *sym, is_full, out=torch.zeros_like(q), lse=torch.zeros(n, hkv * group, device=dev),
+                         return_lse=True, reuse_decoded=True)
+    assert rel_l2(out.cpu(), exp.cpu()) <= 1e-3  # (p and the result in 11 bits)
+    assert torch.allclose(lse, exp_lse, atol=2e-3, rtol=1e-3)
+
+
 def test_fresh_output_of_the_shortest_decoded_lists(dev):
     """2059 pairs: the test of longer lists below, past the line."""
     test_fresh_output_of_longer_lists(dev, ([9000], [300], 29, 1, 0.0), "NHD")
