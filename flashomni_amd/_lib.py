@@ -50,6 +50,8 @@ SIGNATURES = {
     "fo_sparse_attention_direct_max_pairs": ([], c_i32),
     "fo_sparse_attention_direct_may_serve": ([c_i32, c_i32, c_i32, c_i64, c_i64, c_f32], c_int),
     "fo_sparse_attention_direct": ([c_vp], c_int),
+    "fo_sparse_attention_direct_own_bytes": ([c_vp], c_i64),
+    "fo_sparse_attention_direct_own": ([c_vp], c_int),
     "fo_gemm_workspace_bytes": ([c_i32, c_i32, c_i32], c_i64),
     "fo_gemm_q": ([c_vp] * 4 + [c_int] + [c_i32] * 6 + [c_vp, c_vp, c_i32, c_int, c_vp, c_i64, c_vp],
                   c_int),

@@ -425,9 +425,10 @@ class BatchFlashOmniFAWithRaggedKVWrapper:
     ``segment_packbits``.
 
     The float workspace receives the partial results of rows that are cut for several workgroups
-    (lists of up to 2047 (q block, head) pairs, and decoded ones of up to two rows per CU), so runs
+    (lists of up to 1792 (q block, head) pairs, and decoded ones of up to two rows per CU), so runs
     that share one, of one wrapper or of several, must not overlap in time: give wrappers that run on
-    different streams a workspace each, or order the streams.
+    different streams a workspace each, or order the streams.  Longer lists that are taken from the
+    symbols keep their parts in memory of the plan's (66 MiB on 256 CUs, made by the first such run).
     """
 
     def __init__(

@@ -320,6 +320,10 @@ struct Plan {
   // replay): room for the symbols that such a run takes, at keep_at[0] info, [1] kv_info, [2] the indptrs (bytes
   // from the start of the tables; keep_at[0] = 0: a batch that is always decoded).
   int64_t keep_at[3], keep_room[2];
+  // Partial results of the longer lists that are taken from the symbols, which leave the float workspace to others: made when first
+  // needed (66 MiB on 256 CUs).  no_parts: the allocator has refused it, and such runs are decoded from then on.
+  Tensor parts;
+  bool no_parts;
   fo_batch_sizes z;
 };
 
@@ -333,6 +337,7 @@ void plan_dealloc(PyObject* self) {
   p->tables.~Tensor();
   p->qo_keep.~Tensor();
   p->kv_keep.~Tensor();
+  p->parts.~Tensor();
   PyTypeObject* t = Py_TYPE(self);
   t->tp_free(self);
   Py_DECREF(t);
@@ -582,6 +587,7 @@ PyObject* plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   new (&p->used) std::vector<hipStream_t>();
   new (&p->qo_keep) Tensor();
   new (&p->kv_keep) Tensor();
+  new (&p->parts) Tensor();
   p->dev = dev;
   p->batch = batch;
   p->num_qo = hq;
@@ -872,7 +878,21 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool own = !out && p->from_zero && q->size(0) == p->z.total_q;
   const bool small = p->keep_at[0] && !p->list_only && (full || (sym[0]->numel() <= p->keep_room[0] && sym[1]->numel() <= p->keep_room[1]));
   int rc = FO_NOT_DIRECT;
-  if (small && fo_sparse_attention_direct_serves(&a)) {
+  const int64_t parts = small && !p->no_parts ? fo_sparse_attention_direct_own_bytes(&a) : 0;
+  if (parts && !p->parts.defined()) {
+    try {
+      p->parts = new_tensor({parts}, at::kByte, dev);
+    } catch (const c10::OutOfMemoryError&) {
+      p->no_parts = true;  // (a request that fails has the allocator give its cached blocks back first, which waits)
+    }
+  }
+  const bool own_parts = parts && p->parts.defined();
+  if (own_parts || (small && fo_sparse_attention_direct_serves(&a))) {
+    if (own_parts) {
+      hold(p->parts, dev);
+      a.split_ws = p->parts.data_ptr();
+      a.split_ws_bytes = p->parts.numel();
+    }
     if (!out) fresh = own ? at::empty(q->sizes(), q->options()) : at::zeros(q->sizes(), q->options());
     const Tensor& o = out ? *out : fresh;
     a.o = o.data_ptr();
@@ -886,7 +906,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
       a.kv_info_bytes = sym[1]->numel();
     }
     a.keep_indptr = t + p->keep_at[2] / 4;
-    rc = fo_sparse_attention_direct(&a);
+    rc = own_parts ? fo_sparse_attention_direct_own(&a) : fo_sparse_attention_direct(&a);
     if (rc < 0) return raise_last();
     if (rc == FO_OK) note(p, static_cast<hipStream_t>(stream), full ? 2 : 1, full);
   }

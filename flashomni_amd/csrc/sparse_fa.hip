@@ -418,6 +418,9 @@ struct NoMask {};
 // place of 36.8 with those for eight; kernels for five and six of them gain nothing).  From kDirectMost + 1 on lists are long ones
 // (long_list below, 256 CUs).
 constexpr int kDirectMost = 2047;
+// ... of which up to so many (is_full: every row is computed) may leave partial results in a workspace that other batches' launches use,
+// see direct_shares_workspace
+constexpr int kDirectShared = 1792, kDirectSharedFull = 1408;
 constexpr int direct_max_cand(int many) { return many == 0 ? 1024 : 256 * many < kDirectMost ? 256 * many : kDirectMost; }
 constexpr int kDirectShareRows = 1024;  // rows of a share that the table of them holds (see direct_table_holds)
 constexpr int kDirectMaxParts = 8;    // parts of a row, one workgroup each
@@ -3017,6 +3020,8 @@ bool direct_table_holds(int64_t n_cand, int64_t max_nnz, int num_cu) {
           (4 * longest / 9 + 2) / kRowOverheadPipe + 3 < kDirectShareRows);
 }
 
+int64_t direct_candidates(const fo_attention_args& a) { return static_cast<int64_t>(a.n_blk) * a.symbol_heads; }
+
 // Whether the launch takes its rows straight from the symbols.
 // Candidates that a workgroup's threads can go through at the top of a launch, and keep bits that every workgroup can
 // afford to read (2^20 bits = 128 KB from L2: about as long as the scans).  Longer lists are worth a decode launch, which also
@@ -3033,7 +3038,7 @@ bool direct_table_holds(int64_t n_cand, int64_t max_nnz, int num_cu) {
 // (Decoded and in the pipelined form, whose queues have whole rows only, 1800 of 90 with 10 % of the rows take 78.7 in place of 63.4.)
 bool direct_takes(const fo_attention_args& a, int variant) {
   const int num_cu = fo_num_cu();
-  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  const int64_t n_cand = direct_candidates(a);
   return (a.dtype == FO_BF16 || a.dtype == FO_F16) && variant != 1 && n_cand >= 1 &&
          (n_cand <= direct_max_cand(0) ||
           (n_cand <= kDirectMost && variant == 0 && direct_pipe(a, num_cu) &&
@@ -3044,10 +3049,30 @@ bool direct_takes(const fo_attention_args& a, int variant) {
 
 }  // namespace
 
-extern "C" int fo_sparse_attention_direct_serves(const void* args) {
-  const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
+namespace {
+
+bool direct_serves(const fo_attention_args& a) {
   return direct_takes(a, g_variant.load(std::memory_order_relaxed)) && a.split_ws &&
          (reinterpret_cast<uintptr_t>(a.split_ws) & 15) == 0;
+}
+
+// Longer lists are promised to callers not to touch a workspace that other batches' launches may be using: they need one of their own.
+bool direct_shares_workspace(const fo_attention_args& a) {
+  return direct_candidates(a) <= (a.is_full ? kDirectSharedFull : kDirectShared);
+}
+
+int direct_run(const fo_attention_args& a);
+
+}  // namespace
+
+extern "C" int fo_sparse_attention_direct_serves(const void* args) {
+  const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
+  return direct_shares_workspace(a) && direct_serves(a);
+}
+
+extern "C" int64_t fo_sparse_attention_direct_own_bytes(const void* args) {
+  const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
+  return !direct_shares_workspace(a) && direct_serves(a) ? 2 * fo_sparse_fa_split_workspace_bytes() : 0;
 }
 
 extern "C" int fo_sparse_attention_direct_may_serve(int32_t n_blk, int32_t symbol_heads, int32_t batch, int64_t max_nnz,
@@ -3067,9 +3092,18 @@ extern "C" int32_t fo_sparse_attention_direct_max_pairs(void) { return kDirectMo
 
 extern "C" int fo_sparse_attention_direct(const void* args) {
   FO_REQUIRE(args, "sparse_attention: null pointer");
-  const fo_attention_args& a = *static_cast<const fo_attention_args*>(args);
-  if (!fo_sparse_attention_direct_serves(args)) return FO_NOT_DIRECT;
-  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  return fo_sparse_attention_direct_serves(args) ? direct_run(*static_cast<const fo_attention_args*>(args)) : FO_NOT_DIRECT;
+}
+
+extern "C" int fo_sparse_attention_direct_own(const void* args) {
+  FO_REQUIRE(args, "sparse_attention: null pointer");
+  return fo_sparse_attention_direct_own_bytes(args) ? direct_run(*static_cast<const fo_attention_args*>(args)) : FO_NOT_DIRECT;
+}
+
+namespace {
+
+int direct_run(const fo_attention_args& a) {
+  const int64_t n_cand = direct_candidates(a);
   FO_REQUIRE(a.q && a.k && a.v && a.o && a.qo_indptr && a.kv_indptr && a.blk_req && a.blk_qb && a.sched,
              "sparse_attention: null pointer");
   FO_REQUIRE(a.is_full || (a.info && a.kv_info && a.info_indptr && a.kv_info_indptr), "sparse_attention: null symbols");
@@ -3141,3 +3175,5 @@ extern "C" int fo_sparse_attention_direct(const void* args) {
   return bf16 ? launch<__bf16, false, false, false, 2, false, false, false, true>(p, n_cand, s)
               : launch<_Float16, false, false, false, 2, false, false, false, true>(p, n_cand, s);
 }
+
+}  // namespace

@@ -332,7 +332,8 @@ int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, 
  * The same attention straight from the packed symbols, without a decoded list: short lists whose rows
  * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
- * candidates (2047 in the software-pipelined form), more than 2^20 keep bits, no split workspace of
+ * candidates (1792 in the software-pipelined form, 1408 of them where is_full; up to 2047: see
+ * fo_sparse_attention_direct_own), more than 2^20 keep bits, no split workspace of
  * fo_sparse_fa_split_workspace_bytes() bytes.
  * With twice that many bytes, from 2.5 candidates per CU on (1.625 where is_full) and where a row has at most 1024 kv blocks (of one
  * request: the share of keep bits of a candidate; of several: all kv blocks), the launch runs in the
@@ -366,11 +367,18 @@ typedef struct fo_attention_args {
 } fo_attention_args;
 enum { FO_NOT_DIRECT = 1 };
 int fo_sparse_attention_direct_serves(const void* args);  /* 1: fo_sparse_attention_direct takes the batch */
-int32_t fo_sparse_attention_direct_max_pairs(void);       /* ... and never one of more (symbol row, head) pairs */
+int32_t fo_sparse_attention_direct_max_pairs(void);       /* ... and never, nor _own, one of more (symbol row, head) pairs */
 /* 0: no 16-bit call over such a batch, with such a workspace and soft cap, is ever taken, whatever its strides and is_full */
 int fo_sparse_attention_direct_may_serve(int32_t n_blk, int32_t symbol_heads, int32_t batch, int64_t max_nnz,
                                          int64_t split_ws_bytes, float logits_soft_cap);
 int fo_sparse_attention_direct(const void* args);
+/* Longer lists, of up to fo_sparse_attention_direct_max_pairs() pairs, the same way, with partial results in memory that no other
+ * batch's launches use: as decoded lists they leave a workspace alone that others may be using at the time.
+ * fo_sparse_attention_direct_own_bytes: how much the batch needs, 0 where it is not such a list, or args' split_ws is not one
+ * that it could be served with if it were this batch's own (twice fo_sparse_fa_split_workspace_bytes()).
+ * fo_sparse_attention_direct_own: args' split_ws is that memory; FO_NOT_DIRECT where _own_bytes is 0. */
+int64_t fo_sparse_attention_direct_own_bytes(const void* args);
+int fo_sparse_attention_direct_own(const void* args);
 
 /* ---------------------------------------------------------------------------------------------
  * GEMM-Q: y[b, tile] = x[b] . w^T + bias for every (128-row, 128-column) tile whose symbol bit

@@ -366,3 +366,58 @@ def test_full_rows_around_the_choice_of_form(dev, tokens, heads):
         # (p and the result are rounded to 8 bits, q * scale as well: 1e-2 of the result's size at most)
         assert float((out[rows, h].float() - exp).norm() / exp.norm()) <= 1e-2
         assert float((lse[rows, h] - torch.logsumexp(s, -1) * 1.4426950408889634).abs().max()) < 2e-2
+
+
+def _long_list(dev, pairs, is_full, room=128 << 20):
+    """A planned list of `pairs` over 300 keys, as a call without arguments; its wrapper and workspace."""
+    import flashomni_amd as fo
+    blocks, heads = pairs
+    tokens = 128 * blocks
+    m = make_ragged_masks([tokens], [300], heads, 0.9, 0.5, seed=14)
+    g = torch.Generator(device=dev).manual_seed(14)
+    q, k, v = (torch.randn(n, heads, 128, generator=g, device=dev).to(torch.bfloat16) for n in (tokens, 300, 300))
+    sym = [torch.from_numpy(m[x]).to(dev) for x in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
+    ws = torch.full((room,), 0x5a, dtype=torch.uint8, device=dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(ws)
+    w.plan(*(torch.tensor([0, n], dtype=torch.int32) for n in (tokens, 300)), heads, heads, 128, q_data_type=torch.bfloat16)
+    out = torch.zeros_like(q)
+    return w, ws, sym, out, lambda **kw: w.run(q, k, v, *sym, is_full, out=out, **kw)
+
+
+@pytest.mark.parametrize("pairs, is_full, shares", [((28, 64), False, True), ((23, 78), False, False), ((23, 89), False, False),
+                                                    ((22, 64), True, True), ((23, 62), True, False), ((23, 89), True, False)])
+def test_long_lists_leave_the_float_workspace_alone(dev, pairs, is_full, shares):
+    """1792 pairs and fewer (1408 where every row is computed) leave partial results in the float workspace.  Longer lists, which
+    were always decoded once, leave it to others that may be using it at the time."""
+    w, ws, sym, out, run = _long_list(dev, pairs, is_full)
+    run()
+    assert w._planned.native.state != 0
+    assert bool((ws == 0x5a).all()) != shares
+    exp = out.clone()
+    out.zero_()
+    w.decode(*sym, is_full)
+    ws.fill_(0x5a)
+    run(reuse_decoded=True)
+    assert bool((ws == 0x5a).all())    # (more than two rows per CU: taken whole)
+    # (p and the result are rounded to 8 bits on either side, by 2^-9 / sqrt(3) of it each: together 2.3e-3, four times that)
+    assert rel_l2(out.cpu(), exp.cpu()) <= 1e-2
+
+
+def test_long_list_without_room_for_its_parts(dev):
+    """The allocator has nothing left for the parts of rows: the list is decoded, and later runs do not ask again."""
+    w, ws, sym, out, run = _long_list(dev, (23, 78), False)
+    w.decode(*sym)
+    run(reuse_decoded=True)
+    exp = out.clone()
+    torch.cuda.synchronize(dev)
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (8 << 20)) / total, dev)
+    try:
+        out.zero_()
+        run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert w._planned.native.state == 0 and torch.equal(out, exp)
+    run()
+    assert w._planned.native.state == 0 and torch.equal(out, exp)

@@ -281,14 +281,11 @@ def test_captured_reuse_runs_the_list_of_the_moment(dev):
     s.check(s.full, s.run, [None] * 4, reuse=True, is_full=True)
 
 
-class _LongerList(_ShortList):
-    heads = 206    # 1030 candidates: decoded, where a list is asked for, by three launches
-
-
-def test_captured_lists_of_three_launches(dev, monkeypatch):
-    """The same where what a run left behind is decoded by more than one launch, of which the device decides each."""
-    import sys
-    monkeypatch.setattr(sys.modules[__name__], "_ShortList", _LongerList)
+@pytest.mark.parametrize("heads", [206, 408])
+def test_captured_lists_of_three_launches(dev, heads, monkeypatch):
+    """The same where what a run left behind is decoded by more than one launch, of which the device decides each: 1030
+    candidates, and 2040, eight to a thread, whose parts of rows lie in memory of the plan's."""
+    monkeypatch.setattr(_ShortList, "heads", heads)
     test_captured_reuse_runs_the_list_of_the_moment(dev)
 
 
