@@ -344,7 +344,9 @@ int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, 
  * row, as in fo_sparse_fa_run.
  * zero_skipped: the rows of q blocks that are not computed are cleared in o.  keep_info,
  * keep_kv_info, keep_indptr (optional): receive the info_bytes / kv_info_bytes of symbols and the two
- * indptrs ([2 * (batch + 1)]) that this launch read, for a decode of the same list later; with keep_indptr (also
+ * indptrs ([2 * (batch + 1)]) that this launch read, for a decode of the same list later.  kv_info_bytes is the size of
+ * kv_info in any case: no byte behind it is read, whatever the last entry of kv_info_indptr says; 0 without keep_kv_info: not known,
+ * that entry is then taken for the end of the segments.  With keep_indptr (also
  * where is_full needs no copy) the launch sets sched[33] to 1 (is_full: 2), see fo_decode_sparse_kept.
  * Launches that share sched or split_ws must not overlap in time.
  * ------------------------------------------------------------------------------------------- */

@@ -347,6 +347,12 @@ def test_symbols_in_any_order(dev, ql, kl, heads):
     keep, keep_ip = moved(m["packed_keep"], m["keep_indptr"])
     got = w.run(q, k, v, t(info), t(keep), t(info_ip), t(keep_ip))
     assert torch.equal(got, want)
+    # where the last segment ends is nobody's beginning: whatever stands there, no byte behind the segments is asked for
+    for end in (0, len(m["packed_keep"]) + 40000, 2 ** 31 - 1):
+        ip = m["keep_indptr"].copy()
+        ip[-1] = end
+        got = w.run(q, k, v, t(m["packed_info"]), t(m["packed_keep"]), t(m["info_indptr"]), t(ip))
+        assert torch.equal(got, want), end
 
 
 @pytest.mark.parametrize("tokens, heads", [(1627, 32), (1627, 31), (5200, 10), (10500, 5)])
@@ -413,10 +419,15 @@ def test_long_list_without_room_for_its_parts(dev):
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(dev).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (8 << 20)) / total, dev)
+    held = []    # (what is left in the allocator's own blocks)
     try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            for _ in range(1000):
+                held.append(torch.empty(60 << 20, dtype=torch.uint8, device=dev))
         out.zero_()
         run()
     finally:
+        held.clear()
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
     assert w._planned.native.state == 0 and torch.equal(out, exp)
     run()
