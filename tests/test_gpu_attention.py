@@ -649,11 +649,24 @@ def test_row_tiles(dev, dtype):
     exp_lse = torch.full((nq, heads), float("nan"))
     exp = oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=torch.zeros(nq, heads, 128, dtype=dtype),
                                   lse=exp_lse)
-    # (logits of up to 20 in the log2 domain: the bound of the test below)
+    # (logits of up to 20 in the log2 domain: the bounds of the test below)
+    rel, lse_off = _bounds_of_large_logits({torch.bfloat16: "bf16", torch.float16: "fp16"}[dtype])
     for r in range(len(ql)):
         a, b = int(m["qo_indptr"][r]), int(m["qo_indptr"][r + 1])
-        assert rel_l2(out[a:b].cpu(), exp[a:b]) <= 2 * REL_L2, ql[r]
-        assert float((lse[a:b].cpu() - exp_lse[a:b]).abs().max()) < 5e-2, ql[r]
+        assert rel_l2(out[a:b].cpu(), exp[a:b]) <= rel, ql[r]
+        assert float((lse[a:b].cpu() - exp_lse[a:b]).abs().max()) < lse_off, ql[r]
+
+
+def _bounds_of_large_logits(terms):
+    """(relative error, error of the log-sum-exp) of rows whose logits reach 20 in the log2 domain.
+
+    bf16: q times the scale is rounded to 8 bits, a logit is off by 2^-9 of its products' root sum of squares, about
+    20 * 2^-9 / sqrt(128) * 3: 1e-2, so an output of unit size by as much.  fp16 has three bits more.
+    Two-term fp8: the scales stay in fp32.  What the terms' products leave out, k_lo.q_lo, is a residual of 2^-4 / sqrt(3) of a
+    binade, 0.025 of the value, times another: 6e-4 of a product; of 128 products of one sign that add up to 34, four times
+    the root of their sum, 34 / sqrt(128) * 6e-4 * 4: 7.2e-3.  Widened to 11 bits the sums are off by less.  p and the result are
+    rounded as for bf16."""
+    return {"bf16": (2 * REL_L2, 5e-2), "fp16": (2 * REL_L2 / 8, 5e-2 / 8), "fp8": (REL_L2, 1e-2)}[terms]
 
 
 @pytest.mark.parametrize("terms", ["bf16", "fp16", "fp8"])
@@ -692,13 +705,13 @@ def test_rows_of_few_steps(dev, terms):
     exp = oracle.sparse_attention(q, k, v, *sym, m["qo_indptr"], m["kv_indptr"], out=torch.zeros(nq, heads, 128, dtype=dtype),
                                   lse=exp_lse, **extra)
     out, lse = out.cpu(), lse.cpu()
-    # per request: a short one must not hide behind the long ones.  (A logit of up to 20 in the log2 domain is off by 2^-9
-    # of its products' root sum of squares, about 20 * 2^-9 / sqrt(128) * 3: 1e-2, so an output of unit size by as much.)
+    # per request: a short one must not hide behind the long ones
+    rel, lse_off = _bounds_of_large_logits(terms)
     for r in range(len(kl)):
         a, b = int(m["qo_indptr"][r]), int(m["qo_indptr"][r + 1])
         rows = ok[a:b]
-        assert rel_l2(out[a:b][rows], exp[a:b][rows]) <= 2 * REL_L2, kl[r]
-        assert float((lse[a:b][rows] - exp_lse[a:b][rows]).abs().max()) < 5e-2, kl[r]
+        assert rel_l2(out[a:b][rows], exp[a:b][rows]) <= rel, kl[r]
+        assert float((lse[a:b][rows] - exp_lse[a:b][rows]).abs().max()) < lse_off, kl[r]
 
 
 def _split_case(dev, ql, kl, heads, seed, share, dtype=torch.bfloat16, pk=0.6):

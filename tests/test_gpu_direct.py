@@ -10,6 +10,14 @@ from helpers import make_ragged_masks, max_abs, rel_l2
 
 pytestmark = pytest.mark.gpu
 
+def _cus(dev):
+    return torch.cuda.get_device_properties(dev).multi_processor_count
+
+
+def _pairs(ql, heads):
+    return sum(-(-n // 128) for n in ql) * heads
+
+
 CASES = [
     ([1], [1], 1, 1.0),
     ([640], [20000], 1, 1.0),                 # 5 rows of ~80 kept blocks: eight parts each
@@ -45,6 +53,8 @@ def test_rows_from_the_symbols(dev, case, is_full, dtype):
     junk = torch.full((64 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
     del junk
     out, lse = w.run(*args, lse=lse, return_lse=True)
+    if _cus(dev) == 256:
+        assert (w._planned.native.state != 0) == (_pairs(ql, heads) <= 2047)    # (0: decoded)
     again, lse2 = w.run(*args, lse=lse.clone(), return_lse=True)
     assert torch.equal(out, again) and torch.equal(lse, lse2)
     exp_lse = torch.full((nq, heads), 7.0)
@@ -201,7 +211,6 @@ def test_fresh_output_of_longer_lists(dev, case, layout):
     the skipped rows of a fresh output (ragged last tiles, tiles of grouped-query rows, nothing to compute); the same bits as
     over a cleared output."""
     import flashomni_amd as fo
-    from flashomni_amd import _lib
     ql, kl, hkv, group, pa = case
     hq = hkv * group
     pairs = sum(-(-n * group // 128) for n in ql) * hkv
@@ -215,8 +224,8 @@ def test_fresh_output_of_longer_lists(dev, case, layout):
     w.plan(qo, t("kv_indptr"), hq, hkv, 128, q_data_type=torch.bfloat16)
     sym = [t(n) for n in ("packed_info", "packed_keep", "info_indptr", "keep_indptr")]
     exp = w.run(q, k, v, *sym, out=torch.zeros_like(q))
-    decoded = w._planned.native.state == 0
-    assert decoded == (pairs > _lib.lib().fo_sparse_attention_direct_max_pairs())
+    if _cus(dev) == 256:
+        assert (w._planned.native.state == 0) == (pairs > 2047)
     for _ in range(3):
         junk = torch.full((256 << 20,), 0x7f, dtype=torch.uint8, device=dev)   # what a fresh allocation may hold
         del junk
@@ -355,16 +364,24 @@ def test_symbols_in_any_order(dev, ql, kl, heads):
         assert torch.equal(got, want), end
 
 
-@pytest.mark.parametrize("tokens, heads", [(1627, 32), (1627, 31), (5200, 10), (10500, 5)])
+@pytest.mark.parametrize("tokens, heads", [(1627, 32), (1627, 31), (5200, 10), (6600, 8), (10500, 5)])
 def test_full_rows_around_the_choice_of_form(dev, tokens, heads):
-    """Every row computed, 403 to 416 candidates: the two loops meet there."""
+    """Every row computed, 403 to 416 candidates: the two loops meet there.  (Of the two workgroups per CU of the pipelined one
+    the second ones' parts lie in the second half of the float workspace, where rows are long enough to be cut.)"""
     import flashomni_amd as fo
+    from flashomni_amd import _lib
     g = torch.Generator().manual_seed(tokens)
     q, k, v = (torch.randn(tokens, heads, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(3))
     ip = torch.tensor([0, tokens], dtype=torch.int32)
-    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(torch.empty(128 << 20, dtype=torch.uint8, device=dev))
+    ws = torch.full((128 << 20,), 0x5a, dtype=torch.uint8, device=dev)
+    w = fo.BatchFlashOmniFAWithRaggedKVWrapper(ws)
     w.plan(ip, ip, heads, heads, 128, q_data_type=torch.bfloat16)
     out, lse = w.run(q, k, v, is_full=True, return_lse=True)
+    half = _lib.lib().fo_sparse_fa_split_workspace_bytes()
+    if _cus(dev) == 256:
+        assert w._planned.native.state != 0
+        if tokens >= 40 * 128:
+            assert bool((ws[half:2 * half] != 0x5a).any()) == (_pairs([tokens], heads) >= 416)
     rows = torch.cat([torch.arange(0, 130), torch.arange(tokens - 130, tokens)]).to(dev)
     for h in (0, heads // 2, heads - 1):
         s = q[rows, h].float() @ k[:, h].float().t().contiguous() * 128 ** -0.5
