@@ -2096,11 +2096,12 @@ __global__ void __launch_bounds__(kThreads, 4) gemm_packed_kernel(const GemmPara
 //
 // Tiles of 16 x 16 over 32 of k: an accumulator is read and written once per 32 of k instead of once per 16, and the card
 // sustains 1.98 PFLOP/s of them on random operands against 1.76 of 32 x 32 x 16 (registers only, all CUs, both at the power limit;
-// with zeros both reach 2.42).  GEMM-O of 76 112 x 5120 with 80 % 2835 -> 2640 us, of 4608 x 3072, both passes, 97.5 -> 94.
-// They are worth it where two wavefronts share a SIMD and the vector ALU has nothing else to issue: quads, one wavefront to a
+// with zeros both reach 2.42).  GEMM-O of 76 112 x 5120 with 80 % 2823 -> 2738 us, of 4608 x 3072, both passes, 101.2 -> 97.5.
+// They are worth it where two wavefronts share a SIMD and the vector ALU has little else to issue between them: quads, one wavefront to a
 // SIMD, wait for their own loads with 16 cycles of MFMA in flight instead of 32 (GEMM-Q of 76 112 x 5120 2940 -> 3230), as do
 // strips of flagged units that have a CU each, which keep 32 x 32 (16 384 x 3072 with a tenth flagged, new inputs, 49.2 us, in 16 x 16
-// 50.3), and the attention loop's exponentials want the issue slots that twice as many MFMAs take (33 k tokens x 24 heads 1709 -> 1785).
+// 50.3).  The attention loop runs them in runs of sixteen, its exponentials behind them; with MFMAs and exponentials in turn, which
+// want the same issue slots, they took longer there (33 k tokens x 24 heads 1709 -> 1785).
 // ---------------------------------------------------------------------------------------------
 constexpr int kStripPiece = 2 * 32 * kRowBytes;  // 32 rows of W of both column blocks
 constexpr int kStripRing = 6;

@@ -767,7 +767,7 @@ sparse_fa_kernel(const FaParams p) {
     __builtin_amdgcn_s_waitcnt(0x0f70);
   };
   // ---- kDirect: rows straight from the packed symbols (short lists) ----
-  // Every workgroup reads all flags and keep bits itself, two, four or seven candidates (symbol row, head) per
+  // Every workgroup reads all flags and keep bits itself, two, four, seven or eight candidates (symbol row, head) per
   // thread in head-major order, and works out with two or three workgroup scans which rows or parts of rows
   // are its own.  A decode launch in front of this one costs 8-15 us and a launch gap at these sizes, most of
   // it latency of a single workgroup; here the same trips to memory (two, for a batch of one request) replace
@@ -1427,9 +1427,9 @@ sparse_fa_kernel(const FaParams p) {
       // instructions a step.  MFMA tiles of 32 x 32 over 16, half as many, read and write each accumulator twice as often and
       // held the clock at 1.55 GHz where these run at 1.8 (33 k tokens x 24 heads with windows, in 16 % fewer cycles at
       // equal interleaving).  What then made them the faster ones: K's swizzle (see q_chunk_of), and runs of MFMAs in place of
-      // MFMAs and exponentials in turn, see the softmax's bursts.  33 k x 24 1713 -> 1664 us, 16 896 x 24 with a fifth of the
-      // blocks in fp16 712 -> 680, 4608 x 24 from the symbols 116.4 -> 113.1, the layer step of 76 112 x 5120 with two-term
-      // fp8 13 977 -> 13 678.
+      // MFMAs and exponentials in turn, see the softmax's bursts.  33 k x 24 1782 -> 1700 us, 16 896 x 24 with a fifth of the
+      // blocks in fp16 728 -> 693, 4608 x 24 from the symbols 115.9 -> 110.6, the layer step of 76 112 x 5120 with two-term
+      // fp8 14 320 -> 14 002.
       constexpr int kStep = 32;
       // K buffers 0..2 | V buffer 0 | K buffer 3 | V buffers 1..3; Q is staged from K buffer 3 on, so
       // that K(0..2) and V(0) can be requested together with it
@@ -2995,6 +2995,8 @@ extern "C" int64_t fo_sparse_fa_wide_bytes(int64_t max_rows, int32_t num_kv_head
 
 namespace {
 
+int64_t direct_candidates(const fo_attention_args& a) { return static_cast<int64_t>(a.n_blk) * a.symbol_heads; }
+
 // Two workgroups of four wavefronts per CU and the software-pipelined loop, whose row boundaries pass beside the other
 // workgroup's main loop; where there are too few rows for that, the two-phase loop with twice the wavefronts per row.
 // Two-phase against pipelined, us per call.  Where every row is computed (is_full) from 13/8 of a candidate per CU on:
@@ -3006,7 +3008,7 @@ namespace {
 // What it needs besides: partial results of two shares per CU, room in LDS for a row's list (the
 // longest row is bounded by all keep bits where there are several requests), 32-bit copy offsets.
 bool direct_pipe(const fo_attention_args& a, int num_cu) {
-  const int64_t n_cand = static_cast<int64_t>(a.n_blk) * a.symbol_heads;
+  const int64_t n_cand = direct_candidates(a);
   const int64_t nkv = a.max_nnz / (a.batch == 1 ? n_cand : a.symbol_heads), span = (nkv + 1) * kBlockKV * 2;
   const bool enough = a.is_full ? 8 * n_cand >= int64_t(13) * num_cu : 2 * n_cand >= int64_t(5) * num_cu;
   return a.logits_soft_cap <= 0.f && enough && nkv <= kMaxRowBlocksOneGroupDirect &&
@@ -3016,14 +3018,13 @@ bool direct_pipe(const fo_attention_args& a, int num_cu) {
 
 // Whether a share of the pipelined form has fewer rows than its table: a row costs kRowOverheadPipe at least, and a share
 // is no longer than an even part of all cost, kOlderGain / 128 more, or four ninths of the longest row (of 3 and
-// a part thirds 3 are made).
+// a part thirds 3 are made).  (At most 1.01 million keep bits on 256 CUs: a row is counted as one without kept blocks, and all keep
+// bits as set, at the same time.)
 bool direct_table_holds(int64_t n_cand, int64_t max_nnz, int num_cu) {
   const int64_t even = (max_nnz + kRowOverheadPipe * n_cand) / (2 * num_cu), longest = kMaxRowBlocksOneGroupDirect;
   return ((even + 2) * (128 + kOlderGain) / 128 / kRowOverheadPipe + 3 < kDirectShareRows &&
           (4 * longest / 9 + 2) / kRowOverheadPipe + 3 < kDirectShareRows);
 }
-
-int64_t direct_candidates(const fo_attention_args& a) { return static_cast<int64_t>(a.n_blk) * a.symbol_heads; }
 
 // Whether the launch takes its rows straight from the symbols.
 // Candidates that a workgroup's threads can go through at the top of a launch, and keep bits that every workgroup can

@@ -333,8 +333,8 @@ int fo_sparse_fa_run_wide(const void* q, const void* k, const void* v, void* o, 
  * every workgroup can work out for itself.  args: an fo_attention_args.  Returns FO_NOT_DIRECT (and
  * launches nothing) for a batch that has to be decoded first: fp8 q/k, more than 1024 (symbol row, head)
  * candidates (1792 in the software-pipelined form, 1408 of them where is_full; up to 2047: see
- * fo_sparse_attention_direct_own), more than 2^20 keep bits, no split workspace of
- * fo_sparse_fa_split_workspace_bytes() bytes.
+ * fo_sparse_attention_direct_own), more than 2^20 keep bits (beyond 1024 candidates 1.01 million on 256 CUs, as many as the
+ * table of a workgroup's rows is sure to hold), no split workspace of fo_sparse_fa_split_workspace_bytes() bytes.
  * With twice that many bytes, from 2.5 candidates per CU on (1.625 where is_full) and where a row has at most 1024 kv blocks (of one
  * request: the share of keep bits of a candidate; of several: all kv blocks), the launch runs in the
  * software-pipelined form, two workgroups per CU.
